@@ -278,6 +278,21 @@ int jf_block_colsum(const int8_t *q, const void *s, int R, int C, int scale_dtyp
 int jf_rowstats_finish(const float *rowsum, const float *rowsq, int R, int parts, int C, float *mean, float *rstd,
                        jf_stream_t stream);
 
+/* Causal self-attention between the QKV projection and the output projection, binary16 in and out.  q, k, v: [B*T, ld]
+ * with head h of a row at columns h*D .. h*D + D - 1 of each pointer (the three column ranges of the projection's output,
+ * ld = 3*H*D, or tensors of their own); out: [B*T, H*D]; lse: [B*H, T] fp32, log2 of the row sums (for the backward call).
+ * D = 32 or 64, T a multiple of 32, pointers 16-byte aligned.  Scores, sums and products accumulate in fp32; probabilities
+ * enter the second product in binary16.  Replaces scaled_dot_product_attention of the reference's recipe
+ * (INT8_GPT2/qmodel.py:134). */
+int jf_attention_fwd(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale, void *out,
+                     float *lse, jf_stream_t stream);
+
+/* Its gradients: gq, gk, gv ([B*T, ldg], laid out like q, k, v) from gout [B*T, H*D] and the forward's out and lse.
+ * delta: [B*H, T] fp32 scratch.  Every sum has one owner and a fixed order: the same bits on every run. */
+int jf_attention_bwd(const void *q, const void *k, const void *v, int ld, const void *out, const void *gout, const float *lse,
+                     int B, int H, int T, int D, float scale, void *gq, void *gk, void *gv, int ldg, float *delta,
+                     jf_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -27,7 +27,10 @@ from Linear.linear import bias_operands
 from Nonlinear import (int8_add_Ifp_Ig16_Ofp_Og_MeanVar, int8_layernorm_backward_add, int8_layernorm_forward, int8_quantize,
                        int8_quantize_concat)
 
+import BlockQuantizeCUDA as BQC     # (Linear puts its folder on the path)
+
 QB = 32
+_jf = BQC.jetfire
 _F8 = torch.float8_e4m3fn
 
 
@@ -190,6 +193,30 @@ def _mlp_backward(saved, fpg, qg, sg, wdtype, res_dtype, bias_dtype=None):
     return (res_g, qg, sg, gw1, gw2, g_ln, (gb1[0].to(bias_dtype) if gb1 else None), (gb2[0].to(bias_dtype) if gb2 else None))
 
 
+class CausalAttention(torch.autograd.Function):
+    """Causal self-attention on the projection's output where it lies (q, k, v: views [B, T, C] of it; qmodel.py:134), by the
+    library's kernels: heads 32 or 64 wide, binary16.  The three gradients leave as views of one [B, T, 3C] tensor."""
+
+    @staticmethod
+    def applies(q, n_head):
+        return q.dtype == torch.float16 and q.shape[-1] // n_head in (32, 64) and q.shape[1] % QB == 0
+
+    @staticmethod
+    def forward(ctx, q, k, v, n_head):
+        B, T, C = q.shape
+        q, k, v = (t.reshape(B * T, C) for t in (q, k, v))
+        y, lse = _jf.attention_fwd(q, k, v, B, n_head)
+        ctx.save_for_backward(q, k, v, y, lse)
+        ctx.shape, ctx.n_head = (B, T, C), n_head
+        return y.view(B, T, C)
+
+    @staticmethod
+    def backward(ctx, g):
+        B, T, C = ctx.shape
+        g = _jf.attention_bwd(*ctx.saved_tensors, g.reshape(B * T, C).contiguous(), B, ctx.n_head).view(B, T, 3 * C)
+        return (*g.split(C, dim=-1), None)
+
+
 class AttentionOut(torch.autograd.Function):
     """Output projection + residual add, producing the statistics of the next LayerNorm (qmodel.py:134-171)."""
 
@@ -276,8 +303,11 @@ class QBlock(nn.Module):
     def forward(self, x, qx, sx, mean, rstd):
         B, T, C = x.shape
         res, q, k, v = AttentionIn.apply(x, qx, sx, self.w_qkv, self.ln_1, mean, rstd, self.b_qkv)
-        q, k, v = (t.view(B, T, self.n_head, C // self.n_head).transpose(1, 2) for t in (q, k, v))
-        y = F.scaled_dot_product_attention(q, k, v, is_causal=True).transpose(1, 2).contiguous().view(B, T, C)
+        if CausalAttention.applies(q, self.n_head):
+            y = CausalAttention.apply(q, k, v, self.n_head)
+        else:
+            q, k, v = (t.view(B, T, self.n_head, C // self.n_head).transpose(1, 2) for t in (q, k, v))
+            y = F.scaled_dot_product_attention(q, k, v, is_causal=True).transpose(1, 2).contiguous().view(B, T, C)
         return AttentionOutMLP.apply(res, y, self.w_attn_proj, self.w_fc, self.w_mlp_proj, self.ln_2, self.out_dtype,
                                      self.b_attn_proj, self.b_fc, self.b_mlp_proj)
 

@@ -22,7 +22,9 @@ CSRC = os.path.join(HERE, "csrc")
 HIP_LIB = os.path.join(HERE, "libjetfire_hip.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-HIP_SOURCES = ["jf_gemm.hip", "jf_blockops.hip"]
+# (source, flags of its own).  The attention's maxima are taken over finite scores and -inf: without the flag every one of
+# them carries a canonicalisation for NaN operands.
+HIP_SOURCES = [("jf_gemm.hip", []), ("jf_blockops.hip", []), ("jf_attention.hip", ["-fno-honor-nans"])]
 PROF_LIB = os.path.join(HERE, "libjetfire_prof.so")
 PROF_SOURCES = [("jf_gemm.hip", ["-DJF_PROF_LIB"], "jf_gemm_prof.o"), ("jf_calib.hip", [], "jf_calib.o")]
 HIP_FLAGS = [
@@ -52,9 +54,9 @@ def build_hip():
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     jobs, prof_jobs = [], []
-    for src in HIP_SOURCES:
+    for src, extra in HIP_SOURCES:
         obj = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
-        cmd = [hipcc] + flags + ["-c", os.path.join(CSRC, src), "-o", obj]
+        cmd = [hipcc] + flags + extra + ["-c", os.path.join(CSRC, src), "-o", obj]
         print("+", " ".join(cmd), flush=True)
         jobs.append((cmd, obj, subprocess.Popen(cmd)))
     for src, extra, name in PROF_SOURCES:

@@ -10,6 +10,7 @@
 // use exactly these (tests, captured graphs).
 #include "bqc_common.h"
 
+#include <cmath>
 #include <vector>
 
 namespace jfext {
@@ -370,6 +371,60 @@ std::tuple<Tensor, Tensor> gelu_bwd(const Tensor &qx, const Tensor &sx, const Te
     return std::make_tuple(qy, sy);
 }
 
+// ---- causal self-attention (qmodel.py:134) ---------------------------------------------------------------------------
+
+// q, k, v: [B*T, C] binary16 views of one row stride (column ranges of the QKV projection's output), heads D = C/heads wide
+struct AttentionOperands {
+    int B, H, T, D, ld;
+    int64_t C;
+    float scale;
+};
+AttentionOperands attention_operands(const Tensor &q, const Tensor &k, const Tensor &v, int64_t batch, int64_t heads)
+{
+    for (const Tensor *t : {&q, &k, &v})
+        TORCH_CHECK(t->is_cuda() && t->dim() == 2 && t->scalar_type() == torch::kFloat16 && t->stride(1) == 1 && t->sizes() == q.sizes() &&
+                        t->stride(0) == q.stride(0) && t->device() == q.device(),
+                    "attention: q, k, v must be float16 [tokens, C] GPU tensors of one shape, row stride and device");
+    const int64_t M = q.size(0), C = q.size(1);
+    TORCH_CHECK(batch > 0 && heads > 0 && M % batch == 0 && C % heads == 0, "attention: ", q.sizes(), " does not split into ", batch,
+                " sequences and ", heads, " heads");
+    const int64_t D = C / heads;
+    return {(int)batch, (int)heads, (int)(M / batch), (int)D, (int)q.stride(0), C, (float)(1.0 / std::sqrt((double)D))};
+}
+
+std::tuple<Tensor, Tensor> attention_fwd(const Tensor &q, const Tensor &k, const Tensor &v, int64_t batch, int64_t heads)
+{
+    const AttentionOperands a = attention_operands(q, k, v, batch, heads);
+    c10::DeviceGuard guard(q.device());
+    Tensor out = torch::empty({q.size(0), a.C}, q.options()), lse = torch::empty({(int64_t)a.B * a.H, a.T}, q.options().dtype(torch::kFloat32));
+    pybind11::gil_scoped_release nogil;
+    check_rc(jf_attention_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), a.ld, a.B, a.H, a.T, a.D, a.scale, out.data_ptr(),
+                              lse.data_ptr<float>(), current_stream(q)),
+             "attention_fwd");
+    return std::make_tuple(out, lse);
+}
+
+// the gradients side by side, [B*T, 3C]
+Tensor attention_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &out, const Tensor &lse, const Tensor &gout,
+                     int64_t batch, int64_t heads)
+{
+    const AttentionOperands a = attention_operands(q, k, v, batch, heads);
+    for (const Tensor *t : {&out, &gout}) {
+        need(*t, "attention: out / its gradient", 2);
+        TORCH_CHECK(t->scalar_type() == torch::kFloat16 && t->sizes() == q.sizes() && t->device() == q.device(),
+                    "attention: out and its gradient must be float16 tensors of the shape of q");
+    }
+    vec(lse.reshape({-1}), q.size(0) * a.H, q, "lse");
+    c10::DeviceGuard guard(q.device());
+    Tensor g = torch::empty({q.size(0), 3 * a.C}, q.options()), delta = torch::empty_like(lse);
+    c10::Half *gp = g.data_ptr<c10::Half>();
+    pybind11::gil_scoped_release nogil;
+    check_rc(jf_attention_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), a.ld, out.data_ptr(), gout.data_ptr(), lse.data_ptr<float>(), a.B,
+                              a.H, a.T, a.D, a.scale, gp, gp + a.C, gp + 2 * a.C, (int)(3 * a.C), delta.data_ptr<float>(), current_stream(q)),
+             "attention_bwd");
+    return g;
+}
+
 // ---- column sums (bias gradient; QBlockLinear.py:63-66) -------------------------------------------------------------
 
 Tensor block_colsum(const Tensor &q, const Tensor &s)
@@ -540,6 +595,10 @@ void register_jetfire_ops(pybind11::module &m)
     m.def("add", &add, py::arg("x1"), py::arg("q2"), py::arg("s2"), py::arg("rounding") = JF_ROUND_TRUNC, py::arg("with_stats") = false,
           py::arg("out_dtype") = none, py::arg("seed") = none, py::arg("offset") = none,
           "(y1, codes, scales, mean or None, rstd or None)");
+    m.def("attention_fwd", &attention_fwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("batch"), py::arg("heads"),
+          "(out [tokens, C], lse [batch*heads, T]) of causal self-attention; heads 32 or 64 wide");
+    m.def("attention_bwd", &attention_bwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("out"), py::arg("lse"), py::arg("gout"),
+          py::arg("batch"), py::arg("heads"), "gradients of q, k, v side by side, [tokens, 3C]");
     m.def("block_colsum", &block_colsum, py::arg("q"), py::arg("s"), "fp32 column sums of a block tensor (bias gradient)");
     m.def("igemm_block_q", &igemm_block_q, py::arg("A"), py::arg("B"), py::arg("sa"), py::arg("sb"), py::arg("b_layout") = JF_B_KN,
           py::arg("bias") = none, py::arg("biasmax") = none, py::arg("rounding") = JF_ROUND_NEAREST, py::arg("seed") = none,

@@ -1,0 +1,46 @@
+"""The recipe's causal attention kernels against attention evaluated in float32 on the CPU, at the edges of their tiles: one
+row block, ragged last tiles, one, two and four waves per workgroup, head counts that do not divide by the 8 XCDs, operands
+that are column ranges of one tensor."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(qkv, g, B, H, T, D):
+    x = qkv.float().cpu().view(B, T, 3, H, D).permute(2, 0, 3, 1, 4).contiguous().requires_grad_(True)
+    s = (x[0] @ x[1].transpose(-1, -2).contiguous()) * D ** -0.5
+    s = s.masked_fill(~torch.ones(T, T, dtype=torch.bool).tril(), float("-inf"))
+    o = (torch.softmax(s, -1) @ x[2]).transpose(1, 2).reshape(B * T, H * D)
+    o.backward(g.float().cpu())
+    return o.detach(), x.grad.permute(1, 3, 0, 2, 4).reshape(B * T, 3 * H * D)
+
+
+def rel(a, b):
+    return float((a.float().cpu() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("B,H,T,D", [(1, 1, 32, 64), (2, 3, 64, 64), (1, 5, 96, 32), (2, 4, 160, 64), (37, 7, 160, 64), (70, 8, 96, 32),
+                                     (20, 9, 288, 64), (1, 2, 1056, 64)])
+@pytest.mark.parametrize("scale", [1.0, 6.0])
+def test_causal_attention(B, H, T, D, scale):
+    import BlockQuantizeCUDA as BQC
+    jf, C = BQC.jetfire, H * D
+    gen = torch.Generator().manual_seed(B * 1000 + T)
+    qkv = (torch.randn(B * T, 3 * C, generator=gen) * scale).half().cuda()     # (scale 6: peaked rows, the running maximum moves)
+    g = (torch.randn(B * T, C, generator=gen) * 1e-2).half().cuda()
+    q, k, v = qkv.split(C, dim=1)
+    print(f"case B={B} H={H} T={T} D={D} scale={scale}", flush=True)
+    out, lse = jf.attention_fwd(q, k, v, B, H)
+    grads = jf.attention_bwd(q, k, v, out, lse, g, B, H)
+    want, want_g = reference(qkv, g, B, H, T, D)
+    assert rel(out, want) < 1e-3
+    for i in range(3):
+        assert rel(grads[:, i * C:(i + 1) * C], want_g[:, i * C:(i + 1) * C]) < 2e-3, i
+    out2, lse2 = jf.attention_fwd(q.contiguous(), k.contiguous(), v.contiguous(), B, H)
+    assert torch.equal(out, out2) and torch.equal(lse, lse2)                   # operands of their own: same bits
+    assert torch.equal(grads, jf.attention_bwd(q, k, v, out, lse, g, B, H))    # and on every run
+    with pytest.raises(RuntimeError):
+        jf.attention_fwd(q, k, v.float(), B, H)
+    with pytest.raises(RuntimeError):
+        jf.attention_fwd(q[: 16 * B], k[: 16 * B], v[: 16 * B], B, H)          # rows that are not whole blocks
