@@ -182,6 +182,12 @@ int jf_quantize(const void *x, int x_dtype, int R, int C, int8_t *q, void *s, in
                 int scale_dtype, int rounding, uint64_t seed, uint64_t offset, float amax_eps,
                 jf_stream_t stream);
 
+/* jf_quantize (round to nearest, no amax_eps) of n <= 8 separate tensors of one type in one launch: tensor k is x[k],
+ * [R[k], C[k]], its block tensor (q[k], s[k]) (x, R, C, q, s are HOST arrays).  For the weights of a layer or a block, which the
+ * reference quantises one by one (INT8_GPT2/qmodel.py:92,139,199-200). */
+int jf_quantize_many(int n, const void *const *x, const int *R, const int *C, int x_dtype, int8_t *const *q, void *const *s,
+                     int scale_dtype, jf_stream_t stream);
+
 /* jf_quantize of a tensor that exists only as column slabs lying side by side: slab k is x[k], [R, widths[k]] with rows
  * ldx[k] elements apart (nslabs <= 4; x, ldx, widths are HOST arrays); (q, s) is the block tensor of the concatenation,
  * [R, sum of widths].  Rounding noise is drawn by position in the result, so the codes are those jf_quantize gives for
@@ -206,6 +212,10 @@ int jf_transpose_s8(const int8_t *in, int R, int C, int8_t *out, jf_stream_t str
  * the reference gets them from add_mean_var.py:219-221 or qmodel.py:429-430). */
 int jf_rowstats(const int8_t *q, const void *s, int R, int C, int scale_dtype, float eps,
                 float *mean, float *rstd, jf_stream_t stream);
+
+/* Per-row mean and 1/sqrt(biased variance), no epsilon, of a floating tensor x[R,C] (x_dtype: JF_FP_*): the statistics of a
+ * stack's input (INT8_GPT2/qmodel.py:429-430, torch's mean / var there). */
+int jf_rowstats_fp(const void *x, int x_dtype, int R, int C, float *mean, float *rstd, jf_stream_t stream);
 
 /* dequant -> (x-mean)*rstd*gamma + beta -> requant.  beta may be NULL.
  * Replaces int8_layernorm_forward (Jetfire/Nonlinear/layernorm.py:430-465). */

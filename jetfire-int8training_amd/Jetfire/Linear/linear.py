@@ -2,9 +2,9 @@
 
 Data format everywhere: codes int8 [..., R, C] with one scale per 32x32 tile, scales [..., R/32, C/32]
 (float16 as in the reference, float32 accepted).  The GEMM entry points take their scale operands as [K/32, rows/32];
-the reference makes transposed copies for that (linear_fwd.py:17-18, linear_bwd.py:11), here the .t() VIEW of the
-block tensor's own scale array is passed and the kernel reads it in place.  The zero bias the reference allocates on
-every call (linear_fwd.py:20-21) is kept per device and width.  The weight-gradient GEMM reads the gradient
+the reference makes transposed copies for that (linear_fwd.py:17-18, linear_bwd.py:11), here the kernel reads the block
+tensor's own scale array in place, and no bias is no operand (the reference allocates a zero bias on every call,
+linear_fwd.py:20-21).  The weight-gradient GEMM reads the gradient
 [tokens, C_out] in place as its [K, M] operand when no pre-transposed copy is supplied (G8T=None); the reference needs
 the copy (linear_bwd.py:21, made by int8_transpose / int8_quantize_transpose).
 
@@ -13,7 +13,8 @@ Bias (sketched in the reference, JetfireGEMMKernel/BlockQuantize/QBlockLinear.py
 biasmax = max|bias| added to the block absmax (…BiasRowCol.cu:313,357); `bias_grad=True` of the backward functions
 also returns the bias gradient, the column sums of the (dequantised) output gradient.
 
-Every kernel is reached through the C++ extension (BlockQuantizeCUDA and its submodule BlockQuantizeCUDA.jetfire).
+Every function here is one call of the C++ extension (BlockQuantizeCUDA.jetfire), which reads the leading dimensions,
+validates, allocates and enqueues: the views and reshapes this took in Python were most of a small call's time.
 """
 import os
 import sys
@@ -29,30 +30,10 @@ import BlockQuantizeCUDA as BQC  # noqa: E402
 _jf = BQC.jetfire       # GEMMs with fused epilogues, column sums
 
 
-def _flat2(t):
-    """[..., C] -> [prod(...), C] without copying when possible."""
-    return t.reshape(-1, t.shape[-1])
-
-
-def _k_major(s2d):
-    """[rows/32, K/32] -> [K/32, rows/32] without a copy (the extension accepts this view)."""
-    return s2d.contiguous().t()
-
-
-_ZERO_BIAS = {}
-
-
-def _zero_bias(n, device):
-    key = (str(device), n)
-    if key not in _ZERO_BIAS:
-        _ZERO_BIAS[key] = (torch.zeros(n, dtype=torch.float32, device=device), torch.zeros(1, dtype=torch.float32, device=device))
-    return _ZERO_BIAS[key]
-
-
 def bias_operands(bias, n_out, device):
-    """(bias as contiguous float32 [N], biasmax = max|bias| as float32 [1]) for the kernel; the zero pair for None."""
+    """(bias as contiguous float32 [N], biasmax = max|bias| as float32 [1]) for the kernel; no pair for None."""
     if bias is None:
-        return _zero_bias(n_out, device)
+        return None, None
     if bias.numel() != n_out:
         raise RuntimeError(f"bias must have {n_out} elements, got {bias.numel()}")
     b = bias.detach().reshape(-1).to(torch.float32).contiguous()
@@ -76,21 +57,10 @@ def int8_linear_forward(X8_3D, SX16_3D, W8, SW16, output_quantized, B, bias=None
     Returns (O8 [BS,T,N], SO [BS,T/32,N/32]) or, with output_quantized=False, the dequantised
     output in the scale dtype (reference: linear_fwd.py:4-32; bias: QBlockLinear.py:38-39)."""
     _check_block(B)
-    lead = tuple(X8_3D.shape[:-1])
-    s_lead = tuple(SX16_3D.shape[:-1])
-    x2 = _flat2(X8_3D)
-    sx2 = _flat2(SX16_3D)
-    n_out = W8.shape[0]
-    m, k = x2.shape
-    b, bmax = _bias_pair(bias, n_out, W8.device)
-    if not output_quantized:
-        # the quantising GEMM and the codes x scales product of the reference (linear_fwd.py:22-31) in one kernel: same bits
-        out = _jf.igemm_block_q_dequant(x2.contiguous(), W8.contiguous(), _k_major(sx2), _k_major(SW16), _jf.B_NK,
-                                        SW16.dtype, b, bmax)
-        return out.reshape(*lead, n_out)
-    o8, so = BQC.igemm_output_int_quantize_bias_rowcol(x2.contiguous(), W8.t(), b, bmax,
-                                                       _k_major(sx2), _k_major(SW16), m, n_out, k)
-    return o8.reshape(*lead, n_out), so.reshape(*s_lead, SW16.shape[0])
+    b, bmax = (None, None) if bias is None else _bias_pair(bias, W8.shape[0], W8.device)
+    # unquantised: the quantising GEMM and the codes x scales product of the reference (linear_fwd.py:22-31) in one kernel
+    o, so = _jf.linear_forward(X8_3D, SX16_3D, W8, SW16, bool(output_quantized), b, bmax)
+    return (o, so) if output_quantized else o
 
 
 def int8_linear_forward_gelu(X8_3D, SX16_3D, W8, SW16, B, approximate="none", bias=None):
@@ -100,16 +70,10 @@ def int8_linear_forward_gelu(X8_3D, SX16_3D, W8, SW16, B, approximate="none", bi
     _check_block(B)
     if approximate not in ("none", "tanh"):
         raise RuntimeError("approximate must be 'none' or 'tanh'")
-    lead, s_lead = tuple(X8_3D.shape[:-1]), tuple(SX16_3D.shape[:-1])
-    x2, sx2 = _flat2(X8_3D).contiguous(), _flat2(SX16_3D)
-    n_out = W8.shape[0]
-    b, bmax = _bias_pair(bias, n_out, W8.device)
-    o8, so, g8, sg = _jf.igemm_block_q_gelu(x2, W8.contiguous(), _k_major(sx2), _k_major(SW16),
-                                            _jf.GELU_TANH if approximate == "tanh" else _jf.GELU_ERF,
-                                            0.0 if approximate == "tanh" else 5e-5,   # as Nonlinear.int8_gelu_forward
-                                            b, bmax)
-    shp, sshp = (*lead, n_out), (*s_lead, SW16.shape[0])
-    return o8.reshape(shp), so.reshape(sshp), g8.reshape(shp), sg.reshape(sshp)
+    b, bmax = (None, None) if bias is None else _bias_pair(bias, W8.shape[0], W8.device)
+    tanh = approximate == "tanh"
+    # (the threshold as in Nonlinear.int8_gelu_forward)
+    return _jf.linear_forward_gelu(X8_3D, SX16_3D, W8, SW16, _jf.GELU_TANH if tanh else _jf.GELU_ERF, 0.0 if tanh else 5e-5, b, bmax)
 
 
 def int8_linear_backward(X8_3D, SX16_3D, G8_3D, SG16_3D, G8T, W8, SW16, B, stochastic=True, dgrad_quantize=True,
@@ -123,24 +87,7 @@ def int8_linear_backward(X8_3D, SX16_3D, G8_3D, SG16_3D, G8T, W8, SW16, B, stoch
     wgrad_dtype (not in the reference): None = float16 as there; float32 / bfloat16 = dW leaves the kernel in that type.
     bias_grad=True appends the bias gradient (float32 [N], the column sums of G8 x SG; QBlockLinear.py:63-66)."""
     _check_block(B)
-    g2, sg2 = _flat2(G8_3D).contiguous(), _flat2(SG16_3D).contiguous()
-    x2, sx2 = _flat2(X8_3D).contiguous(), _flat2(SX16_3D).contiguous()
-    tokens, c_out = g2.shape
-    c_in = W8.shape[1]
-    gb = (_jf.block_colsum(g2, sg2),) if bias_grad else ()
-    if dgrad_quantize:
-        gx8, gsx = BQC.igemm_output_int_quantize_stochastic(g2, W8, _k_major(sg2), SW16, tokens, c_in, c_out)
-    else:
-        # the stochastic quantising GEMM and the codes x scales product of the reference (linear_bwd.py:17,26-28) in one
-        # kernel: same bits, same noise counters
-        gx = _jf.igemm_block_q_dequant(g2, W8.contiguous(), _k_major(sg2), SW16, _jf.B_KN, SW16.dtype, None, None,
-                                       _jf.ROUND_STOCHASTIC)
-    if G8T is None:
-        G8T = g2.t()                                               # a view: the extension reads g2 as the [K, M] operand
-    gw = BQC.igemm_output_fp_no_quantize(G8T, x2, sg2, sx2, G8T.shape[0], c_in, G8T.shape[1], wgrad_splitk, wgrad_dtype)
-    if not dgrad_quantize:
-        return (gx.reshape(*G8_3D.shape[:-1], c_in), gw) + gb
-    return (gx8.reshape(*G8_3D.shape[:-1], c_in), gsx.reshape(*SG16_3D.shape[:-1], SW16.shape[1]), gw) + gb
+    return tuple(_jf.linear_backward(X8_3D, SX16_3D, G8_3D, SG16_3D, G8T, W8, SW16, dgrad_quantize, wgrad_splitk, wgrad_dtype, bias_grad))
 
 
 def int8_linear_backward_gelu(X8_3D, SX16_3D, G8_3D, SG16_3D, W8, SW16, PRE8_3D, SPRE16_3D, B, approximate="none",
@@ -154,14 +101,6 @@ def int8_linear_backward_gelu(X8_3D, SX16_3D, G8_3D, SG16_3D, W8, SW16, PRE8_3D,
     _check_block(B)
     if approximate not in ("none", "tanh"):
         raise RuntimeError("approximate must be 'none' or 'tanh'")
-    g2, sg2 = _flat2(G8_3D).contiguous(), _flat2(SG16_3D).contiguous()
-    x2, sx2 = _flat2(X8_3D).contiguous(), _flat2(SX16_3D).contiguous()
-    p2, sp2 = _flat2(PRE8_3D).contiguous(), _flat2(SPRE16_3D).contiguous()
-    tokens, c_out = g2.shape
-    c_in = W8.shape[1]
-    gp8, gsp = _jf.igemm_block_q_gelu_bwd(g2, W8.contiguous(), _k_major(sg2), SW16, p2, sp2,
+    return tuple(_jf.linear_backward_gelu(X8_3D, SX16_3D, G8_3D, SG16_3D, W8, SW16, PRE8_3D, SPRE16_3D,
                                           _jf.GELU_TANH if approximate == "tanh" else _jf.GELU_ERF,
-                                          _jf.ROUND_STOCHASTIC if stochastic else _jf.ROUND_NEAREST)
-    gw = BQC.igemm_output_fp_no_quantize(g2.t(), x2, sg2, sx2, c_out, c_in, tokens, wgrad_splitk, wgrad_dtype)
-    gb = (_jf.block_colsum(g2, sg2),) if bias_grad else ()
-    return (gp8.reshape(*G8_3D.shape[:-1], c_in), gsp.reshape(*SG16_3D.shape[:-1], SW16.shape[1]), gw) + gb
+                                          _jf.ROUND_STOCHASTIC if stochastic else _jf.ROUND_NEAREST, wgrad_splitk, wgrad_dtype, bias_grad))

@@ -69,6 +69,26 @@ template <typename OT> __device__ __forceinline__ void store16_as(OT *p, const f
 }
 template <> __device__ __forceinline__ void store16_as<float>(float *p, const float x[16]) { store16_f32(p, x); }
 
+// 64-lane sum, every lane returns it (data-parallel-primitive forms of v_add_f32; a fixed tree: pairs, quads, eights,
+// rows of 16, then row 1 += row 0 and row 3 += row 2, then rows 2-3 += rows 0-1; asm for the reason given at wave_max)
+__device__ __forceinline__ float wave_sum(float v)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+                 "s_nop 1\n\t"
+                 "v_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+                 : "+v"(v));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
 // Position of this wave's block / this lane's 16 elements.
 struct BlockPos {
     int rb, cb, row, col;     // block coordinates; absolute row / first column of the lane
@@ -203,6 +223,82 @@ __global__ __launch_bounds__(NT) void quantize_kernel(QuantSrc src, int R, int C
             __builtin_amdgcn_wave_barrier();
         }
     }
+}
+
+// quantize.py:33-117 of up to QMANY_MAX tensors of one type in one launch, round to nearest: the weights of a block, quantised
+// after every optimizer step.  (Four launches for a GPT-2 small block take 23 us, most of it ramp and drain; a 256-wide block
+// spends 16 us on four tensors that need 2.)
+constexpr int QMANY_MAX = 8;
+struct QuantMany {
+    const void *x[QMANY_MAX];
+    int8_t *q[QMANY_MAX];
+    void *s[QMANY_MAX];
+    int C[QMANY_MAX];
+    int end[QMANY_MAX];      // first group (four column blocks of a row block) behind tensor k
+    int n;
+};
+template <typename T, typename ST> __global__ __launch_bounds__(NT) void quantize_many_kernel(QuantMany m)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char line_patches[2 * QB * LINE_PITCH];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    GroupLineStore lines(line_patches, lane, wave);
+    for (int g = blockIdx.x; g < m.end[m.n - 1]; g += gridDim.x) {
+        int k = 0, begin = 0;
+        const T *x = reinterpret_cast<const T *>(m.x[0]);
+        int8_t *q = m.q[0];
+        ST *s = reinterpret_cast<ST *>(m.s[0]);
+        int C = m.C[0];
+#pragma unroll
+        for (k = 1; k < QMANY_MAX; ++k)
+            if (k < m.n && g >= m.end[k - 1]) {
+                begin = m.end[k - 1]; C = m.C[k];
+                x = reinterpret_cast<const T *>(m.x[k]); q = m.q[k]; s = reinterpret_cast<ST *>(m.s[k]);
+            }
+        const int SC = C / QB, G4 = (SC + WPB - 1) / WPB, rb = (g - begin) / G4, cg = (g - begin) - rb * G4, cb = cg * WPB + wave;
+        v4i codes = {0, 0, 0, 0};
+        if (cb < SC) {                                             // wave-uniform
+            BlockPos pos(rb * SC + cb, SC, C, lane);
+            float v[16], scale;
+            Load16<T>::run(x + pos.e0, v);
+            codes = quantize16(v, 0.0f, JF_ROUND_NEAREST, 0, 0, pos.e0, &scale);
+            if (lane == 0) store_scale(s, rb * SC + cb, scale);
+        }
+        lines.store(codes, q, rb, cg, C);
+    }
+}
+
+// Mean and 1/sqrt(biased variance) of the rows of a floating tensor (the LayerNorm statistics of a stack's input,
+// qmodel.py:429-430: two reductions of torch and a square root there).  One wave per row; the second pass over the row, for
+// the variance about the mean, comes out of the caches.
+template <typename T> __global__ __launch_bounds__(NT) void rowstats_fp_kernel(const T *x, int R, int C, float *mean, float *rstd)
+{
+    const int lane = threadIdx.x & 63, row = blockIdx.x * WPB + (threadIdx.x >> 6);
+    if (row >= R) return;
+    const T *p = x + (size_t)row * C;
+    constexpr int PER = 16 / sizeof(T);                            // C is a multiple of 32: whole 16-byte pieces
+    auto piece = [&](int c, float (&f)[PER]) {
+        T t[PER];
+        *reinterpret_cast<v4i *>(t) = *reinterpret_cast<const v4i *>(p + c);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) f[i] = (float)t[i];
+    };
+    float s = 0.0f;
+    for (int c = lane * PER; c < C; c += WAVE * PER) {
+        float f[PER];
+        piece(c, f);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) s = s + f[i];
+    }
+    const float mu = wave_sum(s) / (float)C;
+    float v = 0.0f;
+    for (int c = lane * PER; c < C; c += WAVE * PER) {
+        float f[PER];
+        piece(c, f);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) { const float d = f[i] - mu; v = __builtin_fmaf(d, d, v); }
+    }
+    const float var = wave_sum(v) / (float)C;
+    if (lane == 0) { mean[row] = mu; rstd[row] = 1.0f / __builtin_sqrtf(var); }
 }
 
 // dequantize.py:28-84
@@ -619,26 +715,6 @@ __global__ __launch_bounds__(NT) void layernorm_bwd_stats_kernel(const int8_t *q
         const float tb = colsum16_over_rows(accb, lane, cpatch);
         if ((lane & 1) == 0) pdb[dst] = tb;
     }
-}
-
-// 64-lane sum, every lane returns it (data-parallel-primitive forms of v_add_f32; a fixed tree: pairs, quads, eights,
-// rows of 16, then row 1 += row 0 and row 3 += row 2, then rows 2-3 += rows 0-1; asm for the reason given at wave_max)
-__device__ __forceinline__ float wave_sum(float v)
-{
-    asm volatile("s_nop 1\n\t"
-                 "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-                 "s_nop 1\n\t"
-                 "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-                 "s_nop 1\n\t"
-                 "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-                 "s_nop 1\n\t"
-                 "v_add_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf\n\t"
-                 "s_nop 1\n\t"
-                 "v_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-                 "s_nop 1\n\t"
-                 "v_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-                 : "+v"(v));
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
 template <typename ST>
@@ -1119,6 +1195,52 @@ int jf_quantize(const void *x, int x_dtype, int R, int C, int8_t *q, void *s, in
         JF_Q(__bf16, float);
     }
 #undef JF_Q
+}
+
+int jf_quantize_many(int n, const void *const *x, const int *R, const int *C, int x_dtype, int8_t *const *q, void *const *s,
+                     int scale_dtype, jf_stream_t stream)
+{
+    if (!x || !R || !C || !q || !s) return JF_ERR_NULL;
+    if (n < 1 || n > QMANY_MAX) return JF_ERR_SHAPE;
+    if (x_dtype < JF_FP_F16 || x_dtype > JF_FP_BF16) return JF_ERR_ENUM;
+    QuantMany m = {};
+    long groups = 0;
+    for (int k = 0; k < n; ++k) {
+        int rc = check_block_tensor(q[k], s[k], R[k], C[k], scale_dtype);
+        if (rc) return rc;
+        if (!x[k]) return JF_ERR_NULL;
+        if (!aligned16(x[k])) return JF_ERR_ALIGN;
+        groups += quantize_groups(R[k], C[k], false);
+        if (groups > 0x7fffffffL) return JF_ERR_SHAPE;
+        m.x[k] = x[k]; m.q[k] = q[k]; m.s[k] = s[k]; m.C[k] = C[k]; m.end[k] = (int)groups;
+    }
+    m.n = n;
+    hipStream_t st = (hipStream_t)stream;
+    const int grid = (int)(groups < 256L * 32 ? groups : 256L * 32);
+#define JF_QM(T, ST) JF_LAUNCH((quantize_many_kernel<T, ST>), grid, 0, st, m)
+    if (scale_dtype == JF_SCALE_F16) {
+        if (x_dtype == JF_FP_F32) JF_QM(float, half_t);
+        if (x_dtype == JF_FP_F16) JF_QM(half_t, half_t);
+        JF_QM(__bf16, half_t);
+    } else {
+        if (x_dtype == JF_FP_F32) JF_QM(float, float);
+        if (x_dtype == JF_FP_F16) JF_QM(half_t, float);
+        JF_QM(__bf16, float);
+    }
+#undef JF_QM
+}
+
+int jf_rowstats_fp(const void *x, int x_dtype, int R, int C, float *mean, float *rstd, jf_stream_t stream)
+{
+    if (!x || !mean || !rstd) return JF_ERR_NULL;
+    if (R <= 0 || !mult32(C)) return JF_ERR_SHAPE;
+    if (x_dtype < JF_FP_F16 || x_dtype > JF_FP_BF16) return JF_ERR_ENUM;
+    if (!aligned16(x)) return JF_ERR_ALIGN;
+    hipStream_t st = (hipStream_t)stream;
+    const int grid = (R + WPB - 1) / WPB;
+    if (x_dtype == JF_FP_F32) JF_LAUNCH(rowstats_fp_kernel<float>, grid, 0, st, (const float *)x, R, C, mean, rstd);
+    if (x_dtype == JF_FP_F16) JF_LAUNCH(rowstats_fp_kernel<half_t>, grid, 0, st, (const half_t *)x, R, C, mean, rstd);
+    JF_LAUNCH(rowstats_fp_kernel<__bf16>, grid, 0, st, (const __bf16 *)x, R, C, mean, rstd);
 }
 
 int jf_quantize_slabs(const void *const *x, const int *ldx, const int *widths, int nslabs, int x_dtype, int R,

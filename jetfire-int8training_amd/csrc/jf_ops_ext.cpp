@@ -5,7 +5,8 @@
 // is one C++ call that validates its tensors, allocates the outputs, reserves Philox counters under the generator's
 // mutex, releases the GIL and enqueues the gfx950 kernel on the current stream through the C ABI.
 //
-// All tensors are 2-D ([R, C] codes / values, [R/32, C/32] scales, 1-D vectors); the Python packages fold 3-D operands.
+// Operands are 2-D ([R, C] codes / values, [R/32, C/32] scales) or 3-D ([B, T, C] with [B, T/32, C/32] scales; results then
+// have that rank too), vectors (per row, per column) of any shape with the right number of elements.
 // seed / offset arguments: None = reserve from the device's default generator (what the operator API does); integers =
 // use exactly these (tests, captured graphs).
 #include "bqc_common.h"
@@ -52,28 +53,58 @@ void need(const Tensor &t, const char *name, int64_t dim)
     TORCH_CHECK(t.is_contiguous(), name, ": expected a contiguous tensor");
 }
 
+// a contiguous tensor of 2 to max_dim dimensions, read as [R, C]
+void rows_of(const Tensor &t, const char *name, int64_t &R, int64_t &C, int64_t max_dim = 3)
+{
+    TORCH_CHECK(t.is_cuda(), name, ": expected a GPU tensor");
+    TORCH_CHECK(t.dim() >= 2 && t.dim() <= max_dim, name, ": expected a 2-D or 3-D tensor, got ", t.dim(), " dimensions");
+    TORCH_CHECK(t.is_contiguous(), name, ": expected a contiguous tensor");
+    C = t.size(-1);
+    R = 1;
+    for (int64_t d = 0; d + 1 < t.dim(); ++d) R *= t.size(d);
+}
+
+// the scales of a [R, C] or [B, T, C] tensor
+std::vector<int64_t> scale_shape(const Tensor &x)
+{
+    std::vector<int64_t> n = x.sizes().vec();
+    const int64_t T = n[n.size() - 2];
+    TORCH_CHECK(T % QB == 0, "dimension ", T, " is not a positive multiple of 32");
+    n[n.size() - 2] = T / QB;
+    n[n.size() - 1] /= QB;
+    return n;
+}
+
+// one value per row, [R] or [B, T]
+std::vector<int64_t> row_shape(const Tensor &x)
+{
+    std::vector<int64_t> n = x.sizes().vec();
+    n.pop_back();
+    return n;
+}
+
 void mult32(int64_t d)
 {
     TORCH_CHECK(d > 0 && d % QB == 0, "dimension ", d, " is not a positive multiple of 32");
 }
 
 // (codes [R,C] int8, scales [R/32,C/32]) -> scale code; R, C out
-int block_tensor(const Tensor &q, const Tensor &s, const char *name, int64_t &R, int64_t &C)
+int block_tensor(const Tensor &q, const Tensor &s, const char *name, int64_t &R, int64_t &C, int64_t max_dim = 3)
 {
-    need(q, name, 2);
+    rows_of(q, name, R, C, max_dim);
     TORCH_CHECK(q.scalar_type() == torch::kInt8, name, ": codes must be int8, got ", q.scalar_type());
-    R = q.size(0); C = q.size(1);
     mult32(R); mult32(C);
-    need(s, name, 2);
-    TORCH_CHECK(s.size(0) == R / QB && s.size(1) == C / QB, name, ": scale shape ", s.sizes(), " does not match codes ", q.sizes());
+    int64_t SR, SC;
+    rows_of(s, name, SR, SC, max_dim);
+    TORCH_CHECK(SR == R / QB && SC == C / QB, name, ": scale shape ", s.sizes(), " does not match codes ", q.sizes());
     TORCH_CHECK(s.device() == q.device(), name, ": codes and scales are on different devices");
     return scale_code(s, name);
 }
 
 const float *vec(const Tensor &v, int64_t n, const Tensor &like, const char *name)
 {
-    need(v, name, 1);
-    TORCH_CHECK(v.scalar_type() == torch::kFloat32 && v.numel() == n && v.device() == like.device(), name,
+    TORCH_CHECK(v.is_cuda(), name, ": expected a GPU tensor");
+    TORCH_CHECK(v.is_contiguous() && v.scalar_type() == torch::kFloat32 && v.numel() == n && v.device() == like.device(), name,
                 ": expected a float32 vector of ", n, " elements on ", like.device());
     return v.data_ptr<float>();
 }
@@ -96,16 +127,16 @@ Tensor scratch(const Tensor &like, size_t bytes)
 std::tuple<Tensor, Tensor, OptTensor> quantize(const Tensor &x, int64_t rounding, OptDtype scale_dtype_o, bool transpose,
                                                double amax_eps, OptU64 seed, OptU64 offset)
 {
-    need(x, "x", 2);
+    int64_t R, C;
+    rows_of(x, "x", R, C);
     const int xc = fp_code(x.scalar_type(), "x");
-    const int64_t R = x.size(0), C = x.size(1);
     mult32(R); mult32(C);
     check_rounding(rounding, true);
     const torch::ScalarType scale_dtype = scale_dtype_o.value_or(torch::kFloat16);
     const int sc = scale_code_of(scale_dtype);
     c10::DeviceGuard guard(x.device());
-    Tensor q = torch::empty({R, C}, x.options().dtype(torch::kInt8));
-    Tensor s = torch::empty({R / QB, C / QB}, x.options().dtype(scale_dtype));
+    Tensor q = torch::empty(x.sizes(), x.options().dtype(torch::kInt8));
+    Tensor s = torch::empty(scale_shape(x), x.options().dtype(scale_dtype));
     OptTensor qT;
     if (transpose) qT = torch::empty({C, R}, x.options().dtype(torch::kInt8));
     const auto so = rng(rounding, x, R * C, seed, offset);
@@ -117,6 +148,47 @@ std::tuple<Tensor, Tensor, OptTensor> quantize(const Tensor &x, int64_t rounding
                  "quantize");
     }
     return std::make_tuple(q, s, qT);
+}
+
+// several floating tensors (weights) in one launch, round to nearest: [(codes, scales), ...]
+std::vector<std::tuple<Tensor, Tensor>> quantize_many(const std::vector<Tensor> &xs, OptDtype scale_dtype_o)
+{
+    TORCH_CHECK(!xs.empty() && xs.size() <= 8, "between 1 and 8 tensors");
+    const torch::ScalarType scale_dtype = scale_dtype_o.value_or(torch::kFloat16);
+    const int sc = scale_code_of(scale_dtype), xc = fp_code(xs[0].scalar_type(), "xs"), n = (int)xs.size();
+    c10::DeviceGuard guard(xs[0].device());
+    std::vector<std::tuple<Tensor, Tensor>> out;
+    const void *xp[8];
+    int Rs[8], Cs[8];
+    int8_t *qp[8];
+    void *sp[8];
+    for (int k = 0; k < n; ++k) {
+        const Tensor &x = xs[k];
+        int64_t R, C;
+        rows_of(x, "xs", R, C);
+        mult32(R); mult32(C);
+        TORCH_CHECK(x.scalar_type() == xs[0].scalar_type() && x.device() == xs[0].device(), "xs: expected tensors of one type and device");
+        Tensor q = torch::empty(x.sizes(), x.options().dtype(torch::kInt8)), s = torch::empty(scale_shape(x), x.options().dtype(scale_dtype));
+        xp[k] = x.data_ptr(); Rs[k] = (int)R; Cs[k] = (int)C; qp[k] = (int8_t *)q.data_ptr(); sp[k] = s.data_ptr();
+        out.emplace_back(std::move(q), std::move(s));
+    }
+    pybind11::gil_scoped_release nogil;
+    check_rc(jf_quantize_many(n, xp, Rs, Cs, xc, qp, sp, sc, current_stream(xs[0])), "quantize_many");
+    return out;
+}
+
+// per-row mean and 1/sqrt(biased variance) of a floating tensor (qmodel.py:429-430)
+std::tuple<Tensor, Tensor> rowstats_fp(const Tensor &x)
+{
+    int64_t R, C;
+    rows_of(x, "x", R, C);
+    mult32(C);
+    const int xc = fp_code(x.scalar_type(), "x");
+    c10::DeviceGuard guard(x.device());
+    Tensor mean = torch::empty(row_shape(x), x.options().dtype(torch::kFloat32)), rstd = torch::empty_like(mean);
+    pybind11::gil_scoped_release nogil;
+    check_rc(jf_rowstats_fp(x.data_ptr(), xc, (int)R, (int)C, mean.data_ptr<float>(), rstd.data_ptr<float>(), current_stream(x)), "rowstats_fp");
+    return std::make_tuple(mean, rstd);
 }
 
 // the block tensor of torch.cat(slabs, dim=1) without the concatenation (jf_quantize_slabs)
@@ -164,7 +236,7 @@ Tensor dequantize(const Tensor &q, const Tensor &s, OptDtype out_dtype_o)
     const int sc = block_tensor(q, s, "x", R, C);
     const int oc = fp_code(out_dtype, "out_dtype");
     c10::DeviceGuard guard(q.device());
-    Tensor out = torch::empty({R, C}, q.options().dtype(out_dtype));
+    Tensor out = torch::empty(q.sizes(), q.options().dtype(out_dtype));
     pybind11::gil_scoped_release nogil;
     check_rc(jf_dequantize((const int8_t *)q.data_ptr(), s.data_ptr(), (int)R, (int)C, sc, out.data_ptr(), oc, current_stream(q)),
              "dequantize");
@@ -174,9 +246,9 @@ Tensor dequantize(const Tensor &q, const Tensor &s, OptDtype out_dtype_o)
 // transpose.py:69-97
 Tensor transpose_s8(const Tensor &q)
 {
-    need(q, "x", 2);
+    int64_t R, C;
+    rows_of(q, "x", R, C);
     TORCH_CHECK(q.scalar_type() == torch::kInt8, "x must be int8");
-    const int64_t R = q.size(0), C = q.size(1);
     TORCH_CHECK(R > 0 && C > 0 && R % 16 == 0 && C % 16 == 0, "transpose: dimensions must be positive multiples of 16");
     c10::DeviceGuard guard(q.device());
     Tensor out = torch::empty({C, R}, q.options());
@@ -192,7 +264,7 @@ std::tuple<Tensor, Tensor> rowstats(const Tensor &q, const Tensor &s, double eps
     int64_t R, C;
     const int sc = block_tensor(q, s, "x", R, C);
     c10::DeviceGuard guard(q.device());
-    Tensor mean = torch::empty({R}, q.options().dtype(torch::kFloat32)), rstd = torch::empty_like(mean);
+    Tensor mean = torch::empty(row_shape(q), q.options().dtype(torch::kFloat32)), rstd = torch::empty_like(mean);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_rowstats((const int8_t *)q.data_ptr(), s.data_ptr(), (int)R, (int)C, sc, (float)eps, mean.data_ptr<float>(),
                          rstd.data_ptr<float>(), current_stream(q)),
@@ -254,19 +326,20 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor, OptTensor> add(const Tensor &x1, c
     const torch::ScalarType out_dtype = out_dtype_o.value_or(torch::kFloat32);
     int64_t R, C;
     const int sc = block_tensor(q2, s2, "x2", R, C);
-    need(x1, "x1", 2);
+    int64_t R1, C1;
+    rows_of(x1, "x1", R1, C1);
     const int xc = fp_code(x1.scalar_type(), "x1"), oc = fp_code(out_dtype, "out_dtype");
-    TORCH_CHECK(x1.size(0) == R && x1.size(1) == C && x1.device() == q2.device(), "x1 must be a float tensor of the shape and device of x2");
+    TORCH_CHECK(R1 == R && C1 == C && x1.device() == q2.device(), "x1 must be a float tensor of the shape and device of x2");
     check_rounding(rounding, true);
     c10::DeviceGuard guard(x1.device());
-    Tensor y1 = torch::empty({R, C}, x1.options().dtype(out_dtype));
-    Tensor q = torch::empty_like(q2), s = torch::empty_like(s2);
+    Tensor y1 = torch::empty(x1.sizes(), x1.options().dtype(out_dtype));
+    Tensor q = torch::empty(x1.sizes(), q2.options()), s = torch::empty(scale_shape(x1), s2.options());
     Tensor rs, rq;
     OptTensor mean, rstd;
     if (with_stats) {
         rs = torch::empty({C / QB, R}, x1.options().dtype(torch::kFloat32));          // part-major
         rq = torch::empty_like(rs);
-        mean = torch::empty({R}, x1.options().dtype(torch::kFloat32));
+        mean = torch::empty(row_shape(x1), x1.options().dtype(torch::kFloat32));
         rstd = torch::empty_like(*mean);
     }
     const auto so = rng(rounding, x1, R * C, seed, offset);
@@ -300,9 +373,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor> layernorm_bwd_add(const Te
     TORCH_CHECK(block_tensor(qg, sg, "g", R2, C2) == sc && R2 == R && C2 == C && qg.device() == qx.device(),
                 "x and g must have the same shape, scale dtype and device");
     const float *g = vec(gamma, C, qx, "gamma"), *m = vec(mean, R, qx, "mean"), *r = vec(rstd, R, qx, "rstd");
-    need(x1, "x1", 2);
+    int64_t R1, C1;
+    rows_of(x1, "x1", R1, C1);
     const int xc = fp_code(x1.scalar_type(), "x1"), oc = fp_code(out_dtype, "out_dtype");
-    TORCH_CHECK(x1.size(0) == R && x1.size(1) == C && x1.device() == qx.device(), "x1 must be a float tensor of the shape and device of x");
+    TORCH_CHECK(R1 == R && C1 == C && x1.device() == qx.device(), "x1 must be a float tensor of the shape and device of x");
     check_rounding(rounding, true);
     check_rounding(add_rounding, true);
     const auto so = rng(rounding, qx, R * C, seed, offset);
@@ -315,7 +389,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor> layernorm_bwd_add(const Te
     c10::DeviceGuard guard(qx.device());
     const size_t nbytes = jf_layernorm_bwd_workspace_bytes((int)R, (int)C);
     Tensor ws = scratch(qx, nbytes);
-    Tensor y1 = torch::empty({R, C}, x1.options().dtype(out_dtype));
+    Tensor y1 = torch::empty(qx.sizes(), x1.options().dtype(out_dtype));
     Tensor q = torch::empty_like(qx), s = torch::empty_like(sx);
     Tensor dgamma = torch::empty({C}, qx.options().dtype(torch::kFloat32));
     OptTensor dbeta;
@@ -558,6 +632,173 @@ std::tuple<Tensor, Tensor> igemm_block_q(const Tensor &A, const Tensor &B, const
     return std::make_tuple(out, sc);
 }
 
+// ---- package Linear (linear_fwd.py:4-32, linear_bwd.py:4-29) -------------------------------------------------------------
+
+// an int8 operand [.., rows, cols] with its scales in the block tensor's own layout
+struct Operand {
+    Tensor q, s;
+    int64_t R, C;
+    int code;
+    Operand(const Tensor &q_, const Tensor &s_, const char *name) : q(q_.contiguous()), s(s_.contiguous()) { code = block_tensor(q, s, name, R, C, 8); }
+    int8_t *qp() const { return (int8_t *)q.data_ptr(); }
+    void *sp() const { return s.data_ptr(); }
+};
+
+void same_kind(const Operand &a, const Operand &b)
+{
+    TORCH_CHECK(a.code == b.code, "scales must have the same dtype");
+    TORCH_CHECK(a.q.device() == b.q.device(), "operands are on different devices");
+}
+
+// the sizes of x with another last dimension
+std::vector<int64_t> with_last(const Tensor &x, int64_t n)
+{
+    std::vector<int64_t> v = x.sizes().vec();
+    v.back() = n;
+    return v;
+}
+
+void linear_bias(const OptTensor &bias, const OptTensor &biasmax, const Operand &x, int64_t N, const float *&b, const float *&bm)
+{
+    b = bm = nullptr;
+    TORCH_CHECK(bias.has_value() == biasmax.has_value(), "bias and biasmax come together");
+    if (!bias) return;
+    b = vec(*bias, N, x.q, "bias");
+    TORCH_CHECK(biasmax->is_cuda() && biasmax->device() == x.q.device() && biasmax->scalar_type() == torch::kFloat32 && biasmax->numel() >= 1,
+                "biasmax must be a float32 GPU tensor with one element");
+    bm = biasmax->data_ptr<float>();
+}
+
+// Y = X W^T (+ bias): (codes, scales), or (values in the scale type, None) with quantized = false
+std::tuple<Tensor, OptTensor> linear_forward(const Tensor &X, const Tensor &SX, const Tensor &W, const Tensor &SW, bool quantized,
+                                             const OptTensor &bias, const OptTensor &biasmax)
+{
+    const Operand x(X, SX, "X"), w(W, SW, "W");
+    same_kind(x, w);
+    TORCH_CHECK(w.q.dim() == 2 && x.C == w.C, "inner dimensions differ: X is ", X.sizes(), ", W is ", W.sizes());
+    const float *b, *bm;
+    linear_bias(bias, biasmax, x, w.R, b, bm);
+    c10::DeviceGuard guard(x.q.device());
+    if (!quantized) {
+        Tensor out = torch::empty(with_last(x.q, w.R), x.s.options());
+        pybind11::gil_scoped_release nogil;
+        check_rc(jf_igemm_block_q_dequant(x.qp(), w.qp(), x.sp(), w.sp(), b, bm, out.data_ptr(), (int)x.R, (int)w.R, (int)x.C, JF_B_NK, x.code,
+                                          JF_SCALES_ROWMAJOR, JF_SCALES_ROWMAJOR, x.code == JF_SCALE_F16 ? JF_FP_F16 : JF_FP_F32,
+                                          JF_ROUND_NEAREST, 0, 0, current_stream(x.q)),
+                 "linear_forward");
+        return std::make_tuple(out, OptTensor());
+    }
+    Tensor o = torch::empty(with_last(x.q, w.R), x.q.options()), so = torch::empty(with_last(x.s, w.R / QB), x.s.options());
+    pybind11::gil_scoped_release nogil;
+    check_rc(jf_igemm_block_q(x.qp(), w.qp(), x.sp(), w.sp(), b, bm, (int8_t *)o.data_ptr(), so.data_ptr(), (int)x.R, (int)w.R, (int)x.C,
+                              JF_B_NK, x.code, JF_SCALES_ROWMAJOR, JF_SCALES_ROWMAJOR, JF_ROUND_NEAREST, 0, 0, nullptr, 0, current_stream(x.q)),
+             "linear_forward");
+    return std::make_tuple(o, OptTensor(so));
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> linear_forward_gelu(const Tensor &X, const Tensor &SX, const Tensor &W, const Tensor &SW,
+                                                               int64_t approx, double amax_eps, const OptTensor &bias, const OptTensor &biasmax)
+{
+    const Operand x(X, SX, "X"), w(W, SW, "W");
+    same_kind(x, w);
+    TORCH_CHECK(w.q.dim() == 2 && x.C == w.C, "inner dimensions differ: X is ", X.sizes(), ", W is ", W.sizes());
+    check_approx(approx);
+    const float *b, *bm;
+    linear_bias(bias, biasmax, x, w.R, b, bm);
+    c10::DeviceGuard guard(x.q.device());
+    Tensor o = torch::empty(with_last(x.q, w.R), x.q.options()), so = torch::empty(with_last(x.s, w.R / QB), x.s.options());
+    Tensor g = torch::empty_like(o), sg = torch::empty_like(so);
+    pybind11::gil_scoped_release nogil;
+    check_rc(jf_igemm_block_q_gelu(x.qp(), w.qp(), x.sp(), w.sp(), b, bm, (int8_t *)o.data_ptr(), so.data_ptr(), (int8_t *)g.data_ptr(),
+                                   sg.data_ptr(), (int)x.R, (int)w.R, (int)x.C, x.code, JF_SCALES_ROWMAJOR, JF_SCALES_ROWMAJOR, (int)approx,
+                                   (float)amax_eps, current_stream(x.q)),
+             "linear_forward_gelu");
+    return std::make_tuple(o, so, g, sg);
+}
+
+// dW = dY^T X of a gradient read where it lies, or of its transposed copy [C_out, tokens]
+Tensor weight_gradient(const Operand &x, const Operand &g, const OptTensor &gT, int64_t splitk, OptDtype dtype)
+{
+    const torch::ScalarType odt = dtype.value_or(torch::kFloat16);
+    const int oc = fp_code(odt, "wgrad_dtype");
+    TORCH_CHECK(splitk >= 0, "splitk must be >= 0");
+    const int M = (int)g.C, N = (int)x.C, K = (int)x.R;
+    const int8_t *a = g.qp();
+    int la = JF_A_KM;
+    if (gT) {
+        TORCH_CHECK(gT->device() == x.q.device(), "operands are on different devices");
+        la = check_a_any_layout(*gT, M, K);
+        a = (const int8_t *)gT->data_ptr();
+    }
+    Tensor out = torch::empty({M, N}, x.q.options().dtype(odt));
+    const size_t nbytes = jf_igemm_block_fp_workspace_bytes(M, N, K, JF_B_KN, (int)splitk);
+    Tensor ws;
+    if (nbytes) ws = scratch(x.q, nbytes);
+    pybind11::gil_scoped_release nogil;
+    check_rc(jf_igemm_block_fp(a, x.qp(), g.sp(), x.sp(), out.data_ptr(), M, N, K, la, JF_B_KN, x.code, JF_SCALES_KMAJOR, JF_SCALES_KMAJOR, oc,
+                               (int)splitk, nbytes ? ws.data_ptr() : nullptr, nbytes, current_stream(x.q)),
+             "weight_gradient");
+    return out;
+}
+
+// (dX codes, dX scales, dW[, db]) or (dX values, dW[, db])
+std::vector<Tensor> linear_backward(const Tensor &X, const Tensor &SX, const Tensor &G, const Tensor &SG, const OptTensor &GT, const Tensor &W,
+                                    const Tensor &SW, bool dgrad_quantize, int64_t splitk, OptDtype wgrad_dtype, bool bias_grad)
+{
+    const Operand x(X, SX, "X"), g(G, SG, "G"), w(W, SW, "W");
+    same_kind(x, g); same_kind(x, w);
+    TORCH_CHECK(x.R == g.R && w.q.dim() == 2 && w.R == g.C && w.C == x.C, "operands do not match: X ", X.sizes(), ", G ", G.sizes(), ", W ", W.sizes());
+    c10::DeviceGuard guard(x.q.device());
+    std::vector<Tensor> out;
+    const auto so = rng(JF_ROUND_STOCHASTIC, g.q, g.R * w.C, c10::nullopt, c10::nullopt);
+    if (dgrad_quantize) {
+        out.push_back(torch::empty(with_last(g.q, w.C), g.q.options()));
+        out.push_back(torch::empty(with_last(g.s, w.C / QB), g.s.options()));
+        pybind11::gil_scoped_release nogil;
+        check_rc(jf_igemm_block_q(g.qp(), w.qp(), g.sp(), w.sp(), nullptr, nullptr, (int8_t *)out[0].data_ptr(), out[1].data_ptr(), (int)g.R,
+                                  (int)w.C, (int)g.C, JF_B_KN, g.code, JF_SCALES_ROWMAJOR, JF_SCALES_KMAJOR, JF_ROUND_STOCHASTIC, so.first,
+                                  so.second, nullptr, 0, current_stream(g.q)),
+                 "linear_backward");
+    } else {
+        out.push_back(torch::empty(with_last(g.q, w.C), g.s.options()));
+        pybind11::gil_scoped_release nogil;
+        check_rc(jf_igemm_block_q_dequant(g.qp(), w.qp(), g.sp(), w.sp(), nullptr, nullptr, out[0].data_ptr(), (int)g.R, (int)w.C, (int)g.C,
+                                          JF_B_KN, g.code, JF_SCALES_ROWMAJOR, JF_SCALES_KMAJOR, g.code == JF_SCALE_F16 ? JF_FP_F16 : JF_FP_F32,
+                                          JF_ROUND_STOCHASTIC, so.first, so.second, current_stream(g.q)),
+                 "linear_backward");
+    }
+    out.push_back(weight_gradient(x, g, GT, splitk, wgrad_dtype));
+    if (bias_grad) out.push_back(block_colsum(g.q, g.s));
+    return out;
+}
+
+// linear_backward followed by the GELU backward of its activation gradient (qmodel.py:249-253): (codes, scales, dW[, db])
+std::vector<Tensor> linear_backward_gelu(const Tensor &X, const Tensor &SX, const Tensor &G, const Tensor &SG, const Tensor &W, const Tensor &SW,
+                                         const Tensor &P, const Tensor &SP, int64_t approx, int64_t gelu_rounding, int64_t splitk,
+                                         OptDtype wgrad_dtype, bool bias_grad)
+{
+    const Operand x(X, SX, "X"), g(G, SG, "G"), w(W, SW, "W"), p(P, SP, "PRE");
+    same_kind(x, g); same_kind(x, w); same_kind(x, p);
+    TORCH_CHECK(x.R == g.R && w.q.dim() == 2 && w.R == g.C && w.C == x.C && p.R == x.R && p.C == x.C, "operands do not match: X ", X.sizes(), ", G ",
+                G.sizes(), ", W ", W.sizes(), ", PRE ", P.sizes());
+    check_approx(approx);
+    check_rounding(gelu_rounding, false);
+    c10::DeviceGuard guard(x.q.device());
+    const auto so = rng(JF_ROUND_STOCHASTIC, g.q, g.R * w.C, c10::nullopt, c10::nullopt);
+    const auto go = rng(gelu_rounding, g.q, g.R * w.C, c10::nullopt, c10::nullopt);
+    std::vector<Tensor> out{torch::empty(with_last(g.q, w.C), g.q.options()), torch::empty(with_last(g.s, w.C / QB), g.s.options())};
+    {
+        pybind11::gil_scoped_release nogil;
+        check_rc(jf_igemm_block_q_gelu_bwd(g.qp(), w.qp(), g.sp(), w.sp(), p.qp(), p.sp(), (int8_t *)out[0].data_ptr(), out[1].data_ptr(), (int)g.R,
+                                           (int)w.C, (int)g.C, g.code, JF_SCALES_ROWMAJOR, JF_SCALES_KMAJOR, (int)approx, so.first, so.second,
+                                           (int)gelu_rounding, go.first, go.second, current_stream(g.q)),
+                 "linear_backward_gelu");
+    }
+    out.push_back(weight_gradient(x, g, c10::nullopt, splitk, wgrad_dtype));
+    if (bias_grad) out.push_back(block_colsum(g.q, g.s));
+    return out;
+}
+
 }  // namespace
 
 void register_jetfire_ops(pybind11::module &m)
@@ -578,6 +819,9 @@ void register_jetfire_ops(pybind11::module &m)
     m.def("quantize_slabs", &quantize_slabs, py::arg("slabs"), py::arg("rounding") = JF_ROUND_NEAREST,
           py::arg("scale_dtype") = none, py::arg("amax_eps") = 0.0, py::arg("seed") = none, py::arg("offset") = none,
           "block tensor of the column-wise concatenation of up to 4 slabs, read where they lie");
+    m.def("quantize_many", &quantize_many, py::arg("xs"), py::arg("scale_dtype") = none,
+          "[(codes, scales), ...] of up to 8 float tensors of one type, one launch, round to nearest");
+    m.def("rowstats_fp", &rowstats_fp, py::arg("x"), "(mean, 1/sqrt(biased variance)) of the rows of a float tensor");
     m.def("dequantize", &dequantize, py::arg("q"), py::arg("s"), py::arg("out_dtype") = none);
     m.def("transpose_s8", &transpose_s8, py::arg("q"));
     m.def("rowstats", &rowstats, py::arg("q"), py::arg("s"), py::arg("eps") = 1e-5);
@@ -600,6 +844,15 @@ void register_jetfire_ops(pybind11::module &m)
     m.def("attention_bwd", &attention_bwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("out"), py::arg("lse"), py::arg("gout"),
           py::arg("batch"), py::arg("heads"), "gradients of q, k, v side by side, [tokens, 3C]");
     m.def("block_colsum", &block_colsum, py::arg("q"), py::arg("s"), "fp32 column sums of a block tensor (bias gradient)");
+    m.def("linear_forward", &linear_forward, py::arg("x"), py::arg("sx"), py::arg("w"), py::arg("sw"), py::arg("quantized"),
+          py::arg("bias") = none, py::arg("biasmax") = none);
+    m.def("linear_forward_gelu", &linear_forward_gelu, py::arg("x"), py::arg("sx"), py::arg("w"), py::arg("sw"), py::arg("approx"),
+          py::arg("amax_eps"), py::arg("bias") = none, py::arg("biasmax") = none);
+    m.def("linear_backward", &linear_backward, py::arg("x"), py::arg("sx"), py::arg("g"), py::arg("sg"), py::arg("gt"), py::arg("w"),
+          py::arg("sw"), py::arg("dgrad_quantize"), py::arg("splitk"), py::arg("wgrad_dtype"), py::arg("bias_grad"));
+    m.def("linear_backward_gelu", &linear_backward_gelu, py::arg("x"), py::arg("sx"), py::arg("g"), py::arg("sg"), py::arg("w"), py::arg("sw"),
+          py::arg("pre"), py::arg("spre"), py::arg("approx"), py::arg("gelu_rounding"), py::arg("splitk"), py::arg("wgrad_dtype"),
+          py::arg("bias_grad"));
     m.def("igemm_block_q", &igemm_block_q, py::arg("A"), py::arg("B"), py::arg("sa"), py::arg("sb"), py::arg("b_layout") = JF_B_KN,
           py::arg("bias") = none, py::arg("biasmax") = none, py::arg("rounding") = JF_ROUND_NEAREST, py::arg("seed") = none,
           py::arg("offset") = none);

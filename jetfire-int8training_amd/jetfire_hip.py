@@ -30,7 +30,7 @@ EXPORTS = [
     "jf_igemm_block_q", "jf_quantize", "jf_dequantize", "jf_transpose_s8", "jf_rowstats", "jf_layernorm_fwd",
     "jf_layernorm_bwd_workspace_bytes", "jf_layernorm_bwd", "jf_layernorm_bwd_add", "jf_gelu_fwd", "jf_gelu_bwd", "jf_add", "jf_rowstats_finish",
     "jf_igemm_block_q_dequant", "jf_quantize_slabs", "jf_philox_rounds", "jf_block_colsum", "jf_block_colsum_workspace_bytes",
-    "jf_attention_fwd", "jf_attention_bwd",
+    "jf_attention_fwd", "jf_attention_bwd", "jf_quantize_many", "jf_rowstats_fp",
 ]
 
 _lib = None
@@ -79,6 +79,8 @@ def lib():
         L.jf_block_colsum.argtypes = [_p, _p, _i, _i, _i, _p, _p, _sz, _p]
         L.jf_attention_fwd.argtypes = [_p, _p, _p, _i, _i, _i, _i, _i, _f, _p, _p, _p]
         L.jf_attention_bwd.argtypes = [_p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _f, _p, _p, _p, _i, _p, _p]
+        L.jf_quantize_many.argtypes = [_i, _p, _p, _p, _i, _p, _p, _i, _p]
+        L.jf_rowstats_fp.argtypes = [_p, _i, _i, _i, _p, _p, _p]
         missing = [name for name in EXPORTS if not hasattr(L, name)]
         if missing:
             raise RuntimeError(f"{LIB_PATH} does not export {missing}")
