@@ -46,31 +46,37 @@ class WeightCodes:
         self._entries = {}
         self.hits = self.misses = 0
 
-    def get(self, w):
-        key = id(w)
-        e = self._entries.get(key)
-        if e is not None and e[0]() is w and e[1] == w._version and e[2] == w.data_ptr():
+    def _hit(self, t):
+        e = self._entries.get(id(t))
+        if e is not None and e[0]() is t and e[1] == t._version and e[2] == t.data_ptr():
             self.hits += 1
             return e[3], e[4]
         self.misses += 1
-        q, s = int8_quantize(w.detach(), QB)
-        self._entries[key] = (weakref.ref(w, lambda _r, k=key, d=self._entries: d.pop(k, None)), w._version, w.data_ptr(), q, s)
-        return q, s
+        return None
+
+    def _keep(self, t, a, b):
+        key = id(t)
+        self._entries[key] = (weakref.ref(t, lambda _r, k=key, d=self._entries: d.pop(k, None)), t._version, t.data_ptr(), a, b)
+        return a, b
+
+    def get(self, w):
+        return self._hit(w) or self._keep(w, *int8_quantize(w.detach(), QB))
+
+    def get_many(self, ws):
+        """[(codes, scales), ...] of up to 8 weights; those that have changed are quantised in one launch per type."""
+        out = [self._hit(w) for w in ws]
+        for dt in {w.dtype for w, o in zip(ws, out) if o is None}:
+            stale = [i for i, o in enumerate(out) if o is None and ws[i].dtype == dt]
+            for i, (q, s) in zip(stale, _jf.quantize_many([ws[i].detach().contiguous() for i in stale])):
+                out[i] = self._keep(ws[i], q, s)
+        return out
 
     def get_bias(self, b):
         """(bias as float32, max|bias| as a one-element tensor) of a bias parameter, made once per version like the
         weight codes; None for None."""
         if b is None:
             return None
-        key = id(b)
-        e = self._entries.get(key)
-        if e is not None and e[0]() is b and e[1] == b._version and e[2] == b.data_ptr():
-            self.hits += 1
-            return e[3], e[4]
-        self.misses += 1
-        b32, bmax = bias_operands(b, b.numel(), b.device)
-        self._entries[key] = (weakref.ref(b, lambda _r, k=key, d=self._entries: d.pop(k, None)), b._version, b.data_ptr(), b32, bmax)
-        return b32, bmax
+        return self._hit(b) or self._keep(b, *bias_operands(b, b.numel(), b.device))
 
     def clear(self):
         self._entries.clear()
@@ -193,30 +199,6 @@ def _mlp_backward(saved, fpg, qg, sg, wdtype, res_dtype, bias_dtype=None):
     return (res_g, qg, sg, gw1, gw2, g_ln, (gb1[0].to(bias_dtype) if gb1 else None), (gb2[0].to(bias_dtype) if gb2 else None))
 
 
-class CausalAttention(torch.autograd.Function):
-    """Causal self-attention on the projection's output where it lies (q, k, v: views [B, T, C] of it; qmodel.py:134), by the
-    library's kernels: heads 32 or 64 wide, binary16.  The three gradients leave as views of one [B, T, 3C] tensor."""
-
-    @staticmethod
-    def applies(q, n_head):
-        return q.dtype == torch.float16 and q.shape[-1] // n_head in (32, 64) and q.shape[1] % QB == 0
-
-    @staticmethod
-    def forward(ctx, q, k, v, n_head):
-        B, T, C = q.shape
-        q, k, v = (t.reshape(B * T, C) for t in (q, k, v))
-        y, lse = _jf.attention_fwd(q, k, v, B, n_head)
-        ctx.save_for_backward(q, k, v, y, lse)
-        ctx.shape, ctx.n_head = (B, T, C), n_head
-        return y.view(B, T, C)
-
-    @staticmethod
-    def backward(ctx, g):
-        B, T, C = ctx.shape
-        g = _jf.attention_bwd(*ctx.saved_tensors, g.reshape(B * T, C).contiguous(), B, ctx.n_head).view(B, T, 3 * C)
-        return (*g.split(C, dim=-1), None)
-
-
 class AttentionOut(torch.autograd.Function):
     """Output projection + residual add, producing the statistics of the next LayerNorm (qmodel.py:134-171)."""
 
@@ -300,14 +282,25 @@ class QBlock(nn.Module):
         self.w_fc = nn.Parameter(torch.randn(4 * n_embd, n_embd) * 0.02)
         self.w_mlp_proj = nn.Parameter(torch.randn(n_embd, 4 * n_embd) * 0.02)
 
+    def _one_node(self, x, sx):
+        """Whether the block runs as the extension's single autograd node (its attention kernels take binary16 heads 32 or
+        64 wide, its LayerNorm backward rows of up to 2048 columns)."""
+        B, T, C = x.shape
+        return (C // self.n_head in (32, 64) and T % QB == 0 and C <= 2048 and T * 3 * C < 2 ** 30 and sx.dtype == torch.float16
+                and self.ln_1.dtype == self.ln_2.dtype == torch.float32
+                and self.w_qkv.dtype == self.w_attn_proj.dtype == self.w_fc.dtype == self.w_mlp_proj.dtype)
+
     def forward(self, x, qx, sx, mean, rstd):
         B, T, C = x.shape
+        if self._one_node(x, sx):
+            # the sequence below (AttentionIn, attention, AttentionOutMLP) as one node: same kernels, same noise
+            ws = [self.w_qkv, self.w_attn_proj, self.w_fc, self.w_mlp_proj]
+            bs = [] if self.b_qkv is None else [self.b_qkv, self.b_attn_proj, self.b_fc, self.b_mlp_proj]
+            return _jf.qblock(x.contiguous(), qx, sx, mean, rstd, [self.ln_1, self.ln_2] + ws, weight_codes.get_many(ws), bs,
+                              [weight_codes.get_bias(b) for b in bs], self.n_head, self.out_dtype)
         res, q, k, v = AttentionIn.apply(x, qx, sx, self.w_qkv, self.ln_1, mean, rstd, self.b_qkv)
-        if CausalAttention.applies(q, self.n_head):
-            y = CausalAttention.apply(q, k, v, self.n_head)
-        else:
-            q, k, v = (t.view(B, T, self.n_head, C // self.n_head).transpose(1, 2) for t in (q, k, v))
-            y = F.scaled_dot_product_attention(q, k, v, is_causal=True).transpose(1, 2).contiguous().view(B, T, C)
+        q, k, v = (t.view(B, T, self.n_head, C // self.n_head).transpose(1, 2) for t in (q, k, v))
+        y = F.scaled_dot_product_attention(q, k, v, is_causal=True).transpose(1, 2).contiguous().view(B, T, C)
         return AttentionOutMLP.apply(res, y, self.w_attn_proj, self.w_fc, self.w_mlp_proj, self.ln_2, self.out_dtype,
                                      self.b_attn_proj, self.b_fc, self.b_mlp_proj)
 
@@ -322,9 +315,9 @@ class QStack(nn.Module):
         self.blocks = nn.ModuleList(QBlock(n_embd, n_head, stream_dtype, bias) for _ in range(n_layer))
 
     def forward(self, x):
+        x = x.contiguous()
         x, qx, sx = StreamBegin.apply(x)
-        mean = x.float().mean(dim=-1)
-        rstd = torch.rsqrt(x.float().var(dim=-1, unbiased=False))
+        mean, rstd = _jf.rowstats_fp(x.detach())
         for blk in self.blocks:
             x, qx, sx, mean, rstd = blk(x, qx, sx, mean, rstd)
         return StreamEnd.apply(x, qx, sx)

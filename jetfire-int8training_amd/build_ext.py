@@ -72,7 +72,7 @@ def build_hip():
     return HIP_LIB
 
 
-TORCH_SOURCES = ["bqc_ext.cpp", "jf_ops_ext.cpp"]
+TORCH_SOURCES = ["bqc_ext.cpp", "jf_ops_ext.cpp", "jf_block_ext.cpp"]
 
 
 def build_torch():

@@ -10,7 +10,10 @@
 
 using namespace jfext;
 
-namespace jfext { void register_jetfire_ops(pybind11::module &m); }     // jf_ops_ext.cpp
+namespace jfext {
+void register_jetfire_ops(pybind11::module &m);     // jf_ops_ext.cpp
+void register_block(pybind11::module &m);           // jf_block_ext.cpp
+}
 
 namespace {
 
@@ -176,4 +179,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     // every other operator of the path (Jetfire/Nonlinear, and the GEMMs with fused epilogues Jetfire/Linear uses)
     pybind11::module ops = m.def_submodule("jetfire", "Nonlinear operators and fused-epilogue GEMMs of the INT8 data flow (gfx950)");
     jfext::register_jetfire_ops(ops);
+    jfext::register_block(ops);
 }

@@ -282,3 +282,60 @@ def test_weight_codes_are_cached_per_weight_version():
     import gc
     gc.collect()
     assert len(recipe.weight_codes._entries) == 0
+
+
+@pytest.mark.parametrize("B,T,C,H,bias,res,out", [(1, 32, 64, 2, False, torch.float32, torch.float32), (2, 96, 192, 3, True, torch.bfloat16, torch.float32),
+                                                  (3, 160, 128, 4, False, torch.float32, torch.bfloat16)])
+def test_block_as_one_node_equals_the_functions(B, T, C, H, bias, res, out):
+    """QBlock's single node runs the kernels of AttentionIn, the attention and AttentionOutMLP in their order with their noise
+    counters: outputs and every gradient are the same bits."""
+    import BlockQuantizeCUDA as BQC
+    import recipe
+    from Nonlinear import int8_quantize
+    jf = BQC.jetfire
+
+    class Attention(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, q, k, v):
+            q, k, v = (t.reshape(B * T, C) for t in (q, k, v))
+            y, lse = jf.attention_fwd(q, k, v, B, H)
+            ctx.save_for_backward(q, k, v, y, lse)
+            return y.view(B, T, C)
+
+        @staticmethod
+        def backward(ctx, g):
+            return jf.attention_bwd(*ctx.saved_tensors, g.reshape(B * T, C).contiguous(), B, H).view(B, T, 3 * C).split(C, dim=-1)
+
+    torch.manual_seed(5)
+    blk = recipe.QBlock(C, H, out, bias).cuda()
+    with torch.no_grad():
+        for p in blk.parameters():
+            if p.dim() == 1:
+                p.add_(0.1 * torch.randn_like(p))
+    x = torch.randn(B, T, C, device="cuda").to(res)
+    g = torch.randn(B, T, C, device="cuda").to(out)
+
+    def run(one):
+        torch.manual_seed(77)
+        xi = x.clone().requires_grad_(True)
+        for p in blk.parameters():
+            p.grad = None
+        h, qx, sx = recipe.StreamBegin.apply(xi)
+        mean, rstd = jf.rowstats_fp(h.detach())
+        assert torch.allclose(mean, h.detach().float().mean(-1), atol=1e-6)
+        assert torch.allclose(rstd, torch.rsqrt(h.detach().float().var(-1, unbiased=False)), rtol=1e-5)
+        if one:
+            assert blk._one_node(h, sx)
+            fp, q, s, m, r = blk(h, qx, sx, mean, rstd)
+        else:
+            a, qq, k, v = recipe.AttentionIn.apply(h, qx, sx, blk.w_qkv, blk.ln_1, mean, rstd, blk.b_qkv)
+            fp, q, s, m, r = recipe.AttentionOutMLP.apply(a, Attention.apply(qq, k, v), blk.w_attn_proj, blk.w_fc, blk.w_mlp_proj, blk.ln_2, out,
+                                                          blk.b_attn_proj, blk.b_fc, blk.b_mlp_proj)
+        recipe.StreamEnd.apply(fp, q, s).backward(g)
+        return [fp.detach(), q.view(torch.int8), s, m, r, xi.grad] + [p.grad for p in blk.parameters()]
+    for i, (a, b) in enumerate(zip(run(True), run(False))):
+        assert a.dtype == b.dtype and torch.equal(a, b), i
+    # several weights quantised in one launch: the codes of one by one
+    for (q, s), w in zip(jf.quantize_many([blk.w_qkv.detach(), blk.w_fc.detach()]), (blk.w_qkv, blk.w_fc)):
+        q2, s2 = int8_quantize(w.detach(), 32)
+        assert torch.equal(q, q2) and torch.equal(s, s2)
