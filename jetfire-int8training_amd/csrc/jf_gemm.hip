@@ -21,8 +21,8 @@
 // bytes per row) through an LDS ring filled by LDS-direct loads (global_load_lds_dwordx4: no register
 // staging).  LDS rows are 128 bytes with an XOR chunk swizzle, so the 16-byte MFMA operand reads are
 // conflict-free.  A is K-contiguous; B is either K-contiguous ([N,K]) or [K,N], which is staged as it lies
-// in memory and read with the transposing LDS read.  Scales are wave-uniform and are fetched by each wave
-// into a private LDS patch.
+// in memory and read with the transposing LDS read.  Scales are wave-uniform; each wave multiplies those it
+// needs once per stage and reads the products from a private LDS patch.
 #include "jf_device.hpp"
 
 #include <atomic>
@@ -198,51 +198,49 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
             gbase[j] = (is_a[j] ? p.A : p.B) + (size_t)r0 * (size_t)(is_a[j] ? p.lda : p.ldb);
         }
     }
-    // Scales of a stage: every wave fetches, again LDS-direct, the scales it needs itself into a private 256-byte
-    // patch (lane l: K block l/16; word l%16 = the wave's WBM A-side scales, then its WBN B-side scales, the rest
-    // padding), so that scale reads need no cross-wave synchronisation, every wave has the same number of loads in
-    // flight, and one LDS read per K block fetches all of them.  The lane keeps a running pointer.
-    constexpr int SCALE_WORDS = 64;
-    constexpr int NSC = WBM + WBN;                            // scales per wave and K block
-    static_assert(NSC <= 4, "one 16-byte LDS read per K block");
-    unsigned char *const scale_ring = smem + NSTAGE * STAGE_BYTES + wave * (NSTAGE * SCALE_WORDS * 4);
-    const int s_blk = lane & 15;
-    const bool s_is_a = !(s_blk >= WBM && s_blk < NSC);       // padding lanes repeat the first A-side scale
-    int s_idx = s_is_a ? m0 / QB + wm * WBM + (s_blk < WBM ? s_blk : 0) : n0 / QB + wn * WBN + s_blk - WBM;
-    { const int lim = s_is_a ? SM : SN; s_idx = s_idx < lim ? s_idx : lim - 1; }
-    const int s_ks = s_is_a ? p.sa_ks : p.sb_ks, s_is = s_is_a ? p.sa_is : p.sb_is;   // element strides: K block, tile block
-    const unsigned char *const s_base = reinterpret_cast<const unsigned char *>(s_is_a ? p.sa : p.sb);
-    auto scale_addr = [&](int kbg) {
-        const unsigned e = (unsigned)((kbg + kb_base) * s_ks + s_idx * s_is);
-        return s_base + e * (unsigned)sizeof(ST);
+    // Scales.  A K block of a wave needs the NBLK products sa * sb * 2^26 (see accumulate()), wave-uniform.  Lane l fetches the
+    // two scales of product (K block (l / NBLK) % 4 of the stage, block l % NBLK) with the stage's operands; when the stage is
+    // handed over the lane forms the product and leaves it in a private 256-byte LDS patch, from which one broadcast read per
+    // K block returns the block's products: per stage 2 conversions, 2 multiplications and a write, where multiplying the
+    // scales at every K block took 12 conversions and 16 multiplications per stage, 24 of the 280 vector instructions of its
+    // K loop (fc forward 8192x6400x1600, binary16 scales: see the measurements at launch_gemm_cfg).
+    constexpr int NBLK = WBM * WBN;
+    static_assert(NBLK == 2 || NBLK == 1, "one or two products per K block and wave");
+    unsigned char *const scale_patch = smem + NSTAGE * STAGE_BYTES + wave * 256;
+    const int s_blk = lane % NBLK, s_kb = (lane / NBLK) % KB_STAGE;
+    unsigned sa_off, sb_off;                                  // byte offsets of the lane's scales in the stage issued next
+    auto scale_offsets = [&](int kbg, unsigned &oa, unsigned &ob) {
+        int ia = m0 / QB + wm * WBM + s_blk / WBN, ib = n0 / QB + wn * WBN + s_blk % WBN;
+        ia = ia < SM ? ia : SM - 1;                           // (clamped for partial tiles: those blocks are never stored)
+        ib = ib < SN ? ib : SN - 1;
+        oa = (unsigned)((kbg + kb_base) * p.sa_ks + ia * p.sa_is) * (unsigned)sizeof(ST);
+        ob = (unsigned)((kbg + kb_base) * p.sb_ks + ib * p.sb_is) * (unsigned)sizeof(ST);
     };
-    const unsigned char *s_ptr = scale_addr((lane >> 4) < nkb ? (lane >> 4) : nkb - 1);
-    const unsigned s_step = (unsigned)(KB_STAGE * s_ks) * (unsigned)sizeof(ST);
+    scale_offsets(s_kb < nkb ? s_kb : nkb - 1, sa_off, sb_off);
+    const unsigned sa_step = (unsigned)(KB_STAGE * p.sa_ks) * (unsigned)sizeof(ST), sb_step = (unsigned)(KB_STAGE * p.sb_ks) * (unsigned)sizeof(ST);
+    ST sa_raw[NSTAGE], sb_raw[NSTAGE];
 
     constexpr int A_LOADS = (BM / 8) / NW;                    // loads 0 .. A_LOADS-1 of a wave fetch A rows, the rest B rows
     static_assert((BM / 8) % NW == 0, "a load instruction fetches rows of one operand");
     // FULL: the stage has all KB_STAGE K blocks (every stage but a short last one)
-    auto issue_stage_as = [&](int stage, auto full_c) {
+    auto issue_stage_as = [&](int stage, auto slot_c, auto full_c) {
         constexpr bool FULL = decltype(full_c)::value;
-        const unsigned slot_lds = (unsigned)(uintptr_t)(lds_u8 *)smem + (unsigned)(stage % NSTAGE) * STAGE_BYTES;
-        const unsigned scale_lds = (unsigned)(uintptr_t)(lds_u8 *)scale_ring + (unsigned)(stage % NSTAGE) * (SCALE_WORDS * 4);
+        constexpr int SLOT = decltype(slot_c)::value;         // stage % NSTAGE
+        const unsigned slot_lds = (unsigned)(uintptr_t)(lds_u8 *)smem + (unsigned)SLOT * STAGE_BYTES;
         const int kb0 = stage * KB_STAGE;
+        if (EPI != EPI_S32) {
+            if (!FULL) {                                      // missing K blocks: fetch the last one again (never used)
+                const int kbg = kb0 + s_kb;
+                scale_offsets(kbg < nkb ? kbg : nkb - 1, sa_off, sb_off);
+            }
+            // exactly the element's bytes are read, whatever the parity of its index or the length of the array
+            sa_raw[SLOT] = *reinterpret_cast<const ST *>(reinterpret_cast<const unsigned char *>(p.sa) + sa_off);
+            sb_raw[SLOT] = *reinterpret_cast<const ST *>(reinterpret_cast<const unsigned char *>(p.sb) + sb_off);
+            sa_off += sa_step;
+            sb_off += sb_step;
+        }
         // asm: scalar base + 32-bit lane offset is the addressing mode that costs no vector instruction, and the
         // compiler does not choose it by itself here.  M0 holds the LDS destination of an LDS-direct load.
-        if (EPI != EPI_S32) {
-            const unsigned char *src = s_ptr;
-            if (!FULL) {                                      // missing K blocks: fetch the last one again (never used)
-                int kbg = kb0 + (lane >> 4);
-                src = scale_addr(kbg < nkb ? kbg : nkb - 1);
-            }
-            // a binary16 scale is fetched with the 16-bit form (zero-extended into the lane's LDS word): exactly the
-            // element's two bytes are read, whatever the parity of its index or the length of the array
-            if (sizeof(ST) == 4)
-                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(scale_lds) : "memory", "m0");
-            else
-                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_ushort %0, off" ::"v"(src), "s"(scale_lds) : "memory", "m0");
-            s_ptr += s_step;
-        }
         unsigned la = loff_a, lb = loff_b;
         if (!FULL && kb0 + (gchunk >> 1) >= nkb) {            // chunks of missing K blocks: the stage's first block again
             if (!AKM) la -= (unsigned)(gchunk >> 1) * QB;
@@ -266,9 +264,17 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
                          ::"v"(j < A_LOADS ? la : lb), "s"(base), "s"(slot_lds + (unsigned)grp * 1024u) : "memory", "m0");
         }
     };
-    auto issue_stage = [&](int stage) {                       // stage < nstages
-        if (stage < nkb / KB_STAGE) issue_stage_as(stage, std::true_type{});
-        else issue_stage_as(stage, std::false_type{});
+    auto issue_stage = [&](int stage, auto slot_c) {          // stage < nstages
+        if (stage < nkb / KB_STAGE) issue_stage_as(stage, slot_c, std::true_type{});
+        else issue_stage_as(stage, slot_c, std::false_type{});
+    };
+    // the products of a stage that has landed, from the lane's registers into the wave's patch
+    auto put_products = [&](auto slot_c) {
+        constexpr int SLOT = decltype(slot_c)::value;
+        if (EPI != EPI_S32) {
+            const float t = ((float)sa_raw[SLOT] * (float)sb_raw[SLOT]) * 67108864.0f;
+            *reinterpret_cast<__attribute__((address_space(3))) float *>((uintptr_t)((unsigned)(uintptr_t)(lds_u8 *)scale_patch + lane * 4)) = t;
+        }
     };
 
     // ---- operand fetch addresses ----------------------------------------------------------------
@@ -301,10 +307,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
         const int c = 2 * (wm * WBM + i) + (g & 1);
         fa_km[i] = AKM ? (unsigned)(uintptr_t)lds + (g >> 1) * 2048 + ((rho * 8 + (c ^ rho)) << 4) + 8 * (r & 1) : 0u;
     }
-    // scale patch of this wave: a uniform address, parked in a vector register once (LDS reads take a VGPR address)
+    // product patch of this wave: a uniform address, parked in a vector register once (LDS reads take a VGPR address)
     unsigned sc_v;
     {
-        const unsigned sc_u = (unsigned)(uintptr_t)(lds_u8 *)scale_ring;
+        const unsigned sc_u = (unsigned)(uintptr_t)(lds_u8 *)scale_patch;
         asm volatile("v_mov_b32 %0, %1" : "=v"(sc_v) : "s"(sc_u));
     }
 
@@ -330,29 +336,29 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
     // of stage s has been read.  Operand fragments and scales of K block k+1 are read from LDS into a second set
     // of registers BEFORE the products of K block k are issued, so the LDS pipe works while the wave multiplies
     // and accumulates; without this all waves of a SIMD queue at the LDS together and then compute together.
-    constexpr int LOADS = LPW + (EPI != EPI_S32 ? 1 : 0);     // LDS-direct loads per wave and stage
+    constexpr int LOADS = LPW + (EPI != EPI_S32 ? 2 : 0);     // loads per wave and stage: LDS-direct ones and the scales
     const int nfull = nkb / KB_STAGE;                         // stages with all KB_STAGE blocks
     const int ktail = nkb - nfull * KB_STAGE;                 // K blocks of the short last stage (0: none)
-#pragma unroll
-    for (int s = 0; s < NSTAGE; ++s)
-        if (s < nstages) issue_stage(s);
+    static_for<0, NSTAGE>([&](auto slot_c) {
+        if (decltype(slot_c)::value < nstages) issue_stage(decltype(slot_c)::value, slot_c);
+    });
 
     // The fragment reads are written as asm so that they stay where they are and so that the wait for them can
     // name a count: the compiler, tracking them itself, waits for ALL outstanding LDS reads (the prefetch included)
     // on every other K block.  LDS reads of a wave return in order, so "at most FETCH_OPS outstanding" after issuing
     // the next K block's reads means that the current K block's have arrived.
-    typedef float scale_vec __attribute__((ext_vector_type(NSC == 3 ? 3 : NSC <= 2 ? 2 : 4)));
+    typedef float scale_vec __attribute__((ext_vector_type(2)));
     v4i fa_reg[2][WBM], fb_reg[2][WBN];
     scale_vec sc_raw[2];
     constexpr int FETCH_OPS = (AKM ? 2 : 1) * WBM + (BKN ? 2 : 1) * WBN + (EPI != EPI_S32 ? 1 : 0);
     static_assert(2 * FETCH_OPS <= 15, "lgkmcnt is a 4-bit counter");
-    // pa/pb: this lane's fragment addresses for the K block (ring slot 0); psc: the wave's scale patch;
-    // slot_bytes / slot_words: compile-time offset of the ring slot in the tile ring and of the K block in the patch
+    // pa/pb: this lane's fragment addresses for the K block (ring slot 0); psc: the wave's product patch;
+    // slot_bytes: compile-time offset of the ring slot in the tile ring; kb: K block of the stage (for the patch)
     // kn_base: runtime offset of the ring slot for the transposing reads (0 where the slot is in the immediates)
     auto fetch = [&](const unsigned pa, const unsigned pb, const unsigned kn_base, const unsigned psc, auto slot_bytes_c,
-                     auto kn_off_c, auto slot_words_c, auto buf_c) {
+                     auto kn_off_c, auto kb_c, auto buf_c) {
         constexpr int BUF = decltype(buf_c)::value;
-        constexpr int SB = decltype(slot_bytes_c)::value, SW = decltype(slot_words_c)::value;
+        constexpr int SB = decltype(slot_bytes_c)::value, KB = decltype(kb_c)::value;
         // the instruction's offset field has 16 bits: slots beyond that are reached through the address register
         constexpr int HI = (SB + (WBM > WBN ? WBM : WBN) * QB * ROW_BYTES) > 65535 ? SB : 0;
         const unsigned pa2 = pa + HI, pb2 = pb + HI;
@@ -384,9 +390,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
         }
         if (EPI != EPI_S32) {
             scale_vec &dst = sc_raw[BUF];
-            if (NSC == 3) asm volatile("ds_read_b96 %0, %1 offset:%2" : "=v"(dst) : "v"(psc), "n"(SW * 4));
-            else if (NSC <= 2) asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(dst) : "v"(psc), "n"(SW * 4));
-            else asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(psc), "n"(SW * 4));
+            asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(dst) : "v"(psc), "n"(KB * NBLK * 4));
         }
     };
     // wait until at most `n` LDS reads are outstanding, and tie register set BUF to that point in program order
@@ -404,7 +408,6 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
     // before the vector ALU can read it.  So the accumulation lags the products by one: product n is issued, THEN
     // product n-1 (long finished) is converted and accumulated.  (d_pend, sab_pend) carry the lagging product across
     // K blocks and stages; the first accumulation adds 0*0 and the last product is accumulated after the loop.
-    constexpr int NBLK = WBM * WBN;
     constexpr int C_MAGIC = 0x3e22f983;                        // accumulator input of the MFMAs (file header)
     v16i d_pend = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     float sab_pend = 0.0f;
@@ -429,16 +432,6 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
                 for (int j = 0; j < WBN; ++j)
                     iacc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa_reg[CUR][i], fb_reg[CUR][j], iacc[i][j], 0, 0, 0);
         } else {
-            float fa[WBM], fb[WBN];
-            // a binary16 scale sits in the low half of its word
-            auto scale_of = [&](float raw) -> float {
-                if (sizeof(ST) == 4) return raw;
-                return (float)__builtin_bit_cast(half_t, (uint16_t)__float_as_uint(raw));
-            };
-#pragma unroll
-            for (int i = 0; i < WBM; ++i) fa[i] = scale_of(sc_raw[CUR][i]);
-#pragma unroll
-            for (int j = 0; j < WBN; ++j) fb[j] = scale_of(sc_raw[CUR][WBM + j]);
             static_for<0, NBLK>([&](auto n_c) {
                 constexpr int n = decltype(n_c)::value, i = n / WBN, j = n % WBN;
                 // asm: as a builtin operand the constant is hoisted into 16 registers instead of being encoded inline.
@@ -447,7 +440,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
                 // a vector read of an MFMA result needs.
                 v16i d_new;
                 asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0x3e22f983" : "=&v"(d_new) : "v"(fa_reg[CUR][i]), "v"(fb_reg[CUR][j]));
-                const float sab_new = (fa[i] * fb[j]) * 67108864.0f;       // * 2^26, see accumulate()
+                const float sab_new = sc_raw[CUR][n];
                 __builtin_amdgcn_sched_barrier(0);
                 accumulate(std::integral_constant<int, (n + NBLK - 1) % NBLK>{});
                 __builtin_amdgcn_sched_barrier(0);
@@ -467,6 +460,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
     };
     using c0 = std::integral_constant<int, 0>;
     wait_stage(0, NSTAGE - 1);
+    put_products(c0{});
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();                              // bare: __syncthreads() would drain every load
     asm volatile("" ::: "memory");
@@ -499,21 +493,21 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
                     // ring slot of stage s may be overwritten by the loads of stage s+NSTAGE.
                     __builtin_amdgcn_s_waitcnt(0xC07F);       // lgkmcnt(0) only
                     wait_stage(s + 1, s + NSTAGE - 1);
+                    put_products(std::integral_constant<int, NEXT_SLOT>{});
                     asm volatile("" ::: "memory");
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
-                    if (s + NSTAGE < nstages) issue_stage(s + NSTAGE);
+                    if (s + NSTAGE < nstages) issue_stage(s + NSTAGE, slot_c);
                 }
                 // unconditional: past the last stage it reads bytes of the ring that nobody uses
                 if constexpr (ACTIVE)
                     fetch(fa_u[0], fb_u[0], 0u, sc_v, std::integral_constant<int, NEXT_SLOT * STAGE_BYTES>{},
-                          std::integral_constant<int, NEXT_SLOT * STAGE_BYTES>{},
-                          std::integral_constant<int, NEXT_SLOT * 64>{}, std::integral_constant<int, NXT>{});
+                          std::integral_constant<int, NEXT_SLOT * STAGE_BYTES>{}, c0{}, std::integral_constant<int, NXT>{});
             } else {
                 if constexpr (ACTIVE)
                     fetch(fa_u[kb + 1], fb_u[kb + 1], 0u, sc_v, std::integral_constant<int, SLOT * STAGE_BYTES>{},
                           std::integral_constant<int, SLOT * STAGE_BYTES + (kb + 1) * 4096>{},
-                          std::integral_constant<int, SLOT * 64 + (kb + 1) * 16>{}, std::integral_constant<int, NXT>{});
+                          std::integral_constant<int, kb + 1>{}, std::integral_constant<int, NXT>{});
             }
             // The arbiter of a SIMD serves its oldest wave first, so the older of two resident workgroups runs about 1.4
             // times as fast as the younger one and the second wave of a workgroup on a SIMD trails the first by a quarter
@@ -539,8 +533,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
             constexpr int CUR = kb & 1;
             if (kb < ktail) {
                 if (kb > 0)
-                    fetch(fa_u[kb] + slot * STAGE_BYTES, fb_u[kb] + slot * STAGE_BYTES, slot * STAGE_BYTES, sc_v + slot * 256,
-                          c0{}, std::integral_constant<int, kb * 4096>{}, std::integral_constant<int, kb * 16>{},
+                    fetch(fa_u[kb] + slot * STAGE_BYTES, fb_u[kb] + slot * STAGE_BYTES, slot * STAGE_BYTES, sc_v,
+                          c0{}, std::integral_constant<int, kb * 4096>{}, std::integral_constant<int, kb>{},
                           std::integral_constant<int, CUR>{});
                 fetched(c0{}, std::integral_constant<int, CUR>{});
                 compute(std::integral_constant<int, CUR>{}, nfull * KB_STAGE + kb);
@@ -868,7 +862,7 @@ template <int EPI, typename ST, int WGM, int WGN, int NSTAGE, int WGPC, int BKN,
 static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 {
     constexpr int BM = QB * WBM * WGM, BN = QB * WBN * WGN, NT = 64 * WGM * WGN;
-    constexpr int RING = NSTAGE * (BM + BN) * ROW_BYTES + WGM * WGN * NSTAGE * 256;   // operand ring + per-wave scale patches
+    constexpr int RING = NSTAGE * (BM + BN) * ROW_BYTES + WGM * WGN * 256;            // operand ring + per-wave product patches
     constexpr int PATCH = WGM * WGN * QB * EPI_LD * (int)sizeof(float);     // the epilogue's per-wave transposition patches
     constexpr int SMEM = RING > PATCH ? RING : PATCH;
     if (!device_is_gfx950()) return JF_ERR_DEVICE;
