@@ -99,8 +99,9 @@ __device__ __forceinline__ void tile_of_workgroup(int tiles_m, int tiles_n, bool
 // vmcnt(n), no wait on the other counters (gfx9 encoding: vmcnt = bits 3:0 and 15:14)
 #define JF_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | 0x0F70)
 
-// WGM x WGN waves, each owning WBM x WBN quantisation blocks (64x32 elements).
-constexpr int WBM = 2, WBN = 1;
+// WGM x WGN waves, each owning WBM x WBN quantisation blocks (WBM = 2: 64x32 elements; WBM = 1: one block, for launches whose
+// 128x128 tiles would leave most of the chip idle, see launch_gemm).
+constexpr int WBN = 1;
 // NSTAGE = depth of the LDS ring (one stage being computed, NSTAGE-1 in flight); WGPC = workgroups per CU
 // (the second launch bound counts waves per SIMD: WGPC workgroups of WGM*WGN waves over 4 SIMDs).
 // AKM = 1: A is [K, lda] (M-contiguous rows), staged and read like a [K,N] B operand (below).
@@ -111,7 +112,7 @@ static int cu_count();
 // PROF = 1: the first wave of every workgroup also records when the workgroup's phases began and ended (wall clock) and
 // how many shader cycles its main loop took: a profiling build of the same code, instantiated only in the measurement
 // library (jf_prof_igemm_block_q).
-template <int EPI, typename ST, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
+template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
 __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt_kernel(GemmArgs p_in)
 {
     GemmArgs p = p_in;                                        // K-split launches narrow it to the split's K range below
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
     const int kn_chunk = (n0 + (((lane & 7) ^ lrow) << 4)) < p.N ? ((lane & 7) ^ lrow) : 0;
     const unsigned loff_b = BKN ? (unsigned)lrow * (unsigned)p.ldb + kn_chunk * 16
                                 : (unsigned)lrow * (unsigned)p.ldb + gchunk * 16;
-    const int8_t *gbase[LPW];      // wave-uniform: first byte of the group's first row (stage 0)
+    const int8_t *gbase[LPW];      // wave-uniform: first byte of the group's first row in the stage issued next
     bool is_a[LPW];
 #pragma unroll
     for (int j = 0; j < LPW; ++j) {
@@ -198,27 +199,66 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
             gbase[j] = (is_a[j] ? p.A : p.B) + (size_t)r0 * (size_t)(is_a[j] ? p.lda : p.ldb);
         }
     }
-    // Scales.  A K block of a wave needs the NBLK products sa * sb * 2^26 (see accumulate()), wave-uniform.  Lane l fetches the
-    // two scales of product (K block (l / NBLK) % 4 of the stage, block l % NBLK) with the stage's operands; when the stage is
-    // handed over the lane forms the product and leaves it in a private 256-byte LDS patch, from which one broadcast read per
-    // K block returns the block's products: per stage 2 conversions, 2 multiplications and a write, where multiplying the
-    // scales at every K block took 12 conversions and 16 multiplications per stage, 24 of the 280 vector instructions of its
-    // K loop (fc forward 8192x6400x1600, binary16 scales: see the measurements at launch_gemm_cfg).
+    // Scales.  A K block of a wave needs the NBLK products sa * sb * 2^26 (see accumulate()), wave-uniform.  They are formed once
+    // per stage: lanes 0..31 fetch the A-side and lanes 32..63 the B-side scale of product l % (4 NBLK) (K block of the stage,
+    // block) of a stage, LDS-direct, one stage ahead of its operands; during the stage before, each lane multiplies its pair and
+    // leaves the product in a private patch, from which one broadcast read per K block returns the block's products.  Per
+    // stage 2 conversions, 2 multiplications and 2 LDS operations, where multiplying the scales at every K block took 12
+    // conversions and 16 multiplications, 28 of the 290 vector instructions of a stage (XL forward 8192x1600x6400, binary16
+    // scales: 162 -> 154 us; 8192^3, binary32: 985 -> 966 us).  Not through registers: a load of the compiler's own makes it
+    // wait for every load in flight when the value is used, the stages ahead included.
     constexpr int NBLK = WBM * WBN;
     static_assert(NBLK == 2 || NBLK == 1, "one or two products per K block and wave");
-    unsigned char *const scale_patch = smem + NSTAGE * STAGE_BYTES + wave * 256;
-    const int s_blk = lane % NBLK, s_kb = (lane / NBLK) % KB_STAGE;
-    unsigned sa_off, sb_off;                                  // byte offsets of the lane's scales in the stage issued next
-    auto scale_offsets = [&](int kbg, unsigned &oa, unsigned &ob) {
-        int ia = m0 / QB + wm * WBM + s_blk / WBN, ib = n0 / QB + wn * WBN + s_blk % WBN;
-        ia = ia < SM ? ia : SM - 1;                           // (clamped for partial tiles: those blocks are never stored)
-        ib = ib < SN ? ib : SN - 1;
-        oa = (unsigned)((kbg + kb_base) * p.sa_ks + ia * p.sa_is) * (unsigned)sizeof(ST);
-        ob = (unsigned)((kbg + kb_base) * p.sb_ks + ib * p.sb_is) * (unsigned)sizeof(ST);
+    constexpr int SC_SLOT = 256;                              // a ring slot of a wave's fetched scales; its products follow all of them
+    static_assert(NSTAGE <= 3, "8-bit word offsets of the paired scale read");
+    unsigned char *const scale_patch = smem + NSTAGE * STAGE_BYTES + wave * (2 * NSTAGE * SC_SLOT);
+    const int s_prod = lane % (KB_STAGE * NBLK), s_blk = s_prod % NBLK, s_kb = s_prod / NBLK;
+    const bool s_is_b = lane >= 32;
+    const unsigned char *const s_base = reinterpret_cast<const unsigned char *>(s_is_b ? p.sb : p.sa);
+    unsigned s_off, s_last, s_step;                           // byte offsets: in the stage fetched next, of the last K block, per stage
+    {
+        // (clamped for partial tiles: those blocks are never stored)
+        int i = s_is_b ? n0 / QB + wn * WBN + s_blk % WBN : m0 / QB + wm * WBM + s_blk / WBN;
+        const int lim = s_is_b ? SN : SM, ks = s_is_b ? p.sb_ks : p.sa_ks, is = s_is_b ? p.sb_is : p.sa_is;
+        i = i < lim ? i : lim - 1;
+        s_off = (unsigned)((s_kb + kb_base) * ks + i * is) * (unsigned)sizeof(ST);
+        s_last = (unsigned)((nkb - 1 + kb_base) * ks + i * is) * (unsigned)sizeof(ST);
+        s_step = (unsigned)(KB_STAGE * ks) * (unsigned)sizeof(ST);
+    }
+    // the scales of the next stage (one after the other) into ring slot `slot`; K blocks beyond the last: the last one again
+    auto issue_scales = [&](auto slot_c) {
+        if (EPI == EPI_S32) return;
+        const unsigned char *const src = s_base + (s_off < s_last ? s_off : s_last);
+        const unsigned dst = (unsigned)(uintptr_t)(lds_u8 *)scale_patch + decltype(slot_c)::value * SC_SLOT;
+        // a binary16 scale is fetched with the 16-bit form (zero-extended into the lane's LDS word): exactly the
+        // element's two bytes are read, whatever the parity of its index or the length of the array
+        if (sizeof(ST) == 4)
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(dst) : "memory", "m0");
+        else
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_ushort %0, off" ::"v"(src), "s"(dst) : "memory", "m0");
+        s_off += s_step;
     };
-    scale_offsets(s_kb < nkb ? s_kb : nkb - 1, sa_off, sb_off);
-    const unsigned sa_step = (unsigned)(KB_STAGE * p.sa_ks) * (unsigned)sizeof(ST), sb_step = (unsigned)(KB_STAGE * p.sb_ks) * (unsigned)sizeof(ST);
-    ST sa_raw[NSTAGE], sb_raw[NSTAGE];
+    const unsigned sc_rd = (unsigned)(uintptr_t)(lds_u8 *)scale_patch + (lane & 31) * 4, sc_wr = (unsigned)(uintptr_t)(lds_u8 *)scale_patch + NSTAGE * SC_SLOT + lane * 4;
+    v2i s_pair;                                               // the lane's two scales, between read_scales and put_products
+    auto read_scales = [&](auto slot_c) {
+        if (EPI == EPI_S32) return;
+        constexpr int W = decltype(slot_c)::value * (SC_SLOT / 4);
+        v2i &dst = s_pair;
+        const unsigned src = sc_rd;
+        asm volatile("ds_read2_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(dst) : "v"(src), "n"(W), "n"(W + 32));
+    };
+    auto put_products = [&](auto slot_c) {                    // the read has been waited for
+        if (EPI == EPI_S32) return;
+        v2i &pair = s_pair;
+        const unsigned dst = sc_wr;
+        asm volatile("" : "+v"(pair));
+        auto value = [](int bits) -> float {
+            if (sizeof(ST) == 4) return __int_as_float(bits);
+            return (float)__builtin_bit_cast(half_t, (uint16_t)bits);
+        };
+        const float t = (value(pair.x) * value(pair.y)) * 67108864.0f;
+        asm volatile("ds_write_b32 %0, %1 offset:%2" ::"v"(dst), "v"(t), "n"(decltype(slot_c)::value * SC_SLOT) : "memory");
+    };
 
     constexpr int A_LOADS = (BM / 8) / NW;                    // loads 0 .. A_LOADS-1 of a wave fetch A rows, the rest B rows
     static_assert((BM / 8) % NW == 0, "a load instruction fetches rows of one operand");
@@ -228,17 +268,6 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
         constexpr int SLOT = decltype(slot_c)::value;         // stage % NSTAGE
         const unsigned slot_lds = (unsigned)(uintptr_t)(lds_u8 *)smem + (unsigned)SLOT * STAGE_BYTES;
         const int kb0 = stage * KB_STAGE;
-        if (EPI != EPI_S32) {
-            if (!FULL) {                                      // missing K blocks: fetch the last one again (never used)
-                const int kbg = kb0 + s_kb;
-                scale_offsets(kbg < nkb ? kbg : nkb - 1, sa_off, sb_off);
-            }
-            // exactly the element's bytes are read, whatever the parity of its index or the length of the array
-            sa_raw[SLOT] = *reinterpret_cast<const ST *>(reinterpret_cast<const unsigned char *>(p.sa) + sa_off);
-            sb_raw[SLOT] = *reinterpret_cast<const ST *>(reinterpret_cast<const unsigned char *>(p.sb) + sb_off);
-            sa_off += sa_step;
-            sb_off += sb_step;
-        }
         // asm: scalar base + 32-bit lane offset is the addressing mode that costs no vector instruction, and the
         // compiler does not choose it by itself here.  M0 holds the LDS destination of an LDS-direct load.
         unsigned la = loff_a, lb = loff_b;
@@ -251,30 +280,25 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
             const int grp = wave + j * NW;
             const int8_t *base;                                // wave-uniform
             if (BKN && j >= A_LOADS) {
-                base = gbase[j] + (size_t)kb0 * QB * (size_t)p.ldb;
+                base = gbase[j];
+                gbase[j] += (size_t)(KB_STAGE * QB) * (size_t)p.ldb;
                 // K rows of a missing K block: the stage's first group again
                 if (!FULL && kb0 * QB + (grp - BM / 8) * 8 >= p.K) base -= (size_t)((grp - BM / 8) * 8) * (size_t)p.ldb;
             } else if (AKM && j < A_LOADS) {
-                base = gbase[j] + (size_t)kb0 * QB * (size_t)p.lda;
+                base = gbase[j];
+                gbase[j] += (size_t)(KB_STAGE * QB) * (size_t)p.lda;
                 if (!FULL && kb0 * QB + grp * 8 >= p.K) base -= (size_t)(grp * 8) * (size_t)p.lda;
             } else {
-                base = gbase[j] + (size_t)kb0 * QB;
+                base = gbase[j];
+                gbase[j] += KB_STAGE * QB;
             }
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                          ::"v"(j < A_LOADS ? la : lb), "s"(base), "s"(slot_lds + (unsigned)grp * 1024u) : "memory", "m0");
         }
     };
-    auto issue_stage = [&](int stage, auto slot_c) {          // stage < nstages
+    auto issue_stage = [&](int stage, auto slot_c) {          // stage < nstages, one after the other
         if (stage < nkb / KB_STAGE) issue_stage_as(stage, slot_c, std::true_type{});
         else issue_stage_as(stage, slot_c, std::false_type{});
-    };
-    // the products of a stage that has landed, from the lane's registers into the wave's patch
-    auto put_products = [&](auto slot_c) {
-        constexpr int SLOT = decltype(slot_c)::value;
-        if (EPI != EPI_S32) {
-            const float t = ((float)sa_raw[SLOT] * (float)sb_raw[SLOT]) * 67108864.0f;
-            *reinterpret_cast<__attribute__((address_space(3))) float *>((uintptr_t)((unsigned)(uintptr_t)(lds_u8 *)scale_patch + lane * 4)) = t;
-        }
     };
 
     // ---- operand fetch addresses ----------------------------------------------------------------
@@ -310,7 +334,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
     // product patch of this wave: a uniform address, parked in a vector register once (LDS reads take a VGPR address)
     unsigned sc_v;
     {
-        const unsigned sc_u = (unsigned)(uintptr_t)(lds_u8 *)scale_patch;
+        const unsigned sc_u = (unsigned)(uintptr_t)(lds_u8 *)scale_patch + NSTAGE * SC_SLOT;
         asm volatile("v_mov_b32 %0, %1" : "=v"(sc_v) : "s"(sc_u));
     }
 
@@ -336,11 +360,17 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
     // of stage s has been read.  Operand fragments and scales of K block k+1 are read from LDS into a second set
     // of registers BEFORE the products of K block k are issued, so the LDS pipe works while the wave multiplies
     // and accumulates; without this all waves of a SIMD queue at the LDS together and then compute together.
-    constexpr int LOADS = LPW + (EPI != EPI_S32 ? 2 : 0);     // loads per wave and stage: LDS-direct ones and the scales
+    constexpr int LOADS = LPW + (EPI != EPI_S32 ? 1 : 0);     // LDS-direct loads per wave and stage
     const int nfull = nkb / KB_STAGE;                         // stages with all KB_STAGE blocks
     const int ktail = nkb - nfull * KB_STAGE;                 // K blocks of the short last stage (0: none)
+    issue_scales(std::integral_constant<int, 0>{});
     static_for<0, NSTAGE>([&](auto slot_c) {
-        if (decltype(slot_c)::value < nstages) issue_stage(decltype(slot_c)::value, slot_c);
+        constexpr int SLOT = decltype(slot_c)::value;
+        if (SLOT < nstages) {
+            issue_stage(SLOT, slot_c);
+            // (ring slot 0 holds the first stage's scales until they are read, below)
+            if (SLOT + 1 < NSTAGE) issue_scales(std::integral_constant<int, (SLOT + 1) % NSTAGE>{});
+        }
     });
 
     // The fragment reads are written as asm so that they stay where they are and so that the wait for them can
@@ -353,23 +383,24 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
     constexpr int FETCH_OPS = (AKM ? 2 : 1) * WBM + (BKN ? 2 : 1) * WBN + (EPI != EPI_S32 ? 1 : 0);
     static_assert(2 * FETCH_OPS <= 15, "lgkmcnt is a 4-bit counter");
     // pa/pb: this lane's fragment addresses for the K block (ring slot 0); psc: the wave's product patch;
-    // slot_bytes: compile-time offset of the ring slot in the tile ring; kb: K block of the stage (for the patch)
+    // slot_bytes: compile-time offset of the ring slot in the tile ring; sc_off: of the K block's products in the patch
     // kn_base: runtime offset of the ring slot for the transposing reads (0 where the slot is in the immediates)
     auto fetch = [&](const unsigned pa, const unsigned pb, const unsigned kn_base, const unsigned psc, auto slot_bytes_c,
-                     auto kn_off_c, auto kb_c, auto buf_c) {
+                     auto kn_off_c, auto sc_off_c, auto buf_c) {
         constexpr int BUF = decltype(buf_c)::value;
-        constexpr int SB = decltype(slot_bytes_c)::value, KB = decltype(kb_c)::value;
+        constexpr int SB = decltype(slot_bytes_c)::value, SC = decltype(sc_off_c)::value;
         // the instruction's offset field has 16 bits: slots beyond that are reached through the address register
         constexpr int HI = (SB + (WBM > WBN ? WBM : WBN) * QB * ROW_BYTES) > 65535 ? SB : 0;
         const unsigned pa2 = pa + HI, pb2 = pb + HI;
         constexpr int KO = decltype(kn_off_c)::value;         // slot + K block offset of a [K,N] / [K,M] staging
+        constexpr int KHI = KO + 1024 > 65535 ? KO : 0;
         if (AKM) {
 #pragma unroll
             for (int i = 0; i < WBM; ++i) {
-                const unsigned pakm = fa_km[i] + kn_base;
+                const unsigned pakm = fa_km[i] + kn_base + KHI;
                 v2i lo, hi;
-                asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(lo) : "v"(pakm), "n"(KO));
-                asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(hi) : "v"(pakm), "n"(KO + 1024));
+                asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(lo) : "v"(pakm), "n"(KO - KHI));
+                asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(hi) : "v"(pakm), "n"(KO - KHI + 1024));
                 fa_reg[BUF][i] = v4i{lo.x, lo.y, hi.x, hi.y};
             }
         } else {
@@ -378,10 +409,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
                 asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa_reg[BUF][i]) : "v"(pa2), "n"(SB - HI + i * (QB * ROW_BYTES)));
         }
         if (BKN) {
-            const unsigned pbkn = fb_kn + kn_base;
+            const unsigned pbkn = fb_kn + kn_base + KHI;
             v2i lo, hi;
-            asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(lo) : "v"(pbkn), "n"(KO));
-            asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(hi) : "v"(pbkn), "n"(KO + 1024));
+            asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(lo) : "v"(pbkn), "n"(KO - KHI));
+            asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(hi) : "v"(pbkn), "n"(KO - KHI + 1024));
             fb_reg[BUF][0] = v4i{lo.x, lo.y, hi.x, hi.y};
         } else {
 #pragma unroll
@@ -390,7 +421,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
         }
         if (EPI != EPI_S32) {
             scale_vec &dst = sc_raw[BUF];
-            asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(dst) : "v"(psc), "n"(KB * NBLK * 4));
+            if (NBLK == 2) {
+                asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(dst) : "v"(psc), "n"(SC));
+            } else {
+                float one;
+                asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(one) : "v"(psc), "n"(SC));
+                dst.x = one;
+            }
         }
     };
     // wait until at most `n` LDS reads are outstanding, and tie register set BUF to that point in program order
@@ -449,18 +486,20 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
             });
         }
     };
-    // Loads retire in order: stage t has landed once only the loads of the stages issued after it are outstanding.
-    auto wait_stage = [&](int t, int last_issued) {
-        int younger = (last_issued < nstages - 1 ? last_issued : nstages - 1) - t;
-        if (younger >= 4) JF_WAIT_VMCNT(4 * LOADS);
-        else if (younger == 3) JF_WAIT_VMCNT(3 * LOADS);
-        else if (younger == 2) JF_WAIT_VMCNT(2 * LOADS);
-        else if (younger == 1) JF_WAIT_VMCNT(LOADS);
-        else JF_WAIT_VMCNT(0);
+    // Loads retire in order: a stage (and the scales of the one after it) has landed once only the loads of the Y stages
+    // issued after it (up to `last`) are outstanding.  Near the end of K, with fewer stages behind it than usual, everything is waited for.
+    auto wait_stage = [&](int last, auto younger_c) {
+        constexpr int Y = decltype(younger_c)::value;
+        if (Y == 0 || last >= nstages) JF_WAIT_VMCNT(0);
+        else JF_WAIT_VMCNT(Y * LOADS);
     };
     using c0 = std::integral_constant<int, 0>;
-    wait_stage(0, NSTAGE - 1);
+    if (NSTAGE - 1 >= nstages) JF_WAIT_VMCNT(0);
+    else JF_WAIT_VMCNT((NSTAGE - 1) * LOADS - (EPI != EPI_S32 ? 1 : 0));      // stage 0 and the scales of stage 1 have landed
+    read_scales(c0{});
+    __builtin_amdgcn_s_waitcnt(0xC07F);                        // lgkmcnt(0) only
     put_products(c0{});
+    if (NSTAGE - 1 < nstages) issue_scales(c0{});              // stage NSTAGE, behind the operands of stage NSTAGE - 1
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();                              // bare: __syncthreads() would drain every load
     asm volatile("" ::: "memory");
@@ -492,22 +531,26 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
                     // landed; after the barrier that holds for every wave, so (a) stage s+1 may be read and (b) the
                     // ring slot of stage s may be overwritten by the loads of stage s+NSTAGE.
                     __builtin_amdgcn_s_waitcnt(0xC07F);       // lgkmcnt(0) only
-                    wait_stage(s + 1, s + NSTAGE - 1);
-                    put_products(std::integral_constant<int, NEXT_SLOT>{});
+                    wait_stage(s + NSTAGE - 1, std::integral_constant<int, NSTAGE - 2>{});
                     asm volatile("" ::: "memory");
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
-                    if (s + NSTAGE < nstages) issue_stage(s + NSTAGE, slot_c);
+                    if (s + NSTAGE < nstages) {
+                        issue_stage(s + NSTAGE, slot_c);
+                        issue_scales(std::integral_constant<int, NEXT_SLOT>{});      // of stage s + NSTAGE + 1
+                    }
                 }
                 // unconditional: past the last stage it reads bytes of the ring that nobody uses
                 if constexpr (ACTIVE)
                     fetch(fa_u[0], fb_u[0], 0u, sc_v, std::integral_constant<int, NEXT_SLOT * STAGE_BYTES>{},
-                          std::integral_constant<int, NEXT_SLOT * STAGE_BYTES>{}, c0{}, std::integral_constant<int, NXT>{});
+                          std::integral_constant<int, NEXT_SLOT * STAGE_BYTES>{}, std::integral_constant<int, NEXT_SLOT * SC_SLOT>{},
+                          std::integral_constant<int, NXT>{});
             } else {
                 if constexpr (ACTIVE)
                     fetch(fa_u[kb + 1], fb_u[kb + 1], 0u, sc_v, std::integral_constant<int, SLOT * STAGE_BYTES>{},
                           std::integral_constant<int, SLOT * STAGE_BYTES + (kb + 1) * 4096>{},
-                          std::integral_constant<int, kb + 1>{}, std::integral_constant<int, NXT>{});
+                          std::integral_constant<int, SLOT * SC_SLOT + (kb + 1) * NBLK * 4>{}, std::integral_constant<int, NXT>{});
+                if constexpr (ACTIVE && kb == 0) read_scales(std::integral_constant<int, NEXT_SLOT>{});
             }
             // The arbiter of a SIMD serves its oldest wave first, so the older of two resident workgroups runs about 1.4
             // times as fast as the younger one and the second wave of a workgroup on a SIMD trails the first by a quarter
@@ -518,10 +561,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
             if constexpr (PACE == PACE_ORDERED && kb == 0) { if (second_slot) __builtin_amdgcn_s_setprio(3); else __builtin_amdgcn_s_setprio(1); }
             if constexpr (PACE == PACE_ORDERED && kb == 2) { if (second_slot) __builtin_amdgcn_s_setprio(2); else __builtin_amdgcn_s_setprio(0); }
             if constexpr (ACTIVE) {
-                fetched(std::integral_constant<int, FETCH_OPS>{}, std::integral_constant<int, CUR>{});
+                fetched(std::integral_constant<int, FETCH_OPS + (kb == 0 && EPI != EPI_S32 ? 1 : 0)>{}, std::integral_constant<int, CUR>{});
                 __builtin_amdgcn_sched_barrier(0);            // the reads above stay above the products below,
                 compute(std::integral_constant<int, CUR>{}, s * KB_STAGE + kb);
                 __builtin_amdgcn_sched_barrier(0);            // and K blocks are scheduled one by one (register pressure)
+                if constexpr (kb == 1) put_products(std::integral_constant<int, NEXT_SLOT>{});     // the next stage's
             }
         });
     });
@@ -533,8 +577,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
             constexpr int CUR = kb & 1;
             if (kb < ktail) {
                 if (kb > 0)
-                    fetch(fa_u[kb] + slot * STAGE_BYTES, fb_u[kb] + slot * STAGE_BYTES, slot * STAGE_BYTES, sc_v,
-                          c0{}, std::integral_constant<int, kb * 4096>{}, std::integral_constant<int, kb>{},
+                    fetch(fa_u[kb] + slot * STAGE_BYTES, fb_u[kb] + slot * STAGE_BYTES, slot * STAGE_BYTES,
+                          sc_v + slot * SC_SLOT, c0{}, std::integral_constant<int, kb * 4096>{}, std::integral_constant<int, kb * NBLK * 4>{},
                           std::integral_constant<int, CUR>{});
                 fetched(c0{}, std::integral_constant<int, CUR>{});
                 compute(std::integral_constant<int, CUR>{}, nfull * KB_STAGE + kb);
@@ -543,8 +587,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
     }
     };
     if (!wave_active) main_loop(std::false_type{}, std::integral_constant<int, PACE_HARDWARE>{});
-    else if (p.pace == PACE_EVEN) main_loop(std::true_type{}, std::integral_constant<int, PACE_EVEN>{});
-    else if (p.pace == PACE_ORDERED) main_loop(std::true_type{}, std::integral_constant<int, PACE_ORDERED>{});
+    else if (WBM == 2 && p.pace == PACE_EVEN) main_loop(std::true_type{}, std::integral_constant<int, PACE_EVEN>{});
+    else if (WBM == 2 && p.pace == PACE_ORDERED) main_loop(std::true_type{}, std::integral_constant<int, PACE_ORDERED>{});
     else main_loop(std::true_type{}, std::integral_constant<int, PACE_HARDWARE>{});
     __builtin_amdgcn_s_waitcnt(0xC07F);                        // the last, unused prefetch must land before its registers are reused
     if (EPI != EPI_S32 && wave_active) {
@@ -858,18 +902,18 @@ static int launch_transpose(const int8_t *in, int R, int C, int8_t *out, hipStre
     return (int)hipGetLastError();
 }
 
-template <int EPI, typename ST, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
+template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
 static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 {
     constexpr int BM = QB * WBM * WGM, BN = QB * WBN * WGN, NT = 64 * WGM * WGN;
-    constexpr int RING = NSTAGE * (BM + BN) * ROW_BYTES + WGM * WGN * 256;            // operand ring + per-wave product patches
+    constexpr int RING = NSTAGE * ((BM + BN) * ROW_BYTES + WGM * WGN * 512);         // operand ring + per-wave scale and product patches
     constexpr int PATCH = WGM * WGN * QB * EPI_LD * (int)sizeof(float);     // the epilogue's per-wave transposition patches
     constexpr int SMEM = RING > PATCH ? RING : PATCH;
     if (!device_is_gfx950()) return JF_ERR_DEVICE;
     GemmArgs p = a;
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
-    auto kern = igemm_nt_kernel<EPI, ST, WGM, WGN, NSTAGE, WGPC, BKN, AKM, PROF>;
+    auto kern = igemm_nt_kernel<EPI, ST, WBM, WGM, WGN, NSTAGE, WGPC, BKN, AKM, PROF>;
     // more than 64 KiB of dynamic LDS has to be opted into, per function and device: once, not on every launch
     // (the reference sets its attribute on every call, igemm_BlockSquare32OutputIntQuantizeBiasRowCol.cu:418)
     static std::atomic<bool> opted_in[MAX_DEVICES] = {};
@@ -892,7 +936,8 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
     const long wgs = (long)p.tiles_m * p.tiles_n * p.splits, slots = (long)WGPC * cu_count();
     const bool short_second_round = wgs > slots && 2 * wgs < 3 * slots;
     const int k_per_wg = p.splits > 1 ? p.kb_per_split * QB : p.K;
-    p.pace = short_second_round ? (k_per_wg >= 4096 ? PACE_ORDERED : PACE_HARDWARE)
+    if (WBM == 1) p.pace = PACE_HARDWARE;                     // (no paced instances: all its workgroups are resident)
+    else p.pace = short_second_round ? (k_per_wg >= 4096 ? PACE_ORDERED : PACE_HARDWARE)
                                 : (wgs <= 2 * slots ? PACE_EVEN : PACE_HARDWARE);
     hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n * p.splits), dim3(NT), SMEM, st, p);
     return (int)hipGetLastError();
@@ -951,31 +996,46 @@ static void splitk_plan(int M, int N, int K, int request, int &splits, int &kb_p
     splits = (nkb + kb_per_split - 1) / kb_per_split;
 }
 
-// Tile configuration: 128x128 tiles, 8 waves, a 2-deep ring and two workgroups per CU (the epilogue of one overlaps
-// the main loop of the other).  A [K,N] B operand (and, for the weight gradient, a [K,M] A operand) is read in place.
+// Tile configuration.  Large launches: 128x128 tiles, 8 waves of two blocks, a 2-deep ring and two workgroups per CU (the
+// epilogue of one overlaps the main loop of the other).  A launch whose 32x128 tiles are all resident at once, two workgroups
+// of 4 waves and a 3-deep ring per CU, takes those instead: its 128x128 tiles would occupy at most a quarter of the chip with
+// 16 products per K block and SIMD pair in sequence, where a wave with one block is bound by the issue of its own 32 vector
+// instructions per product.  Measured (one-sequence forward GEMMs, us, 128x128 | 32x128): 32x768x768 9.7 | 6.7, 512x768x3072
+// 28.8 | 16.6, 512x3072x768 (384 small tiles) 10.7 | 8.4, 1248x768x768 10.7 | 7.1; beyond two per CU the larger tile's data
+// reuse wins: 1248x2304x768 (702) 10.9 | 12.6.  (A deeper ring changes nothing there; a 64x128 tile of 8 waves is 6 % better
+// between 256 and 512 small tiles and up to 19 % worse below.)
+// A [K,N] B operand (and, for the weight gradient, a [K,M] A operand) is read in place.
 // a_km (A given as [K,M]) exists for the weight-gradient form only: fp output, B as [K,N].
+template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs &a, hipStream_t st)
+{
+    if constexpr (EPI != EPI_S32) {
+        if (a.splits <= 1 && (long)((a.M + 31) / 32) * ((a.N + 127) / 128) <= 2L * cu_count())
+            return launch_gemm_cfg<EPI, ST, 1, 1, 4, 3, 2, BKN>(a, st);
+    }
+    return launch_gemm_cfg<EPI, ST, 2, 2, 4, 2, 2, BKN>(a, st);
+}
 template <int EPI, typename ST> static int launch_gemm(const GemmArgs &a, hipStream_t st, bool b_kn, bool a_km = false)
 {
     if constexpr (EPI == EPI_QG) {                            // the forward form only: A [M,K], B [N,K]
         if (a_km || b_kn) return JF_ERR_UNSUPPORTED;
-        return launch_gemm_cfg<EPI, ST, 2, 4, 2, 2, 0>(a, st);
+        return launch_gemm_b<EPI, ST, 0>(a, st);
     } else if constexpr (EPI == EPI_QB) {                     // the activation-gradient form only: A [M,K], B [K,N]
         if (a_km || !b_kn) return JF_ERR_UNSUPPORTED;
-        return launch_gemm_cfg<EPI, ST, 2, 4, 2, 2, 1>(a, st);
+        return launch_gemm_b<EPI, ST, 1>(a, st);
     } else {
         if (a_km) {
             if constexpr (EPI == EPI_FP) {
-                if (b_kn) return launch_gemm_cfg<EPI, ST, 2, 4, 2, 2, 1, 1>(a, st);
+                if (b_kn) return launch_gemm_cfg<EPI, ST, 2, 2, 4, 2, 2, 1, 1>(a, st);
             }
             return JF_ERR_UNSUPPORTED;
         }
 #ifdef JF_PROF_LIB
         if constexpr (EPI == EPI_Q && std::is_same<ST, float>::value) {
             if (a.phases)                                     // the profiling library: the PROF build of the same kernel
-                return b_kn ? launch_gemm_cfg<EPI, ST, 2, 4, 2, 2, 1, 0, 1>(a, st) : launch_gemm_cfg<EPI, ST, 2, 4, 2, 2, 0, 0, 1>(a, st);
+                return b_kn ? launch_gemm_cfg<EPI, ST, 2, 2, 4, 2, 2, 1, 0, 1>(a, st) : launch_gemm_cfg<EPI, ST, 2, 2, 4, 2, 2, 0, 0, 1>(a, st);
         }
 #endif
-        return b_kn ? launch_gemm_cfg<EPI, ST, 2, 4, 2, 2, 1>(a, st) : launch_gemm_cfg<EPI, ST, 2, 4, 2, 2, 0>(a, st);
+        return b_kn ? launch_gemm_b<EPI, ST, 1>(a, st) : launch_gemm_b<EPI, ST, 0>(a, st);
     }
 }
 

@@ -481,3 +481,19 @@ def test_phase_recording_build_gives_the_same_bits_and_ordered_phases(jf):
         us = ph["us"]
         assert us.shape == (12, 6) and (us[:, 1:] >= us[:, :-1]).all() and us[:, 5].max() < 1e4
         assert ((ph["k_loop_MHz"] > 300) & (ph["k_loop_MHz"] < 3500)).all()
+
+
+@pytest.mark.parametrize("M,N", [(1056, 544), (2080, 1056)])      # 165 workgroups of 32x128 tiles; 153 of 128x128 (585 would be small ones)
+@pytest.mark.parametrize("K", [32, 96, 128, 160, 288, 384, 416])  # ring of two and of three stages: one, fewer than, as many as, more than its depth
+def test_both_tile_sizes_at_every_ring_fill(jf, oracle, M, N, K):
+    print(f"case M={M} N={N} K={K}", flush=True)
+    A, Bkn, sa, sb = make_problem(M + N + K, M, N, K)
+    dA, dsa, dsb = dev(A), dev(sa.astype(np.float16)), dev(sb.astype(np.float16))
+    for layout in (0, 1):
+        B = b_of(Bkn, layout)
+        want = oracle.igemm_block_f32(A, B, sa, sb, layout)
+        same(jf.igemm_block_fp(dA, dev(B), dsa, dsb, layout, torch.float32), want, "fp32 accumulators")
+        q, sc = jf.igemm_block_q(dA, dev(B), dsa, dsb, layout, rounding=jf.ROUND_STOCHASTIC, seed=4, offset=8)
+        wq, wsc = oracle.igemm_block_q(A, B, sa, sb, layout, stochastic=True, seed=4, offset=8, scale_dtype="f16")
+        same(q, wq, "SR codes")
+        same(sc, wsc, "SR scales")
