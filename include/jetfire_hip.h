@@ -247,6 +247,12 @@ int jf_layernorm_bwd_add(const int8_t *qx, const void *sx, const int8_t *qg, con
                          const void *x1, int x1_dtype, int add_rounding, uint64_t add_seed, uint64_t add_offset,
                          void *y1, int y1_dtype, int8_t *q, void *s, float *dgamma, float *dbeta,
                          void *workspace, size_t workspace_bytes, jf_stream_t stream);
+/* The same with dgamma left as one term per 32-row strip, [R/32][C]: jf_wgrad_many adds them.  No workspace. */
+int jf_layernorm_bwd_add_strips(const int8_t *qx, const void *sx, const int8_t *qg, const void *sg, const float *gamma, const float *mean,
+                                const float *rstd, int R, int C, int scale_dtype, int rounding, uint64_t seed, uint64_t offset,
+                                const void *x1, int x1_dtype, int add_rounding, uint64_t add_seed, uint64_t add_offset, void *y1,
+                                int y1_dtype, int8_t *q, void *s, float *strip_dgamma, jf_stream_t stream);
+
 
 /* dequant -> GELU -> requant (amax_eps is added to the block amax: 5e-5 in the reference).
  * Replaces int8_gelu_forward (Jetfire/Nonlinear/gelu_fwd.py:128-162). */
@@ -287,6 +293,15 @@ int jf_block_colsum(const int8_t *q, const void *s, int R, int C, int scale_dtyp
  * jf_add. */
 int jf_rowstats_finish(const float *rowsum, const float *rowsq, int R, int parts, int C, float *mean, float *rstd,
                        jf_stream_t stream);
+
+/* Up to 4 weight gradients over the same K tokens in one launch: out[i] [M[i], N[i]] = G[i]^T X[i] with G[i] codes [K, M[i]],
+ * X[i] codes [K, N[i]] and scales in the block tensors' own layout ([K/32, M[i]/32], [K/32, N[i]/32]); arithmetic of
+ * jf_igemm_block_fp with JF_A_KM, JF_B_KN and a K split chosen for the launch as a whole.  Behind it, up to 4 column sums
+ * sum[i][c] = sum over K/32 strips of terms[i][strip][c], in the same launch as the sums of the K split. */
+size_t jf_wgrad_many_workspace_bytes(int n, const int *M, const int *N, int K);
+int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
+                  const int *M, const int *N, int K, int scale_dtype, int out_dtype, int ncol, const float *const *terms,
+                  const int *width, float *const *sum, void *workspace, size_t workspace_bytes, jf_stream_t stream);
 
 /* Causal self-attention between the QKV projection and the output projection, binary16 in and out.  q, k, v: [B*T, ld]
  * with head h of a row at columns h*D .. h*D + D - 1 of each pointer (the three column ranges of the projection's output,

@@ -72,7 +72,7 @@ struct BackwardTemp {
     int8_t *qp, *qd, *qr, *qq;
     void *sp, *sd, *sr, *sq;
     void *res, *gy, *gqkv;
-    float *delta;
+    float *delta, *ln1_terms, *ln2_terms;
     void *ws;
     size_t carve(uint8_t *b, const Dims &d, size_t res_bytes, size_t ws_bytes)
     {
@@ -83,6 +83,7 @@ struct BackwardTemp {
         qq = k.take<int8_t>(d.codes(3 * d.c)); sq = k.take(d.scales(3 * d.c));      // at Q, K, V
         res = k.take(d.m * d.c * res_bytes); gy = k.take(d.m * d.c * 2); gqkv = k.take(d.m * 3 * d.c * 2);
         delta = k.take<float>(d.m * d.H * 4);
+        ln1_terms = k.take<float>(d.m / 32 * d.c * 4); ln2_terms = k.take<float>(d.m / 32 * d.c * 4);
         ws = k.take(ws_bytes);
         return k.used;
     }
@@ -234,9 +235,9 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         Saved v;
         v.carve((uint8_t *)s[14].data_ptr(), d);
         const int m = d.M, c = d.C;
-        const int wdim[4][2] = {{3 * c, c}, {c, c}, {4 * c, c}, {c, 4 * c}};          // [C_out, C_in]
-        size_t ws_bytes = jf_layernorm_bwd_workspace_bytes(m, c);
-        for (auto &n : wdim) ws_bytes = std::max(ws_bytes, jf_igemm_block_fp_workspace_bytes(n[0], n[1], m, JF_B_KN, 0));
+        // [C_out, C_in] of the weights
+        const int wrows[4] = {3 * c, c, 4 * c, c}, wcols[4] = {c, c, c, 4 * c};
+        size_t ws_bytes = jf_wgrad_many_workspace_bytes(4, wrows, wcols, m);
         if (with_bias) ws_bytes = std::max(ws_bytes, jf_block_colsum_workspace_bytes(m, 4 * c));
         BackwardTemp t;
         const size_t res_bytes = torch::elementSize(res_type);
@@ -249,9 +250,9 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         out[SX] = torch::empty({B, T / QB, C / QB}, opt.dtype(torch::kFloat16));
         out[LN1] = torch::empty({C}, opt.dtype(torch::kFloat32));
         out[LN2] = torch::empty({C}, opt.dtype(torch::kFloat32));
-        for (int i = 0; i < 4; ++i) out[W_QKV + i] = torch::empty({wdim[i][0], wdim[i][1]}, opt.dtype(w_type));
+        for (int i = 0; i < 4; ++i) out[W_QKV + i] = torch::empty({wrows[i], wcols[i]}, opt.dtype(w_type));
         if (with_bias)
-            for (int i = 0; i < 4; ++i) out[B_QKV + i] = torch::empty({wdim[i][0]}, opt.dtype(torch::kFloat32));
+            for (int i = 0; i < 4; ++i) out[B_QKV + i] = torch::empty({wrows[i]}, opt.dtype(torch::kFloat32));
         const int resc = fp_of(out[X], "residual"), wc = fp_of(out[W_QKV], "weight"), fpgc = fp_of(fpg, "gradient");
 
         // Philox counters, drawn in the order of the separate Functions (the reservations below are what each would make)
@@ -269,10 +270,14 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const jf_stream_t st = current_stream(qx);
         constexpr int RM = JF_SCALES_ROWMAJOR, KM = JF_SCALES_KMAJOR, F16 = JF_SCALE_F16, SR = JF_ROUND_STOCHASTIC;
         auto codes = [](const Tensor &a) { return (const int8_t *)a.data_ptr(); };
+        // The weight gradients run together at the end: one launch has tiles for the whole chip where each of the four alone
+        // needs a K split and leaves a last round half empty, and one more adds what is left to add, the LayerNorm weights'
+        // gradients included.
+        const int8_t *wg[4], *wx[4];
+        const void *wgs[4], *wxs[4];
         auto wgrad = [&](int i, const int8_t *g, const void *gs, const int8_t *xq, const void *xs) {
-            check_rc(jf_igemm_block_fp(g, xq, gs, xs, out[W_QKV + i].data_ptr(), wdim[i][0], wdim[i][1], m, JF_A_KM, JF_B_KN, F16, KM, KM, wc, 0, t.ws,
-                                       ws_bytes, st), "weight gradient");
-            if (with_bias) check_rc(jf_block_colsum(g, gs, m, wdim[i][0], F16, out[B_QKV + i].data_ptr<float>(), t.ws, ws_bytes, st), "bias gradient");
+            wg[i] = g; wgs[i] = gs; wx[i] = xq; wxs[i] = xs;
+            if (with_bias) check_rc(jf_block_colsum(g, gs, m, wrows[i], F16, out[B_QKV + i].data_ptr<float>(), t.ws, ws_bytes, st), "bias gradient");
         };
         // MLP: second projection with the GELU's backward in its epilogue, fc, LayerNorm with the residual add behind it
         check_rc(jf_igemm_block_q_gelu_bwd(codes(qg), codes(w[3].q), sg.data_ptr(), w[3].s.data_ptr(), v.qh, v.sh, t.qp, t.sp, m, 4 * c, c, F16, RM, KM,
@@ -281,9 +286,9 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         check_rc(jf_igemm_block_q(t.qp, codes(w[2].q), t.sp, w[2].s.data_ptr(), nullptr, nullptr, t.qd, t.sd, m, c, 4 * c, JF_B_KN, F16, RM, KM, SR,
                                   z[2].seed, z[2].offset, nullptr, 0, st), "gradient of fc");
         wgrad(2, t.qp, t.sp, v.qn2, v.sn2);
-        check_rc(jf_layernorm_bwd_add(v.q2, v.s2, t.qd, t.sd, ln2.data_ptr<float>(), v.mean2, v.rstd2, m, c, F16, SR, z[3].seed, z[3].offset,
+        check_rc(jf_layernorm_bwd_add_strips(v.q2, v.s2, t.qd, t.sd, ln2.data_ptr<float>(), v.mean2, v.rstd2, m, c, F16, SR, z[3].seed, z[3].offset,
                                       fpg.data_ptr(), fpgc, JF_ROUND_STOCHASTIC_TRUNC, z[4].seed, z[4].offset, t.res, resc, t.qr, t.sr,
-                                      out[LN2].data_ptr<float>(), nullptr, t.ws, ws_bytes, st), "gradient of layernorm");
+                                      t.ln2_terms, st), "gradient of layernorm");
         // attention: output projection, the attention itself, QKV, LayerNorm with the residual add behind it
         check_rc(jf_igemm_block_q_dequant(t.qr, codes(w[1].q), t.sr, w[1].s.data_ptr(), nullptr, nullptr, t.gy, m, c, c, JF_B_KN, F16, RM, KM, JF_FP_F16,
                                           SR, z[5].seed, z[5].offset, st), "gradient of the attention's projection");
@@ -295,10 +300,15 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         check_rc(jf_igemm_block_q(t.qq, codes(w[0].q), t.sq, w[0].s.data_ptr(), nullptr, nullptr, t.qd, t.sd, m, c, 3 * c, JF_B_KN, F16, RM, KM, SR,
                                   z[7].seed, z[7].offset, nullptr, 0, st), "gradient of qkv");
         wgrad(0, t.qq, t.sq, v.qn, v.sn);
-        check_rc(jf_layernorm_bwd_add(codes(qx), sx.data_ptr(), t.qd, t.sd, ln1.data_ptr<float>(), mean.data_ptr<float>(), rstd.data_ptr<float>(), m, c, F16,
+        check_rc(jf_layernorm_bwd_add_strips(codes(qx), sx.data_ptr(), t.qd, t.sd, ln1.data_ptr<float>(), mean.data_ptr<float>(), rstd.data_ptr<float>(), m, c, F16,
                                       SR, z[8].seed, z[8].offset, t.res, resc, JF_ROUND_STOCHASTIC_TRUNC, z[9].seed, z[9].offset, out[X].data_ptr(), resc,
-                                      (int8_t *)out[QX].data_ptr(), out[SX].data_ptr(), out[LN1].data_ptr<float>(), nullptr, t.ws, ws_bytes, st),
+                                      (int8_t *)out[QX].data_ptr(), out[SX].data_ptr(), t.ln1_terms, st),
                  "gradient of layernorm");
+        void *const gw[4] = {out[W_QKV].data_ptr(), out[W_PROJ].data_ptr(), out[W_FC].data_ptr(), out[W_FC2].data_ptr()};
+        const float *const terms[2] = {t.ln1_terms, t.ln2_terms};
+        float *const gln[2] = {out[LN1].data_ptr<float>(), out[LN2].data_ptr<float>()};
+        const int widths[2] = {c, c};
+        check_rc(jf_wgrad_many(4, wg, wgs, wx, wxs, gw, wrows, wcols, m, F16, wc, 2, terms, widths, gln, t.ws, ws_bytes, st), "weight gradients");
         if (with_bias && b_type != torch::kFloat32)
             for (int i = 0; i < 4; ++i) out[B_QKV + i] = out[B_QKV + i].to(b_type);
         return out;

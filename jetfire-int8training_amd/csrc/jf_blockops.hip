@@ -900,8 +900,10 @@ __global__ __launch_bounds__(WAVE * LNS_WAVES) void layernorm_bwd_strip_kernel(
             const size_t dst = (size_t)rb * C + cb * QB + ((lane >> 1) & 1) * 16 + (lane >> 2);
             const float tg = colsum16_over_rows(x, lane, cpatch);
             if ((lane & 1) == 0) pdg[dst] = tg;
-            const float tb = colsum16_over_rows(g, lane, cpatch);
-            if ((lane & 1) == 0) pdb[dst] = tb;
+            if (pdb) {                                             // (uniform) dbeta wanted
+                const float tb = colsum16_over_rows(g, lane, cpatch);
+                if ((lane & 1) == 0) pdb[dst] = tb;
+            }
         }
         __builtin_amdgcn_sched_barrier(0);                         // block by block: interleaved, their temporaries do not fit
     });
@@ -1343,15 +1345,17 @@ size_t jf_layernorm_bwd_workspace_bytes(int R, int C)
 }  // extern "C"
 
 // rows of up to 2048 columns: one pass over the inputs, the strip's codes held in registers.  add != nullptr: the residual
-// add that follows happens in the same kernel (qdx / sdx are not written).
+// add that follows happens in the same kernel (qdx / sdx are not written).  strip_dgamma != nullptr: dgamma is left as one
+// term per strip, [R/32][C] (jf_wgrad_many adds them), dgamma and dbeta are not written.
 static int launch_layernorm_bwd_strip(const int8_t *qx, const void *sx, const int8_t *qg, const void *sg, const float *gamma,
                                       const float *mean, const float *rstd, int R, int C, int scale_dtype, int rounding,
                                       uint64_t seed, uint64_t offset, int8_t *qdx, void *sdx, float *dgamma, float *dbeta,
-                                      void *workspace, const LnAddArgs *add, hipStream_t st)
+                                      void *workspace, const LnAddArgs *add, float *strip_dgamma, hipStream_t st)
 {
-    const bool want_dw = dgamma || dbeta;
+    const bool want_dw = dgamma || dbeta || strip_dgamma;
     const int SC = C / QB;
-    float *sdg = (float *)workspace, *sdb = sdg + (size_t)(R / QB) * C;      // [R/32][C] each: fits the workspace size
+    float *sdg = strip_dgamma ? strip_dgamma : (float *)workspace;          // [R/32][C] each: fits the workspace size
+    float *sdb = dbeta && !strip_dgamma ? sdg + (size_t)(R / QB) * C : nullptr;
     const size_t patch = add ? LNS_PATCH_ADD : want_dw ? COLSUM_PATCH : 0;
     const size_t lds = ((size_t)C + 2 * SC * QB + 2 * 8 * QB + 2 * QB + LNS_WAVES * patch) * sizeof(float);
     const LnAddArgs ad = add ? *add : LnAddArgs{};
@@ -1376,9 +1380,33 @@ static int launch_layernorm_bwd_strip(const int8_t *qx, const void *sx, const in
     else { if (add) JF_LNS_DW(float, true); else JF_LNS_DW(float, false); }
 #undef JF_LNS_DW
 #undef JF_LNS
-    if (want_dw)
-        hipLaunchKernelGGL(layernorm_bwd_colsum_finish_kernel, dim3(SC, 2), dim3(1024), 0, st, sdg, sdb, R / QB, C, dgamma, dbeta);
+    if (want_dw && !strip_dgamma)
+        hipLaunchKernelGGL(layernorm_bwd_colsum_finish_kernel, dim3(SC, dbeta ? 2 : 1), dim3(1024), 0, st, sdg, sdb, R / QB, C, dgamma, dbeta);
     return (int)hipGetLastError();
+}
+
+static int layernorm_bwd_add(const int8_t *qx, const void *sx, const int8_t *qg, const void *sg, const float *gamma, const float *mean,
+                             const float *rstd, int R, int C, int scale_dtype, int rounding, uint64_t seed, uint64_t offset, const void *x1,
+                             int x1_dtype, int add_rounding, uint64_t add_seed, uint64_t add_offset, void *y1, int y1_dtype, int8_t *q, void *s,
+                             float *dgamma, float *dbeta, float *strip_dgamma, void *workspace, jf_stream_t stream)
+{
+    int rc = check_block_tensor(qx, sx, R, C, scale_dtype);
+    if (rc) return rc;
+    if ((rc = check_block_tensor(qg, sg, R, C, scale_dtype))) return rc;
+    if (!gamma || !mean || !rstd || !x1 || !y1 || !q || !s) return JF_ERR_NULL;
+    if (!rounding_ok(rounding) || !rounding_ok(add_rounding)) return JF_ERR_ENUM;
+    if (x1_dtype < JF_FP_F16 || x1_dtype > JF_FP_BF16 || y1_dtype < JF_FP_F16 || y1_dtype > JF_FP_BF16) return JF_ERR_ENUM;
+    if (!aligned16(gamma) || !aligned16(x1) || !aligned16(y1) || !aligned16(q)) return JF_ERR_ALIGN;
+    if (C / QB > LNS_WAVES * LNS_BPW) return JF_ERR_SHAPE;         // wider rows: jf_layernorm_bwd, then jf_add
+    if (!strip_dgamma && !workspace) return JF_ERR_WORKSPACE;
+    if (!aligned16(workspace)) return JF_ERR_ALIGN;
+    if (!device_is_gfx950()) return JF_ERR_DEVICE;
+    LnAddArgs ad;
+    ad.x1 = x1; ad.y1 = y1; ad.q = q; ad.s = s;
+    ad.x1_dtype = x1_dtype; ad.y1_dtype = y1_dtype; ad.rounding = add_rounding;
+    ad.seed = add_seed; ad.offset = add_offset;
+    return launch_layernorm_bwd_strip(qx, sx, qg, sg, gamma, mean, rstd, R, C, scale_dtype, rounding, seed, offset, nullptr,
+                                      nullptr, dgamma, dbeta, workspace, &ad, strip_dgamma, (hipStream_t)stream);
 }
 
 extern "C" {
@@ -1389,23 +1417,19 @@ int jf_layernorm_bwd_add(const int8_t *qx, const void *sx, const int8_t *qg, con
                          uint64_t add_offset, void *y1, int y1_dtype, int8_t *q, void *s, float *dgamma, float *dbeta,
                          void *workspace, size_t workspace_bytes, jf_stream_t stream)
 {
-    int rc = check_block_tensor(qx, sx, R, C, scale_dtype);
-    if (rc) return rc;
-    if ((rc = check_block_tensor(qg, sg, R, C, scale_dtype))) return rc;
-    if (!gamma || !mean || !rstd || !x1 || !y1 || !q || !s) return JF_ERR_NULL;
-    if (!rounding_ok(rounding) || !rounding_ok(add_rounding)) return JF_ERR_ENUM;
-    if (x1_dtype < JF_FP_F16 || x1_dtype > JF_FP_BF16 || y1_dtype < JF_FP_F16 || y1_dtype > JF_FP_BF16) return JF_ERR_ENUM;
-    if (!aligned16(gamma) || !aligned16(x1) || !aligned16(y1) || !aligned16(q)) return JF_ERR_ALIGN;
-    if (C / QB > LNS_WAVES * LNS_BPW) return JF_ERR_SHAPE;         // wider rows: jf_layernorm_bwd, then jf_add
-    if (!workspace || workspace_bytes < jf_layernorm_bwd_workspace_bytes(R, C)) return JF_ERR_WORKSPACE;
-    if (!aligned16(workspace)) return JF_ERR_ALIGN;
-    if (!device_is_gfx950()) return JF_ERR_DEVICE;
-    LnAddArgs ad;
-    ad.x1 = x1; ad.y1 = y1; ad.q = q; ad.s = s;
-    ad.x1_dtype = x1_dtype; ad.y1_dtype = y1_dtype; ad.rounding = add_rounding;
-    ad.seed = add_seed; ad.offset = add_offset;
-    return launch_layernorm_bwd_strip(qx, sx, qg, sg, gamma, mean, rstd, R, C, scale_dtype, rounding, seed, offset, nullptr,
-                                      nullptr, dgamma, dbeta, workspace, &ad, (hipStream_t)stream);
+    if (workspace_bytes < jf_layernorm_bwd_workspace_bytes(R, C)) workspace = nullptr;
+    return layernorm_bwd_add(qx, sx, qg, sg, gamma, mean, rstd, R, C, scale_dtype, rounding, seed, offset, x1, x1_dtype, add_rounding, add_seed,
+                             add_offset, y1, y1_dtype, q, s, dgamma, dbeta, nullptr, workspace, stream);
+}
+
+int jf_layernorm_bwd_add_strips(const int8_t *qx, const void *sx, const int8_t *qg, const void *sg, const float *gamma, const float *mean,
+                                const float *rstd, int R, int C, int scale_dtype, int rounding, uint64_t seed, uint64_t offset,
+                                const void *x1, int x1_dtype, int add_rounding, uint64_t add_seed, uint64_t add_offset, void *y1,
+                                int y1_dtype, int8_t *q, void *s, float *strip_dgamma, jf_stream_t stream)
+{
+    if (!strip_dgamma) return JF_ERR_NULL;
+    return layernorm_bwd_add(qx, sx, qg, sg, gamma, mean, rstd, R, C, scale_dtype, rounding, seed, offset, x1, x1_dtype, add_rounding, add_seed,
+                             add_offset, y1, y1_dtype, q, s, nullptr, nullptr, strip_dgamma, nullptr, stream);
 }
 
 int jf_layernorm_bwd(const int8_t *qx, const void *sx, const int8_t *qg, const void *sg, const float *gamma,
@@ -1427,7 +1451,7 @@ int jf_layernorm_bwd(const int8_t *qx, const void *sx, const int8_t *qg, const v
     const int SC = C / QB, groups = lnb_groups(R);
     if (SC <= LNS_WAVES * LNS_BPW)
         return launch_layernorm_bwd_strip(qx, sx, qg, sg, gamma, mean, rstd, R, C, scale_dtype, rounding, seed, offset, qdx,
-                                          sdx, dgamma, dbeta, workspace, nullptr, st);
+                                          sdx, dgamma, dbeta, workspace, nullptr, nullptr, st);
     const size_t smem = ((size_t)C + 2 * QB + 16 * QB) * sizeof(float);   // gamma, c1, c2 and the row-sum partials in LDS
     if (smem > LDS_VECTOR_LIMIT) return JF_ERR_SHAPE;
     float *part1 = (float *)workspace, *part2 = part1 + (size_t)R * SC;

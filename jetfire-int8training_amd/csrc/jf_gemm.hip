@@ -75,15 +75,20 @@ struct GemmArgs {
     int phase_capacity;
 };
 
-// Logical tile (and K split) of this workgroup.  Workgroups are dealt round-robin to the 8 XCDs, each with a
-// private L2: give every XCD one contiguous run of the launch's work, and walk tiles in groups of 8 tile-rows so
-// that concurrently resident workgroups of an XCD share A and B panels.  With K splits the order is split-major.
-__device__ __forceinline__ void tile_of_workgroup(int tiles_m, int tiles_n, bool has_splits, int &tm, int &tn, int &split)
+// Position of this workgroup in the launch's work.  Workgroups are dealt round-robin to the 8 XCDs, each with a private L2:
+// every XCD gets one contiguous run of the work.
+__device__ __forceinline__ int logical_workgroup()
 {
     const int nwg = gridDim.x, wg = blockIdx.x;
     const int xcd = wg & 7, idx = wg >> 3;
     const int per = nwg >> 3, rem = nwg & 7;
-    int logical = xcd * per + (xcd < rem ? xcd : rem) + idx;
+    return xcd * per + (xcd < rem ? xcd : rem) + idx;
+}
+
+// Tile (and K split) at a position of a GEMM's work: tiles in groups of 8 tile-rows, so that concurrently resident workgroups
+// of an XCD share A and B panels.  With K splits the order is split-major.
+__device__ __forceinline__ void tile_at(int logical, int tiles_m, int tiles_n, bool has_splits, int &tm, int &tn, int &split)
+{
     split = has_splits ? logical / (tiles_m * tiles_n) : 0;
     logical -= split * (tiles_m * tiles_n);
     constexpr int GROUP = 8;
@@ -108,12 +113,13 @@ constexpr int WBN = 1;
 // BKN = 0: B is [N, ldb] (K-contiguous rows, like A).  BKN = 1: B is [K, ldb] (N-contiguous rows); its tile is staged
 // as it lies in memory and the K-contiguous MFMA operand is produced by the transposing LDS read of gfx950.
 static int cu_count();
+static int pace_of(long wgs, long slots, int k_per_wg);
 
 // PROF = 1: the first wave of every workgroup also records when the workgroup's phases began and ended (wall clock) and
 // how many shader cycles its main loop took: a profiling build of the same code, instantiated only in the measurement
 // library (jf_prof_igemm_block_q).
-template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
-__global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt_kernel(GemmArgs p_in)
+template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM, int PROF>
+__device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logical)
 {
     GemmArgs p = p_in;                                        // K-split launches narrow it to the split's K range below
     unsigned long long *const prof_buf = p_in.phases;
@@ -144,7 +150,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
     const int wm = wave % WGM, wn = wave / WGM;
 
     int tile_m, tile_n, split;
-    tile_of_workgroup(p.tiles_m, p.tiles_n, EPI == EPI_FP && p.splits > 1, tile_m, tile_n, split);
+    tile_at(logical, p.tiles_m, p.tiles_n, EPI == EPI_FP && p.splits > 1, tile_m, tile_n, split);
     int kb_base = 0;                                          // first K block of this workgroup (scale indices count from 0)
     if (EPI == EPI_FP && p.splits > 1) {                      // uniform: the same problem on a K range, fp32 partial output
         kb_base = split * p.kb_per_split;
@@ -847,6 +853,30 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt
 #undef phase
 }
 
+template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
+__global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt_kernel(GemmArgs p)
+{
+    igemm_body<EPI, ST, WBM, WGM, WGN, NSTAGE, WGPC, BKN, AKM, PROF>(p, logical_workgroup());
+}
+
+// Several weight gradients over the same tokens in one launch (jf_wgrad_many): the work of one follows the other's.
+constexpr int WGRAD_MAX = 4;
+struct GemmGroup {
+    GemmArgs g[WGRAD_MAX];
+    int end[WGRAD_MAX];       // first workgroup behind problem k
+    int n;
+};
+template <typename ST>
+__global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp)
+{
+    const int logical = logical_workgroup();
+    int k = 0, begin = 0;
+#pragma unroll
+    for (int i = 1; i < WGRAD_MAX; ++i)
+        if (i < grp.n && logical >= grp.end[i - 1]) { k = i; begin = grp.end[i - 1]; }
+    igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0>(grp.g[k], logical - begin);
+}
+
 // -------------------------------------------------------------------------------------------------
 // int8 transpose: out[C,R] = in[R,C].  TR_ROWS x 64 tiles through LDS: 16-byte loads, the transposing LDS read of gfx950
 // (ds_read_b64_tr_b8, as for the GEMM's [K,N] operands) and 16-byte stores.  The instruction works on groups of 16 lanes:
@@ -902,51 +932,72 @@ static int launch_transpose(const int8_t *in, int R, int C, int8_t *out, hipStre
     return (int)hipGetLastError();
 }
 
+// LDS of a workgroup: operand ring and per-wave scale and product patches, or the epilogue's per-wave transposition patches
+constexpr int gemm_lds(int WBM, int WGM, int WGN, int NSTAGE)
+{
+    const int ring = NSTAGE * ((QB * WBM * WGM + QB * WBN * WGN) * ROW_BYTES + WGM * WGN * 512), patch = WGM * WGN * QB * EPI_LD * (int)sizeof(float);
+    return ring > patch ? ring : patch;
+}
+
+// more than 64 KiB of dynamic LDS has to be opted into, per function and device: once, not on every launch
+// (the reference sets its attribute on every call, igemm_BlockSquare32OutputIntQuantizeBiasRowCol.cu:418)
+static int allow_lds(const void *kern, int bytes, std::atomic<bool> (&opted_in)[MAX_DEVICES])
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return JF_ERR_DEVICE;
+    if (!opted_in[dev].load(std::memory_order_acquire)) {
+        hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        if (e != hipSuccess) return (int)e;
+        opted_in[dev].store(true, std::memory_order_release);
+    }
+    return JF_OK;
+}
+
+// Pace of the workgroups that share a CU.  Left to the hardware, the older one runs ahead: a launch ends with every CU
+// half empty while the younger workgroups finish alone, at two thirds of the shared throughput (two waves per SIMD
+// meeting at a barrier).  Kept in step by wave priorities (PACE_EVEN) they finish together: 5-16 % faster for launches
+// of up to two rounds of workgroups.  The exception is a launch of between 1 and 1.5 rounds: there the early finishers
+// are what starts the short second round early, and an even pace is 5-9 % slower than the hardware's order.  A strict
+// order with fairness inside each workgroup (PACE_ORDERED) does that job 4-6 % better than the hardware when tiles are
+// long (K >= 4096) and 5-16 % worse when they are short.  Beyond two rounds the schemes are within 3 % of each other,
+// either way depending on shape and data: left to the hardware.  (All measured; results do not depend on the scheme.)
+static int pace_of(long wgs, long slots, int k_per_wg)
+{
+    if (wgs > slots && 2 * wgs < 3 * slots) return k_per_wg >= 4096 ? PACE_ORDERED : PACE_HARDWARE;      // a short second round
+    return wgs <= 2 * slots ? PACE_EVEN : PACE_HARDWARE;
+}
+
 template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
 static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 {
     constexpr int BM = QB * WBM * WGM, BN = QB * WBN * WGN, NT = 64 * WGM * WGN;
-    constexpr int RING = NSTAGE * ((BM + BN) * ROW_BYTES + WGM * WGN * 512);         // operand ring + per-wave scale and product patches
-    constexpr int PATCH = WGM * WGN * QB * EPI_LD * (int)sizeof(float);     // the epilogue's per-wave transposition patches
-    constexpr int SMEM = RING > PATCH ? RING : PATCH;
+    constexpr int SMEM = gemm_lds(WBM, WGM, WGN, NSTAGE);
     if (!device_is_gfx950()) return JF_ERR_DEVICE;
     GemmArgs p = a;
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
     auto kern = igemm_nt_kernel<EPI, ST, WBM, WGM, WGN, NSTAGE, WGPC, BKN, AKM, PROF>;
-    // more than 64 KiB of dynamic LDS has to be opted into, per function and device: once, not on every launch
-    // (the reference sets its attribute on every call, igemm_BlockSquare32OutputIntQuantizeBiasRowCol.cu:418)
     static std::atomic<bool> opted_in[MAX_DEVICES] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return JF_ERR_DEVICE;
-    if (!opted_in[dev].load(std::memory_order_acquire)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
-        if (e != hipSuccess) return (int)e;
-        opted_in[dev].store(true, std::memory_order_release);
-    }
+    if (int rc = allow_lds(reinterpret_cast<const void *>(kern), SMEM, opted_in)) return rc;
     if (EPI != EPI_FP || p.splits < 1) p.splits = 1;
-    // Pace of the workgroups that share a CU.  Left to the hardware, the older one runs ahead: a launch ends with every CU
-    // half empty while the younger workgroups finish alone, at two thirds of the shared throughput (two waves per SIMD
-    // meeting at a barrier).  Kept in step by wave priorities (PACE_EVEN) they finish together: 5-16 % faster for launches
-    // of up to two rounds of workgroups.  The exception is a launch of between 1 and 1.5 rounds: there the early finishers
-    // are what starts the short second round early, and an even pace is 5-9 % slower than the hardware's order.  A strict
-    // order with fairness inside each workgroup (PACE_ORDERED) does that job 4-6 % better than the hardware when tiles are
-    // long (K >= 4096) and 5-16 % worse when they are short.  Beyond two rounds the schemes are within 3 % of each other,
-    // either way depending on shape and data: left to the hardware.  (All measured; results do not depend on the scheme.)
-    const long wgs = (long)p.tiles_m * p.tiles_n * p.splits, slots = (long)WGPC * cu_count();
-    const bool short_second_round = wgs > slots && 2 * wgs < 3 * slots;
-    const int k_per_wg = p.splits > 1 ? p.kb_per_split * QB : p.K;
-    if (WBM == 1) p.pace = PACE_HARDWARE;                     // (no paced instances: all its workgroups are resident)
-    else p.pace = short_second_round ? (k_per_wg >= 4096 ? PACE_ORDERED : PACE_HARDWARE)
-                                : (wgs <= 2 * slots ? PACE_EVEN : PACE_HARDWARE);
+    p.pace = WBM == 1 ? (int)PACE_HARDWARE                    // (no paced instances: all its workgroups are resident)
+                      : pace_of((long)p.tiles_m * p.tiles_n * p.splits, (long)WGPC * cu_count(), p.splits > 1 ? p.kb_per_split * QB : p.K);
     hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n * p.splits), dim3(NT), SMEM, st, p);
     return (int)hipGetLastError();
 }
 
-// out[i] = convert(part[0][i] + part[1][i] + ... + part[S-1][i]), added in ascending split order.
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *part, size_t n, int splits, void *out, int out_dtype)
+template <typename ST> static int launch_wgrad_group(const GemmGroup &grp, unsigned wgs, hipStream_t st)
 {
-    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    constexpr int SMEM = gemm_lds(2, 2, 4, 2);
+    static std::atomic<bool> opted_in[MAX_DEVICES] = {};
+    if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_wgrad_group_kernel<ST>), SMEM, opted_in)) return rc;
+    hipLaunchKernelGGL(igemm_wgrad_group_kernel<ST>, dim3(wgs), dim3(512), SMEM, st, grp);
+    return (int)hipGetLastError();
+}
+
+// out[i] = convert(part[0][i] + part[1][i] + ... + part[S-1][i]), added in ascending split order, for the four elements at i.
+__device__ __forceinline__ void reduce_splits(const float *part, size_t n, int splits, void *out, int out_dtype, size_t i)
+{
     if (i >= n) return;                                        // n is a multiple of 1024
     v4f t = *reinterpret_cast<const v4f *>(part + i);
     for (int s = 1; s < splits; ++s) {
@@ -961,6 +1012,59 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *part, s
     } else {
         __bf16 h[4] = {(__bf16)t.x, (__bf16)t.y, (__bf16)t.z, (__bf16)t.w};
         *reinterpret_cast<v2i *>(reinterpret_cast<__bf16 *>(out) + i) = *reinterpret_cast<v2i *>(h);
+    }
+}
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *part, size_t n, int splits, void *out, int out_dtype)
+{
+    reduce_splits(part, n, splits, out, out_dtype, ((size_t)blockIdx.x * 256 + threadIdx.x) * 4);
+}
+
+// What follows the weight gradients of a block, one launch: the K splits of each (as splitk_reduce_kernel) and column sums over
+// per-strip terms (the gradients of the LayerNorm weights; the order of layernorm_bwd_colsum_finish_kernel: thread (g, column)
+// adds the strips g, g + 32, ... ascending, then the 32 partial sums are added ascending).
+struct WgradFinish {
+    const float *part[WGRAD_MAX];
+    void *out[WGRAD_MAX];
+    size_t count[WGRAD_MAX];  // elements of gradient k
+    int end[WGRAD_MAX];       // first workgroup behind gradient k (4096 elements each)
+    const float *terms[WGRAD_MAX];                             // [strips][width]
+    float *sum[WGRAD_MAX];
+    int width[WGRAD_MAX], cend[WGRAD_MAX];                     // first workgroup behind column sum k (32 columns each)
+    int n, ncol, splits, strips, out_dtype;
+};
+__global__ __launch_bounds__(1024) void wgrad_finish_kernel(WgradFinish f)
+{
+    __shared__ float red[32][QB + 1];
+    const int wg = blockIdx.x, nred = f.n > 0 ? f.end[f.n - 1] : 0;
+    int k = 0, begin = 0;
+    if (wg < nred) {
+#pragma unroll
+        for (int i = 1; i < WGRAD_MAX; ++i)
+            if (i < f.n && wg >= f.end[i - 1]) { k = i; begin = f.end[i - 1]; }
+        reduce_splits(f.part[k], f.count[k], f.splits, f.out[k], f.out_dtype, ((size_t)(wg - begin) * 1024 + threadIdx.x) * 4);
+        return;
+    }
+    begin = nred;
+#pragma unroll
+    for (int i = 1; i < WGRAD_MAX; ++i)
+        if (i < f.ncol && wg >= f.cend[i - 1]) { k = i; begin = f.cend[i - 1]; }
+    const float *src = f.terms[k];
+    const int C = f.width[k], x = threadIdx.x & 31, c = (wg - begin) * QB + x, g = threadIdx.x >> 5;
+    float acc = 0.0f;
+    for (int s0 = g; s0 < f.strips; s0 += 256) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) { const int s = s0 + 32 * i; v[i] = s < f.strips ? src[(size_t)s * C + c] : 0.0f; }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc = acc + v[i];
+    }
+    red[g][x] = acc;
+    __syncthreads();
+    if (g == 0) {
+        float t = red[0][x];
+#pragma unroll
+        for (int i = 1; i < 32; ++i) t = t + red[i][x];
+        f.sum[k][c] = t;
     }
 }
 
@@ -994,6 +1098,30 @@ static void splitk_plan(int M, int N, int K, int request, int &splits, int &kb_p
     if (want < 1) want = 1;
     kb_per_split = ((nkb + want - 1) / want + 3) / 4 * 4;
     splits = (nkb + kb_per_split - 1) / kb_per_split;
+}
+
+// K split of a group of weight gradients (one for all of them: they share K).  The launch takes, on the fullest CU, as many
+// tiles as fall to it times their K blocks: about 0.27 us per block for a lone tile and 0.2 us per tile beyond (GPT-2 XL and
+// small gradients), 3 us of ramp and epilogue per pair of tiles; parts cost a write and a read of every partial sum at about
+// 8 TB/s (they stay in the caches).  One split for a GPT-2 block at 8 x 1024 or 12 x 1024 tokens (XL: 532 us in four launches
+// -> 500; small: 225 us with four sums of parts -> 180), four for a 256-wide one over 1024.  Parts are at least 8 K blocks (two stages) of at least 16.
+static void wgrad_group_plan(int n, const int *M, const int *N, int K, int &splits, int &kb_per_split)
+{
+    const int nkb = K / QB;
+    long tiles = 0;
+    double elems = 0;
+    for (int i = 0; i < n; ++i) {
+        tiles += (long)((M[i] + 127) / 128) * ((N[i] + 127) / 128);
+        elems += (double)M[i] * N[i];
+    }
+    double best = 0;
+    splits = 1; kb_per_split = nkb;
+    for (int s = 1; s <= 16 && (s == 1 || (nkb >= 16 && nkb / s >= 8)); ++s) {
+        const int kb = s == 1 ? nkb : ((nkb + s - 1) / s + KB_STAGE - 1) / KB_STAGE * KB_STAGE, parts = (nkb + kb - 1) / kb;
+        const long per_cu = (tiles * parts + cu_count() - 1) / cu_count();
+        const double t = kb * (0.2 * per_cu + (per_cu & 1 ? 0.07 : 0.0)) + 3.0 * ((per_cu + 1) / 2) + (parts > 1 ? parts * elems * 8 / 8e6 : 0.0);
+        if (s == 1 || t < best) { best = t; splits = parts; kb_per_split = kb; }
+    }
 }
 
 // Tile configuration.  Large launches: 128x128 tiles, 8 waves of two blocks, a 2-deep ring and two workgroups per CU (the
@@ -1183,6 +1311,69 @@ int jf_igemm_block_fp(const int8_t *A, const int8_t *B, const void *sa, const vo
         return JF_ERR_WORKSPACE;
     return block_fp_run(A, B, sa, sb, C, M, N, K, a_layout, b_layout, scale_dtype, sa_layout, sb_layout, out_dtype, splits,
                         kb_per, workspace, (hipStream_t)stream);
+}
+
+size_t jf_wgrad_many_workspace_bytes(int n, const int *M, const int *N, int K)
+{
+    if (n < 1 || n > WGRAD_MAX || !M || !N || !mult32(K)) return 0;
+    int splits, kb;
+    wgrad_group_plan(n, M, N, K, splits, kb);
+    size_t bytes = 0;
+    for (int i = 0; splits > 1 && i < n; ++i) bytes += (size_t)splits * (size_t)M[i] * (size_t)N[i] * sizeof(float);
+    return bytes;
+}
+
+int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
+                  const int *M, const int *N, int K, int scale_dtype, int out_dtype, int ncol, const float *const *terms,
+                  const int *width, float *const *sum, void *workspace, size_t workspace_bytes, jf_stream_t stream)
+{
+    if (n < 1 || n > WGRAD_MAX || ncol < 0 || ncol > WGRAD_MAX) return JF_ERR_SHAPE;
+    if (!G || !SG || !X || !SX || !out || !M || !N || (ncol && (!terms || !width || !sum))) return JF_ERR_NULL;
+    int splits, kb_per;
+    for (int i = 0; i < n; ++i) {
+        int rc = block_fp_check(G[i], X[i], SG[i], SX[i], out[i], M[i], N[i], K, JF_A_KM, JF_B_KN, scale_dtype, out_dtype);
+        if (rc) return rc;
+    }
+    for (int i = 0; i < ncol; ++i) {
+        if (!terms[i] || !sum[i]) return JF_ERR_NULL;
+        if (!mult32(width[i])) return JF_ERR_SHAPE;
+    }
+    if (!device_is_gfx950()) return JF_ERR_DEVICE;
+    wgrad_group_plan(n, M, N, K, splits, kb_per);
+    if (splits > 1 && (!workspace || !aligned16(workspace) || workspace_bytes < jf_wgrad_many_workspace_bytes(n, M, N, K))) return JF_ERR_WORKSPACE;
+    GemmGroup grp = {};
+    WgradFinish fin = {};
+    float *part = (float *)workspace;
+    long wgs = 0, fwgs = 0;
+    for (int i = 0; i < n; ++i) {
+        GemmArgs &a = grp.g[i];
+        a.A = G[i]; a.B = X[i]; a.sa = SG[i]; a.sb = SX[i]; a.C = splits > 1 ? (void *)part : out[i];
+        a.M = M[i]; a.N = N[i]; a.K = K; a.lda = M[i]; a.ldb = N[i]; a.out_dtype = out_dtype; a.splits = splits; a.kb_per_split = kb_per;
+        a.sa_ks = M[i] / QB; a.sa_is = 1; a.sb_ks = N[i] / QB; a.sb_is = 1;
+        a.tiles_m = (M[i] + 127) / 128; a.tiles_n = (N[i] + 127) / 128;
+        wgs += (long)a.tiles_m * a.tiles_n * splits;
+        grp.end[i] = (int)wgs;
+        if (splits > 1) {
+            const size_t count = (size_t)M[i] * (size_t)N[i];
+            fwgs += (long)((count + 4095) / 4096);
+            fin.part[i] = part; fin.out[i] = out[i]; fin.count[i] = count; fin.end[i] = (int)fwgs;
+            part += (size_t)splits * count;
+        }
+    }
+    for (int i = 0; i < ncol; ++i) {
+        fwgs += width[i] / QB;
+        fin.terms[i] = terms[i]; fin.sum[i] = sum[i]; fin.width[i] = width[i]; fin.cend[i] = (int)fwgs;
+    }
+    if (wgs > 0x7fffffffL || fwgs > 0x7fffffffL) return JF_ERR_SHAPE;
+    grp.n = n;
+    fin.n = splits > 1 ? n : 0; fin.ncol = ncol; fin.splits = splits; fin.strips = K / QB; fin.out_dtype = out_dtype;
+    const int pace = pace_of(wgs, 2L * cu_count(), kb_per * QB);
+    for (int i = 0; i < n; ++i) grp.g[i].pace = pace;
+    hipStream_t st = (hipStream_t)stream;
+    int rc = scale_dtype == JF_SCALE_F16 ? launch_wgrad_group<half_t>(grp, (unsigned)wgs, st) : launch_wgrad_group<float>(grp, (unsigned)wgs, st);
+    if (rc || fwgs == 0) return rc;
+    hipLaunchKernelGGL(wgrad_finish_kernel, dim3((unsigned)fwgs), dim3(1024), 0, st, fin);
+    return (int)hipGetLastError();
 }
 
 // ---- the allocation-free weight-gradient entry point ---------------------------------------------------------------

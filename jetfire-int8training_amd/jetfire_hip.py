@@ -28,9 +28,9 @@ EXPORTS = [
     "jf_error_string", "jf_igemm_workspace_bytes", "jf_igemm_s32", "jf_igemm_block_acc", "jf_igemm_block_fp",
     "jf_igemm_splitk_plan", "jf_igemm_block_fp_workspace_bytes", "jf_igemm_block_q_gelu", "jf_igemm_block_fp_noalloc", "jf_igemm_block_q_gelu_bwd",
     "jf_igemm_block_q", "jf_quantize", "jf_dequantize", "jf_transpose_s8", "jf_rowstats", "jf_layernorm_fwd",
-    "jf_layernorm_bwd_workspace_bytes", "jf_layernorm_bwd", "jf_layernorm_bwd_add", "jf_gelu_fwd", "jf_gelu_bwd", "jf_add", "jf_rowstats_finish",
+    "jf_layernorm_bwd_workspace_bytes", "jf_layernorm_bwd", "jf_layernorm_bwd_add", "jf_layernorm_bwd_add_strips", "jf_gelu_fwd", "jf_gelu_bwd", "jf_add", "jf_rowstats_finish",
     "jf_igemm_block_q_dequant", "jf_quantize_slabs", "jf_philox_rounds", "jf_block_colsum", "jf_block_colsum_workspace_bytes",
-    "jf_attention_fwd", "jf_attention_bwd", "jf_quantize_many", "jf_rowstats_fp",
+    "jf_attention_fwd", "jf_attention_bwd", "jf_quantize_many", "jf_rowstats_fp", "jf_wgrad_many", "jf_wgrad_many_workspace_bytes",
 ]
 
 _lib = None
@@ -52,6 +52,9 @@ def lib():
         L.jf_igemm_block_acc.argtypes = [_p, _p, _p, _i, _i, _i, _i, _p, _sz, _p]
         L.jf_igemm_block_fp.argtypes = [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p, _sz, _p]
         L.jf_igemm_block_fp_noalloc.argtypes = [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p]
+        L.jf_wgrad_many_workspace_bytes.argtypes = [_i, _p, _p, _i]
+        L.jf_wgrad_many_workspace_bytes.restype = _sz
+        L.jf_wgrad_many.argtypes = [_i, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _p, _p, _sz, _p]
         L.jf_igemm_block_q_gelu_bwd.argtypes = [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _u64, _u64, _i, _u64, _u64, _p]
         L.jf_igemm_block_q_dequant.argtypes = [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _u64, _u64, _p]
         L.jf_igemm_block_q_gelu.argtypes = [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _f, _p]
@@ -279,6 +282,37 @@ def igemm_block_fp_noalloc(A, B, sa, sb, out, b_layout=B_KN, a_layout=A_MK, spli
     check(lib().jf_igemm_block_fp_noalloc(_ptr(A), _ptr(B), _ptr(sa), _ptr(sb), _ptr(out), M, N, K, a_layout, b_layout,
                                           code, la, lb, _FP_CODE[out.dtype], splitk, _stream()))
     return out
+
+
+def wgrad_many(gs, xs, out_dtype=torch.float32, terms=()):
+    """Weight gradients of up to 4 layers over the same tokens in one launch: gs, xs = [(codes [K, .], scales [K/32, ./32]), ...],
+    the output gradients and inputs of the layers; terms: up to 4 [K/32, width] float32 tensors, whose column sums come with
+    them.  Returns ([dW [M, N], ...], [sum [width], ...])."""
+    n, K = len(gs), gs[0][0].shape[0]
+    codes = set()
+    for q, s in list(gs) + list(xs):
+        R, _, code = _block_tensor(q, s, "operand")
+        codes.add(code)
+        if R != K:
+            raise RuntimeError("operands must have the same number of tokens")
+    if n != len(xs) or len(codes) != 1:
+        raise RuntimeError("one input per gradient and one scale dtype expected")
+    for t in terms:
+        _need(t, torch.float32, "terms", 2)
+        if t.shape[0] != K // QB:
+            raise RuntimeError("terms: expected one row per strip of 32 tokens")
+    Ms, Ns = [q.shape[1] for q, _ in gs], [q.shape[1] for q, _ in xs]
+    dev = gs[0][0].device
+    out = [torch.empty((m, k), dtype=out_dtype, device=dev) for m, k in zip(Ms, Ns)]
+    sums = [torch.empty(t.shape[1], dtype=torch.float32, device=dev) for t in terms]
+    ptrs = lambda ts: (C.c_void_p * max(1, len(ts)))(*[t.data_ptr() for t in ts])  # noqa: E731
+    ints = lambda v: (C.c_int * max(1, len(v)))(*v)  # noqa: E731
+    nb = lib().jf_wgrad_many_workspace_bytes(n, ints(Ms), ints(Ns), K)
+    ws = torch.empty(nb, dtype=torch.int8, device=dev) if nb else None
+    check(lib().jf_wgrad_many(n, ptrs([q for q, _ in gs]), ptrs([s for _, s in gs]), ptrs([q for q, _ in xs]), ptrs([s for _, s in xs]),
+                              ptrs(out), ints(Ms), ints(Ns), K, codes.pop(), _FP_CODE[out_dtype], len(terms), ptrs(terms),
+                              ints([t.shape[1] for t in terms]), ptrs(sums), _ptr(ws), nb, _stream()))
+    return out, sums
 
 
 def igemm_block_q_gelu(A, B, sa, sb, approx=GELU_ERF, amax_eps=5e-5, bias=None, biasmax=None):

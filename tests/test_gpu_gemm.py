@@ -497,3 +497,26 @@ def test_both_tile_sizes_at_every_ring_fill(jf, oracle, M, N, K):
         wq, wsc = oracle.igemm_block_q(A, B, sa, sb, layout, stochastic=True, seed=4, offset=8, scale_dtype="f16")
         same(q, wq, "SR codes")
         same(sc, wsc, "SR scales")
+
+
+@pytest.mark.parametrize("K", [32, 480, 512, 1056])               # one K block, the longest without and the shortest with a K split, a ragged split
+@pytest.mark.parametrize("widths", [[(96, 32)], [(384, 160), (128, 160), (512, 128), (32, 544)]])
+@pytest.mark.parametrize("f16,out", [(True, torch.float32), (False, torch.bfloat16)])
+def test_weight_gradients_in_one_launch(jf, oracle, K, widths, f16, out):
+    print(f"case K={K} widths={widths}", flush=True)
+    rng = np.random.default_rng(K)
+    st = np.float16 if f16 else np.float32
+    operand = lambda c: (rand_codes(rng, (K, c)), rand_scales(rng, (K // QB, c // QB), f16=f16))  # noqa: E731
+    gs, xs = [operand(m) for m, _ in widths], [operand(n) for _, n in widths]
+    terms = [rng.standard_normal((K // QB, c)).astype(np.float32) for c in (32, 544)]
+    d = lambda ts: [(dev(q), dev(s.astype(st))) for q, s in ts]  # noqa: E731
+    got, sums = jf.wgrad_many(d(gs), d(xs), out, [dev(t) for t in terms])
+    for (g, sg), (x, sx), o in zip(gs, xs, got):
+        want = torch.from_numpy(oracle.igemm_block_f32(np.ascontiguousarray(g.T), x, sg, sx, 1))
+        if K < 512:
+            assert torch.equal(o.cpu(), want.to(out))
+        else:
+            assert float((o.cpu().double() - want.double()).norm() / want.double().norm()) < (1e-5 if out == torch.float32 else 4e-3)
+    for t, s in zip(terms, sums):
+        np.testing.assert_allclose(s.cpu().numpy(), t.astype(np.float64).sum(0), atol=1e-5)
+    assert jf.wgrad_many(d(gs[:1]), d(xs[:1]), out)[0][0].shape == got[0].shape
