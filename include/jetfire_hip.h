@@ -222,6 +222,10 @@ int jf_rowstats_fp(const void *x, int x_dtype, int R, int C, float *mean, float 
 int jf_layernorm_fwd(const int8_t *q, const void *s, const float *gamma, const float *beta,
                      const float *mean, const float *rstd, int R, int C, int scale_dtype,
                      int8_t *qy, void *sy, jf_stream_t stream);
+/* jf_rowstats_finish(rowsum, rowsq) -> (mean, rstd) and jf_layernorm_fwd of them as one kernel, same bits. */
+int jf_layernorm_fwd_sums(const int8_t *q, const void *s, const float *gamma, const float *beta, const float *rowsum, const float *rowsq,
+                          int R, int C, int scale_dtype, float *mean, float *rstd, int8_t *qy, void *sy, jf_stream_t stream);
+
 
 /* Bytes of scratch for jf_layernorm_bwd. */
 size_t jf_layernorm_bwd_workspace_bytes(int R, int C);
@@ -311,12 +315,22 @@ int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const in
  * (INT8_GPT2/qmodel.py:134). */
 int jf_attention_fwd(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale, void *out,
                      float *lse, jf_stream_t stream);
+/* The same with the block quantisation of the result (round to nearest, binary16 scales) next to it. */
+int jf_attention_fwd_q(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale, void *out,
+                       float *lse, int8_t *codes, void *scales, jf_stream_t stream);
+
 
 /* Its gradients: gq, gk, gv ([B*T, ldg], laid out like q, k, v) from gout [B*T, H*D] and the forward's out and lse.
  * delta: [B*H, T] fp32 scratch.  Every sum has one owner and a fixed order: the same bits on every run. */
 int jf_attention_bwd(const void *q, const void *k, const void *v, int ld, const void *out, const void *gout, const float *lse,
                      int B, int H, int T, int D, float scale, void *gq, void *gk, void *gv, int ldg, float *delta,
                      jf_stream_t stream);
+/* The same with the gradients quantised (stochastic rounding, binary16 scales) instead of stored: codes [B*T, 3 H D], what
+ * quantising the three binary16 gradients side by side gives. */
+int jf_attention_bwd_q(const void *q, const void *k, const void *v, int ld, const void *out, const void *gout, const float *lse,
+                       int B, int H, int T, int D, float scale, int8_t *codes, void *scales, uint64_t seed, uint64_t offset, float *delta,
+                       jf_stream_t stream);
+
 
 #ifdef __cplusplus
 }

@@ -39,6 +39,9 @@ struct AttnArgs {
     float *delta;                   // [B*H, T]: sum over D of o * go (left by the dQ kernel, read by the dK/dV kernel)
     int ld, ldg, B, H, T;
     float scale;                    // of the scores
+    int8_t *cq;                     // codes and scales of the result [B*T, C] or of the gradients [B*T, 3C] (kernels with QUANT)
+    half_t *cs;
+    uint64_t seed, offset;          // of the gradients' rounding noise
 };
 
 constexpr int ATT_ROWS = 64;        // rows of a shared tile
@@ -135,20 +138,57 @@ __device__ __forceinline__ h8 pack8(const v16f &x, int s)
     for (int j = 0; j < 8; ++j) r[j] = (half_t)x[8 * s + j];
     return r;
 }
-// a transposed result block (lane: row l%32 of the output, columns 8g + 4h + 0..3) times a factor, stored as binary16
-__device__ __forceinline__ void store_t(half_t *row, int h, const v16f &x, float f)
+// a result block times a factor, rounded to binary32 (pinned: the compiler would fold the product into some of the conversions
+// to binary16 and not into others, with one rounding less)
+__device__ __forceinline__ void scale_t(v16f &x, float f)
+{
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        float t = x[v] * f;
+        asm volatile("" : "+v"(t));
+        x[v] = t;
+    }
+}
+// a transposed result block (lane: row l%32 of the output, columns 8g + 4h + 0..3), stored as binary16
+__device__ __forceinline__ void store_t(half_t *row, int h, const v16f &x)
 {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         h4 t;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) t[j] = (half_t)(x[4 * g + j] * f);
+        for (int j = 0; j < 4; ++j) t[j] = (half_t)x[4 * g + j];
         *reinterpret_cast<h4 *>(row + 8 * g + 4 * h) = t;
     }
 }
 
-template <int D, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(AttnArgs a)
+// The block quantisation (quantize.py:33-117) of a wave's result while it is still in registers: a transposed result block is
+// one 32x32 quantisation block (lane: row l%32, columns 8g + 4h + 0..3).  Two 32-lane exchanges per pair of registers give each
+// lane 16 consecutive columns (half l/32 of its row), which is what the rounding noise is drawn for.  Values are rounded to
+// binary16 first: codes, scales and noise are those of quantising the stored binary16 tensor.  row, col: the block's first
+// element in a [., C] tensor.
+__device__ __forceinline__ void quantize_t(const v16f &x, int8_t *codes, half_t *scales, int row, int col, int C, int lane, int rounding,
+                                           uint64_t seed, uint64_t offset)
+{
+    float y[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) y[v] = (float)(half_t)x[v];
+    float z[16];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[4 * g + j]), __float_as_uint(y[8 + 4 * g + j]), false, false);
+            z[8 * g + j] = __uint_as_float(p[0]);
+            z[8 * g + 4 + j] = __uint_as_float(p[1]);
+        }
+    const size_t e0 = (size_t)(row + (lane & 31)) * C + col + 16 * (lane >> 5);
+    float s;
+    *reinterpret_cast<v4i *>(codes + e0) = quantize16(z, 0.0f, rounding, seed, offset, e0, &s);
+    if (lane == 0) scales[(size_t)(row / QB) * (C / QB) + col / QB] = (half_t)s;
+}
+
+template <int D, int NW, bool QUANT>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_fwd_kernel(AttnArgs a)
 {
     using IO = TileIO<D, NW>;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
@@ -227,13 +267,17 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(AttnArgs a)
     const float r = 1.0f / l;
     half_t *dst = a.out + ((size_t)b * a.T + query) * (a.H * D) + head * D;
 #pragma unroll
-    for (int mb = 0; mb < D / 32; ++mb) store_t(dst + 32 * mb, h, o[mb], r);
+    for (int mb = 0; mb < D / 32; ++mb) {
+        scale_t(o[mb], r);
+        store_t(dst + 32 * mb, h, o[mb]);
+        if (QUANT) quantize_t(o[mb], a.cq, a.cs, b * a.T + q0, head * D + 32 * mb, a.H * D, lane, JF_ROUND_NEAREST, 0, 0);
+    }
     if (h == 0) a.lse[(size_t)bh * a.T + query] = m * c + __builtin_amdgcn_logf(l);     // (v_log_f32: base 2)
 }
 
 // dQ by blocks of queries; leaves delta for the dK/dV kernel
-template <int D, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_dq_kernel(AttnArgs a)
+template <int D, int NW, bool QUANT>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_dq_kernel(AttnArgs a)
 {
     using IO = TileIO<D, NW>;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
@@ -303,14 +347,19 @@ __global__ __launch_bounds__(64 * NW) void attn_dq_kernel(AttnArgs a)
         }
     }
     if (!active) return;
-    half_t *dst = a.gq + ((size_t)b * a.T + query) * a.ldg + head * D;
 #pragma unroll
-    for (int mb = 0; mb < D / 32; ++mb) store_t(dst + 32 * mb, h, acc[mb], a.scale);
+    for (int mb = 0; mb < D / 32; ++mb) {
+        scale_t(acc[mb], a.scale);
+        if (QUANT)
+            quantize_t(acc[mb], a.cq, a.cs, b * a.T + q0, head * D + 32 * mb, 3 * a.H * D, lane, JF_ROUND_STOCHASTIC, a.seed, a.offset);
+        else
+            store_t(a.gq + ((size_t)b * a.T + query) * a.ldg + head * D + 32 * mb, h, acc[mb]);
+    }
 }
 
 // dK and dV by blocks of keys
-template <int D, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_dkv_kernel(AttnArgs a)
+template <int D, int NW, bool QUANT>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void attn_dkv_kernel(AttnArgs a)
 {
     using IO = TileIO<D, NW>;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
@@ -397,11 +446,22 @@ __global__ __launch_bounds__(64 * NW) void attn_dkv_kernel(AttnArgs a)
         }
     }
     if (!active) return;
+#pragma unroll
+    for (int mb = 0; mb < D / 32; ++mb) scale_t(dk[mb], a.scale);
+    if (QUANT) {
+        const int C = a.H * D;
+#pragma unroll
+        for (int mb = 0; mb < D / 32; ++mb) {
+            quantize_t(dk[mb], a.cq, a.cs, b * a.T + k0, C + head * D + 32 * mb, 3 * C, lane, JF_ROUND_STOCHASTIC, a.seed, a.offset);
+            quantize_t(dv[mb], a.cq, a.cs, b * a.T + k0, 2 * C + head * D + 32 * mb, 3 * C, lane, JF_ROUND_STOCHASTIC, a.seed, a.offset);
+        }
+        return;
+    }
     const size_t row = ((size_t)b * a.T + key) * a.ldg + head * D;
 #pragma unroll
     for (int mb = 0; mb < D / 32; ++mb) {
-        store_t(a.gk + row + 32 * mb, h, dk[mb], a.scale);
-        store_t(a.gv + row + 32 * mb, h, dv[mb], 1.0f);
+        store_t(a.gk + row + 32 * mb, h, dk[mb]);
+        store_t(a.gv + row + 32 * mb, h, dv[mb]);
     }
 }
 
@@ -423,12 +483,17 @@ static int attn_waves(int B, int H, int T)
 }
 static unsigned attn_grid(int B, int H, int T, int nw) { return 8u * ((B * H + 7) / 8) * ((T + 32 * nw - 1) / (32 * nw)); }
 
+#define JF_ATT_Q(KERN, D, NW, a, grid, st)                                                                                   \
+    do {                                                                                                                    \
+        if ((a).cq) hipLaunchKernelGGL((KERN<D, NW, true>), dim3(grid), dim3(64 * NW), 0, st, a);                           \
+        else hipLaunchKernelGGL((KERN<D, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);                                 \
+    } while (0)
 #define JF_ATT_D(KERN, D, nw, a, st)                                                                                        \
     do {                                                                                                                    \
         const unsigned grid = attn_grid((a).B, (a).H, (a).T, nw);                                                           \
-        if (nw == 4) hipLaunchKernelGGL((KERN<D, 4>), dim3(grid), dim3(256), 0, st, a);                                     \
-        else if (nw == 2) hipLaunchKernelGGL((KERN<D, 2>), dim3(grid), dim3(128), 0, st, a);                                \
-        else hipLaunchKernelGGL((KERN<D, 1>), dim3(grid), dim3(64), 0, st, a);                                              \
+        if (nw == 4) JF_ATT_Q(KERN, D, 4, a, grid, st);                                                                     \
+        else if (nw == 2) JF_ATT_Q(KERN, D, 2, a, grid, st);                                                                \
+        else JF_ATT_Q(KERN, D, 1, a, grid, st);                                                                             \
     } while (0)
 #define JF_ATT(KERN, D, nw, a, st) do { if (D == 64) JF_ATT_D(KERN, 64, nw, a, st); else JF_ATT_D(KERN, 32, nw, a, st); } while (0)
 
@@ -436,39 +501,72 @@ static unsigned attn_grid(int B, int H, int T, int nw) { return 8u * ((B * H + 7
 
 using namespace jf;
 
-extern "C" {
-
-int jf_attention_fwd(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale, void *out,
-                     float *lse, jf_stream_t stream)
+static int attention_fwd(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale, void *out, float *lse,
+                         int8_t *codes, void *scales, jf_stream_t stream)
 {
     int rc = attn_check(q, k, v, ld, B, H, T, D);
     if (rc) return rc;
     if (!out || !lse) return JF_ERR_NULL;
-    if (!aligned16(out)) return JF_ERR_ALIGN;
+    if (!aligned16(out) || !aligned16(codes)) return JF_ERR_ALIGN;
     AttnArgs a = {};
     a.q = (const half_t *)q; a.k = (const half_t *)k; a.v = (const half_t *)v; a.ld = ld;
     a.out = (half_t *)out; a.lse = lse; a.B = B; a.H = H; a.T = T; a.scale = scale;
+    a.cq = codes; a.cs = (half_t *)scales;
     const int nw = attn_waves(B, H, T);
     JF_ATT(attn_fwd_kernel, D, nw, a, (hipStream_t)stream);
     return (int)hipGetLastError();
 }
 
-int jf_attention_bwd(const void *q, const void *k, const void *v, int ld, const void *out, const void *gout, const float *lse,
-                     int B, int H, int T, int D, float scale, void *gq, void *gk, void *gv, int ldg, float *delta, jf_stream_t stream)
+static int attention_bwd(const void *q, const void *k, const void *v, int ld, const void *out, const void *gout, const float *lse, int B, int H,
+                         int T, int D, float scale, void *gq, void *gk, void *gv, int ldg, float *delta, int8_t *codes, void *scales,
+                         uint64_t seed, uint64_t offset, jf_stream_t stream)
 {
     int rc = attn_check(q, k, v, ld, B, H, T, D);
     if (rc) return rc;
-    if (!out || !gout || !lse || !gq || !gk || !gv || !delta) return JF_ERR_NULL;
-    if (ldg < H * D || ldg % 8 || (long)T * H * D >= (1L << 30)) return JF_ERR_SHAPE;
-    if (!aligned16(out) || !aligned16(gout) || !aligned16(gq) || !aligned16(gk) || !aligned16(gv)) return JF_ERR_ALIGN;
+    if (!out || !gout || !lse || !delta) return JF_ERR_NULL;
+    if ((long)T * H * D >= (1L << 30)) return JF_ERR_SHAPE;
+    if (!aligned16(out) || !aligned16(gout) || !aligned16(codes)) return JF_ERR_ALIGN;
     AttnArgs a = {};
     a.q = (const half_t *)q; a.k = (const half_t *)k; a.v = (const half_t *)v; a.ld = ld;
     a.o = (const half_t *)out; a.go = (const half_t *)gout; a.lse = const_cast<float *>(lse); a.delta = delta;
     a.gq = (half_t *)gq; a.gk = (half_t *)gk; a.gv = (half_t *)gv; a.ldg = ldg; a.B = B; a.H = H; a.T = T; a.scale = scale;
+    a.cq = codes; a.cs = (half_t *)scales; a.seed = seed; a.offset = offset;
     const int nw = attn_waves(B, H, T);
     JF_ATT(attn_dq_kernel, D, nw, a, (hipStream_t)stream);
     JF_ATT(attn_dkv_kernel, D, nw, a, (hipStream_t)stream);
     return (int)hipGetLastError();
+}
+
+extern "C" {
+
+int jf_attention_fwd(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale, void *out,
+                     float *lse, jf_stream_t stream)
+{
+    return attention_fwd(q, k, v, ld, B, H, T, D, scale, out, lse, nullptr, nullptr, stream);
+}
+
+int jf_attention_fwd_q(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale, void *out,
+                       float *lse, int8_t *codes, void *scales, jf_stream_t stream)
+{
+    if (!codes || !scales) return JF_ERR_NULL;
+    return attention_fwd(q, k, v, ld, B, H, T, D, scale, out, lse, codes, scales, stream);
+}
+
+int jf_attention_bwd(const void *q, const void *k, const void *v, int ld, const void *out, const void *gout, const float *lse,
+                     int B, int H, int T, int D, float scale, void *gq, void *gk, void *gv, int ldg, float *delta, jf_stream_t stream)
+{
+    if (!gq || !gk || !gv) return JF_ERR_NULL;
+    if (ldg < H * D || ldg % 8) return JF_ERR_SHAPE;
+    if (!aligned16(gq) || !aligned16(gk) || !aligned16(gv)) return JF_ERR_ALIGN;
+    return attention_bwd(q, k, v, ld, out, gout, lse, B, H, T, D, scale, gq, gk, gv, ldg, delta, nullptr, nullptr, 0, 0, stream);
+}
+
+int jf_attention_bwd_q(const void *q, const void *k, const void *v, int ld, const void *out, const void *gout, const float *lse,
+                       int B, int H, int T, int D, float scale, int8_t *codes, void *scales, uint64_t seed, uint64_t offset, float *delta,
+                       jf_stream_t stream)
+{
+    if (!codes || !scales) return JF_ERR_NULL;
+    return attention_bwd(q, k, v, ld, out, gout, lse, B, H, T, D, scale, nullptr, nullptr, nullptr, 0, delta, codes, scales, seed, offset, stream);
 }
 
 }  // extern "C"

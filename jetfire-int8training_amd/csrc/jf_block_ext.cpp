@@ -71,7 +71,7 @@ struct ForwardTemp {
 struct BackwardTemp {
     int8_t *qp, *qd, *qr, *qq;
     void *sp, *sd, *sr, *sq;
-    void *res, *gy, *gqkv;
+    void *res, *gy;
     float *delta, *ln1_terms, *ln2_terms;
     void *ws;
     size_t carve(uint8_t *b, const Dims &d, size_t res_bytes, size_t ws_bytes)
@@ -81,7 +81,7 @@ struct BackwardTemp {
         qd = k.take<int8_t>(d.codes(d.c)); sd = k.take(d.scales(d.c));              // at a LayerNorm's output
         qr = k.take<int8_t>(d.codes(d.c)); sr = k.take(d.scales(d.c));              // at the sum inside the block
         qq = k.take<int8_t>(d.codes(3 * d.c)); sq = k.take(d.scales(3 * d.c));      // at Q, K, V
-        res = k.take(d.m * d.c * res_bytes); gy = k.take(d.m * d.c * 2); gqkv = k.take(d.m * 3 * d.c * 2);
+        res = k.take(d.m * d.c * res_bytes); gy = k.take(d.m * d.c * 2);
         delta = k.take<float>(d.m * d.H * 4);
         ln1_terms = k.take<float>(d.m / 32 * d.c * 4); ln2_terms = k.take<float>(d.m / 32 * d.c * 4);
         ws = k.take(ws_bytes);
@@ -157,25 +157,24 @@ BlockForward forward_impl(const Dims &d, const Tensor &x, const Tensor &qx, cons
         check_rc(jf_igemm_block_q(a, codes(w[i].q), sa, w[i].s.data_ptr(), bp[i], bm[i], out, so, m, n, k, JF_B_NK, F16, RM, RM, JF_ROUND_NEAREST,
                                   0, 0, nullptr, 0, st), "projection");
     };
-    auto add = [&](const void *x1, int x1c, void *y, int yc, int8_t *q, void *s, float *mo, float *ro) {
+    auto add = [&](const void *x1, int x1c, void *y, int yc, int8_t *q, void *s) {
         check_rc(jf_add(x1, x1c, t.qo, t.so, m, c, F16, JF_ROUND_TRUNC, 0, 0, y, yc, q, s, t.rowsum, t.rowsq, st), "residual add");
-        check_rc(jf_rowstats_finish(t.rowsum, t.rowsq, m, c / QB, c, mo, ro, st), "row statistics");
     };
     check_rc(jf_layernorm_fwd(qx_, sx.data_ptr(), g1, nullptr, mu, rs, m, c, F16, v.qn, v.sn, st), "layernorm");
     check_rc(jf_igemm_block_q_dequant(v.qn, codes(w[0].q), v.sn, w[0].s.data_ptr(), bp[0], bm[0], v.qkv, m, 3 * c, c, JF_B_NK, F16, RM, RM, JF_FP_F16,
                                       JF_ROUND_NEAREST, 0, 0, st), "qkv projection");
     c10::Half *qkv = (c10::Half *)v.qkv;
-    check_rc(jf_attention_fwd(qkv, qkv + c, qkv + 2 * c, 3 * c, d.B, d.H, d.T, c / d.H, (float)(1.0 / std::sqrt((double)(c / d.H))), v.y, v.lse, st),
+    check_rc(jf_attention_fwd_q(qkv, qkv + c, qkv + 2 * c, 3 * c, d.B, d.H, d.T, c / d.H, (float)(1.0 / std::sqrt((double)(c / d.H))), v.y, v.lse,
+                                v.qy, v.sy, st),
              "attention");
-    check_rc(jf_quantize(v.y, JF_FP_F16, m, c, v.qy, v.sy, nullptr, F16, JF_ROUND_NEAREST, 0, 0, 0.0f, st), "quantize");
     gemm_q(v.qy, v.sy, 1, c, c, t.qo, t.so);
-    add(x.data_ptr(), xc, t.mid, JF_FP_F32, v.q2, v.s2, v.mean2, v.rstd2);
-    check_rc(jf_layernorm_fwd(v.q2, v.s2, g2, nullptr, v.mean2, v.rstd2, m, c, F16, v.qn2, v.sn2, st), "layernorm");
+    add(x.data_ptr(), xc, t.mid, JF_FP_F32, v.q2, v.s2);
+    check_rc(jf_layernorm_fwd_sums(v.q2, v.s2, g2, nullptr, t.rowsum, t.rowsq, m, c, F16, v.mean2, v.rstd2, v.qn2, v.sn2, st), "layernorm");
     check_rc(jf_igemm_block_q_gelu(v.qn2, codes(w[2].q), v.sn2, w[2].s.data_ptr(), bp[2], bm[2], v.qh, v.sh, v.qa, v.sa, m, 4 * c, c, F16, RM, RM,
                                    JF_GELU_ERF, 5e-5f, st), "fc");
     gemm_q(v.qa, v.sa, 3, c, 4 * c, t.qo, t.so);
-    add(t.mid, JF_FP_F32, r.fp.data_ptr(), fp_of(r.fp, "out"), (int8_t *)r.q.data_ptr(), r.s.data_ptr(), r.mean.data_ptr<float>(),
-        r.rstd.data_ptr<float>());
+    add(t.mid, JF_FP_F32, r.fp.data_ptr(), fp_of(r.fp, "out"), (int8_t *)r.q.data_ptr(), r.s.data_ptr());
+    check_rc(jf_rowstats_finish(t.rowsum, t.rowsq, m, c / QB, c, r.mean.data_ptr<float>(), r.rstd.data_ptr<float>(), st), "row statistics");
     return r;
 }
 
@@ -293,10 +292,9 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         check_rc(jf_igemm_block_q_dequant(t.qr, codes(w[1].q), t.sr, w[1].s.data_ptr(), nullptr, nullptr, t.gy, m, c, c, JF_B_KN, F16, RM, KM, JF_FP_F16,
                                           SR, z[5].seed, z[5].offset, st), "gradient of the attention's projection");
         wgrad(1, t.qr, t.sr, v.qy, v.sy);
-        c10::Half *qkv = (c10::Half *)v.qkv, *gqkv = (c10::Half *)t.gqkv;
-        check_rc(jf_attention_bwd(qkv, qkv + c, qkv + 2 * c, 3 * c, v.y, t.gy, v.lse, d.B, d.H, d.T, c / d.H, (float)(1.0 / std::sqrt((double)(c / d.H))),
-                                  gqkv, gqkv + c, gqkv + 2 * c, 3 * c, t.delta, st), "gradient of attention");
-        check_rc(jf_quantize(gqkv, JF_FP_F16, m, 3 * c, t.qq, t.sq, nullptr, F16, SR, z[6].seed, z[6].offset, 0.0f, st), "quantize");
+        const c10::Half *qkv = (const c10::Half *)v.qkv;
+        check_rc(jf_attention_bwd_q(qkv, qkv + c, qkv + 2 * c, 3 * c, v.y, t.gy, v.lse, d.B, d.H, d.T, c / d.H, (float)(1.0 / std::sqrt((double)(c / d.H))),
+                                    t.qq, t.sq, z[6].seed, z[6].offset, t.delta, st), "gradient of attention");
         check_rc(jf_igemm_block_q(t.qq, codes(w[0].q), t.sq, w[0].s.data_ptr(), nullptr, nullptr, t.qd, t.sd, m, c, 3 * c, JF_B_KN, F16, RM, KM, SR,
                                   z[7].seed, z[7].offset, nullptr, 0, st), "gradient of qkv");
         wgrad(0, t.qq, t.sq, v.qn, v.sn);

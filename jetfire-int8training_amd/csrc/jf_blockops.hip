@@ -449,11 +449,18 @@ void gelu_bwd_kernel(const int8_t *qx, const ST *sx, const int8_t *qg, const ST 
 // is done, or pinning the requests above the arithmetic (the compiler moves those of the later blocks behind the first
 // block's), changes nothing; what counts is how evenly the waves fill the SIMDs: 9.1 us with 2 row blocks per wave (6.5
 // waves per SIMD), 10.0 us with 4 (3.25: a quarter of the SIMDs get a fourth wave), 11.6 us with 8.
+// STATS: mean and rstd are not given but follow from a residual add's partial row sums (rowsum, rowsq: [C/32][R]), added here
+// in the order of rowstats_finish_kernel and written by the workgroups of the first column blocks.  Every workgroup adds its
+// own 64 rows' sums again, 2 C/32 floats per row out of the L2: less than the launch of its own that this takes the place of.
 constexpr int CW_ROWS = 2;
-template <typename ST>
+struct RowSums {
+    const float *rowsum, *rowsq;
+    float *mean, *rstd;
+};
+template <typename ST, bool STATS>
 __global__ __launch_bounds__(NT) void layernorm_fwd_kernel(const int8_t *q, const ST *s, const float *gamma,
                                                            const float *beta, const float *mean, const float *rstd,
-                                                           int R, int C, int8_t *qy, ST *sy)
+                                                           int R, int C, int8_t *qy, ST *sy, RowSums rsum)
 {
     __shared__ __attribute__((aligned(16))) unsigned char line_patches[2 * QB * LINE_PITCH];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -481,8 +488,29 @@ __global__ __launch_bounds__(NT) void layernorm_fwd_kernel(const int8_t *q, cons
         const int row = rb * QB + (lane >> 1);
         c[k] = *reinterpret_cast<const v4i *>(q + (size_t)row * C + col);
         sc[k] = load_scale(s, rb * SC + cb);
-        mu[k] = mean[row];
-        rs[k] = rstd[row];
+        if (!STATS) { mu[k] = mean[row]; rs[k] = rstd[row]; }
+    }
+    if constexpr (STATS) {
+        __shared__ float stat[2][CW_ROWS * QB];
+        const int r = threadIdx.x & (CW_ROWS * QB - 1), which = threadIdx.x / (CW_ROWS * QB);     // two waves: 0 = sums, 1 = squares
+        const int row = grp * CW_ROWS * QB + r;
+        float acc = 0.0f;
+        if (which < 2) {
+            const float *src = (which ? rsum.rowsq : rsum.rowsum) + (row < R ? row : R - 1);
+#pragma unroll 16
+            for (int j = 0; j < SC; ++j) acc = acc + src[(size_t)j * R];
+            stat[which][r] = acc;
+        }
+        __syncthreads();
+        if (which == 0) {
+            const float n = (float)C, m = acc / n, var = stat[1][r] / n - m * m, rv = 1.0f / __builtin_sqrtf(var);
+            stat[0][r] = m;                                        // (each thread reads and writes its own row)
+            stat[1][r] = rv;
+            if (cg == 0 && row < R) { rsum.mean[row] = m; rsum.rstd[row] = rv; }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < CW_ROWS; ++k) { mu[k] = stat[0][k * QB + (lane >> 1)]; rs[k] = stat[1][k * QB + (lane >> 1)]; }
     }
     v4i out[CW_ROWS];
     float so[CW_ROWS];
@@ -1316,8 +1344,10 @@ int jf_rowstats(const int8_t *q, const void *s, int R, int C, int scale_dtype, f
     JF_LAUNCH(rowstats_kernel<float>, R / QB, smem, st, q, (const float *)s, R, C, eps, mean, rstd);
 }
 
-int jf_layernorm_fwd(const int8_t *q, const void *s, const float *gamma, const float *beta, const float *mean,
-                     const float *rstd, int R, int C, int scale_dtype, int8_t *qy, void *sy, jf_stream_t stream)
+}  // extern "C"
+
+static int layernorm_fwd(const int8_t *q, const void *s, const float *gamma, const float *beta, const float *mean, const float *rstd, int R, int C,
+                         int scale_dtype, int8_t *qy, void *sy, const RowSums *sums, jf_stream_t stream)
 {
     int rc = check_block_tensor(q, s, R, C, scale_dtype);
     if (rc) return rc;
@@ -1325,12 +1355,28 @@ int jf_layernorm_fwd(const int8_t *q, const void *s, const float *gamma, const f
     if (!aligned16(qy) || !aligned16(gamma) || (beta && !aligned16(beta))) return JF_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
     const int grid = ((C / QB + WPB - 1) / WPB) * ((R / QB + CW_ROWS - 1) / CW_ROWS);
-    const size_t smem = 0;
-    if (scale_dtype == JF_SCALE_F16)
-        JF_LAUNCH(layernorm_fwd_kernel<half_t>, grid, smem, st, q, (const half_t *)s, gamma, beta, mean, rstd, R, C, qy,
-                  (half_t *)sy);
-    JF_LAUNCH(layernorm_fwd_kernel<float>, grid, smem, st, q, (const float *)s, gamma, beta, mean, rstd, R, C, qy,
-              (float *)sy);
+    const RowSums rs = sums ? *sums : RowSums{};
+#define JF_LNF(ST, STATS) JF_LAUNCH((layernorm_fwd_kernel<ST, STATS>), grid, 0, st, q, (const ST *)s, gamma, beta, mean, rstd, R, C, qy, (ST *)sy, rs)
+    if (scale_dtype == JF_SCALE_F16) { if (sums) JF_LNF(half_t, true); JF_LNF(half_t, false); }
+    if (sums) JF_LNF(float, true);
+    JF_LNF(float, false);
+#undef JF_LNF
+}
+
+extern "C" {
+
+int jf_layernorm_fwd(const int8_t *q, const void *s, const float *gamma, const float *beta, const float *mean,
+                     const float *rstd, int R, int C, int scale_dtype, int8_t *qy, void *sy, jf_stream_t stream)
+{
+    return layernorm_fwd(q, s, gamma, beta, mean, rstd, R, C, scale_dtype, qy, sy, nullptr, stream);
+}
+
+int jf_layernorm_fwd_sums(const int8_t *q, const void *s, const float *gamma, const float *beta, const float *rowsum, const float *rowsq,
+                          int R, int C, int scale_dtype, float *mean, float *rstd, int8_t *qy, void *sy, jf_stream_t stream)
+{
+    if (!rowsum || !rowsq) return JF_ERR_NULL;
+    const RowSums sums = {rowsum, rowsq, mean, rstd};
+    return layernorm_fwd(q, s, gamma, beta, mean, rstd, R, C, scale_dtype, qy, sy, &sums, stream);
 }
 
 // workspace: per-row block partials [2][C/32][R] and per-row-group column partials [2][C][groups]

@@ -478,17 +478,22 @@ std::tuple<Tensor, Tensor> attention_fwd(const Tensor &q, const Tensor &k, const
     return std::make_tuple(out, lse);
 }
 
-// the gradients side by side, [B*T, 3C]
-Tensor attention_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &out, const Tensor &lse, const Tensor &gout,
-                     int64_t batch, int64_t heads)
+void attention_gradient_operands(const Tensor &q, const Tensor &out, const Tensor &lse, const Tensor &gout, const AttentionOperands &a)
 {
-    const AttentionOperands a = attention_operands(q, k, v, batch, heads);
     for (const Tensor *t : {&out, &gout}) {
         need(*t, "attention: out / its gradient", 2);
         TORCH_CHECK(t->scalar_type() == torch::kFloat16 && t->sizes() == q.sizes() && t->device() == q.device(),
                     "attention: out and its gradient must be float16 tensors of the shape of q");
     }
-    vec(lse.reshape({-1}), q.size(0) * a.H, q, "lse");
+    vec(lse, q.size(0) * a.H, q, "lse");
+}
+
+// the gradients side by side, [B*T, 3C]
+Tensor attention_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &out, const Tensor &lse, const Tensor &gout,
+                     int64_t batch, int64_t heads)
+{
+    const AttentionOperands a = attention_operands(q, k, v, batch, heads);
+    attention_gradient_operands(q, out, lse, gout, a);
     c10::DeviceGuard guard(q.device());
     Tensor g = torch::empty({q.size(0), 3 * a.C}, q.options()), delta = torch::empty_like(lse);
     c10::Half *gp = g.data_ptr<c10::Half>();
@@ -497,6 +502,40 @@ Tensor attention_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Te
                               a.H, a.T, a.D, a.scale, gp, gp + a.C, gp + 2 * a.C, (int)(3 * a.C), delta.data_ptr<float>(), current_stream(q)),
              "attention_bwd");
     return g;
+}
+
+// attention_fwd with the block quantisation of its result: (out, lse, codes, scales)
+std::tuple<Tensor, Tensor, Tensor, Tensor> attention_fwd_q(const Tensor &q, const Tensor &k, const Tensor &v, int64_t batch, int64_t heads)
+{
+    const AttentionOperands a = attention_operands(q, k, v, batch, heads);
+    c10::DeviceGuard guard(q.device());
+    const int64_t M = q.size(0);
+    Tensor out = torch::empty({M, a.C}, q.options()), lse = torch::empty({(int64_t)a.B * a.H, a.T}, q.options().dtype(torch::kFloat32));
+    Tensor codes = torch::empty({M, a.C}, q.options().dtype(torch::kInt8)), scales = torch::empty({M / QB, a.C / QB}, q.options());
+    pybind11::gil_scoped_release nogil;
+    check_rc(jf_attention_fwd_q(q.data_ptr(), k.data_ptr(), v.data_ptr(), a.ld, a.B, a.H, a.T, a.D, a.scale, out.data_ptr(), lse.data_ptr<float>(),
+                                (int8_t *)codes.data_ptr(), scales.data_ptr(), current_stream(q)),
+             "attention_fwd_q");
+    return std::make_tuple(out, lse, codes, scales);
+}
+
+// attention_bwd with the gradients quantised: (codes, scales)
+std::tuple<Tensor, Tensor> attention_bwd_q(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &out, const Tensor &lse,
+                                           const Tensor &gout, int64_t batch, int64_t heads, OptU64 seed, OptU64 offset)
+{
+    const AttentionOperands a = attention_operands(q, k, v, batch, heads);
+    attention_gradient_operands(q, out, lse, gout, a);
+    c10::DeviceGuard guard(q.device());
+    const int64_t M = q.size(0);
+    Tensor codes = torch::empty({M, 3 * a.C}, q.options().dtype(torch::kInt8)), scales = torch::empty({M / QB, 3 * a.C / QB}, q.options());
+    Tensor delta = torch::empty_like(lse);
+    const auto so = rng(JF_ROUND_STOCHASTIC, q, 3 * M * a.C, seed, offset);
+    pybind11::gil_scoped_release nogil;
+    check_rc(jf_attention_bwd_q(q.data_ptr(), k.data_ptr(), v.data_ptr(), a.ld, out.data_ptr(), gout.data_ptr(), lse.data_ptr<float>(), a.B, a.H, a.T,
+                                a.D, a.scale, (int8_t *)codes.data_ptr(), scales.data_ptr(), so.first, so.second, delta.data_ptr<float>(),
+                                current_stream(q)),
+             "attention_bwd_q");
+    return std::make_tuple(codes, scales);
 }
 
 // ---- column sums (bias gradient; QBlockLinear.py:63-66) -------------------------------------------------------------
@@ -843,6 +882,10 @@ void register_jetfire_ops(pybind11::module &m)
           "(out [tokens, C], lse [batch*heads, T]) of causal self-attention; heads 32 or 64 wide");
     m.def("attention_bwd", &attention_bwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("out"), py::arg("lse"), py::arg("gout"),
           py::arg("batch"), py::arg("heads"), "gradients of q, k, v side by side, [tokens, 3C]");
+    m.def("attention_fwd_q", &attention_fwd_q, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("batch"), py::arg("heads"),
+          "attention_fwd and the block quantisation of its result: (out, lse, codes, scales)");
+    m.def("attention_bwd_q", &attention_bwd_q, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("out"), py::arg("lse"), py::arg("gout"),
+          py::arg("batch"), py::arg("heads"), py::arg("seed") = none, py::arg("offset") = none, "(codes, scales) of attention_bwd's result, rounded stochastically");
     m.def("block_colsum", &block_colsum, py::arg("q"), py::arg("s"), "fp32 column sums of a block tensor (bias gradient)");
     m.def("linear_forward", &linear_forward, py::arg("x"), py::arg("sx"), py::arg("w"), py::arg("sw"), py::arg("quantized"),
           py::arg("bias") = none, py::arg("biasmax") = none);

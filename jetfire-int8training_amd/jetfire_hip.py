@@ -31,6 +31,7 @@ EXPORTS = [
     "jf_layernorm_bwd_workspace_bytes", "jf_layernorm_bwd", "jf_layernorm_bwd_add", "jf_layernorm_bwd_add_strips", "jf_gelu_fwd", "jf_gelu_bwd", "jf_add", "jf_rowstats_finish",
     "jf_igemm_block_q_dequant", "jf_quantize_slabs", "jf_philox_rounds", "jf_block_colsum", "jf_block_colsum_workspace_bytes",
     "jf_attention_fwd", "jf_attention_bwd", "jf_quantize_many", "jf_rowstats_fp", "jf_wgrad_many", "jf_wgrad_many_workspace_bytes",
+    "jf_layernorm_fwd_sums", "jf_attention_fwd_q", "jf_attention_bwd_q",
 ]
 
 _lib = None
@@ -54,6 +55,7 @@ def lib():
         L.jf_igemm_block_fp_noalloc.argtypes = [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _p]
         L.jf_wgrad_many_workspace_bytes.argtypes = [_i, _p, _p, _i]
         L.jf_wgrad_many_workspace_bytes.restype = _sz
+        L.jf_layernorm_fwd_sums.argtypes = [_p, _p, _p, _p, _p, _p, _i, _i, _i, _p, _p, _p, _p, _p]
         L.jf_wgrad_many.argtypes = [_i, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _p, _p, _sz, _p]
         L.jf_igemm_block_q_gelu_bwd.argtypes = [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _u64, _u64, _i, _u64, _u64, _p]
         L.jf_igemm_block_q_dequant.argtypes = [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _u64, _u64, _p]
@@ -609,6 +611,22 @@ def block_colsum(q, s):
     out = torch.empty(Cc, dtype=torch.float32, device=q.device)
     check(lib().jf_block_colsum(_ptr(q), _ptr(s), R, Cc, code, _ptr(out), _ptr(ws), nbytes, _stream()))
     return out
+
+
+def layernorm_fwd_sums(q, s, gamma, beta, rowsum, rowsq):
+    """rowstats_finish and layernorm_fwd as one kernel: (qy, sy, mean, rstd)."""
+    R, Cc, code = _block_tensor(q, s, "x")
+    for t, n, name in ((gamma, Cc, "gamma"), (beta, Cc, "beta"), (rowsum, Cc // QB * R, "rowsum"), (rowsq, Cc // QB * R, "rowsq")):
+        if t is not None:
+            _need(t, torch.float32, name, None)
+            if t.numel() != n:
+                raise RuntimeError(f"{name} must have {n} elements")
+    qy, sy = torch.empty_like(q), torch.empty_like(s)
+    mean = torch.empty(R, dtype=torch.float32, device=q.device)
+    rstd = torch.empty_like(mean)
+    check(lib().jf_layernorm_fwd_sums(_ptr(q), _ptr(s), _ptr(gamma), _ptr(beta), _ptr(rowsum), _ptr(rowsq), R, Cc, code, _ptr(mean), _ptr(rstd),
+                                      _ptr(qy), _ptr(sy), _stream()))
+    return qy, sy, mean, rstd
 
 
 def rowstats_finish(rowsum, rowsq, n_cols):

@@ -44,3 +44,11 @@ def test_causal_attention(B, H, T, D, scale):
         jf.attention_fwd(q, k, v.float(), B, H)
     with pytest.raises(RuntimeError):
         jf.attention_fwd(q[: 16 * B], k[: 16 * B], v[: 16 * B], B, H)          # rows that are not whole blocks
+    # the same with the block quantisation inside: what quantising the stored tensors gives
+    out3, lse3, qo, so = jf.attention_fwd_q(q, k, v, B, H)
+    assert torch.equal(out, out3) and torch.equal(lse, lse3)
+    wq, ws, _ = jf.quantize(out, jf.ROUND_NEAREST)
+    assert torch.equal(qo, wq) and torch.equal(so, ws)
+    qg, sg = jf.attention_bwd_q(q, k, v, out, lse, g, B, H, 3, 40)
+    wq, ws, _ = jf.quantize(grads, jf.ROUND_STOCHASTIC, torch.float16, False, 0.0, 3, 40)
+    assert torch.equal(qg, wq) and torch.equal(sg, ws)

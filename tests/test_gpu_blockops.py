@@ -428,3 +428,20 @@ def test_gelu_fwd_on_one_sided_and_degenerate_blocks(jf, oracle, approx, eps, f1
     wq, ws = oracle.gelu_fwd(q, s, approx, eps, scale_dtype="f16" if f16 else "f32")
     same(sy, ws, "scales")
     same(qy, wq, "codes")
+
+
+@pytest.mark.parametrize("R,C", [(32, 32), (64, 96), (96, 512), (160, 544), (64, 2080)])    # whole and half groups of rows, full and partial groups of columns
+@pytest.mark.parametrize("f16,with_beta", [(True, False), (False, True)])
+def test_layernorm_from_partial_row_sums(jf, oracle, R, C, f16, with_beta):
+    """jf_layernorm_fwd_sums against the two kernels it stands for."""
+    print(f"case R={R} C={C} f16={f16}", flush=True)
+    rng = np.random.default_rng(R + C)
+    x1 = dev(rng.standard_normal((R, C)).astype(np.float32) * 3)
+    q2, s2 = block_tensor(oracle, rng, R, C, 0.5)
+    gamma = dev((1 + 0.1 * rng.standard_normal(C)).astype(np.float32))
+    beta = dev(rng.standard_normal(C).astype(np.float32)) if with_beta else None
+    y, q, s, rs, rq = jf.add(x1, dev(q2), dev(s2).to(torch.float16 if f16 else torch.float32), with_stats=True)
+    mean, rstd = jf.rowstats_finish(rs, rq, C)
+    want = jf.layernorm_fwd(q, s, gamma, beta, mean, rstd) + (mean, rstd)
+    for a, b in zip(jf.layernorm_fwd_sums(q, s, gamma, beta, rs, rq), want):
+        assert torch.equal(a, b)
