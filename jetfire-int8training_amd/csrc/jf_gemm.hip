@@ -107,6 +107,8 @@ __device__ __forceinline__ void tile_at(int logical, int tiles_m, int tiles_n, b
 // WGM x WGN waves, each owning WBM x WBN quantisation blocks (WBM = 2: 64x32 elements; WBM = 1: one block, for launches whose
 // 128x128 tiles would leave most of the chip idle, see launch_gemm).
 constexpr int WBN = 1;
+// threads of a workgroup: with one block per wave, as many waves again that do nothing but load (see load_loop)
+constexpr int gemm_threads(int WBM, int WGM, int WGN) { return 64 * WGM * WGN * (WBM == 1 ? 2 : 1); }
 // NSTAGE = depth of the LDS ring (one stage being computed, NSTAGE-1 in flight); WGPC = workgroups per CU
 // (the second launch bound counts waves per SIMD: WGPC workgroups of WGM*WGN waves over 4 SIMDs).
 // AKM = 1: A is [K, lda] (M-contiguous rows), staged and read like a [K,N] B operand (below).
@@ -139,6 +141,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     static_assert(GROUPS % NW == 0, "stage must split evenly over the waves");
     static_assert(NSTAGE >= 2 && NSTAGE <= 5, "ring depth");
     static_assert(!BKN || (BN == ROW_BYTES && WBN == 1), "a staged [K,N] row is one 128-byte LDS row");
+    static_assert(WBM == 2 || !AKM, "one block per wave: A as [M,K] only");
     static_assert(!AKM || BM == ROW_BYTES, "a staged [K,M] row is one 128-byte LDS row");
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -146,7 +149,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool loader = WBM == 1 && wave_id >= NW;            // a wave that fetches for the others
+    const int wave = WBM == 1 ? wave_id % NW : wave_id;
     const int wm = wave % WGM, wn = wave / WGM;
 
     int tile_m, tile_n, split;
@@ -231,9 +236,18 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         s_last = (unsigned)((nkb - 1 + kb_base) * ks + i * is) * (unsigned)sizeof(ST);
         s_step = (unsigned)(KB_STAGE * ks) * (unsigned)sizeof(ST);
     }
+    // WBM = 1: all of a block's products at once, before the main loop, into a table of the wave: lane l those of the K blocks l,
+    // l + 64, ...
+    constexpr bool TABLE = WBM == 1;
+    float *const table = reinterpret_cast<float *>(smem + NSTAGE * STAGE_BYTES) + wave * ((nkb + KB_STAGE - 1) / KB_STAGE * KB_STAGE + KB_STAGE);
+    auto make_table = [&] {
+        const int mi = m0 / QB + wm < SM ? m0 / QB + wm : SM - 1, ni = n0 / QB + wn < SN ? n0 / QB + wn : SN - 1;
+        const ST *ta = reinterpret_cast<const ST *>(p.sa) + (size_t)mi * p.sa_is, *tb = reinterpret_cast<const ST *>(p.sb) + (size_t)ni * p.sb_is;
+        for (int k = lane; k < nkb; k += WAVE) table[k] = ((float)ta[(size_t)k * p.sa_ks] * (float)tb[(size_t)k * p.sb_ks]) * 67108864.0f;
+    };
     // the scales of the next stage (one after the other) into ring slot `slot`; K blocks beyond the last: the last one again
     auto issue_scales = [&](auto slot_c) {
-        if (EPI == EPI_S32) return;
+        if (EPI == EPI_S32 || TABLE) return;
         const unsigned char *const src = s_base + (s_off < s_last ? s_off : s_last);
         const unsigned dst = (unsigned)(uintptr_t)(lds_u8 *)scale_patch + decltype(slot_c)::value * SC_SLOT;
         // a binary16 scale is fetched with the 16-bit form (zero-extended into the lane's LDS word): exactly the
@@ -269,10 +283,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     constexpr int A_LOADS = (BM / 8) / NW;                    // loads 0 .. A_LOADS-1 of a wave fetch A rows, the rest B rows
     static_assert((BM / 8) % NW == 0, "a load instruction fetches rows of one operand");
     // FULL: the stage has all KB_STAGE K blocks (every stage but a short last one)
-    auto issue_stage_as = [&](int stage, auto slot_c, auto full_c) {
+    auto issue_stage_as = [&](int stage, unsigned slot, auto full_c) {       // slot: stage % NSTAGE
         constexpr bool FULL = decltype(full_c)::value;
-        constexpr int SLOT = decltype(slot_c)::value;         // stage % NSTAGE
-        const unsigned slot_lds = (unsigned)(uintptr_t)(lds_u8 *)smem + (unsigned)SLOT * STAGE_BYTES;
+        const unsigned slot_lds = (unsigned)(uintptr_t)(lds_u8 *)smem + slot * STAGE_BYTES;
         const int kb0 = stage * KB_STAGE;
         // asm: scalar base + 32-bit lane offset is the addressing mode that costs no vector instruction, and the
         // compiler does not choose it by itself here.  M0 holds the LDS destination of an LDS-direct load.
@@ -302,9 +315,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                          ::"v"(j < A_LOADS ? la : lb), "s"(base), "s"(slot_lds + (unsigned)grp * 1024u) : "memory", "m0");
         }
     };
-    auto issue_stage = [&](int stage, auto slot_c) {          // stage < nstages, one after the other
-        if (stage < nkb / KB_STAGE) issue_stage_as(stage, slot_c, std::true_type{});
-        else issue_stage_as(stage, slot_c, std::false_type{});
+    auto issue_stage = [&](int stage, unsigned slot) {        // stage < nstages, one after the other
+        if (stage < nkb / KB_STAGE) issue_stage_as(stage, slot, std::true_type{});
+        else issue_stage_as(stage, slot, std::false_type{});
     };
 
     // ---- operand fetch addresses ----------------------------------------------------------------
@@ -366,14 +379,14 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     // of stage s has been read.  Operand fragments and scales of K block k+1 are read from LDS into a second set
     // of registers BEFORE the products of K block k are issued, so the LDS pipe works while the wave multiplies
     // and accumulates; without this all waves of a SIMD queue at the LDS together and then compute together.
-    constexpr int LOADS = LPW + (EPI != EPI_S32 ? 1 : 0);     // LDS-direct loads per wave and stage
+    constexpr int LOADS = LPW + (EPI != EPI_S32 && !TABLE ? 1 : 0);     // LDS-direct loads per wave and stage
     const int nfull = nkb / KB_STAGE;                         // stages with all KB_STAGE blocks
     const int ktail = nkb - nfull * KB_STAGE;                 // K blocks of the short last stage (0: none)
     issue_scales(std::integral_constant<int, 0>{});
     static_for<0, NSTAGE>([&](auto slot_c) {
         constexpr int SLOT = decltype(slot_c)::value;
-        if (SLOT < nstages) {
-            issue_stage(SLOT, slot_c);
+        if (SLOT < nstages && (!TABLE || loader)) {
+            issue_stage(SLOT, (unsigned)SLOT);
             // (ring slot 0 holds the first stage's scales until they are read, below)
             if (SLOT + 1 < NSTAGE) issue_scales(std::integral_constant<int, (SLOT + 1) % NSTAGE>{});
         }
@@ -451,20 +464,31 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     // before the vector ALU can read it.  So the accumulation lags the products by one: product n is issued, THEN
     // product n-1 (long finished) is converted and accumulated.  (d_pend, sab_pend) carry the lagging product across
     // K blocks and stages; the first accumulation adds 0*0 and the last product is accumulated after the loop.
-    constexpr int C_MAGIC = 0x3e22f983;                        // accumulator input of the MFMAs (file header)
     v16i d_pend = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     float sab_pend = 0.0f;
     auto accumulate = [&](auto blk_c) {
         constexpr int i = decltype(blk_c)::value / WBN, j = decltype(blk_c)::value % WBN;
         float t[16];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) t[v] = __int_as_float(d_pend[v]) - __int_as_float(C_MAGIC);   // = d * 2^-26, exactly
+        for (int v = 0; v < 16; ++v)                          // = d * 2^-26, exactly (asm: the compiler adds a 32-bit literal, twice the code bytes)
+            asm("v_subrev_f32_e32 %0, 0.15915494, %1" : "=v"(t[v]) : "v"(d_pend[v]));
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_fmaf(sab_pend, t[v], acc[i][j][v]);
         // pin the accumulation here: the optimiser would otherwise postpone it past the next K blocks and keep their
         // products alive in registers it does not have
 #pragma unroll
         for (int v = 0; v < 16; ++v) asm volatile("" : "+v"(acc[i][j][v]));
+    };
+    // the same of one block with everything as arguments
+    auto compute_block = [&](const v4i &fa, const v4i &fb, const float sab_new) {
+        v16i d_new;
+        asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0x3e22f983" : "=&v"(d_new) : "v"(fa), "v"(fb));
+        __builtin_amdgcn_sched_barrier(0);
+        accumulate(std::integral_constant<int, 0>{});
+        // (a copy of its own, made here: the register the product was read into is the target of the next read by the time it is used)
+        asm volatile("v_mov_b32_e32 %0, %1" : "=v"(sab_pend) : "v"(sab_new));
+        __builtin_amdgcn_sched_barrier(0);
+        d_pend = d_new;
     };
     auto compute = [&](auto cur_c, const int kbg) {
         constexpr int CUR = decltype(cur_c)::value;
@@ -500,12 +524,17 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         else JF_WAIT_VMCNT(Y * LOADS);
     };
     using c0 = std::integral_constant<int, 0>;
-    if (NSTAGE - 1 >= nstages) JF_WAIT_VMCNT(0);
-    else JF_WAIT_VMCNT((NSTAGE - 1) * LOADS - (EPI != EPI_S32 ? 1 : 0));      // stage 0 and the scales of stage 1 have landed
-    read_scales(c0{});
-    __builtin_amdgcn_s_waitcnt(0xC07F);                        // lgkmcnt(0) only
-    put_products(c0{});
-    if (NSTAGE - 1 < nstages) issue_scales(c0{});              // stage NSTAGE, behind the operands of stage NSTAGE - 1
+    if constexpr (TABLE) {
+        if (loader) wait_stage(NSTAGE - 1, std::integral_constant<int, NSTAGE - 1>{});    // stage 0 has landed
+        else make_table();
+    } else {
+        if (NSTAGE - 1 >= nstages) JF_WAIT_VMCNT(0);
+        else JF_WAIT_VMCNT((NSTAGE - 1) * LOADS - (EPI != EPI_S32 ? 1 : 0));      // stage 0 and the scales of stage 1 have landed
+        read_scales(c0{});
+        __builtin_amdgcn_s_waitcnt(0xC07F);                    // lgkmcnt(0) only
+        put_products(c0{});
+        if (NSTAGE - 1 < nstages) issue_scales(c0{});          // stage NSTAGE, behind the operands of stage NSTAGE - 1
+    }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();                              // bare: __syncthreads() would drain every load
     asm volatile("" ::: "memory");
@@ -542,7 +571,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
                     if (s + NSTAGE < nstages) {
-                        issue_stage(s + NSTAGE, slot_c);
+                        issue_stage(s + NSTAGE, (unsigned)SLOT);
                         issue_scales(std::integral_constant<int, NEXT_SLOT>{});      // of stage s + NSTAGE + 1
                     }
                 }
@@ -592,12 +621,121 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         });
     }
     };
-    if (!wave_active) main_loop(std::false_type{}, std::integral_constant<int, PACE_HARDWARE>{});
+    // WBM = 1.  A wave that multiplies is (nearly) alone on its SIMD, so what counts is the length of its own chain: a vector
+    // instruction takes 4.1 cycles there, an LDS read 15, an LDS-direct load 25 to 64 (four waves that load at once wait for each
+    // other) and a branch 27 to 120, all of it in sequence.  So the loads are left to four waves of their own, the products of the
+    // scales come from a table, operands are read two K blocks at a time, two ahead, and a turn of the ring has no branch.
+    // 228 cycles per K block, and per launch, us, before | after: 32x768x768 6.6 | 5.7, 512x768x3072 17.7 | 12.8, 1248x768x3072
+    // 17.9 | 13.0, 2048x768x768 8.4 | 7.6.
+    auto load_loop = [&] {
+        unsigned slot = 0;
+        auto hand_over = [&](int s, auto steady_c) {
+            // stage s + 1 has landed; behind the barrier every wave holds all of stage s in registers: its slot may be overwritten
+            if constexpr (decltype(steady_c)::value) JF_WAIT_VMCNT((NSTAGE - 2) * LOADS);
+            else wait_stage(s + NSTAGE - 1, std::integral_constant<int, NSTAGE - 2>{});
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if constexpr (decltype(steady_c)::value) issue_stage_as(s + NSTAGE, slot, std::true_type{});
+            else if (s + NSTAGE < nstages) issue_stage(s + NSTAGE, slot);
+            slot = slot + 1 == NSTAGE ? 0 : slot + 1;
+        };
+        int s = 0;
+        for (; s + NSTAGE < nfull; ++s) hand_over(s, std::true_type{});
+        for (; s + 1 < nstages; ++s) hand_over(s, std::false_type{});
+    };
+    auto table_loop = [&] {
+        typedef float v2f __attribute__((ext_vector_type(2)));
+        v4i fa2[2][2], fb2[2][2];
+        v2f pr[2];
+        const std::integral_constant<int, 0> p0;
+        const std::integral_constant<int, 1> p1;
+        if (!wave_active) {
+            for (int s = 0; s + 1 < nstages; ++s) __builtin_amdgcn_s_barrier();
+            return;
+        }
+        unsigned tab;                                           // products of the stage in ring slot 0
+        {
+            const unsigned u = (unsigned)(uintptr_t)(lds_u8 *)reinterpret_cast<unsigned char *>(table);
+            asm volatile("v_mov_b32 %0, %1" : "=v"(tab) : "s"(u));
+        }
+        // K blocks 2 pair, 2 pair + 1 of a stage into register set `pair`; extra: run-time offsets of operands and products
+        auto fetch_pair = [&](auto pair_c, auto slot_c, unsigned extra, unsigned extra_tab) {
+            constexpr int PAIR = decltype(pair_c)::value, SLOT = decltype(slot_c)::value, SB = SLOT * STAGE_BYTES;
+            static_assert(NSTAGE * STAGE_BYTES <= 65536, "offsets of 16 bits");
+            v2f &t = pr[PAIR];
+            const unsigned pt = tab + extra_tab;
+            asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(t) : "v"(pt), "n"(SLOT * KB_STAGE * 4 + 8 * PAIR));
+            static_for<0, 2>([&](auto i_c) {
+                constexpr int I = decltype(i_c)::value, kb = 2 * PAIR + I;
+                v4i &a = fa2[PAIR][I], &b = fb2[PAIR][I];
+                const unsigned pa = fa_u[kb] + extra, pb = (BKN ? fb_kn : fb_u[kb]) + extra;
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(a) : "v"(pa), "n"(SB));
+                if (BKN) {
+                    v2i lo, hi;
+                    asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(lo) : "v"(pb), "n"(SB + kb * 4096));
+                    asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(hi) : "v"(pb), "n"(SB + kb * 4096 + 1024));
+                    b = v4i{lo.x, lo.y, hi.x, hi.y};
+                } else {
+                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(b) : "v"(pb), "n"(SB));
+                }
+            });
+        };
+        auto arrived = [&](auto pair_c) {                       // every outstanding read: the pair's
+            constexpr int PAIR = decltype(pair_c)::value;
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+            static_for<0, 2>([&](auto i_c) {
+                v4i &a = fa2[PAIR][decltype(i_c)::value], &b = fb2[PAIR][decltype(i_c)::value];
+                asm volatile("" : "+v"(a), "+v"(b));
+            });
+            v2f &t = pr[PAIR];
+            asm volatile("" : "+v"(t));
+        };
+        // a stage that is not the last one (and therefore whole), in ring slot SLOT
+        auto stage = [&](auto slot_c) {
+            constexpr int NEXT_SLOT = (decltype(slot_c)::value + 1) % NSTAGE;
+            arrived(p0);
+            fetch_pair(p1, slot_c, 0u, 0u);
+            __builtin_amdgcn_sched_barrier(0);
+            compute_block(fa2[0][0], fb2[0][0], pr[0][0]);
+            compute_block(fa2[0][1], fb2[0][1], pr[0][1]);
+            arrived(p1);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if constexpr (NEXT_SLOT == 0) tab += NSTAGE * KB_STAGE * 4;
+            fetch_pair(p0, std::integral_constant<int, NEXT_SLOT>{}, 0u, 0u);
+            __builtin_amdgcn_sched_barrier(0);
+            compute_block(fa2[1][0], fb2[1][0], pr[1][0]);
+            compute_block(fa2[1][1], fb2[1][1], pr[1][1]);
+        };
+        fetch_pair(p0, p0, 0u, 0u);
+        int s = 0;
+        for (; s + NSTAGE < nstages; s += NSTAGE) static_for<0, NSTAGE>(stage);
+        static_for<0, NSTAGE - 1>([&](auto slot_c) {
+            if (s + decltype(slot_c)::value + 1 < nstages) stage(slot_c);
+        });
+        // the last stage: its first K blocks are on their way
+        const int left = nkb - (nstages - 1) * KB_STAGE;
+        const unsigned slot = (unsigned)(nstages - 1 - s);
+        arrived(p0);
+        if (left > 2) fetch_pair(p1, p0, slot * STAGE_BYTES, slot * (KB_STAGE * 4));
+        __builtin_amdgcn_sched_barrier(0);
+        compute_block(fa2[0][0], fb2[0][0], pr[0][0]);
+        if (left > 1) compute_block(fa2[0][1], fb2[0][1], pr[0][1]);
+        if (left > 2) {
+            arrived(p1);
+            compute_block(fa2[1][0], fb2[1][0], pr[1][0]);
+            if (left > 3) compute_block(fa2[1][1], fb2[1][1], pr[1][1]);
+        }
+    };
+    if constexpr (TABLE) { if (loader) load_loop(); else table_loop(); }
+    else if (!wave_active) main_loop(std::false_type{}, std::integral_constant<int, PACE_HARDWARE>{});
     else if (WBM == 2 && p.pace == PACE_EVEN) main_loop(std::true_type{}, std::integral_constant<int, PACE_EVEN>{});
     else if (WBM == 2 && p.pace == PACE_ORDERED) main_loop(std::true_type{}, std::integral_constant<int, PACE_ORDERED>{});
     else main_loop(std::true_type{}, std::integral_constant<int, PACE_HARDWARE>{});
     __builtin_amdgcn_s_waitcnt(0xC07F);                        // the last, unused prefetch must land before its registers are reused
-    if (EPI != EPI_S32 && wave_active) {
+    if (EPI != EPI_S32 && wave_active && !loader) {
         accumulate(std::integral_constant<int, NBLK - 1>{});
         // The scaled factor sa*sb*2^26 overflows when sa*sb >= 2^102.  An infinite factor leaves every accumulator
         // it touches infinite or NaN (inf*0 included), so "some accumulator of the wave is not finite" catches all such
@@ -661,6 +799,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     if (PROF) { phase(2, (unsigned long long)wall_clock64()); phase(7, (unsigned long long)(clock64() - prof_c0)); }
     if (p.pace != PACE_HARDWARE) __builtin_amdgcn_s_setprio(0);
     __syncthreads();           // the epilogue reuses the ring as scratch
+    if (loader) return;
     if (PROF) phase(3, (unsigned long long)wall_clock64());
 
     // ---- epilogue ------------------------------------------------------------------------------------------
@@ -854,7 +993,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
 }
 
 template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
-__global__ __launch_bounds__(64 * WGM * WGN, WGPC * WGM * WGN / 4) void igemm_nt_kernel(GemmArgs p)
+__global__ __launch_bounds__(gemm_threads(WBM, WGM, WGN), WGPC * gemm_threads(WBM, WGM, WGN) / 256) void igemm_nt_kernel(GemmArgs p)
 {
     igemm_body<EPI, ST, WBM, WGM, WGN, NSTAGE, WGPC, BKN, AKM, PROF>(p, logical_workgroup());
 }
@@ -932,10 +1071,12 @@ static int launch_transpose(const int8_t *in, int R, int C, int8_t *out, hipStre
     return (int)hipGetLastError();
 }
 
-// LDS of a workgroup: operand ring and per-wave scale and product patches, or the epilogue's per-wave transposition patches
+constexpr int TABLE_KB = 512;                        // K blocks a wave's table of scale products holds (WBM = 1)
+// LDS of a workgroup: operand ring and per-wave scale and product patches or tables, or the epilogue's per-wave transposition patches
 constexpr int gemm_lds(int WBM, int WGM, int WGN, int NSTAGE)
 {
-    const int ring = NSTAGE * ((QB * WBM * WGM + QB * WBN * WGN) * ROW_BYTES + WGM * WGN * 512), patch = WGM * WGN * QB * EPI_LD * (int)sizeof(float);
+    const int scales = WBM == 1 ? 4 * (TABLE_KB + KB_STAGE) * WGM * WGN : NSTAGE * WGM * WGN * 512;
+    const int ring = NSTAGE * (QB * WBM * WGM + QB * WBN * WGN) * ROW_BYTES + scales, patch = WGM * WGN * QB * EPI_LD * (int)sizeof(float);
     return ring > patch ? ring : patch;
 }
 
@@ -970,7 +1111,7 @@ static int pace_of(long wgs, long slots, int k_per_wg)
 template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
 static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 {
-    constexpr int BM = QB * WBM * WGM, BN = QB * WBN * WGN, NT = 64 * WGM * WGN;
+    constexpr int BM = QB * WBM * WGM, BN = QB * WBN * WGN, NT = gemm_threads(WBM, WGM, WGN);
     constexpr int SMEM = gemm_lds(WBM, WGM, WGN, NSTAGE);
     if (!device_is_gfx950()) return JF_ERR_DEVICE;
     GemmArgs p = a;
@@ -1128,8 +1269,8 @@ static void wgrad_group_plan(int n, const int *M, const int *N, int K, int &spli
 // epilogue of one overlaps the main loop of the other).  A launch whose 32x128 tiles are all resident at once, two workgroups
 // of 4 waves and a 3-deep ring per CU, takes those instead: its 128x128 tiles would occupy at most a quarter of the chip with
 // 16 products per K block and SIMD pair in sequence, where a wave with one block is bound by the issue of its own 32 vector
-// instructions per product.  Measured (one-sequence forward GEMMs, us, 128x128 | 32x128): 32x768x768 9.7 | 6.7, 512x768x3072
-// 28.8 | 16.6, 512x3072x768 (384 small tiles) 10.7 | 8.4, 1248x768x768 10.7 | 7.1; beyond two per CU the larger tile's data
+// instructions per product.  Measured (one-sequence forward GEMMs, us, 128x128 | 32x128): 32x768x768 9.7 | 5.7, 512x768x3072
+// 28.8 | 12.8, 512x3072x768 (384 small tiles) 10.7 | 8.4, 1248x768x768 10.7 | 6.5; beyond two per CU the larger tile's data
 // reuse wins: 1248x2304x768 (702) 10.9 | 12.6.  (A deeper ring changes nothing there; a 64x128 tile of 8 waves is 6 % better
 // between 256 and 512 small tiles and up to 19 % worse below.)
 // A [K,N] B operand (and, for the weight gradient, a [K,M] A operand) is read in place.
@@ -1137,7 +1278,7 @@ static void wgrad_group_plan(int n, const int *M, const int *N, int K, int &spli
 template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs &a, hipStream_t st)
 {
     if constexpr (EPI != EPI_S32) {
-        if (a.splits <= 1 && (long)((a.M + 31) / 32) * ((a.N + 127) / 128) <= 2L * cu_count())
+        if (a.splits <= 1 && a.K <= TABLE_KB * QB && (long)((a.M + 31) / 32) * ((a.N + 127) / 128) <= 2L * cu_count())
             return launch_gemm_cfg<EPI, ST, 1, 1, 4, 3, 2, BKN>(a, st);
     }
     return launch_gemm_cfg<EPI, ST, 2, 2, 4, 2, 2, BKN>(a, st);

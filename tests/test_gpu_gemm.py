@@ -483,8 +483,10 @@ def test_phase_recording_build_gives_the_same_bits_and_ordered_phases(jf):
         assert ((ph["k_loop_MHz"] > 300) & (ph["k_loop_MHz"] < 3500)).all()
 
 
-@pytest.mark.parametrize("M,N", [(1056, 544), (2080, 1056)])      # 165 workgroups of 32x128 tiles; 153 of 128x128 (585 would be small ones)
-@pytest.mark.parametrize("K", [32, 96, 128, 160, 288, 384, 416])  # ring of two and of three stages: one, fewer than, as many as, more than its depth
+# 165 workgroups of 32x128 tiles; 153 of 128x128 (585 would be small ones).  K: rings of two and of three stages with one stage, fewer
+# than, as many as, more than their depth, every length of the last one; the longest row the small tiles take and the next one
+@pytest.mark.parametrize("M,N,K", [(m, n, k) for m, n in ((1056, 544), (2080, 1056)) for k in (32, 64, 96, 128, 160, 288, 384, 416, 896)]
+                         + [(32, 160, 16384), (32, 160, 16416)])
 def test_both_tile_sizes_at_every_ring_fill(jf, oracle, M, N, K):
     print(f"case M={M} N={N} K={K}", flush=True)
     A, Bkn, sa, sb = make_problem(M + N + K, M, N, K)
