@@ -102,16 +102,32 @@ enum { X, QX, SX, MEAN, RSTD, LN1, LN2, W_QKV, W_PROJ, W_FC, W_FC2, B_QKV, B_PRO
 struct WeightOperand { Tensor q, s; };
 struct BiasOperand { Tensor b, bmax; };
 
-void check_codes(const Tensor &q, const Tensor &s, int64_t R, int64_t C, const char *name)
+// What the kernels are told about a tensor is checked here, as the separate operators check theirs: all tensors of a call live on
+// the GPU that its kernels are launched on (`like`), and codes and scales split into rows of the width they are read with.
+bool matrix_of(const Tensor &t, int64_t R, int64_t C)
 {
-    TORCH_CHECK(q.is_cuda() && s.is_cuda() && q.is_contiguous() && s.is_contiguous() && q.element_size() == 1 && q.numel() == R * C &&
-                    s.scalar_type() == torch::kFloat16 && s.numel() == R / QB * (C / QB),
-                name, ": expected contiguous codes of [", R, ", ", C, "] with float16 scales");
+    return t.dim() >= 2 && t.size(-1) == C && t.numel() == R * C && t.is_contiguous();
 }
-const float *f32_vec(const Tensor &v, int64_t n, const char *name)
+void check_codes(const Tensor &q, const Tensor &s, int64_t R, int64_t C, const Tensor &like, const char *name)
 {
-    TORCH_CHECK(v.is_cuda() && v.scalar_type() == torch::kFloat32 && v.is_contiguous() && v.numel() == n, name, ": expected ", n, " contiguous float32 values");
+    TORCH_CHECK(q.is_cuda() && s.is_cuda(), name, ": expected GPU tensors");
+    TORCH_CHECK(q.device() == like.device() && s.device() == like.device(), name, ": codes and scales must be on ", like.device(), ", got ", q.device(),
+                " and ", s.device());
+    TORCH_CHECK(q.element_size() == 1 && s.scalar_type() == torch::kFloat16 && matrix_of(q, R, C) && matrix_of(s, R / QB, C / QB), name,
+                ": expected contiguous codes of [", R, ", ", C, "] with float16 scales, got ", q.sizes(), " and ", s.sizes());
+}
+const float *f32_vec(const Tensor &v, int64_t n, const Tensor &like, const char *name)
+{
+    TORCH_CHECK(v.is_cuda(), name, ": expected a GPU tensor");
+    TORCH_CHECK(v.scalar_type() == torch::kFloat32 && v.is_contiguous() && v.numel() == n && v.device() == like.device(), name, ": expected ", n,
+                " contiguous float32 values on ", like.device());
     return v.data_ptr<float>();
+}
+void check_residual(const Tensor &x, int64_t R, int64_t C, const Tensor &like, const char *name)
+{
+    TORCH_CHECK(x.is_cuda(), name, ": expected a GPU tensor");
+    TORCH_CHECK(x.device() == like.device() && matrix_of(x, R, C), name, ": expected a contiguous [B, T, C] tensor of ", R, " rows of ", C, " on ",
+                like.device());
 }
 
 struct BlockForward {
@@ -124,14 +140,14 @@ BlockForward forward_impl(const Dims &d, const Tensor &x, const Tensor &qx, cons
                           torch::ScalarType out_dtype)
 {
     const int64_t M = d.M, C = d.C;
-    check_codes(qx, sx, M, C, "qx");
-    check_codes(w[0].q, w[0].s, 3 * C, C, "w_qkv"); check_codes(w[1].q, w[1].s, C, C, "w_attn_proj");
-    check_codes(w[2].q, w[2].s, 4 * C, C, "w_fc"); check_codes(w[3].q, w[3].s, C, 4 * C, "w_mlp_proj");
-    const float *g1 = f32_vec(ln1, C, "ln_1"), *g2 = f32_vec(ln2, C, "ln_2"), *mu = f32_vec(mean, M, "mean"), *rs = f32_vec(rstd, M, "rstd");
+    check_residual(x, M, C, x, "x");
+    check_codes(qx, sx, M, C, x, "qx");
+    check_codes(w[0].q, w[0].s, 3 * C, C, x, "w_qkv"); check_codes(w[1].q, w[1].s, C, C, x, "w_attn_proj");
+    check_codes(w[2].q, w[2].s, 4 * C, C, x, "w_fc"); check_codes(w[3].q, w[3].s, C, 4 * C, x, "w_mlp_proj");
+    const float *g1 = f32_vec(ln1, C, x, "ln_1"), *g2 = f32_vec(ln2, C, x, "ln_2"), *mu = f32_vec(mean, M, x, "mean"), *rs = f32_vec(rstd, M, x, "rstd");
     const float *bp[4] = {}, *bm[4] = {};
     const int64_t widths[4] = {3 * C, C, 4 * C, C};
-    for (size_t i = 0; i < bias.size(); ++i) { bp[i] = f32_vec(bias[i].b, widths[i], "bias"); bm[i] = f32_vec(bias[i].bmax, 1, "biasmax"); }
-    TORCH_CHECK(x.is_contiguous() && x.numel() == M * C, "x: expected a contiguous [B, T, C] tensor");
+    for (size_t i = 0; i < bias.size(); ++i) { bp[i] = f32_vec(bias[i].b, widths[i], x, "bias"); bm[i] = f32_vec(bias[i].bmax, 1, x, "biasmax"); }
     const int xc = fp_of(x, "x");
 
     c10::DeviceGuard guard(x.device());
@@ -226,8 +242,8 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const Tensor &qx = s[0], &sx = s[1], &mean = s[2], &rstd = s[3], &ln1 = s[4], &ln2 = s[5];
         const WeightOperand w[4] = {{s[6], s[7]}, {s[8], s[9]}, {s[10], s[11]}, {s[12], s[13]}};
         const Tensor fpg = grads[0].contiguous(), qg = grads[1].contiguous(), sg = grads[2].contiguous();
-        check_codes(qg, sg, M, C, "gradient");
-        TORCH_CHECK(fpg.numel() == M * C, "gradient: expected [B, T, C]");
+        check_residual(fpg, M, C, qx, "gradient");
+        check_codes(qg, sg, M, C, qx, "gradient");
 
         c10::DeviceGuard guard(qx.device());
         const auto opt = qx.options().requires_grad(false);

@@ -72,6 +72,18 @@ def test_cpu_tensors_are_rejected_not_computed():
         BQC.igemm_output_int_quantize_fused(a, a, s, s, 32, 32, 32)
 
 
+def test_block_node_refuses_host_tensors():
+    import BlockQuantizeCUDA as BQC
+    B, T, C, H = 1, 32, 64, 2
+    f8, f16 = torch.float8_e4m3fn, torch.float16
+    widths = [(3 * C, C), (C, C), (4 * C, C), (C, 4 * C)]
+    params = [torch.ones(C), torch.ones(C)] + [torch.zeros(*w) for w in widths]
+    codes = [(torch.zeros(*w, dtype=torch.int8), torch.ones(w[0] // 32, w[1] // 32, dtype=f16)) for w in widths]
+    x, q, s = torch.zeros(B, T, C), torch.zeros(B, T, C, dtype=torch.int8).view(f8), torch.ones(B, T // 32, C // 32, dtype=f16)
+    with pytest.raises(RuntimeError, match="x: expected a GPU tensor"):
+        BQC.jetfire.qblock(x, q, s, torch.zeros(B, T), torch.ones(B, T), params, codes, [], [], H, torch.float32)
+
+
 # ------------------------------------------------------------------------------------------- GPU side
 def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()

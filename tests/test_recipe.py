@@ -339,3 +339,56 @@ def test_block_as_one_node_equals_the_functions(B, T, C, H, bias, res, out):
     for (q, s), w in zip(jf.quantize_many([blk.w_qkv.detach(), blk.w_fc.detach()]), (blk.w_qkv, blk.w_fc)):
         q2, s2 = int8_quantize(w.detach(), 32)
         assert torch.equal(q, q2) and torch.equal(s, s2)
+
+
+def block_arguments(B=1, T=64, C=128, H=4, bias=True):
+    """What QBlock.forward hands to the extension: [x, qx, sx, mean, rstd, params, codes, biases, (bias, max) pairs, heads, type]."""
+    import BlockQuantizeCUDA as BQC
+    import recipe
+    torch.manual_seed(6)
+    blk = recipe.QBlock(C, H, torch.float32, bias).cuda()
+    x = torch.randn(B, T, C, device="cuda")
+    x, qx, sx = recipe.StreamBegin.apply(x)
+    mean, rstd = BQC.jetfire.rowstats_fp(x)
+    ws, bs = [blk.w_qkv, blk.w_attn_proj, blk.w_fc, blk.w_mlp_proj], [blk.b_qkv, blk.b_attn_proj, blk.b_fc, blk.b_mlp_proj]
+    codes = [tuple(p) for p in recipe.weight_codes.get_many(ws)]
+    return [x, qx, sx, mean, rstd, [blk.ln_1, blk.ln_2] + ws, codes, bs, [recipe.weight_codes.get_bias(b) for b in bs], H, torch.float32]
+
+
+def test_block_refuses_tensors_of_another_device_or_shape():
+    """Every tensor of the block's single node is looked at before anything is launched: on the GPU of x, of its own width."""
+    import BlockQuantizeCUDA as BQC
+    qblock = BQC.jetfire.qblock
+    assert len(qblock(*block_arguments())) == 5
+    X, QX, SX, MEAN, RSTD, PARAMS, CODES, BPARAMS, BPAIRS = range(9)
+
+    def host(t):
+        return t.detach().cpu()
+
+    def other_shape(t):                                            # the same number of elements in rows of another width
+        return t.detach().reshape(*t.shape[:-2], t.shape[-2] // 2, t.shape[-1] * 2)
+
+    def swap(i, f, *path):
+        a = block_arguments()
+        if not path:
+            a[i] = f(a[i])
+        else:
+            inner = list(a[i])
+            if len(path) == 1:
+                inner[path[0]] = f(inner[path[0]])
+            else:
+                pair = list(inner[path[0]])
+                pair[path[1]] = f(pair[path[1]])
+                inner[path[0]] = tuple(pair)
+            a[i] = inner
+        return a
+
+    cases = [(i, host) for i in (X, QX, SX, MEAN, RSTD)] + [(PARAMS, host, 0), (PARAMS, host, 1)]
+    cases += [(CODES, host, k, part) for k in range(4) for part in range(2)] + [(BPAIRS, host, k, part) for k in range(4) for part in range(2)]
+    cases += [(i, other_shape) for i in (QX, SX)] + [(CODES, other_shape, k, part) for k in range(4) for part in range(2)]
+    cases += [(MEAN, lambda t: t[..., :-32].contiguous()), (PARAMS, lambda t: t.detach()[:-32], 0), (BPAIRS, lambda t: t[:-32], 2, 0)]
+    for case in cases:
+        args = swap(*case)
+        with pytest.raises(RuntimeError, match="expected|must be"):
+            qblock(*args)
+            raise AssertionError(f"accepted: {case}")
