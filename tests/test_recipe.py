@@ -392,3 +392,29 @@ def test_block_refuses_tensors_of_another_device_or_shape():
         with pytest.raises(RuntimeError, match="expected|must be"):
             qblock(*args)
             raise AssertionError(f"accepted: {case}")
+
+
+def test_block_calls_its_hooks():
+    """Forward, full backward and full backward pre-hooks of a block see its five outputs and their gradients."""
+    import recipe
+    torch.manual_seed(8)
+    model = recipe.QStack(2, 128, 4).cuda()
+    seen = []
+    for i, blk in enumerate(model.blocks):
+        blk.register_forward_hook(lambda m, a, out, i=i: seen.append(("forward", i, type(out), len(out))))
+        blk.register_full_backward_pre_hook(lambda m, go, i=i: seen.append(("pre", i, type(go), len(go))))
+        blk.register_full_backward_hook(lambda m, gi, go, i=i: seen.append(("backward", i, type(go), len(go))))
+    x = torch.randn(2, 64, 128, device="cuda", requires_grad=True)
+    w = torch.randn(2, 64, 128, device="cuda")
+    torch.manual_seed(9)
+    (model(x) * w).sum().backward()
+    assert seen == [("forward", 0, tuple, 5), ("forward", 1, tuple, 5), ("pre", 1, tuple, 5), ("backward", 1, tuple, 5), ("pre", 0, tuple, 5),
+                    ("backward", 0, tuple, 5)]
+    got = [x.grad] + [p.grad for p in model.parameters()]
+    plain = recipe.QStack(2, 128, 4).cuda()                        # the hooks change nothing
+    plain.load_state_dict(model.state_dict())
+    x2 = x.detach().clone().requires_grad_(True)
+    torch.manual_seed(9)
+    (plain(x2) * w).sum().backward()
+    for a, b in zip(got, [x2.grad] + [p.grad for p in plain.parameters()]):
+        assert torch.equal(a, b)
