@@ -22,9 +22,7 @@ CSRC = os.path.join(HERE, "csrc")
 HIP_LIB = os.path.join(HERE, "libjetfire_hip.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-# (source, flags of its own).  The attention's maxima are taken over finite scores and -inf: without the flag every one of
-# them carries a canonicalisation for NaN operands.
-HIP_SOURCES = [("jf_gemm.hip", []), ("jf_blockops.hip", []), ("jf_attention.hip", ["-fno-honor-nans"])]
+HIP_SOURCES = ["jf_gemm.hip", "jf_blockops.hip", "jf_attention.hip"]
 PROF_LIB = os.path.join(HERE, "libjetfire_prof.so")
 PROF_SOURCES = [("jf_gemm.hip", ["-DJF_PROF_LIB"], "jf_gemm_prof.o"), ("jf_calib.hip", [], "jf_calib.o")]
 HIP_FLAGS = [
@@ -54,9 +52,9 @@ def build_hip():
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     jobs, prof_jobs = [], []
-    for src, extra in HIP_SOURCES:
+    for src in HIP_SOURCES:
         obj = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
-        cmd = [hipcc] + flags + extra + ["-c", os.path.join(CSRC, src), "-o", obj]
+        cmd = [hipcc] + flags + ["-c", os.path.join(CSRC, src), "-o", obj]
         print("+", " ".join(cmd), flush=True)
         jobs.append((cmd, obj, subprocess.Popen(cmd)))
     for src, extra, name in PROF_SOURCES:

@@ -217,7 +217,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_fwd_kernel(Attn
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[mb][v] = 0.0f;
     const float c = a.scale * 1.44269504f;
-    float m = -__builtin_inff(), l = 0.0f;                     // running maximum (shared by the halves), this lane's part of the sum
+    // Running maximum (shared by the halves), this lane's part of the sum.  The maximum starts below every finite score but
+    // finite: keys whose score is -inf before the first finite one then count for nothing instead of giving -inf - -inf.
+    float m = -1e30f, l = 0.0f;
     io.load(lds, kp, a.ld, vp, a.ld, 0, a.T - 1);
     for (int t = 0; t < nt; ++t) {
         attn_tile_ready();                                     // tile t has landed; nobody reads the other buffer any more
@@ -236,10 +238,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_fwd_kernel(Attn
 #pragma unroll
                 for (int v = 0; v < 16; ++v) s[v] = 8 * (v >> 2) + 4 * h + (v & 3) > (lane & 31) ? -__builtin_inff() : s[v];
             }
+            // (v_maximum3_f32: a NaN stays one, and no operand has to be canonicalised first as for fmaxf)
             float mx = s[0];
 #pragma unroll
-            for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
-            mx = fmaxf(mx, half_swap(mx));
+            for (int v = 1; v < 16; ++v) mx = __builtin_elementwise_maximum(mx, s[v]);
+            mx = __builtin_elementwise_maximum(mx, half_swap(mx));
             // The maximum only guards the exponential's range: it is raised, and the sums rescaled, when a score exceeds it
             // by more than a factor of 2^8 (every later probability keeps its relative precision in binary16 up to there).
             if (__any((mx - m) * c > 8.0f)) {

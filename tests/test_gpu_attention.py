@@ -52,3 +52,68 @@ def test_causal_attention(B, H, T, D, scale):
     qg, sg = jf.attention_bwd_q(q, k, v, out, lse, g, B, H, 3, 40)
     wq, ws, _ = jf.quantize(grads, jf.ROUND_STOCHASTIC, torch.float16, False, 0.0, 3, 40)
     assert torch.equal(qg, wq) and torch.equal(sg, ws)
+
+
+def causal_rows(qkv, B, H, T, D):
+    """Attention in float32 on the CPU, every query over its own keys only: what lies behind a query cannot reach it."""
+    x = qkv.float().cpu().view(B, T, 3, H, D).permute(2, 0, 3, 1, 4)
+    rows = []
+    for i in range(T):
+        s = (x[1][:, :, : i + 1] * x[0][:, :, i: i + 1]).sum(-1) * D ** -0.5
+        p = torch.softmax(s, -1)
+        rows.append(torch.where(p == 0, torch.zeros(()), p).unsqueeze(-1).mul(x[2][:, :, : i + 1]).sum(2))
+    return torch.stack(rows, 2).transpose(1, 2).reshape(B * T, H * D)
+
+
+INF, NAN = float("inf"), float("nan")
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("what,value", [("q", NAN), ("k", NAN), ("v", NAN), ("q", INF), ("k", INF), ("v", INF), ("v", -INF)])
+def test_a_value_that_is_not_finite_reaches_the_result(D, what, value):
+    """An infinity or NaN in q, k or v: the result is not finite wherever it is not in float32, and untouched in the row blocks
+    before it.  The quantised results are those of the stored ones, and a NaN gradient reaches every gradient it belongs to."""
+    import BlockQuantizeCUDA as BQC
+    jf, B, H, T, at = BQC.jetfire, 1, 2, 160, 70
+    C = H * D
+    gen = torch.Generator().manual_seed(D)
+    qkv = torch.randn(T, 3 * C, generator=gen).half()
+    g = (torch.randn(T, C, generator=gen) * 1e-2).half().cuda()
+    qkv[:, 5] = qkv[:, C + 5] = 1.0                                # (head 0: one column of q and k with a known sign)
+    qkv[at, {"q": 0, "k": C, "v": 2 * C}[what] + 5] = value
+    print(f"case {what}={value} D={D}", flush=True)
+    q, k, v = qkv.cuda().split(C, dim=1)
+    out, lse, qo, so = jf.attention_fwd_q(q, k, v, B, H)
+    want = causal_rows(qkv, B, H, T, D)
+    bad = ~want.isfinite()
+    assert bad.any() and not out.cpu()[bad].isfinite().any()
+    assert out.cpu()[:64].isfinite().all() and rel(out[:64], want[:64]) < 1e-3                        # row blocks before it
+    assert out.cpu()[:, D:].isfinite().all() and rel(out[:, D:], want[:, D:]) < 1e-3                  # the other head
+    wq, ws, _ = jf.quantize(out, jf.ROUND_NEAREST)
+    assert torch.equal(qo, wq) and torch.equal(so.view(torch.int16), ws.view(torch.int16))
+    grads = jf.attention_bwd(q, k, v, out, lse, g, B, H)
+    qg, sg = jf.attention_bwd_q(q, k, v, out, lse, g, B, H, 3, 40)
+    wq, ws, _ = jf.quantize(grads, jf.ROUND_STOCHASTIC, torch.float16, False, 0.0, 3, 40)
+    assert torch.equal(qg, wq) and torch.equal(sg.view(torch.int16), ws.view(torch.int16))
+    if what == "q":                                                # a query's row of scores: its own dq, dk and dv of its keys
+        rows = grads.cpu()
+        assert rows[at, :D].isnan().all() and rows[: at + 1, C: C + D].isnan().all() and rows[: at + 1, 2 * C: 2 * C + D].isnan().all()
+        assert rows[96:, :D].isfinite().all() and rows[:, D: C].isfinite().all()
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("keys", [range(0, 32), range(0, 64), range(0, 96), [3, 40, 159]])
+def test_scores_of_minus_infinity_count_for_nothing(D, keys):
+    """Keys whose scores are -inf (k infinite against a positive q): the other keys decide; a query with no other key has no result."""
+    import BlockQuantizeCUDA as BQC
+    jf, B, H, T = BQC.jetfire, 1, 1, 160
+    gen = torch.Generator().manual_seed(D)
+    qkv = torch.randn(T, 3 * D, generator=gen).half()
+    qkv[:, 5] = 1.0
+    qkv[list(keys), D + 5] = -INF
+    print(f"case keys={keys} D={D}", flush=True)
+    out, _ = jf.attention_fwd(*qkv.cuda().split(D, dim=1), B, H)
+    want = causal_rows(qkv, B, H, T, D)
+    finite = want.isfinite().all(1)
+    assert finite.sum() >= 64 and not out.cpu()[~finite].isfinite().any()
+    assert rel(out.cpu()[finite], want[finite]) < 1e-3
