@@ -40,6 +40,7 @@ extern "C" {
 #define JF_ERR_DEVICE        -6   /* the current device is not gfx950                */
 #define JF_ERR_UNSUPPORTED   -7   /* valid codes, but this combination of layouts is not implemented */
 #define JF_ERR_SCRATCH_LIMIT -8   /* jf_igemm_block_fp_noalloc: the K split needs more than JF_NOALLOC_SCRATCH_BYTES */
+#define JF_ERR_VALUE         -9   /* a number outside the range its entry point states */
 
 /* A operand layout of jf_igemm_block_fp (every other GEMM entry point takes A as [M,K]) */
 #define JF_A_MK 0                 /* A is [M,K] row-major                                                          */
@@ -310,7 +311,8 @@ int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const in
 /* Causal self-attention between the QKV projection and the output projection, binary16 in and out.  q, k, v: [B*T, ld]
  * with head h of a row at columns h*D .. h*D + D - 1 of each pointer (the three column ranges of the projection's output,
  * ld = 3*H*D, or tensors of their own); out: [B*T, H*D]; lse: [B*H, T] fp32, log2 of the row sums (for the backward call).
- * D = 32 or 64, T a multiple of 32, pointers 16-byte aligned.  Scores, sums and products accumulate in fp32; probabilities
+ * D = 32 or 64, T a multiple of 32, pointers 16-byte aligned; scale, the factor of the scores, positive, normal and with a finite
+ * 1.4427 * scale (else JF_ERR_VALUE).  Scores, sums and products accumulate in fp32; probabilities
  * enter the second product in binary16.  Replaces scaled_dot_product_attention of the reference's recipe
  * (INT8_GPT2/qmodel.py:134). */
 int jf_attention_fwd(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale, void *out,

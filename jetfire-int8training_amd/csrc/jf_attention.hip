@@ -468,11 +468,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void attn_dkv_kernel(Attn
     }
 }
 
-static int attn_check(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D)
+static int attn_check(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale)
 {
     if (!q || !k || !v) return JF_ERR_NULL;
     if (B <= 0 || H <= 0 || T <= 0 || T % 32 || (D != 32 && D != 64) || ld < H * D || ld % 8) return JF_ERR_SHAPE;
     if ((long)T * ld >= (1L << 30)) return JF_ERR_SHAPE;       // a batch element is addressed with 32-bit byte offsets
+    // The kernels work with scale * log2(e) behind the causal mask's -inf and behind a maximum of the unscaled scores: it has to
+    // be positive (0 * -inf is no number, a negative factor turns the maximum round) and a normal finite number.
+    if (!(scale >= 1.17549435e-38f && scale * 1.44269504f < __builtin_inff())) return JF_ERR_VALUE;
     if (!aligned16(q) || !aligned16(k) || !aligned16(v)) return JF_ERR_ALIGN;
     return device_is_gfx950() ? JF_OK : JF_ERR_DEVICE;
 }
@@ -507,7 +510,7 @@ using namespace jf;
 static int attention_fwd(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale, void *out, float *lse,
                          int8_t *codes, void *scales, jf_stream_t stream)
 {
-    int rc = attn_check(q, k, v, ld, B, H, T, D);
+    int rc = attn_check(q, k, v, ld, B, H, T, D, scale);
     if (rc) return rc;
     if (!out || !lse) return JF_ERR_NULL;
     if (!aligned16(out) || !aligned16(codes)) return JF_ERR_ALIGN;
@@ -524,7 +527,7 @@ static int attention_bwd(const void *q, const void *k, const void *v, int ld, co
                          int T, int D, float scale, void *gq, void *gk, void *gv, int ldg, float *delta, int8_t *codes, void *scales,
                          uint64_t seed, uint64_t offset, jf_stream_t stream)
 {
-    int rc = attn_check(q, k, v, ld, B, H, T, D);
+    int rc = attn_check(q, k, v, ld, B, H, T, D, scale);
     if (rc) return rc;
     if (!out || !gout || !lse || !delta) return JF_ERR_NULL;
     if ((long)T * H * D >= (1L << 30)) return JF_ERR_SHAPE;

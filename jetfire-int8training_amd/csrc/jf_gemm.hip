@@ -1350,6 +1350,7 @@ const char *jf_error_string(int code)
     case JF_ERR_DEVICE: return "jetfire_hip: device is not gfx950";
     case JF_ERR_UNSUPPORTED: return "jetfire_hip: this combination of operand layouts is not implemented";
     case JF_ERR_SCRATCH_LIMIT: return "jetfire_hip: the K split of this problem needs more than the built-in scratch buffer (JF_NOALLOC_SCRATCH_BYTES); use jf_igemm_block_fp with a workspace, or splitk = 1";
+    case JF_ERR_VALUE: return "jetfire_hip: a number is outside the range this entry point states";
     default: return code > 0 ? hipGetErrorString((hipError_t)code) : "jetfire_hip: unknown error";
     }
 }

@@ -68,3 +68,18 @@ def test_argument_errors_without_gpu(jf):
     # (16 parts of 1600 x 1600 fp32 = 164 MB) before it touches the device
     assert L.jf_igemm_block_fp_noalloc(p, p, p, p, p, 1600, 1600, 8192, 0, 1, 1, 0, 0, 1, 16, None) == -8
     assert b"scratch" in L.jf_error_string(-8)
+
+
+def test_attention_refuses_a_scale_it_cannot_use(jf):
+    """The factor of the scores has to be positive, normal and finite; checked before the device is touched."""
+    L = jf.lib()
+    buf = (ctypes.c_char * 4096)()
+    p = (ctypes.addressof(buf) + 15) & ~15
+    for scale in (0.0, -0.0, -0.125, 1e-40, float("inf"), float("nan"), 3.4e38):
+        assert L.jf_attention_fwd(p, p, p, 32, 1, 1, 32, 32, scale, p, p, None) == -9, scale
+        assert L.jf_attention_bwd(p, p, p, 32, p, p, p, 1, 1, 32, 32, scale, p, p, p, 32, p, None) == -9, scale
+    assert b"range" in L.jf_error_string(-9)
+    import torch
+    if not torch.cuda.is_available():                               # (as above: p is host memory)
+        for scale in (1.1754944e-38, 0.125, 2e38):
+            assert L.jf_attention_fwd(p, p, p, 32, 1, 1, 32, 32, scale, p, p, None) == -6, scale
