@@ -84,6 +84,11 @@ def lib():
         L.jf_block_colsum.argtypes = [_p, _p, _i, _i, _i, _p, _p, _sz, _p]
         L.jf_attention_fwd.argtypes = [_p, _p, _p, _i, _i, _i, _i, _i, _f, _p, _p, _p]
         L.jf_attention_bwd.argtypes = [_p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _f, _p, _p, _p, _i, _p, _p]
+        L.jf_attention_fwd_q.argtypes = [_p, _p, _p, _i, _i, _i, _i, _i, _f, _p, _p, _p, _p, _p]
+        L.jf_attention_bwd_q.argtypes = [_p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _i, _f, _p, _p, _u64, _u64, _p, _p]
+        L.jf_layernorm_bwd_add_strips.argtypes = [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _u64, _u64, _p, _i, _i, _u64, _u64,
+                                                  _p, _i, _p, _p, _p, _p]
+        L.jf_philox_rounds.argtypes = []
         L.jf_quantize_many.argtypes = [_i, _p, _p, _p, _i, _p, _p, _i, _p]
         L.jf_rowstats_fp.argtypes = [_p, _i, _i, _i, _p, _p, _p]
         missing = [name for name in EXPORTS if not hasattr(L, name)]

@@ -24,6 +24,24 @@ def test_binding_lists_every_symbol(jf):
     assert sorted(jf.EXPORTS) == _declared()
 
 
+def test_binding_declares_the_arguments_of_every_symbol(jf):
+    """Without argument types ctypes would cut a device pointer to 32 bits: the binding's are those of the header, one by one."""
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "jetfire_hip.h")).read(), flags=re.S)
+    kinds = {"int": ctypes.c_int, "float": ctypes.c_float, "uint64_t": ctypes.c_uint64, "size_t": ctypes.c_size_t, "jf_stream_t": ctypes.c_void_p}
+    seen = 0
+    for name, args in re.findall(r"\b(jf_[a-z0-9_]+)\s*\(([^()]*)\)\s*;", text):
+        args = [a.strip() for a in args.split(",")] if args.strip() not in ("", "void") else []
+        got = getattr(jf.lib(), name).argtypes
+        assert got is not None and len(got) == len(args), name
+        for a, t in zip(args, got):
+            if "*" in a:
+                assert t is ctypes.c_void_p or issubclass(t, ctypes._Pointer), (name, a)
+            else:
+                assert t is kinds[a.split()[0]], (name, a)
+        seen += 1
+    assert seen == len(jf.EXPORTS)
+
+
 def test_measurement_library_is_separate(jf):
     """The measurement aids live in their own library and header: the product library exports only what jetfire_hip.h
     declares (the reference's interfaces and the allocation-free entry point)."""
