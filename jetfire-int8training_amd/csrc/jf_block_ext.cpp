@@ -5,6 +5,7 @@
 // allocation per intermediate.  What the backward needs lives in one buffer, what only the call needs in another.
 #include "bqc_common.h"
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -67,6 +68,24 @@ struct ForwardTemp {
         return k.used;
     }
 };
+
+// Both of them where no backward follows: what is dead makes room for what comes after it.  Two block tensors of [M, C] serve in
+// turn as qn, qy, q2 and as qo, qn2, qo; Q, K, V and the attention's result make room for the float sum and the hidden layer.  14
+// bytes per element of [M, C] and the scales, where a call whose backward follows holds 25.
+size_t carve_inference(uint8_t *b, const Dims &d, Saved &v, ForwardTemp &t)
+{
+    Carver k(b);
+    v.qn = v.qy = v.q2 = k.take<int8_t>(d.codes(d.c)); v.sn = v.sy = v.s2 = k.take(d.scales(d.c));
+    t.qo = v.qn2 = k.take<int8_t>(d.codes(d.c)); t.so = v.sn2 = k.take(d.scales(d.c));
+    v.lse = k.take<float>(d.m * d.H * 4); v.mean2 = k.take<float>(d.m * 4); v.rstd2 = k.take<float>(d.m * 4);
+    t.rowsum = k.take<float>(d.c / 32 * d.m * 4); t.rowsq = k.take<float>(d.c / 32 * d.m * 4);
+    Carver attention(b ? b + k.used : nullptr), mlp(attention.base);
+    v.qkv = attention.take(d.m * 3 * d.c * 2); v.y = attention.take(d.m * d.c * 2);
+    t.mid = mlp.take<float>(d.m * d.c * 4);
+    v.qh = mlp.take<int8_t>(d.codes(4 * d.c)); v.sh = mlp.take(d.scales(4 * d.c));
+    v.qa = mlp.take<int8_t>(d.codes(4 * d.c)); v.sa = mlp.take(d.scales(4 * d.c));
+    return k.used + std::max(attention.used, mlp.used);
+}
 
 struct BackwardTemp {
     int8_t *qp, *qd, *qr, *qq;
@@ -135,9 +154,10 @@ struct BlockForward {
 };
 
 // Forward of a block.  weights: qkv, projection, fc, second projection.  biases: empty or one (bias, max|bias|) pair each.
+// keep: leave what the backward needs in `saved` (else it stays undefined).
 BlockForward forward_impl(const Dims &d, const Tensor &x, const Tensor &qx, const Tensor &sx, const Tensor &mean, const Tensor &rstd,
                           const Tensor &ln1, const Tensor &ln2, const std::vector<WeightOperand> &w, const std::vector<BiasOperand> &bias,
-                          torch::ScalarType out_dtype)
+                          torch::ScalarType out_dtype, bool keep)
 {
     const int64_t M = d.M, C = d.C;
     check_residual(x, M, C, x, "x");
@@ -155,10 +175,14 @@ BlockForward forward_impl(const Dims &d, const Tensor &x, const Tensor &qx, cons
     Saved v;
     ForwardTemp t;
     BlockForward r;
-    r.saved = torch::empty({(int64_t)v.carve(nullptr, d)}, opt.dtype(torch::kUInt8));
-    Tensor temp = torch::empty({(int64_t)t.carve(nullptr, d)}, opt.dtype(torch::kUInt8));
-    v.carve((uint8_t *)r.saved.data_ptr(), d);
-    t.carve((uint8_t *)temp.data_ptr(), d);
+    Tensor temp = torch::empty({(int64_t)(keep ? t.carve(nullptr, d) : carve_inference(nullptr, d, v, t))}, opt.dtype(torch::kUInt8));
+    if (keep) {
+        r.saved = torch::empty({(int64_t)v.carve(nullptr, d)}, opt.dtype(torch::kUInt8));
+        v.carve((uint8_t *)r.saved.data_ptr(), d);
+        t.carve((uint8_t *)temp.data_ptr(), d);
+    } else {
+        carve_inference((uint8_t *)temp.data_ptr(), d, v, t);
+    }
     r.fp = torch::empty({d.B, d.T, C}, opt.dtype(out_dtype));
     r.q = torch::empty({d.B, d.T, C}, opt.dtype(torch::kFloat8_e4m3fn));
     r.s = torch::empty({d.B, d.T / QB, C / QB}, opt.dtype(torch::kFloat16));
@@ -204,17 +228,18 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
     static variable_list forward(AutogradContext *ctx, Tensor x_, Tensor qx, Tensor sx, Tensor mean, Tensor rstd, Tensor ln1, Tensor ln2, Tensor w1,
                                  Tensor w2, Tensor w3, Tensor w4, OptTensor b1, OptTensor b2, OptTensor b3, OptTensor b4,
                                  const std::vector<WeightOperand> &w,
-                                 const std::vector<BiasOperand> &bias, int64_t heads, torch::ScalarType out_dtype)
+                                 const std::vector<BiasOperand> &bias, int64_t heads, torch::ScalarType out_dtype, bool keep)
     {
         const variable_list in{x_, qx, sx, mean, rstd, ln1, ln2, w1, w2, w3, w4};
         const Tensor &x = in[X];
         const Dims d = dims_of(x, heads);
-        BlockForward r = forward_impl(d, x, in[QX], in[SX], in[MEAN], in[RSTD], in[LN1], in[LN2], w, bias, out_dtype);
+        BlockForward r = forward_impl(d, x, in[QX], in[SX], in[MEAN], in[RSTD], in[LN1], in[LN2], w, bias, out_dtype, keep);
+        if (!keep) return {r.fp, r.q, r.s, r.mean, r.rstd};
         ctx->set_materialize_grads(false);
-        variable_list keep{in[QX], in[SX], in[MEAN], in[RSTD], in[LN1], in[LN2]};
-        for (auto &o : w) { keep.push_back(o.q); keep.push_back(o.s); }
-        keep.push_back(r.saved);
-        ctx->save_for_backward(std::move(keep));
+        variable_list held{in[QX], in[SX], in[MEAN], in[RSTD], in[LN1], in[LN2]};
+        for (auto &o : w) { held.push_back(o.q); held.push_back(o.s); }
+        held.push_back(r.saved);
+        ctx->save_for_backward(std::move(held));
         auto &data = ctx->saved_data;
         data["shape"] = std::vector<int64_t>{d.B, d.T, d.C, d.H};
         data["types"] = std::vector<int64_t>{(int64_t)x.scalar_type(), (int64_t)in[W_QKV].scalar_type(), (int64_t)(b1 ? b1->scalar_type() : torch::kFloat32)};
@@ -259,7 +284,7 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         Tensor temp = torch::empty({(int64_t)t.carve(nullptr, d, res_bytes, ws_bytes)}, opt.dtype(torch::kUInt8));
         t.carve((uint8_t *)temp.data_ptr(), d, res_bytes, ws_bytes);
 
-        variable_list out(N_GRAD + 4);                         // (one entry per argument of forward)
+        variable_list out(N_GRAD + 5);                         // (one entry per argument of forward)
         out[X] = torch::empty({B, T, C}, opt.dtype(res_type));
         out[QX] = torch::empty({B, T, C}, opt.dtype(torch::kFloat8_e4m3fn));
         out[SX] = torch::empty({B, T / QB, C / QB}, opt.dtype(torch::kFloat16));
@@ -343,8 +368,13 @@ variable_list qblock(const Tensor &x, const Tensor &qx, const Tensor &sx, const 
     for (auto &p : codes) w.push_back({std::get<0>(p), std::get<1>(p)});
     for (auto &p : bias_pairs) bias.push_back({std::get<0>(p), std::get<1>(p)});
     const auto b = [&](size_t i) { return bias_params.empty() ? OptTensor() : OptTensor(bias_params[i]); };
+    // the condition under which autograd will ask for a backward
+    variable_list inputs{x, qx, sx, mean, rstd};
+    inputs.insert(inputs.end(), params.begin(), params.end());
+    inputs.insert(inputs.end(), bias_params.begin(), bias_params.end());
+    const bool keep = c10::GradMode::is_enabled() && std::any_of(inputs.begin(), inputs.end(), [](const Tensor &t) { return t.requires_grad(); });
     return BlockNode::apply(x, qx, sx, mean, rstd, params[0], params[1], params[2], params[3], params[4], params[5], b(0), b(1), b(2), b(3), w, bias,
-                            heads, out_dtype);
+                            heads, out_dtype, keep);
 }
 
 }  // namespace

@@ -418,3 +418,43 @@ def test_block_calls_its_hooks():
     (plain(x2) * w).sum().backward()
     for a, b in zip(got, [x2.grad] + [p.grad for p in plain.parameters()]):
         assert torch.equal(a, b)
+
+
+def test_block_without_a_backward_keeps_nothing_for_one():
+    """Under no_grad (and where nothing requires a gradient) a block holds what its next operators need, not what a backward
+    would: 14 bytes per element of [tokens, C] and its results; same bits as with a gradient.  A gradient of one parameter
+    alone, or of the input alone, is still computed."""
+    import recipe
+    torch.manual_seed(12)
+    B, T, C, H = 16, 512, 256, 4
+    blk = recipe.QBlock(C, H, torch.float32, True).cuda()
+    args = block_arguments(B, T, C, H)[:5]
+    want = [t.detach().clone() for t in blk(*args)]                # (also quantises the weights)
+
+    def peak(f):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out = f()
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - before, out
+
+    def check(held, out):
+        for a, b in zip(out, want):
+            assert torch.equal(a.view(torch.int8), b.view(torch.int8)) and not a.requires_grad
+        # 14 inside, a float32 sum and codes as results, 0.5 for scales, statistics and row sums; the allocator counts up to 1 MiB
+        # more for each of the three large tensors (it does not split off less)
+        assert held < (14 + 5 + 0.5) * B * T * C + (3 << 20), held / (B * T * C)
+
+    with torch.no_grad():
+        check(*peak(lambda: blk(*args)))
+    with torch.inference_mode():
+        check(*peak(lambda: blk(*args)))
+    for p in blk.parameters():
+        p.requires_grad_(False)
+    check(*peak(lambda: blk(*args)))
+    blk.w_fc.requires_grad_(True)
+    blk(*args)[0].sum()                                            # a graph that is never used
+    fp, q, s, _, _ = blk(*args)
+    recipe.StreamEnd.apply(fp, q, s).backward(torch.ones_like(fp))
+    assert blk.w_fc.grad.isfinite().all() and blk.w_fc.grad.abs().sum() > 0 and blk.w_qkv.grad is None
