@@ -75,6 +75,12 @@ std::vector<int64_t> scale_shape(const Tensor &x)
     return n;
 }
 
+// scales of a result laid out like the codes q (an operand's own scales may have another rank: [B, T, C] with [B T/32, C/32])
+Tensor scales_for(const Tensor &q, const Tensor &s)
+{
+    return torch::empty(scale_shape(q), s.options());
+}
+
 // one value per row, [R] or [B, T]
 std::vector<int64_t> row_shape(const Tensor &x)
 {
@@ -281,7 +287,7 @@ std::tuple<Tensor, Tensor> layernorm_fwd(const Tensor &q, const Tensor &s, const
     const float *g = vec(gamma, C, q, "gamma"), *b = beta ? vec(*beta, C, q, "beta") : nullptr;
     const float *m = vec(mean, R, q, "mean"), *r = vec(rstd, R, q, "rstd");
     c10::DeviceGuard guard(q.device());
-    Tensor qy = torch::empty_like(q), sy = torch::empty_like(s);
+    Tensor qy = torch::empty_like(q), sy = scales_for(q, s);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_layernorm_fwd((const int8_t *)q.data_ptr(), s.data_ptr(), g, b, m, r, (int)R, (int)C, sc, (int8_t *)qy.data_ptr(),
                               sy.data_ptr(), current_stream(q)),
@@ -303,7 +309,7 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor> layernorm_bwd(const Tensor &qx, co
     c10::DeviceGuard guard(qx.device());
     const size_t nbytes = jf_layernorm_bwd_workspace_bytes((int)R, (int)C);
     Tensor ws = scratch(qx, nbytes);
-    Tensor qdx = torch::empty_like(qx), sdx = torch::empty_like(sx);
+    Tensor qdx = torch::empty_like(qx), sdx = scales_for(qx, sx);
     Tensor dgamma = torch::empty({C}, qx.options().dtype(torch::kFloat32));
     OptTensor dbeta;
     if (want_dbeta) dbeta = torch::empty_like(dgamma);
@@ -383,14 +389,14 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor> layernorm_bwd_add(const Te
     const auto ao = rng(add_rounding, qx, R * C, add_seed, add_offset);
     if (C / QB > 64) {
         auto [qdx, sdx, dgamma, dbeta] = layernorm_bwd(qx, sx, qg, sg, gamma, mean, rstd, rounding, want_dbeta, so.first, so.second);
-        auto [y1, q, s, _m, _r] = add(x1, qdx, sdx, add_rounding, false, out_dtype, ao.first, ao.second);
+        auto [y1, q, s, _m, _r] = add(x1.view(qx.sizes()), qdx, sdx, add_rounding, false, out_dtype, ao.first, ao.second);
         return std::make_tuple(y1, q, s, dgamma, dbeta);
     }
     c10::DeviceGuard guard(qx.device());
     const size_t nbytes = jf_layernorm_bwd_workspace_bytes((int)R, (int)C);
     Tensor ws = scratch(qx, nbytes);
     Tensor y1 = torch::empty(qx.sizes(), x1.options().dtype(out_dtype));
-    Tensor q = torch::empty_like(qx), s = torch::empty_like(sx);
+    Tensor q = torch::empty_like(qx), s = scales_for(qx, sx);
     Tensor dgamma = torch::empty({C}, qx.options().dtype(torch::kFloat32));
     OptTensor dbeta;
     if (want_dbeta) dbeta = torch::empty_like(dgamma);
@@ -417,7 +423,7 @@ std::tuple<Tensor, Tensor> gelu_fwd(const Tensor &q, const Tensor &s, int64_t ap
     const int sc = block_tensor(q, s, "x", R, C);
     check_approx(approx);
     c10::DeviceGuard guard(q.device());
-    Tensor qy = torch::empty_like(q), sy = torch::empty_like(s);
+    Tensor qy = torch::empty_like(q), sy = scales_for(q, s);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_gelu_fwd((const int8_t *)q.data_ptr(), s.data_ptr(), (int)R, (int)C, sc, (int)approx, (float)amax_eps,
                          (int8_t *)qy.data_ptr(), sy.data_ptr(), current_stream(q)),
@@ -436,7 +442,7 @@ std::tuple<Tensor, Tensor> gelu_bwd(const Tensor &qx, const Tensor &sx, const Te
     check_approx(approx);
     check_rounding(rounding, true);
     c10::DeviceGuard guard(qx.device());
-    Tensor qy = torch::empty_like(qx), sy = torch::empty_like(sx);
+    Tensor qy = torch::empty_like(qx), sy = scales_for(qx, sx);
     const auto so = rng(rounding, qx, R * C, seed, offset);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_gelu_bwd((const int8_t *)qx.data_ptr(), sx.data_ptr(), (const int8_t *)qg.data_ptr(), sg.data_ptr(), (int)R, (int)C, sc,

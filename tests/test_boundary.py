@@ -527,3 +527,33 @@ def test_expanded_gradient_is_copied_not_rejected():
     assert fb.stride(0) == 32 and fb.is_contiguous() and torch.equal(fb, b)
     assert fa.data_ptr() == a.data_ptr() and fc.data_ptr() == c.data_ptr() and fc.stride(0) == 96
     assert tuple(q.shape) == (64, 96) and tuple(s.shape) == (2, 3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", [64, 2080])                   # (LayerNorm's backward with the add: one kernel, two kernels)
+def test_results_have_the_rank_of_the_codes(width):
+    """[B, T, C] codes with [B T/32, C/32] scales and the other way round: every result has the rank of the codes, as the values
+    of the flat call.  Sequences that are not whole blocks have no scales of that rank and are refused."""
+    import Nonlinear as NL
+    B, T, C = 2, 64, width
+    torch.manual_seed(3)
+    q, s = NL.int8_quantize(torch.randn(B * T, C, device="cuda"), 32)
+    g, sg = NL.int8_quantize(torch.randn(B * T, C, device="cuda"), 32)
+    w, m, v, x1 = torch.ones(C, device="cuda"), torch.zeros(B * T, device="cuda"), torch.ones(B * T, device="cuda"), torch.randn(B * T, C, device="cuda")
+
+    def all_ops(q, s, g, sg, x1):
+        return [*NL.int8_layernorm_forward(q, s, w, m, v, 32)[:2], *NL.int8_layernorm_backward(q, s, g, sg, w, 32, m, v)[:2],
+                *NL.int8_layernorm_backward_add(q, s, g, sg, w, 32, m, v, x1)[:3], *NL.int8_gelu_forward(q, s, 32),
+                *NL.int8_gelu_backward(q, s, g, sg, 32), *NL.int8_add_Ifp_Ig16_Ofp_Og(x1.view(q.shape), q, s, 32)]
+
+    flat = all_ops(q, s, g, sg, x1)
+    deep = all_ops(q.view(B, T, C), s, g.view(B, T, C), sg, x1)
+    back = all_ops(q, s.view(B, T // 32, C // 32), g, sg.view(B, T // 32, C // 32), x1.view(B, T, C))
+    for a, b, c in zip(flat, deep, back):
+        assert a.dim() == 2 and torch.equal(a, c) and b.shape == (B, a.shape[0] // B, a.shape[1]) and torch.equal(a, b.flatten(0, 1))
+    ragged = q.view(4, 32, C)[:3].reshape(2, 48, C)
+    for f in (lambda: NL.int8_layernorm_forward(ragged, s[:3], w, m[:96], v[:96], 32), lambda: NL.int8_gelu_forward(ragged, s[:3], 32),
+              lambda: NL.int8_layernorm_backward(ragged, s[:3], ragged, s[:3], w, 32, m[:96], v[:96]),
+              lambda: NL.int8_gelu_backward(ragged, s[:3], ragged, s[:3], 32)):
+        with pytest.raises(RuntimeError, match="multiple of 32"):
+            f()
