@@ -297,7 +297,7 @@ class QBlock(nn.Module):
             ws = [self.w_qkv, self.w_attn_proj, self.w_fc, self.w_mlp_proj]
             bs = [] if self.b_qkv is None else [self.b_qkv, self.b_attn_proj, self.b_fc, self.b_mlp_proj]
             # (a tuple: a module's backward hooks are called for tensors and tuples of them only)
-            return tuple(_jf.qblock(x.contiguous(), qx, sx, mean, rstd, [self.ln_1, self.ln_2] + ws, weight_codes.get_many(ws), bs,
+            return tuple(_jf.qblock(x, qx, sx, mean, rstd, [self.ln_1, self.ln_2] + ws, weight_codes.get_many(ws), bs,
                                     [weight_codes.get_bias(b) for b in bs], self.n_head, self.out_dtype))
         res, q, k, v = AttentionIn.apply(x, qx, sx, self.w_qkv, self.ln_1, mean, rstd, self.b_qkv)
         q, k, v = (t.view(B, T, self.n_head, C // self.n_head).transpose(1, 2) for t in (q, k, v))

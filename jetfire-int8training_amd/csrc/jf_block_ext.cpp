@@ -357,12 +357,16 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
 // (fp, codes as float8, scales, mean, rstd) of a block.  params: ln_1, ln_2, w_qkv, w_attn_proj, w_fc, w_mlp_proj (the
 // parameters: where their gradients go); codes: (codes, scales) of the four weights; biases: the four bias parameters and
 // their (float32 bias, max|bias|) pairs, or empty.
-variable_list qblock(const Tensor &x, const Tensor &qx, const Tensor &sx, const Tensor &mean, const Tensor &rstd, const std::vector<Tensor> &params,
+variable_list qblock(const Tensor &x_, const Tensor &qx_, const Tensor &sx_, const Tensor &mean_, const Tensor &rstd_, std::vector<Tensor> params,
                      const std::vector<std::tuple<Tensor, Tensor>> &codes, const std::vector<Tensor> &bias_params,
                      const std::vector<std::tuple<Tensor, Tensor>> &bias_pairs, int64_t heads, torch::ScalarType out_dtype)
 {
     TORCH_CHECK(params.size() == 6 && codes.size() == 4 && (bias_params.empty() || bias_params.size() == 4) && bias_pairs.size() == bias_params.size(),
                 "qblock: expected 6 parameters, 4 coded weights and 0 or 4 biases");
+    // strides, and types of the statistics, are brought to what the kernels read, as the separate operators do
+    const Tensor x = x_.contiguous(), qx = qx_.contiguous(), sx = sx_.contiguous();
+    const Tensor mean = mean_.to(torch::kFloat32).contiguous(), rstd = rstd_.to(torch::kFloat32).contiguous();
+    params[0] = params[0].contiguous(); params[1] = params[1].contiguous();
     std::vector<WeightOperand> w;
     std::vector<BiasOperand> bias;
     for (auto &p : codes) w.push_back({std::get<0>(p), std::get<1>(p)});

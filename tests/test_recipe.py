@@ -458,3 +458,39 @@ def test_block_without_a_backward_keeps_nothing_for_one():
     fp, q, s, _, _ = blk(*args)
     recipe.StreamEnd.apply(fp, q, s).backward(torch.ones_like(fp))
     assert blk.w_fc.grad.isfinite().all() and blk.w_fc.grad.abs().sum() > 0 and blk.w_qkv.grad is None
+
+
+def test_block_takes_strided_operands_and_statistics_of_other_types():
+    """Codes, scales, residual, statistics and LayerNorm weights that are not contiguous, or statistics in float64: the same bits."""
+    import recipe
+    torch.manual_seed(13)
+    B, T, C, H = 2, 64, 128, 4
+    blk = recipe.QBlock(C, H).cuda()
+    args = block_arguments(B, T, C, H)[:5]
+    w = torch.randn(B, T, C, device="cuda")
+
+    def strided(t):                                                # the same values, every other element of the storage
+        if t.element_size() == 1:
+            return torch.stack([t.view(torch.int8)] * 2, -1)[..., 0].view(t.dtype)
+        return torch.stack([t, t], -1)[..., 0]
+
+    def run(blk, args):
+        torch.manual_seed(14)
+        for p in blk.parameters():
+            p.grad = None
+        x = args[0].detach().clone(memory_format=torch.preserve_format).requires_grad_(True)
+        fp, q, s, m, r = blk(x, *args[1:])
+        recipe.StreamEnd.apply(fp, q, s).backward(w)
+        return [fp, q.view(torch.int8), s, m, r, x.grad] + [p.grad for p in blk.parameters()]
+
+    want = run(blk, args)
+    odd = recipe.QBlock(C, H).cuda()
+    odd.load_state_dict(blk.state_dict())
+    for name in ("ln_1", "ln_2"):
+        setattr(odd, name, torch.nn.Parameter(strided(getattr(odd, name).detach())))
+        assert not getattr(odd, name).is_contiguous()
+    views = [strided(t.detach()) for t in args]
+    assert not any(t.is_contiguous() for t in views)
+    for other in (views, [*views[:3], views[3].double(), views[4].double()]):
+        for i, (a, b) in enumerate(zip(want, run(odd, other))):
+            assert torch.equal(a, b), i
