@@ -284,7 +284,10 @@ class QBlock(nn.Module):
 
     def _one_node(self, x, sx):
         """Whether the block runs as the extension's single autograd node (its attention kernels take binary16 heads 32 or
-        64 wide, its LayerNorm backward rows of up to 2048 columns)."""
+        64 wide, its LayerNorm backward rows of up to 2048 columns).  Not under an autocast to another type: that is asked of the
+        attention, which torch's own operator heeds."""
+        if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.float16:
+            return False
         B, T, C = x.shape
         return (C // self.n_head in (32, 64) and T % QB == 0 and C <= 2048 and T * 3 * C < 2 ** 30 and sx.dtype == torch.float16
                 and self.ln_1.dtype == self.ln_2.dtype == torch.float32

@@ -494,3 +494,26 @@ def test_block_takes_strided_operands_and_statistics_of_other_types():
     for other in (views, [*views[:3], views[3].double(), views[4].double()]):
         for i, (a, b) in enumerate(zip(want, run(odd, other))):
             assert torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_autocast_reaches_the_attention(dtype, monkeypatch):
+    """The recipe's attention runs in binary16; under an autocast to another type it is torch's attention that is called, within
+    the autocast (here a stand-in that records it)."""
+    import recipe
+    torch.manual_seed(15)
+    calls = []
+
+    def attention(q, k, v, is_causal):
+        calls.append((torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda"), is_causal))
+        return v.to(torch.get_autocast_dtype("cuda"))
+    monkeypatch.setattr(recipe.F, "scaled_dot_product_attention", attention)
+    blk = recipe.QBlock(128, 4).cuda()
+    args = block_arguments()[:5]
+    with torch.no_grad():
+        plain = blk(*args)
+        assert not calls
+        with torch.autocast("cuda", dtype=dtype):
+            cast = blk(*args)
+    assert calls == ([] if dtype == torch.float16 else [(True, dtype, True)])
+    assert cast[0].isfinite().all() and torch.equal(cast[0], plain[0]) == (dtype == torch.float16)
