@@ -289,7 +289,8 @@ class QBlock(nn.Module):
         if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.float16:
             return False
         B, T, C = x.shape
-        return (C // self.n_head in (32, 64) and T % QB == 0 and C <= 2048 and T * 3 * C < 2 ** 30 and sx.dtype == torch.float16
+        biased = sum(b is not None for b in (self.b_qkv, self.b_attn_proj, self.b_fc, self.b_mlp_proj))
+        return (biased in (0, 4) and C // self.n_head in (32, 64) and T % QB == 0 and C <= 2048 and T * 3 * C < 2 ** 30 and sx.dtype == torch.float16
                 and self.ln_1.dtype == self.ln_2.dtype == torch.float32
                 and self.w_qkv.dtype == self.w_attn_proj.dtype == self.w_fc.dtype == self.w_mlp_proj.dtype)
 

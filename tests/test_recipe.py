@@ -517,3 +517,26 @@ def test_autocast_reaches_the_attention(dtype, monkeypatch):
             cast = blk(*args)
     assert calls == ([] if dtype == torch.float16 else [(True, dtype, True)])
     assert cast[0].isfinite().all() and torch.equal(cast[0], plain[0]) == (dtype == torch.float16)
+
+
+def test_block_with_some_of_its_biases():
+    """A block some of whose biases were taken out applies the ones that are left."""
+    import recipe
+    torch.manual_seed(16)
+    blk = recipe.QBlock(128, 4, torch.float32, True).cuda()
+    args = block_arguments()[:5]
+    with torch.no_grad():
+        for b in (blk.b_qkv, blk.b_attn_proj, blk.b_fc, blk.b_mlp_proj):
+            b.normal_()
+        for keep in (("b_qkv",), ("b_attn_proj", "b_mlp_proj"), ("b_qkv", "b_fc", "b_mlp_proj")):
+            some, zeros = recipe.QBlock(128, 4, torch.float32, True).cuda(), recipe.QBlock(128, 4, torch.float32, True).cuda()
+            for other in (some, zeros):
+                other.load_state_dict(blk.state_dict())
+            for name in ("b_qkv", "b_attn_proj", "b_fc", "b_mlp_proj"):
+                if name not in keep:
+                    setattr(some, name, None)
+                    getattr(zeros, name).zero_()
+            got, want = some(*args), zeros(*args)
+            none = recipe.QBlock(128, 4).cuda()
+            none.load_state_dict({n: p for n, p in blk.state_dict().items() if not n.startswith("b_")})
+            assert cos(got[0], want[0]) > 0.9999 and cos(none(*args)[0], want[0]) < 0.999
