@@ -311,8 +311,8 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         constexpr int RM = JF_SCALES_ROWMAJOR, KM = JF_SCALES_KMAJOR, F16 = JF_SCALE_F16, SR = JF_ROUND_STOCHASTIC;
         auto codes = [](const Tensor &a) { return (const int8_t *)a.data_ptr(); };
         // The weight gradients run together at the end: one launch has tiles for the whole chip where each of the four alone
-        // needs a K split and leaves a last round half empty, and one more adds what is left to add, the LayerNorm weights'
-        // gradients included.
+        // leaves a last round half empty, and one more adds what is left to add, the parts of K splits and the LayerNorm weights'
+        // gradients.
         const int8_t *wg[4], *wx[4];
         const void *wgs[4], *wxs[4];
         auto wgrad = [&](int i, const int8_t *g, const void *gs, const int8_t *xq, const void *xs) {

@@ -25,6 +25,7 @@
 // needs once per stage and reads the products from a private LDS patch.
 #include "jf_device.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -998,22 +999,27 @@ __global__ __launch_bounds__(gemm_threads(WBM, WGM, WGN), WGPC * gemm_threads(WB
     igemm_body<EPI, ST, WBM, WGM, WGN, NSTAGE, WGPC, BKN, AKM, PROF>(p, logical_workgroup());
 }
 
-// Several weight gradients over the same tokens in one launch (jf_wgrad_many): the work of one follows the other's.
+// Several weight gradients over the same tokens in one launch (jf_wgrad_many).  Every XCD gets one contiguous run of each problem's
+// work, one problem after the other, so that the XCDs finish together although the parts of the problems differ in length.  (One
+// run over all problems: GPT-2 XL's four, one of them in parts a third as long, took 60 us more than the 500 they take.)
 constexpr int WGRAD_MAX = 4;
 struct GemmGroup {
     GemmArgs g[WGRAD_MAX];
-    int end[WGRAD_MAX];       // first workgroup behind problem k
+    int end[WGRAD_MAX];       // first workgroup behind problem k, of an XCD's: ceil(work / 8) for each problem
     int n;
 };
 template <typename ST>
 __global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp)
 {
-    const int logical = logical_workgroup();
+    const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
     int k = 0, begin = 0;
 #pragma unroll
     for (int i = 1; i < WGRAD_MAX; ++i)
-        if (i < grp.n && logical >= grp.end[i - 1]) { k = i; begin = grp.end[i - 1]; }
-    igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0>(grp.g[k], logical - begin);
+        if (i < grp.n && at >= grp.end[i - 1]) { k = i; begin = grp.end[i - 1]; }
+    const GemmArgs &p = grp.g[k];
+    const int work = p.tiles_m * p.tiles_n * p.splits, per = work >> 3, rem = work & 7, idx = at - begin;
+    if (idx >= per + (xcd < rem ? 1 : 0)) return;
+    igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0>(p, xcd * per + (xcd < rem ? xcd : rem) + idx);
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -1171,7 +1177,8 @@ struct WgradFinish {
     const float *terms[WGRAD_MAX];                             // [strips][width]
     float *sum[WGRAD_MAX];
     int width[WGRAD_MAX], cend[WGRAD_MAX];                     // first workgroup behind column sum k (32 columns each)
-    int n, ncol, splits, strips, out_dtype;
+    int splits[WGRAD_MAX];
+    int n, ncol, strips, out_dtype;
 };
 __global__ __launch_bounds__(1024) void wgrad_finish_kernel(WgradFinish f)
 {
@@ -1182,7 +1189,7 @@ __global__ __launch_bounds__(1024) void wgrad_finish_kernel(WgradFinish f)
 #pragma unroll
         for (int i = 1; i < WGRAD_MAX; ++i)
             if (i < f.n && wg >= f.end[i - 1]) { k = i; begin = f.end[i - 1]; }
-        reduce_splits(f.part[k], f.count[k], f.splits, f.out[k], f.out_dtype, ((size_t)(wg - begin) * 1024 + threadIdx.x) * 4);
+        reduce_splits(f.part[k], f.count[k], f.splits[k], f.out[k], f.out_dtype, ((size_t)(wg - begin) * 1024 + threadIdx.x) * 4);
         return;
     }
     begin = nred;
@@ -1241,13 +1248,22 @@ static void splitk_plan(int M, int N, int K, int request, int &splits, int &kb_p
     splits = (nkb + kb_per_split - 1) / kb_per_split;
 }
 
-// K split of a group of weight gradients (one for all of them: they share K).  The launch takes, on the fullest CU, as many
-// tiles as fall to it times their K blocks: about 0.27 us per block for a lone tile and 0.2 us per tile beyond (GPT-2 XL and
-// small gradients), 3 us of ramp and epilogue per pair of tiles; parts cost a write and a read of every partial sum at about
-// 8 TB/s (they stay in the caches).  One split for a GPT-2 block at 8 x 1024 or 12 x 1024 tokens (XL: 532 us in four launches
-// -> 500; small: 225 us with four sums of parts -> 180), four for a 256-wide one over 1024.  Parts are at least 8 K blocks (two stages) of at least 16.
-static void wgrad_group_plan(int n, const int *M, const int *N, int K, int &splits, int &kb_per_split)
+// K splits of a group of weight gradients.  First one for all of them, by time: the launch takes, on the fullest CU, as many tiles as
+// fall to it times their K blocks: about 0.27 us per block for a lone tile and 0.2 us per tile beyond (GPT-2 XL and small
+// gradients), 3 us of ramp and epilogue per pair of tiles; parts cost a write and a read of every partial sum at about 8 TB/s (they
+// stay in the caches).  Parts are at least 8 K blocks (two stages) of at least 16.
+// Then, by rounding: the squared error of the sum of p parts of kb blocks grows as kb + p (each addition rounds the partial sum it has
+// reached), and no gradient is summed in an order that rounds more than its own launch would (splitk_plan): where the split of the
+// group is such a one, the gradient keeps its own.  A 256-wide block over 1024 tokens takes four parts of 8 blocks where a launch of
+// its own takes two of 16 (error against float64 8.3e-8 -> 7.2e-8 relative); a GPT-2 block at 8 x 1024 (XL) or 12 x 1024 tokens (small), which
+// unsplit would be fastest (small: 180 us, but 3.5e-7 where the parts give 1.2e-7 to 2.1e-7), keeps each gradient's own parts.  Launch and sums of the parts: XL 511
+// us, small 206, where four launches of their own and their sums took 532 and 225.
+struct WgradPlan {
+    int splits[WGRAD_MAX], kb_per_split[WGRAD_MAX];
+};
+static void wgrad_group_plan(int n, const int *M, const int *N, int K, WgradPlan &plan)
 {
+    int splits, kb_per_split;
     const int nkb = K / QB;
     long tiles = 0;
     double elems = 0;
@@ -1262,6 +1278,10 @@ static void wgrad_group_plan(int n, const int *M, const int *N, int K, int &spli
         const long per_cu = (tiles * parts + cu_count() - 1) / cu_count();
         const double t = kb * (0.2 * per_cu + (per_cu & 1 ? 0.07 : 0.0)) + 3.0 * ((per_cu + 1) / 2) + (parts > 1 ? parts * elems * 8 / 8e6 : 0.0);
         if (s == 1 || t < best) { best = t; splits = parts; kb_per_split = kb; }
+    }
+    for (int i = 0; i < n; ++i) {
+        splitk_plan(M[i], N[i], K, 0, plan.splits[i], plan.kb_per_split[i]);
+        if (kb_per_split + splits <= plan.kb_per_split[i] + plan.splits[i]) { plan.splits[i] = splits; plan.kb_per_split[i] = kb_per_split; }
     }
 }
 
@@ -1458,10 +1478,11 @@ int jf_igemm_block_fp(const int8_t *A, const int8_t *B, const void *sa, const vo
 size_t jf_wgrad_many_workspace_bytes(int n, const int *M, const int *N, int K)
 {
     if (n < 1 || n > WGRAD_MAX || !M || !N || !mult32(K)) return 0;
-    int splits, kb;
-    wgrad_group_plan(n, M, N, K, splits, kb);
+    WgradPlan plan;
+    wgrad_group_plan(n, M, N, K, plan);
     size_t bytes = 0;
-    for (int i = 0; splits > 1 && i < n; ++i) bytes += (size_t)splits * (size_t)M[i] * (size_t)N[i] * sizeof(float);
+    for (int i = 0; i < n; ++i)
+        if (plan.splits[i] > 1) bytes += (size_t)plan.splits[i] * (size_t)M[i] * (size_t)N[i] * sizeof(float);
     return bytes;
 }
 
@@ -1471,7 +1492,6 @@ int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const in
 {
     if (n < 1 || n > WGRAD_MAX || ncol < 0 || ncol > WGRAD_MAX) return JF_ERR_SHAPE;
     if (!G || !SG || !X || !SX || !out || !M || !N || (ncol && (!terms || !width || !sum))) return JF_ERR_NULL;
-    int splits, kb_per;
     for (int i = 0; i < n; ++i) {
         int rc = block_fp_check(G[i], X[i], SG[i], SX[i], out[i], M[i], N[i], K, JF_A_KM, JF_B_KN, scale_dtype, out_dtype);
         if (rc) return rc;
@@ -1481,24 +1501,33 @@ int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const in
         if (!mult32(width[i])) return JF_ERR_SHAPE;
     }
     if (!device_is_gfx950()) return JF_ERR_DEVICE;
-    wgrad_group_plan(n, M, N, K, splits, kb_per);
-    if (splits > 1 && (!workspace || !aligned16(workspace) || workspace_bytes < jf_wgrad_many_workspace_bytes(n, M, N, K))) return JF_ERR_WORKSPACE;
+    WgradPlan plan;
+    wgrad_group_plan(n, M, N, K, plan);
+    const size_t need = jf_wgrad_many_workspace_bytes(n, M, N, K);
+    if (need && (!workspace || !aligned16(workspace) || workspace_bytes < need)) return JF_ERR_WORKSPACE;
+    int order[WGRAD_MAX];                                      // longest parts first: the short ones even out the end of the launch
+    for (int i = 0; i < n; ++i) order[i] = i;
+    std::stable_sort(order, order + n, [&](int a, int b) { return plan.kb_per_split[a] > plan.kb_per_split[b]; });
     GemmGroup grp = {};
     WgradFinish fin = {};
     float *part = (float *)workspace;
     long wgs = 0, fwgs = 0;
-    for (int i = 0; i < n; ++i) {
-        GemmArgs &a = grp.g[i];
+    int longest = 0;
+    for (int j = 0; j < n; ++j) {
+        const int i = order[j], splits = plan.splits[i];
+        GemmArgs &a = grp.g[j];
         a.A = G[i]; a.B = X[i]; a.sa = SG[i]; a.sb = SX[i]; a.C = splits > 1 ? (void *)part : out[i];
-        a.M = M[i]; a.N = N[i]; a.K = K; a.lda = M[i]; a.ldb = N[i]; a.out_dtype = out_dtype; a.splits = splits; a.kb_per_split = kb_per;
+        a.M = M[i]; a.N = N[i]; a.K = K; a.lda = M[i]; a.ldb = N[i]; a.out_dtype = out_dtype; a.splits = splits; a.kb_per_split = plan.kb_per_split[i];
         a.sa_ks = M[i] / QB; a.sa_is = 1; a.sb_ks = N[i] / QB; a.sb_is = 1;
         a.tiles_m = (M[i] + 127) / 128; a.tiles_n = (N[i] + 127) / 128;
-        wgs += (long)a.tiles_m * a.tiles_n * splits;
-        grp.end[i] = (int)wgs;
+        wgs += ((long)a.tiles_m * a.tiles_n * splits + 7) / 8;
+        grp.end[j] = (int)wgs;
+        if (plan.kb_per_split[i] > longest) longest = plan.kb_per_split[i];
         if (splits > 1) {
             const size_t count = (size_t)M[i] * (size_t)N[i];
             fwgs += (long)((count + 4095) / 4096);
-            fin.part[i] = part; fin.out[i] = out[i]; fin.count[i] = count; fin.end[i] = (int)fwgs;
+            fin.part[fin.n] = part; fin.out[fin.n] = out[i]; fin.count[fin.n] = count; fin.splits[fin.n] = splits; fin.end[fin.n] = (int)fwgs;
+            ++fin.n;
             part += (size_t)splits * count;
         }
     }
@@ -1506,10 +1535,11 @@ int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const in
         fwgs += width[i] / QB;
         fin.terms[i] = terms[i]; fin.sum[i] = sum[i]; fin.width[i] = width[i]; fin.cend[i] = (int)fwgs;
     }
+    wgs *= 8;
     if (wgs > 0x7fffffffL || fwgs > 0x7fffffffL) return JF_ERR_SHAPE;
     grp.n = n;
-    fin.n = splits > 1 ? n : 0; fin.ncol = ncol; fin.splits = splits; fin.strips = K / QB; fin.out_dtype = out_dtype;
-    const int pace = pace_of(wgs, 2L * cu_count(), kb_per * QB);
+    fin.ncol = ncol; fin.strips = K / QB; fin.out_dtype = out_dtype;
+    const int pace = pace_of(wgs, 2L * cu_count(), longest * QB);
     for (int i = 0; i < n; ++i) grp.g[i].pace = pace;
     hipStream_t st = (hipStream_t)stream;
     int rc = scale_dtype == JF_SCALE_F16 ? launch_wgrad_group<half_t>(grp, (unsigned)wgs, st) : launch_wgrad_group<float>(grp, (unsigned)wgs, st);

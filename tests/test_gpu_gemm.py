@@ -522,3 +522,23 @@ def test_weight_gradients_in_one_launch(jf, oracle, K, widths, f16, out):
     for t, s in zip(terms, sums):
         np.testing.assert_allclose(s.cpu().numpy(), t.astype(np.float64).sum(0), atol=1e-5)
     assert jf.wgrad_many(d(gs[:1]), d(xs[:1]), out)[0][0].shape == got[0].shape
+
+
+@pytest.mark.parametrize("C,K", [(256, 1024), (768, 12288), (1600, 8192), (768, 1248), (512, 4096), (192, 2048)])
+def test_weight_gradients_in_one_launch_round_no_more_than_alone(jf, C, K):
+    """The gradients of a block's four layers against float64: the one launch sums K in an order whose rounding error is no larger
+    than that of each gradient in a launch of its own (2 % for the scatter of a norm over a million rounding errors)."""
+    print(f"case C={C} K={K}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(C + K)
+    codes = lambda c: torch.randint(-127, 128, (K, c), device="cuda", dtype=torch.int8, generator=gen)  # noqa: E731
+    scales = lambda c: (1 + torch.rand(K // QB, c // QB, device="cuda", generator=gen))  # noqa: E731
+    widths = [(3 * C, C), (C, C), (4 * C, C), (C, 4 * C)]
+    gs, xs = [(codes(m), scales(m)) for m, _ in widths], [(codes(n), scales(n)) for _, n in widths]
+    got, _ = jf.wgrad_many(gs, xs)
+    value = lambda q, s: q.double() * s.double().repeat_interleave(QB, 0).repeat_interleave(QB, 1)  # noqa: E731
+    for (g, sg), (x, sx), many in zip(gs, xs, got):
+        alone = jf.igemm_block_fp(g, x, sg, sx, jf.B_KN, torch.float32, a_layout=jf.A_KM, splitk=0)
+        exact = value(g, sg).t().contiguous() @ value(x, sx)
+        error = lambda o: float((o.double() - exact).norm() / exact.norm())  # noqa: E731
+        print(f"  {g.shape[1]} x {x.shape[1]}: alone {error(alone):.3e}, together {error(many):.3e}", flush=True)
+        assert error(many) <= 1.02 * error(alone) and error(alone) < 1e-6

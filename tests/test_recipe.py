@@ -285,7 +285,9 @@ def test_weight_codes_are_cached_per_weight_version():
 
 
 @pytest.mark.parametrize("B,T,C,H,bias,res,out", [(1, 32, 64, 2, False, torch.float32, torch.float32), (2, 96, 192, 3, True, torch.bfloat16, torch.float32),
-                                                  (3, 160, 128, 4, False, torch.float32, torch.bfloat16)])
+                                                  (3, 160, 128, 4, False, torch.float32, torch.bfloat16),
+                                                  # 64 K blocks: the weight gradients are sums of four parts, together as alone
+                                                  (2, 1024, 512, 8, True, torch.bfloat16, torch.bfloat16)])
 def test_block_as_one_node_equals_the_functions(B, T, C, H, bias, res, out):
     """QBlock's single node runs the kernels of AttentionIn, the attention and AttentionOutMLP in their order with their noise
     counters: outputs and every gradient are the same bits."""
