@@ -384,7 +384,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void attn_dkv_kernel(Attn
     auto load = [&](int t) {
         io.load(lds + (t & 1) * 2 * IO::TILE, qp, a.ld, gp, a.H * D, t * ATT_ROWS, a.T - 1);
         if (wave == 0) {
-            const int r = t * ATT_ROWS + lane;
+            // (the lane number is made anew: held over the loop it is one register too many, and its reload waits for the whole tile)
+            unsigned l;
+            asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+            const int r = t * ATT_ROWS + (int)l;
             const unsigned off = (unsigned)(r < a.T ? r : a.T - 1) * 4u, dst = stat_lds + (t & 1) * (2 * ATT_ROWS * 4);
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(lsep), "s"(dst) : "memory", "m0");
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
