@@ -46,6 +46,13 @@ struct AttnArgs {
 
 constexpr int ATT_ROWS = 64;        // rows of a shared tile
 constexpr int ATT_SUB = 32;         // rows of one step
+// Waves of a workgroup, sharing every tile: 128 rows, at every size.  Fewer waves make more workgroups where there are few, but each
+// then loads its tiles alone.  Measured with one, two and four waves, us (forward | gradient, heads 64 wide): 4 heads of 256 rows
+// 9.8 9.5 7.7 | 25.7 25.1 20.7, 36 of 416 15.0 13.5 10.2 | 39.0 35.8 27.4, 24 of 1024 29.4 27.9 21.0 | 75.3 71.1 51.9, 144 of 1024
+// 83.0 51.9 36.8 | 213 140 107; heads 32 wide in the same order.  Fewer waves are ahead by at most 1.3 us, and only where a sequence
+// has 32 or 64 rows.
+constexpr int NW = 4;
+constexpr int WG_ROWS = 32 * NW;
 
 // Workgroup -> (head, block of rows).  Workgroups are dealt to the 8 XCDs in turn: the blocks of one head stay on one XCD
 // (its K and V are read by all of them), and the longest blocks start first.
@@ -66,7 +73,7 @@ template <int D> __device__ __forceinline__ int swz(int r)
     return (r >> 2) & 3;
 }
 
-template <int D, int NW> struct TileIO {
+template <int D> struct TileIO {
     static constexpr int CPR = D / 8, ROWB = D * 2, TILE = ATT_ROWS * ROWB;
     static constexpr int RPI = 64 / CPR;                       // rows one load instruction of a wave moves
     static constexpr int INSTR = ATT_ROWS / RPI;               // load instructions per tensor
@@ -187,13 +194,13 @@ __device__ __forceinline__ void quantize_t(const v16f &x, int8_t *codes, half_t 
     if (lane == 0) scales[(size_t)(row / QB) * (C / QB) + col / QB] = (half_t)s;
 }
 
-template <int D, int NW, bool QUANT>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_fwd_kernel(AttnArgs a)
+template <int D, bool QUANT>
+__global__ __launch_bounds__(64 * NW, 4) void attn_fwd_kernel(AttnArgs a)
 {
-    using IO = TileIO<D, NW>;
+    using IO = TileIO<D>;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
-    const int nblk = (a.T + 32 * NW - 1) / (32 * NW);
+    const int nblk = (a.T + WG_ROWS - 1) / WG_ROWS;
     int bh, blk;
     if (!attn_work(a, nblk, true, bh, blk)) return;
     const int b = bh / a.H, head = bh - b * a.H;
@@ -201,7 +208,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_fwd_kernel(Attn
     const half_t *kp = a.k + first, *vp = a.v + first;
     const IO io(lane, wave);
     const unsigned lds = (unsigned)(uintptr_t)(lds_byte *)smem;
-    const int q0 = blk * 32 * NW + 32 * wave, qend = (blk + 1) * 32 * NW < a.T ? (blk + 1) * 32 * NW : a.T;
+    const int q0 = blk * WG_ROWS + 32 * wave, qend = (blk + 1) * WG_ROWS < a.T ? (blk + 1) * WG_ROWS : a.T;
     const int nt = (qend + ATT_ROWS - 1) / ATT_ROWS;
     const bool active = q0 < a.T;
     const int query = q0 + (lane & 31);
@@ -279,13 +286,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_fwd_kernel(Attn
 }
 
 // dQ by blocks of queries; leaves delta for the dK/dV kernel
-template <int D, int NW, bool QUANT>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_dq_kernel(AttnArgs a)
+template <int D, bool QUANT>
+__global__ __launch_bounds__(64 * NW, 4) void attn_dq_kernel(AttnArgs a)
 {
-    using IO = TileIO<D, NW>;
+    using IO = TileIO<D>;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
-    const int nblk = (a.T + 32 * NW - 1) / (32 * NW);
+    const int nblk = (a.T + WG_ROWS - 1) / WG_ROWS;
     int bh, blk;
     if (!attn_work(a, nblk, true, bh, blk)) return;
     const int b = bh / a.H, head = bh - b * a.H;
@@ -293,7 +300,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_dq_kernel(AttnA
     const half_t *kp = a.k + first, *vp = a.v + first;
     const IO io(lane, wave);
     const unsigned lds = (unsigned)(uintptr_t)(lds_byte *)smem;
-    const int q0 = blk * 32 * NW + 32 * wave, qend = (blk + 1) * 32 * NW < a.T ? (blk + 1) * 32 * NW : a.T;
+    const int q0 = blk * WG_ROWS + 32 * wave, qend = (blk + 1) * WG_ROWS < a.T ? (blk + 1) * WG_ROWS : a.T;
     const int nt = (qend + ATT_ROWS - 1) / ATT_ROWS;
     const bool active = q0 < a.T;
     const int query = active ? q0 + (lane & 31) : 0;
@@ -361,14 +368,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 4 : 1) void attn_dq_kernel(AttnA
 }
 
 // dK and dV by blocks of keys
-template <int D, int NW, bool QUANT>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void attn_dkv_kernel(AttnArgs a)
+template <int D, bool QUANT>
+__global__ __launch_bounds__(64 * NW, 3) void attn_dkv_kernel(AttnArgs a)
 {
-    using IO = TileIO<D, NW>;
+    using IO = TileIO<D>;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
     __shared__ __attribute__((aligned(16))) float stat[2][2][ATT_ROWS];        // lse, delta of the tile's queries
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
-    const int nblk = (a.T + 32 * NW - 1) / (32 * NW);
+    const int nblk = (a.T + WG_ROWS - 1) / WG_ROWS;
     int bh, blk;
     if (!attn_work(a, nblk, false, bh, blk)) return;
     const int b = bh / a.H, head = bh - b * a.H;
@@ -377,8 +384,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void attn_dkv_kernel(Attn
     const float *lsep = a.lse + (size_t)bh * a.T, *dlp = a.delta + (size_t)bh * a.T;
     const IO io(lane, wave);
     const unsigned lds = (unsigned)(uintptr_t)(lds_byte *)smem, stat_lds = (unsigned)(uintptr_t)(lds_byte *)stat;
-    const int k0 = blk * 32 * NW + 32 * wave;
-    const int t0 = blk * 32 * NW / ATT_ROWS, nt = (a.T + ATT_ROWS - 1) / ATT_ROWS;
+    const int k0 = blk * WG_ROWS + 32 * wave;
+    const int t0 = blk * WG_ROWS / ATT_ROWS, nt = (a.T + ATT_ROWS - 1) / ATT_ROWS;
     const bool active = k0 < a.T;
     const int key = active ? k0 + (lane & 31) : 0;
     auto load = [&](int t) {
@@ -483,28 +490,13 @@ static int attn_check(const void *q, const void *k, const void *v, int ld, int B
     return device_is_gfx950() ? JF_OK : JF_ERR_DEVICE;
 }
 
-// Rows per workgroup: 128 (four waves share every tile) unless that leaves compute units idle
-static int attn_waves(int B, int H, int T)
-{
-    const long blocks = (long)B * H;
-    if (blocks * ((T + 127) / 128) >= 512) return 4;
-    return blocks * ((T + 63) / 64) >= 512 ? 2 : 1;
-}
-static unsigned attn_grid(int B, int H, int T, int nw) { return 8u * ((B * H + 7) / 8) * ((T + 32 * nw - 1) / (32 * nw)); }
-
-#define JF_ATT_Q(KERN, D, NW, a, grid, st)                                                                                   \
+#define JF_ATT_D(KERN, D, a, st)                                                                                            \
     do {                                                                                                                    \
-        if ((a).cq) hipLaunchKernelGGL((KERN<D, NW, true>), dim3(grid), dim3(64 * NW), 0, st, a);                           \
-        else hipLaunchKernelGGL((KERN<D, NW, false>), dim3(grid), dim3(64 * NW), 0, st, a);                                 \
+        const unsigned grid = 8u * (((a).B * (a).H + 7) / 8) * (((a).T + WG_ROWS - 1) / WG_ROWS);                           \
+        if ((a).cq) hipLaunchKernelGGL((KERN<D, true>), dim3(grid), dim3(64 * NW), 0, st, a);                               \
+        else hipLaunchKernelGGL((KERN<D, false>), dim3(grid), dim3(64 * NW), 0, st, a);                                     \
     } while (0)
-#define JF_ATT_D(KERN, D, nw, a, st)                                                                                        \
-    do {                                                                                                                    \
-        const unsigned grid = attn_grid((a).B, (a).H, (a).T, nw);                                                           \
-        if (nw == 4) JF_ATT_Q(KERN, D, 4, a, grid, st);                                                                     \
-        else if (nw == 2) JF_ATT_Q(KERN, D, 2, a, grid, st);                                                                \
-        else JF_ATT_Q(KERN, D, 1, a, grid, st);                                                                             \
-    } while (0)
-#define JF_ATT(KERN, D, nw, a, st) do { if (D == 64) JF_ATT_D(KERN, 64, nw, a, st); else JF_ATT_D(KERN, 32, nw, a, st); } while (0)
+#define JF_ATT(KERN, D, a, st) do { if (D == 64) JF_ATT_D(KERN, 64, a, st); else JF_ATT_D(KERN, 32, a, st); } while (0)
 
 }  // namespace jf
 
@@ -521,8 +513,7 @@ static int attention_fwd(const void *q, const void *k, const void *v, int ld, in
     a.q = (const half_t *)q; a.k = (const half_t *)k; a.v = (const half_t *)v; a.ld = ld;
     a.out = (half_t *)out; a.lse = lse; a.B = B; a.H = H; a.T = T; a.scale = scale;
     a.cq = codes; a.cs = (half_t *)scales;
-    const int nw = attn_waves(B, H, T);
-    JF_ATT(attn_fwd_kernel, D, nw, a, (hipStream_t)stream);
+    JF_ATT(attn_fwd_kernel, D, a, (hipStream_t)stream);
     return (int)hipGetLastError();
 }
 
@@ -540,9 +531,8 @@ static int attention_bwd(const void *q, const void *k, const void *v, int ld, co
     a.o = (const half_t *)out; a.go = (const half_t *)gout; a.lse = const_cast<float *>(lse); a.delta = delta;
     a.gq = (half_t *)gq; a.gk = (half_t *)gk; a.gv = (half_t *)gv; a.ldg = ldg; a.B = B; a.H = H; a.T = T; a.scale = scale;
     a.cq = codes; a.cs = (half_t *)scales; a.seed = seed; a.offset = offset;
-    const int nw = attn_waves(B, H, T);
-    JF_ATT(attn_dq_kernel, D, nw, a, (hipStream_t)stream);
-    JF_ATT(attn_dkv_kernel, D, nw, a, (hipStream_t)stream);
+    JF_ATT(attn_dq_kernel, D, a, (hipStream_t)stream);
+    JF_ATT(attn_dkv_kernel, D, a, (hipStream_t)stream);
     return (int)hipGetLastError();
 }
 

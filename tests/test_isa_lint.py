@@ -97,5 +97,5 @@ def test_main_loops_do_not_spill(gemm_isa):
 def test_attention_tile_loops_do_not_spill(attention_isa):
     """A reload inside a tile loop would wait for the next tile's loads as well (values are parked across the loop of the dK/dV
     kernel with heads 64 wide)."""
-    assert sum("v_mfma_f32_32x32x16_f16" in line for line in attention_isa) > 500
+    assert sum("v_mfma_f32_32x32x16_f16" in line for line in attention_isa) >= 200
     _no_scratch_in_loops(attention_isa)
