@@ -1,5 +1,5 @@
 """The recipe's causal attention kernels against attention evaluated in float32 on the CPU, at the edges of their tiles: one
-row block, ragged last tiles, one, two and four waves per workgroup, head counts that do not divide by the 8 XCDs, operands
+row block, ragged last tiles, workgroups with waves that have no rows, head counts that do not divide by the 8 XCDs, operands
 that are column ranges of one tensor."""
 import pytest
 import torch
