@@ -301,8 +301,8 @@ int jf_rowstats_finish(const float *rowsum, const float *rowsq, int R, int parts
 
 /* Up to 4 weight gradients over the same K tokens in one launch: out[i] [M[i], N[i]] = G[i]^T X[i] with G[i] codes [K, M[i]],
  * X[i] codes [K, N[i]] and scales in the block tensors' own layout ([K/32, M[i]/32], [K/32, N[i]/32]); arithmetic of
- * jf_igemm_block_fp with JF_A_KM, JF_B_KN and, for each gradient, either the K split of splitk = 0 or one chosen for the launch as a
- * whole that rounds no more (parts of kb K blocks, p of them, with a smaller kb + p).  Behind it, up to 4 column sums
+ * jf_igemm_block_fp with JF_A_KM, JF_B_KN and, for each gradient, either the parts of splitk = 0 or others, chosen for the launch as a
+ * whole, whose sum rounds no more (parts of kb K blocks, p of them: the squared error grows as kb + p).  Behind it, up to 4 column sums
  * sum[i][c] = sum over K/32 strips of terms[i][strip][c], in the same launch as the sums of the K split. */
 size_t jf_wgrad_many_workspace_bytes(int n, const int *M, const int *N, int K);
 int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,

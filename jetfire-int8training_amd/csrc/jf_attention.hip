@@ -15,10 +15,13 @@
 // read (ds_read_b64_tr_b16: 4 rows of one column per lane), so neither V, K, Q nor dO is ever transposed in memory and P and
 // dS never leave the registers.  Row statistics of a query are lane-local but for one exchange between lane halves.
 //
-// What bounds it: at D = 64 a 32x32 tile of scores is 8 MFMAs forward (256 cycles) against about 20 vector instructions per
-// score register, one of them the quarter-rate exponential; the two overlap between the waves of a SIMD.  The gradient is two
-// kernels (dQ by query, dK/dV by key: 12 + 16 MFMAs per tile instead of 20) so that every sum has one owner and a fixed
-// order: no atomics, the same bits on every run.
+// What bounds it: vector instructions.  At D = 64 a 32x32 tile of scores is 8 MFMAs forward (256 cycles) and about 130 vector
+// instructions (8 per score register, one of them the quarter-rate exponential), at 4 cycles each.  8 x 25 heads of 1024 rows,
+// counters per SIMD, in 1000 cycles (forward | dQ | dK/dV): vector ALU 64 | 75 | 99, matrix pipe 26 | 40 | 53, of 122 | 144 | 199;
+// 51.7 | 64.0 | 81.5 us, no LDS bank conflicts.  The rest is waiting: the register operands' own loads are waited for inside the
+// tile loop, where the compiler's count takes the next tile's loads with them, so that a tile's loads overlap only part of the one
+// before.  The gradient is two kernels (dQ by query, dK/dV by key: 12 + 16 MFMAs per tile instead of 20) so that every sum has one
+// owner and a fixed order: no atomics, the same bits on every run.
 #include "jf_device.hpp"
 
 #pragma clang diagnostic ignored "-Winline-asm"     // M0 appears in clobber lists on purpose

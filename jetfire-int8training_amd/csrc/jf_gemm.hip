@@ -74,6 +74,8 @@ struct GemmArgs {
     int pace;             // PACE_*: wave priorities that order the resident workgroups of a CU (set by the launcher, see there)
     unsigned long long *phases;   // PROF kernels: 8 words per workgroup (jf_prof_igemm_block_q), first phase_capacity workgroups
     int phase_capacity;
+    int fold_kb;          // K blocks after which the accumulators are added up in `fold` (a multiple of NSTAGE stages; 0: never)   (FOLD)
+    float *fold;          // BM x BN values per workgroup, in an order of their own   (FOLD)
 };
 
 // Position of this workgroup in the launch's work.  Workgroups are dealt round-robin to the 8 XCDs, each with a private L2:
@@ -121,7 +123,9 @@ static int pace_of(long wgs, long slots, int k_per_wg);
 // PROF = 1: the first wave of every workgroup also records when the workgroup's phases began and ended (wall clock) and
 // how many shader cycles its main loop took: a profiling build of the same code, instantiated only in the measurement
 // library (jf_prof_igemm_block_q).
-template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM, int PROF>
+// FOLD = 1: a workgroup may sum its K range in parts (p.fold_kb K blocks each, added in ascending order): the same additions as a K
+// split's, without a workgroup, an epilogue and a partial result in a common buffer for every part.
+template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM, int PROF, int FOLD = 0>
 __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logical)
 {
     GemmArgs p = p_in;                                        // K-split launches narrow it to the split's K range below
@@ -517,6 +521,51 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
             });
         }
     };
+    // FOLD.  At the end of a part: the lagging product is accumulated, the accumulators are added to what this lane has left in p.fold
+    // before (a wave's values lie block by block, 16 bytes per lane) and start from zero again.  The first K block of the next stage is on
+    // its way into register set 0: it is waited for here, since the compiler may move those registers about.
+    static_assert(!FOLD || (EPI == EPI_FP && WBM == 2), "weight gradients");
+    int folds = 0;
+    float *const fold_base = FOLD ? p.fold + ((size_t)logical * NW + wave) * (NBLK * QB * QB) : nullptr;   // (wave-uniform)
+    auto fold_lane = [&]() -> unsigned {                      // this lane's first value (made anew: not a register over the main loop)
+        unsigned l;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+        return l * 4;
+    };
+    auto add_parts = [&] {
+        const float *const fold_at = fold_base + fold_lane();
+#pragma unroll
+        for (int i = 0; i < WBM; ++i)
+#pragma unroll
+            for (int j = 0; j < WBN; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const v4f t = *reinterpret_cast<const v4f *>(fold_at + ((i * WBN + j) * 4 + g) * (4 * WAVE));
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[i][j][4 * g + v] = t[v] + acc[i][j][4 * g + v];
+                }
+    };
+    auto end_part = [&] {
+        fetched(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+        accumulate(std::integral_constant<int, NBLK - 1>{});
+        sab_pend = 0.0f;
+        if (folds > 0) add_parts();
+        float *const fold_at = fold_base + fold_lane();
+#pragma unroll
+        for (int i = 0; i < WBM; ++i)
+#pragma unroll
+            for (int j = 0; j < WBN; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    v4f t;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) { t[v] = acc[i][j][4 * g + v]; acc[i][j][4 * g + v] = 0.0f; }
+                    *reinterpret_cast<v4f *>(fold_at + ((i * WBN + j) * 4 + g) * (4 * WAVE)) = t;
+                }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) d_pend[v] = 0;
+        ++folds;
+    };
     // Loads retire in order: a stage (and the scales of the one after it) has landed once only the loads of the Y stages
     // issued after it (up to `last`) are outstanding.  Near the end of K, with fewer stages behind it than usual, everything is waited for.
     auto wait_stage = [&](int last, auto younger_c) {
@@ -553,7 +602,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     constexpr int PACE = decltype(pace_c)::value;
     if constexpr (ACTIVE) fetch(fa_u[0], fb_u[0], 0u, sc_v, c0{}, c0{}, c0{}, c0{});
 
-    for (int s0 = 0; s0 < nfull; s0 += NSTAGE) static_for<0, NSTAGE>([&](auto slot_c) {
+    int s0 = 0;
+    auto stages_to = [&](const int stop) {
+    for (; s0 < stop; s0 += NSTAGE) static_for<0, NSTAGE>([&](auto slot_c) {
         constexpr int SLOT = decltype(slot_c)::value;         // ring slot of this stage, a compile-time constant
         constexpr int NEXT_SLOT = (SLOT + 1) % NSTAGE;
         const int s = s0 + SLOT;
@@ -605,6 +656,16 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
             }
         });
     });
+    };
+    if constexpr (FOLD && ACTIVE) {
+        const int part = p.fold_kb > 0 ? p.fold_kb / KB_STAGE : 0x3fffffff;        // stages of a part: whole turns of the ring
+        for (int end = part; s0 < nfull; end += part) {
+            stages_to(end < nfull ? end : nfull);
+            if (end < nfull || (end == nfull && ktail)) end_part();
+        }
+    } else {
+        stages_to(nfull);
+    }
     if (ACTIVE && ktail) {
         // short last stage (K not a multiple of 128): its first K block is already on its way to register set 0
         const unsigned slot = (unsigned)(nfull % NSTAGE);
@@ -738,6 +799,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     __builtin_amdgcn_s_waitcnt(0xC07F);                        // the last, unused prefetch must land before its registers are reused
     if (EPI != EPI_S32 && wave_active && !loader) {
         accumulate(std::integral_constant<int, NBLK - 1>{});
+        if constexpr (FOLD) { if (folds > 0) add_parts(); }
         // The scaled factor sa*sb*2^26 overflows when sa*sb >= 2^102.  An infinite factor leaves every accumulator
         // it touches infinite or NaN (inf*0 included), so "some accumulator of the wave is not finite" catches all such
         // cases; the wave then recomputes its blocks the plain way (operands straight from memory, zero accumulator
@@ -791,9 +853,13 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                     const float sab = (float)sa_t[(kb + kb_base) * p.sa_ks + mb[i] * p.sa_is] * (float)sb_t[(kb + kb_base) * p.sb_ks + nb[j] * p.sb_is];
 #pragma unroll
                     for (int v = 0; v < 16; ++v) r[v] = __builtin_fmaf(sab, (float)d[v], r[v]);
+                    if (FOLD && p.fold_kb > 0 && (kb + 1) % p.fold_kb == 0 && kb + 1 < nkb) {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) { acc[i][j][v] = kb + 1 == p.fold_kb ? r[v] : acc[i][j][v] + r[v]; r[v] = 0.0f; }
+                    }
                 }
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = r[v];
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = FOLD && folds > 0 ? acc[i][j][v] + r[v] : r[v];
             });
         }
     }
@@ -1019,7 +1085,7 @@ __global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp
     const GemmArgs &p = grp.g[k];
     const int work = p.tiles_m * p.tiles_n * p.splits, per = work >> 3, rem = work & 7, idx = at - begin;
     if (idx >= per + (xcd < rem ? 1 : 0)) return;
-    igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0>(p, xcd * per + (xcd < rem ? xcd : rem) + idx);
+    igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0, 1>(p, xcd * per + (xcd < rem ? xcd : rem) + idx);
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -1253,14 +1319,17 @@ static void splitk_plan(int M, int N, int K, int request, int &splits, int &kb_p
 // gradients), 3 us of ramp and epilogue per pair of tiles; parts cost a write and a read of every partial sum at about 8 TB/s (they
 // stay in the caches).  Parts are at least 8 K blocks (two stages) of at least 16.
 // Then, by rounding: the squared error of the sum of p parts of kb blocks grows as kb + p (each addition rounds the partial sum it has
-// reached), and no gradient is summed in an order that rounds more than its own launch would (splitk_plan): where the split of the
-// group is such a one, the gradient keeps its own.  A 256-wide block over 1024 tokens takes four parts of 8 blocks where a launch of
-// its own takes two of 16 (error against float64 8.3e-8 -> 7.2e-8 relative); a GPT-2 block at 8 x 1024 (XL) or 12 x 1024 tokens (small), which
-// unsplit would be fastest (small: 180 us, but 3.5e-7 where the parts give 1.2e-7 to 2.1e-7), keeps each gradient's own parts.  Launch and sums of the parts: XL 511
-// us, small 206, where four launches of their own and their sums took 532 and 225.
+// reached; 1 part: kb), and no gradient is summed in an order that rounds more than its own launch would (splitk_plan).  Where the
+// split of the group is such a one, its workgroups sum their K range in parts themselves (FOLD, above): q parts of f blocks in each
+// of p workgroups, f + q + p.  A gradient that would take more than FOLD_MAX of them (few tiles, which then end last) keeps its own
+// split.  Error against float64, 768 wide over 12288 tokens, of one chain | of the parts: 3.5e-7 | 1.2e-7 to 2.1e-7.  Launch and sums, us,
+// in one chain | with parts in workgroups | with a workgroup for every part | four launches of their own: 512 wide, 4096 tokens
+// 42 | 52 | 55 | 87; 1024, 8192 196 | 209 | 232 | 246; 768, 12288 171 | 183 | 199 | 235; 1600, 8192 515 | 518 | 514 | 543.
+// FOLD_MAX = 4 | 6 or more: 1152 wide, 8192 tokens (6 parts of one gradient) 264 | 250; = 6 or less | 8: 1024, 8192 (8 parts) 209 | 223.
 struct WgradPlan {
-    int splits[WGRAD_MAX], kb_per_split[WGRAD_MAX];
+    int splits[WGRAD_MAX], kb_per_split[WGRAD_MAX], fold_kb[WGRAD_MAX];
 };
+constexpr int FOLD_MAX = 6;                                    // parts inside a workgroup
 static void wgrad_group_plan(int n, const int *M, const int *N, int K, WgradPlan &plan)
 {
     int splits, kb_per_split;
@@ -1280,8 +1349,20 @@ static void wgrad_group_plan(int n, const int *M, const int *N, int K, WgradPlan
         if (s == 1 || t < best) { best = t; splits = parts; kb_per_split = kb; }
     }
     for (int i = 0; i < n; ++i) {
-        splitk_plan(M[i], N[i], K, 0, plan.splits[i], plan.kb_per_split[i]);
-        if (kb_per_split + splits <= plan.kb_per_split[i] + plan.splits[i]) { plan.splits[i] = splits; plan.kb_per_split[i] = kb_per_split; }
+        const auto parts = [](int p) { return p > 1 ? p : 0; };
+        int own, own_kb, fold = 0;
+        splitk_plan(M[i], N[i], K, 0, own, own_kb);
+        const int limit = own_kb + parts(own);
+        bool keep = kb_per_split + parts(splits) <= limit;
+        if (!keep) {                                           // parts inside the workgroups
+            constexpr int TURN = 2 * KB_STAGE;                 // (of the kernel's ring)
+            if (splits == 1 && own_kb % TURN == 0) fold = own_kb;
+            else for (fold = (kb_per_split - 1) / TURN * TURN; fold > 0 && fold + (kb_per_split + fold - 1) / fold + parts(splits) > limit; fold -= TURN) {}
+            keep = fold > 0 && (kb_per_split + fold - 1) / fold <= FOLD_MAX;
+        }
+        plan.splits[i] = keep ? splits : own;
+        plan.kb_per_split[i] = keep ? kb_per_split : own_kb;
+        plan.fold_kb[i] = keep ? fold : 0;
     }
 }
 
@@ -1475,15 +1556,27 @@ int jf_igemm_block_fp(const int8_t *A, const int8_t *B, const void *sa, const vo
                         kb_per, workspace, (hipStream_t)stream);
 }
 
+static size_t wgrad_fold_values(int M, int N, int splits)      // of GemmArgs::fold
+{
+    return (size_t)((M + 127) / 128) * ((N + 127) / 128) * splits * (128 * 128);
+}
+
+static size_t wgrad_workspace(int n, const int *M, const int *N, const WgradPlan &plan)
+{
+    size_t bytes = 0;
+    for (int i = 0; i < n; ++i) {
+        if (plan.splits[i] > 1) bytes += (size_t)plan.splits[i] * (size_t)M[i] * (size_t)N[i] * sizeof(float);
+        if (plan.fold_kb[i]) bytes += wgrad_fold_values(M[i], N[i], plan.splits[i]) * sizeof(float);
+    }
+    return bytes;
+}
+
 size_t jf_wgrad_many_workspace_bytes(int n, const int *M, const int *N, int K)
 {
     if (n < 1 || n > WGRAD_MAX || !M || !N || !mult32(K)) return 0;
     WgradPlan plan;
     wgrad_group_plan(n, M, N, K, plan);
-    size_t bytes = 0;
-    for (int i = 0; i < n; ++i)
-        if (plan.splits[i] > 1) bytes += (size_t)plan.splits[i] * (size_t)M[i] * (size_t)N[i] * sizeof(float);
-    return bytes;
+    return wgrad_workspace(n, M, N, plan);
 }
 
 int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
@@ -1503,7 +1596,7 @@ int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const in
     if (!device_is_gfx950()) return JF_ERR_DEVICE;
     WgradPlan plan;
     wgrad_group_plan(n, M, N, K, plan);
-    const size_t need = jf_wgrad_many_workspace_bytes(n, M, N, K);
+    const size_t need = wgrad_workspace(n, M, N, plan);
     if (need && (!workspace || !aligned16(workspace) || workspace_bytes < need)) return JF_ERR_WORKSPACE;
     int order[WGRAD_MAX];                                      // longest parts first: the short ones even out the end of the launch
     for (int i = 0; i < n; ++i) order[i] = i;
@@ -1516,16 +1609,21 @@ int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const in
     for (int j = 0; j < n; ++j) {
         const int i = order[j], splits = plan.splits[i];
         GemmArgs &a = grp.g[j];
-        a.A = G[i]; a.B = X[i]; a.sa = SG[i]; a.sb = SX[i]; a.C = splits > 1 ? (void *)part : out[i];
+        a.A = G[i]; a.B = X[i]; a.sa = SG[i]; a.sb = SX[i]; a.C = out[i];
         a.M = M[i]; a.N = N[i]; a.K = K; a.lda = M[i]; a.ldb = N[i]; a.out_dtype = out_dtype; a.splits = splits; a.kb_per_split = plan.kb_per_split[i];
         a.sa_ks = M[i] / QB; a.sa_is = 1; a.sb_ks = N[i] / QB; a.sb_is = 1;
         a.tiles_m = (M[i] + 127) / 128; a.tiles_n = (N[i] + 127) / 128;
+        if (plan.fold_kb[i]) {
+            a.fold_kb = plan.fold_kb[i]; a.fold = part;
+            part += wgrad_fold_values(M[i], N[i], splits);
+        }
         wgs += ((long)a.tiles_m * a.tiles_n * splits + 7) / 8;
         grp.end[j] = (int)wgs;
         if (plan.kb_per_split[i] > longest) longest = plan.kb_per_split[i];
         if (splits > 1) {
             const size_t count = (size_t)M[i] * (size_t)N[i];
             fwgs += (long)((count + 4095) / 4096);
+            a.C = part;
             fin.part[fin.n] = part; fin.out[fin.n] = out[i]; fin.count[fin.n] = count; fin.splits[fin.n] = splits; fin.end[fin.n] = (int)fwgs;
             ++fin.n;
             part += (size_t)splits * count;

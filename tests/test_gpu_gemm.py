@@ -542,3 +542,31 @@ def test_weight_gradients_in_one_launch_round_no_more_than_alone(jf, C, K):
         error = lambda o: float((o.double() - exact).norm() / exact.norm())  # noqa: E731
         print(f"  {g.shape[1]} x {x.shape[1]}: alone {error(alone):.3e}, together {error(many):.3e}", flush=True)
         assert error(many) <= 1.02 * error(alone) and error(alone) < 1e-6
+
+
+# (workgroups per tile along K, K blocks of each, K blocks of a part inside them) of each gradient on 256 compute units: parts inside one
+# workgroup; a short last stage alone in the last part, and a short last part; parts inside the parts of a K split, ragged tiles and a
+# ragged last split; a gradient with a split of its own beside gradients with parts inside workgroups
+@pytest.mark.parametrize("C,K,plan", [(512, 2048, [(1, 64, 16)] * 4), (512, 2080, [(1, 65, 16)] * 4), (480, 2144, [(1, 67, 16)] * 4), (512, 1056, [(1, 33, 16)] * 4),
+                                      (416, 4128, [(3, 44, 16)] * 4), (768, 4096, [(1, 128, 32), (8, 16, 0), (1, 128, 40), (1, 128, 40)])])
+@pytest.mark.parametrize("f16,out", [(True, torch.float16), (False, torch.float32)])
+def test_weight_gradients_summed_in_parts(jf, oracle, C, K, plan, f16, out):
+    """Bit for bit the sums in the order of the plan, also where a scale product is too large for the kernel's fast accumulation."""
+    print(f"case C={C} K={K} f16={f16}", flush=True)
+    rng = np.random.default_rng(C + K)
+    st = np.float16 if f16 else np.float32
+    widths = [(3 * C, C), (C, C), (4 * C, C), (C, 4 * C)]
+    operand = lambda c: (rand_codes(rng, (K, c)), rand_scales(rng, (K // QB, c // QB), f16=f16))  # noqa: E731
+    gs, xs = [operand(m) for m, _ in widths], [operand(n) for _, n in widths]
+    if not f16:
+        gs[0][1][20, 1] = xs[0][1][20, 2] = 2.0 ** 53          # one block product beyond 2^102, in the second part or later
+    d = lambda ts: [(dev(q), dev(s.astype(st))) for q, s in ts]  # noqa: E731
+    for (g, sg), (x, sx), (parts, kb, fold), o in zip(gs, xs, plan, jf.wgrad_many(d(gs), d(xs), out)[0]):
+        A, total = np.ascontiguousarray(g.T), None
+        for s in range(parts):
+            lo, hi = s * kb, min((s + 1) * kb, K // QB)
+            f = fold or hi - lo
+            part = oracle.igemm_block_f32_splitk(np.ascontiguousarray(A[:, lo * QB:hi * QB]), np.ascontiguousarray(x[lo * QB:hi * QB]),
+                                                 np.ascontiguousarray(sg[lo:hi]), np.ascontiguousarray(sx[lo:hi]), 1, -(-(hi - lo) // f), f)
+            total = part if total is None else total + part
+        same(o, torch.from_numpy(total).to(out).numpy(), f"dW {g.shape[1]} x {x.shape[1]}")
