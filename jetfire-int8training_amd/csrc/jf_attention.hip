@@ -17,8 +17,8 @@
 //
 // What bounds it: vector instructions.  At D = 64 a 32x32 tile of scores is 8 MFMAs forward (256 cycles) and about 130 vector
 // instructions (8 per score register, one of them the quarter-rate exponential), at 4 cycles each.  8 x 25 heads of 1024 rows,
-// counters per SIMD, in 1000 cycles (forward | dQ | dK/dV): vector ALU 64 | 75 | 99, matrix pipe 26 | 40 | 53, of 122 | 144 | 199;
-// 51.7 | 64.0 | 81.5 us, no LDS bank conflicts.  The rest is waiting: the register operands' own loads are waited for inside the
+// counters per SIMD, in 1000 cycles (forward | dQ | dK/dV): vector ALU 64 | 75 | 99, matrix pipe 26 | 40 | 53, of 121 | 143 | 194;
+// 50.7 | 62.9 | 80.0 us, no LDS bank conflicts.  The rest is waiting: the register operands' own loads are waited for inside the
 // tile loop, where the compiler's count takes the next tile's loads with them, so that a tile's loads overlap only part of the one
 // before.  The gradient is two kernels (dQ by query, dK/dV by key: 12 + 16 MFMAs per tile instead of 20) so that every sum has one
 // owner and a fixed order: no atomics, the same bits on every run.
