@@ -179,18 +179,10 @@ __device__ __forceinline__ void store_t(half_t *row, int h, const v16f &x)
 __device__ __forceinline__ void quantize_t(const v16f &x, int8_t *codes, half_t *scales, int row, int col, int C, int lane, int rounding,
                                            uint64_t seed, uint64_t offset)
 {
-    float y[16];
+    float y[16], z[16];
 #pragma unroll
     for (int v = 0; v < 16; ++v) y[v] = (float)(half_t)x[v];
-    float z[16];
-#pragma unroll
-    for (int g = 0; g < 2; ++g)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[4 * g + j]), __float_as_uint(y[8 + 4 * g + j]), false, false);
-            z[8 * g + j] = __uint_as_float(p[0]);
-            z[8 * g + 4 + j] = __uint_as_float(p[1]);
-        }
+    row_halves(y, z);
     const size_t e0 = (size_t)(row + (lane & 31)) * C + col + 16 * (lane >> 5);
     float s;
     *reinterpret_cast<v4i *>(codes + e0) = quantize16(z, 0.0f, rounding, seed, offset, e0, &s);

@@ -62,6 +62,20 @@ __device__ __forceinline__ float wave_max(float v)
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// A 32x32 block whose lane l holds row l%32, columns 8*(v/4) + 4*(l/32) + v%4 in register v (a transposed MFMA result), as columns
+// 16*(l/32) .. +15 of that row: an exchange between the lane halves per pair of registers.
+__device__ __forceinline__ void row_halves(const float (&a)[16], float (&x)[16])
+{
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[4 * g + j]), __float_as_uint(a[8 + 4 * g + j]), false, false);
+            x[8 * g + j] = __uint_as_float(p[0]);
+            x[8 * g + 4 + j] = __uint_as_float(p[1]);
+        }
+}
+
 // ---------------------------------------------------------------------------------------------
 // Philox4x32-R.  (Salmon et al., "Parallel random numbers: as easy as 1, 2, 3", SC'11.)  The rounding noise uses
 // R = 7, the smallest round count the authors report as passing BigCrush (10 is their default with a safety margin):
@@ -82,9 +96,10 @@ __device__ __forceinline__ void philox4x32(uint32_t c0, uint32_t c1, uint32_t c2
     for (int r = 0; r < ROUNDS; ++r) {
         uint64_t p0 = (uint64_t)0xD2511F53u * c0;
         uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-        uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
+        // (a ^ b ^ c in one instruction: the key is in a scalar register, with which a plain v_xor_b32 takes as long)
+        uint32_t n0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c1, k0, 0x96);
         uint32_t n1 = (uint32_t)p1;
-        uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+        uint32_t n2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c3, k1, 0x96);
         uint32_t n3 = (uint32_t)p0;
         c0 = n0; c1 = n1; c2 = n2; c3 = n3;
         k0 += 0x9E3779B9u;

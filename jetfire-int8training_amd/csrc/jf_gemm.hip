@@ -112,6 +112,21 @@ __device__ __forceinline__ void tile_at(int logical, int tiles_m, int tiles_n, b
 constexpr int WBN = 1;
 // threads of a workgroup: with one block per wave, as many waves again that do nothing but load (see load_loop)
 constexpr int gemm_threads(int WBM, int WGM, int WGN) { return 64 * WGM * WGN * (WBM == 1 ? 2 : 1); }
+constexpr int TABLE_KB = 512;                        // K blocks a wave's table of scale products holds (WBM = 1)
+// LDS of a workgroup: the operand ring; per-wave scale and product patches or tables; from gelu_lds_at on what the GELU tables of the
+// epilogue need beyond those (WBM = 2: the byte tables, 256 bytes per wave; WBM = 1: both, 1280 bytes).  Epilogues that go through
+// LDS use the ring.
+constexpr int gelu_lds_at(int WBM, int WGM, int WGN, int NSTAGE)
+{
+    const int scales = WBM == 1 ? 4 * (TABLE_KB + KB_STAGE) * WGM * WGN : NSTAGE * WGM * WGN * 512;
+    return NSTAGE * (QB * WBM * WGM + QB * WBN * WGN) * ROW_BYTES + scales;
+}
+constexpr int gemm_lds(int EPI, int WBM, int WGM, int WGN, int NSTAGE)
+{
+    const int tables = EPI == EPI_QG || EPI == EPI_QB ? (WBM == 1 ? 1280 : 256) * WGM * WGN : 0;
+    const int used = gelu_lds_at(WBM, WGM, WGN, NSTAGE) + tables, patch = WGM * WGN * QB * EPI_LD * (int)sizeof(float);
+    return used > patch ? used : patch;
+}
 // NSTAGE = depth of the LDS ring (one stage being computed, NSTAGE-1 in flight); WGPC = workgroups per CU
 // (the second launch bound counts waves per SIMD: WGPC workgroups of WGM*WGN waves over 4 SIMDs).
 // AKM = 1: A is [K, lda] (M-contiguous rows), staged and read like a [K,N] B operand (below).
@@ -148,6 +163,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     static_assert(!BKN || (BN == ROW_BYTES && WBN == 1), "a staged [K,N] row is one 128-byte LDS row");
     static_assert(WBM == 2 || !AKM, "one block per wave: A as [M,K] only");
     static_assert(!AKM || BM == ROW_BYTES, "a staged [K,M] row is one 128-byte LDS row");
+    // The epilogues that requantise want a lane to hold 16 consecutive columns of a row.  They form the transposed product (B block
+    // times A block, the same integers): its registers run along the columns, see the epilogue.
+    constexpr bool QUANT = EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD;
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     typedef __attribute__((address_space(3))) unsigned char lds_u8;
@@ -487,7 +505,8 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     // the same of one block with everything as arguments
     auto compute_block = [&](const v4i &fa, const v4i &fb, const float sab_new) {
         v16i d_new;
-        asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0x3e22f983" : "=&v"(d_new) : "v"(fa), "v"(fb));
+        if constexpr (QUANT) asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0x3e22f983" : "=&v"(d_new) : "v"(fb), "v"(fa));
+        else asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0x3e22f983" : "=&v"(d_new) : "v"(fa), "v"(fb));
         __builtin_amdgcn_sched_barrier(0);
         accumulate(std::integral_constant<int, 0>{});
         // (a copy of its own, made here: the register the product was read into is the target of the next read by the time it is used)
@@ -511,7 +530,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                 // AFTER the one below (32 vector instructions and another MFMA later), far beyond the wait states
                 // a vector read of an MFMA result needs.
                 v16i d_new;
-                asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0x3e22f983" : "=&v"(d_new) : "v"(fa_reg[CUR][i]), "v"(fb_reg[CUR][j]));
+                v4i &fa = fa_reg[CUR][i], &fb = fb_reg[CUR][j];
+                if constexpr (QUANT) asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0x3e22f983" : "=&v"(d_new) : "v"(fb), "v"(fa));
+                else asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0x3e22f983" : "=&v"(d_new) : "v"(fa), "v"(fb));
                 const float sab_new = sc_raw[CUR][n];
                 __builtin_amdgcn_sched_barrier(0);
                 accumulate(std::integral_constant<int, (n + NBLK - 1) % NBLK>{});
@@ -797,6 +818,8 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     else if (WBM == 2 && p.pace == PACE_ORDERED) main_loop(std::true_type{}, std::integral_constant<int, PACE_ORDERED>{});
     else main_loop(std::true_type{}, std::integral_constant<int, PACE_HARDWARE>{});
     __builtin_amdgcn_s_waitcnt(0xC07F);                        // the last, unused prefetch must land before its registers are reused
+    float lane_max[WBM][WBN];                                  // largest magnitude of this lane's results, per block   (QUANT)
+    bool nonfinite = false;                                    // wave-uniform: some result is infinite or NaN   (QUANT)
     if (EPI != EPI_S32 && wave_active && !loader) {
         accumulate(std::integral_constant<int, NBLK - 1>{});
         if constexpr (FOLD) { if (folds > 0) add_parts(); }
@@ -804,14 +827,39 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         // it touches infinite or NaN (inf*0 included), so "some accumulator of the wave is not finite" catches all such
         // cases; the wave then recomputes its blocks the plain way (operands straight from memory, zero accumulator
         // input, v_cvt_f32_i32, unscaled factor), which also reproduces results that really are infinite.
-        float chk = 0.0f;
+        // (A requantising epilogue needs the largest magnitude anyway: taken with the maximum that keeps a NaN, it is the check.)
+        auto largest = [&](auto nan_c) {
+            float all = 0.0f;
 #pragma unroll
-        for (int i = 0; i < WBM; ++i)
+            for (int i = 0; i < WBM; ++i)
 #pragma unroll
-            for (int j = 0; j < WBN; ++j)
+                for (int j = 0; j < WBN; ++j) {
+                    float m = 0.0f;
 #pragma unroll
-                for (int v = 0; v < 16; ++v) chk = __builtin_fmaf(acc[i][j][v], 0.0f, chk);
-        if (__builtin_expect(__ballot(chk != chk) != 0, 0)) {
+                    for (int v = 0; v < 16; ++v) {
+                        const float t = __builtin_fabsf(acc[i][j][v]);
+                        m = decltype(nan_c)::value ? __builtin_elementwise_maximum(m, t) : fmaxf(m, t);
+                    }
+                    lane_max[i][j] = m;
+                    all = __builtin_elementwise_maximum(all, m);
+                }
+            return all;
+        };
+        bool again;
+        if constexpr (QUANT) {
+            const float all = largest(std::true_type{});
+            again = __ballot(!(all < __builtin_inff())) != 0;
+        } else {
+            float chk = 0.0f;
+#pragma unroll
+            for (int i = 0; i < WBM; ++i)
+#pragma unroll
+                for (int j = 0; j < WBN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) chk = __builtin_fmaf(acc[i][j][v], 0.0f, chk);
+            again = __ballot(chk != chk) != 0;
+        }
+        if (__builtin_expect(again, 0)) {
             const ST *const sa_t = reinterpret_cast<const ST *>(p.sa), *const sb_t = reinterpret_cast<const ST *>(p.sb);
             static_for<0, NBLK>([&](auto blk_c) {              // compile-time block index: no indexed register arrays
                 constexpr int blk = decltype(blk_c)::value, i = blk / WBN, j = blk % WBN;
@@ -849,7 +897,8 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                         fb = *reinterpret_cast<const v4i *>(p.B + bcol * (size_t)p.ldb + k0);
                     }
                     const v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-                    const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb, z, 0, 0, 0);
+                    const v16i d = QUANT ? __builtin_amdgcn_mfma_i32_32x32x32_i8(fb, fa, z, 0, 0, 0)
+                                         : __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb, z, 0, 0, 0);
                     const float sab = (float)sa_t[(kb + kb_base) * p.sa_ks + mb[i] * p.sa_is] * (float)sb_t[(kb + kb_base) * p.sb_ks + nb[j] * p.sb_is];
 #pragma unroll
                     for (int v = 0; v < 16; ++v) r[v] = __builtin_fmaf(sab, (float)d[v], r[v]);
@@ -861,29 +910,40 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[i][j][v] = FOLD && folds > 0 ? acc[i][j][v] + r[v] : r[v];
             });
+            if constexpr (QUANT) { nonfinite = true; largest(std::false_type{}); }
         }
     }
     if (PROF) { phase(2, (unsigned long long)wall_clock64()); phase(7, (unsigned long long)(clock64() - prof_c0)); }
     if (p.pace != PACE_HARDWARE) __builtin_amdgcn_s_setprio(0);
-    __syncthreads();           // the epilogue reuses the ring as scratch
+    if constexpr (!QUANT) __syncthreads();                     // the epilogue reuses the ring as scratch
     if (loader) return;
     if (PROF) phase(3, (unsigned long long)wall_clock64());
 
     // ---- epilogue ------------------------------------------------------------------------------------------
-    // One 32x32 block at a time goes through a wave-private LDS patch that turns the MFMA result layout
-    //   (lane l, register v  <->  row 8*(v/4) + 4*(l/32) + v%4, column l%32)
-    // into a row layout (lane l <-> row l/2, columns 16*(l%2) .. +15): 16 consecutive columns per lane are what the
-    // Philox noise (8 elements per call) and 16-byte packing want.  Results are stored straight from the row layout: 16,
-    // 32 or 64 contiguous bytes per lane, two lanes per row of the block (measured 1 % faster than collecting one- and
-    // two-byte outputs in a workgroup-wide LDS image of the tile and writing that out in whole rows behind a barrier).
+    // Row layout of a block, 16 consecutive columns per lane, which is what the Philox noise (8 elements per call) and 16-byte stores
+    // want.  Results are stored straight from it: 16, 32 or 64 contiguous bytes per lane, two lanes per row of the block (measured
+    // 1 % faster than collecting one- and two-byte outputs in a workgroup-wide LDS image of the tile and writing that out in whole rows
+    // behind a barrier).
+    //   QUANT: the transposed product leaves lane l with row l%32, register v with column 8*(v/4) + 4*(l/32) + v%4; eight exchanges
+    //   between the lane halves make that columns 16*(l/32) .. +15.  No LDS and no barrier: a wave requantises while others of its
+    //   workgroup still multiply.  (With the product the other way round the block went through a wave-private LDS patch behind a
+    //   barrier of the workgroup.  us, that | this, the check for results that are not finite and the clamps saved with it:
+    //   12288x3072x768 forward with GELU 77.9 | 75.6, backward through the GELU 94.4 | 90.3; 12288x768x768 23.5 | 22.6;
+    //   8192x6400x1600 forward with GELU 185.9 | 183.4, backward 209.7 | 205.0; 12288x768x3072 71.7 | 71.0.)
+    //   Otherwise: one block at a time goes through a wave-private LDS patch that turns the MFMA result layout
+    //     (lane l, register v  <->  row 8*(v/4) + 4*(l/32) + v%4, column l%32)
+    //   into lane l <-> row l/2, columns 16*(l%2) .. +15.
     auto wave_sync = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    float *patch = reinterpret_cast<float *>(smem) + wave * (QB * EPI_LD);
-    const int rrow = lane >> 1, rcol = (lane & 1) * 16;
-    constexpr bool QUANT = EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD;
+    float *patch = reinterpret_cast<float *>(smem) + wave * (QB * EPI_LD);     // (not QUANT)
+    const int rrow = QUANT ? lane & 31 : lane >> 1, rcol = (QUANT ? lane >> 5 : lane & 1) * 16;
+    // GELU tables of the wave: its scale patch (nothing is on its way there any more) and, for the byte table, a piece of its own
+    float *const gelu_tab = TABLE ? reinterpret_cast<float *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 320 : reinterpret_cast<float *>(scale_patch);
+    int *const gelu_qtab = TABLE ? reinterpret_cast<int *>(gelu_tab + 256) : reinterpret_cast<int *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 64;
+    if (EPI == EPI_QG || EPI == EPI_QB) JF_WAIT_VMCNT(0);
     const float biasmax = (QUANT && p.biasmax) ? p.biasmax[0] : 0.0f;
     float gelu_f0 = 0.0f;                                     // gelu(+0), evaluated on the device like every table entry
     if (EPI == EPI_QG) {
@@ -945,19 +1005,16 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
             const bool valid = bm < p.M && bn < p.N;          // wave-uniform
             if (!valid) continue;
             float amax = 0.0f;
-            if (QUANT) {
-                float m = 0.0f;
+            if (QUANT) amax = wave_max(lane_max[i][j]) + biasmax;
+            if constexpr (!QUANT) {
 #pragma unroll
-                for (int v = 0; v < 16; ++v) m = fmaxf(m, fabsf(acc[i][j][v]));
-                amax = wave_max(m) + biasmax;
+                for (int v = 0; v < 16; ++v) {
+                    const int r = 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                    if (EPI == EPI_S32) patch[r * EPI_LD + (lane & 31)] = __int_as_float(iacc[i][j][v]);
+                    else patch[r * EPI_LD + (lane & 31)] = acc[i][j][v];
+                }
+                wave_sync();
             }
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int r = 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (EPI == EPI_S32) patch[r * EPI_LD + (lane & 31)] = __int_as_float(iacc[i][j][v]);
-                else patch[r * EPI_LD + (lane & 31)] = acc[i][j][v];
-            }
-            wave_sync();
             if (EPI == EPI_FP && p.out_dtype == JF_FP_F32) {
                 // No arithmetic follows, so the patch is read back in the shape that stores best: every store instruction
                 // writes 8 whole 128-byte rows of the block instead of 64 separate 16-byte pieces (3-6 us off the weight
@@ -973,12 +1030,16 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                 continue;
             }
             float x[16];
+            if constexpr (QUANT) {
+                row_halves(acc[i][j], x);
+            } else {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const v4f t = *reinterpret_cast<const v4f *>(patch + rrow * EPI_LD + rcol + 4 * k);
-                x[4 * k] = t.x; x[4 * k + 1] = t.y; x[4 * k + 2] = t.z; x[4 * k + 3] = t.w;
+                for (int k = 0; k < 4; ++k) {
+                    const v4f t = *reinterpret_cast<const v4f *>(patch + rrow * EPI_LD + rcol + 4 * k);
+                    x[4 * k] = t.x; x[4 * k + 1] = t.y; x[4 * k + 2] = t.z; x[4 * k + 3] = t.w;
+                }
+                wave_sync();
             }
-            wave_sync();
             const size_t e0 = (size_t)(bm + rrow) * p.N + bn + rcol;
             if (EPI == EPI_S32) {
                 v4i *dst = reinterpret_cast<v4i *>(reinterpret_cast<int32_t *>(p.C) + e0);
@@ -1004,29 +1065,41 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
 #pragma unroll
                     for (int k = 0; k < 16; ++k) x[k] = 127.0f * x[k];
                     d.div16(x, t);
+                    // Without a bias no |x| exceeds amax and no quotient that of amax itself, which is 127 or, for one block in
+                    // eight, the number after it; the noise stays below 1/2.  So only then (and where the quotient overflows, and
+                    // for results that are not finite) does any sum leave what rounds into +-127.
+                    float top;
+                    {
+                        const float a127 = 127.0f * amax;
+                        d.divn<1>(&a127, &top);
+                    }
+                    const bool clamp = __builtin_amdgcn_readfirstlane((p.bias != nullptr) | nonfinite | !(top <= 127.0f)) != 0;
                     if (p.rounding == JF_ROUND_STOCHASTIC) {
                         float n[16];
                         sr_noise16(p.seed, p.offset, (uint64_t)e0, n);
 #pragma unroll
                         for (int k = 0; k < 16; ++k) t[k] = t[k] + n[k];
                     }
-                    codes.x = (int)round_clamp_pack4(t[0], t[1], t[2], t[3]);
-                    codes.y = (int)round_clamp_pack4(t[4], t[5], t[6], t[7]);
-                    codes.z = (int)round_clamp_pack4(t[8], t[9], t[10], t[11]);
-                    codes.w = (int)round_clamp_pack4(t[12], t[13], t[14], t[15]);
+                    if (clamp) {
+#pragma unroll
+                        for (int k = 0; k < 16; ++k) t[k] = __builtin_amdgcn_fmed3f(t[k], -127.0f, 127.0f);
+                    }
+                    codes.x = (int)round_clamp_pack4<false>(t[0], t[1], t[2], t[3]);
+                    codes.y = (int)round_clamp_pack4<false>(t[4], t[5], t[6], t[7]);
+                    codes.z = (int)round_clamp_pack4<false>(t[8], t[9], t[10], t[11]);
+                    codes.w = (int)round_clamp_pack4<false>(t[12], t[13], t[14], t[15]);
                 }
                 if (EPI == EPI_QB) {
                     // GELU backward of the gradient block as a reader of the stored tensor would see it (codes x the scale
-                    // rounded to ST) against the saved forward input, with the wave's patch (free again) as the code table
+                    // rounded to ST) against the saved forward input
                     const float stored = (float)(ST)scale;
                     float scale2;
                     codes = p.gelu_approx == JF_GELU_TANH
-                        ? gelu_bwd_block<JF_GELU_TANH>(xq_codes[i][j], xq_scale[i][j], codes, stored, gelu_f0, patch, lane,
+                        ? gelu_bwd_block<JF_GELU_TANH>(xq_codes[i][j], xq_scale[i][j], codes, stored, gelu_f0, gelu_tab, lane,
                                                        p.rounding2, p.seed2, p.offset2, (uint64_t)e0, &scale2)
-                        : gelu_bwd_block<JF_GELU_ERF>(xq_codes[i][j], xq_scale[i][j], codes, stored, gelu_f0, patch, lane,
+                        : gelu_bwd_block<JF_GELU_ERF>(xq_codes[i][j], xq_scale[i][j], codes, stored, gelu_f0, gelu_tab, lane,
                                                       p.rounding2, p.seed2, p.offset2, (uint64_t)e0, &scale2);
                     scale = scale2;
-                    wave_sync();                              // the table is the next block's patch
                 }
                 if (EPI == EPI_QD) {
                     // the block as a reader of the stored tensor would dequantise it: codes x the scale rounded to ST
@@ -1038,18 +1111,14 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                     if (lane == 0) store_scale(reinterpret_cast<ST *>(p.sc), (bm / QB) * SN + bn / QB, scale);
                 }
                 if (EPI == EPI_QG) {
-                    // GELU of the block as a reader of the stored tensor would see it (codes x the scale rounded to ST),
-                    // with the wave's patch (free again) as the code tables
+                    // GELU of the block as a reader of the stored tensor would see it (codes x the scale rounded to ST)
                     const float stored = (float)(ST)scale;
-                    float *tab = patch;
-                    int *qtab = reinterpret_cast<int *>(patch + 256);
                     float scale2;
                     const v4i codes2 = p.gelu_approx == JF_GELU_TANH
-                        ? gelu_fwd_block<JF_GELU_TANH>(codes, stored, gelu_f0, p.gelu_eps, tab, qtab, lane, &scale2)
-                        : gelu_fwd_block<JF_GELU_ERF>(codes, stored, gelu_f0, p.gelu_eps, tab, qtab, lane, &scale2);
+                        ? gelu_fwd_block<JF_GELU_TANH>(codes, stored, gelu_f0, p.gelu_eps, gelu_tab, gelu_qtab, lane, &scale2)
+                        : gelu_fwd_block<JF_GELU_ERF>(codes, stored, gelu_f0, p.gelu_eps, gelu_tab, gelu_qtab, lane, &scale2);
                     *reinterpret_cast<v4i *>(reinterpret_cast<int8_t *>(p.C2) + e0) = codes2;
                     if (lane == 0) store_scale(reinterpret_cast<ST *>(p.sc2), (bm / QB) * SN + bn / QB, scale2);
-                    wave_sync();                              // the tables are the next block's patch
                 }
             }
         }
@@ -1143,15 +1212,6 @@ static int launch_transpose(const int8_t *in, int R, int C, int8_t *out, hipStre
     return (int)hipGetLastError();
 }
 
-constexpr int TABLE_KB = 512;                        // K blocks a wave's table of scale products holds (WBM = 1)
-// LDS of a workgroup: operand ring and per-wave scale and product patches or tables, or the epilogue's per-wave transposition patches
-constexpr int gemm_lds(int WBM, int WGM, int WGN, int NSTAGE)
-{
-    const int scales = WBM == 1 ? 4 * (TABLE_KB + KB_STAGE) * WGM * WGN : NSTAGE * WGM * WGN * 512;
-    const int ring = NSTAGE * (QB * WBM * WGM + QB * WBN * WGN) * ROW_BYTES + scales, patch = WGM * WGN * QB * EPI_LD * (int)sizeof(float);
-    return ring > patch ? ring : patch;
-}
-
 // more than 64 KiB of dynamic LDS has to be opted into, per function and device: once, not on every launch
 // (the reference sets its attribute on every call, igemm_BlockSquare32OutputIntQuantizeBiasRowCol.cu:418)
 static int allow_lds(const void *kern, int bytes, std::atomic<bool> (&opted_in)[MAX_DEVICES])
@@ -1184,7 +1244,7 @@ template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC,
 static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 {
     constexpr int BM = QB * WBM * WGM, BN = QB * WBN * WGN, NT = gemm_threads(WBM, WGM, WGN);
-    constexpr int SMEM = gemm_lds(WBM, WGM, WGN, NSTAGE);
+    constexpr int SMEM = gemm_lds(EPI, WBM, WGM, WGN, NSTAGE);
     if (!device_is_gfx950()) return JF_ERR_DEVICE;
     GemmArgs p = a;
     p.tiles_m = (p.M + BM - 1) / BM;
@@ -1201,7 +1261,7 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 
 template <typename ST> static int launch_wgrad_group(const GemmGroup &grp, unsigned wgs, hipStream_t st)
 {
-    constexpr int SMEM = gemm_lds(2, 2, 4, 2);
+    constexpr int SMEM = gemm_lds(EPI_FP, 2, 2, 4, 2);
     static std::atomic<bool> opted_in[MAX_DEVICES] = {};
     if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_wgrad_group_kernel<ST>), SMEM, opted_in)) return rc;
     hipLaunchKernelGGL(igemm_wgrad_group_kernel<ST>, dim3(wgs), dim3(512), SMEM, st, grp);

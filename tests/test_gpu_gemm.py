@@ -140,6 +140,35 @@ def test_row_major_scale_operands(jf, oracle, layout, f16):
         jf.igemm_block_fp(dA, dB, ka[:, ::2].repeat_interleave(2, 1)[:, : M // QB].t().t()[::1].as_strided((K // QB, M // QB), (M // QB * 2, 2)), kb, layout)
 
 
+def _largest_noise(oracle, seed):
+    """(offset, element) whose rounding noise under `seed` is the largest there is, 1/2 - 2^-17."""
+    for offset in range(1 << 17):
+        o = oracle.philox4x32([offset, 0, 0, 0], [seed, 0], oracle.NOISE_ROUNDS)
+        h = np.stack([o & 0xFFFF, o >> 16], 1).reshape(-1)
+        if (h == 0xFFFF).any():
+            return offset, int(np.argmax(h == 0xFFFF))
+    raise AssertionError("no such counter")
+
+
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("above", [False, True])
+def test_largest_noise_on_the_largest_result(jf, oracle, sign, above):
+    """127 * amax / amax is 127 or the number after it; with the noise 1/2 - 2^-17 the latter would round to 128, code -128."""
+    offset, e = _largest_noise(oracle, 5)
+    A, B = np.zeros((QB, QB), np.int8), np.zeros((QB, QB), np.int8)
+    A[0, 0], A[1:, 0] = 64, 16
+    B[0, :], B[0, e] = 16, sign * 64
+    scale = np.linspace(1, 2, 4001, dtype=np.float32)[1:]
+    amax = scale * np.float32(4096)
+    top = (np.float32(127) * amax) / amax
+    sa, sb = np.full((1, 1), scale[top > 127][0] if above else scale[top == 127][0], np.float32), np.ones((1, 1), np.float32)
+    got, sc = jf.igemm_block_q(dev(A), dev(B), dev(sa), dev(sb), jf.B_KN, rounding=jf.ROUND_STOCHASTIC, seed=5, offset=offset)
+    want, wsc = oracle.igemm_block_q(A, B, sa, sb, 1, stochastic=True, seed=5, offset=offset, scale_dtype="f32")
+    same(got, want, "codes")
+    same(sc, wsc, "scales")
+    assert abs(int(got[0, e])) == 127
+
+
 @pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("regime", ["huge_everywhere", "huge_one_block", "huge_last_kblock", "denormal_products"])
 def test_extreme_scale_products(jf, oracle, regime, layout):
