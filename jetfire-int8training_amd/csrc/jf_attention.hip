@@ -15,13 +15,15 @@
 // read (ds_read_b64_tr_b16: 4 rows of one column per lane), so neither V, K, Q nor dO is ever transposed in memory and P and
 // dS never leave the registers.  Row statistics of a query are lane-local but for one exchange between lane halves.
 //
-// What bounds it: vector instructions.  At D = 64 a 32x32 tile of scores is 8 MFMAs forward (256 cycles) and about 130 vector
-// instructions (8 per score register, one of them the quarter-rate exponential), at 4 cycles each.  8 x 25 heads of 1024 rows,
-// counters per SIMD, in 1000 cycles (forward | dQ | dK/dV): vector ALU 64 | 75 | 99, matrix pipe 26 | 40 | 53, of 121 | 143 | 194;
-// 50.7 | 62.9 | 80.0 us, no LDS bank conflicts.  The rest is waiting: the register operands' own loads are waited for inside the
-// tile loop, where the compiler's count takes the next tile's loads with them, so that a tile's loads overlap only part of the one
-// before.  The gradient is two kernels (dQ by query, dK/dV by key: 12 + 16 MFMAs per tile instead of 20) so that every sum has one
-// owner and a fixed order: no atomics, the same bits on every run.
+// What bounds it.  Per 32x32 tile of scores, at D = 64, forward | dQ | dK/dV: 8 | 12 | 16 MFMAs of 32 cycles and 60 to 75 vector
+// instructions, 16 of them exponentials at a quarter of the rate; the two kinds share the issue of a SIMD: about 540 | 730 | 810 cycles.
+// Eight sequences of 1024 rows with 25 heads have 103 tiles per SIMD: 25 | 34 | 38 us of 44 | 55 | 74 (the tile loop without its loads
+// takes 26 us of the forward's; loads and stores outside it, 118 MB, another 15).  Operands are read from LDS a step ahead of the
+// products, at immediate offsets, and tiles are loaded with scalar addresses: a step's instructions are the arithmetic.  us, before |
+// with that, forward and gradient: 8 x 1024 rows x 25 heads 52.8 | 44.5, 135.7 | 129.2; 2 x 1024 x 12 heads 21.6 | 17.5, 51.1 | 42.6;
+// 3 x 416 x 12 10.1 | 8.8, 27.3 | 23.3; 4 x 256 x 4 7.8 | 7.0, 21.1 | 18.3.
+// The gradient is two kernels (dQ by query, dK/dV by key: 12 + 16 MFMAs per tile instead of 20) so that every sum has one owner and a
+// fixed order: no atomics, the same bits on every run.
 #include "jf_device.hpp"
 
 #pragma clang diagnostic ignored "-Winline-asm"     // M0 appears in clobber lists on purpose
@@ -39,7 +41,7 @@ struct AttnArgs {
     half_t *out;                    // [B*T, C]                                           (forward)
     half_t *gq, *gk, *gv;           // [B*T, ldg]                                         (gradient kernels)
     float *lse;                     // [B*H, T]: log2 of the row sum of exp2(scale * log2(e) * s)
-    float *delta;                   // [B*H, T]: sum over D of o * go (left by the dQ kernel, read by the dK/dV kernel)
+    float *delta;                   // [B*H, T]: minus the sum over D of o * go (left by the dQ kernel, read by the dK/dV kernel)
     int ld, ldg, B, H, T;
     float scale;                    // of the scores
     int8_t *cq;                     // codes and scales of the result [B*T, C] or of the gradients [B*T, 3C] (kernels with QUANT)
@@ -83,10 +85,15 @@ template <int D> struct TileIO {
     static constexpr int LPW = 2 * INSTR / NW;                 // load instructions per wave: two tensors
     static_assert(2 * INSTR % NW == 0, "loads must split evenly");
     int lane, wave;
+    unsigned lx, ly;                                           // this lane's bytes behind the first row of a load, in either tensor
     unsigned rd[D / 16];                                       // operand reads: chunk 2kk + h of row l%32
     unsigned tr[D / 32][2];                                    // transposing reads: column block mb, rows +0..7 / +8..15
-    __device__ __forceinline__ TileIO(int lane_, int wave_) : lane(lane_), wave(wave_)
+    __device__ __forceinline__ TileIO(int lane_, int wave_, int ldx, int ldy) : lane(lane_), wave(wave_)
     {
+        const int r0 = (wave * RPI + lane / CPR) % 16;         // (a wave's loads are a multiple of 16 rows apart, the period of swz)
+        const unsigned chunk = (unsigned)(((lane % CPR) ^ swz<D>(r0)) << 4);
+        lx = (unsigned)(lane / CPR) * (unsigned)ldx * 2u + chunk;
+        ly = (unsigned)(lane / CPR) * (unsigned)ldy * 2u + chunk;
         const int h = lane >> 5, r = lane & 31;
 #pragma unroll
         for (int kk = 0; kk < D / 16; ++kk) rd[kk] = r * ROWB + (((2 * kk + h) ^ swz<D>(r)) << 4);
@@ -99,46 +106,92 @@ template <int D> struct TileIO {
                 tr[mb][e] = row * ROWB + ((c ^ swz<D>(row)) << 4) + (p & 1) * 8;
             }
     }
-    // rows row0 .. row0+63 of two tensors (first row of the batch at x / y, ldx / ldy elements apart) into LDS at `lds`;
-    // rows beyond the last are replaced by the last (never used)
-    __device__ __forceinline__ void load(unsigned lds, const half_t *x, int ldx, const half_t *y, int ldy, int row0, int last) const
+    // rows row0 .. row0+63 of two tensors (first row of the batch at x / y, ldx / ldy elements apart) into LDS at `lds`.  The first
+    // row of a load is wave-uniform: addresses cost no vector instructions.  Loads beyond the T rows (whole ones, T and the rows of a
+    // tile are multiples of 32) fetch the tile's first rows instead (never used).
+    __device__ __forceinline__ void load(unsigned lds, const half_t *x, int ldx, const half_t *y, int ldy, int row0, int T) const
     {
+        static_assert(32 % RPI == 0 && (NW * RPI) % 16 == 0 && INSTR % NW == 0, "whole loads beyond the last row; one swizzle and one tensor per load");
 #pragma unroll
         for (int j = 0; j < LPW; ++j) {
-            const int idx = wave + j * NW;                     // wave-uniform
-            const bool second = idx >= INSTR;
-            const int i = second ? idx - INSTR : idx;
-            const int row = i * RPI + lane / CPR, src = row0 + row < last ? row0 + row : last;
-            const unsigned off = (unsigned)src * (unsigned)(second ? ldy : ldx) * 2u + (((lane % CPR) ^ swz<D>(row)) << 4);
-            const half_t *base = second ? y : x;
+            const bool second = j >= INSTR / NW;
+            const int i = wave + (second ? j - INSTR / NW : j) * NW;
+            const int row = row0 + i * RPI, src = row < T ? row : row0;
+            const half_t *base = second ? y + (unsigned)src * (unsigned)ldy : x + (unsigned)src * (unsigned)ldx;
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         ::"v"(off), "s"(base), "s"(lds + (unsigned)(second ? TILE : 0) + (unsigned)i * 1024u) : "memory", "m0");
+                         ::"v"(second ? ly : lx), "s"(base), "s"(lds + (unsigned)(second ? TILE : 0) + (unsigned)i * 1024u) : "memory", "m0");
         }
     }
-    __device__ __forceinline__ h8 row_operand(unsigned tile, int sub, int kk) const
+    // LDS addresses of a buffer's operands in vector registers, so that everything else about a read is its immediate offset (left to
+    // itself the compiler adds up every read's address: 12 to 24 vector instructions a step)
+    struct At {
+        unsigned rd[D / 16], tr[D / 32][2];
+    };
+    __device__ __forceinline__ At at(unsigned buffer) const
     {
-        return *(const __attribute__((address_space(3))) h8 *)(uintptr_t)(tile + rd[kk] + sub * ATT_SUB * ROWB);
+        At r;
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) { r.rd[kk] = buffer + rd[kk]; asm volatile("" : "+v"(r.rd[kk])); }
+#pragma unroll
+        for (int mb = 0; mb < D / 32; ++mb)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) { r.tr[mb][e] = buffer + tr[mb][e]; asm volatile("" : "+v"(r.tr[mb][e])); }
+        return r;
     }
-    __device__ __forceinline__ h8 tr_operand(unsigned tile, int sub, int s, int mb) const
+    // row operands of step `sub` of a buffer's first or second tensor, K step kk
+    template <bool SECOND> static __device__ __forceinline__ h8 row_operand(const At &a, int sub, int kk)
+    {
+        return *(const __attribute__((address_space(3))) h8 *)(uintptr_t)(a.rd[kk] + (SECOND ? TILE : 0) + sub * ATT_SUB * ROWB);
+    }
+    template <bool SECOND> static __device__ __forceinline__ void row_operands(h8 (&x)[D / 16], const At &a, int sub)
+    {
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) x[kk] = row_operand<SECOND>(a, sub, kk);
+    }
+    // the transposed operands of step `sub`, columns 32mb .. +31; x[st][mb]
+    template <bool SECOND> static __device__ __forceinline__ void tr_operands(h8 (&x)[2][D / 32], const At &a, int sub)
     {
         typedef short s4 __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) s4 lds_s4;
-        const unsigned b = tile + (sub * ATT_SUB + 16 * s) * ROWB;
-        const h4 lo = __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(uintptr_t)(b + tr[mb][0])));
-        const h4 hi = __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(uintptr_t)(b + tr[mb][1])));
-        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int mb = 0; mb < D / 32; ++mb) {
+                h4 half[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    half[e] = __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (lds_s4 *)(uintptr_t)(a.tr[mb][e] + (SECOND ? TILE : 0) + (sub * ATT_SUB + 16 * st) * ROWB)));
+                x[st][mb] = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
+            }
     }
 };
 
+#define ATT_FENCE() __builtin_amdgcn_sched_barrier(0)    // LDS reads above it are under way before what follows
 #define ATT_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0)
 
-__device__ __forceinline__ void attn_tile_ready()
+// KNOWN: with the builtin, so that the compiler knows that its own loads before the tile loop have arrived too.  Left to it, it waits
+// for them where they are first used, inside the loop, with a count that takes the next tile's loads along.
+template <bool KNOWN = true> __device__ __forceinline__ void attn_tile_ready()
 {
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if constexpr (KNOWN) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0F70);                    // vmcnt(0)
+        asm volatile("s_barrier" ::: "memory");
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    }
 }
-__device__ __forceinline__ float half_swap(float x)            // the value of lane l ^ 32
+// maximum / sum over a lane and its partner in the other lane half
+__device__ __forceinline__ float half_max(float x)
 {
-    return __shfl_xor(x, 32, WAVE);
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __builtin_elementwise_maximum(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+__device__ __forceinline__ float half_sum(float x)
+{
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
 }
 // eight registers of a result as the B operand of a 16-deep step
 __device__ __forceinline__ h8 pack8(const v16f &x, int s)
@@ -201,7 +254,7 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_fwd_kernel(AttnArgs a)
     const int b = bh / a.H, head = bh - b * a.H;
     const size_t first = (size_t)b * a.T * a.ld + (size_t)head * D;
     const half_t *kp = a.k + first, *vp = a.v + first;
-    const IO io(lane, wave);
+    const IO io(lane, wave, a.ld, a.ld);
     const unsigned lds = (unsigned)(uintptr_t)(lds_byte *)smem;
     const int q0 = blk * WG_ROWS + 32 * wave, qend = (blk + 1) * WG_ROWS < a.T ? (blk + 1) * WG_ROWS : a.T;
     const int nt = (qend + ATT_ROWS - 1) / ATT_ROWS;
@@ -219,56 +272,75 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_fwd_kernel(AttnArgs a)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[mb][v] = 0.0f;
     const float c = a.scale * 1.44269504f;
-    // Running maximum (shared by the halves), this lane's part of the sum.  The maximum starts below every finite score but
-    // finite: keys whose score is -inf before the first finite one then count for nothing instead of giving -inf - -inf.
+    // Maximum (shared by the halves), this lane's part of the sum.  The maximum only guards the exponential's range: it is the rows'
+    // maximum over the first step and raised, and the sums rescaled, when a lane's 16 probabilities of a step add up to more than 2^8
+    // (every later one keeps its relative precision in binary16 up to there).  The sum is taken anyway; so a step has no maximum to
+    // form and to exchange before its exponentials can start.  The maximum starts below every finite score but finite: keys whose
+    // score is -inf before the first finite one then count for nothing instead of giving -inf - -inf.  (A sum that is NaN takes the
+    // slow way and stays one.)
     float m = -1e30f, l = 0.0f;
-    io.load(lds, kp, a.ld, vp, a.ld, 0, a.T - 1);
+    io.load(lds, kp, a.ld, vp, a.ld, 0, a.T);
     for (int t = 0; t < nt; ++t) {
         attn_tile_ready();                                     // tile t has landed; nobody reads the other buffer any more
-        if (t + 1 < nt) io.load(lds + ((t + 1) & 1) * 2 * IO::TILE, kp, a.ld, vp, a.ld, (t + 1) * ATT_ROWS, a.T - 1);
-        const unsigned kt = lds + (t & 1) * 2 * IO::TILE, vt = kt + IO::TILE;
+        if (t + 1 < nt) io.load(lds + ((t + 1) & 1) * 2 * IO::TILE, kp, a.ld, vp, a.ld, (t + 1) * ATT_ROWS, a.T);
+        const typename IO::At at = io.at(lds + (t & 1) * 2 * IO::TILE);
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub) {
             const int k0 = t * ATT_ROWS + sub * ATT_SUB;
             if (!active || k0 > q0) continue;                  // (wave-uniform) all keys behind the queries
+            h8 kr[D / 16], vr[2][D / 32];
+            IO::template row_operands<false>(kr, at, sub);
             v16f s;
 #pragma unroll
             for (int v = 0; v < 16; ++v) s[v] = 0.0f;
+            ATT_FENCE();
 #pragma unroll
-            for (int kk = 0; kk < D / 16; ++kk) s = ATT_MFMA(io.row_operand(kt, sub, kk), q[kk], s);
+            for (int kk = 0; kk < D / 16; ++kk) s = ATT_MFMA(kr[kk], q[kk], s);
+            IO::template tr_operands<true>(vr, at, sub);
+            ATT_FENCE();
             if (k0 == q0) {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) s[v] = 8 * (v >> 2) + 4 * h + (v & 3) > (lane & 31) ? -__builtin_inff() : s[v];
             }
-            // (v_maximum3_f32: a NaN stays one, and no operand has to be canonicalised first as for fmaxf)
-            float mx = s[0];
+            h8 p[2];
+            float sum;
+            auto probabilities = [&] {
+                const float mc = -m * c;
+                sum = 0.0f;
 #pragma unroll
-            for (int v = 1; v < 16; ++v) mx = __builtin_elementwise_maximum(mx, s[v]);
-            mx = __builtin_elementwise_maximum(mx, half_swap(mx));
-            // The maximum only guards the exponential's range: it is raised, and the sums rescaled, when a score exceeds it
-            // by more than a factor of 2^8 (every later probability keeps its relative precision in binary16 up to there).
-            if (__any((mx - m) * c > 8.0f)) {
-                const float mn = fmaxf(m, mx), al = __builtin_amdgcn_exp2f((m - mn) * c);
+                for (int st = 0; st < 2; ++st)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * st + j], c, mc));
+                        sum += e;
+                        p[st][j] = (half_t)e;
+                    }
+            };
+            const bool first = sub == 0 && t == 0;             // (wave-uniform)
+            if (!first) probabilities();
+            if (first || __any(!(sum <= 256.0f))) {               // (wave-uniform)
+                // (v_maximum3_f32: a NaN stays one, and no operand has to be canonicalised first as for fmaxf)
+                float mx = s[0];
+#pragma unroll
+                for (int v = 1; v < 16; ++v) mx = __builtin_elementwise_maximum(mx, s[v]);
+                const float mn = fmaxf(m, half_max(mx)), al = __builtin_amdgcn_exp2f((m - mn) * c);
                 l *= al;
 #pragma unroll
                 for (int mb = 0; mb < D / 32; ++mb)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) o[mb][v] *= al;
                 m = mn;
+                probabilities();
             }
-            const float mc = -m * c;
+            l += sum;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) { s[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], c, mc)); l += s[v]; }
+            for (int st = 0; st < 2; ++st)
 #pragma unroll
-            for (int st = 0; st < 2; ++st) {
-                const h8 p = pack8(s, st);
-#pragma unroll
-                for (int mb = 0; mb < D / 32; ++mb) o[mb] = ATT_MFMA(io.tr_operand(vt, sub, st, mb), p, o[mb]);
-            }
+                for (int mb = 0; mb < D / 32; ++mb) o[mb] = ATT_MFMA(vr[st][mb], p[st], o[mb]);
         }
     }
     if (!active) return;
-    l += half_swap(l);
+    l = half_sum(l);
     const float r = 1.0f / l;
     half_t *dst = a.out + ((size_t)b * a.T + query) * (a.H * D) + head * D;
 #pragma unroll
@@ -280,9 +352,15 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_fwd_kernel(AttnArgs a)
     if (h == 0) a.lse[(size_t)bh * a.T + query] = m * c + __builtin_amdgcn_logf(l);     // (v_log_f32: base 2)
 }
 
-// dQ by blocks of queries; leaves delta for the dK/dV kernel
-template <int D, bool QUANT>
-__global__ __launch_bounds__(64 * NW, 4) void attn_dq_kernel(AttnArgs a)
+// dQ by blocks of queries; leaves delta for the dK/dV kernel.
+// EARLY: operands are read before they are needed and a tile's loads overlap the whole tile before it (140 registers, 3 waves per SIMD).
+// It is the faster kernel by itself at every size, us without | with: 2 sequences of 1024 rows x 12 heads 45.2 | 42.3 (with dK/dV), 8 x 25
+// heads 131.6 | 129.4.  But where it fills the chip, the chip then lowers its clock for everything around it (1.99 -> 1.91 GHz in the
+// GEMMs of a training step, read from their clock counters, for as long as the steps go on): three GPT-2 XL blocks 5809 | 5959 us a step,
+// three of GPT-2 small 2860 | 2900, three 1024 wide over 8 x 512 tokens 1641 | 1685; two blocks 768 wide over 2 x 1024 tokens 614 | 606.
+// So it is taken while no CU has more than one workgroup of it.
+template <int D, bool QUANT, bool EARLY>
+__global__ __launch_bounds__(64 * NW, EARLY ? 3 : 4) void attn_dq_kernel(AttnArgs a)
 {
     using IO = TileIO<D>;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
@@ -293,13 +371,13 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_dq_kernel(AttnArgs a)
     const int b = bh / a.H, head = bh - b * a.H;
     const size_t first = (size_t)b * a.T * a.ld + (size_t)head * D;
     const half_t *kp = a.k + first, *vp = a.v + first;
-    const IO io(lane, wave);
+    const IO io(lane, wave, a.ld, a.ld);
     const unsigned lds = (unsigned)(uintptr_t)(lds_byte *)smem;
     const int q0 = blk * WG_ROWS + 32 * wave, qend = (blk + 1) * WG_ROWS < a.T ? (blk + 1) * WG_ROWS : a.T;
     const int nt = (qend + ATT_ROWS - 1) / ATT_ROWS;
     const bool active = q0 < a.T;
     const int query = active ? q0 + (lane & 31) : 0;
-    io.load(lds, kp, a.ld, vp, a.ld, 0, a.T - 1);
+    io.load(lds, kp, a.ld, vp, a.ld, 0, a.T);
     h8 q[D / 16], go[D / 16];
     float dl = 0.0f;
     {
@@ -314,18 +392,18 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_dq_kernel(AttnArgs a)
             for (int j = 0; j < 8; ++j) dl = __builtin_fmaf((float)o[j], (float)go[kk][j], dl);
         }
     }
-    dl += half_swap(dl);
+    dl = half_sum(dl);
     const float lse = a.lse[(size_t)bh * a.T + query], c = a.scale * 1.44269504f;
-    if (active && h == 0) a.delta[(size_t)bh * a.T + query] = dl;
+    if (active && h == 0) a.delta[(size_t)bh * a.T + query] = -dl;
     v16f acc[D / 32];
 #pragma unroll
     for (int mb = 0; mb < D / 32; ++mb)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[mb][v] = 0.0f;
     for (int t = 0; t < nt; ++t) {
-        attn_tile_ready();
-        if (t + 1 < nt) io.load(lds + ((t + 1) & 1) * 2 * IO::TILE, kp, a.ld, vp, a.ld, (t + 1) * ATT_ROWS, a.T - 1);
-        const unsigned kt = lds + (t & 1) * 2 * IO::TILE, vt = kt + IO::TILE;
+        attn_tile_ready<EARLY>();
+        if (t + 1 < nt) io.load(lds + ((t + 1) & 1) * 2 * IO::TILE, kp, a.ld, vp, a.ld, (t + 1) * ATT_ROWS, a.T);
+        const typename IO::At at = io.at(lds + (t & 1) * 2 * IO::TILE);
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub) {
             const int k0 = t * ATT_ROWS + sub * ATT_SUB;
@@ -333,21 +411,35 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_dq_kernel(AttnArgs a)
             v16f s, dp;
 #pragma unroll
             for (int v = 0; v < 16; ++v) { s[v] = 0.0f; dp[v] = 0.0f; }
+            h8 kc[2][D / 32];
+            if constexpr (EARLY) {
+                h8 kr[D / 16], vr[D / 16];
+                IO::template row_operands<false>(kr, at, sub);
+                IO::template row_operands<true>(vr, at, sub);
+                ATT_FENCE();
 #pragma unroll
-            for (int kk = 0; kk < D / 16; ++kk) s = ATT_MFMA(io.row_operand(kt, sub, kk), q[kk], s);
+                for (int kk = 0; kk < D / 16; ++kk) s = ATT_MFMA(kr[kk], q[kk], s);
 #pragma unroll
-            for (int kk = 0; kk < D / 16; ++kk) dp = ATT_MFMA(io.row_operand(vt, sub, kk), go[kk], dp);
+                for (int kk = 0; kk < D / 16; ++kk) dp = ATT_MFMA(vr[kk], go[kk], dp);
+                IO::template tr_operands<false>(kc, at, sub);
+            } else {
+#pragma unroll
+                for (int kk = 0; kk < D / 16; ++kk) s = ATT_MFMA(IO::template row_operand<false>(at, sub, kk), q[kk], s);
+#pragma unroll
+                for (int kk = 0; kk < D / 16; ++kk) dp = ATT_MFMA(IO::template row_operand<true>(at, sub, kk), go[kk], dp);
+            }
             if (k0 == q0) {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) s[v] = 8 * (v >> 2) + 4 * h + (v & 3) > (lane & 31) ? -__builtin_inff() : s[v];
             }
 #pragma unroll
             for (int v = 0; v < 16; ++v) s[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], c, -lse)) * (dp[v] - dl);
+            if constexpr (!EARLY) IO::template tr_operands<false>(kc, at, sub);
 #pragma unroll
             for (int st = 0; st < 2; ++st) {
                 const h8 ds = pack8(s, st);
 #pragma unroll
-                for (int mb = 0; mb < D / 32; ++mb) acc[mb] = ATT_MFMA(io.tr_operand(kt, sub, st, mb), ds, acc[mb]);
+                for (int mb = 0; mb < D / 32; ++mb) acc[mb] = ATT_MFMA(kc[st][mb], ds, acc[mb]);
             }
         }
     }
@@ -364,7 +456,7 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_dq_kernel(AttnArgs a)
 
 // dK and dV by blocks of keys
 template <int D, bool QUANT>
-__global__ __launch_bounds__(64 * NW, 3) void attn_dkv_kernel(AttnArgs a)
+__global__ __launch_bounds__(64 * NW, 2) void attn_dkv_kernel(AttnArgs a)
 {
     using IO = TileIO<D>;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
@@ -377,14 +469,14 @@ __global__ __launch_bounds__(64 * NW, 3) void attn_dkv_kernel(AttnArgs a)
     const size_t first = (size_t)b * a.T * a.ld + (size_t)head * D;
     const half_t *qp = a.q + first, *gp = a.go + (size_t)b * a.T * (a.H * D) + (size_t)head * D;
     const float *lsep = a.lse + (size_t)bh * a.T, *dlp = a.delta + (size_t)bh * a.T;
-    const IO io(lane, wave);
+    const IO io(lane, wave, a.ld, a.H * D);
     const unsigned lds = (unsigned)(uintptr_t)(lds_byte *)smem, stat_lds = (unsigned)(uintptr_t)(lds_byte *)stat;
     const int k0 = blk * WG_ROWS + 32 * wave;
     const int t0 = blk * WG_ROWS / ATT_ROWS, nt = (a.T + ATT_ROWS - 1) / ATT_ROWS;
     const bool active = k0 < a.T;
     const int key = active ? k0 + (lane & 31) : 0;
     auto load = [&](int t) {
-        io.load(lds + (t & 1) * 2 * IO::TILE, qp, a.ld, gp, a.H * D, t * ATT_ROWS, a.T - 1);
+        io.load(lds + (t & 1) * 2 * IO::TILE, qp, a.ld, gp, a.H * D, t * ATT_ROWS, a.T);
         if (wave == 0) {
             // (the lane number is made anew: held over the loop it is one register too many, and its reload waits for the whole tile)
             unsigned l;
@@ -415,40 +507,51 @@ __global__ __launch_bounds__(64 * NW, 3) void attn_dkv_kernel(AttnArgs a)
     for (int t = t0; t < nt; ++t) {
         attn_tile_ready();
         if (t + 1 < nt) load(t + 1);
-        const unsigned qt = lds + (t & 1) * 2 * IO::TILE, gt = qt + IO::TILE;
+        const typename IO::At at = io.at(lds + (t & 1) * 2 * IO::TILE);
         const float *st_l = stat[t & 1][0], *st_d = stat[t & 1][1];
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub) {
             const int q0 = t * ATT_ROWS + sub * ATT_SUB;
             if (!active || q0 < k0 || q0 >= a.T) continue;     // (wave-uniform) queries before the keys, or none
+            h8 qr[D / 16], gr[D / 16];
+            IO::template row_operands<false>(qr, at, sub);
             v16f s, dp;
+            // (the gradient's product starts from -delta, which the registers of a result are read into as they lie)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) { s[v] = 0.0f; dp[v] = 0.0f; }
+            for (int g = 0; g < 4; ++g) {
+                const v4f de = *reinterpret_cast<const v4f *>(st_d + sub * ATT_SUB + 8 * g + 4 * h);
 #pragma unroll
-            for (int kk = 0; kk < D / 16; ++kk) s = ATT_MFMA(io.row_operand(qt, sub, kk), k[kk], s);
+                for (int j = 0; j < 4; ++j) { s[4 * g + j] = 0.0f; dp[4 * g + j] = de[j]; }
+            }
+            ATT_FENCE();
+            IO::template row_operands<true>(gr, at, sub);
 #pragma unroll
-            for (int kk = 0; kk < D / 16; ++kk) dp = ATT_MFMA(io.row_operand(gt, sub, kk), vv[kk], dp);
+            for (int kk = 0; kk < D / 16; ++kk) s = ATT_MFMA(qr[kk], k[kk], s);
+#pragma unroll
+            for (int kk = 0; kk < D / 16; ++kk) dp = ATT_MFMA(gr[kk], vv[kk], dp);
+            ATT_FENCE();
+            h8 gc[2][D / 32], qc[2][D / 32];
+            v4f ls[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) ls[g] = *reinterpret_cast<const v4f *>(st_l + sub * ATT_SUB + 8 * g + 4 * h);
+            IO::template tr_operands<true>(gc, at, sub);
             if (q0 == k0) {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) s[v] = 8 * (v >> 2) + 4 * h + (v & 3) < (lane & 31) ? -__builtin_inff() : s[v];
             }
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const v4f ls = *reinterpret_cast<const v4f *>(st_l + sub * ATT_SUB + 8 * g + 4 * h);
-                const v4f de = *reinterpret_cast<const v4f *>(st_d + sub * ATT_SUB + 8 * g + 4 * h);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    s[4 * g + j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * g + j], c, -ls[j]));
-                    dp[4 * g + j] = s[4 * g + j] * (dp[4 * g + j] - de[j]);
-                }
+            for (int v = 0; v < 16; ++v) {
+                s[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], c, -ls[v >> 2][v & 3]));
+                dp[v] = s[v] * dp[v];
             }
+            IO::template tr_operands<false>(qc, at, sub);
 #pragma unroll
             for (int st = 0; st < 2; ++st) {
                 const h8 p = pack8(s, st), ds = pack8(dp, st);
 #pragma unroll
                 for (int mb = 0; mb < D / 32; ++mb) {
-                    dv[mb] = ATT_MFMA(io.tr_operand(gt, sub, st, mb), p, dv[mb]);
-                    dk[mb] = ATT_MFMA(io.tr_operand(qt, sub, st, mb), ds, dk[mb]);
+                    dv[mb] = ATT_MFMA(gc[st][mb], p, dv[mb]);
+                    dk[mb] = ATT_MFMA(qc[st][mb], ds, dk[mb]);
                 }
             }
         }
@@ -485,13 +588,16 @@ static int attn_check(const void *q, const void *k, const void *v, int ld, int B
     return device_is_gfx950() ? JF_OK : JF_ERR_DEVICE;
 }
 
-#define JF_ATT_D(KERN, D, a, st)                                                                                            \
-    do {                                                                                                                    \
-        const unsigned grid = 8u * (((a).B * (a).H + 7) / 8) * (((a).T + WG_ROWS - 1) / WG_ROWS);                           \
-        if ((a).cq) hipLaunchKernelGGL((KERN<D, true>), dim3(grid), dim3(64 * NW), 0, st, a);                               \
-        else hipLaunchKernelGGL((KERN<D, false>), dim3(grid), dim3(64 * NW), 0, st, a);                                     \
-    } while (0)
-#define JF_ATT(KERN, D, a, st) do { if (D == 64) JF_ATT_D(KERN, 64, a, st); else JF_ATT_D(KERN, 32, a, st); } while (0)
+static void attn_launch(void (*kernel)(AttnArgs), const AttnArgs &a, hipStream_t st)
+{
+    const unsigned grid = 8u * ((a.B * a.H + 7) / 8) * ((a.T + WG_ROWS - 1) / WG_ROWS);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * NW), 0, st, a);
+}
+template <int D, bool QUANT> static void attn_launch_dq(const AttnArgs &a, hipStream_t st)
+{
+    const bool alone = (long)a.B * a.H * ((a.T + WG_ROWS - 1) / WG_ROWS) <= cu_count();   // (see the kernel)
+    attn_launch(alone ? attn_dq_kernel<D, QUANT, true> : attn_dq_kernel<D, QUANT, false>, a, st);
+}
 
 }  // namespace jf
 
@@ -508,7 +614,8 @@ static int attention_fwd(const void *q, const void *k, const void *v, int ld, in
     a.q = (const half_t *)q; a.k = (const half_t *)k; a.v = (const half_t *)v; a.ld = ld;
     a.out = (half_t *)out; a.lse = lse; a.B = B; a.H = H; a.T = T; a.scale = scale;
     a.cq = codes; a.cs = (half_t *)scales;
-    JF_ATT(attn_fwd_kernel, D, a, (hipStream_t)stream);
+    if (D == 64) attn_launch(codes ? attn_fwd_kernel<64, true> : attn_fwd_kernel<64, false>, a, (hipStream_t)stream);
+    else attn_launch(codes ? attn_fwd_kernel<32, true> : attn_fwd_kernel<32, false>, a, (hipStream_t)stream);
     return (int)hipGetLastError();
 }
 
@@ -526,8 +633,14 @@ static int attention_bwd(const void *q, const void *k, const void *v, int ld, co
     a.o = (const half_t *)out; a.go = (const half_t *)gout; a.lse = const_cast<float *>(lse); a.delta = delta;
     a.gq = (half_t *)gq; a.gk = (half_t *)gk; a.gv = (half_t *)gv; a.ldg = ldg; a.B = B; a.H = H; a.T = T; a.scale = scale;
     a.cq = codes; a.cs = (half_t *)scales; a.seed = seed; a.offset = offset;
-    JF_ATT(attn_dq_kernel, D, a, (hipStream_t)stream);
-    JF_ATT(attn_dkv_kernel, D, a, (hipStream_t)stream);
+    hipStream_t st = (hipStream_t)stream;
+    if (D == 64) {
+        codes ? attn_launch_dq<64, true>(a, st) : attn_launch_dq<64, false>(a, st);
+        attn_launch(codes ? attn_dkv_kernel<64, true> : attn_dkv_kernel<64, false>, a, st);
+    } else {
+        codes ? attn_launch_dq<32, true>(a, st) : attn_launch_dq<32, false>(a, st);
+        attn_launch(codes ? attn_dkv_kernel<32, true> : attn_dkv_kernel<32, false>, a, st);
+    }
     return (int)hipGetLastError();
 }
 

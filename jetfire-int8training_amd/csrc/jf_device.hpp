@@ -7,6 +7,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <type_traits>
 #include <stdint.h>
 
@@ -570,6 +571,19 @@ static inline bool device_is_gfx950()
         known[dev] = ok ? 1 : -1;
     }
     return known[dev] == 1;
+}
+// compute units of the current device (asked once per device; 256 if the query fails)
+static inline int cu_count()
+{
+    static std::atomic<int> known[MAX_DEVICES] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return 256;
+    int cus = known[dev].load(std::memory_order_relaxed);
+    if (cus == 0) {
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+        known[dev].store(cus, std::memory_order_relaxed);
+    }
+    return cus;
 }
 static inline bool mult32(int v) { return v > 0 && (v % QB) == 0; }
 static inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

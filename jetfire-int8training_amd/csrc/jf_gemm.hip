@@ -132,7 +132,6 @@ constexpr int gemm_lds(int EPI, int WBM, int WGM, int WGN, int NSTAGE)
 // AKM = 1: A is [K, lda] (M-contiguous rows), staged and read like a [K,N] B operand (below).
 // BKN = 0: B is [N, ldb] (K-contiguous rows, like A).  BKN = 1: B is [K, ldb] (N-contiguous rows); its tile is staged
 // as it lies in memory and the K-contiguous MFMA operand is produced by the transposing LDS read of gfx950.
-static int cu_count();
 static int pace_of(long wgs, long slots, int k_per_wg);
 
 // PROF = 1: the first wave of every workgroup also records when the workgroup's phases began and ended (wall clock) and
@@ -1340,20 +1339,6 @@ __global__ __launch_bounds__(1024) void wgrad_finish_kernel(WgradFinish f)
         for (int i = 1; i < 32; ++i) t = t + red[i][x];
         f.sum[k][c] = t;
     }
-}
-
-// compute units of the current device (asked once per device; 256 if the query fails)
-static int cu_count()
-{
-    static std::atomic<int> known[MAX_DEVICES] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return 256;
-    int cus = known[dev].load(std::memory_order_relaxed);
-    if (cus == 0) {
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-        known[dev].store(cus, std::memory_order_relaxed);
-    }
-    return cus;
 }
 
 // K split of the fp-output GEMM.  request 1: none; request > 1: that many parts (fewer if K is short); request 0: as
