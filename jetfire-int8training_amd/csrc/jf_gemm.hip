@@ -60,6 +60,8 @@ struct GemmArgs {
     uint64_t seed, offset;
     int M, N, K, lda, ldb;
     int tiles_m, tiles_n;
+    int m_base;           // first row of the tiles (a launch of two tile sizes: its second part)
+    int big_tiles;        // 128x128 tiles of a launch of both tile sizes, rows 0 .. m_base - 1 (the 32x128 tiles start there)
     int splits, kb_per_split;   // split-K (EPI_FP only): workgroup w works on K blocks [s*kb_per_split, ...) of tile w % tiles,
                                 // s = w / tiles, and stores fp32 partial sums at C + s*M*N
     int out_dtype;        // JF_FP_*        (EPI_FP)
@@ -78,13 +80,13 @@ struct GemmArgs {
     float *fold;          // BM x BN values per workgroup, in an order of their own   (FOLD)
 };
 
-// Position of this workgroup in the launch's work.  Workgroups are dealt round-robin to the 8 XCDs, each with a private L2:
-// every XCD gets one contiguous run of the work.
-__device__ __forceinline__ int logical_workgroup()
+// Position of workgroup wg in `work` pieces of work, or -1 behind the last.  Workgroups are dealt round-robin to the 8 XCDs, each with a
+// private L2: every XCD gets one contiguous run of the work.
+__device__ __forceinline__ int logical_workgroup(int work, int wg, bool all = false)     // (all: no workgroup lies behind the last)
 {
-    const int nwg = gridDim.x, wg = blockIdx.x;
     const int xcd = wg & 7, idx = wg >> 3;
-    const int per = nwg >> 3, rem = nwg & 7;
+    const int per = work >> 3, rem = work & 7;
+    if (!all && idx >= per + (xcd < rem ? 1 : 0)) return -1;
     return xcd * per + (xcd < rem ? xcd : rem) + idx;
 }
 
@@ -188,7 +190,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         p.C = reinterpret_cast<float *>(p.C) + (size_t)split * (size_t)p.M * (size_t)p.N;
         p.out_dtype = JF_FP_F32;
     }
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int m0 = p.m_base + tile_m * BM, n0 = tile_n * BN;
     const int SM = p.M / QB, SN = p.N / QB;
     const int nkb = p.K / QB;
     const int nstages = (nkb + KB_STAGE - 1) / KB_STAGE;
@@ -1130,7 +1132,27 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
 template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM = 0, int PROF = 0>
 __global__ __launch_bounds__(gemm_threads(WBM, WGM, WGN), WGPC * gemm_threads(WBM, WGM, WGN) / 256) void igemm_nt_kernel(GemmArgs p)
 {
-    igemm_body<EPI, ST, WBM, WGM, WGN, NSTAGE, WGPC, BKN, AKM, PROF>(p, logical_workgroup());
+    p.m_base = 0;
+    igemm_body<EPI, ST, WBM, WGM, WGN, NSTAGE, WGPC, BKN, AKM, PROF>(p, logical_workgroup(gridDim.x, blockIdx.x, true));
+}
+
+// Rows 0 .. m_base - 1 in 128x128 tiles, the others in 32x128 tiles (launch_gemm_mixed).
+template <int EPI, typename ST, int BKN> __global__ __launch_bounds__(512, 4) void igemm_mixed_kernel(GemmArgs p)
+{
+    const int first_small = (p.big_tiles + 7) & ~7;           // (both parts are dealt to the XCDs from the first one on)
+    const int wg = blockIdx.x;
+    if (wg < first_small) {
+        const int logical = logical_workgroup(p.big_tiles, wg);
+        if (logical < 0) return;
+        p.tiles_m = p.m_base / (4 * QB);
+        p.m_base = 0;
+        igemm_body<EPI, ST, 2, 2, 4, 2, 2, BKN, 0, 0>(p, logical);
+    } else {
+        const int logical = logical_workgroup(p.tiles_m * p.tiles_n, wg - first_small);
+        if (logical < 0) return;
+        p.pace = PACE_HARDWARE;                               // (no paced instances)
+        igemm_body<EPI, ST, 1, 1, 4, 3, 2, BKN, 0, 0>(p, logical);
+    }
 }
 
 // Several weight gradients over the same tokens in one launch (jf_wgrad_many).  Every XCD gets one contiguous run of each problem's
@@ -1151,9 +1173,8 @@ __global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp
     for (int i = 1; i < WGRAD_MAX; ++i)
         if (i < grp.n && at >= grp.end[i - 1]) { k = i; begin = grp.end[i - 1]; }
     const GemmArgs &p = grp.g[k];
-    const int work = p.tiles_m * p.tiles_n * p.splits, per = work >> 3, rem = work & 7, idx = at - begin;
-    if (idx >= per + (xcd < rem ? 1 : 0)) return;
-    igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0, 1>(p, xcd * per + (xcd < rem ? xcd : rem) + idx);
+    const int logical = logical_workgroup(p.tiles_m * p.tiles_n * p.splits, (at - begin) * 8 + xcd);
+    if (logical >= 0) igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0, 1>(p, logical);
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -1255,6 +1276,45 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
     p.pace = WBM == 1 ? (int)PACE_HARDWARE                    // (no paced instances: all its workgroups are resident)
                       : pace_of((long)p.tiles_m * p.tiles_n * p.splits, (long)WGPC * cu_count(), p.splits > 1 ? p.kb_per_split * QB : p.K);
     hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n * p.splits), dim3(NT), SMEM, st, p);
+    return (int)hipGetLastError();
+}
+
+// A launch of 128x128 tiles that begins a short last round (of one workgroup per CU, or of two) takes that round's part of M as 32x128
+// tiles, in the same launch: tiles left alone on their CUs run at two thirds of the rate and leave most of the chip idle for the whole
+// length of a tile.  Rows of 128x128 tiles if so, else 0.  The line: after two big tiles per CU up to two small ones each (all of
+// them resident at once), after one, four or six one small one each.  us, 128x128 | mixed:
+//   768 wide, K = 3072: 5504 rows (258 tiles) 39.8 | 32.0, 6144 (288) 42.2 | 33.5, 12288 (576) 72.4 | 61.9; K = 768: 2048x2304 (288)
+//   15.4 | 11.5, 12288x768 23.2 | 21.6; K = 1536: 11008 rows (516) 41.2 | 32.8, 13312 (624) 38.8 | 35.3, 22016 (1032) 63.0 | 56.3;
+//   11008x2304x768 (1548) 50.6 | 45.9; 4224x1024x4096 (264) 52.1 | 43.0.
+// Beyond it: 13824x768x1536 (648 tiles) 38.8 | 39.0, 15360 (720) 39.4 | 42.5, 8192x768x3072 (384) 43.5 | 47.5, 24576x768x1536 (1152)
+// 61.7 | 61.8, 11264x3072x768 (2112) 63.0 | 62.3.
+static int mixed_big_rows(int M, int N, int K)
+{
+    const int rows = (M + 127) / 128, tiles_n = (N + 127) / 128, cus = cu_count();
+    if (K > TABLE_KB * QB) return 0;
+    for (const int rounds : {1, 2, 4, 6}) {                    // big tiles per CU
+        const int big = rounds * cus / tiles_n;
+        const long small = (long)((M - big * 128) / QB) * tiles_n;
+        if (big < rows && big * tiles_n > (rounds - 1) * cus && small <= (rounds == 2 ? 2L : 1L) * cus) return big;
+    }
+    return 0;
+}
+
+template <int EPI, typename ST, int BKN> static int launch_gemm_mixed(const GemmArgs &a, int big_rows, hipStream_t st)
+{
+    if (!device_is_gfx950()) return JF_ERR_DEVICE;
+    GemmArgs p = a;
+    p.splits = 1;
+    p.tiles_n = (p.N + 127) / 128;
+    p.m_base = big_rows * 128;
+    p.big_tiles = big_rows * p.tiles_n;
+    p.tiles_m = (p.M - p.m_base) / QB;
+    p.pace = pace_of(p.big_tiles, 2L * cu_count(), p.K);
+    constexpr int BIG = gemm_lds(EPI, 2, 2, 4, 2), SMALL = gemm_lds(EPI, 1, 1, 4, 3), SMEM = BIG > SMALL ? BIG : SMALL;
+    static std::atomic<bool> opted_in[MAX_DEVICES] = {};
+    if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_mixed_kernel<EPI, ST, BKN>), SMEM, opted_in)) return rc;
+    const unsigned wgs = ((p.big_tiles + 7) & ~7) + p.tiles_m * p.tiles_n;
+    hipLaunchKernelGGL((igemm_mixed_kernel<EPI, ST, BKN>), dim3(wgs), dim3(512), SMEM, st, p);
     return (int)hipGetLastError();
 }
 
@@ -1426,6 +1486,9 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs
     if constexpr (EPI != EPI_S32) {
         if (a.splits <= 1 && a.K <= TABLE_KB * QB && (long)((a.M + 31) / 32) * ((a.N + 127) / 128) <= 2L * cu_count())
             return launch_gemm_cfg<EPI, ST, 1, 1, 4, 3, 2, BKN>(a, st);
+    }
+    if constexpr (EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD) {
+        if (const int big = mixed_big_rows(a.M, a.N, a.K)) return launch_gemm_mixed<EPI, ST, BKN>(a, big, st);
     }
     return launch_gemm_cfg<EPI, ST, 2, 2, 4, 2, 2, BKN>(a, st);
 }

@@ -530,6 +530,31 @@ def test_both_tile_sizes_at_every_ring_fill(jf, oracle, M, N, K):
         same(sc, wsc, "SR scales")
 
 
+# 128x128 and 32x128 tiles in one launch (256 CUs): behind one big tile per CU the fewest and the most small ones and one row block more
+# (128x128 only), columns that end inside a tile; behind two the fewest and the most; behind four
+@pytest.mark.parametrize("M,N,K", [(5408, 768, 32), (6720, 768, 416), (6752, 768, 32), (4704, 800, 160), (10912, 768, 160), (13600, 768, 32),
+                                   (4352, 4096, 96)])
+def test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K):
+    print(f"case M={M} N={N} K={K}", flush=True)
+    A, Bkn, sa, sb = make_problem(M + N + K, M, N, K)
+    d = lambda t: dev(t.astype(np.float16))  # noqa: E731
+    dA, dsa, dsb, dkn, dnk = dev(A), d(sa), d(sb), dev(Bkn), dev(b_of(Bkn, 0))
+    q, sc = jf.igemm_block_q(dA, dnk, dsa, dsb, jf.B_NK)
+    wq, wsc = oracle.igemm_block_q(A, b_of(Bkn, 0), sa, sb, 0, scale_dtype="f16")
+    same(q, wq, "codes")
+    same(sc, wsc, "scales")
+    for got, want in zip(jf.igemm_block_q_gelu(dA, dnk, dsa, dsb), (q, sc) + tuple(jf.gelu_fwd(q, sc))):
+        assert torch.equal(got, want)
+    assert torch.equal(jf.igemm_block_q_dequant(dA, dnk, dsa, dsb, jf.B_NK, torch.float32), jf.dequantize(q, sc, torch.float32))
+    g, gs = jf.igemm_block_q(dA, dkn, dsa, dsb, jf.B_KN, rounding=jf.ROUND_STOCHASTIC, seed=4, offset=8)
+    wq, wsc = oracle.igemm_block_q(A, Bkn, sa, sb, 1, stochastic=True, seed=4, offset=8, scale_dtype="f16")
+    same(g, wq, "SR codes")
+    same(gs, wsc, "SR scales")
+    got = jf.igemm_block_q_gelu_bwd(dA, dkn, dsa, dsb, q, sc, seed=4, offset=8, gelu_seed=5, gelu_offset=4)
+    want = jf.gelu_bwd(q, sc, g, gs, rounding=jf.ROUND_STOCHASTIC, seed=5, offset=4)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("K", [32, 480, 512, 1056])               # one K block, the longest without and the shortest with a K split, a ragged split
 @pytest.mark.parametrize("widths", [[(96, 32)], [(384, 160), (128, 160), (512, 128), (32, 544)]])
 @pytest.mark.parametrize("f16,out", [(True, torch.float32), (False, torch.bfloat16)])
