@@ -862,18 +862,25 @@ __global__ __launch_bounds__(WAVE * LNB_DX_WAVES) void layernorm_bwd_dx_kernel(
 // without ADD, but instead of being stored it is dequantised again as a reader of the stored tensor would (codes x the
 // scale rounded to ST), added to x1, and the sum and its own block quantisation are what leaves -- the same bits as this
 // kernel without ADD followed by add_kernel, without dx's round trip through memory and the second launch.
+// Waves and pieces (launch_layernorm_bwd_strip).  WAVES = 16 fills a CU with one strip.  WAVES = 8, for up to 1024 columns, lets two
+// strips share a CU where there are more strips than CUs (16 waves hold no more than two blocks each then, and a second round of them
+// would follow).  Where there are fewer strips than CUs, `pieces` workgroups share a strip: all of them form all row sums (phase 1 without
+// column sums is a quarter of the work), each finishes every pieces-th of its waves' blocks.  us with the residual add, stochastic, 16
+// waves and one workgroup per strip | now: 256x2048 29.4 | 13.5, 64x1024 16.3 | 10.4, 1248x1120 17.8 | 10.9, 2048x768 13.0 | 10.7, 4096x1024
+// 17.9 | 13.0, 3072x1280 20.7 | 15.4 (pieces); 12288x768 27.8 | 26.3, 8224x768 25.9 | 24.1 (eight waves).
 constexpr int LNS_WAVES = 16, LNS_BPW = 4;
 constexpr int LNS_PATCH_ADD = QB * ADD_PITCH;      // floats per wave: the sum's patch, also used for the column sums
 static_assert(LNS_PATCH_ADD >= COLSUM_PATCH, "one patch per wave serves both");
-template <typename ST, bool WANT_DW, bool ADD>
-__global__ __launch_bounds__(WAVE * LNS_WAVES) void layernorm_bwd_strip_kernel(
+template <typename ST, bool WANT_DW, bool ADD, int WAVES>
+__global__ __launch_bounds__(WAVE * WAVES, 4) void layernorm_bwd_strip_kernel(
     const int8_t *qx, const ST *sx, const int8_t *qg, const ST *sg, const float *gamma, const float *mean,
     const float *rstd, int R, int C, int rounding, uint64_t seed, uint64_t offset, int8_t *qdx, ST *sdx, float *pdg,
-    float *pdb, LnAddArgs ad)
+    float *pdb, LnAddArgs ad, int pieces)
 {
     extern __shared__ __attribute__((aligned(16))) float lds_f[];  // gamma[C], part[2][C/32][32], T[2][8][32], c[2][32], patches
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int SC = C / QB, rb = blockIdx.x;
+    const int SC = C / QB, rb = blockIdx.x / pieces, piece = blockIdx.x - rb * pieces;
+    const auto own = [&](int i) { return i % pieces == piece; };   // block i of a wave is this workgroup's to finish
     float *gl = lds_f, *part = gl + C, *tj = part + 2 * SC * QB, *cs = tj + 2 * 8 * QB;
     float *cpatch = cs + 2 * QB + wave * (ADD ? LNS_PATCH_ADD : COLSUM_PATCH);   // (only with WANT_DW or ADD)
     const int row = rb * QB + (lane >> 1);
@@ -881,7 +888,7 @@ __global__ __launch_bounds__(WAVE * LNS_WAVES) void layernorm_bwd_strip_kernel(
     float scx[LNS_BPW], scg[LNS_BPW];
     static_for<0, LNS_BPW>([&](auto i_c) {
         constexpr int I = decltype(i_c)::value;
-        const int cb = wave + I * LNS_WAVES;
+        const int cb = wave + I * WAVES;
         if (cb < SC) {
             const size_t e0 = (size_t)row * C + cb * QB + (lane & 1) * 16;
             cx[I] = *reinterpret_cast<const v4i *>(qx + e0);
@@ -891,14 +898,14 @@ __global__ __launch_bounds__(WAVE * LNS_WAVES) void layernorm_bwd_strip_kernel(
         }
     });
     const float mu = mean[row], rs = rstd[row];
-    for (int c = threadIdx.x * 4; c < C; c += WAVE * LNS_WAVES * 4)
+    for (int c = threadIdx.x * 4; c < C; c += WAVE * WAVES * 4)
         *reinterpret_cast<v4f *>(gl + c) = *reinterpret_cast<const v4f *>(gamma + c);
     __syncthreads();
     const float b = -(mu * rs);
     // phase 1: block partials of the two row sums; column sums of the strip
     static_for<0, LNS_BPW>([&](auto i_c) {
         constexpr int I = decltype(i_c)::value;
-        const int cb = wave + I * LNS_WAVES;
+        const int cb = wave + I * WAVES;
         if (cb >= SC) return;                                      // uniform
         const int col = cb * QB + (lane & 1) * 16;
         const float a = scx[I] * rs, sgk = scg[I];
@@ -923,7 +930,7 @@ __global__ __launch_bounds__(WAVE * LNS_WAVES) void layernorm_bwd_strip_kernel(
             part[cb * QB + (lane >> 1)] = p1;
             part[(SC + cb) * QB + (lane >> 1)] = p2;
         }
-        if (WANT_DW) {
+        if (WANT_DW && own(I)) {
             // output of lane j (j even): value index j/4 of column set (j/2)%2
             const size_t dst = (size_t)rb * C + cb * QB + ((lane >> 1) & 1) * 16 + (lane >> 2);
             const float tg = colsum16_over_rows(x, lane, cpatch);
@@ -956,8 +963,8 @@ __global__ __launch_bounds__(WAVE * LNS_WAVES) void layernorm_bwd_strip_kernel(
     // phase 2: dx of the blocks still held as codes
     static_for<0, LNS_BPW>([&](auto i_c) {
         constexpr int I = decltype(i_c)::value;
-        const int cb = wave + I * LNS_WAVES;
-        if (cb >= SC) return;                                      // uniform
+        const int cb = wave + I * WAVES;
+        if (cb >= SC || !own(I)) return;                           // uniform
         const int col = cb * QB + (lane & 1) * 16;
         const size_t e0 = (size_t)row * C + col;
         const float a = scx[I] * rs, sgk = scg[I];
@@ -1403,13 +1410,29 @@ static int launch_layernorm_bwd_strip(const int8_t *qx, const void *sx, const in
     float *sdg = strip_dgamma ? strip_dgamma : (float *)workspace;          // [R/32][C] each: fits the workspace size
     float *sdb = dbeta && !strip_dgamma ? sdg + (size_t)(R / QB) * C : nullptr;
     const size_t patch = add ? LNS_PATCH_ADD : want_dw ? COLSUM_PATCH : 0;
-    const size_t lds = ((size_t)C + 2 * SC * QB + 2 * 8 * QB + 2 * QB + LNS_WAVES * patch) * sizeof(float);
     const LnAddArgs ad = add ? *add : LnAddArgs{};
+    const int strips = R / QB, cus = cu_count(), blocks = (SC + LNS_WAVES - 1) / LNS_WAVES;      // of a wave
+    const bool narrow = strips > cus && SC <= 8 * LNS_BPW;
+    int pieces = cus / strips < blocks ? cus / strips : blocks;
+    if (pieces < 1) pieces = 1;
+    if (pieces > 1) {                                              // a result in the place of an operand: one workgroup per strip reads before it writes
+        const size_t n = (size_t)R * C, ns = n / (QB * QB) * (scale_dtype == JF_SCALE_F16 ? 2 : 4);
+        const auto overlap = [](const void *a, size_t na, const void *b, size_t nb) {
+            const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+            return a && x < y + nb && y < x + na;
+        };
+        const void *const out[] = {qdx, sdx, ad.q, ad.s, ad.y1};
+        const size_t size[] = {n, ns, n, ns, n * (ad.y1_dtype == JF_FP_F32 ? 4 : 2)};
+        for (int i = 0; i < 5; ++i)
+            if (overlap(out[i], size[i], qx, n) || overlap(out[i], size[i], qg, n) || overlap(out[i], size[i], sx, ns) || overlap(out[i], size[i], sg, ns))
+                pieces = 1;
+    }
+    const size_t lds = ((size_t)C + 2 * SC * QB + 2 * 8 * QB + 2 * QB + (narrow ? 8 : LNS_WAVES) * patch) * sizeof(float);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return JF_ERR_DEVICE;
-#define JF_LNS(ST, DW, ADD)                                                                                            \
+#define JF_LNS(ST, DW, ADD, WAVES)                                                                                     \
     do {                                                                                                               \
-        auto kern = layernorm_bwd_strip_kernel<ST, DW, ADD>;                                                           \
+        auto kern = layernorm_bwd_strip_kernel<ST, DW, ADD, WAVES>;                                                    \
         static std::atomic<bool> opted_in[MAX_DEVICES] = {};      /* more than 64 KiB of LDS: once per device */        \
         if (lds > 64 * 1024 && !opted_in[dev].load(std::memory_order_acquire)) {                                       \
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),                                   \
@@ -1417,14 +1440,16 @@ static int launch_layernorm_bwd_strip(const int8_t *qx, const void *sx, const in
             if (e != hipSuccess) return (int)e;                                                                        \
             opted_in[dev].store(true, std::memory_order_release);                                                      \
         }                                                                                                              \
-        hipLaunchKernelGGL(kern, dim3(R / QB), dim3(WAVE * LNS_WAVES), lds, st, qx, (const ST *)sx, qg,                \
+        hipLaunchKernelGGL(kern, dim3(strips * pieces), dim3(WAVE * WAVES), lds, st, qx, (const ST *)sx, qg,           \
                            (const ST *)sg, gamma, mean, rstd, R, C, rounding, seed, offset, qdx, (ST *)sdx,            \
-                           DW ? sdg : nullptr, DW ? sdb : nullptr, ad);                                                \
+                           DW ? sdg : nullptr, DW ? sdb : nullptr, ad, pieces);                                        \
     } while (0)
-#define JF_LNS_DW(ST, ADD) do { if (want_dw) JF_LNS(ST, true, ADD); else JF_LNS(ST, false, ADD); } while (0)
+#define JF_LNS_W(ST, DW, ADD) do { if (narrow) JF_LNS(ST, DW, ADD, 8); else JF_LNS(ST, DW, ADD, LNS_WAVES); } while (0)
+#define JF_LNS_DW(ST, ADD) do { if (want_dw) JF_LNS_W(ST, true, ADD); else JF_LNS_W(ST, false, ADD); } while (0)
     if (scale_dtype == JF_SCALE_F16) { if (add) JF_LNS_DW(half_t, true); else JF_LNS_DW(half_t, false); }
     else { if (add) JF_LNS_DW(float, true); else JF_LNS_DW(float, false); }
 #undef JF_LNS_DW
+#undef JF_LNS_W
 #undef JF_LNS
     if (want_dw && !strip_dgamma)
         hipLaunchKernelGGL(layernorm_bwd_colsum_finish_kernel, dim3(SC, dbeta ? 2 : 1), dim3(1024), 0, st, sdg, sdb, R / QB, C, dgamma, dbeta);

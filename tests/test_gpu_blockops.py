@@ -354,6 +354,31 @@ def test_layernorm_backward_single_pass_and_two_launch_forms(jf, oracle, R, C):
     test_rowstats_layernorm(jf, oracle, R, C, True)
 
 
+# (256 CUs) strips in three pieces, in two of three possible ones; more strips than CUs: eight waves a strip, with two, four blocks each,
+# and one column block too many for them
+@pytest.mark.parametrize("R,C", [(32, 1120), (4096, 1120), (8224, 512), (8224, 1024), (8224, 1056)])
+def test_layernorm_backward_workgroups_per_strip(jf, oracle, R, C):
+    test_rowstats_layernorm(jf, oracle, R, C, True)
+    test_layernorm_backward_with_the_residual_add(jf, R, C, torch.bfloat16, torch.bfloat16, torch.float16)
+
+
+def test_layernorm_backward_in_the_place_of_its_gradient(jf):
+    """dx over the incoming gradient (codes and scales): a strip then has one workgroup, which reads it before it writes."""
+    g = torch.Generator().manual_seed(3)
+    R, C = 64, 2048
+    qx, sx = jf.quantize(torch.randn(R, C, generator=g).cuda())
+    qg, sg = jf.quantize(torch.randn(R, C, generator=g).cuda())
+    gamma = torch.randn(C, generator=g).cuda()
+    mean, rstd = jf.rowstats(qx, sx)
+    want = jf.layernorm_bwd(qx, sx, qg, sg, gamma, mean, rstd, jf.ROUND_STOCHASTIC, False, seed=7, offset=3)
+    n = jf.lib().jf_layernorm_bwd_workspace_bytes(R, C)
+    ws, dg = torch.empty(n, dtype=torch.int8, device="cuda"), torch.empty(C, device="cuda")
+    p = lambda t: t.data_ptr()  # noqa: E731
+    jf.check(jf.lib().jf_layernorm_bwd(p(qx), p(sx), p(qg), p(sg), p(gamma), p(mean), p(rstd), R, C, jf.SCALE_F16, jf.ROUND_STOCHASTIC, 7, 3, p(qg),
+                                       p(sg), p(dg), None, p(ws), n, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(qg, want[0]) and torch.equal(sg, want[1]) and torch.equal(dg, want[2])
+
+
 @pytest.mark.parametrize("R,C,f16,approx", list(_random_block_shapes(12, 7)))
 def test_random_shapes(jf, oracle, R, C, f16, approx):
     """The GELU and LayerNorm checks above on random tensor shapes (up to 320 x 4128: rows of more column blocks than a
