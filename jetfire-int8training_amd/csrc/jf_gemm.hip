@@ -116,8 +116,8 @@ constexpr int WBN = 1;
 constexpr int gemm_threads(int WBM, int WGM, int WGN) { return 64 * WGM * WGN * (WBM == 1 ? 2 : 1); }
 constexpr int TABLE_KB = 512;                        // K blocks a wave's table of scale products holds (WBM = 1)
 // LDS of a workgroup: the operand ring; per-wave scale and product patches or tables; from gelu_lds_at on what the GELU tables of the
-// epilogue need beyond those (WBM = 2: the byte tables, 256 bytes per wave; WBM = 1: both, 1280 bytes).  Epilogues that go through
-// LDS use the ring.
+// epilogue need beyond those (WBM = 2: the forward's byte tables, 256 bytes per wave; WBM = 1: both, 1280 bytes).  Epilogues that go
+// through LDS use the ring.
 constexpr int gelu_lds_at(int WBM, int WGM, int WGN, int NSTAGE)
 {
     const int scales = WBM == 1 ? 4 * (TABLE_KB + KB_STAGE) * WGM * WGN : NSTAGE * WGM * WGN * 512;
@@ -125,7 +125,7 @@ constexpr int gelu_lds_at(int WBM, int WGM, int WGN, int NSTAGE)
 }
 constexpr int gemm_lds(int EPI, int WBM, int WGM, int WGN, int NSTAGE)
 {
-    const int tables = EPI == EPI_QG || EPI == EPI_QB ? (WBM == 1 ? 1280 : 256) * WGM * WGN : 0;
+    const int tables = (WBM == 1 ? (EPI == EPI_QG || EPI == EPI_QB) * 1280 : (EPI == EPI_QG) * 256) * WGM * WGN;
     const int used = gelu_lds_at(WBM, WGM, WGN, NSTAGE) + tables, patch = WGM * WGN * QB * EPI_LD * (int)sizeof(float);
     return used > patch ? used : patch;
 }
@@ -1489,6 +1489,17 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs
     }
     if constexpr (EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD) {
         if (const int big = mixed_big_rows(a.M, a.N, a.K)) return launch_gemm_mixed<EPI, ST, BKN>(a, big, st);
+    }
+    // 64x128 tiles, four waves of two blocks, three workgroups per CU: where they are all resident at once (up to 384 big tiles), the
+    // 128x128 tiles would be alone on many of their CUs, and a SIMD's waves belong to workgroups that do not wait for each other.  us,
+    // 128x128 | 64x128: 7168x768x768 (336 big tiles) 15.3 | 12.8, 8192x768x768 (384) 15.4 | 13.1, x3072 43.6 | 41.0, 768x8192x2048 (384) 30.3 |
+    // 27.8, 3072x1024x4096 (192) 37.5 | 34.9, 2048x1600x1600 (208) 17.6 | 16.9, 1248x2304x768 (180) 10.7 | 10.3; two rounds of them: 2560x2560x2560
+    // (400) 37.1 | 47.4.  Not with the GELU forward behind it, whose byte tables leave room for two workgroups only; with its backward,
+    // the longest epilogue, above one big tile per CU: 2048x3072x768 (384) 22.0 | 19.8, 1248x3072x768 (240) 15.2 | 15.6.
+    if constexpr (EPI == EPI_Q || EPI == EPI_QB || EPI == EPI_QD) {
+        const long tiles_n = (a.N + 127) / 128;
+        if ((a.M + 63) / 64 * tiles_n <= 3L * cu_count() && (EPI != EPI_QB || (a.M + 127) / 128 * tiles_n > cu_count()))
+            return launch_gemm_cfg<EPI, ST, 2, 1, 4, 2, 3, BKN>(a, st);
     }
     return launch_gemm_cfg<EPI, ST, 2, 2, 4, 2, 2, BKN>(a, st);
 }

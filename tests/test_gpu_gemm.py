@@ -530,6 +530,12 @@ def test_both_tile_sizes_at_every_ring_fill(jf, oracle, M, N, K):
         same(sc, wsc, "SR scales")
 
 
+# 425 tiles of 128x128 (825 of 64x128, which would not all be resident), the last row and column of them ragged: every ring fill
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 288, 384, 416])
+def test_the_large_tiles_at_every_ring_fill(jf, oracle, K):
+    test_both_tile_sizes_at_every_ring_fill(jf, oracle, 2080, 3104, K)
+
+
 # 128x128 and 32x128 tiles in one launch (256 CUs): behind one big tile per CU the fewest and the most small ones and one row block more
 # (128x128 only), columns that end inside a tile; behind two the fewest and the most; behind four
 @pytest.mark.parametrize("M,N,K", [(5408, 768, 32), (6720, 768, 416), (6752, 768, 32), (4704, 800, 160), (10912, 768, 160), (13600, 768, 32),
