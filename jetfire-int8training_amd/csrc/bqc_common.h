@@ -6,7 +6,9 @@
 #include <torch/extension.h>
 
 #include <ATen/detail/CUDAHooksInterface.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <mutex>
@@ -18,6 +20,24 @@ namespace jfext {
 
 
 constexpr int QB = 32;
+
+// The memory of a result or of a workspace: torch::empty, but straight from the function that the dispatcher's GPU entry
+// ends in.  An operator here is one or two launches of a few microseconds of host time each and allocates up to seven
+// tensors.  Whatever could watch or change such an allocation keeps the dispatcher: a dispatch mode (a tracer, a fake
+// tensor), a request to fill new memory, any device but the GPU.  Host time per call with the
+// dispatcher and so (runs in turn): quantise 6.6 and 6.2 us, add with statistics 14.1 and 12.7, LayerNorm
+// backward with add 15.1 and 14.2, seven such calls on 32 x 128 elements 61.3 and 57.2.
+inline torch::Tensor fresh(at::IntArrayRef sizes, const at::TensorOptions &opt)
+{
+    if (!opt.device().is_cuda() || c10::impl::dispatch_mode_enabled() || at::globalContext().deterministicAlgorithms())
+        return torch::empty(sizes, opt);
+    return torch::Tensor(at::detail::empty_cuda(sizes, opt));
+}
+
+inline torch::Tensor fresh_like(const torch::Tensor &t)
+{
+    return t.is_contiguous() ? fresh(t.sizes(), t.options()) : torch::empty_like(t);
+}
 
 inline void check_rc(int rc, const char *what)
 {
@@ -122,7 +142,7 @@ struct Workspace {
     {
         bytes = nbytes;
         if (bytes) {
-            t = torch::empty({(int64_t)bytes}, like.options().dtype(torch::kInt8));
+            t = fresh({(int64_t)bytes}, like.options().dtype(torch::kInt8));
             ptr = t.data_ptr();
         }
     }

@@ -37,8 +37,8 @@ std::tuple<torch::Tensor, torch::Tensor> block_q(const torch::Tensor &X, const t
         biasmax_p = biasmax->data_ptr<float>();
     }
     c10::DeviceGuard guard(X.device());
-    torch::Tensor O = torch::empty({M, N}, X.options().dtype(torch::kInt8));
-    torch::Tensor SO = torch::empty({M / QB, N / QB}, SX.options().memory_format(c10::MemoryFormat::Contiguous));
+    torch::Tensor O = fresh({M, N}, X.options().dtype(torch::kInt8));
+    torch::Tensor SO = fresh({M / QB, N / QB}, SX.options().memory_format(c10::MemoryFormat::Contiguous));
     Workspace ws(X, M, N, K, layout);
     uint64_t seed = 0, offset = 0;
     if (rounding == JF_ROUND_STOCHASTIC) std::tie(seed, offset) = next_philox(X, (int64_t)M * N);
@@ -63,7 +63,7 @@ torch::Tensor igemm_basic_int8_gemm(torch::Tensor X, torch::Tensor W, const int 
     check_a(X, M, K);
     check_b_kn(W, X, K, N);
     c10::DeviceGuard guard(X.device());
-    torch::Tensor O = torch::empty({M, N}, X.options().dtype(torch::kInt32));
+    torch::Tensor O = fresh({M, N}, X.options().dtype(torch::kInt32));
     Workspace ws(X, M, N, K, JF_B_KN);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_igemm_s32((const int8_t *)X.data_ptr(), (const int8_t *)W.data_ptr(), (int32_t *)O.data_ptr(), M, N, K,
@@ -90,7 +90,7 @@ torch::Tensor igemm_output_fp_no_quantize(torch::Tensor X, torch::Tensor W, torc
     int sxl, swl;
     const int code = check_scales(SX, SW, X, M, N, K, sxl, swl);
     c10::DeviceGuard guard(X.device());
-    torch::Tensor O = torch::empty({M, N}, X.options().dtype(odt));
+    torch::Tensor O = fresh({M, N}, X.options().dtype(odt));
     TORCH_CHECK(splitk >= 0, "splitk must be >= 0");
     Workspace ws(X, jf_igemm_block_fp_workspace_bytes(M, N, K, JF_B_KN, splitk));
     pybind11::gil_scoped_release nogil;

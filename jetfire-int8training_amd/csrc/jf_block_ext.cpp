@@ -175,19 +175,19 @@ BlockForward forward_impl(const Dims &d, const Tensor &x, const Tensor &qx, cons
     Saved v;
     ForwardTemp t;
     BlockForward r;
-    Tensor temp = torch::empty({(int64_t)(keep ? t.carve(nullptr, d) : carve_inference(nullptr, d, v, t))}, opt.dtype(torch::kUInt8));
+    Tensor temp = fresh({(int64_t)(keep ? t.carve(nullptr, d) : carve_inference(nullptr, d, v, t))}, opt.dtype(torch::kUInt8));
     if (keep) {
-        r.saved = torch::empty({(int64_t)v.carve(nullptr, d)}, opt.dtype(torch::kUInt8));
+        r.saved = fresh({(int64_t)v.carve(nullptr, d)}, opt.dtype(torch::kUInt8));
         v.carve((uint8_t *)r.saved.data_ptr(), d);
         t.carve((uint8_t *)temp.data_ptr(), d);
     } else {
         carve_inference((uint8_t *)temp.data_ptr(), d, v, t);
     }
-    r.fp = torch::empty({d.B, d.T, C}, opt.dtype(out_dtype));
-    r.q = torch::empty({d.B, d.T, C}, opt.dtype(torch::kFloat8_e4m3fn));
-    r.s = torch::empty({d.B, d.T / QB, C / QB}, opt.dtype(torch::kFloat16));
-    r.mean = torch::empty({d.B, d.T}, opt.dtype(torch::kFloat32));
-    r.rstd = torch::empty({d.B, d.T}, opt.dtype(torch::kFloat32));
+    r.fp = fresh({d.B, d.T, C}, opt.dtype(out_dtype));
+    r.q = fresh({d.B, d.T, C}, opt.dtype(torch::kFloat8_e4m3fn));
+    r.s = fresh({d.B, d.T / QB, C / QB}, opt.dtype(torch::kFloat16));
+    r.mean = fresh({d.B, d.T}, opt.dtype(torch::kFloat32));
+    r.rstd = fresh({d.B, d.T}, opt.dtype(torch::kFloat32));
     const jf_stream_t st = current_stream(x);
     constexpr int RM = JF_SCALES_ROWMAJOR, F16 = JF_SCALE_F16;
     const int m = d.M, c = d.C;
@@ -281,18 +281,18 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         if (with_bias) ws_bytes = std::max(ws_bytes, jf_block_colsum_workspace_bytes(m, 4 * c));
         BackwardTemp t;
         const size_t res_bytes = torch::elementSize(res_type);
-        Tensor temp = torch::empty({(int64_t)t.carve(nullptr, d, res_bytes, ws_bytes)}, opt.dtype(torch::kUInt8));
+        Tensor temp = fresh({(int64_t)t.carve(nullptr, d, res_bytes, ws_bytes)}, opt.dtype(torch::kUInt8));
         t.carve((uint8_t *)temp.data_ptr(), d, res_bytes, ws_bytes);
 
         variable_list out(N_GRAD + 5);                         // (one entry per argument of forward)
-        out[X] = torch::empty({B, T, C}, opt.dtype(res_type));
-        out[QX] = torch::empty({B, T, C}, opt.dtype(torch::kFloat8_e4m3fn));
-        out[SX] = torch::empty({B, T / QB, C / QB}, opt.dtype(torch::kFloat16));
-        out[LN1] = torch::empty({C}, opt.dtype(torch::kFloat32));
-        out[LN2] = torch::empty({C}, opt.dtype(torch::kFloat32));
-        for (int i = 0; i < 4; ++i) out[W_QKV + i] = torch::empty({wrows[i], wcols[i]}, opt.dtype(w_type));
+        out[X] = fresh({B, T, C}, opt.dtype(res_type));
+        out[QX] = fresh({B, T, C}, opt.dtype(torch::kFloat8_e4m3fn));
+        out[SX] = fresh({B, T / QB, C / QB}, opt.dtype(torch::kFloat16));
+        out[LN1] = fresh({C}, opt.dtype(torch::kFloat32));
+        out[LN2] = fresh({C}, opt.dtype(torch::kFloat32));
+        for (int i = 0; i < 4; ++i) out[W_QKV + i] = fresh({wrows[i], wcols[i]}, opt.dtype(w_type));
         if (with_bias)
-            for (int i = 0; i < 4; ++i) out[B_QKV + i] = torch::empty({wrows[i]}, opt.dtype(torch::kFloat32));
+            for (int i = 0; i < 4; ++i) out[B_QKV + i] = fresh({wrows[i]}, opt.dtype(torch::kFloat32));
         const int resc = fp_of(out[X], "residual"), wc = fp_of(out[W_QKV], "weight"), fpgc = fp_of(fpg, "gradient");
 
         // Philox counters, drawn in the order of the separate Functions (the reservations below are what each would make)

@@ -78,7 +78,7 @@ std::vector<int64_t> scale_shape(const Tensor &x)
 // scales of a result laid out like the codes q (an operand's own scales may have another rank: [B, T, C] with [B T/32, C/32])
 Tensor scales_for(const Tensor &q, const Tensor &s)
 {
-    return torch::empty(scale_shape(q), s.options());
+    return fresh(scale_shape(q), s.options());
 }
 
 // one value per row, [R] or [B, T]
@@ -124,7 +124,7 @@ std::pair<uint64_t, uint64_t> rng(int64_t rounding, const Tensor &like, int64_t 
 
 Tensor scratch(const Tensor &like, size_t bytes)
 {
-    return torch::empty({(int64_t)(bytes ? bytes : 16)}, like.options().dtype(torch::kInt8));
+    return fresh({(int64_t)(bytes ? bytes : 16)}, like.options().dtype(torch::kInt8));
 }
 
 // ---- quantize / dequantize / transpose -----------------------------------------------------------------------------
@@ -141,10 +141,10 @@ std::tuple<Tensor, Tensor, OptTensor> quantize(const Tensor &x, int64_t rounding
     const torch::ScalarType scale_dtype = scale_dtype_o.value_or(torch::kFloat16);
     const int sc = scale_code_of(scale_dtype);
     c10::DeviceGuard guard(x.device());
-    Tensor q = torch::empty(x.sizes(), x.options().dtype(torch::kInt8));
-    Tensor s = torch::empty(scale_shape(x), x.options().dtype(scale_dtype));
+    Tensor q = fresh(x.sizes(), x.options().dtype(torch::kInt8));
+    Tensor s = fresh(scale_shape(x), x.options().dtype(scale_dtype));
     OptTensor qT;
-    if (transpose) qT = torch::empty({C, R}, x.options().dtype(torch::kInt8));
+    if (transpose) qT = fresh({C, R}, x.options().dtype(torch::kInt8));
     const auto so = rng(rounding, x, R * C, seed, offset);
     {
         pybind11::gil_scoped_release nogil;
@@ -174,7 +174,7 @@ std::vector<std::tuple<Tensor, Tensor>> quantize_many(const std::vector<Tensor> 
         rows_of(x, "xs", R, C);
         mult32(R); mult32(C);
         TORCH_CHECK(x.scalar_type() == xs[0].scalar_type() && x.device() == xs[0].device(), "xs: expected tensors of one type and device");
-        Tensor q = torch::empty(x.sizes(), x.options().dtype(torch::kInt8)), s = torch::empty(scale_shape(x), x.options().dtype(scale_dtype));
+        Tensor q = fresh(x.sizes(), x.options().dtype(torch::kInt8)), s = fresh(scale_shape(x), x.options().dtype(scale_dtype));
         xp[k] = x.data_ptr(); Rs[k] = (int)R; Cs[k] = (int)C; qp[k] = (int8_t *)q.data_ptr(); sp[k] = s.data_ptr();
         out.emplace_back(std::move(q), std::move(s));
     }
@@ -191,7 +191,7 @@ std::tuple<Tensor, Tensor> rowstats_fp(const Tensor &x)
     mult32(C);
     const int xc = fp_code(x.scalar_type(), "x");
     c10::DeviceGuard guard(x.device());
-    Tensor mean = torch::empty(row_shape(x), x.options().dtype(torch::kFloat32)), rstd = torch::empty_like(mean);
+    Tensor mean = fresh(row_shape(x), x.options().dtype(torch::kFloat32)), rstd = fresh_like(mean);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_rowstats_fp(x.data_ptr(), xc, (int)R, (int)C, mean.data_ptr<float>(), rstd.data_ptr<float>(), current_stream(x)), "rowstats_fp");
     return std::make_tuple(mean, rstd);
@@ -222,8 +222,8 @@ std::tuple<Tensor, Tensor> quantize_slabs(const std::vector<Tensor> &slabs, int6
     const torch::ScalarType scale_dtype = scale_dtype_o.value_or(torch::kFloat16);
     const int sc = scale_code_of(scale_dtype);
     c10::DeviceGuard guard(x0.device());
-    Tensor q = torch::empty({R, Ct}, x0.options().dtype(torch::kInt8));
-    Tensor s = torch::empty({R / QB, Ct / QB}, x0.options().dtype(scale_dtype));
+    Tensor q = fresh({R, Ct}, x0.options().dtype(torch::kInt8));
+    Tensor s = fresh({R / QB, Ct / QB}, x0.options().dtype(scale_dtype));
     const auto so = rng(rounding, x0, R * Ct, seed, offset);
     {
         pybind11::gil_scoped_release nogil;
@@ -242,7 +242,7 @@ Tensor dequantize(const Tensor &q, const Tensor &s, OptDtype out_dtype_o)
     const int sc = block_tensor(q, s, "x", R, C);
     const int oc = fp_code(out_dtype, "out_dtype");
     c10::DeviceGuard guard(q.device());
-    Tensor out = torch::empty(q.sizes(), q.options().dtype(out_dtype));
+    Tensor out = fresh(q.sizes(), q.options().dtype(out_dtype));
     pybind11::gil_scoped_release nogil;
     check_rc(jf_dequantize((const int8_t *)q.data_ptr(), s.data_ptr(), (int)R, (int)C, sc, out.data_ptr(), oc, current_stream(q)),
              "dequantize");
@@ -257,7 +257,7 @@ Tensor transpose_s8(const Tensor &q)
     TORCH_CHECK(q.scalar_type() == torch::kInt8, "x must be int8");
     TORCH_CHECK(R > 0 && C > 0 && R % 16 == 0 && C % 16 == 0, "transpose: dimensions must be positive multiples of 16");
     c10::DeviceGuard guard(q.device());
-    Tensor out = torch::empty({C, R}, q.options());
+    Tensor out = fresh({C, R}, q.options());
     pybind11::gil_scoped_release nogil;
     check_rc(jf_transpose_s8((const int8_t *)q.data_ptr(), (int)R, (int)C, (int8_t *)out.data_ptr(), current_stream(q)), "transpose");
     return out;
@@ -270,7 +270,7 @@ std::tuple<Tensor, Tensor> rowstats(const Tensor &q, const Tensor &s, double eps
     int64_t R, C;
     const int sc = block_tensor(q, s, "x", R, C);
     c10::DeviceGuard guard(q.device());
-    Tensor mean = torch::empty(row_shape(q), q.options().dtype(torch::kFloat32)), rstd = torch::empty_like(mean);
+    Tensor mean = fresh(row_shape(q), q.options().dtype(torch::kFloat32)), rstd = fresh_like(mean);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_rowstats((const int8_t *)q.data_ptr(), s.data_ptr(), (int)R, (int)C, sc, (float)eps, mean.data_ptr<float>(),
                          rstd.data_ptr<float>(), current_stream(q)),
@@ -287,7 +287,7 @@ std::tuple<Tensor, Tensor> layernorm_fwd(const Tensor &q, const Tensor &s, const
     const float *g = vec(gamma, C, q, "gamma"), *b = beta ? vec(*beta, C, q, "beta") : nullptr;
     const float *m = vec(mean, R, q, "mean"), *r = vec(rstd, R, q, "rstd");
     c10::DeviceGuard guard(q.device());
-    Tensor qy = torch::empty_like(q), sy = scales_for(q, s);
+    Tensor qy = fresh_like(q), sy = scales_for(q, s);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_layernorm_fwd((const int8_t *)q.data_ptr(), s.data_ptr(), g, b, m, r, (int)R, (int)C, sc, (int8_t *)qy.data_ptr(),
                               sy.data_ptr(), current_stream(q)),
@@ -309,10 +309,10 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor> layernorm_bwd(const Tensor &qx, co
     c10::DeviceGuard guard(qx.device());
     const size_t nbytes = jf_layernorm_bwd_workspace_bytes((int)R, (int)C);
     Tensor ws = scratch(qx, nbytes);
-    Tensor qdx = torch::empty_like(qx), sdx = scales_for(qx, sx);
-    Tensor dgamma = torch::empty({C}, qx.options().dtype(torch::kFloat32));
+    Tensor qdx = fresh_like(qx), sdx = scales_for(qx, sx);
+    Tensor dgamma = fresh({C}, qx.options().dtype(torch::kFloat32));
     OptTensor dbeta;
-    if (want_dbeta) dbeta = torch::empty_like(dgamma);
+    if (want_dbeta) dbeta = fresh_like(dgamma);
     const auto so = rng(rounding, qx, R * C, seed, offset);
     {
         pybind11::gil_scoped_release nogil;
@@ -338,15 +338,15 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor, OptTensor> add(const Tensor &x1, c
     TORCH_CHECK(R1 == R && C1 == C && x1.device() == q2.device(), "x1 must be a float tensor of the shape and device of x2");
     check_rounding(rounding, true);
     c10::DeviceGuard guard(x1.device());
-    Tensor y1 = torch::empty(x1.sizes(), x1.options().dtype(out_dtype));
-    Tensor q = torch::empty(x1.sizes(), q2.options()), s = torch::empty(scale_shape(x1), s2.options());
+    Tensor y1 = fresh(x1.sizes(), x1.options().dtype(out_dtype));
+    Tensor q = fresh(x1.sizes(), q2.options()), s = fresh(scale_shape(x1), s2.options());
     Tensor rs, rq;
     OptTensor mean, rstd;
     if (with_stats) {
-        rs = torch::empty({C / QB, R}, x1.options().dtype(torch::kFloat32));          // part-major
-        rq = torch::empty_like(rs);
-        mean = torch::empty(row_shape(x1), x1.options().dtype(torch::kFloat32));
-        rstd = torch::empty_like(*mean);
+        rs = fresh({C / QB, R}, x1.options().dtype(torch::kFloat32));          // part-major
+        rq = fresh_like(rs);
+        mean = fresh(row_shape(x1), x1.options().dtype(torch::kFloat32));
+        rstd = fresh_like(*mean);
     }
     const auto so = rng(rounding, x1, R * C, seed, offset);
     {
@@ -395,11 +395,11 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor> layernorm_bwd_add(const Te
     c10::DeviceGuard guard(qx.device());
     const size_t nbytes = jf_layernorm_bwd_workspace_bytes((int)R, (int)C);
     Tensor ws = scratch(qx, nbytes);
-    Tensor y1 = torch::empty(qx.sizes(), x1.options().dtype(out_dtype));
-    Tensor q = torch::empty_like(qx), s = scales_for(qx, sx);
-    Tensor dgamma = torch::empty({C}, qx.options().dtype(torch::kFloat32));
+    Tensor y1 = fresh(qx.sizes(), x1.options().dtype(out_dtype));
+    Tensor q = fresh_like(qx), s = scales_for(qx, sx);
+    Tensor dgamma = fresh({C}, qx.options().dtype(torch::kFloat32));
     OptTensor dbeta;
-    if (want_dbeta) dbeta = torch::empty_like(dgamma);
+    if (want_dbeta) dbeta = fresh_like(dgamma);
     {
         pybind11::gil_scoped_release nogil;
         check_rc(jf_layernorm_bwd_add((const int8_t *)qx.data_ptr(), sx.data_ptr(), (const int8_t *)qg.data_ptr(), sg.data_ptr(), g, m, r,
@@ -423,7 +423,7 @@ std::tuple<Tensor, Tensor> gelu_fwd(const Tensor &q, const Tensor &s, int64_t ap
     const int sc = block_tensor(q, s, "x", R, C);
     check_approx(approx);
     c10::DeviceGuard guard(q.device());
-    Tensor qy = torch::empty_like(q), sy = scales_for(q, s);
+    Tensor qy = fresh_like(q), sy = scales_for(q, s);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_gelu_fwd((const int8_t *)q.data_ptr(), s.data_ptr(), (int)R, (int)C, sc, (int)approx, (float)amax_eps,
                          (int8_t *)qy.data_ptr(), sy.data_ptr(), current_stream(q)),
@@ -442,7 +442,7 @@ std::tuple<Tensor, Tensor> gelu_bwd(const Tensor &qx, const Tensor &sx, const Te
     check_approx(approx);
     check_rounding(rounding, true);
     c10::DeviceGuard guard(qx.device());
-    Tensor qy = torch::empty_like(qx), sy = scales_for(qx, sx);
+    Tensor qy = fresh_like(qx), sy = scales_for(qx, sx);
     const auto so = rng(rounding, qx, R * C, seed, offset);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_gelu_bwd((const int8_t *)qx.data_ptr(), sx.data_ptr(), (const int8_t *)qg.data_ptr(), sg.data_ptr(), (int)R, (int)C, sc,
@@ -476,7 +476,7 @@ std::tuple<Tensor, Tensor> attention_fwd(const Tensor &q, const Tensor &k, const
 {
     const AttentionOperands a = attention_operands(q, k, v, batch, heads);
     c10::DeviceGuard guard(q.device());
-    Tensor out = torch::empty({q.size(0), a.C}, q.options()), lse = torch::empty({(int64_t)a.B * a.H, a.T}, q.options().dtype(torch::kFloat32));
+    Tensor out = fresh({q.size(0), a.C}, q.options()), lse = fresh({(int64_t)a.B * a.H, a.T}, q.options().dtype(torch::kFloat32));
     pybind11::gil_scoped_release nogil;
     check_rc(jf_attention_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), a.ld, a.B, a.H, a.T, a.D, a.scale, out.data_ptr(),
                               lse.data_ptr<float>(), current_stream(q)),
@@ -501,7 +501,7 @@ Tensor attention_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Te
     const AttentionOperands a = attention_operands(q, k, v, batch, heads);
     attention_gradient_operands(q, out, lse, gout, a);
     c10::DeviceGuard guard(q.device());
-    Tensor g = torch::empty({q.size(0), 3 * a.C}, q.options()), delta = torch::empty_like(lse);
+    Tensor g = fresh({q.size(0), 3 * a.C}, q.options()), delta = fresh_like(lse);
     c10::Half *gp = g.data_ptr<c10::Half>();
     pybind11::gil_scoped_release nogil;
     check_rc(jf_attention_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), a.ld, out.data_ptr(), gout.data_ptr(), lse.data_ptr<float>(), a.B,
@@ -516,8 +516,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> attention_fwd_q(const Tensor &q, cons
     const AttentionOperands a = attention_operands(q, k, v, batch, heads);
     c10::DeviceGuard guard(q.device());
     const int64_t M = q.size(0);
-    Tensor out = torch::empty({M, a.C}, q.options()), lse = torch::empty({(int64_t)a.B * a.H, a.T}, q.options().dtype(torch::kFloat32));
-    Tensor codes = torch::empty({M, a.C}, q.options().dtype(torch::kInt8)), scales = torch::empty({M / QB, a.C / QB}, q.options());
+    Tensor out = fresh({M, a.C}, q.options()), lse = fresh({(int64_t)a.B * a.H, a.T}, q.options().dtype(torch::kFloat32));
+    Tensor codes = fresh({M, a.C}, q.options().dtype(torch::kInt8)), scales = fresh({M / QB, a.C / QB}, q.options());
     pybind11::gil_scoped_release nogil;
     check_rc(jf_attention_fwd_q(q.data_ptr(), k.data_ptr(), v.data_ptr(), a.ld, a.B, a.H, a.T, a.D, a.scale, out.data_ptr(), lse.data_ptr<float>(),
                                 (int8_t *)codes.data_ptr(), scales.data_ptr(), current_stream(q)),
@@ -533,8 +533,8 @@ std::tuple<Tensor, Tensor> attention_bwd_q(const Tensor &q, const Tensor &k, con
     attention_gradient_operands(q, out, lse, gout, a);
     c10::DeviceGuard guard(q.device());
     const int64_t M = q.size(0);
-    Tensor codes = torch::empty({M, 3 * a.C}, q.options().dtype(torch::kInt8)), scales = torch::empty({M / QB, 3 * a.C / QB}, q.options());
-    Tensor delta = torch::empty_like(lse);
+    Tensor codes = fresh({M, 3 * a.C}, q.options().dtype(torch::kInt8)), scales = fresh({M / QB, 3 * a.C / QB}, q.options());
+    Tensor delta = fresh_like(lse);
     const auto so = rng(JF_ROUND_STOCHASTIC, q, 3 * M * a.C, seed, offset);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_attention_bwd_q(q.data_ptr(), k.data_ptr(), v.data_ptr(), a.ld, out.data_ptr(), gout.data_ptr(), lse.data_ptr<float>(), a.B, a.H, a.T,
@@ -553,7 +553,7 @@ Tensor block_colsum(const Tensor &q, const Tensor &s)
     c10::DeviceGuard guard(q.device());
     const size_t nbytes = jf_block_colsum_workspace_bytes((int)R, (int)C);
     Tensor ws = scratch(q, nbytes);
-    Tensor out = torch::empty({C}, q.options().dtype(torch::kFloat32));
+    Tensor out = fresh({C}, q.options().dtype(torch::kFloat32));
     pybind11::gil_scoped_release nogil;
     check_rc(jf_block_colsum((const int8_t *)q.data_ptr(), s.data_ptr(), (int)R, (int)C, sc, out.data_ptr<float>(), ws.data_ptr(), nbytes,
                              current_stream(q)),
@@ -603,9 +603,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> igemm_block_q_gelu(const Tensor &A, c
     const GemmOperands g = gemm_operands(A, B, sa, sb, JF_B_NK, bias, biasmax);
     check_approx(approx);
     c10::DeviceGuard guard(A.device());
-    Tensor q = torch::empty({g.M, g.N}, A.options());
-    Tensor s = torch::empty({g.M / QB, g.N / QB}, sa.options().memory_format(c10::MemoryFormat::Contiguous));
-    Tensor qg = torch::empty_like(q), sg = torch::empty_like(s);
+    Tensor q = fresh({g.M, g.N}, A.options());
+    Tensor s = fresh({g.M / QB, g.N / QB}, sa.options().memory_format(c10::MemoryFormat::Contiguous));
+    Tensor qg = fresh_like(q), sg = fresh_like(s);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_igemm_block_q_gelu((const int8_t *)A.data_ptr(), (const int8_t *)B.data_ptr(), sa.data_ptr(), sb.data_ptr(), g.bias,
                                    g.biasmax, (int8_t *)q.data_ptr(), s.data_ptr(), (int8_t *)qg.data_ptr(), sg.data_ptr(), g.M, g.N, g.K,
@@ -628,8 +628,8 @@ std::tuple<Tensor, Tensor> igemm_block_q_gelu_bwd(const Tensor &A, const Tensor 
     c10::DeviceGuard guard(A.device());
     const auto so = rng(JF_ROUND_STOCHASTIC, A, (int64_t)g.M * g.N, seed, offset);
     const auto go = rng(gelu_rounding, A, (int64_t)g.M * g.N, gelu_seed, gelu_offset);
-    Tensor out = torch::empty({g.M, g.N}, A.options());
-    Tensor sc = torch::empty({g.M / QB, g.N / QB}, sa.options().memory_format(c10::MemoryFormat::Contiguous));
+    Tensor out = fresh({g.M, g.N}, A.options());
+    Tensor sc = fresh({g.M / QB, g.N / QB}, sa.options().memory_format(c10::MemoryFormat::Contiguous));
     pybind11::gil_scoped_release nogil;
     check_rc(jf_igemm_block_q_gelu_bwd((const int8_t *)A.data_ptr(), (const int8_t *)B.data_ptr(), sa.data_ptr(), sb.data_ptr(),
                                        (const int8_t *)xq.data_ptr(), xs.data_ptr(), (int8_t *)out.data_ptr(), sc.data_ptr(), g.M, g.N, g.K,
@@ -650,7 +650,7 @@ Tensor igemm_block_q_dequant(const Tensor &A, const Tensor &B, const Tensor &sa,
     check_rounding(rounding, false);
     c10::DeviceGuard guard(A.device());
     const auto so = rng(rounding, A, (int64_t)g.M * g.N, seed, offset);
-    Tensor out = torch::empty({g.M, g.N}, A.options().dtype(odt));
+    Tensor out = fresh({g.M, g.N}, A.options().dtype(odt));
     pybind11::gil_scoped_release nogil;
     check_rc(jf_igemm_block_q_dequant((const int8_t *)A.data_ptr(), (const int8_t *)B.data_ptr(), sa.data_ptr(), sb.data_ptr(), g.bias,
                                       g.biasmax, out.data_ptr(), g.M, g.N, g.K, (int)layout, g.code, g.la, g.lb, oc, (int)rounding,
@@ -667,8 +667,8 @@ std::tuple<Tensor, Tensor> igemm_block_q(const Tensor &A, const Tensor &B, const
     check_rounding(rounding, false);
     c10::DeviceGuard guard(A.device());
     const auto so = rng(rounding, A, (int64_t)g.M * g.N, seed, offset);
-    Tensor out = torch::empty({g.M, g.N}, A.options());
-    Tensor sc = torch::empty({g.M / QB, g.N / QB}, sa.options().memory_format(c10::MemoryFormat::Contiguous));
+    Tensor out = fresh({g.M, g.N}, A.options());
+    Tensor sc = fresh({g.M / QB, g.N / QB}, sa.options().memory_format(c10::MemoryFormat::Contiguous));
     pybind11::gil_scoped_release nogil;
     check_rc(jf_igemm_block_q((const int8_t *)A.data_ptr(), (const int8_t *)B.data_ptr(), sa.data_ptr(), sb.data_ptr(), g.bias, g.biasmax,
                               (int8_t *)out.data_ptr(), sc.data_ptr(), g.M, g.N, g.K, (int)layout, g.code, g.la, g.lb, (int)rounding,
@@ -725,7 +725,7 @@ std::tuple<Tensor, OptTensor> linear_forward(const Tensor &X, const Tensor &SX, 
     linear_bias(bias, biasmax, x, w.R, b, bm);
     c10::DeviceGuard guard(x.q.device());
     if (!quantized) {
-        Tensor out = torch::empty(with_last(x.q, w.R), x.s.options());
+        Tensor out = fresh(with_last(x.q, w.R), x.s.options());
         pybind11::gil_scoped_release nogil;
         check_rc(jf_igemm_block_q_dequant(x.qp(), w.qp(), x.sp(), w.sp(), b, bm, out.data_ptr(), (int)x.R, (int)w.R, (int)x.C, JF_B_NK, x.code,
                                           JF_SCALES_ROWMAJOR, JF_SCALES_ROWMAJOR, x.code == JF_SCALE_F16 ? JF_FP_F16 : JF_FP_F32,
@@ -733,7 +733,7 @@ std::tuple<Tensor, OptTensor> linear_forward(const Tensor &X, const Tensor &SX, 
                  "linear_forward");
         return std::make_tuple(out, OptTensor());
     }
-    Tensor o = torch::empty(with_last(x.q, w.R), x.q.options()), so = torch::empty(with_last(x.s, w.R / QB), x.s.options());
+    Tensor o = fresh(with_last(x.q, w.R), x.q.options()), so = fresh(with_last(x.s, w.R / QB), x.s.options());
     pybind11::gil_scoped_release nogil;
     check_rc(jf_igemm_block_q(x.qp(), w.qp(), x.sp(), w.sp(), b, bm, (int8_t *)o.data_ptr(), so.data_ptr(), (int)x.R, (int)w.R, (int)x.C,
                               JF_B_NK, x.code, JF_SCALES_ROWMAJOR, JF_SCALES_ROWMAJOR, JF_ROUND_NEAREST, 0, 0, nullptr, 0, current_stream(x.q)),
@@ -751,8 +751,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> linear_forward_gelu(const Tensor &X, 
     const float *b, *bm;
     linear_bias(bias, biasmax, x, w.R, b, bm);
     c10::DeviceGuard guard(x.q.device());
-    Tensor o = torch::empty(with_last(x.q, w.R), x.q.options()), so = torch::empty(with_last(x.s, w.R / QB), x.s.options());
-    Tensor g = torch::empty_like(o), sg = torch::empty_like(so);
+    Tensor o = fresh(with_last(x.q, w.R), x.q.options()), so = fresh(with_last(x.s, w.R / QB), x.s.options());
+    Tensor g = fresh_like(o), sg = fresh_like(so);
     pybind11::gil_scoped_release nogil;
     check_rc(jf_igemm_block_q_gelu(x.qp(), w.qp(), x.sp(), w.sp(), b, bm, (int8_t *)o.data_ptr(), so.data_ptr(), (int8_t *)g.data_ptr(),
                                    sg.data_ptr(), (int)x.R, (int)w.R, (int)x.C, x.code, JF_SCALES_ROWMAJOR, JF_SCALES_ROWMAJOR, (int)approx,
@@ -775,7 +775,7 @@ Tensor weight_gradient(const Operand &x, const Operand &g, const OptTensor &gT, 
         la = check_a_any_layout(*gT, M, K);
         a = (const int8_t *)gT->data_ptr();
     }
-    Tensor out = torch::empty({M, N}, x.q.options().dtype(odt));
+    Tensor out = fresh({M, N}, x.q.options().dtype(odt));
     const size_t nbytes = jf_igemm_block_fp_workspace_bytes(M, N, K, JF_B_KN, (int)splitk);
     Tensor ws;
     if (nbytes) ws = scratch(x.q, nbytes);
@@ -797,15 +797,15 @@ std::vector<Tensor> linear_backward(const Tensor &X, const Tensor &SX, const Ten
     std::vector<Tensor> out;
     const auto so = rng(JF_ROUND_STOCHASTIC, g.q, g.R * w.C, c10::nullopt, c10::nullopt);
     if (dgrad_quantize) {
-        out.push_back(torch::empty(with_last(g.q, w.C), g.q.options()));
-        out.push_back(torch::empty(with_last(g.s, w.C / QB), g.s.options()));
+        out.push_back(fresh(with_last(g.q, w.C), g.q.options()));
+        out.push_back(fresh(with_last(g.s, w.C / QB), g.s.options()));
         pybind11::gil_scoped_release nogil;
         check_rc(jf_igemm_block_q(g.qp(), w.qp(), g.sp(), w.sp(), nullptr, nullptr, (int8_t *)out[0].data_ptr(), out[1].data_ptr(), (int)g.R,
                                   (int)w.C, (int)g.C, JF_B_KN, g.code, JF_SCALES_ROWMAJOR, JF_SCALES_KMAJOR, JF_ROUND_STOCHASTIC, so.first,
                                   so.second, nullptr, 0, current_stream(g.q)),
                  "linear_backward");
     } else {
-        out.push_back(torch::empty(with_last(g.q, w.C), g.s.options()));
+        out.push_back(fresh(with_last(g.q, w.C), g.s.options()));
         pybind11::gil_scoped_release nogil;
         check_rc(jf_igemm_block_q_dequant(g.qp(), w.qp(), g.sp(), w.sp(), nullptr, nullptr, out[0].data_ptr(), (int)g.R, (int)w.C, (int)g.C,
                                           JF_B_KN, g.code, JF_SCALES_ROWMAJOR, JF_SCALES_KMAJOR, g.code == JF_SCALE_F16 ? JF_FP_F16 : JF_FP_F32,
@@ -831,7 +831,7 @@ std::vector<Tensor> linear_backward_gelu(const Tensor &X, const Tensor &SX, cons
     c10::DeviceGuard guard(x.q.device());
     const auto so = rng(JF_ROUND_STOCHASTIC, g.q, g.R * w.C, c10::nullopt, c10::nullopt);
     const auto go = rng(gelu_rounding, g.q, g.R * w.C, c10::nullopt, c10::nullopt);
-    std::vector<Tensor> out{torch::empty(with_last(g.q, w.C), g.q.options()), torch::empty(with_last(g.s, w.C / QB), g.s.options())};
+    std::vector<Tensor> out{fresh(with_last(g.q, w.C), g.q.options()), fresh(with_last(g.s, w.C / QB), g.s.options())};
     {
         pybind11::gil_scoped_release nogil;
         check_rc(jf_igemm_block_q_gelu_bwd(g.qp(), w.qp(), g.sp(), w.sp(), p.qp(), p.sp(), (int8_t *)out[0].data_ptr(), out[1].data_ptr(), (int)g.R,
