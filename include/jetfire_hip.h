@@ -275,12 +275,21 @@ int jf_gelu_bwd(const int8_t *qx, const void *sx, const int8_t *qg, const void *
  * may be NULL).  y1 receives y in y1_dtype (JF_FP_F32: as the reference's kernels write it; JF_FP_F16 / JF_FP_BF16: y
  * rounded to nearest even, i.e. the kernel followed by the cast the reference's recipe applies to it,
  * INT8_GPT2/qmodel.py:228, without the fp32 tensor in between).  The quantisation and the partial sums always use the
- * fp32 y.
+ * fp32 y.  (q, s) may be (q2, s2).
  * Replaces int8_add_Ifp_Ig16_Ofp_Og (Jetfire/Nonlinear/add.py:164-211) and
  * int8_add_Ifp_Ig16_Ofp_Og_MeanVar (Jetfire/Nonlinear/add_mean_var.py:179-230). */
 int jf_add(const void *x1, int x1_dtype, const int8_t *q2, const void *s2, int R, int C,
            int scale_dtype, int rounding, uint64_t seed, uint64_t offset,
            void *y1, int y1_dtype, int8_t *q, void *s, float *rowsum, float *rowsq, jf_stream_t stream);
+
+/* The forward GEMM of jf_igemm_block_q (A [M,K], B [N,K], round to nearest) and jf_add of its result to x1, as one kernel where the
+ * launch is small: y, (q, s), rowsum and rowsq are what jf_add(x1, <the requantised output>, add_rounding) returns, bit for bit.  The
+ * requantised output itself is left nowhere.  q, s and y overlap no input.  add_rounding: JF_ROUND_NEAREST or JF_ROUND_TRUNC.
+ * Replaces the pair igemm_output_int_quantize_bias_rowcol (include/igemm.h:66-77) + int8_add_Ifp_Ig16_Ofp_Og_MeanVar
+ * (Jetfire/Nonlinear/add_mean_var.py:179-230) at the end of either half of a block (INT8_GPT2/qmodel.py:228). */
+int jf_igemm_block_q_add(const int8_t *A, const int8_t *B, const void *sa, const void *sb, const float *bias, const float *biasmax,
+                         const void *x1, int x1_dtype, int add_rounding, void *y, int y_dtype, int8_t *q, void *s, float *rowsum,
+                         float *rowsq, int M, int N, int K, int scale_dtype, int sa_layout, int sb_layout, jf_stream_t stream);
 
 /* out[c] = sum over all rows of q[r,c] * s[r/32,c/32] (fp32): the column sums of a block tensor, i.e. the bias gradient
  * of a linear layer from its quantised output gradient (sketched in the reference as G8.sum(0),

@@ -56,27 +56,24 @@ struct Saved {
 
 // needed by the forward only
 struct ForwardTemp {
-    int8_t *qo;
-    void *so;
     float *mid, *rowsum, *rowsq;
     size_t carve(uint8_t *b, const Dims &d)
     {
         Carver k(b);
-        qo = k.take<int8_t>(d.codes(d.c)); so = k.take(d.scales(d.c));
         mid = k.take<float>(d.m * d.c * 4);
         rowsum = k.take<float>(d.c / 32 * d.m * 4); rowsq = k.take<float>(d.c / 32 * d.m * 4);
         return k.used;
     }
 };
 
-// Both of them where no backward follows: what is dead makes room for what comes after it.  Two block tensors of [M, C] serve in
-// turn as qn, qy, q2 and as qo, qn2, qo; Q, K, V and the attention's result make room for the float sum and the hidden layer.  14
+// Both of them where no backward follows: what is dead makes room for what comes after it.  Of two block tensors of [M, C] one
+// serves in turn as qn, qy and qn2, the other as q2; Q, K, V and the attention's result make room for the float sum and the hidden layer.  14
 // bytes per element of [M, C] and the scales, where a call whose backward follows holds 25.
 size_t carve_inference(uint8_t *b, const Dims &d, Saved &v, ForwardTemp &t)
 {
     Carver k(b);
-    v.qn = v.qy = v.q2 = k.take<int8_t>(d.codes(d.c)); v.sn = v.sy = v.s2 = k.take(d.scales(d.c));
-    t.qo = v.qn2 = k.take<int8_t>(d.codes(d.c)); t.so = v.sn2 = k.take(d.scales(d.c));
+    v.qn = v.qy = v.qn2 = k.take<int8_t>(d.codes(d.c)); v.sn = v.sy = v.sn2 = k.take(d.scales(d.c));
+    v.q2 = k.take<int8_t>(d.codes(d.c)); v.s2 = k.take(d.scales(d.c));
     v.lse = k.take<float>(d.m * d.H * 4); v.mean2 = k.take<float>(d.m * 4); v.rstd2 = k.take<float>(d.m * 4);
     t.rowsum = k.take<float>(d.c / 32 * d.m * 4); t.rowsq = k.take<float>(d.c / 32 * d.m * 4);
     Carver attention(b ? b + k.used : nullptr), mlp(attention.base);
@@ -193,12 +190,9 @@ BlockForward forward_impl(const Dims &d, const Tensor &x, const Tensor &qx, cons
     const int m = d.M, c = d.C;
     auto codes = [](const Tensor &a) { return (const int8_t *)a.data_ptr(); };
     const int8_t *qx_ = codes(qx);
-    auto gemm_q = [&](const int8_t *a, const void *sa, int i, int n, int k, int8_t *out, void *so) {
-        check_rc(jf_igemm_block_q(a, codes(w[i].q), sa, w[i].s.data_ptr(), bp[i], bm[i], out, so, m, n, k, JF_B_NK, F16, RM, RM, JF_ROUND_NEAREST,
-                                  0, 0, nullptr, 0, st), "projection");
-    };
-    auto add = [&](const void *x1, int x1c, void *y, int yc, int8_t *q, void *s) {
-        check_rc(jf_add(x1, x1c, t.qo, t.so, m, c, F16, JF_ROUND_TRUNC, 0, 0, y, yc, q, s, t.rowsum, t.rowsq, st), "residual add");
+    auto project_add = [&](const int8_t *a, const void *sa, int i, int k, const void *x1, int x1c, void *y, int yc, int8_t *q, void *s) {
+        check_rc(jf_igemm_block_q_add(a, codes(w[i].q), sa, w[i].s.data_ptr(), bp[i], bm[i], x1, x1c, JF_ROUND_TRUNC, y, yc, q, s, t.rowsum,
+                                      t.rowsq, m, c, k, F16, RM, RM, st), "projection and residual add");
     };
     check_rc(jf_layernorm_fwd(qx_, sx.data_ptr(), g1, nullptr, mu, rs, m, c, F16, v.qn, v.sn, st), "layernorm");
     check_rc(jf_igemm_block_q_dequant(v.qn, codes(w[0].q), v.sn, w[0].s.data_ptr(), bp[0], bm[0], v.qkv, m, 3 * c, c, JF_B_NK, F16, RM, RM, JF_FP_F16,
@@ -207,13 +201,11 @@ BlockForward forward_impl(const Dims &d, const Tensor &x, const Tensor &qx, cons
     check_rc(jf_attention_fwd_q(qkv, qkv + c, qkv + 2 * c, 3 * c, d.B, d.H, d.T, c / d.H, (float)(1.0 / std::sqrt((double)(c / d.H))), v.y, v.lse,
                                 v.qy, v.sy, st),
              "attention");
-    gemm_q(v.qy, v.sy, 1, c, c, t.qo, t.so);
-    add(x.data_ptr(), xc, t.mid, JF_FP_F32, v.q2, v.s2);
+    project_add(v.qy, v.sy, 1, c, x.data_ptr(), xc, t.mid, JF_FP_F32, v.q2, v.s2);
     check_rc(jf_layernorm_fwd_sums(v.q2, v.s2, g2, nullptr, t.rowsum, t.rowsq, m, c, F16, v.mean2, v.rstd2, v.qn2, v.sn2, st), "layernorm");
     check_rc(jf_igemm_block_q_gelu(v.qn2, codes(w[2].q), v.sn2, w[2].s.data_ptr(), bp[2], bm[2], v.qh, v.sh, v.qa, v.sa, m, 4 * c, c, F16, RM, RM,
                                    JF_GELU_ERF, 5e-5f, st), "fc");
-    gemm_q(v.qa, v.sa, 3, c, 4 * c, t.qo, t.so);
-    add(t.mid, JF_FP_F32, r.fp.data_ptr(), fp_of(r.fp, "out"), (int8_t *)r.q.data_ptr(), r.s.data_ptr());
+    project_add(v.qa, v.sa, 3, 4 * c, t.mid, JF_FP_F32, r.fp.data_ptr(), fp_of(r.fp, "out"), (int8_t *)r.q.data_ptr(), r.s.data_ptr());
     check_rc(jf_rowstats_finish(t.rowsum, t.rowsq, m, c / QB, c, r.mean.data_ptr<float>(), r.rstd.data_ptr<float>(), st), "row statistics");
     return r;
 }

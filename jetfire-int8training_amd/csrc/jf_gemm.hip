@@ -43,7 +43,9 @@ constexpr int EPI_LD = 36;                          // floats per staged row (32
 //         the saved forward input of the GELU: only the result of the GELU backward leaves
 // EPI_QD: EPI_Q followed by the dequantisation of the block just requantised (codes x stored scale), written as float /
 //         binary16 / bfloat16: the requantised tensor itself is never written.
-enum Epilogue { EPI_S32 = 0, EPI_FP = 1, EPI_Q = 2, EPI_QG = 3, EPI_QB = 4, EPI_QD = 5 };
+// EPI_QA: EPI_Q (deterministic) followed by the residual addition of the block just requantised: the sum, its requantisation and its
+//         partial row sums leave (32x128 tiles only, see jf_igemm_block_q_add)
+enum Epilogue { EPI_S32 = 0, EPI_FP = 1, EPI_Q = 2, EPI_QG = 3, EPI_QB = 4, EPI_QD = 5, EPI_QA = 6 };
 // Wave-priority schemes of the main loop (launch_gemm_cfg picks one per launch)
 enum Pace { PACE_HARDWARE = 0, PACE_EVEN = 1, PACE_ORDERED = 2 };
 
@@ -78,6 +80,10 @@ struct GemmArgs {
     int phase_capacity;
     int fold_kb;          // K blocks after which the accumulators are added up in `fold` (a multiple of NSTAGE stages; 0: never)   (FOLD)
     float *fold;          // BM x BN values per workgroup, in an order of their own   (FOLD)
+    const void *x1;       // [M, N], x1_dtype: what the requantised result is added to   (EPI_QA; rounding2: JF_ROUND_NEAREST / _TRUNC)
+    int x1_dtype;
+    void *y;              // [M, N], out_dtype: the sum   (EPI_QA)
+    float *rowsum, *rowsq;   // [N/32, M] or null: per row and 32 columns, of the sum and its square   (EPI_QA)
 };
 
 // Position of workgroup wg in `work` pieces of work, or -1 behind the last.  Workgroups are dealt round-robin to the 8 XCDs, each with a
@@ -166,7 +172,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     static_assert(!AKM || BM == ROW_BYTES, "a staged [K,M] row is one 128-byte LDS row");
     // The epilogues that requantise want a lane to hold 16 consecutive columns of a row.  They form the transposed product (B block
     // times A block, the same integers): its registers run along the columns, see the epilogue.
-    constexpr bool QUANT = EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD;
+    constexpr bool QUANT = EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD || EPI == EPI_QA;
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     typedef __attribute__((address_space(3))) unsigned char lds_u8;
@@ -398,6 +404,21 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
 #pragma unroll
     for (int j = 0; j < WBN; ++j) { nb[j] = n0 / QB + wn * WBN + j; nb[j] = nb[j] < SN ? nb[j] : SN - 1; }
 
+    // EPI_QA: the lane's 16 elements of x1 are on their way during the main loop (the waves that multiply wait for no load in it)
+    v4i x1_raw[4];
+    auto fetch_x1 = [&] {
+        const size_t at = (size_t)(m0 + wm * QB + (lane & 31)) * p.N + n0 + wn * QB + (lane >> 5) * 16;
+        if (p.x1_dtype == JF_FP_F32) {
+            const v4i *src = reinterpret_cast<const v4i *>(reinterpret_cast<const float *>(p.x1) + at);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x1_raw[k] = src[k];
+        } else {
+            const v4i *src = reinterpret_cast<const v4i *>(reinterpret_cast<const uint16_t *>(p.x1) + at);
+            x1_raw[0] = src[0]; x1_raw[1] = src[1];
+            x1_raw[2] = x1_raw[3] = v4i{0, 0, 0, 0};
+        }
+    };
+
     // ---- main loop ----------------------------------------------------------------------------
     // The whole ring is filled up front; afterwards the loads of stage s+NSTAGE are issued when the last K block
     // of stage s has been read.  Operand fragments and scales of K block k+1 are read from LDS into a second set
@@ -599,6 +620,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     if constexpr (TABLE) {
         if (loader) wait_stage(NSTAGE - 1, std::integral_constant<int, NSTAGE - 1>{});    // stage 0 has landed
         else make_table();
+        if constexpr (EPI == EPI_QA) { if (!loader && m0 + wm * QB < p.M && n0 + wn * QB < p.N) fetch_x1(); }
     } else {
         if (NSTAGE - 1 >= nstages) JF_WAIT_VMCNT(0);
         else JF_WAIT_VMCNT((NSTAGE - 1) * LOADS - (EPI != EPI_S32 ? 1 : 0));      // stage 0 and the scales of stage 1 have landed
@@ -916,7 +938,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     }
     if (PROF) { phase(2, (unsigned long long)wall_clock64()); phase(7, (unsigned long long)(clock64() - prof_c0)); }
     if (p.pace != PACE_HARDWARE) __builtin_amdgcn_s_setprio(0);
-    if constexpr (!QUANT) __syncthreads();                     // the epilogue reuses the ring as scratch
+    if constexpr (!QUANT || EPI == EPI_QA) __syncthreads();    // the epilogue reuses the ring as scratch
     if (loader) return;
     if (PROF) phase(3, (unsigned long long)wall_clock64());
 
@@ -939,7 +961,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    float *patch = reinterpret_cast<float *>(smem) + wave * (QB * EPI_LD);     // (not QUANT)
+    float *patch = reinterpret_cast<float *>(smem) + wave * (QB * EPI_LD);     // (not QUANT, or EPI_QA)
     const int rrow = QUANT ? lane & 31 : lane >> 1, rcol = (QUANT ? lane >> 5 : lane & 1) * 16;
     // GELU tables of the wave: its scale patch (nothing is on its way there any more) and, for the byte table, a piece of its own
     float *const gelu_tab = TABLE ? reinterpret_cast<float *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 320 : reinterpret_cast<float *>(scale_patch);
@@ -973,9 +995,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     }
 
     // 16 consecutive results of a row as float / binary16 / bfloat16 (rounded to nearest even): 64 or 32 contiguous bytes
-    auto store_fp = [&](const float (&x)[16], const size_t e0) {
+    auto store_fp = [&](void *out, const float (&x)[16], const size_t e0) {
         if (p.out_dtype == JF_FP_F32) {
-            v4f *dst = reinterpret_cast<v4f *>(reinterpret_cast<float *>(p.C) + e0);
+            v4f *dst = reinterpret_cast<v4f *>(reinterpret_cast<float *>(out) + e0);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 v4f t = {x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]};
@@ -994,9 +1016,21 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                 for (int k = 0; k < 16; ++k) h[k] = (__bf16)x[k];
                 lo = *reinterpret_cast<v4i *>(&h[0]); hi = *reinterpret_cast<v4i *>(&h[8]);
             }
-            v4i *dst = reinterpret_cast<v4i *>(reinterpret_cast<unsigned char *>(p.C) + e0 * 2);   // 32 of a row's 64 bytes
+            v4i *dst = reinterpret_cast<v4i *>(reinterpret_cast<unsigned char *>(out) + e0 * 2);   // 32 of a row's 64 bytes
             dst[0] = lo; dst[1] = hi;
         }
+    };
+    // A block's float results from the patch in the shape that stores best: every store instruction writes 8 whole 128-byte rows of the
+    // block instead of 64 separate 16-byte pieces (3-6 us off the weight gradients of GPT-2 XL; the same for 16-bit outputs, 16 rows x
+    // 64 bytes per instruction, measured slower than the two 16-byte pieces per lane of the row layout)
+    auto store_patch_rows = [&](void *out, const int bm, const int bn) {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            const int row = 8 * h + (lane >> 3), c4 = (lane & 7) * 4;
+            const v4f t = *reinterpret_cast<const v4f *>(patch + row * EPI_LD + c4);
+            *reinterpret_cast<v4f *>(reinterpret_cast<float *>(out) + (size_t)(bm + row) * p.N + bn + c4) = t;
+        }
+        wave_sync();
     };
 #pragma unroll
     for (int i = 0; i < WBM; ++i)
@@ -1017,17 +1051,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                 wave_sync();
             }
             if (EPI == EPI_FP && p.out_dtype == JF_FP_F32) {
-                // No arithmetic follows, so the patch is read back in the shape that stores best: every store instruction
-                // writes 8 whole 128-byte rows of the block instead of 64 separate 16-byte pieces (3-6 us off the weight
-                // gradients of GPT-2 XL; the same for 16-bit outputs, 16 rows x 64 bytes per instruction, measured slower
-                // than the two 16-byte pieces per lane of the row layout below)
-#pragma unroll
-                for (int h = 0; h < 4; ++h) {
-                    const int row = 8 * h + (lane >> 3), c4 = (lane & 7) * 4;
-                    const v4f t = *reinterpret_cast<const v4f *>(patch + row * EPI_LD + c4);
-                    *reinterpret_cast<v4f *>(reinterpret_cast<float *>(p.C) + (size_t)(bm + row) * p.N + bn + c4) = t;
-                }
-                wave_sync();
+                store_patch_rows(p.C, bm, bn);                // (no arithmetic follows)
                 continue;
             }
             float x[16];
@@ -1051,7 +1075,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                     dst[k] = t;
                 }
             } else if (EPI == EPI_FP) {
-                store_fp(x, e0);
+                store_fp(p.C, x, e0);
             } else {
                 v4i codes = {0, 0, 0, 0};
                 float scale = 0.0f;
@@ -1102,11 +1126,50 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                                                       p.rounding2, p.seed2, p.offset2, (uint64_t)e0, &scale2);
                     scale = scale2;
                 }
+                if constexpr (EPI == EPI_QA) {
+                    // the sum with the block as a reader of the stored tensor would dequantise it; its partial row sums, columns 0..15
+                    // and 16..31 (add_kernel's order); its own requantisation
+                    float y[16];
+                    unpack16(codes, (float)(ST)scale, y);
+                    // (one branch per type: the compiler makes a choice per element sixteen branches)
+                    if (p.x1_dtype == JF_FP_F32) {
+#pragma unroll
+                        for (int k = 0; k < 16; ++k) y[k] = __int_as_float(x1_raw[k / 4][k % 4]) + y[k];
+                    } else if (p.x1_dtype == JF_FP_F16) {
+#pragma unroll
+                        for (int k = 0; k < 16; ++k) y[k] = (float)__builtin_bit_cast(half_t, (uint16_t)(x1_raw[k / 8][(k / 2) % 4] >> (16 * (k & 1)))) + y[k];
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 16; ++k) {
+                            const unsigned w = (unsigned)x1_raw[k / 8][(k / 2) % 4];
+                            y[k] = __uint_as_float(k & 1 ? w & 0xffff0000u : w << 16) + y[k];
+                        }
+                    }
+                    if (p.out_dtype == JF_FP_F32) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) *reinterpret_cast<v4f *>(patch + rrow * EPI_LD + rcol + 4 * k) = v4f{y[4 * k], y[4 * k + 1], y[4 * k + 2], y[4 * k + 3]};
+                        wave_sync();
+                        store_patch_rows(p.y, bm, bn);
+                    } else {
+                        store_fp(p.y, y, e0);
+                    }
+                    if (p.rowsum) {
+                        float t1 = 0.0f, t2 = 0.0f;
+#pragma unroll
+                        for (int k = 0; k < 16; ++k) { t1 = t1 + y[k]; t2 = __builtin_fmaf(y[k], y[k], t2); }
+                        const float o1 = __shfl_xor(t1, 32, WAVE), o2 = __shfl_xor(t2, 32, WAVE);
+                        if (lane < 32) {
+                            p.rowsum[(size_t)(bn / QB) * p.M + bm + lane] = t1 + o1;
+                            p.rowsq[(size_t)(bn / QB) * p.M + bm + lane] = t2 + o2;
+                        }
+                    }
+                    codes = quantize16(y, 0.0f, p.rounding2, 0, 0, 0, &scale);
+                }
                 if (EPI == EPI_QD) {
                     // the block as a reader of the stored tensor would dequantise it: codes x the scale rounded to ST
                     float y[16];
                     unpack16(codes, (float)(ST)scale, y);
-                    store_fp(y, e0);
+                    store_fp(p.C, y, e0);
                 } else {
                     *reinterpret_cast<v4i *>(reinterpret_cast<int8_t *>(p.C) + e0) = codes;     // 16 of a row's 32 bytes
                     if (lane == 0) store_scale(reinterpret_cast<ST *>(p.sc), (bm / QB) * SN + bn / QB, scale);
@@ -1471,6 +1534,11 @@ static void wgrad_group_plan(int n, const int *M, const int *N, int K, WgradPlan
     }
 }
 
+static bool small_tiles_resident(int M, int N, int K)          // two workgroups per CU
+{
+    return K <= TABLE_KB * QB && (long)((M + 31) / 32) * ((N + 127) / 128) <= 2L * cu_count();
+}
+
 // Tile configuration.  Large launches: 128x128 tiles, 8 waves of two blocks, a 2-deep ring and two workgroups per CU (the
 // epilogue of one overlaps the main loop of the other).  A launch whose 32x128 tiles are all resident at once, two workgroups
 // of 4 waves and a 3-deep ring per CU, takes those instead: its 128x128 tiles would occupy at most a quarter of the chip with
@@ -1484,7 +1552,7 @@ static void wgrad_group_plan(int n, const int *M, const int *N, int K, WgradPlan
 template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs &a, hipStream_t st)
 {
     if constexpr (EPI != EPI_S32) {
-        if (a.splits <= 1 && a.K <= TABLE_KB * QB && (long)((a.M + 31) / 32) * ((a.N + 127) / 128) <= 2L * cu_count())
+        if (a.splits <= 1 && small_tiles_resident(a.M, a.N, a.K))
             return launch_gemm_cfg<EPI, ST, 1, 1, 4, 3, 2, BKN>(a, st);
     }
     if constexpr (EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD) {
@@ -1854,6 +1922,37 @@ int jf_igemm_block_q_dequant(const int8_t *A, const int8_t *B, const void *sa, c
         return JF_ERR_ENUM;
     hipStream_t st = (hipStream_t)stream;
     return scale_dtype == JF_SCALE_F16 ? launch_gemm<EPI_QD, half_t>(a, st, kn) : launch_gemm<EPI_QD, float>(a, st, kn);
+}
+
+// The residual addition reads and writes 13 to 17 bytes per element that the GEMM has in registers, in a launch of its own.  In the
+// epilogue where the launch is one of 32x128 tiles that are all resident at once: there the addition's launch is what costs.  us, two
+// launches | this | the GEMM alone, float in and out, binary16 scales: 32x768x768 8.7 | 6.9 | 5.6, 64x256x256 7.0 | 5.6 | 4.1, 512x256x1024
+// 9.6 | 7.7 | 6.4, 1248x768x768 10.0 | 7.8 | 5.9, 1248x768x3072 17.4 | 14.7 | 12.4, 2048x768x3072 21.5 | 18.8 | 15.6.  Larger launches keep the
+// two: the epilogue of a 128x128 tile has no room in LDS to turn the float sum into whole rows without a barrier of the workgroup, and
+// as separate 16-byte pieces it would hold up the other tiles' loads.
+int jf_igemm_block_q_add(const int8_t *A, const int8_t *B, const void *sa, const void *sb, const float *bias, const float *biasmax,
+                         const void *x1, int x1_dtype, int add_rounding, void *y, int y_dtype, int8_t *q, void *s, float *rowsum,
+                         float *rowsq, int M, int N, int K, int scale_dtype, int sa_layout, int sb_layout, jf_stream_t stream)
+{
+    int rc = check_gemm_common(A, B, q, M, N, K, JF_B_NK);
+    if (rc) return rc;
+    if (!sa || !sb || !s || !x1 || !y || (rowsum == nullptr) != (rowsq == nullptr)) return JF_ERR_NULL;
+    if ((scale_dtype != JF_SCALE_F16 && scale_dtype != JF_SCALE_F32) || (add_rounding != JF_ROUND_NEAREST && add_rounding != JF_ROUND_TRUNC) ||
+        x1_dtype < JF_FP_F16 || x1_dtype > JF_FP_BF16 || y_dtype < JF_FP_F16 || y_dtype > JF_FP_BF16) return JF_ERR_ENUM;
+    if (!aligned16(x1) || !aligned16(y) || !scale_ptr_ok(sa, scale_dtype) || !scale_ptr_ok(sb, scale_dtype)) return JF_ERR_ALIGN;
+    if (!small_tiles_resident(M, N, K)) {
+        rc = jf_igemm_block_q(A, B, sa, sb, bias, biasmax, q, s, M, N, K, JF_B_NK, scale_dtype, sa_layout, sb_layout, JF_ROUND_NEAREST, 0, 0,
+                              nullptr, 0, stream);
+        return rc ? rc : jf_add(x1, x1_dtype, q, s, M, N, scale_dtype, add_rounding, 0, 0, y, y_dtype, q, s, rowsum, rowsq, stream);
+    }
+    GemmArgs a = {};
+    a.A = A; a.B = B; a.sa = sa; a.sb = sb; a.C = q; a.sc = s; a.bias = bias; a.biasmax = biasmax;
+    a.x1 = x1; a.x1_dtype = x1_dtype; a.rounding2 = add_rounding; a.y = y; a.out_dtype = y_dtype; a.rowsum = rowsum; a.rowsq = rowsq;
+    a.M = M; a.N = N; a.K = K; a.lda = K; a.ldb = K; a.rounding = JF_ROUND_NEAREST;
+    if (!scale_strides(sa_layout, K, M / QB, a.sa_ks, a.sa_is) || !scale_strides(sb_layout, K, N / QB, a.sb_ks, a.sb_is))
+        return JF_ERR_ENUM;
+    hipStream_t st = (hipStream_t)stream;
+    return scale_dtype == JF_SCALE_F16 ? launch_gemm_cfg<EPI_QA, half_t, 1, 1, 4, 3, 2, 0>(a, st) : launch_gemm_cfg<EPI_QA, float, 1, 1, 4, 3, 2, 0>(a, st);
 }
 
 int jf_igemm_block_q_gelu(const int8_t *A, const int8_t *B, const void *sa, const void *sb, const float *bias,

@@ -31,7 +31,7 @@ EXPORTS = [
     "jf_layernorm_bwd_workspace_bytes", "jf_layernorm_bwd", "jf_layernorm_bwd_add", "jf_layernorm_bwd_add_strips", "jf_gelu_fwd", "jf_gelu_bwd", "jf_add", "jf_rowstats_finish",
     "jf_igemm_block_q_dequant", "jf_quantize_slabs", "jf_philox_rounds", "jf_block_colsum", "jf_block_colsum_workspace_bytes",
     "jf_attention_fwd", "jf_attention_bwd", "jf_quantize_many", "jf_rowstats_fp", "jf_wgrad_many", "jf_wgrad_many_workspace_bytes",
-    "jf_layernorm_fwd_sums", "jf_attention_fwd_q", "jf_attention_bwd_q",
+    "jf_layernorm_fwd_sums", "jf_attention_fwd_q", "jf_attention_bwd_q", "jf_igemm_block_q_add",
 ]
 
 _lib = None
@@ -78,6 +78,7 @@ def lib():
         L.jf_gelu_bwd.argtypes = [_p, _p, _p, _p, _i, _i, _i, _i, _i, _u64, _u64, _p, _p, _p]
         L.jf_layernorm_bwd_add.argtypes = [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _u64, _u64, _p, _i, _i, _u64, _u64,
                                            _p, _i, _p, _p, _p, _p, _p, _sz, _p]
+        L.jf_igemm_block_q_add.argtypes = [_p, _p, _p, _p, _p, _p, _p, _i, _i, _p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p]
         L.jf_add.argtypes = [_p, _i, _p, _p, _i, _i, _i, _i, _u64, _u64, _p, _i, _p, _p, _p, _p, _p]
         L.jf_block_colsum_workspace_bytes.argtypes = [_i, _i]
         L.jf_block_colsum_workspace_bytes.restype = _sz
@@ -339,6 +340,32 @@ def igemm_block_q_gelu(A, B, sa, sb, approx=GELU_ERF, amax_eps=5e-5, bias=None, 
     check(lib().jf_igemm_block_q_gelu(_ptr(A), _ptr(B), _ptr(sa), _ptr(sb), _ptr(bias), _ptr(biasmax), _ptr(q), _ptr(s),
                                       _ptr(qg), _ptr(sg), M, N, K, code, la, lb, approx, amax_eps, _stream()))
     return q, s, qg, sg
+
+
+def igemm_block_q_add(A, B, sa, sb, x1, rounding=ROUND_TRUNC, bias=None, biasmax=None, out_dtype=torch.float32):
+    """Forward GEMM (B as [N,K], round to nearest) with the residual addition to x1 fused into its epilogue.
+    Returns (y, q, s, rowsum, rowsq): what igemm_block_q and then add(with_stats=True) would return."""
+    M, N, K, _, _ = _gemm_operands(A, B, B_NK)
+    code, la, lb = _gemm_scales(sa, sb, M, N, K)
+    if bias is not None:
+        _need(bias, torch.float32, "bias", 1)
+        if bias.numel() != N:
+            raise RuntimeError("bias must have N elements")
+    if biasmax is not None:
+        _need(biasmax, torch.float32, "biasmax", None)
+    _need(x1, None, "x1")
+    if x1.dtype not in _FP_CODE or tuple(x1.shape) != (M, N):
+        raise RuntimeError("x1 must be a float tensor of the shape of the result")
+    if out_dtype not in _FP_CODE:
+        raise RuntimeError("out_dtype must be float32, float16 or bfloat16")
+    y = torch.empty((M, N), dtype=out_dtype, device=A.device)
+    q = torch.empty((M, N), dtype=torch.int8, device=A.device)
+    s = torch.empty((M // QB, N // QB), dtype=sa.dtype, device=A.device)
+    rs = torch.empty((N // QB, M), dtype=torch.float32, device=A.device)
+    rq = torch.empty_like(rs)
+    check(lib().jf_igemm_block_q_add(_ptr(A), _ptr(B), _ptr(sa), _ptr(sb), _ptr(bias), _ptr(biasmax), _ptr(x1), _FP_CODE[x1.dtype], rounding,
+                                     _ptr(y), _FP_CODE[out_dtype], _ptr(q), _ptr(s), _ptr(rs), _ptr(rq), M, N, K, code, la, lb, _stream()))
+    return y, q, s, rs, rq
 
 
 def igemm_block_q_gelu_bwd(A, B, sa, sb, xq, xs, approx=GELU_ERF, gelu_rounding=ROUND_STOCHASTIC, seed=None, offset=None,

@@ -431,6 +431,36 @@ def test_forward_gemm_with_fused_gelu(jf, oracle, M, N, K, f16, approx):
     assert qg.cpu().numpy().any()
 
 
+@pytest.mark.parametrize("M,N,K,x1,y,f16,bias", [
+    (32, 32, 32, torch.float32, torch.float32, True, False),             # one block
+    (64, 160, 96, torch.float16, torch.bfloat16, False, True),           # a tile of one block's width
+    (1248, 768, 160, torch.bfloat16, torch.float32, True, True),
+    (256, 288, 1056, torch.float32, torch.float16, True, False),
+    (2048, 1024, 32, torch.float32, torch.float32, True, False),         # the last launch of one kernel ...
+    (2080, 1024, 32, torch.float32, torch.float32, True, True),          # ... and the first of two, in place
+    (32, 32, 16416, torch.bfloat16, torch.bfloat16, False, False),       # ... by the length of K
+])
+def test_quantised_with_residual_addition(jf, oracle, M, N, K, x1, y, f16, bias):
+    """The fused entry point returns, bit for bit, what the GEMM and then the addition return (both of which are checked against the
+    oracle elsewhere)."""
+    print(f"case q+add M={M} N={N} K={K} {x1} {y} f16={f16} bias={bias}", flush=True)
+    A, Bkn, sa, sb = make_problem(M + N * 3 + K, M, N, K, f16)
+    st = np.float16 if f16 else np.float32
+    sa = sa * np.float32(0.05)
+    dA, dB, dsa, dsb = dev(A), dev(b_of(Bkn, 0)), dev(sa.astype(st)), dev(sb.astype(st))
+    gen = torch.Generator("cuda").manual_seed(M + K)
+    res = torch.randn((M, N), device="cuda", generator=gen).to(x1)
+    res[:32, :32] = 0
+    b = torch.randn(N, device="cuda", generator=gen) if bias else None
+    bmax = b.abs().max().reshape(1) if bias else None
+    for rounding in (jf.ROUND_TRUNC, jf.ROUND_NEAREST):
+        got = jf.igemm_block_q_add(dA, dB, dsa, dsb, res, rounding, b, bmax, out_dtype=y)
+        q0, s0 = jf.igemm_block_q(dA, dB, dsa, dsb, jf.B_NK, bias=b, biasmax=bmax)
+        for g, w, name in zip(got, jf.add(res, q0, s0, rounding, with_stats=True, out_dtype=y), ("sum", "codes", "scales", "row sums", "row squares")):
+            assert torch.equal(g, w), name
+    assert got[1].any()
+
+
 @pytest.mark.parametrize("approx", [0, 1])
 @pytest.mark.parametrize("f16", [True, False])
 @pytest.mark.parametrize("M,N,K", [(128, 256, 96), (96, 160, 224), (256, 384, 544), (32, 32, 32)])
