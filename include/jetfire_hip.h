@@ -164,6 +164,15 @@ int jf_igemm_block_q_gelu_bwd(const int8_t *A, const int8_t *B, const void *sa, 
                               int sb_layout, int gelu_approx, uint64_t seed, uint64_t offset, int gelu_rounding,
                               uint64_t gelu_seed, uint64_t gelu_offset, jf_stream_t stream);
 
+/* Both gradients of a linear layer, dX = dY W and dW = dY^T X, in one launch where both are small: X codes [R, C_in], G = dY codes
+ * [R, C_out], W codes [C_out, C_in], scales in the tensors' own layout.  (dx, dx_scales) is what jf_igemm_block_q returns with stochastic
+ * rounding or, where dx_scales is NULL, dx (dx_dtype) what jf_igemm_block_q_dequant returns; dw is what jf_igemm_block_fp returns for G
+ * read as [K, M] with the same splitk, and so is the workspace it takes; all bit for bit.
+ * Replaces igemm_output_int_quantize_stochastic + igemm_output_fp_no_quantize of int8_linear_backward (Jetfire/Linear/linear_bwd.py:4-29). */
+int jf_linear_bwd(const int8_t *X, const void *sx, const int8_t *G, const void *sg, const int8_t *W, const void *sw, int R, int C_in, int C_out,
+                  int scale_dtype, void *dx, void *dx_scales, int dx_dtype, uint64_t seed, uint64_t offset, void *dw, int dw_dtype, int splitk,
+                  void *workspace, size_t workspace_bytes, jf_stream_t stream);
+
 /* jf_igemm_block_q with the dequantisation of its result fused into the epilogue: out[M,N] (out_dtype: JF_FP_*) =
  * codes x scales of the block tensor jf_igemm_block_q would have stored (scales rounded to scale_dtype as it stores
  * them), i.e. what jf_dequantize of that result returns, bit for bit; the INT8 tensor itself is never written.

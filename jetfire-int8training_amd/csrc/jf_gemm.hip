@@ -1218,6 +1218,24 @@ template <int EPI, typename ST, int BKN> __global__ __launch_bounds__(512, 4) vo
     }
 }
 
+// Both gradients of a linear layer (launch_linear_bwd): 32x128 or 128x128 tiles of the activation gradient (EPI_Q or EPI_QD, B as
+// [K,N]), then 128x128 tiles of the weight gradient.
+struct GemmBackward {
+    GemmArgs x, w;
+};
+template <int EPI, typename ST, bool SMALL> __global__ __launch_bounds__(512, 4) void igemm_backward_kernel(GemmBackward b)
+{
+    const int work_x = b.x.tiles_m * b.x.tiles_n, first_w = (work_x + 7) & ~7;      // (both parts are dealt to the XCDs from the first one on)
+    const int wg = blockIdx.x;
+    if (wg < first_w) {
+        const int logical = logical_workgroup(work_x, wg);
+        if (logical >= 0) igemm_body<EPI, ST, SMALL ? 1 : 2, SMALL ? 1 : 2, 4, SMALL ? 3 : 2, 2, 1, 0, 0>(b.x, logical);
+    } else {
+        const int logical = logical_workgroup(b.w.tiles_m * b.w.tiles_n * b.w.splits, wg - first_w);
+        if (logical >= 0) igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0>(b.w, logical);
+    }
+}
+
 // Several weight gradients over the same tokens in one launch (jf_wgrad_many).  Every XCD gets one contiguous run of each problem's
 // work, one problem after the other, so that the XCDs finish together although the parts of the problems differ in length.  (One
 // run over all problems: GPT-2 XL's four, one of them in parts a third as long, took 60 us more than the 500 they take.)
@@ -1412,6 +1430,12 @@ __device__ __forceinline__ void reduce_splits(const float *part, size_t n, int s
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *part, size_t n, int splits, void *out, int out_dtype)
 {
     reduce_splits(part, n, splits, out, out_dtype, ((size_t)blockIdx.x * 256 + threadIdx.x) * 4);
+}
+
+static int launch_splitk_reduce(const float *part, size_t n, int splits, void *out, int out_dtype, hipStream_t st)
+{
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)(n / 1024)), dim3(256), 0, st, part, n, splits, out, out_dtype);
+    return (int)hipGetLastError();
 }
 
 // What follows the weight gradients of a block, one launch: the K splits of each (as splitk_reduce_kernel) and column sums over
@@ -1624,6 +1648,22 @@ static bool scale_ptr_ok(const void *p, int scale_dtype)
 }
 
 #ifndef JF_PROF_LIB
+// x, w: as for their own launches.
+template <int EPI, typename ST, bool SMALL> static int launch_linear_bwd(const GemmArgs &x, const GemmArgs &w, hipStream_t st)
+{
+    GemmBackward b = {x, w};
+    b.x.tiles_m = SMALL ? x.M / QB : (x.M + 127) / 128; b.x.tiles_n = (x.N + 127) / 128; b.x.splits = 1;
+    b.w.tiles_m = (w.M + 127) / 128; b.w.tiles_n = (w.N + 127) / 128;
+    const long work = (long)b.x.tiles_m * b.x.tiles_n + (long)b.w.tiles_m * b.w.tiles_n * b.w.splits;
+    b.x.pace = b.w.pace = SMALL ? (int)PACE_HARDWARE : pace_of(work, 2L * cu_count(), std::max(x.K, w.splits > 1 ? w.kb_per_split * QB : w.K));
+    constexpr int SX = SMALL ? gemm_lds(EPI, 1, 1, 4, 3) : gemm_lds(EPI, 2, 2, 4, 2), SW = gemm_lds(EPI_FP, 2, 2, 4, 2), SMEM = SX > SW ? SX : SW;
+    static std::atomic<bool> opted_in[MAX_DEVICES] = {};
+    if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_backward_kernel<EPI, ST, SMALL>), SMEM, opted_in)) return rc;
+    const unsigned wgs = ((b.x.tiles_m * b.x.tiles_n + 7) & ~7) + b.w.tiles_m * b.w.tiles_n * b.w.splits;
+    hipLaunchKernelGGL((igemm_backward_kernel<EPI, ST, SMALL>), dim3(wgs), dim3(512), SMEM, st, b);
+    return (int)hipGetLastError();
+}
+
 extern "C" {
 
 const char *jf_error_string(int code)
@@ -1711,9 +1751,7 @@ static int block_fp_run(const int8_t *A, const int8_t *B, const void *sa, const 
     if (splits > 1) a.C = partials;
     int rc = scale_dtype == JF_SCALE_F16 ? launch_gemm<EPI_FP, half_t>(a, st, kn, a_km) : launch_gemm<EPI_FP, float>(a, st, kn, a_km);
     if (rc || splits == 1) return rc;
-    const size_t n = (size_t)M * (size_t)N;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)(n / 1024)), dim3(256), 0, st, (const float *)partials, n, splits, C, out_dtype);
-    return (int)hipGetLastError();
+    return launch_splitk_reduce((const float *)partials, (size_t)M * (size_t)N, splits, C, out_dtype, st);
 }
 
 static int block_fp_check(const int8_t *A, const int8_t *B, const void *sa, const void *sb, void *C, int M, int N, int K,
@@ -1877,6 +1915,65 @@ int jf_igemm_block_fp_noalloc(const int8_t *A, const int8_t *B, const void *sa, 
     // reduction reads it, so what an earlier (larger) call left behind is never read
     return block_fp_run(A, B, sa, sb, C, M, N, K, a_layout, b_layout, scale_dtype, sa_layout, sb_layout, out_dtype, splits,
                         kb_per, partials, (hipStream_t)stream);
+}
+
+// One launch for both gradients: neither needs the other's result, small ones leave most of the chip idle, and larger ones end in a
+// round that is not full, once instead of twice.  The activation gradient's tiles, which are longer, come first: 32x128 where one per CU
+// holds them all, and two per CU where K is long and a 128x128 tile would outlast everything else.  us, two launches | one, rows x
+// C_in x C_out:
+//   32x128: 32x768x768 10.3 | 6.4, 512x768x2304 20.8 | 13.2, 1024x1024x1024 22.8 | 18.7, 1248x768x3072 35.6 | 31.8; two per CU
+//   2048x1024x4096 55.5 | 52.5 (128x128: 59.0), 1024x1600x6400 65.7 | 56.7 (62.5);
+//   128x128: 2048x768x768 23.6 | 19.4 (32x128: 21.3), 1024x2048x1024 31.8 | 25.8 (28.5), 4096x768x768 35.0 | 26.0, 4096x1024x4096 84.4 | 78.3,
+//   12288x768x3072 127.5 | 119.4, 8192x1024x4096 141.4 | 138.2.
+// Above three 128x128 tiles of the activation gradient per CU the rounds even out by themselves: 4096x4096x1024 (1024) 86.1 | 83.7,
+// 8192x1600x4800 (832) 248.7 | 263.2, 8192x6400x1600 (3200) 359.4 | 363.9, 4096x4096x4096 (1024) 259.0 | 260.8.
+int jf_linear_bwd(const int8_t *X, const void *sx, const int8_t *G, const void *sg, const int8_t *W, const void *sw, int R, int C_in, int C_out,
+                  int scale_dtype, void *dx, void *dx_scales, int dx_dtype, uint64_t seed, uint64_t offset, void *dw, int dw_dtype, int splitk,
+                  void *workspace, size_t workspace_bytes, jf_stream_t stream)
+{
+    int rc = block_fp_check(G, X, sg, sx, dw, C_out, C_in, R, JF_A_KM, JF_B_KN, scale_dtype, dw_dtype);
+    if (!rc) rc = check_gemm_common(G, W, dx, R, C_in, C_out, JF_B_KN);
+    if (rc) return rc;
+    if (!sw) return JF_ERR_NULL;
+    if (!scale_ptr_ok(sw, scale_dtype)) return JF_ERR_ALIGN;
+    if (!dx_scales && dx_dtype != JF_FP_F16 && dx_dtype != JF_FP_F32 && dx_dtype != JF_FP_BF16) return JF_ERR_ENUM;
+    int splits = 1, kb_per = 0;
+    if ((rc = jf_igemm_splitk_plan(C_out, C_in, R, splitk, &splits, &kb_per))) return rc;
+    if (splits > 1 && (!workspace || !aligned16(workspace) || workspace_bytes < jf_igemm_block_fp_workspace_bytes(C_out, C_in, R, JF_B_KN, splitk)))
+        return JF_ERR_WORKSPACE;
+    hipStream_t st = (hipStream_t)stream;
+    const bool small = small_tiles_resident(R, C_in, C_out) && (C_out > 2048 || (long)(R / QB) * ((C_in + 127) / 128) <= cu_count());
+    const long tiles_w = (long)((C_out + 127) / 128) * ((C_in + 127) / 128) * splits;
+    if ((long)((R + 127) / 128) * ((C_in + 127) / 128) > 3L * cu_count() || tiles_w > 0x3fffffffL) {
+        if (dx_scales)
+            rc = jf_igemm_block_q(G, W, sg, sw, nullptr, nullptr, (int8_t *)dx, dx_scales, R, C_in, C_out, JF_B_KN, scale_dtype, JF_SCALES_ROWMAJOR,
+                                  JF_SCALES_KMAJOR, JF_ROUND_STOCHASTIC, seed, offset, nullptr, 0, stream);
+        else
+            rc = jf_igemm_block_q_dequant(G, W, sg, sw, nullptr, nullptr, dx, R, C_in, C_out, JF_B_KN, scale_dtype, JF_SCALES_ROWMAJOR,
+                                          JF_SCALES_KMAJOR, dx_dtype, JF_ROUND_STOCHASTIC, seed, offset, stream);
+        return rc ? rc : block_fp_run(G, X, sg, sx, dw, C_out, C_in, R, JF_A_KM, JF_B_KN, scale_dtype, JF_SCALES_KMAJOR, JF_SCALES_KMAJOR, dw_dtype,
+                                      splits, kb_per, workspace, st);
+    }
+    if (!device_is_gfx950()) return JF_ERR_DEVICE;
+    GemmArgs x = {}, w = {};
+    x.A = G; x.B = W; x.sa = sg; x.sb = sw; x.C = dx; x.sc = dx_scales; x.out_dtype = dx_dtype; x.rounding = JF_ROUND_STOCHASTIC;
+    x.seed = seed; x.offset = offset; x.M = R; x.N = C_in; x.K = C_out; x.lda = C_out; x.ldb = C_in;
+    w.A = G; w.B = X; w.sa = sg; w.sb = sx; w.C = splits > 1 ? workspace : dw; w.out_dtype = dw_dtype; w.splits = splits; w.kb_per_split = kb_per;
+    w.M = C_out; w.N = C_in; w.K = R; w.lda = C_out; w.ldb = C_in;
+    if (!scale_strides(JF_SCALES_ROWMAJOR, C_out, R / QB, x.sa_ks, x.sa_is) || !scale_strides(JF_SCALES_KMAJOR, C_out, C_in / QB, x.sb_ks, x.sb_is) ||
+        !scale_strides(JF_SCALES_KMAJOR, R, C_out / QB, w.sa_ks, w.sa_is) || !scale_strides(JF_SCALES_KMAJOR, R, C_in / QB, w.sb_ks, w.sb_is))
+        return JF_ERR_ENUM;
+    const bool f16 = scale_dtype == JF_SCALE_F16;
+    const auto launch = [&](auto epi_c, auto small_c) {
+        constexpr int EPI = decltype(epi_c)::value;
+        constexpr bool SMALL = decltype(small_c)::value;
+        return f16 ? launch_linear_bwd<EPI, half_t, SMALL>(x, w, st) : launch_linear_bwd<EPI, float, SMALL>(x, w, st);
+    };
+    const std::integral_constant<int, EPI_Q> q;
+    const std::integral_constant<int, EPI_QD> qd;
+    if (dx_scales) rc = small ? launch(q, std::true_type{}) : launch(q, std::false_type{});
+    else rc = small ? launch(qd, std::true_type{}) : launch(qd, std::false_type{});
+    return rc || splits == 1 ? rc : launch_splitk_reduce((const float *)workspace, (size_t)C_out * (size_t)C_in, splits, dw, dw_dtype, st);
 }
 
 int jf_igemm_block_q(const int8_t *A, const int8_t *B, const void *sa, const void *sb,

@@ -796,6 +796,26 @@ std::vector<Tensor> linear_backward(const Tensor &X, const Tensor &SX, const Ten
     c10::DeviceGuard guard(x.q.device());
     std::vector<Tensor> out;
     const auto so = rng(JF_ROUND_STOCHASTIC, g.q, g.R * w.C, c10::nullopt, c10::nullopt);
+    if (!GT) {
+        const torch::ScalarType odt = wgrad_dtype.value_or(torch::kFloat16);
+        const int oc = fp_code(odt, "wgrad_dtype");
+        TORCH_CHECK(splitk >= 0, "splitk must be >= 0");
+        out.push_back(fresh(with_last(g.q, w.C), dgrad_quantize ? g.q.options() : g.s.options()));
+        if (dgrad_quantize) out.push_back(fresh(with_last(g.s, w.C / QB), g.s.options()));
+        out.push_back(fresh({g.C, x.C}, x.q.options().dtype(odt)));
+        const size_t nbytes = jf_igemm_block_fp_workspace_bytes((int)g.C, (int)x.C, (int)x.R, JF_B_KN, (int)splitk);
+        Tensor ws;
+        if (nbytes) ws = scratch(x.q, nbytes);
+        {
+            pybind11::gil_scoped_release nogil;
+            check_rc(jf_linear_bwd(x.qp(), x.sp(), g.qp(), g.sp(), w.qp(), w.sp(), (int)g.R, (int)w.C, (int)g.C, g.code, out[0].data_ptr(),
+                                   dgrad_quantize ? out[1].data_ptr() : nullptr, g.code == JF_SCALE_F16 ? JF_FP_F16 : JF_FP_F32, so.first, so.second,
+                                   out.back().data_ptr(), oc, (int)splitk, nbytes ? ws.data_ptr() : nullptr, nbytes, current_stream(x.q)),
+                     "linear_backward");
+        }
+        if (bias_grad) out.push_back(block_colsum(g.q, g.s));
+        return out;
+    }
     if (dgrad_quantize) {
         out.push_back(fresh(with_last(g.q, w.C), g.q.options()));
         out.push_back(fresh(with_last(g.s, w.C / QB), g.s.options()));

@@ -461,6 +461,44 @@ def test_quantised_with_residual_addition(jf, oracle, M, N, K, x1, y, f16, bias)
     assert got[1].any()
 
 
+@pytest.mark.parametrize("R,C_in,C_out,splitk,f16,quantize", [
+    (32, 32, 32, 0, True, True),                     # one tile each
+    (96, 160, 224, 0, False, False),
+    (512, 768, 2304, 0, True, False),
+    (512, 768, 2304, 1, False, True),
+    (2048, 128, 256, 0, True, True),                 # weight gradient in parts
+    (1024, 1024, 64, 1, True, False),                # 256 tiles of 32x128 ...
+    (1056, 1024, 64, 1, False, False),               # ... and one row of them more: 128x128
+    (1056, 1024, 2080, 0, True, True),               # 32x128 again, for a long K
+    (2080, 1056, 96, 0, False, True),                # ragged tiles
+    (12288, 1024, 32, 0, True, True),                # the last launch of one kernel on 256 CUs ...
+    (12320, 1024, 32, 0, True, True),                # ... and the first of two
+])
+def test_both_gradients_of_a_linear_layer_in_one_launch(jf, R, C_in, C_out, splitk, f16, quantize):
+    """Bit for bit what the two entry points return (both of which are checked against the oracle elsewhere)."""
+    print(f"case bwd R={R} C_in={C_in} C_out={C_out} splitk={splitk} f16={f16} quantize={quantize}", flush=True)
+    rng = np.random.default_rng(R + C_in * 3 + C_out)
+    st = np.float16 if f16 else np.float32
+    block = lambda r, c: (dev(rand_codes(rng, (r, c))), dev(rand_scales(rng, (r // QB, c // QB), lo=-8, hi=-4, f16=f16).astype(st)))  # noqa: E731
+    (x, sx), (g, sg), (w, sw) = block(R, C_in), block(R, C_out), block(C_out, C_in)
+    L, p, seed, offset = jf.lib(), jf._ptr, 17, 8
+    code = jf.SCALE_F16 if f16 else jf.SCALE_F32
+    want_w = jf.igemm_block_fp(g, x, sg, sx, jf.B_KN, torch.float32, jf.A_KM, splitk)
+    if quantize:
+        want = jf.igemm_block_q(g, w, sg.t(), sw, jf.B_KN, rounding=jf.ROUND_STOCHASTIC, seed=seed, offset=offset)
+    else:
+        want = (jf.igemm_block_q_dequant(g, w, sg.t(), sw, jf.B_KN, torch.float16, rounding=jf.ROUND_STOCHASTIC, seed=seed, offset=offset),)
+    dx = torch.empty_like(want[0])
+    ds = torch.empty_like(want[1]) if quantize else None
+    dw = torch.empty_like(want_w)
+    nb = L.jf_igemm_block_fp_workspace_bytes(C_out, C_in, R, jf.B_KN, splitk)
+    ws = torch.empty(max(nb, 16), dtype=torch.int8, device="cuda")
+    jf.check(L.jf_linear_bwd(p(x), p(sx), p(g), p(sg), p(w), p(sw), R, C_in, C_out, code, p(dx), p(ds), jf.FP_F16, seed, offset, p(dw),
+                             jf.FP_F32, splitk, p(ws), nb, jf._stream()))
+    assert torch.equal(dw, want_w) and torch.equal(dx, want[0])
+    assert ds is None or torch.equal(ds, want[1])
+
+
 @pytest.mark.parametrize("approx", [0, 1])
 @pytest.mark.parametrize("f16", [True, False])
 @pytest.mark.parametrize("M,N,K", [(128, 256, 96), (96, 160, 224), (256, 384, 544), (32, 32, 32)])
