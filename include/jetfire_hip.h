@@ -327,6 +327,18 @@ int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const in
                   const int *M, const int *N, int K, int scale_dtype, int out_dtype, int ncol, const float *const *terms,
                   const int *width, float *const *sum, void *workspace, size_t workspace_bytes, jf_stream_t stream);
 
+/* jf_wgrad_many in two calls around work that depends on the first: jf_wgrad_many_dgrad forms the gradients (K split parts stay in the
+ * workspace) and, in the same launch where that is faster, the activation gradient of the first of them, (dx, dx_scales) [K, N[0]] =
+ * G[0] W with W codes [M[0], N[0]], as jf_igemm_block_q forms it with stochastic rounding; jf_wgrad_many_finish, given the same arguments
+ * and the workspace as it was left, adds the parts and the column sums. */
+int jf_wgrad_many_dgrad(const int8_t *W, const void *sw, int8_t *dx, void *dx_scales, uint64_t seed, uint64_t offset, int n,
+                        const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
+                        const int *M, const int *N, int K, int scale_dtype, int out_dtype, void *workspace, size_t workspace_bytes,
+                        jf_stream_t stream);
+int jf_wgrad_many_finish(int n, const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
+                         const int *M, const int *N, int K, int scale_dtype, int out_dtype, int ncol, const float *const *terms,
+                         const int *width, float *const *sum, void *workspace, size_t workspace_bytes, jf_stream_t stream);
+
 /* Causal self-attention between the QKV projection and the output projection, binary16 in and out.  q, k, v: [B*T, ld]
  * with head h of a row at columns h*D .. h*D + D - 1 of each pointer (the three column ranges of the projection's output,
  * ld = 3*H*D, or tensors of their own); out: [B*T, H*D]; lse: [B*H, T] fp32, log2 of the row sums (for the backward call).

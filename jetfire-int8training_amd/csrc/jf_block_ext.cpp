@@ -302,9 +302,9 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const jf_stream_t st = current_stream(qx);
         constexpr int RM = JF_SCALES_ROWMAJOR, KM = JF_SCALES_KMAJOR, F16 = JF_SCALE_F16, SR = JF_ROUND_STOCHASTIC;
         auto codes = [](const Tensor &a) { return (const int8_t *)a.data_ptr(); };
-        // The weight gradients run together at the end: one launch has tiles for the whole chip where each of the four alone
-        // leaves a last round half empty, and one more adds what is left to add, the parts of K splits and the LayerNorm weights'
-        // gradients.
+        // The weight gradients run together, with the last activation gradient: one launch has tiles for the whole chip where each
+        // alone leaves a last round half empty, and one more at the end adds what is left to add, the parts of K splits and the
+        // LayerNorm weights' gradients.
         const int8_t *wg[4], *wx[4];
         const void *wgs[4], *wxs[4];
         auto wgrad = [&](int i, const int8_t *g, const void *gs, const int8_t *xq, const void *xs) {
@@ -328,18 +328,18 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const c10::Half *qkv = (const c10::Half *)v.qkv;
         check_rc(jf_attention_bwd_q(qkv, qkv + c, qkv + 2 * c, 3 * c, v.y, t.gy, v.lse, d.B, d.H, d.T, c / d.H, (float)(1.0 / std::sqrt((double)(c / d.H))),
                                     t.qq, t.sq, z[6].seed, z[6].offset, t.delta, st), "gradient of attention");
-        check_rc(jf_igemm_block_q(t.qq, codes(w[0].q), t.sq, w[0].s.data_ptr(), nullptr, nullptr, t.qd, t.sd, m, c, 3 * c, JF_B_KN, F16, RM, KM, SR,
-                                  z[7].seed, z[7].offset, nullptr, 0, st), "gradient of qkv");
         wgrad(0, t.qq, t.sq, v.qn, v.sn);
+        void *const gw[4] = {out[W_QKV].data_ptr(), out[W_PROJ].data_ptr(), out[W_FC].data_ptr(), out[W_FC2].data_ptr()};
+        check_rc(jf_wgrad_many_dgrad(codes(w[0].q), w[0].s.data_ptr(), t.qd, t.sd, z[7].seed, z[7].offset, 4, wg, wgs, wx, wxs, gw, wrows, wcols, m, F16,
+                                     wc, t.ws, ws_bytes, st), "gradient of qkv and weight gradients");
         check_rc(jf_layernorm_bwd_add_strips(codes(qx), sx.data_ptr(), t.qd, t.sd, ln1.data_ptr<float>(), mean.data_ptr<float>(), rstd.data_ptr<float>(), m, c, F16,
                                       SR, z[8].seed, z[8].offset, t.res, resc, JF_ROUND_STOCHASTIC_TRUNC, z[9].seed, z[9].offset, out[X].data_ptr(), resc,
                                       (int8_t *)out[QX].data_ptr(), out[SX].data_ptr(), t.ln1_terms, st),
                  "gradient of layernorm");
-        void *const gw[4] = {out[W_QKV].data_ptr(), out[W_PROJ].data_ptr(), out[W_FC].data_ptr(), out[W_FC2].data_ptr()};
         const float *const terms[2] = {t.ln1_terms, t.ln2_terms};
         float *const gln[2] = {out[LN1].data_ptr<float>(), out[LN2].data_ptr<float>()};
         const int widths[2] = {c, c};
-        check_rc(jf_wgrad_many(4, wg, wgs, wx, wxs, gw, wrows, wcols, m, F16, wc, 2, terms, widths, gln, t.ws, ws_bytes, st), "weight gradients");
+        check_rc(jf_wgrad_many_finish(4, wg, wgs, wx, wxs, gw, wrows, wcols, m, F16, wc, 2, terms, widths, gln, t.ws, ws_bytes, st), "weight gradients");
         if (with_bias && b_type != torch::kFloat32)
             for (int i = 0; i < 4; ++i) out[B_QKV + i] = out[B_QKV + i].to(b_type);
         return out;

@@ -1218,24 +1218,6 @@ template <int EPI, typename ST, int BKN> __global__ __launch_bounds__(512, 4) vo
     }
 }
 
-// Both gradients of a linear layer (launch_linear_bwd): 32x128 or 128x128 tiles of the activation gradient (EPI_Q or EPI_QD, B as
-// [K,N]), then 128x128 tiles of the weight gradient.
-struct GemmBackward {
-    GemmArgs x, w;
-};
-template <int EPI, typename ST, bool SMALL> __global__ __launch_bounds__(512, 4) void igemm_backward_kernel(GemmBackward b)
-{
-    const int work_x = b.x.tiles_m * b.x.tiles_n, first_w = (work_x + 7) & ~7;      // (both parts are dealt to the XCDs from the first one on)
-    const int wg = blockIdx.x;
-    if (wg < first_w) {
-        const int logical = logical_workgroup(work_x, wg);
-        if (logical >= 0) igemm_body<EPI, ST, SMALL ? 1 : 2, SMALL ? 1 : 2, 4, SMALL ? 3 : 2, 2, 1, 0, 0>(b.x, logical);
-    } else {
-        const int logical = logical_workgroup(b.w.tiles_m * b.w.tiles_n * b.w.splits, wg - first_w);
-        if (logical >= 0) igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0>(b.w, logical);
-    }
-}
-
 // Several weight gradients over the same tokens in one launch (jf_wgrad_many).  Every XCD gets one contiguous run of each problem's
 // work, one problem after the other, so that the XCDs finish together although the parts of the problems differ in length.  (One
 // run over all problems: GPT-2 XL's four, one of them in parts a third as long, took 60 us more than the 500 they take.)
@@ -1245,10 +1227,9 @@ struct GemmGroup {
     int end[WGRAD_MAX];       // first workgroup behind problem k, of an XCD's: ceil(work / 8) for each problem
     int n;
 };
-template <typename ST>
-__global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp)
+template <typename ST> __device__ __forceinline__ void wgrad_group_body(const GemmGroup &grp, const int wg)
 {
-    const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+    const int xcd = wg & 7, at = wg >> 3;
     int k = 0, begin = 0;
 #pragma unroll
     for (int i = 1; i < WGRAD_MAX; ++i)
@@ -1256,6 +1237,25 @@ __global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp
     const GemmArgs &p = grp.g[k];
     const int logical = logical_workgroup(p.tiles_m * p.tiles_n * p.splits, (at - begin) * 8 + xcd);
     if (logical >= 0) igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0, 1>(p, logical);
+}
+template <typename ST> __global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp) { wgrad_group_body<ST>(grp, blockIdx.x); }
+
+// An activation gradient (EPI_Q or EPI_QD, B as [K,N]; 32x128 or 128x128 tiles), then weight gradients, in one launch: both gradients of
+// a linear layer, or the last one of a block with all of the block's weight gradients.
+struct GemmBackward {
+    GemmArgs x;
+    GemmGroup w;
+};
+template <int EPI, typename ST, bool SMALL> __global__ __launch_bounds__(512, 4) void igemm_backward_kernel(GemmBackward b)
+{
+    const int work_x = b.x.tiles_m * b.x.tiles_n, first_w = (work_x + 7) & ~7;      // (both parts are dealt to the XCDs from the first one on)
+    const int wg = blockIdx.x;
+    if (wg < first_w) {
+        const int logical = logical_workgroup(work_x, wg);
+        if (logical >= 0) igemm_body<EPI, ST, SMALL ? 1 : 2, SMALL ? 1 : 2, 4, SMALL ? 3 : 2, 2, 1, 0, 0>(b.x, logical);
+    } else {
+        wgrad_group_body<ST>(b.w, wg - first_w);
+    }
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -1648,20 +1648,60 @@ static bool scale_ptr_ok(const void *p, int scale_dtype)
 }
 
 #ifndef JF_PROF_LIB
-// x, w: as for their own launches.
-template <int EPI, typename ST, bool SMALL> static int launch_linear_bwd(const GemmArgs &x, const GemmArgs &w, hipStream_t st)
+// x: as for a launch of its own; w: w_wgs workgroups, the longest of them k_per_part deep.
+template <int EPI, typename ST, bool SMALL> static int launch_backward(const GemmArgs &x, const GemmGroup &w, long w_wgs, int k_per_part, hipStream_t st)
 {
     GemmBackward b = {x, w};
     b.x.tiles_m = SMALL ? x.M / QB : (x.M + 127) / 128; b.x.tiles_n = (x.N + 127) / 128; b.x.splits = 1;
-    b.w.tiles_m = (w.M + 127) / 128; b.w.tiles_n = (w.N + 127) / 128;
-    const long work = (long)b.x.tiles_m * b.x.tiles_n + (long)b.w.tiles_m * b.w.tiles_n * b.w.splits;
-    b.x.pace = b.w.pace = SMALL ? (int)PACE_HARDWARE : pace_of(work, 2L * cu_count(), std::max(x.K, w.splits > 1 ? w.kb_per_split * QB : w.K));
+    const long x_wgs = ((long)b.x.tiles_m * b.x.tiles_n + 7) & ~7L;
+    b.x.pace = SMALL ? (int)PACE_HARDWARE : pace_of(x_wgs + w_wgs, 2L * cu_count(), std::max(x.K, k_per_part));
+    for (int i = 0; i < w.n; ++i) b.w.g[i].pace = b.x.pace;
     constexpr int SX = SMALL ? gemm_lds(EPI, 1, 1, 4, 3) : gemm_lds(EPI, 2, 2, 4, 2), SW = gemm_lds(EPI_FP, 2, 2, 4, 2), SMEM = SX > SW ? SX : SW;
     static std::atomic<bool> opted_in[MAX_DEVICES] = {};
     if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_backward_kernel<EPI, ST, SMALL>), SMEM, opted_in)) return rc;
-    const unsigned wgs = ((b.x.tiles_m * b.x.tiles_n + 7) & ~7) + b.w.tiles_m * b.w.tiles_n * b.w.splits;
-    hipLaunchKernelGGL((igemm_backward_kernel<EPI, ST, SMALL>), dim3(wgs), dim3(512), SMEM, st, b);
+    hipLaunchKernelGGL((igemm_backward_kernel<EPI, ST, SMALL>), dim3((unsigned)(x_wgs + w_wgs)), dim3(512), SMEM, st, b);
     return (int)hipGetLastError();
+}
+// One launch for an activation gradient and weight gradients: neither needs the other's result, small ones leave most of the chip
+// idle, and larger ones end in a round that is not full, once instead of twice.  The activation gradient's tiles, which are longer, come
+// first: 32x128 where one per CU holds them all, and two per CU where K is long and a 128x128 tile would outlast everything else.  us,
+// two launches | one, both gradients of a layer, rows x C_in x C_out:
+//   32x128: 32x768x768 10.3 | 6.4, 512x768x2304 20.8 | 13.2, 1024x1024x1024 22.8 | 18.7, 1248x768x3072 35.6 | 31.8; two per CU
+//   2048x1024x4096 55.5 | 52.5 (128x128: 59.0), 1024x1600x6400 65.7 | 56.7 (62.5);
+//   128x128: 2048x768x768 23.6 | 19.4 (32x128: 21.3), 1024x2048x1024 31.8 | 25.8 (28.5), 4096x768x768 35.0 | 26.0, 4096x1024x4096 84.4 | 78.3,
+//   12288x768x3072 127.5 | 119.4, 8192x1024x4096 141.4 | 138.2.
+// Above three 128x128 tiles of the activation gradient per CU the rounds even out by themselves: 4096x4096x1024 (1024) 86.1 | 83.7,
+// 8192x1600x4800 (832) 248.7 | 263.2, 8192x6400x1600 (3200) 359.4 | 363.9, 4096x4096x4096 (1024) 259.0 | 260.8.
+static bool backward_in_one_launch(int R, int C_in, long w_wgs)
+{
+    return (long)((R + 127) / 128) * ((C_in + 127) / 128) <= 3L * cu_count() && w_wgs <= 0x3fffffffL;
+}
+template <int EPI> static int launch_backward_any(const GemmArgs &x, const GemmGroup &w, long w_wgs, int k_per_part, bool f16, hipStream_t st)
+{
+    const bool small = small_tiles_resident(x.M, x.N, x.K) && (x.K > 2048 || (long)(x.M / QB) * ((x.N + 127) / 128) <= cu_count());
+    if (small) return f16 ? launch_backward<EPI, half_t, true>(x, w, w_wgs, k_per_part, st) : launch_backward<EPI, float, true>(x, w, w_wgs, k_per_part, st);
+    return f16 ? launch_backward<EPI, half_t, false>(x, w, w_wgs, k_per_part, st) : launch_backward<EPI, float, false>(x, w, w_wgs, k_per_part, st);
+}
+// dX [R, C_in] = G [R, C_out] W [C_out, C_in], requantised or (dx_scales null) dequantised, scales in the tensors' own layout
+static GemmArgs dgrad_args(const int8_t *G, const void *sg, const int8_t *W, const void *sw, int R, int C_in, int C_out, void *dx, void *dx_scales,
+                           int dx_dtype, uint64_t seed, uint64_t offset)
+{
+    GemmArgs x = {};
+    x.A = G; x.B = W; x.sa = sg; x.sb = sw; x.C = dx; x.sc = dx_scales; x.out_dtype = dx_dtype; x.rounding = JF_ROUND_STOCHASTIC;
+    x.seed = seed; x.offset = offset; x.M = R; x.N = C_in; x.K = C_out; x.lda = C_out; x.ldb = C_in;
+    x.sa_ks = 1; x.sa_is = C_out / QB; x.sb_ks = C_in / QB; x.sb_is = 1;
+    return x;
+}
+// dW [C_out, C_in] = G^T X, in `splits` parts
+static GemmArgs wgrad_args(const int8_t *G, const void *sg, const int8_t *X, const void *sx, int R, int C_in, int C_out, void *out, int out_dtype,
+                           int splits, int kb_per_split)
+{
+    GemmArgs a = {};
+    a.A = G; a.B = X; a.sa = sg; a.sb = sx; a.C = out; a.out_dtype = out_dtype; a.splits = splits; a.kb_per_split = kb_per_split;
+    a.M = C_out; a.N = C_in; a.K = R; a.lda = C_out; a.ldb = C_in;
+    a.sa_ks = C_out / QB; a.sa_is = 1; a.sb_ks = C_in / QB; a.sb_is = 1;
+    a.tiles_m = (C_out + 127) / 128; a.tiles_n = (C_in + 127) / 128;
+    return a;
 }
 
 extern "C" {
@@ -1804,9 +1844,16 @@ size_t jf_wgrad_many_workspace_bytes(int n, const int *M, const int *N, int K)
     return wgrad_workspace(n, M, N, plan);
 }
 
-int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
-                  const int *M, const int *N, int K, int scale_dtype, int out_dtype, int ncol, const float *const *terms,
-                  const int *width, float *const *sum, void *workspace, size_t workspace_bytes, jf_stream_t stream)
+// The launches of jf_wgrad_many and jf_wgrad_many_dgrad: plan, group of GEMMs and what follows it
+struct WgradLaunch {
+    GemmGroup grp;
+    WgradFinish fin;
+    long wgs, fwgs;
+    int longest;              // K blocks of a workgroup
+};
+static int wgrad_launch(int n, const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
+                        const int *M, const int *N, int K, int scale_dtype, int out_dtype, int ncol, const float *const *terms,
+                        const int *width, float *const *sum, void *workspace, size_t workspace_bytes, WgradLaunch &l)
 {
     if (n < 1 || n > WGRAD_MAX || ncol < 0 || ncol > WGRAD_MAX) return JF_ERR_SHAPE;
     if (!G || !SG || !X || !SX || !out || !M || !N || (ncol && (!terms || !width || !sum))) return JF_ERR_NULL;
@@ -1826,49 +1873,96 @@ int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const in
     int order[WGRAD_MAX];                                      // longest parts first: the short ones even out the end of the launch
     for (int i = 0; i < n; ++i) order[i] = i;
     std::stable_sort(order, order + n, [&](int a, int b) { return plan.kb_per_split[a] > plan.kb_per_split[b]; });
-    GemmGroup grp = {};
-    WgradFinish fin = {};
+    l = {};
     float *part = (float *)workspace;
-    long wgs = 0, fwgs = 0;
-    int longest = 0;
     for (int j = 0; j < n; ++j) {
         const int i = order[j], splits = plan.splits[i];
-        GemmArgs &a = grp.g[j];
-        a.A = G[i]; a.B = X[i]; a.sa = SG[i]; a.sb = SX[i]; a.C = out[i];
-        a.M = M[i]; a.N = N[i]; a.K = K; a.lda = M[i]; a.ldb = N[i]; a.out_dtype = out_dtype; a.splits = splits; a.kb_per_split = plan.kb_per_split[i];
-        a.sa_ks = M[i] / QB; a.sa_is = 1; a.sb_ks = N[i] / QB; a.sb_is = 1;
-        a.tiles_m = (M[i] + 127) / 128; a.tiles_n = (N[i] + 127) / 128;
+        GemmArgs &a = l.grp.g[j];
+        a = wgrad_args(G[i], SG[i], X[i], SX[i], K, N[i], M[i], out[i], out_dtype, splits, plan.kb_per_split[i]);
         if (plan.fold_kb[i]) {
             a.fold_kb = plan.fold_kb[i]; a.fold = part;
             part += wgrad_fold_values(M[i], N[i], splits);
         }
-        wgs += ((long)a.tiles_m * a.tiles_n * splits + 7) / 8;
-        grp.end[j] = (int)wgs;
-        if (plan.kb_per_split[i] > longest) longest = plan.kb_per_split[i];
+        l.wgs += ((long)a.tiles_m * a.tiles_n * splits + 7) / 8;
+        l.grp.end[j] = (int)l.wgs;
+        if (plan.kb_per_split[i] > l.longest) l.longest = plan.kb_per_split[i];
         if (splits > 1) {
             const size_t count = (size_t)M[i] * (size_t)N[i];
-            fwgs += (long)((count + 4095) / 4096);
+            l.fwgs += (long)((count + 4095) / 4096);
             a.C = part;
-            fin.part[fin.n] = part; fin.out[fin.n] = out[i]; fin.count[fin.n] = count; fin.splits[fin.n] = splits; fin.end[fin.n] = (int)fwgs;
+            WgradFinish &fin = l.fin;
+            fin.part[fin.n] = part; fin.out[fin.n] = out[i]; fin.count[fin.n] = count; fin.splits[fin.n] = splits; fin.end[fin.n] = (int)l.fwgs;
             ++fin.n;
             part += (size_t)splits * count;
         }
     }
     for (int i = 0; i < ncol; ++i) {
-        fwgs += width[i] / QB;
-        fin.terms[i] = terms[i]; fin.sum[i] = sum[i]; fin.width[i] = width[i]; fin.cend[i] = (int)fwgs;
+        l.fwgs += width[i] / QB;
+        l.fin.terms[i] = terms[i]; l.fin.sum[i] = sum[i]; l.fin.width[i] = width[i]; l.fin.cend[i] = (int)l.fwgs;
     }
-    wgs *= 8;
-    if (wgs > 0x7fffffffL || fwgs > 0x7fffffffL) return JF_ERR_SHAPE;
-    grp.n = n;
-    fin.ncol = ncol; fin.strips = K / QB; fin.out_dtype = out_dtype;
-    const int pace = pace_of(wgs, 2L * cu_count(), longest * QB);
-    for (int i = 0; i < n; ++i) grp.g[i].pace = pace;
-    hipStream_t st = (hipStream_t)stream;
-    int rc = scale_dtype == JF_SCALE_F16 ? launch_wgrad_group<half_t>(grp, (unsigned)wgs, st) : launch_wgrad_group<float>(grp, (unsigned)wgs, st);
-    if (rc || fwgs == 0) return rc;
-    hipLaunchKernelGGL(wgrad_finish_kernel, dim3((unsigned)fwgs), dim3(1024), 0, st, fin);
+    l.wgs *= 8;
+    if (l.wgs > 0x7fffffffL || l.fwgs > 0x7fffffffL) return JF_ERR_SHAPE;
+    l.grp.n = n;
+    l.fin.ncol = ncol; l.fin.strips = K / QB; l.fin.out_dtype = out_dtype;
+    return JF_OK;
+}
+static int launch_wgrads(WgradLaunch &l, bool f16, hipStream_t st)
+{
+    const int pace = pace_of(l.wgs, 2L * cu_count(), l.longest * QB);
+    for (int i = 0; i < l.grp.n; ++i) l.grp.g[i].pace = pace;
+    return f16 ? launch_wgrad_group<half_t>(l.grp, (unsigned)l.wgs, st) : launch_wgrad_group<float>(l.grp, (unsigned)l.wgs, st);
+}
+static int launch_finish(const WgradLaunch &l, hipStream_t st)
+{
+    if (l.fwgs == 0) return JF_OK;
+    hipLaunchKernelGGL(wgrad_finish_kernel, dim3((unsigned)l.fwgs), dim3(1024), 0, st, l.fin);
     return (int)hipGetLastError();
+}
+
+int jf_wgrad_many(int n, const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
+                  const int *M, const int *N, int K, int scale_dtype, int out_dtype, int ncol, const float *const *terms,
+                  const int *width, float *const *sum, void *workspace, size_t workspace_bytes, jf_stream_t stream)
+{
+    WgradLaunch l;
+    int rc = wgrad_launch(n, G, SG, X, SX, out, M, N, K, scale_dtype, out_dtype, ncol, terms, width, sum, workspace, workspace_bytes, l);
+    if (!rc) rc = launch_wgrads(l, scale_dtype == JF_SCALE_F16, (hipStream_t)stream);
+    return rc ? rc : launch_finish(l, (hipStream_t)stream);
+}
+
+// A group of weight gradients fills the chip by itself and ends in a short round; the activation gradient's tiles are worth having in it
+// where they are few, or the sums over the tokens short.  us of a training step of three blocks, two launches | one, tokens x width (128x128
+// tiles of the activation gradient): 1024x768 (48) 733 | 718, 1024x1600 (104) 1348 | 1322, 4096x768 (192) 1279 | 1270, 4096x1024 (256) 1663 |
+// 1629, 4096x1600 (416) 3252 | 3219, 8192x256 (128) 674 | 662; on the other side 8192x512 (256) 1225 | 1234, 6144x768 (288) 1576 | 1585,
+// 8192x768 (384) 1903 | 1939, 12288x768 (576) 2700 | 2720.
+int jf_wgrad_many_dgrad(const int8_t *W, const void *sw, int8_t *dx, void *dx_scales, uint64_t seed, uint64_t offset, int n,
+                        const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
+                        const int *M, const int *N, int K, int scale_dtype, int out_dtype, void *workspace, size_t workspace_bytes,
+                        jf_stream_t stream)
+{
+    WgradLaunch l;
+    int rc = wgrad_launch(n, G, SG, X, SX, out, M, N, K, scale_dtype, out_dtype, 0, nullptr, nullptr, nullptr, workspace, workspace_bytes, l);
+    if (!rc) rc = check_gemm_common(G[0], W, dx, K, N[0], M[0], JF_B_KN);
+    if (rc) return rc;
+    if (!sw || !dx_scales) return JF_ERR_NULL;
+    if (!scale_ptr_ok(sw, scale_dtype)) return JF_ERR_ALIGN;
+    hipStream_t st = (hipStream_t)stream;
+    const bool f16 = scale_dtype == JF_SCALE_F16;
+    const bool few = (long)((K + 127) / 128) * ((N[0] + 127) / 128) <= cu_count() / 2;
+    if (backward_in_one_launch(K, N[0], l.wgs) && (few || K <= 4096))
+        return launch_backward_any<EPI_Q>(dgrad_args(G[0], SG[0], W, sw, K, N[0], M[0], dx, dx_scales, 0, seed, offset), l.grp, l.wgs,
+                                          l.longest * QB, f16, st);
+    rc = jf_igemm_block_q(G[0], W, SG[0], sw, nullptr, nullptr, dx, dx_scales, K, N[0], M[0], JF_B_KN, scale_dtype, JF_SCALES_ROWMAJOR,
+                          JF_SCALES_KMAJOR, JF_ROUND_STOCHASTIC, seed, offset, nullptr, 0, stream);
+    return rc ? rc : launch_wgrads(l, f16, st);
+}
+
+int jf_wgrad_many_finish(int n, const int8_t *const *G, const void *const *SG, const int8_t *const *X, const void *const *SX, void *const *out,
+                         const int *M, const int *N, int K, int scale_dtype, int out_dtype, int ncol, const float *const *terms,
+                         const int *width, float *const *sum, void *workspace, size_t workspace_bytes, jf_stream_t stream)
+{
+    WgradLaunch l;
+    const int rc = wgrad_launch(n, G, SG, X, SX, out, M, N, K, scale_dtype, out_dtype, ncol, terms, width, sum, workspace, workspace_bytes, l);
+    return rc ? rc : launch_finish(l, (hipStream_t)stream);
 }
 
 // ---- the allocation-free weight-gradient entry point ---------------------------------------------------------------
@@ -1917,16 +2011,6 @@ int jf_igemm_block_fp_noalloc(const int8_t *A, const int8_t *B, const void *sa, 
                         kb_per, partials, (hipStream_t)stream);
 }
 
-// One launch for both gradients: neither needs the other's result, small ones leave most of the chip idle, and larger ones end in a
-// round that is not full, once instead of twice.  The activation gradient's tiles, which are longer, come first: 32x128 where one per CU
-// holds them all, and two per CU where K is long and a 128x128 tile would outlast everything else.  us, two launches | one, rows x
-// C_in x C_out:
-//   32x128: 32x768x768 10.3 | 6.4, 512x768x2304 20.8 | 13.2, 1024x1024x1024 22.8 | 18.7, 1248x768x3072 35.6 | 31.8; two per CU
-//   2048x1024x4096 55.5 | 52.5 (128x128: 59.0), 1024x1600x6400 65.7 | 56.7 (62.5);
-//   128x128: 2048x768x768 23.6 | 19.4 (32x128: 21.3), 1024x2048x1024 31.8 | 25.8 (28.5), 4096x768x768 35.0 | 26.0, 4096x1024x4096 84.4 | 78.3,
-//   12288x768x3072 127.5 | 119.4, 8192x1024x4096 141.4 | 138.2.
-// Above three 128x128 tiles of the activation gradient per CU the rounds even out by themselves: 4096x4096x1024 (1024) 86.1 | 83.7,
-// 8192x1600x4800 (832) 248.7 | 263.2, 8192x6400x1600 (3200) 359.4 | 363.9, 4096x4096x4096 (1024) 259.0 | 260.8.
 int jf_linear_bwd(const int8_t *X, const void *sx, const int8_t *G, const void *sg, const int8_t *W, const void *sw, int R, int C_in, int C_out,
                   int scale_dtype, void *dx, void *dx_scales, int dx_dtype, uint64_t seed, uint64_t offset, void *dw, int dw_dtype, int splitk,
                   void *workspace, size_t workspace_bytes, jf_stream_t stream)
@@ -1942,9 +2026,12 @@ int jf_linear_bwd(const int8_t *X, const void *sx, const int8_t *G, const void *
     if (splits > 1 && (!workspace || !aligned16(workspace) || workspace_bytes < jf_igemm_block_fp_workspace_bytes(C_out, C_in, R, JF_B_KN, splitk)))
         return JF_ERR_WORKSPACE;
     hipStream_t st = (hipStream_t)stream;
-    const bool small = small_tiles_resident(R, C_in, C_out) && (C_out > 2048 || (long)(R / QB) * ((C_in + 127) / 128) <= cu_count());
-    const long tiles_w = (long)((C_out + 127) / 128) * ((C_in + 127) / 128) * splits;
-    if ((long)((R + 127) / 128) * ((C_in + 127) / 128) > 3L * cu_count() || tiles_w > 0x3fffffffL) {
+    GemmGroup w = {};
+    w.n = 1;
+    w.g[0] = wgrad_args(G, sg, X, sx, R, C_in, C_out, splits > 1 ? workspace : dw, dw_dtype, splits, kb_per);
+    const long w_wgs = ((long)w.g[0].tiles_m * w.g[0].tiles_n * splits + 7) / 8 * 8;
+    w.end[0] = (int)(w_wgs / 8);
+    if (!backward_in_one_launch(R, C_in, w_wgs)) {
         if (dx_scales)
             rc = jf_igemm_block_q(G, W, sg, sw, nullptr, nullptr, (int8_t *)dx, dx_scales, R, C_in, C_out, JF_B_KN, scale_dtype, JF_SCALES_ROWMAJOR,
                                   JF_SCALES_KMAJOR, JF_ROUND_STOCHASTIC, seed, offset, nullptr, 0, stream);
@@ -1955,24 +2042,10 @@ int jf_linear_bwd(const int8_t *X, const void *sx, const int8_t *G, const void *
                                       splits, kb_per, workspace, st);
     }
     if (!device_is_gfx950()) return JF_ERR_DEVICE;
-    GemmArgs x = {}, w = {};
-    x.A = G; x.B = W; x.sa = sg; x.sb = sw; x.C = dx; x.sc = dx_scales; x.out_dtype = dx_dtype; x.rounding = JF_ROUND_STOCHASTIC;
-    x.seed = seed; x.offset = offset; x.M = R; x.N = C_in; x.K = C_out; x.lda = C_out; x.ldb = C_in;
-    w.A = G; w.B = X; w.sa = sg; w.sb = sx; w.C = splits > 1 ? workspace : dw; w.out_dtype = dw_dtype; w.splits = splits; w.kb_per_split = kb_per;
-    w.M = C_out; w.N = C_in; w.K = R; w.lda = C_out; w.ldb = C_in;
-    if (!scale_strides(JF_SCALES_ROWMAJOR, C_out, R / QB, x.sa_ks, x.sa_is) || !scale_strides(JF_SCALES_KMAJOR, C_out, C_in / QB, x.sb_ks, x.sb_is) ||
-        !scale_strides(JF_SCALES_KMAJOR, R, C_out / QB, w.sa_ks, w.sa_is) || !scale_strides(JF_SCALES_KMAJOR, R, C_in / QB, w.sb_ks, w.sb_is))
-        return JF_ERR_ENUM;
+    const GemmArgs x = dgrad_args(G, sg, W, sw, R, C_in, C_out, dx, dx_scales, dx_dtype, seed, offset);
     const bool f16 = scale_dtype == JF_SCALE_F16;
-    const auto launch = [&](auto epi_c, auto small_c) {
-        constexpr int EPI = decltype(epi_c)::value;
-        constexpr bool SMALL = decltype(small_c)::value;
-        return f16 ? launch_linear_bwd<EPI, half_t, SMALL>(x, w, st) : launch_linear_bwd<EPI, float, SMALL>(x, w, st);
-    };
-    const std::integral_constant<int, EPI_Q> q;
-    const std::integral_constant<int, EPI_QD> qd;
-    if (dx_scales) rc = small ? launch(q, std::true_type{}) : launch(q, std::false_type{});
-    else rc = small ? launch(qd, std::true_type{}) : launch(qd, std::false_type{});
+    const int depth = splits > 1 ? kb_per * QB : R;
+    rc = dx_scales ? launch_backward_any<EPI_Q>(x, w, w_wgs, depth, f16, st) : launch_backward_any<EPI_QD>(x, w, w_wgs, depth, f16, st);
     return rc || splits == 1 ? rc : launch_splitk_reduce((const float *)workspace, (size_t)C_out * (size_t)C_in, splits, dw, dw_dtype, st);
 }
 

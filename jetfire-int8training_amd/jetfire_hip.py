@@ -31,7 +31,7 @@ EXPORTS = [
     "jf_layernorm_bwd_workspace_bytes", "jf_layernorm_bwd", "jf_layernorm_bwd_add", "jf_layernorm_bwd_add_strips", "jf_gelu_fwd", "jf_gelu_bwd", "jf_add", "jf_rowstats_finish",
     "jf_igemm_block_q_dequant", "jf_quantize_slabs", "jf_philox_rounds", "jf_block_colsum", "jf_block_colsum_workspace_bytes",
     "jf_attention_fwd", "jf_attention_bwd", "jf_quantize_many", "jf_rowstats_fp", "jf_wgrad_many", "jf_wgrad_many_workspace_bytes",
-    "jf_layernorm_fwd_sums", "jf_attention_fwd_q", "jf_attention_bwd_q", "jf_igemm_block_q_add", "jf_linear_bwd",
+    "jf_layernorm_fwd_sums", "jf_attention_fwd_q", "jf_attention_bwd_q", "jf_igemm_block_q_add", "jf_linear_bwd", "jf_wgrad_many_dgrad", "jf_wgrad_many_finish",
 ]
 
 _lib = None
@@ -57,6 +57,8 @@ def lib():
         L.jf_wgrad_many_workspace_bytes.restype = _sz
         L.jf_layernorm_fwd_sums.argtypes = [_p, _p, _p, _p, _p, _p, _i, _i, _i, _p, _p, _p, _p, _p]
         L.jf_wgrad_many.argtypes = [_i, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _p, _p, _sz, _p]
+        L.jf_wgrad_many_dgrad.argtypes = [_p, _p, _p, _p, _u64, _u64, _i, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _p, _sz, _p]
+        L.jf_wgrad_many_finish.argtypes = L.jf_wgrad_many.argtypes
         L.jf_igemm_block_q_gelu_bwd.argtypes = [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _u64, _u64, _i, _u64, _u64, _p]
         L.jf_igemm_block_q_dequant.argtypes = [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _u64, _u64, _p]
         L.jf_igemm_block_q_gelu.argtypes = [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _f, _p]

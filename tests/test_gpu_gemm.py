@@ -5,6 +5,7 @@ accumulation is compared bit-exact too (same fmaf chain); fp16 output = RNE of i
 Shapes: the reference's own test lists (JetfireGEMMKernel/tests/*.py) plus shapes that are not
 multiples of the 128x128 tile (where the reference drops tiles) and a K with an odd number of blocks.
 """
+import ctypes
 import os
 
 import numpy as np
@@ -497,6 +498,33 @@ def test_both_gradients_of_a_linear_layer_in_one_launch(jf, R, C_in, C_out, spli
                              jf.FP_F32, splitk, p(ws), nb, jf._stream()))
     assert torch.equal(dw, want_w) and torch.equal(dx, want[0])
     assert ds is None or torch.equal(ds, want[1])
+
+
+@pytest.mark.parametrize("R,C,f16", [(64, 96, True), (1024, 256, True), (2112, 544, False), (4096, 1056, True), (4128, 1056, True)])
+def test_weight_gradients_with_an_activation_gradient(jf, R, C, f16):
+    """In 32x128 tiles, in 128x128 tiles and, the last one, apart: bit for bit what the two entry points return."""
+    print(f"case wgrads+dgrad R={R} C={C} f16={f16}", flush=True)
+    rng = np.random.default_rng(R + C)
+    st = np.float16 if f16 else np.float32
+    block = lambda r, c: (dev(rand_codes(rng, (r, c))), dev(rand_scales(rng, (r // QB, c // QB), lo=-8, hi=-4, f16=f16).astype(st)))  # noqa: E731
+    gs, xs = [block(R, 3 * C), block(R, 32)], [block(R, C), block(R, 64)]
+    w, sw = block(3 * C, C)
+    terms = torch.rand((R // QB, C), device="cuda")
+    want, (wsum,) = jf.wgrad_many(gs, xs, terms=[terms])
+    wq, ws_ = jf.igemm_block_q(gs[0][0], w, gs[0][1].t(), sw, jf.B_KN, rounding=jf.ROUND_STOCHASTIC, seed=5, offset=16)
+    L, p = jf.lib(), jf._ptr
+    ptrs = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])  # noqa: E731
+    ints = lambda *v: (ctypes.c_int * len(v))(*v)  # noqa: E731
+    out, total, q, s = [torch.empty_like(t) for t in want], torch.empty_like(wsum), torch.empty_like(wq), torch.empty_like(ws_)
+    Ms, Ns = ints(3 * C, 32), ints(C, 64)
+    nb = L.jf_wgrad_many_workspace_bytes(2, Ms, Ns, R)
+    ws = torch.empty(max(nb, 16), dtype=torch.int8, device="cuda")
+    operands = (ptrs([t for t, _ in gs]), ptrs([t for _, t in gs]), ptrs([t for t, _ in xs]), ptrs([t for _, t in xs]), ptrs(out), Ms, Ns, R,
+                jf.SCALE_F16 if f16 else jf.SCALE_F32, jf.FP_F32)
+    jf.check(L.jf_wgrad_many_dgrad(p(w), p(sw), p(q), p(s), 5, 16, 2, *operands, p(ws), nb, jf._stream()))
+    jf.check(L.jf_wgrad_many_finish(2, *operands, 1, ptrs([terms]), ints(C), ptrs([total]), p(ws), nb, jf._stream()))
+    assert torch.equal(q, wq) and torch.equal(s, ws_) and torch.equal(total, wsum)
+    assert all(torch.equal(a, b) for a, b in zip(out, want))
 
 
 @pytest.mark.parametrize("approx", [0, 1])
