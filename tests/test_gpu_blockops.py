@@ -470,3 +470,26 @@ def test_layernorm_from_partial_row_sums(jf, oracle, R, C, f16, with_beta):
     want = jf.layernorm_fwd(q, s, gamma, beta, mean, rstd) + (mean, rstd)
     for a, b in zip(jf.layernorm_fwd_sums(q, s, gamma, beta, rs, rq), want):
         assert torch.equal(a, b)
+
+
+def test_results_are_seen_by_a_dispatch_mode():
+    """Results are allocated without the dispatcher, except where something listens to it; the values do not depend on it."""
+    from Nonlinear import int8_quantize
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    seen = []
+
+    class Listener(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.name())
+            return func(*args, **(kwargs or {}))
+
+    x = torch.randn(64, 96, device="cuda")
+    q, s = int8_quantize(x, 32)
+    assert not q.requires_grad and q.is_contiguous() and q.device == x.device
+    with Listener():
+        q1, s1 = int8_quantize(x, 32)
+    assert sum(n.startswith("aten::empty") for n in seen) == 2
+    with torch.inference_mode():
+        q2, s2 = int8_quantize(x, 32)
+    assert q2.is_inference() and torch.equal(q, q1) and torch.equal(s, s1) and torch.equal(q, q2) and torch.equal(s, s2)

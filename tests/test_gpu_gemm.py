@@ -452,12 +452,18 @@ def test_quantised_with_residual_addition(jf, oracle, M, N, K, x1, y, f16, bias)
     gen = torch.Generator("cuda").manual_seed(M + K)
     res = torch.randn((M, N), device="cuda", generator=gen).to(x1)
     res[:32, :32] = 0
+    if M > 32:                                                    # blocks with a NaN, an infinity, both
+        res[32, 0] = res[33, 64] = float("nan")
+        res[34, 32] = res[35, 64] = float("inf")
     b = torch.randn(N, device="cuda", generator=gen) if bias else None
     bmax = b.abs().max().reshape(1) if bias else None
     for rounding in (jf.ROUND_TRUNC, jf.ROUND_NEAREST):
         got = jf.igemm_block_q_add(dA, dB, dsa, dsb, res, rounding, b, bmax, out_dtype=y)
         q0, s0 = jf.igemm_block_q(dA, dB, dsa, dsb, jf.B_NK, bias=b, biasmax=bmax)
         for g, w, name in zip(got, jf.add(res, q0, s0, rounding, with_stats=True, out_dtype=y), ("sum", "codes", "scales", "row sums", "row squares")):
+            if g.is_floating_point():
+                assert torch.equal(g.isnan(), w.isnan()), name
+                g, w = g.nan_to_num(7.0), w.nan_to_num(7.0)
             assert torch.equal(g, w), name
     assert got[1].any()
 
