@@ -16,7 +16,7 @@
 // fma(sa*sb, float(d), acc).  The only way the two differ is an overflow of sa*sb*2^26; that is detected
 // after the K loop and the wave then recomputes its blocks with the plain sequence (see there).
 //
-// Work decomposition: workgroup = 8 waves (2 x 4), tile 128x128, each wave owns 64x32 = 2 quantisation
+// Work decomposition (large launches; see launch_gemm_b): workgroup = 8 waves (2 x 4), tile 128x128, each wave owns 64x32 = 2 quantisation
 // blocks (32 fp32 accumulators per lane); two workgroups per CU.  K is consumed in stages of 4 blocks (128
 // bytes per row) through an LDS ring filled by LDS-direct loads (global_load_lds_dwordx4: no register
 // staging).  LDS rows are 128 bytes with an XOR chunk swizzle, so the 16-byte MFMA operand reads are
@@ -1569,8 +1569,7 @@ static bool small_tiles_resident(int M, int N, int K)          // two workgroups
 // 16 products per K block and SIMD pair in sequence, where a wave with one block is bound by the issue of its own 32 vector
 // instructions per product.  Measured (one-sequence forward GEMMs, us, 128x128 | 32x128): 32x768x768 9.7 | 5.7, 512x768x3072
 // 28.8 | 12.8, 512x3072x768 (384 small tiles) 10.7 | 8.4, 1248x768x768 10.7 | 6.5; beyond two per CU the larger tile's data
-// reuse wins: 1248x2304x768 (702) 10.9 | 12.6.  (A deeper ring changes nothing there; a 64x128 tile of 8 waves is 6 % better
-// between 256 and 512 small tiles and up to 19 % worse below.)
+// reuse wins: 1248x2304x768 (702) 10.9 | 12.6.  In between: launch_gemm_mixed, and 64x128 tiles (below).
 // A [K,N] B operand (and, for the weight gradient, a [K,M] A operand) is read in place.
 // a_km (A given as [K,M]) exists for the weight-gradient form only: fp output, B as [K,N].
 template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs &a, hipStream_t st)
