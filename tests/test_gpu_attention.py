@@ -54,6 +54,66 @@ def test_causal_attention(B, H, T, D, scale):
     assert torch.equal(qg, wq) and torch.equal(sg, ws)
 
 
+def half(x):
+    return x.to(torch.float16).to(x.dtype)
+
+
+def attention64(q, k, v, g, rounded):
+    """One head in float64: (out, dq, dk, dv).  rounded: with the roundings to binary16 that the kernels state, and no others: the
+    probabilities and score gradients that enter a second product, and the results (the forward's is what the backward reads).  The
+    forward's probabilities are relative to the maximum over a row's first 32 keys unless the row has one 2^8 times larger."""
+    r = half if rounded else (lambda x: x)
+    T, scale = q.shape[0], q.shape[1] ** -0.5
+    mask = ~torch.ones(T, T, dtype=torch.bool).tril()
+    s = ((q @ k.t()) * scale).masked_fill(mask, float("-inf"))
+    first, top = s[:, :32].amax(1, keepdim=True), s.amax(1, keepdim=True)
+    e = torch.exp(s - torch.where(top - first > 8 * 0.6931, top, first))
+    out = r((r(e) @ v) / e.sum(1, keepdim=True))
+    p = torch.softmax(s, 1)
+    ds = r(p * (g @ v.t() - (out * g).sum(1, keepdim=True)))
+    return out, r(ds @ k * scale), r(ds.t() @ q * scale), r(r(p).t() @ g)
+
+
+@pytest.mark.parametrize("B,H,T,D,scale,kind", [(1, 3, 1024, 64, 1.0, "plain"), (1, 3, 1024, 64, 6.0, "plain"), (1, 2, 512, 64, 20.0, "plain"),
+                                                (1, 3, 1024, 32, 1.0, "plain"), (1, 3, 512, 32, 0.1, "plain"), (1, 3, 1024, 64, 1.0, "rising"),
+                                                (1, 3, 1024, 32, 3.0, "rising"), (2, 4, 416, 64, 1.0, "channel"), (37, 7, 160, 64, 1.0, "plain"),
+                                                (37, 7, 160, 64, 3.0, "channel"), (70, 8, 96, 32, 3.0, "plain")])
+def test_attention_rounds_only_where_it_says(B, H, T, D, scale, kind):
+    """The error against float64 is that of float64 with the stated roundings.  Bound: a result's own rounding is in both; what else can
+    differ is whether a row's largest probability is exactly 1 (the kernel's maximum may be raised on the way, then it is not), which is
+    one more rounding of the same size, the square root of 2 in norm.  (Seen: 0.94 to 1.02, and 1.11 where keys rise.)  Binary32 leaves a
+    probability a relative error of 2^-23 times its exponent.  rising: keys that grow along the sequence, so that the running maximum is
+    raised again and again; channel: one channel in fifty twenty times larger, as activations have."""
+    import BlockQuantizeCUDA as BQC
+    jf, C = BQC.jetfire, H * D
+    gen = torch.Generator().manual_seed(B * 1000 + T + D)
+    x = torch.randn(B * T, 3 * C, generator=gen) * scale
+    if kind == "rising":
+        x[:, C: 2 * C] *= torch.linspace(0.2, 3.0, T).repeat(B).unsqueeze(1)
+    elif kind == "channel":
+        x[:, 7::50] *= 20
+    qkv, g = x.half(), (torch.randn(B * T, C, generator=gen) * 1e-2).half()
+    print(f"case B={B} H={H} T={T} D={D} scale={scale} {kind}", flush=True)
+    q, k, v = qkv.cuda().split(C, dim=1)
+    out, lse = jf.attention_fwd(q, k, v, B, H)
+    grads = jf.attention_bwd(q, k, v, out, lse, g.cuda(), B, H)
+    got = torch.cat([out, grads], 1).cpu().double().view(B, T, 4, H, D)
+    err, model, norm, exponent = torch.zeros(4, dtype=torch.float64), torch.zeros(4, dtype=torch.float64), torch.zeros(4, dtype=torch.float64), 0.0
+    for b in range(B):
+        for h in range(H):
+            a = [t.double().contiguous() for t in qkv.view(B, T, 3, H, D)[b, :, :, h].unbind(1)] + [g.view(B, T, H, D)[b, :, h].double()]
+            want, rounded = attention64(*a, False), attention64(*a, True)
+            exponent = max(exponent, float((a[0] @ a[1].t()).abs().max()) * D ** -0.5 * 1.4427)
+            for i in range(4):
+                err[i] += (got[b, :, i, h] - want[i]).square().sum()
+                model[i] += (rounded[i] - want[i]).square().sum()
+                norm[i] += want[i].square().sum()
+    err, model = (err / norm).sqrt(), (model / norm).sqrt()
+    print("  out dq dk dv", " ".join("%.2e" % e for e in err.tolist()), "| rounded", " ".join("%.2e" % e for e in model.tolist()),
+          "ratio", " ".join("%.3f" % e for e in (err / model).tolist()), "exponent %.0f" % exponent, flush=True)
+    assert (err <= 2.0 ** 0.5 * model + 2.0 ** -23 * exponent).all()
+
+
 def causal_rows(qkv, B, H, T, D):
     """Attention in float32 on the CPU, every query over its own keys only: what lies behind a query cannot reach it."""
     x = qkv.float().cpu().view(B, T, 3, H, D).permute(2, 0, 3, 1, 4)
