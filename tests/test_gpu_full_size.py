@@ -167,11 +167,15 @@ def test_cfg5_stress_cube(jf, oracle):
 # One odd-shaped launch per regime of the launcher's choice of wave priorities (by the number of 128 x 128 workgroups
 # against the 512 that are resident at once: up to one round; 1 to 1.5 rounds with short and with long tiles; 1.5 to 2;
 # more than 2), each with a number of tile rows that is not a multiple of the 8-row groups the tile order walks, a
-# workgroup count that is not a multiple of the 8 XCDs, and ragged last tiles in both directions.
+# workgroup count that is not a multiple of the 8 XCDs, and ragged last tiles in both directions.  The float outputs of all of them
+# come from 128x128 tiles; the requantised ones of 143 tiles from 64x128 tiles and of 609 from two tile sizes in one launch, so 667
+# are there for the requantising launches of 1 to 1.5 rounds.
 PACE_SHAPES = [
     (11 * 128 - 32, 13 * 128 - 64, 512),        # 143 workgroups
     (21 * 128 - 32, 29 * 128 - 96, 256),        # 609: 1.19 rounds, short tiles
     (21 * 128 - 32, 29 * 128 - 96, 4096),       # 609: long tiles
+    (23 * 128 - 32, 29 * 128 - 96, 256),        # 667: 1.30 rounds, short tiles
+    (23 * 128 - 32, 29 * 128 - 96, 4096),       # 667: long tiles
     (27 * 128 - 64, 33 * 128 - 32, 384),        # 891: 1.74 rounds
     (37 * 128 - 96, 31 * 128 - 64, 160),        # 1147: 2.24 rounds
 ]

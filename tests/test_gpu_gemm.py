@@ -614,7 +614,7 @@ def test_phase_recording_build_gives_the_same_bits_and_ordered_phases(jf):
         assert ((ph["k_loop_MHz"] > 300) & (ph["k_loop_MHz"] < 3500)).all()
 
 
-# 165 workgroups of 32x128 tiles; 153 of 128x128 (585 would be small ones).  K: rings of two and of three stages with one stage, fewer
+# 165 workgroups of 32x128 tiles; 297 of 64x128 for the requantised result, 153 of 128x128 for the float one (585 would be small ones).  K: rings of two and of three stages with one stage, fewer
 # than, as many as, more than their depth, every length of the last one; the longest row the small tiles take and the next one
 @pytest.mark.parametrize("M,N,K", [(m, n, k) for m, n in ((1056, 544), (2080, 1056)) for k in (32, 64, 96, 128, 160, 288, 384, 416, 896)]
                          + [(32, 160, 16384), (32, 160, 16416)])
@@ -639,9 +639,9 @@ def test_the_large_tiles_at_every_ring_fill(jf, oracle, K):
 
 
 # 128x128 and 32x128 tiles in one launch (256 CUs): behind one big tile per CU the fewest and the most small ones and one row block more
-# (128x128 only), columns that end inside a tile; behind two the fewest and the most; behind four
+# (64x128 only, 128x128 with the GELU forward), columns that end inside a tile; behind two the fewest and the most; behind four; behind six
 @pytest.mark.parametrize("M,N,K", [(5408, 768, 32), (6720, 768, 416), (6752, 768, 32), (4704, 800, 160), (10912, 768, 160), (13600, 768, 32),
-                                   (4352, 4096, 96)])
+                                   (4352, 4096, 96), (6176, 4096, 32)])
 def test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K):
     print(f"case M={M} N={N} K={K}", flush=True)
     A, Bkn, sa, sb = make_problem(M + N + K, M, N, K)
