@@ -17,11 +17,13 @@
 //
 // What bounds it.  Per 32x32 tile of scores, at D = 64, forward | dQ | dK/dV: 8 | 12 | 16 MFMAs of 32 cycles and 60 to 75 vector
 // instructions, 16 of them exponentials at a quarter of the rate; the two kinds share the issue of a SIMD: about 540 | 730 | 810 cycles.
-// Eight sequences of 1024 rows with 25 heads have 103 tiles per SIMD: 25 | 34 | 38 us of 44 | 55 | 74 (the tile loop without its loads
+// Eight sequences of 1024 rows with 25 heads have 103 tiles per SIMD: 25 | 34 | 38 us of 44 | 59 | 81 (the tile loop without its loads
 // takes 26 us of the forward's; loads and stores outside it, 118 MB, another 15).  Operands are read from LDS a step ahead of the
-// products, at immediate offsets, and tiles are loaded with scalar addresses: a step's instructions are the arithmetic.  us, before |
-// with that, forward and gradient: 8 x 1024 rows x 25 heads 52.8 | 44.5, 135.7 | 129.2; 2 x 1024 x 12 heads 21.6 | 17.5, 51.1 | 42.6;
-// 3 x 416 x 12 10.1 | 8.8, 27.3 | 23.3; 4 x 256 x 4 7.8 | 7.0, 21.1 | 18.3.
+// products, at immediate offsets (dQ: where it does not fill the chip, see there), and tiles are loaded with scalar addresses: a step's
+// instructions are the arithmetic.  us, before | with that, forward and gradient, each as it is launched at its size: 8 x 1024 rows x 25
+// heads 50.9 | 44.0, 144.3 | 139.6; 12 x 1024 x 12 36.9 | 33.0, 109.5 | 100.9; 2 x 1024 x 12 21.0 | 17.0, 51.7 | 42.8; 3 x 416 x 12 10.3 | 8.9,
+// 27.7 | 23.6; 4 x 256 x 4 7.8 | 7.0, 21.1 | 18.4.  Errors against float64 are the same before and with that, the gradients of keys
+// that rise along the sequence 2 % smaller.
 // The gradient is two kernels (dQ by query, dK/dV by key: 12 + 16 MFMAs per tile instead of 20) so that every sum has one owner and a
 // fixed order: no atomics, the same bits on every run.
 #include "jf_device.hpp"
@@ -354,8 +356,8 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_fwd_kernel(AttnArgs a)
 
 // dQ by blocks of queries; leaves delta for the dK/dV kernel.
 // EARLY: operands are read before they are needed and a tile's loads overlap the whole tile before it (140 registers, 3 waves per SIMD).
-// It is the faster kernel by itself at every size, us without | with: 2 sequences of 1024 rows x 12 heads 45.2 | 42.3 (with dK/dV), 8 x 25
-// heads 131.6 | 129.4.  But where it fills the chip, the chip then lowers its clock for everything around it (1.99 -> 1.91 GHz in the
+// It is the faster kernel by itself at every size, us without | with, both with dK/dV: 2 sequences of 1024 rows x 12 heads 45.2 | 42.3, 8 x
+// 25 heads 131.6 | 129.4 (on another box than the figures above).  But where it fills the chip, the chip then lowers its clock for everything around it (1.99 -> 1.91 GHz in the
 // GEMMs of a training step, read from their clock counters, for as long as the steps go on): three GPT-2 XL blocks 5809 | 5959 us a step,
 // three of GPT-2 small 2860 | 2900, three 1024 wide over 8 x 512 tokens 1641 | 1685; two blocks 768 wide over 2 x 1024 tokens 614 | 606.
 // So it is taken while no CU has more than one workgroup of it.

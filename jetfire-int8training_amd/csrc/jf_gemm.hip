@@ -1369,6 +1369,10 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 //   11008x2304x768 (1548) 50.6 | 45.9; 4224x1024x4096 (264) 52.1 | 43.0.
 // Beyond it: 13824x768x1536 (648 tiles) 38.8 | 39.0, 15360 (720) 39.4 | 42.5, 8192x768x3072 (384) 43.5 | 47.5, 24576x768x1536 (1152)
 // 61.7 | 61.8, 11264x3072x768 (2112) 63.0 | 62.3.
+// After three and after five the rule takes none, which is right for GPT-2 XL's 832 tiles only (640 rows behind three, 260 small tiles):
+// 8192x1600x1600 48.7 | 51.7, x4800 123.6 | 128.8, x6400 157.2 | 162.9.  With fewer behind them a mix would win there too: behind three
+// 16640x768x1536 (780) 46.3 | 41.1, 17408x768x1536 (816) 47.1 | 42.2, x3072 84.9 | 77.8; behind five 27648x768x1536 (1296) 73.5 | 64.5,
+// 12800x1600x6400 (1300) 265.2 | 254.6, 7040x3072x768 (1320) 42.5 | 37.8.
 static int mixed_big_rows(int M, int N, int K)
 {
     const int rows = (M + 127) / 128, tiles_n = (N + 127) / 128, cus = cu_count();
