@@ -357,7 +357,7 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_fwd_kernel(AttnArgs a)
 // dQ by blocks of queries; leaves delta for the dK/dV kernel.
 // EARLY: operands are read before they are needed and a tile's loads overlap the whole tile before it (140 registers, 3 waves per SIMD).
 // It is the faster kernel by itself at every size, us without | with, both with dK/dV: 2 sequences of 1024 rows x 12 heads 45.2 | 42.3, 8 x
-// 25 heads 131.6 | 129.4 (on another box than the figures above).  But where it fills the chip, the chip then lowers its clock for everything around it (1.99 -> 1.91 GHz in the
+// 25 heads 131.6 | 129.4 (on another card than the figures above).  But where it fills the chip, the chip then lowers its clock for everything around it (1.99 -> 1.91 GHz in the
 // GEMMs of a training step, read from their clock counters, for as long as the steps go on): three GPT-2 XL blocks 5809 | 5959 us a step,
 // three of GPT-2 small 2860 | 2900, three 1024 wide over 8 x 512 tokens 1641 | 1685; two blocks 768 wide over 2 x 1024 tokens 614 | 606.
 // So it is taken while no CU has more than one workgroup of it.
