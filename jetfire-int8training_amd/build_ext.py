@@ -22,7 +22,9 @@ CSRC = os.path.join(HERE, "csrc")
 HIP_LIB = os.path.join(HERE, "libjetfire_hip.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-HIP_SOURCES = ["jf_gemm.hip", "jf_blockops.hip", "jf_attention.hip"]
+JF_PARTS = 8                                                     # of jf_gemm.hip, see there
+HIP_SOURCES = [("jf_gemm.hip", ["-DJF_PART=%d" % k], "jf_gemm_%d.o" % k) for k in range(JF_PARTS)]
+HIP_SOURCES += [("jf_blockops.hip", [], "jf_blockops.o"), ("jf_attention.hip", [], "jf_attention.o")]
 PROF_LIB = os.path.join(HERE, "libjetfire_prof.so")
 PROF_SOURCES = [("jf_gemm.hip", ["-DJF_PROF_LIB"], "jf_gemm_prof.o"), ("jf_calib.hip", [], "jf_calib.o")]
 HIP_FLAGS = [
@@ -44,24 +46,20 @@ def _run(cmd):
 
 
 def build_hip():
-    """One hipcc process per source file, side by side (the GEMM file alone takes a minute), then one link."""
+    """One hipcc process per source file or part of one, side by side, then one link."""
     flags = [f for f in HIP_FLAGS if f != "-shared"]
     if os.environ.get("JF_PHILOX_ROUNDS"):                       # 7 (default) to 10 rounds of the rounding-noise generator
         flags.append("-DJF_PHILOX_ROUNDS=%d" % int(os.environ["JF_PHILOX_ROUNDS"]))
     hipcc = os.path.join(ROCM, "bin", "hipcc")
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
-    jobs, prof_jobs = [], []
-    for src in HIP_SOURCES:
-        obj = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
-        cmd = [hipcc] + flags + ["-c", os.path.join(CSRC, src), "-o", obj]
-        print("+", " ".join(cmd), flush=True)
-        jobs.append((cmd, obj, subprocess.Popen(cmd)))
-    for src, extra, name in PROF_SOURCES:
+    def start(src, extra, name):
         obj = os.path.join(objdir, name)
         cmd = [hipcc] + flags + extra + ["-c", os.path.join(CSRC, src), "-o", obj]
         print("+", " ".join(cmd), flush=True)
-        prof_jobs.append((cmd, obj, subprocess.Popen(cmd)))
+        return cmd, obj, subprocess.Popen(cmd)
+
+    jobs, prof_jobs = [start(*s) for s in HIP_SOURCES], [start(*s) for s in PROF_SOURCES]
     for cmd, obj, proc in jobs + prof_jobs:
         if proc.wait() != 0:
             raise subprocess.CalledProcessError(proc.returncode, cmd)

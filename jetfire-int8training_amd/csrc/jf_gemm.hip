@@ -32,6 +32,14 @@
 
 #pragma clang diagnostic ignored "-Winline-asm"     // M0 appears in clobber lists on purpose
 
+// The kernels are many instantiations of one function: a library is built from this file in JF_PARTS pieces, compiled side by side (each
+// with -DJF_PART=0 .. and its share of the explicit instantiations below; the entry points are in piece 0).  Without JF_PART: all of it.
+#ifdef JF_PART
+#define JF_IN_PART(n) (JF_PART == (n))
+#else
+#define JF_IN_PART(n) 1
+#endif
+
 namespace jf {
 
 constexpr int KB_STAGE = 4;                         // 32-deep K blocks per LDS stage (128 bytes of K per row)
@@ -124,11 +132,16 @@ constexpr int TABLE_KB = 512;                        // K blocks a wave's table 
 // LDS of a workgroup: the operand ring; per-wave scale and product patches or tables; from gelu_lds_at on what the GELU tables of the
 // epilogue need beyond those (WBM = 2: the forward's byte tables, 256 bytes per wave; WBM = 1: both, 1280 bytes).  Epilogues that go
 // through LDS use the ring.
+constexpr int SPLIT_GROUP = 8 * ROW_BYTES + 64;       // SPLIT: bytes from one 8-row group of a stage to the next
 constexpr int gelu_lds_at(int WBM, int WGM, int WGN, int NSTAGE)
 {
     const int scales = WBM == 1 ? 4 * (TABLE_KB + KB_STAGE) * WGM * WGN : NSTAGE * WGM * WGN * 512;
     return NSTAGE * (QB * WBM * WGM + QB * WBN * WGN) * ROW_BYTES + scales;
 }
+// SPLIT: tables of scale products, patches, ring (it also serves as the GELU's tables)
+constexpr int SPLIT_RING_AT = 2 * (4 * (TABLE_KB + KB_STAGE) + QB * EPI_LD * 4);
+constexpr int SPLIT_RING = 6;                        // stages: at 0.23 us each, five on their way cover the latency of the memory behind the L2s
+constexpr int SPLIT_LDS = SPLIT_RING_AT + SPLIT_RING * 12 * SPLIT_GROUP;
 constexpr int gemm_lds(int EPI, int WBM, int WGM, int WGN, int NSTAGE)
 {
     const int tables = (WBM == 1 ? (EPI == EPI_QG || EPI == EPI_QB) * 1280 : (EPI == EPI_QG) * 256) * WGM * WGN;
@@ -147,7 +160,8 @@ static int pace_of(long wgs, long slots, int k_per_wg);
 // library (jf_prof_igemm_block_q).
 // FOLD = 1: a workgroup may sum its K range in parts (p.fold_kb K blocks each, added in ascending order): the same additions as a K
 // split's, without a workgroup, an epilogue and a partial result in a common buffer for every part.
-template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM, int PROF, int FOLD = 0>
+// SPLIT = 2: two waves share a block, 16 rows each (split_loop, below).
+template <int EPI, typename ST, int WBM, int WGM, int WGN, int NSTAGE, int WGPC, int BKN, int AKM, int PROF, int FOLD = 0, int SPLIT = 1>
 __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logical)
 {
     GemmArgs p = p_in;                                        // K-split launches narrow it to the split's K range below
@@ -161,18 +175,22 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     }
     constexpr int NW = WGM * WGN;
     constexpr int BM = QB * WBM * WGM, BN = QB * WBN * WGN;
-    constexpr int A_BYTES = BM * ROW_BYTES;                  // one stage of A
-    constexpr int STAGE_BYTES = (BM + BN) * ROW_BYTES;
+    constexpr int GROUP_BYTES = SPLIT > 1 ? SPLIT_GROUP : 8 * ROW_BYTES;
+    constexpr int A_BYTES = BM / 8 * GROUP_BYTES;            // one stage of A
+    constexpr int STAGE_BYTES = (BM + BN) / 8 * GROUP_BYTES;
     constexpr int GROUPS = (BM + BN) / 8;                    // 8-row groups (1 KiB each) per stage
-    constexpr int LPW = GROUPS / NW;                         // LDS-direct loads per wave per stage
-    static_assert(GROUPS % NW == 0, "stage must split evenly over the waves");
+    constexpr int LW = SPLIT > 1 ? 4 : NW;                   // waves that load
+    constexpr int LPW = GROUPS / LW;                         // LDS-direct loads per wave per stage
+    static_assert(GROUPS % LW == 0, "stage must split evenly over the waves");
     static_assert(NSTAGE >= 2 && NSTAGE <= 5, "ring depth");
-    static_assert(!BKN || (BN == ROW_BYTES && WBN == 1), "a staged [K,N] row is one 128-byte LDS row");
+    static_assert(SPLIT == 1 || (SPLIT == 2 && WBM == 1 && WGM == 1 && WGN == 2), "32x64 tiles");
+    static_assert(SPLIT > 1 || !BKN || (BN == ROW_BYTES && WBN == 1), "a staged [K,N] row is one 128-byte LDS row");
     static_assert(WBM == 2 || !AKM, "one block per wave: A as [M,K] only");
     static_assert(!AKM || BM == ROW_BYTES, "a staged [K,M] row is one 128-byte LDS row");
     // The epilogues that requantise want a lane to hold 16 consecutive columns of a row.  They form the transposed product (B block
     // times A block, the same integers): its registers run along the columns, see the epilogue.
     constexpr bool QUANT = EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD || EPI == EPI_QA;
+    static_assert(SPLIT == 1 || QUANT, "the halves of a block meet as the transposed product");
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     typedef __attribute__((address_space(3))) unsigned char lds_u8;
@@ -180,8 +198,10 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool loader = WBM == 1 && wave_id >= NW;            // a wave that fetches for the others
-    const int wave = WBM == 1 ? wave_id % NW : wave_id;
+    const bool loader = WBM == 1 && wave_id >= NW * SPLIT;    // a wave that fetches for the others
+    unsigned char *const ring_lds = smem + (SPLIT > 1 ? SPLIT_RING_AT : 0);
+    const int load_wave = WBM == 1 ? wave_id % LW : wave_id;
+    const int wave = SPLIT > 1 ? wave_id / SPLIT % NW : load_wave, part = wave_id % SPLIT;     // (SPLIT: the wave's block and its part of it)
     const int wm = wave % WGM, wn = wave / WGM;
 
     int tile_m, tile_n, split;
@@ -212,7 +232,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     // The vector ALU is the bottleneck of this kernel, so the loads must not cost vector instructions.
     static_assert(NW % 2 == 0, "the chunk swizzle of a lane must not depend on the load index");
     const int lrow = lane >> 3;
-    const int gchunk = (lane & 7) ^ (((wave & 1) * 4 + (lane >> 4)) & 7);     // global chunk this lane fetches
+    // (SPLIT: chunk c of row r of a group at slot c ^ ((r>>1)&3), groups 64 bytes apart: also free of conflicts, and a K block's
+    // operands lie 64 bytes from those of the one two before)
+    const int gchunk = SPLIT > 1 ? (lane & 7) ^ ((lane >> 4) & 3) : (lane & 7) ^ (((load_wave & 1) * 4 + (lane >> 4)) & 7);     // global chunk this lane fetches
     // A as [K,M]: as for B as [K,N] below (8 K rows x 128 M bytes per load, slot c' of row r holds chunk c' ^ r)
     const int km_chunk = (m0 + (((lane & 7) ^ lrow) << 4)) < p.M ? ((lane & 7) ^ lrow) : 0;
     const unsigned loff_a = AKM ? (unsigned)lrow * (unsigned)p.lda + km_chunk * 16
@@ -221,16 +243,20 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     // of row r holds global chunk c' ^ r, which makes the transposing reads below conflict-free.  Chunks beyond N (partial
     // tile) fetch the tile's first chunk instead (never used).
     const int kn_chunk = (n0 + (((lane & 7) ^ lrow) << 4)) < p.N ? ((lane & 7) ^ lrow) : 0;
-    const unsigned loff_b = BKN ? (unsigned)lrow * (unsigned)p.ldb + kn_chunk * 16
+    // (SPLIT: rows of 64 bytes, 16 of them a group, chunk c of row r at slot c ^ ((r>>2)&3))
+    constexpr int KN_ROWS = SPLIT > 1 ? 16 : 8;
+    const int kn_row = SPLIT > 1 ? lane >> 2 : lrow;
+    const int kn_at = SPLIT > 1 ? (n0 + (((lane & 3) ^ (lane >> 4)) << 4) < p.N ? (lane & 3) ^ (lane >> 4) : 0) : kn_chunk;
+    const unsigned loff_b = BKN ? (unsigned)kn_row * (unsigned)p.ldb + kn_at * 16
                                 : (unsigned)lrow * (unsigned)p.ldb + gchunk * 16;
     const int8_t *gbase[LPW];      // wave-uniform: first byte of the group's first row in the stage issued next
     bool is_a[LPW];
 #pragma unroll
     for (int j = 0; j < LPW; ++j) {
-        const int grp = wave + j * NW;
+        const int grp = load_wave + j * LW;
         is_a[j] = grp < BM / 8;
         if (BKN && !is_a[j]) {
-            const int k0 = (grp - BM / 8) * 8;                     // K row of the stage (redirected at issue time if beyond K)
+            const int k0 = (grp - BM / 8) * KN_ROWS;                     // K row of the stage (redirected at issue time if beyond K)
             gbase[j] = p.B + (size_t)k0 * (size_t)p.ldb + n0;
         } else if (AKM && is_a[j]) {
             gbase[j] = p.A + (size_t)(grp * 8) * (size_t)p.lda + m0;
@@ -251,7 +277,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     constexpr int NBLK = WBM * WBN;
     static_assert(NBLK == 2 || NBLK == 1, "one or two products per K block and wave");
     constexpr int SC_SLOT = 256;                              // a ring slot of a wave's fetched scales; its products follow all of them
-    static_assert(NSTAGE <= 3, "8-bit word offsets of the paired scale read");
+    static_assert(WBM == 1 || NSTAGE <= 3, "8-bit word offsets of the paired scale read");
     unsigned char *const scale_patch = smem + NSTAGE * STAGE_BYTES + wave * (2 * NSTAGE * SC_SLOT);
     const int s_prod = lane % (KB_STAGE * NBLK), s_blk = s_prod % NBLK, s_kb = s_prod / NBLK;
     const bool s_is_b = lane >= 32;
@@ -269,11 +295,11 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     // WBM = 1: all of a block's products at once, before the main loop, into a table of the wave: lane l those of the K blocks l,
     // l + 64, ...
     constexpr bool TABLE = WBM == 1;
-    float *const table = reinterpret_cast<float *>(smem + NSTAGE * STAGE_BYTES) + wave * ((nkb + KB_STAGE - 1) / KB_STAGE * KB_STAGE + KB_STAGE);
+    float *const table = reinterpret_cast<float *>(smem + (SPLIT > 1 ? 0 : NSTAGE * STAGE_BYTES)) + wave * ((nkb + KB_STAGE - 1) / KB_STAGE * KB_STAGE + KB_STAGE);
     auto make_table = [&] {
         const int mi = m0 / QB + wm < SM ? m0 / QB + wm : SM - 1, ni = n0 / QB + wn < SN ? n0 / QB + wn : SN - 1;
         const ST *ta = reinterpret_cast<const ST *>(p.sa) + (size_t)mi * p.sa_is, *tb = reinterpret_cast<const ST *>(p.sb) + (size_t)ni * p.sb_is;
-        for (int k = lane; k < nkb; k += WAVE) table[k] = ((float)ta[(size_t)k * p.sa_ks] * (float)tb[(size_t)k * p.sb_ks]) * 67108864.0f;
+        for (int k = lane + WAVE * part; k < nkb; k += WAVE * SPLIT) table[k] = (SPLIT > 1 ? -1.0f : 1.0f) * ((float)ta[(size_t)k * p.sa_ks] * (float)tb[(size_t)k * p.sb_ks]) * 67108864.0f;
     };
     // the scales of the next stage (one after the other) into ring slot `slot`; K blocks beyond the last: the last one again
     auto issue_scales = [&](auto slot_c) {
@@ -310,12 +336,12 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         asm volatile("ds_write_b32 %0, %1 offset:%2" ::"v"(dst), "v"(t), "n"(decltype(slot_c)::value * SC_SLOT) : "memory");
     };
 
-    constexpr int A_LOADS = (BM / 8) / NW;                    // loads 0 .. A_LOADS-1 of a wave fetch A rows, the rest B rows
-    static_assert((BM / 8) % NW == 0, "a load instruction fetches rows of one operand");
+    constexpr int A_LOADS = (BM / 8) / LW;                    // loads 0 .. A_LOADS-1 of a wave fetch A rows, the rest B rows
+    static_assert((BM / 8) % LW == 0, "a load instruction fetches rows of one operand");
     // FULL: the stage has all KB_STAGE K blocks (every stage but a short last one)
     auto issue_stage_as = [&](int stage, unsigned slot, auto full_c) {       // slot: stage % NSTAGE
         constexpr bool FULL = decltype(full_c)::value;
-        const unsigned slot_lds = (unsigned)(uintptr_t)(lds_u8 *)smem + slot * STAGE_BYTES;
+        const unsigned slot_lds = (unsigned)(uintptr_t)(lds_u8 *)ring_lds + slot * STAGE_BYTES;
         const int kb0 = stage * KB_STAGE;
         // asm: scalar base + 32-bit lane offset is the addressing mode that costs no vector instruction, and the
         // compiler does not choose it by itself here.  M0 holds the LDS destination of an LDS-direct load.
@@ -326,13 +352,13 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         }
 #pragma unroll
         for (int j = 0; j < LPW; ++j) {
-            const int grp = wave + j * NW;
+            const int grp = load_wave + j * LW;
             const int8_t *base;                                // wave-uniform
             if (BKN && j >= A_LOADS) {
                 base = gbase[j];
                 gbase[j] += (size_t)(KB_STAGE * QB) * (size_t)p.ldb;
                 // K rows of a missing K block: the stage's first group again
-                if (!FULL && kb0 * QB + (grp - BM / 8) * 8 >= p.K) base -= (size_t)((grp - BM / 8) * 8) * (size_t)p.ldb;
+                if (!FULL && kb0 * QB + (grp - BM / 8) * KN_ROWS >= p.K) base -= (size_t)((grp - BM / 8) * KN_ROWS) * (size_t)p.ldb;
             } else if (AKM && j < A_LOADS) {
                 base = gbase[j];
                 gbase[j] += (size_t)(KB_STAGE * QB) * (size_t)p.lda;
@@ -342,7 +368,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                 gbase[j] += KB_STAGE * QB;
             }
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         ::"v"(j < A_LOADS ? la : lb), "s"(base), "s"(slot_lds + (unsigned)grp * 1024u) : "memory", "m0");
+                         ::"v"(j < A_LOADS ? la : lb), "s"(base), "s"(slot_lds + (unsigned)grp * (unsigned)GROUP_BYTES) : "memory", "m0");
         }
     };
     auto issue_stage = [&](int stage, unsigned slot) {        // stage < nstages, one after the other
@@ -428,7 +454,12 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     const int nfull = nkb / KB_STAGE;                         // stages with all KB_STAGE blocks
     const int ktail = nkb - nfull * KB_STAGE;                 // K blocks of the short last stage (0: none)
     issue_scales(std::integral_constant<int, 0>{});
-    static_for<0, NSTAGE>([&](auto slot_c) {
+    if constexpr (SPLIT > 1) {
+        if (loader) {
+#pragma unroll 1
+            for (int s = 0; s < SPLIT_RING && s < nstages; ++s) issue_stage(s, (unsigned)s);
+        }
+    } else static_for<0, NSTAGE>([&](auto slot_c) {
         constexpr int SLOT = decltype(slot_c)::value;
         if (SLOT < nstages && (!TABLE || loader)) {
             issue_stage(SLOT, (unsigned)SLOT);
@@ -616,10 +647,14 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         if (Y == 0 || last >= nstages) JF_WAIT_VMCNT(0);
         else JF_WAIT_VMCNT(Y * LOADS);
     };
+    auto wait_behind = [&](const int n) {                      // the loads of n stages may be outstanding (SPLIT)
+        static_for<0, SPLIT_RING>([&](auto n_c) { if (n == decltype(n_c)::value) JF_WAIT_VMCNT(decltype(n_c)::value * LPW); });
+    };
     using c0 = std::integral_constant<int, 0>;
     if constexpr (TABLE) {
-        if (loader) wait_stage(NSTAGE - 1, std::integral_constant<int, NSTAGE - 1>{});    // stage 0 has landed
-        else make_table();
+        if (!loader) make_table();
+        else if (SPLIT > 1) wait_behind(SPLIT_RING < nstages ? SPLIT_RING - 1 : nstages - 1);
+        else wait_stage(NSTAGE - 1, std::integral_constant<int, NSTAGE - 1>{});           // stage 0 has landed
         if constexpr (EPI == EPI_QA) { if (!loader && m0 + wm * QB < p.M && n0 + wn * QB < p.N) fetch_x1(); }
     } else {
         if (NSTAGE - 1 >= nstages) JF_WAIT_VMCNT(0);
@@ -639,6 +674,8 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     // which of the CU's two workgroup slots this is: the base of its LDS allocation (the low field of the LDS_ALLOC
     // register; its size field starts at bit 12)
     const bool second_slot = (__builtin_amdgcn_s_getreg((31 << 11) | 6) & 0xFFF) != 0;
+    // (not QUANT, EPI_QA or SPLIT)
+    float *const patch = reinterpret_cast<float *>(smem + (SPLIT > 1 ? NW * 4 * (TABLE_KB + KB_STAGE) : 0)) + wave * (QB * EPI_LD);
     long long prof_c0 = 0;
     if (PROF) { phase(1, (unsigned long long)wall_clock64()); prof_c0 = clock64(); }
     auto main_loop = [&](auto active_c, auto pace_c) {
@@ -768,7 +805,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         // K blocks 2 pair, 2 pair + 1 of a stage into register set `pair`; extra: run-time offsets of operands and products
         auto fetch_pair = [&](auto pair_c, auto slot_c, unsigned extra, unsigned extra_tab) {
             constexpr int PAIR = decltype(pair_c)::value, SLOT = decltype(slot_c)::value, SB = SLOT * STAGE_BYTES;
-            static_assert(NSTAGE * STAGE_BYTES <= 65536, "offsets of 16 bits");
+            static_assert(SPLIT > 1 || NSTAGE * STAGE_BYTES <= 65536, "offsets of 16 bits");
             v2f &t = pr[PAIR];
             const unsigned pt = tab + extra_tab;
             asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(t) : "v"(pt), "n"(SLOT * KB_STAGE * 4 + 8 * PAIR));
@@ -835,7 +872,179 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
             if (left > 3) compute_block(fa2[1][1], fb2[1][1], pr[1][1]);
         }
     };
-    if constexpr (TABLE) { if (loader) load_loop(); else table_loop(); }
+    auto split_loads = [&] {
+        int s = 0;
+        auto hand_over = [&](auto behind_c) {                  // stage s + 1 has landed: at most the loads of so many stages are outstanding
+            JF_WAIT_VMCNT(decltype(behind_c)::value * LPW);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        int slot = 0;
+#pragma unroll 1
+        for (; s + SPLIT_RING < nstages; ++s) {
+            hand_over(std::integral_constant<int, SPLIT_RING - 2>{});
+            issue_stage(s + SPLIT_RING, (unsigned)slot);
+            slot = slot + 1 == SPLIT_RING ? 0 : slot + 1;
+        }
+        const int left = nstages - 2 - s;                      // stages behind stage s + 1
+        static_for<0, SPLIT_RING - 1>([&](auto n_c) {
+            constexpr int BEHIND = SPLIT_RING - 2 - decltype(n_c)::value;
+            if (BEHIND <= left) hand_over(std::integral_constant<int, BEHIND>{});
+        });
+    };
+    // SPLIT.  With fewer blocks than SIMDs the vector ALU idles for half of table_loop: a wave alone on its SIMD issues every 4.1 cycles,
+    // and 32 vector instructions per K block in one chain are what the launch waits for.  Two or four waves share a block: each forms the
+    // products of 16 rows and STRIPS x 16 columns (v_mfma_i32_16x16x32_i8: the same integers) and accumulates them in the same chain over
+    // K, 16 or 8 vector instructions per K block.  One turn per stage, and nothing unrolled beyond two of them: code that is executed once
+    // costs an instruction fetch per 64 bytes.
+    constexpr int STRIPS = 2;
+    auto split_loop = [&] {
+        if (!wave_active) {
+            for (int s = 0; s + 1 < nstages; ++s) __builtin_amdgcn_s_barrier();
+            return;
+        }
+        // operand addresses of the current slot.  Lane l holds row (column) l%16 of its strip and K bytes 8*(l/16) .. +7 of a K block:
+        // qa[i], qb[i] for K blocks i, i + 2 (a second strip: an offset); as [K,N] qb[strip] (a group of 16 lanes reads 8 K rows of
+        // 16 columns, as for fb_kn)
+        unsigned qa[2], qb[2], tab;
+        {
+            const int g = lane >> 4, r = lane & 15;
+            const unsigned base = (unsigned)(uintptr_t)(lds_u8 *)ring_lds, row = (r >> 3) * GROUP_BYTES + (r & 7) * ROW_BYTES + 8 * (g & 1);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const unsigned slot = ((2 * i + (g >> 1)) ^ ((r >> 1) & 3)) << 4;
+                qa[i] = base + part * 2 * GROUP_BYTES + row + slot;
+                qb[i] = base + A_BYTES + wn * 4 * GROUP_BYTES + row + slot;
+                if (BKN) {
+                    const int k = 8 * g + (r >> 1);
+                    qb[i] = base + A_BYTES + (k >> 4) * GROUP_BYTES + (k & 15) * 64 + (((2 * wn + i) ^ ((k >> 2) & 3)) << 4) + 8 * (r & 1);
+                }
+            }
+            const unsigned u = (unsigned)(uintptr_t)(lds_u8 *)reinterpret_cast<unsigned char *>(table);
+            asm volatile("v_mov_b32 %0, %1" : "=v"(tab) : "s"(u));
+        }
+        // operands and products of a whole stage per register set: they are read while the stage before is multiplied
+        typedef float v4f_t __attribute__((ext_vector_type(4)));
+        v2i fa[2][KB_STAGE], fb[2][KB_STAGE][STRIPS];
+        v4f_t pr[2];
+        constexpr int READS = 1 + KB_STAGE * (1 + STRIPS);     // LDS reads of a stage
+        auto fetch_one = [&](auto set_c, auto n_c) {           // the n-th of them, of the current slot
+            constexpr int SET = decltype(set_c)::value, N = decltype(n_c)::value, kb = (N - 1) / (1 + STRIPS), J = (N - 1) % (1 + STRIPS) - 1;
+            if constexpr (N == 0) {
+                v4f_t &t = pr[SET];
+                const unsigned pt = tab;
+                asm volatile("ds_read_b128 %0, %1" : "=v"(t) : "v"(pt));
+            } else if constexpr (J < 0) {
+                v2i &a = fa[SET][kb];
+                const unsigned pa = qa[kb & 1];
+                asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(a) : "v"(pa), "n"(64 * (kb >> 1)));
+            } else {
+                v2i &b = fb[SET][kb][J];
+                const unsigned pb = BKN ? qb[J] : qb[kb & 1];
+                if (BKN) asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(b) : "v"(pb), "n"(kb * 2 * GROUP_BYTES));
+                else asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(b) : "v"(pb), "n"(64 * (kb >> 1) + J * 2 * GROUP_BYTES));
+            }
+        };
+        auto arrived = [&](auto set_c) {
+            constexpr int SET = decltype(set_c)::value;
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+            v4f_t &t = pr[SET];
+            asm volatile("" : "+v"(t));
+            static_for<0, KB_STAGE>([&](auto kb_c) {
+                v2i &a = fa[SET][decltype(kb_c)::value];
+                asm volatile("" : "+v"(a));
+                static_for<0, STRIPS>([&](auto j_c) {
+                    v2i &b = fb[SET][decltype(kb_c)::value][decltype(j_c)::value];
+                    asm volatile("" : "+v"(b));
+                });
+            });
+        };
+        // The products lead the accumulation by one K block.  0.15915494 - (0x3e22f983 + d) = -d * 2^-26, exactly, against a negated
+        // factor: the product of accumulate() (this way round the constant is an inline one for the compiler too).
+        constexpr int ONE = 0x3e22f983;
+        const v4i one = {ONE, ONE, ONE, ONE};
+        v4i lag[STRIPS];
+        float lag_s = 0.0f, t[4 * STRIPS];
+#pragma unroll
+        for (int j = 0; j < STRIPS; ++j) lag[j] = one;
+        auto unbias = [&](auto j_c) {
+            constexpr int J = decltype(j_c)::value;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) t[4 * J + v] = __int_as_float(ONE) - __int_as_float(lag[J][v]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto add = [&](auto j_c) {
+            constexpr int J = decltype(j_c)::value;
+#pragma unroll
+            for (int v = 4 * J; v < 4 * J + 4; ++v) acc[0][0][v] = __builtin_fmaf(lag_s, t[v], acc[0][0][v]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // One K block.  AHEAD: with the first two K blocks of a stage go the reads of the next stage, which then have the time of the other
+        // two to arrive.  (Spread evenly, one for every four vector instructions, 20 cycles more per K block: an LDS read takes 12 to 16
+        // cycles of a wave that is alone on its SIMD, wherever it stands.)
+        auto product = [&](auto set_c, auto kb_c, auto ahead_c) {
+            constexpr int SET = decltype(set_c)::value, kb = decltype(kb_c)::value;
+            static_for<0, STRIPS>([&](auto j_c) {              // (four vector instructions fill the 16 cycles of each)
+                constexpr int J = decltype(j_c)::value;
+                const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, fb[SET][kb][J]), __builtin_bit_cast(long, fa[SET][kb]), one, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (decltype(ahead_c)::value && kb < 2 && J == 0) {
+                    constexpr int HALF = (READS + 1) / 2;
+                    static_for<kb * HALF, (kb == 0 ? HALF : READS)>([&](auto n_c) { fetch_one(std::integral_constant<int, SET ^ 1>{}, n_c); });
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                unbias(j_c);
+                lag[J] = d;
+            });
+            static_for<0, STRIPS>(add);
+            lag_s = pr[SET][kb];
+        };
+        int slot = 0;
+        auto stage = [&](auto set_c) {                         // a stage that is not the last one (and therefore whole)
+            constexpr int SET = decltype(set_c)::value;
+            arrived(set_c);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            slot = slot + 1 == SPLIT_RING ? 0 : slot + 1;
+            const unsigned step = slot == 0 ? (unsigned)-((SPLIT_RING - 1) * STAGE_BYTES) : (unsigned)STAGE_BYTES;
+            qa[0] += step; qa[1] += step; qb[0] += step; qb[1] += step; tab += KB_STAGE * 4;
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<0, KB_STAGE>([&](auto kb_c) { product(set_c, kb_c, std::true_type{}); });
+        };
+        const std::integral_constant<int, 0> set0;
+        const std::integral_constant<int, 1> set1;
+        int n = nstages - 1;                                   // the last stage is in set 0
+        if (n & 1) static_for<0, READS>([&](auto n_c) { fetch_one(set1, n_c); });
+        else static_for<0, READS>([&](auto n_c) { fetch_one(set0, n_c); });
+#pragma unroll 1
+        while (n > 0) {
+            if (!(n & 1)) { stage(set0); --n; }
+            stage(set1);
+            --n;
+        }
+        const int left = nkb - (nstages - 1) * KB_STAGE;
+        arrived(set0);
+        static_for<0, KB_STAGE>([&](auto kb_c) { if (decltype(kb_c)::value < left) product(set0, kb_c, std::false_type{}); });
+        static_for<0, STRIPS>(unbias);
+        static_for<0, STRIPS>(add);
+        // [row][column] of the block
+        float *const at = patch + (part * 16 + (lane & 15)) * EPI_LD + 4 * (lane >> 4);
+#pragma unroll
+        for (int j = 0; j < STRIPS; ++j)
+            *reinterpret_cast<v4f *>(at + 16 * j) = v4f{acc[0][0][4 * j], acc[0][0][4 * j + 1], acc[0][0][4 * j + 2], acc[0][0][4 * j + 3]};
+    };
+    if constexpr (SPLIT > 1) {
+        if (loader) split_loads();
+        else split_loop();
+        __syncthreads();                                       // the halves meet in the patch; the first wave of a block goes on with it
+        if (loader || part > 0 || !wave_active) return;
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+            acc[0][0][v] = patch[(lane & 31) * EPI_LD + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)];
+    }
+    else if constexpr (TABLE) { if (loader) load_loop(); else table_loop(); }
     else if (!wave_active) main_loop(std::false_type{}, std::integral_constant<int, PACE_HARDWARE>{});
     else if (WBM == 2 && p.pace == PACE_EVEN) main_loop(std::true_type{}, std::integral_constant<int, PACE_EVEN>{});
     else if (WBM == 2 && p.pace == PACE_ORDERED) main_loop(std::true_type{}, std::integral_constant<int, PACE_ORDERED>{});
@@ -844,7 +1053,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     float lane_max[WBM][WBN];                                  // largest magnitude of this lane's results, per block   (QUANT)
     bool nonfinite = false;                                    // wave-uniform: some result is infinite or NaN   (QUANT)
     if (EPI != EPI_S32 && wave_active && !loader) {
-        accumulate(std::integral_constant<int, NBLK - 1>{});
+        if constexpr (SPLIT == 1) accumulate(std::integral_constant<int, NBLK - 1>{});
         if constexpr (FOLD) { if (folds > 0) add_parts(); }
         // The scaled factor sa*sb*2^26 overflows when sa*sb >= 2^102.  An infinite factor leaves every accumulator
         // it touches infinite or NaN (inf*0 included), so "some accumulator of the wave is not finite" catches all such
@@ -938,7 +1147,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     }
     if (PROF) { phase(2, (unsigned long long)wall_clock64()); phase(7, (unsigned long long)(clock64() - prof_c0)); }
     if (p.pace != PACE_HARDWARE) __builtin_amdgcn_s_setprio(0);
-    if constexpr (!QUANT || EPI == EPI_QA) __syncthreads();    // the epilogue reuses the ring as scratch
+    if constexpr (SPLIT == 1 && (!QUANT || EPI == EPI_QA)) __syncthreads();    // the epilogue reuses the ring as scratch
     if (loader) return;
     if (PROF) phase(3, (unsigned long long)wall_clock64());
 
@@ -961,10 +1170,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    float *patch = reinterpret_cast<float *>(smem) + wave * (QB * EPI_LD);     // (not QUANT, or EPI_QA)
     const int rrow = QUANT ? lane & 31 : lane >> 1, rcol = (QUANT ? lane >> 5 : lane & 1) * 16;
     // GELU tables of the wave: its scale patch (nothing is on its way there any more) and, for the byte table, a piece of its own
-    float *const gelu_tab = TABLE ? reinterpret_cast<float *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 320 : reinterpret_cast<float *>(scale_patch);
+    float *const gelu_tab = SPLIT > 1 ? reinterpret_cast<float *>(ring_lds) + wave * 320 : TABLE ? reinterpret_cast<float *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 320 : reinterpret_cast<float *>(scale_patch);
     int *const gelu_qtab = TABLE ? reinterpret_cast<int *>(gelu_tab + 256) : reinterpret_cast<int *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 64;
     if (EPI == EPI_QG || EPI == EPI_QB) JF_WAIT_VMCNT(0);
     const float biasmax = (QUANT && p.biasmax) ? p.biasmax[0] : 0.0f;
@@ -1199,6 +1407,13 @@ __global__ __launch_bounds__(gemm_threads(WBM, WGM, WGN), WGPC * gemm_threads(WB
     igemm_body<EPI, ST, WBM, WGM, WGN, NSTAGE, WGPC, BKN, AKM, PROF>(p, logical_workgroup(gridDim.x, blockIdx.x, true));
 }
 
+// 32x64 tiles, two waves per block.
+template <int EPI, typename ST, int BKN> __global__ __launch_bounds__(512, 4) void igemm_split_kernel(GemmArgs p)
+{
+    p.m_base = 0;
+    igemm_body<EPI, ST, 1, 1, 2, 2, 2, BKN, 0, 0, 0, 2>(p, logical_workgroup(gridDim.x, blockIdx.x, true));
+}
+
 // Rows 0 .. m_base - 1 in 128x128 tiles, the others in 32x128 tiles (launch_gemm_mixed).
 template <int EPI, typename ST, int BKN> __global__ __launch_bounds__(512, 4) void igemm_mixed_kernel(GemmArgs p)
 {
@@ -1242,22 +1457,24 @@ template <typename ST> __global__ __launch_bounds__(512, 4) void igemm_wgrad_gro
 
 // An activation gradient (EPI_Q or EPI_QD, B as [K,N]; 32x128 or 128x128 tiles), then weight gradients, in one launch: both gradients of
 // a linear layer, or the last one of a block with all of the block's weight gradients.
+enum BackwardTile { TILE_128x128, TILE_32x128, TILE_32x64 };   // of the activation gradient
 struct GemmBackward {
     GemmArgs x;
     GemmGroup w;
 };
-template <int EPI, typename ST, bool SMALL> __global__ __launch_bounds__(512, 4) void igemm_backward_kernel(GemmBackward b)
+template <int EPI, typename ST, int TILE> __global__ __launch_bounds__(512, 4) void igemm_backward_kernel(GemmBackward b)
 {
     const int work_x = b.x.tiles_m * b.x.tiles_n, first_w = (work_x + 7) & ~7;      // (both parts are dealt to the XCDs from the first one on)
     const int wg = blockIdx.x;
     if (wg < first_w) {
         const int logical = logical_workgroup(work_x, wg);
-        if (logical >= 0) igemm_body<EPI, ST, SMALL ? 1 : 2, SMALL ? 1 : 2, 4, SMALL ? 3 : 2, 2, 1, 0, 0>(b.x, logical);
+        if (logical >= 0) igemm_body<EPI, ST, TILE == TILE_128x128 ? 2 : 1, TILE == TILE_128x128 ? 2 : 1, TILE == TILE_32x64 ? 2 : 4, TILE == TILE_32x128 ? 3 : 2, 2, 1, 0, 0, 0, TILE == TILE_32x64 ? 2 : 1>(b.x, logical);
     } else {
         wgrad_group_body<ST>(b.w, wg - first_w);
     }
 }
 
+#if JF_IN_PART(0)
 // -------------------------------------------------------------------------------------------------
 // int8 transpose: out[C,R] = in[R,C].  TR_ROWS x 64 tiles through LDS: 16-byte loads, the transposing LDS read of gfx950
 // (ds_read_b64_tr_b8, as for the GEMM's [K,N] operands) and 16-byte stores.  The instruction works on groups of 16 lanes:
@@ -1312,6 +1529,7 @@ static int launch_transpose(const int8_t *in, int R, int C, int8_t *out, hipStre
     hipLaunchKernelGGL(transpose_s8_kernel, dim3(tiles), dim3(256), 0, st, in, out, R, C);
     return (int)hipGetLastError();
 }
+#endif
 
 // more than 64 KiB of dynamic LDS has to be opted into, per function and device: once, not on every launch
 // (the reference sets its attribute on every call, igemm_BlockSquare32OutputIntQuantizeBiasRowCol.cu:418)
@@ -1403,7 +1621,21 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_mixed(const Gemm
     return (int)hipGetLastError();
 }
 
-template <typename ST> static int launch_wgrad_group(const GemmGroup &grp, unsigned wgs, hipStream_t st)
+template <int EPI, typename ST, int BKN> static int launch_gemm_split(const GemmArgs &a, hipStream_t st)
+{
+    if (!device_is_gfx950()) return JF_ERR_DEVICE;
+    GemmArgs p = a;
+    p.splits = 1;
+    p.tiles_m = p.M / QB;
+    p.tiles_n = (p.N + 63) / 64;
+    p.pace = PACE_HARDWARE;
+    static std::atomic<bool> opted_in[MAX_DEVICES] = {};
+    if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_split_kernel<EPI, ST, BKN>), SPLIT_LDS, opted_in)) return rc;
+    hipLaunchKernelGGL((igemm_split_kernel<EPI, ST, BKN>), dim3(p.tiles_m * p.tiles_n), dim3(512), SPLIT_LDS, st, p);
+    return (int)hipGetLastError();
+}
+
+template <typename ST> int launch_wgrad_group(const GemmGroup &grp, unsigned wgs, hipStream_t st)
 {
     constexpr int SMEM = gemm_lds(EPI_FP, 2, 2, 4, 2);
     static std::atomic<bool> opted_in[MAX_DEVICES] = {};
@@ -1412,6 +1644,7 @@ template <typename ST> static int launch_wgrad_group(const GemmGroup &grp, unsig
     return (int)hipGetLastError();
 }
 
+#if JF_IN_PART(0)
 // out[i] = convert(part[0][i] + part[1][i] + ... + part[S-1][i]), added in ascending split order, for the four elements at i.
 __device__ __forceinline__ void reduce_splits(const float *part, size_t n, int splits, void *out, int out_dtype, size_t i)
 {
@@ -1492,6 +1725,8 @@ __global__ __launch_bounds__(1024) void wgrad_finish_kernel(WgradFinish f)
     }
 }
 
+#endif
+
 // K split of the fp-output GEMM.  request 1: none; request > 1: that many parts (fewer if K is short); request 0: as
 // many parts as it takes to give every CU two workgroups, when the tiles alone fill less than half of them.  Parts are
 // whole multiples of 4 K blocks (one LDS stage), at least 16 K blocks long.
@@ -1562,7 +1797,12 @@ static void wgrad_group_plan(int n, const int *M, const int *N, int K, WgradPlan
     }
 }
 
-static bool small_tiles_resident(int M, int N, int K)          // two workgroups per CU
+// 32x64 tiles, two waves per block: where one per CU holds them all.  us, 32x128 tiles | these: 32x768x768 5.7 | 5.3, 64x256x256 4.1 | 3.9,
+// 512x768x768 (192 of them) 5.8 | 5.5, 512x768x2304 10.3 | 8.7, 416x1120x2080 (234) 9.5 | 8.3, 160x544x4096 15.4 | 12.0; B as [K,N] 512x768x768
+// 6.1 | 6.1, x2304 10.8 | 9.5; with two per CU 1248x768x768 (468) 5.8 | 6.5, 1024x1024x1024 (512) 6.6 | 7.4, 1280x768x2304 (480) 10.4 | 11.2.
+static long split_tiles(int M, int N) { return (long)(M / QB) * ((N + 63) / 64); }
+static bool split_tiles_resident(int M, int N, int K) { return K <= TABLE_KB * QB && split_tiles(M, N) <= (long)cu_count(); }
+static bool small_tiles_resident(int M, int N, int K)          // 32x128 tiles, two workgroups per CU
 {
     return K <= TABLE_KB * QB && (long)((M + 31) / 32) * ((N + 127) / 128) <= 2L * cu_count();
 }
@@ -1579,6 +1819,7 @@ static bool small_tiles_resident(int M, int N, int K)          // two workgroups
 template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs &a, hipStream_t st)
 {
     if constexpr (EPI != EPI_S32) {
+        if constexpr (EPI != EPI_FP) { if (split_tiles_resident(a.M, a.N, a.K)) return launch_gemm_split<EPI, ST, BKN>(a, st); }
         if (a.splits <= 1 && small_tiles_resident(a.M, a.N, a.K))
             return launch_gemm_cfg<EPI, ST, 1, 1, 4, 3, 2, BKN>(a, st);
     }
@@ -1598,7 +1839,7 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs
     }
     return launch_gemm_cfg<EPI, ST, 2, 2, 4, 2, 2, BKN>(a, st);
 }
-template <int EPI, typename ST> static int launch_gemm(const GemmArgs &a, hipStream_t st, bool b_kn, bool a_km = false)
+template <int EPI, typename ST> int launch_gemm(const GemmArgs &a, hipStream_t st, bool b_kn, bool a_km = false)
 {
     if constexpr (EPI == EPI_QG) {                            // the forward form only: A [M,K], B [N,K]
         if (a_km || b_kn) return JF_ERR_UNSUPPORTED;
@@ -1622,6 +1863,119 @@ template <int EPI, typename ST> static int launch_gemm(const GemmArgs &a, hipStr
         return b_kn ? launch_gemm_b<EPI, ST, 1>(a, st) : launch_gemm_b<EPI, ST, 0>(a, st);
     }
 }
+
+// EPI_QA: 32-row tiles only (jf_igemm_block_q_add)
+template <typename ST> int launch_gemm_add(const GemmArgs &a, hipStream_t st)
+{
+    if (split_tiles_resident(a.M, a.N, a.K)) return launch_gemm_split<EPI_QA, ST, 0>(a, st);
+    return launch_gemm_cfg<EPI_QA, ST, 1, 1, 4, 3, 2, 0>(a, st);
+}
+
+#ifndef JF_PROF_LIB
+// x: as for a launch of its own; w: w_wgs workgroups, the longest of them k_per_part deep.
+template <int EPI, typename ST, int TILE> static int launch_backward(const GemmArgs &x, const GemmGroup &w, long w_wgs, int k_per_part, hipStream_t st)
+{
+    GemmBackward b = {x, w};
+    constexpr bool BIG = TILE == TILE_128x128;
+    constexpr int BN = TILE == TILE_32x64 ? 64 : 128;
+    b.x.tiles_m = BIG ? (x.M + 127) / 128 : x.M / QB; b.x.tiles_n = (x.N + BN - 1) / BN; b.x.splits = 1;
+    const long x_wgs = ((long)b.x.tiles_m * b.x.tiles_n + 7) & ~7L;
+    b.x.pace = !BIG ? (int)PACE_HARDWARE : pace_of(x_wgs + w_wgs, 2L * cu_count(), std::max(x.K, k_per_part));
+    for (int i = 0; i < w.n; ++i) b.w.g[i].pace = b.x.pace;
+    constexpr int SX = BIG ? gemm_lds(EPI, 2, 2, 4, 2) : TILE == TILE_32x128 ? gemm_lds(EPI, 1, 1, 4, 3) : SPLIT_LDS, SW = gemm_lds(EPI_FP, 2, 2, 4, 2), SMEM = SX > SW ? SX : SW;
+    static std::atomic<bool> opted_in[MAX_DEVICES] = {};
+    if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_backward_kernel<EPI, ST, TILE>), SMEM, opted_in)) return rc;
+    hipLaunchKernelGGL((igemm_backward_kernel<EPI, ST, TILE>), dim3((unsigned)(x_wgs + w_wgs)), dim3(512), SMEM, st, b);
+    return (int)hipGetLastError();
+}
+// One launch for an activation gradient and weight gradients: neither needs the other's result, small ones leave most of the chip
+// idle, and larger ones end in a round that is not full, once instead of twice.  The activation gradient's tiles, which are longer, come
+// first: 32x128 where one per CU holds them all, and two per CU where K is long and a 128x128 tile would outlast everything else.  us,
+// two launches | one, both gradients of a layer, rows x C_in x C_out:
+//   32x128: 32x768x768 10.3 | 6.4, 512x768x2304 20.8 | 13.2, 1024x1024x1024 22.8 | 18.7, 1248x768x3072 35.6 | 31.8; two per CU
+//   2048x1024x4096 55.5 | 52.5 (128x128: 59.0), 1024x1600x6400 65.7 | 56.7 (62.5);
+//   128x128: 2048x768x768 23.6 | 19.4 (32x128: 21.3), 1024x2048x1024 31.8 | 25.8 (28.5), 4096x768x768 35.0 | 26.0, 4096x1024x4096 84.4 | 78.3,
+//   12288x768x3072 127.5 | 119.4, 8192x1024x4096 141.4 | 138.2.
+// Above three 128x128 tiles of the activation gradient per CU the rounds even out by themselves: 4096x4096x1024 (1024) 86.1 | 83.7,
+// 8192x1600x4800 (832) 248.7 | 263.2, 8192x6400x1600 (3200) 359.4 | 363.9, 4096x4096x4096 (1024) 259.0 | 260.8.
+static bool backward_in_one_launch(int R, int C_in, long w_wgs)
+{
+    return (long)((R + 127) / 128) * ((C_in + 127) / 128) <= 3L * cu_count() && w_wgs <= 0x3fffffffL;
+}
+template <int EPI, typename ST> int launch_backward_any(const GemmArgs &x, const GemmGroup &w, long w_wgs, int k_per_part, hipStream_t st)
+{
+    if (split_tiles_resident(x.M, x.N, x.K) && split_tiles(x.M, x.N) + w_wgs <= cu_count())
+        return launch_backward<EPI, ST, TILE_32x64>(x, w, w_wgs, k_per_part, st);
+    const bool small = small_tiles_resident(x.M, x.N, x.K) && (x.K > 2048 || (long)(x.M / QB) * ((x.N + 127) / 128) <= cu_count());
+    if (small) return launch_backward<EPI, ST, TILE_32x128>(x, w, w_wgs, k_per_part, st);
+    return launch_backward<EPI, ST, TILE_128x128>(x, w, w_wgs, k_per_part, st);
+}
+
+#ifdef JF_PART
+#define JF_INST(part) JF_INST_##part
+#if JF_IN_PART(0)
+#define JF_INST_0
+#else
+#define JF_INST_0 extern
+#endif
+#if JF_IN_PART(1)
+#define JF_INST_1
+#else
+#define JF_INST_1 extern
+#endif
+#if JF_IN_PART(2)
+#define JF_INST_2
+#else
+#define JF_INST_2 extern
+#endif
+#if JF_IN_PART(3)
+#define JF_INST_3
+#else
+#define JF_INST_3 extern
+#endif
+#if JF_IN_PART(4)
+#define JF_INST_4
+#else
+#define JF_INST_4 extern
+#endif
+#if JF_IN_PART(5)
+#define JF_INST_5
+#else
+#define JF_INST_5 extern
+#endif
+#if JF_IN_PART(6)
+#define JF_INST_6
+#else
+#define JF_INST_6 extern
+#endif
+#if JF_IN_PART(7)
+#define JF_INST_7
+#else
+#define JF_INST_7 extern
+#endif
+#define JF_GEMM(part, EPI, ST) JF_INST(part) template int launch_gemm<EPI, ST>(const GemmArgs &, hipStream_t, bool, bool)
+#define JF_BWD(part, EPI, ST) JF_INST(part) template int launch_backward_any<EPI, ST>(const GemmArgs &, const GemmGroup &, long, int, hipStream_t)
+JF_GEMM(0, EPI_S32, float);
+JF_GEMM(1, EPI_FP, half_t);
+JF_GEMM(1, EPI_FP, float);
+JF_GEMM(2, EPI_Q, half_t);
+JF_GEMM(3, EPI_Q, float);
+JF_GEMM(4, EPI_QD, half_t);
+JF_GEMM(5, EPI_QD, float);
+JF_GEMM(6, EPI_QG, half_t);
+JF_GEMM(7, EPI_QG, float);
+JF_GEMM(6, EPI_QB, half_t);
+JF_GEMM(7, EPI_QB, float);
+JF_BWD(2, EPI_Q, half_t);
+JF_BWD(3, EPI_Q, float);
+JF_BWD(4, EPI_QD, half_t);
+JF_BWD(5, EPI_QD, float);
+JF_INST(0) template int launch_gemm_add<half_t>(const GemmArgs &, hipStream_t);
+JF_INST(0) template int launch_gemm_add<float>(const GemmArgs &, hipStream_t);
+JF_INST(1) template int launch_wgrad_group<half_t>(const GemmGroup &, unsigned, hipStream_t);
+JF_INST(1) template int launch_wgrad_group<float>(const GemmGroup &, unsigned, hipStream_t);
+#endif
+#endif  // !JF_PROF_LIB
 
 static int check_gemm_common(const void *A, const void *B, const void *C, int M, int N, int K, int b_layout)
 {
@@ -1650,41 +2004,7 @@ static bool scale_ptr_ok(const void *p, int scale_dtype)
     return (reinterpret_cast<uintptr_t>(p) & (scale_dtype == JF_SCALE_F32 ? 3u : 1u)) == 0;
 }
 
-#ifndef JF_PROF_LIB
-// x: as for a launch of its own; w: w_wgs workgroups, the longest of them k_per_part deep.
-template <int EPI, typename ST, bool SMALL> static int launch_backward(const GemmArgs &x, const GemmGroup &w, long w_wgs, int k_per_part, hipStream_t st)
-{
-    GemmBackward b = {x, w};
-    b.x.tiles_m = SMALL ? x.M / QB : (x.M + 127) / 128; b.x.tiles_n = (x.N + 127) / 128; b.x.splits = 1;
-    const long x_wgs = ((long)b.x.tiles_m * b.x.tiles_n + 7) & ~7L;
-    b.x.pace = SMALL ? (int)PACE_HARDWARE : pace_of(x_wgs + w_wgs, 2L * cu_count(), std::max(x.K, k_per_part));
-    for (int i = 0; i < w.n; ++i) b.w.g[i].pace = b.x.pace;
-    constexpr int SX = SMALL ? gemm_lds(EPI, 1, 1, 4, 3) : gemm_lds(EPI, 2, 2, 4, 2), SW = gemm_lds(EPI_FP, 2, 2, 4, 2), SMEM = SX > SW ? SX : SW;
-    static std::atomic<bool> opted_in[MAX_DEVICES] = {};
-    if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_backward_kernel<EPI, ST, SMALL>), SMEM, opted_in)) return rc;
-    hipLaunchKernelGGL((igemm_backward_kernel<EPI, ST, SMALL>), dim3((unsigned)(x_wgs + w_wgs)), dim3(512), SMEM, st, b);
-    return (int)hipGetLastError();
-}
-// One launch for an activation gradient and weight gradients: neither needs the other's result, small ones leave most of the chip
-// idle, and larger ones end in a round that is not full, once instead of twice.  The activation gradient's tiles, which are longer, come
-// first: 32x128 where one per CU holds them all, and two per CU where K is long and a 128x128 tile would outlast everything else.  us,
-// two launches | one, both gradients of a layer, rows x C_in x C_out:
-//   32x128: 32x768x768 10.3 | 6.4, 512x768x2304 20.8 | 13.2, 1024x1024x1024 22.8 | 18.7, 1248x768x3072 35.6 | 31.8; two per CU
-//   2048x1024x4096 55.5 | 52.5 (128x128: 59.0), 1024x1600x6400 65.7 | 56.7 (62.5);
-//   128x128: 2048x768x768 23.6 | 19.4 (32x128: 21.3), 1024x2048x1024 31.8 | 25.8 (28.5), 4096x768x768 35.0 | 26.0, 4096x1024x4096 84.4 | 78.3,
-//   12288x768x3072 127.5 | 119.4, 8192x1024x4096 141.4 | 138.2.
-// Above three 128x128 tiles of the activation gradient per CU the rounds even out by themselves: 4096x4096x1024 (1024) 86.1 | 83.7,
-// 8192x1600x4800 (832) 248.7 | 263.2, 8192x6400x1600 (3200) 359.4 | 363.9, 4096x4096x4096 (1024) 259.0 | 260.8.
-static bool backward_in_one_launch(int R, int C_in, long w_wgs)
-{
-    return (long)((R + 127) / 128) * ((C_in + 127) / 128) <= 3L * cu_count() && w_wgs <= 0x3fffffffL;
-}
-template <int EPI> static int launch_backward_any(const GemmArgs &x, const GemmGroup &w, long w_wgs, int k_per_part, bool f16, hipStream_t st)
-{
-    const bool small = small_tiles_resident(x.M, x.N, x.K) && (x.K > 2048 || (long)(x.M / QB) * ((x.N + 127) / 128) <= cu_count());
-    if (small) return f16 ? launch_backward<EPI, half_t, true>(x, w, w_wgs, k_per_part, st) : launch_backward<EPI, float, true>(x, w, w_wgs, k_per_part, st);
-    return f16 ? launch_backward<EPI, half_t, false>(x, w, w_wgs, k_per_part, st) : launch_backward<EPI, float, false>(x, w, w_wgs, k_per_part, st);
-}
+#if !defined(JF_PROF_LIB) && JF_IN_PART(0)
 // dX [R, C_in] = G [R, C_out] W [C_out, C_in], requantised or (dx_scales null) dequantised, scales in the tensors' own layout
 static GemmArgs dgrad_args(const int8_t *G, const void *sg, const int8_t *W, const void *sw, int R, int C_in, int C_out, void *dx, void *dx_scales,
                            int dx_dtype, uint64_t seed, uint64_t offset)
@@ -1951,9 +2271,10 @@ int jf_wgrad_many_dgrad(const int8_t *W, const void *sw, int8_t *dx, void *dx_sc
     hipStream_t st = (hipStream_t)stream;
     const bool f16 = scale_dtype == JF_SCALE_F16;
     const bool few = (long)((K + 127) / 128) * ((N[0] + 127) / 128) <= cu_count() / 2;
-    if (backward_in_one_launch(K, N[0], l.wgs) && (few || K <= 4096))
-        return launch_backward_any<EPI_Q>(dgrad_args(G[0], SG[0], W, sw, K, N[0], M[0], dx, dx_scales, 0, seed, offset), l.grp, l.wgs,
-                                          l.longest * QB, f16, st);
+    if (backward_in_one_launch(K, N[0], l.wgs) && (few || K <= 4096)) {
+        const GemmArgs x = dgrad_args(G[0], SG[0], W, sw, K, N[0], M[0], dx, dx_scales, 0, seed, offset);
+        return f16 ? launch_backward_any<EPI_Q, half_t>(x, l.grp, l.wgs, l.longest * QB, st) : launch_backward_any<EPI_Q, float>(x, l.grp, l.wgs, l.longest * QB, st);
+    }
     rc = jf_igemm_block_q(G[0], W, SG[0], sw, nullptr, nullptr, dx, dx_scales, K, N[0], M[0], JF_B_KN, scale_dtype, JF_SCALES_ROWMAJOR,
                           JF_SCALES_KMAJOR, JF_ROUND_STOCHASTIC, seed, offset, nullptr, 0, stream);
     return rc ? rc : launch_wgrads(l, f16, st);
@@ -2048,7 +2369,8 @@ int jf_linear_bwd(const int8_t *X, const void *sx, const int8_t *G, const void *
     const GemmArgs x = dgrad_args(G, sg, W, sw, R, C_in, C_out, dx, dx_scales, dx_dtype, seed, offset);
     const bool f16 = scale_dtype == JF_SCALE_F16;
     const int depth = splits > 1 ? kb_per * QB : R;
-    rc = dx_scales ? launch_backward_any<EPI_Q>(x, w, w_wgs, depth, f16, st) : launch_backward_any<EPI_QD>(x, w, w_wgs, depth, f16, st);
+    if (dx_scales) rc = f16 ? launch_backward_any<EPI_Q, half_t>(x, w, w_wgs, depth, st) : launch_backward_any<EPI_Q, float>(x, w, w_wgs, depth, st);
+    else rc = f16 ? launch_backward_any<EPI_QD, half_t>(x, w, w_wgs, depth, st) : launch_backward_any<EPI_QD, float>(x, w, w_wgs, depth, st);
     return rc || splits == 1 ? rc : launch_splitk_reduce((const float *)workspace, (size_t)C_out * (size_t)C_in, splits, dw, dw_dtype, st);
 }
 
@@ -2125,7 +2447,7 @@ int jf_igemm_block_q_add(const int8_t *A, const int8_t *B, const void *sa, const
     if (!scale_strides(sa_layout, K, M / QB, a.sa_ks, a.sa_is) || !scale_strides(sb_layout, K, N / QB, a.sb_ks, a.sb_is))
         return JF_ERR_ENUM;
     hipStream_t st = (hipStream_t)stream;
-    return scale_dtype == JF_SCALE_F16 ? launch_gemm_cfg<EPI_QA, half_t, 1, 1, 4, 3, 2, 0>(a, st) : launch_gemm_cfg<EPI_QA, float, 1, 1, 4, 3, 2, 0>(a, st);
+    return scale_dtype == JF_SCALE_F16 ? launch_gemm_add<half_t>(a, st) : launch_gemm_add<float>(a, st);
 }
 
 int jf_igemm_block_q_gelu(const int8_t *A, const int8_t *B, const void *sa, const void *sb, const float *bias,
@@ -2183,7 +2505,7 @@ int jf_transpose_s8(const int8_t *in, int R, int C, int8_t *out, jf_stream_t str
 }
 
 }  // extern "C"
-#else   // JF_PROF_LIB: libjetfire_prof.so
+#elif defined(JF_PROF_LIB)   // libjetfire_prof.so
 
 #include "../../include/jetfire_prof.h"
 
@@ -2210,4 +2532,4 @@ extern "C" int jf_prof_igemm_block_q(const int8_t *A, const int8_t *B, const flo
     return launch_gemm<EPI_Q, float>(a, (hipStream_t)stream, kn);
 }
 
-#endif  // JF_PROF_LIB
+#endif

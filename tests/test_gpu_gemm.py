@@ -632,6 +632,23 @@ def test_both_tile_sizes_at_every_ring_fill(jf, oracle, M, N, K):
         same(sc, wsc, "SR scales")
 
 
+# 32x64 tiles whose blocks two waves share (up to one per CU, 256): 15 of them with a ragged last column at every fill of the six-deep ring
+# and every length of its last stage, all 256, and the long row; with 288 tiles and a longer row 32x128 again
+@pytest.mark.parametrize("M,N,K", [(96, 160, k) for k in (32, 64, 96, 128, 160, 640, 768, 800, 896, 1056, 1632)]
+                         + [(1024, 512, 288), (32, 64, 16384), (1024, 544, 288)])
+def test_tiles_whose_blocks_two_waves_share(jf, oracle, M, N, K):
+    test_both_tile_sizes_at_every_ring_fill(jf, oracle, M, N, K)
+    test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K)       # (every other epilogue)
+    test_quantised_with_residual_addition(jf, oracle, M, N, K, torch.bfloat16, torch.float32, True, True)
+
+
+# activation gradients in 32x64 tiles beside weight gradients, one workgroup per CU: 248 and 8 of them, and one row of tiles more (32x128)
+@pytest.mark.parametrize("R,C_in,C_out,f16", [(992, 512, 64, True), (1024, 512, 64, True), (160, 544, 1056, False)])
+def test_both_gradients_with_tiles_that_two_waves_share(jf, R, C_in, C_out, f16):
+    for quantize in (True, False):
+        test_both_gradients_of_a_linear_layer_in_one_launch(jf, R, C_in, C_out, 0, f16, quantize)
+
+
 # 425 tiles of 128x128 (825 of 64x128, which would not all be resident), the last row and column of them ragged: every ring fill
 @pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 288, 384, 416])
 def test_the_large_tiles_at_every_ring_fill(jf, oracle, K):
