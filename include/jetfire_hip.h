@@ -291,8 +291,8 @@ int jf_add(const void *x1, int x1_dtype, const int8_t *q2, const void *s2, int R
            int scale_dtype, int rounding, uint64_t seed, uint64_t offset,
            void *y1, int y1_dtype, int8_t *q, void *s, float *rowsum, float *rowsq, jf_stream_t stream);
 
-/* The forward GEMM of jf_igemm_block_q (A [M,K], B [N,K], round to nearest) and jf_add of its result to x1, as one kernel where the
- * launch is small: y, (q, s), rowsum and rowsq are what jf_add(x1, <the requantised output>, add_rounding) returns, bit for bit.  The
+/* The forward GEMM of jf_igemm_block_q (A [M,K], B [N,K], round to nearest) and jf_add of its result to x1, as one kernel: y, (q, s),
+ * rowsum and rowsq are what jf_add(x1, <the requantised output>, add_rounding) returns, bit for bit.  The
  * requantised output itself is left nowhere.  q, s and y overlap no input.  add_rounding: JF_ROUND_NEAREST or JF_ROUND_TRUNC.
  * Replaces the pair igemm_output_int_quantize_bias_rowcol (include/igemm.h:66-77) + int8_add_Ifp_Ig16_Ofp_Og_MeanVar
  * (Jetfire/Nonlinear/add_mean_var.py:179-230) at the end of either half of a block (INT8_GPT2/qmodel.py:228). */

@@ -221,6 +221,14 @@ __device__ __forceinline__ uint32_t round_clamp_pack4(float a, float b, float c,
     return __builtin_amdgcn_perm(cd, ab, 0x05040100u);                                    // bytes: a, b, c, d
 }
 
+// The same rounded towards zero (the conversion does that), for |y| < 128.
+__device__ __forceinline__ uint32_t trunc_pack4(float a, float b, float c, float d)
+{
+    const uint32_t ab = __builtin_amdgcn_perm((uint32_t)(int)b, (uint32_t)(int)a, 0x0c0c0400u);
+    const uint32_t cd = __builtin_amdgcn_perm((uint32_t)(int)d, (uint32_t)(int)c, 0x0c0c0400u);
+    return __builtin_amdgcn_perm(cd, ab, 0x05040100u);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Block quantisation of 16 values per lane, one wave = one 32x32 block (lane l: row l/2,
 // columns 16*(l%2) .. +15).  Returns the packed codes; *scale_out = amax/127 (all lanes).
@@ -254,13 +262,14 @@ __device__ __forceinline__ v4i quantize16(const float v[16], float amax_eps, int
         }
     }
     if (rounding == JF_ROUND_TRUNC || rounding == JF_ROUND_STOCHASTIC_TRUNC) {
-        int c[16];
+        if (rounding == JF_ROUND_TRUNC) {                      // (for NaN only: -127)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) c[i] = clamp127(__builtin_truncf(y[i]));
-        out.x = (int)pack4(c[0], c[1], c[2], c[3]);
-        out.y = (int)pack4(c[4], c[5], c[6], c[7]);
-        out.z = (int)pack4(c[8], c[9], c[10], c[11]);
-        out.w = (int)pack4(c[12], c[13], c[14], c[15]);
+            for (int i = 0; i < 16; ++i) y[i] = __builtin_amdgcn_fmed3f(y[i], -127.0f, 127.0f);
+        }
+        out.x = (int)trunc_pack4(y[0], y[1], y[2], y[3]);
+        out.y = (int)trunc_pack4(y[4], y[5], y[6], y[7]);
+        out.z = (int)trunc_pack4(y[8], y[9], y[10], y[11]);
+        out.w = (int)trunc_pack4(y[12], y[13], y[14], y[15]);
     } else {
         // no clamp here: |v| <= amax and s = amax/127 correctly rounded give |v/s| <= 127 * (1 + 2^-23) < 127.5 (scales
         // outside the normal range were clamped above), and the stochastic path has limited |y| + noise to 127

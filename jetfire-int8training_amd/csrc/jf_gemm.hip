@@ -52,7 +52,7 @@ constexpr int EPI_LD = 36;                          // floats per staged row (32
 // EPI_QD: EPI_Q followed by the dequantisation of the block just requantised (codes x stored scale), written as float /
 //         binary16 / bfloat16: the requantised tensor itself is never written.
 // EPI_QA: EPI_Q (deterministic) followed by the residual addition of the block just requantised: the sum, its requantisation and its
-//         partial row sums leave (32x128 tiles only, see jf_igemm_block_q_add)
+//         partial row sums leave
 enum Epilogue { EPI_S32 = 0, EPI_FP = 1, EPI_Q = 2, EPI_QG = 3, EPI_QB = 4, EPI_QD = 5, EPI_QA = 6 };
 // Wave-priority schemes of the main loop (launch_gemm_cfg picks one per launch)
 enum Pace { PACE_HARDWARE = 0, PACE_EVEN = 1, PACE_ORDERED = 2 };
@@ -430,10 +430,11 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
 #pragma unroll
     for (int j = 0; j < WBN; ++j) { nb[j] = n0 / QB + wn * WBN + j; nb[j] = nb[j] < SN ? nb[j] : SN - 1; }
 
-    // EPI_QA: the lane's 16 elements of x1 are on their way during the main loop (the waves that multiply wait for no load in it)
+    // EPI_QA: the lane's 16 elements of x1 of the wave's block i.  With one block per wave they are on their way during the main loop (the
+    // waves that multiply wait for no load in it), with two each while the block before is worked on.
     v4i x1_raw[4];
-    auto fetch_x1 = [&] {
-        const size_t at = (size_t)(m0 + wm * QB + (lane & 31)) * p.N + n0 + wn * QB + (lane >> 5) * 16;
+    auto fetch_x1 = [&](int i) {
+        const size_t at = (size_t)(m0 + (wm * WBM + i) * QB + (lane & 31)) * p.N + n0 + wn * QB + (lane >> 5) * 16;
         if (p.x1_dtype == JF_FP_F32) {
             const v4i *src = reinterpret_cast<const v4i *>(reinterpret_cast<const float *>(p.x1) + at);
 #pragma unroll
@@ -655,7 +656,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         if (!loader) make_table();
         else if (SPLIT > 1) wait_behind(SPLIT_RING < nstages ? SPLIT_RING - 1 : nstages - 1);
         else wait_stage(NSTAGE - 1, std::integral_constant<int, NSTAGE - 1>{});           // stage 0 has landed
-        if constexpr (EPI == EPI_QA) { if (!loader && m0 + wm * QB < p.M && n0 + wn * QB < p.N) fetch_x1(); }
+        if constexpr (EPI == EPI_QA) { if (!loader && m0 + wm * QB < p.M && n0 + wn * QB < p.N) fetch_x1(0); }
     } else {
         if (NSTAGE - 1 >= nstages) JF_WAIT_VMCNT(0);
         else JF_WAIT_VMCNT((NSTAGE - 1) * LOADS - (EPI != EPI_S32 ? 1 : 0));      // stage 0 and the scales of stage 1 have landed
@@ -1052,6 +1053,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     __builtin_amdgcn_s_waitcnt(0xC07F);                        // the last, unused prefetch must land before its registers are reused
     float lane_max[WBM][WBN];                                  // largest magnitude of this lane's results, per block   (QUANT)
     bool nonfinite = false;                                    // wave-uniform: some result is infinite or NaN   (QUANT)
+    if constexpr (EPI == EPI_QA && WBM == 2) { if (wave_active) fetch_x1(0); }
     if (EPI != EPI_S32 && wave_active && !loader) {
         if constexpr (SPLIT == 1) accumulate(std::integral_constant<int, NBLK - 1>{});
         if constexpr (FOLD) { if (folds > 0) add_parts(); }
@@ -1147,7 +1149,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     }
     if (PROF) { phase(2, (unsigned long long)wall_clock64()); phase(7, (unsigned long long)(clock64() - prof_c0)); }
     if (p.pace != PACE_HARDWARE) __builtin_amdgcn_s_setprio(0);
-    if constexpr (SPLIT == 1 && (!QUANT || EPI == EPI_QA)) __syncthreads();    // the epilogue reuses the ring as scratch
+    if constexpr (SPLIT == 1 && (!QUANT || (EPI == EPI_QA && WBM == 1))) __syncthreads();    // the epilogue reuses the ring as scratch
     if (loader) return;
     if (PROF) phase(3, (unsigned long long)wall_clock64());
 
@@ -1353,7 +1355,24 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                             y[k] = __uint_as_float(k & 1 ? w & 0xffff0000u : w << 16) + y[k];
                         }
                     }
-                    if (p.out_dtype == JF_FP_F32) {
+                    if (i + 1 < WBM && bm + QB < p.M) fetch_x1(i + 1);
+                    if (p.out_dtype == JF_FP_F32 && WBM == 2) {
+                        // whole rows without a patch of the block's size and its barrier: eight at a time through the wave's scale patch
+                        static_assert(EPI != EPI_QA || WBM == 1 || 2 * NSTAGE * SC_SLOT >= 8 * 128, "eight rows of 128 bytes");
+#pragma unroll
+                        for (int h = 0; h < 4; ++h) {
+                            if ((rrow >> 3) == h) {
+#pragma unroll
+                                for (int k = 0; k < 4; ++k)
+                                    *reinterpret_cast<v4f *>(scale_patch + (rrow & 7) * 128 + (((rcol / 4 + k) ^ (rrow & 7)) << 4)) = v4f{y[4 * k], y[4 * k + 1], y[4 * k + 2], y[4 * k + 3]};
+                            }
+                            wave_sync();
+                            const int row = lane >> 3;
+                            const v4f t = *reinterpret_cast<const v4f *>(scale_patch + row * 128 + (((lane & 7) ^ row) << 4));
+                            *reinterpret_cast<v4f *>(reinterpret_cast<float *>(p.y) + (size_t)(bm + 8 * h + row) * p.N + bn + (lane & 7) * 4) = t;
+                            wave_sync();
+                        }
+                    } else if (p.out_dtype == JF_FP_F32) {
 #pragma unroll
                         for (int k = 0; k < 4; ++k) *reinterpret_cast<v4f *>(patch + rrow * EPI_LD + rcol + 4 * k) = v4f{y[4 * k], y[4 * k + 1], y[4 * k + 2], y[4 * k + 3]};
                         wave_sync();
@@ -1823,7 +1842,7 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs
         if (a.splits <= 1 && small_tiles_resident(a.M, a.N, a.K))
             return launch_gemm_cfg<EPI, ST, 1, 1, 4, 3, 2, BKN>(a, st);
     }
-    if constexpr (EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD) {
+    if constexpr (EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD || EPI == EPI_QA) {
         if (const int big = mixed_big_rows(a.M, a.N, a.K)) return launch_gemm_mixed<EPI, ST, BKN>(a, big, st);
     }
     // 64x128 tiles, four waves of two blocks, three workgroups per CU: where they are all resident at once (up to 384 big tiles), the
@@ -1832,7 +1851,7 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs
     // 27.8, 3072x1024x4096 (192) 37.5 | 34.9, 2048x1600x1600 (208) 17.6 | 16.9, 1248x2304x768 (180) 10.7 | 10.3; two rounds of them: 2560x2560x2560
     // (400) 37.1 | 47.4.  Not with the GELU forward behind it, whose byte tables leave room for two workgroups only; with its backward,
     // the longest epilogue, above one big tile per CU: 2048x3072x768 (384) 22.0 | 19.8, 1248x3072x768 (240) 15.2 | 15.6.
-    if constexpr (EPI == EPI_Q || EPI == EPI_QB || EPI == EPI_QD) {
+    if constexpr (EPI == EPI_Q || EPI == EPI_QB || EPI == EPI_QD || EPI == EPI_QA) {
         const long tiles_n = (a.N + 127) / 128;
         if ((a.M + 63) / 64 * tiles_n <= 3L * cu_count() && (EPI != EPI_QB || (a.M + 127) / 128 * tiles_n > cu_count()))
             return launch_gemm_cfg<EPI, ST, 2, 1, 4, 2, 3, BKN>(a, st);
@@ -1841,7 +1860,7 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs
 }
 template <int EPI, typename ST> int launch_gemm(const GemmArgs &a, hipStream_t st, bool b_kn, bool a_km = false)
 {
-    if constexpr (EPI == EPI_QG) {                            // the forward form only: A [M,K], B [N,K]
+    if constexpr (EPI == EPI_QG || EPI == EPI_QA) {           // the forward form only: A [M,K], B [N,K]
         if (a_km || b_kn) return JF_ERR_UNSUPPORTED;
         return launch_gemm_b<EPI, ST, 0>(a, st);
     } else if constexpr (EPI == EPI_QB) {                     // the activation-gradient form only: A [M,K], B [K,N]
@@ -1862,13 +1881,6 @@ template <int EPI, typename ST> int launch_gemm(const GemmArgs &a, hipStream_t s
 #endif
         return b_kn ? launch_gemm_b<EPI, ST, 1>(a, st) : launch_gemm_b<EPI, ST, 0>(a, st);
     }
-}
-
-// EPI_QA: 32-row tiles only (jf_igemm_block_q_add)
-template <typename ST> int launch_gemm_add(const GemmArgs &a, hipStream_t st)
-{
-    if (split_tiles_resident(a.M, a.N, a.K)) return launch_gemm_split<EPI_QA, ST, 0>(a, st);
-    return launch_gemm_cfg<EPI_QA, ST, 1, 1, 4, 3, 2, 0>(a, st);
 }
 
 #ifndef JF_PROF_LIB
@@ -1970,8 +1982,8 @@ JF_BWD(2, EPI_Q, half_t);
 JF_BWD(3, EPI_Q, float);
 JF_BWD(4, EPI_QD, half_t);
 JF_BWD(5, EPI_QD, float);
-JF_INST(0) template int launch_gemm_add<half_t>(const GemmArgs &, hipStream_t);
-JF_INST(0) template int launch_gemm_add<float>(const GemmArgs &, hipStream_t);
+JF_GEMM(0, EPI_QA, half_t);
+JF_GEMM(1, EPI_QA, float);
 JF_INST(1) template int launch_wgrad_group<half_t>(const GemmGroup &, unsigned, hipStream_t);
 JF_INST(1) template int launch_wgrad_group<float>(const GemmGroup &, unsigned, hipStream_t);
 #endif
@@ -2419,12 +2431,11 @@ int jf_igemm_block_q_dequant(const int8_t *A, const int8_t *B, const void *sa, c
     return scale_dtype == JF_SCALE_F16 ? launch_gemm<EPI_QD, half_t>(a, st, kn) : launch_gemm<EPI_QD, float>(a, st, kn);
 }
 
-// The residual addition reads and writes 13 to 17 bytes per element that the GEMM has in registers, in a launch of its own.  In the
-// epilogue where the launch is one of 32x128 tiles that are all resident at once: there the addition's launch is what costs.  us, two
-// launches | this | the GEMM alone, float in and out, binary16 scales: 32x768x768 8.7 | 6.9 | 5.6, 64x256x256 7.0 | 5.6 | 4.1, 512x256x1024
-// 9.6 | 7.7 | 6.4, 1248x768x768 10.0 | 7.8 | 5.9, 1248x768x3072 17.4 | 14.7 | 12.4, 2048x768x3072 21.5 | 18.8 | 15.6.  Larger launches keep the
-// two: the epilogue of a 128x128 tile has no room in LDS to turn the float sum into whole rows without a barrier of the workgroup, and
-// as separate 16-byte pieces it would hold up the other tiles' loads.
+// The residual addition reads and writes 13 to 17 bytes per element, of which the GEMM has a third in registers, in a launch of its own.
+// us, two launches | this | the GEMM alone, binary16 scales.  Float in and out: 32x768x768 8.7 | 6.3 | 5.3, 512x256x1024 9.6 | 7.2 | 6.0,
+// 1248x768x768 10.0 | 7.8 | 5.9, x3072 17.4 | 14.7 | 12.4.  Float in, bfloat16 out: 4096x768x768 18.6 | 16.4 | 12.2, 12288x768x768 40.2 | 34.8 |
+// 24.6, x3072 86.5 | 81.5 | 68, 8192x1600x1600 76.3 | 69 | 53, x6400 190 | 187 | 166, 8192x1024x1024 37.1 | 31.7 | 22.9, 12288x768x96 27.0 | 20.6 | 11.6.
+// What it adds to a large launch is memory time: the tiles of a round end together, and their 8 bytes per element have nothing to hide behind.
 int jf_igemm_block_q_add(const int8_t *A, const int8_t *B, const void *sa, const void *sb, const float *bias, const float *biasmax,
                          const void *x1, int x1_dtype, int add_rounding, void *y, int y_dtype, int8_t *q, void *s, float *rowsum,
                          float *rowsq, int M, int N, int K, int scale_dtype, int sa_layout, int sb_layout, jf_stream_t stream)
@@ -2435,11 +2446,6 @@ int jf_igemm_block_q_add(const int8_t *A, const int8_t *B, const void *sa, const
     if ((scale_dtype != JF_SCALE_F16 && scale_dtype != JF_SCALE_F32) || (add_rounding != JF_ROUND_NEAREST && add_rounding != JF_ROUND_TRUNC) ||
         x1_dtype < JF_FP_F16 || x1_dtype > JF_FP_BF16 || y_dtype < JF_FP_F16 || y_dtype > JF_FP_BF16) return JF_ERR_ENUM;
     if (!aligned16(x1) || !aligned16(y) || !scale_ptr_ok(sa, scale_dtype) || !scale_ptr_ok(sb, scale_dtype)) return JF_ERR_ALIGN;
-    if (!small_tiles_resident(M, N, K)) {
-        rc = jf_igemm_block_q(A, B, sa, sb, bias, biasmax, q, s, M, N, K, JF_B_NK, scale_dtype, sa_layout, sb_layout, JF_ROUND_NEAREST, 0, 0,
-                              nullptr, 0, stream);
-        return rc ? rc : jf_add(x1, x1_dtype, q, s, M, N, scale_dtype, add_rounding, 0, 0, y, y_dtype, q, s, rowsum, rowsq, stream);
-    }
     GemmArgs a = {};
     a.A = A; a.B = B; a.sa = sa; a.sb = sb; a.C = q; a.sc = s; a.bias = bias; a.biasmax = biasmax;
     a.x1 = x1; a.x1_dtype = x1_dtype; a.rounding2 = add_rounding; a.y = y; a.out_dtype = y_dtype; a.rowsum = rowsum; a.rowsq = rowsq;
@@ -2447,7 +2453,7 @@ int jf_igemm_block_q_add(const int8_t *A, const int8_t *B, const void *sa, const
     if (!scale_strides(sa_layout, K, M / QB, a.sa_ks, a.sa_is) || !scale_strides(sb_layout, K, N / QB, a.sb_ks, a.sb_is))
         return JF_ERR_ENUM;
     hipStream_t st = (hipStream_t)stream;
-    return scale_dtype == JF_SCALE_F16 ? launch_gemm_add<half_t>(a, st) : launch_gemm_add<float>(a, st);
+    return scale_dtype == JF_SCALE_F16 ? launch_gemm<EPI_QA, half_t>(a, st, false) : launch_gemm<EPI_QA, float>(a, st, false);
 }
 
 int jf_igemm_block_q_gelu(const int8_t *A, const int8_t *B, const void *sa, const void *sb, const float *bias,

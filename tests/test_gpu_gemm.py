@@ -642,6 +642,15 @@ def test_tiles_whose_blocks_two_waves_share(jf, oracle, M, N, K):
     test_quantised_with_residual_addition(jf, oracle, M, N, K, torch.bfloat16, torch.float32, True, True)
 
 
+# the residual addition in the epilogue of every larger tile: 128x128 with ragged rows and columns, both sizes in one launch, 64x128; one K block
+# and a short last stage
+@pytest.mark.parametrize("M,N,K,x1,y", [(2080, 3104, 32, torch.float32, torch.float32), (2080, 3104, 160, torch.bfloat16, torch.bfloat16),
+                                        (5408, 768, 96, torch.float16, torch.float32), (2080, 1056, 288, torch.float32, torch.float16)])
+def test_residual_addition_in_the_large_tiles(jf, oracle, M, N, K, x1, y):
+    test_quantised_with_residual_addition(jf, oracle, M, N, K, x1, y, True, True)
+    test_quantised_with_residual_addition(jf, oracle, M, N, K, x1, y, False, False)
+
+
 # activation gradients in 32x64 tiles beside weight gradients, one workgroup per CU: 248 and 8 of them, and one row of tiles more (32x128)
 @pytest.mark.parametrize("R,C_in,C_out,f16", [(992, 512, 64, True), (1024, 512, 64, True), (160, 544, 1056, False)])
 def test_both_gradients_with_tiles_that_two_waves_share(jf, R, C_in, C_out, f16):
