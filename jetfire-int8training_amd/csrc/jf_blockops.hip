@@ -358,25 +358,30 @@ __device__ __forceinline__ void group_request(const int8_t *q, const ST *s, int 
         sc[j] = load_scale(s, rb * SC + cb);
     }
 }
-static inline int grid_for_groups(int R, int C)
+static inline int grid_for_groups(int R, int C, int blocks = 4)
 {
-    const long groups = (long)(R / QB) * ((C / QB + 3) / 4), g = (groups + WPB - 1) / WPB;
+    const long groups = (long)(R / QB) * ((C / QB + blocks - 1) / blocks), g = (groups + WPB - 1) / WPB;
     return (int)(g < 256L * 16 ? g : 256L * 16);
 }
+// One block per wave up to eight blocks per SIMD: four in a row are what such a tensor waits for, and it stays in the caches, where the
+// quarter-line writes cost nothing.  us, four | one block per wave, forward and backward: 256x1024 5.2, 7.2 | 2.9, 3.5; 1248x2080 5.6, 7.7 | 3.8,
+// 4.9; 2048x4096 7.1, 10.6 | 5.5, 8.7; beyond the caches 8192x6400 29.4, 44.4 | 34, 47 (within them 22.8, 40.8 | 20.6, 37.4).
+static inline bool gelu_by_blocks(int R, int C) { return (long)(R / QB) * (C / QB) <= 32L * cu_count(); }
 
 // gelu_fwd.py:34-126
-template <int APPROX, typename ST>
+// BLOCKS = 1: a wave takes one block and stores it in the row layout.  For tensors whose groups of four would leave SIMDs without a wave.
+template <int APPROX, typename ST, int BLOCKS>
 __global__ __launch_bounds__(NT) void gelu_fwd_kernel(const int8_t *q, const ST *s, int R, int C, float amax_eps,
                                                       int8_t *qy, ST *sy)
 {
     __shared__ __attribute__((aligned(16))) float table[WPB][256];
     __shared__ __attribute__((aligned(16))) int qtable[WPB][64];      // 256 one-byte entries per wave
-    __shared__ __attribute__((aligned(16))) unsigned char patches[WPB][QB * LINE_PITCH];
+    __shared__ __attribute__((aligned(16))) unsigned char patches[BLOCKS > 1 ? WPB : 1][BLOCKS > 1 ? QB * LINE_PITCH : 16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     float *tab = table[wave];
     int *qtab = qtable[wave];
-    unsigned char *patch = patches[wave];
-    const int SC = C / QB, SG = (SC + 3) / 4, ngrp = (R / QB) * SG, stride = gridDim.x * WPB;
+    unsigned char *patch = patches[BLOCKS > 1 ? wave : 0];
+    const int SC = C / QB, SG = BLOCKS > 1 ? (SC + 3) / 4 : SC, ngrp = (R / QB) * SG, stride = gridDim.x * WPB;
     int g = blockIdx.x * WPB + wave;
     if (g >= ngrp) return;
     float zero = 0.0f;
@@ -384,6 +389,13 @@ __global__ __launch_bounds__(NT) void gelu_fwd_kernel(const int8_t *q, const ST 
     const float f0 = gelu<APPROX>(zero);
     for (; g < ngrp; g += stride) {
         const int rb = g / SG, cg = g - rb * SG;
+        if constexpr (BLOCKS == 1) {
+            const size_t e0 = (size_t)(rb * QB + (lane >> 1)) * C + cg * QB + (lane & 1) * 16;
+            float scale;
+            *reinterpret_cast<v4i *>(qy + e0) = gelu_fwd_block<APPROX>(*reinterpret_cast<const v4i *>(q + e0), load_scale(s, rb * SC + cg), f0, amax_eps, tab, qtab, lane, &scale);
+            if (lane == 0) store_scale(sy, rb * SC + cg, scale);
+            continue;
+        }
         v4i cur[4];
         float csc[4];
         group_request(q, s, C, rb, cg, lane, cur, csc);            // the later blocks arrive while the first is worked on
@@ -403,18 +415,18 @@ __global__ __launch_bounds__(NT) void gelu_fwd_kernel(const int8_t *q, const ST 
 // gelu_bwd.py:28-171
 // (Held to five waves per SIMD: with the codes of four blocks of both inputs in flight the kernel wants 97 registers, one
 // more than five waves allow, and runs 1 us faster at 8192x6400 with five waves than with four.)
-template <int APPROX, typename ST>
+template <int APPROX, typename ST, int BLOCKS>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5, 5)))
 void gelu_bwd_kernel(const int8_t *qx, const ST *sx, const int8_t *qg, const ST *sg,
                                                       int R, int C, int rounding, uint64_t seed, uint64_t offset,
                                                       int8_t *qy, ST *sy)
 {
     __shared__ __attribute__((aligned(16))) float table[WPB][256];
-    __shared__ __attribute__((aligned(16))) unsigned char patches[WPB][QB * LINE_PITCH];
+    __shared__ __attribute__((aligned(16))) unsigned char patches[BLOCKS > 1 ? WPB : 1][BLOCKS > 1 ? QB * LINE_PITCH : 16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     float *tab = table[wave];
-    unsigned char *patch = patches[wave];
-    const int SC = C / QB, SG = (SC + 3) / 4, ngrp = (R / QB) * SG, stride = gridDim.x * WPB;
+    unsigned char *patch = patches[BLOCKS > 1 ? wave : 0];
+    const int SC = C / QB, SG = BLOCKS > 1 ? (SC + 3) / 4 : SC, ngrp = (R / QB) * SG, stride = gridDim.x * WPB;
     int g = blockIdx.x * WPB + wave;
     if (g >= ngrp) return;
     float zero = 0.0f;
@@ -422,6 +434,14 @@ void gelu_bwd_kernel(const int8_t *qx, const ST *sx, const int8_t *qg, const ST 
     const float f0 = dgelu<APPROX>(zero);
     for (; g < ngrp; g += stride) {
         const int rb = g / SG, cg = g - rb * SG;
+        if constexpr (BLOCKS == 1) {
+            const size_t e0 = (size_t)(rb * QB + (lane >> 1)) * C + cg * QB + (lane & 1) * 16;
+            float scale;
+            *reinterpret_cast<v4i *>(qy + e0) = gelu_bwd_block<APPROX>(*reinterpret_cast<const v4i *>(qx + e0), load_scale(sx, rb * SC + cg), *reinterpret_cast<const v4i *>(qg + e0),
+                                                                       load_scale(sg, rb * SC + cg), f0, tab, lane, rounding, seed, offset, e0, &scale);
+            if (lane == 0) store_scale(sy, rb * SC + cg, scale);
+            continue;
+        }
         v4i cx[4], cgr[4];
         float scx[4], scg[4];
         group_request(qx, sx, C, rb, cg, lane, cx, scx);
@@ -1126,6 +1146,68 @@ __global__ __launch_bounds__(NT) void add_kernel(const T *x1, const int8_t *q2, 
     }
 }
 
+// add_kernel and rowstats_finish_kernel as one launch, bit for bit: a workgroup owns a 32-row strip (wave w: column blocks w, w + 16, ..., all
+// of them requested at once), so that the partial sums of its rows never leave it (add_in_strips).
+constexpr int ADS_WAVES = 16, ADS_BPW = 4;
+template <typename T, typename ST, typename OT>
+__global__ __launch_bounds__(WAVE * ADS_WAVES, 4) void add_strip_kernel(const T *x1, const int8_t *q2, const ST *s2, int R, int C,
+                                                                        int rounding, uint64_t seed, uint64_t offset, OT *y1, int8_t *q,
+                                                                        ST *s, float *mean, float *rstd)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds_f[];  // partial sums [2][C/32][32], squares of a row [32], patches
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int SC = C / QB, rb = blockIdx.x, row = rb * QB + (lane >> 1);
+    float *part = lds_f, *sq = part + 2 * SC * QB, *ypatch = sq + QB + wave * (QB * ADD_PITCH);
+    float a[ADS_BPW][16];
+    v4i c[ADS_BPW];
+    float sc[ADS_BPW];
+    static_for<0, ADS_BPW>([&](auto i_c) {
+        constexpr int I = decltype(i_c)::value;
+        const int cb = wave + I * ADS_WAVES;
+        if (cb < SC) {
+            const size_t e0 = (size_t)row * C + cb * QB + (lane & 1) * 16;
+            Load16<T>::run(x1 + e0, a[I]);
+            c[I] = *reinterpret_cast<const v4i *>(q2 + e0);
+            sc[I] = load_scale(s2, rb * SC + cb);
+        }
+    });
+    static_for<0, ADS_BPW>([&](auto i_c) {
+        constexpr int I = decltype(i_c)::value;
+        const int cb = wave + I * ADS_WAVES;
+        if (cb >= SC) return;                                      // uniform
+        const size_t e0 = (size_t)row * C + cb * QB + (lane & 1) * 16;
+        float b[16];
+        unpack16(c[I], sc[I], b);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) b[k] = a[I][k] + b[k];
+        float t1 = 0.0f, t2 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) { t1 = t1 + b[k]; t2 = __builtin_fmaf(b[k], b[k], t2); }
+        const float o1 = __shfl_xor(t1, 1, WAVE), o2 = __shfl_xor(t2, 1, WAVE);
+        if ((lane & 1) == 0) {
+            part[cb * QB + (lane >> 1)] = t1 + o1;
+            part[(SC + cb) * QB + (lane >> 1)] = t2 + o2;
+        }
+        store_block_rows(ypatch, b, y1 + (size_t)rb * QB * C + cb * QB, C, lane);
+        float scale;
+        *reinterpret_cast<v4i *>(q + e0) = quantize16(b, 0.0f, rounding, seed, offset, e0, &scale);
+        if (lane == 0) store_scale(s, rb * SC + cb, scale);
+    });
+    __syncthreads();
+    float acc = 0.0f;                                              // threads 0..31: sums, 32..63: squares, in ascending order
+    if (threadIdx.x < 2 * QB) {
+        const float *p = part + (threadIdx.x >> 5) * SC * QB + (threadIdx.x & 31);
+        for (int j = 0; j < SC; ++j) acc = acc + p[j * QB];
+        if (threadIdx.x >= QB) sq[threadIdx.x & 31] = acc;
+    }
+    __syncthreads();
+    if (threadIdx.x < QB) {
+        const float n = (float)C, m = acc / n, var = sq[threadIdx.x] / n - m * m;
+        mean[rb * QB + threadIdx.x] = m;
+        rstd[rb * QB + threadIdx.x] = 1.0f / __builtin_sqrtf(var);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 static inline int grid_for_blocks(int R, int C)
 {
@@ -1196,6 +1278,17 @@ __global__ __launch_bounds__(256) void rowstats_finish_kernel(const float *rowsu
         mean[r0 + row] = m;
         rstd[r0 + row] = 1.0f / __builtin_sqrtf(var);
     }
+}
+
+// Where one workgroup per strip takes the place of two launches (jf_add_rowstats): a CU to itself for every strip, and either few blocks in
+// a row or enough strips to occupy the chip.  us, two launches | one, bfloat16 in and out (float): 32x128 4.5 | 3.1, 512x1024 6.7 | 7.0 (6.7 | 7.4),
+// 1248x1120 7.6 | 7.3 (8.1 | 8.5), 2048x768 7.1 | 5.9, 4096x1024 9.4 | 8.8, 8192x768 11.6 | 8.4, 8192x1600 21.0 | 16.4 (28.0 | 22.3), 4096x2048 16.3 |
+// 15.9; on the other side of the line 1248x1536 8.4 | 9.9, 2048x1600 10.4 | 10.9, 256x2048 8.1 | 11.8.  (A launch and two allocations less are
+// another 5 us of the host.)
+static bool add_in_strips(int R, int C)
+{
+    const int strips = R / QB, blocks = C / QB, cus = cu_count();
+    return blocks <= ADS_WAVES * ADS_BPW && strips <= cus && (blocks <= 36 || 8 * strips >= 3 * cus);
 }
 
 #define JF_LAUNCH(kern, grid, smem, st, ...)                         \
@@ -1550,8 +1643,13 @@ int jf_gelu_fwd(const int8_t *q, const void *s, int R, int C, int scale_dtype, i
     if (approx != JF_GELU_ERF && approx != JF_GELU_TANH) return JF_ERR_ENUM;
     if (!aligned16(qy)) return JF_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
-    const int grid = grid_for_groups(R, C);
-#define JF_GF(A, ST) JF_LAUNCH((gelu_fwd_kernel<A, ST>), grid, 0, st, q, (const ST *)s, R, C, amax_eps, qy, (ST *)sy)
+    const bool one = gelu_by_blocks(R, C);
+    const int grid = grid_for_groups(R, C, one ? 1 : 4);
+#define JF_GF(A, ST)                                                                                              \
+    do {                                                                                                          \
+        if (one) JF_LAUNCH((gelu_fwd_kernel<A, ST, 1>), grid, 0, st, q, (const ST *)s, R, C, amax_eps, qy, (ST *)sy); \
+        JF_LAUNCH((gelu_fwd_kernel<A, ST, 4>), grid, 0, st, q, (const ST *)s, R, C, amax_eps, qy, (ST *)sy);      \
+    } while (0)
     if (scale_dtype == JF_SCALE_F16) {
         if (approx == JF_GELU_ERF) JF_GF(JF_GELU_ERF, half_t);
         JF_GF(JF_GELU_TANH, half_t);
@@ -1572,10 +1670,13 @@ int jf_gelu_bwd(const int8_t *qx, const void *sx, const int8_t *qg, const void *
     if ((approx != JF_GELU_ERF && approx != JF_GELU_TANH) || !rounding_ok(rounding)) return JF_ERR_ENUM;
     if (!aligned16(qy)) return JF_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
-    const int grid = grid_for_groups(R, C);
+    const bool one = gelu_by_blocks(R, C);
+    const int grid = grid_for_groups(R, C, one ? 1 : 4);
 #define JF_GB(A, ST)                                                                                              \
-    JF_LAUNCH((gelu_bwd_kernel<A, ST>), grid, 0, st, qx, (const ST *)sx, qg, (const ST *)sg, R, C, rounding, seed, \
-              offset, qy, (ST *)sy)
+    do {                                                                                                          \
+        if (one) JF_LAUNCH((gelu_bwd_kernel<A, ST, 1>), grid, 0, st, qx, (const ST *)sx, qg, (const ST *)sg, R, C, rounding, seed, offset, qy, (ST *)sy); \
+        JF_LAUNCH((gelu_bwd_kernel<A, ST, 4>), grid, 0, st, qx, (const ST *)sx, qg, (const ST *)sg, R, C, rounding, seed, offset, qy, (ST *)sy); \
+    } while (0)
     if (scale_dtype == JF_SCALE_F16) {
         if (approx == JF_GELU_ERF) JF_GB(JF_GELU_ERF, half_t);
         JF_GB(JF_GELU_TANH, half_t);
@@ -1602,6 +1703,63 @@ int jf_add(const void *x1, int x1_dtype, const int8_t *q2, const void *s2, int R
 #define JF_ADD(T, ST, OT)                                                                                         \
     JF_LAUNCH((add_kernel<T, ST, OT>), grid, 0, st, (const T *)x1, q2, (const ST *)s2, R, C, rounding, seed, offset, \
               (OT *)y1, q, (ST *)s, rowsum, rowsq)
+#define JF_ADD_OUT(T, ST)                                                                                         \
+    do {                                                                                                          \
+        if (y1_dtype == JF_FP_F32) JF_ADD(T, ST, float);                                                          \
+        if (y1_dtype == JF_FP_F16) JF_ADD(T, ST, half_t);                                                         \
+        JF_ADD(T, ST, __bf16);                                                                                    \
+    } while (0)
+    if (scale_dtype == JF_SCALE_F16) {
+        if (x1_dtype == JF_FP_F32) JF_ADD_OUT(float, half_t);
+        if (x1_dtype == JF_FP_F16) JF_ADD_OUT(half_t, half_t);
+        JF_ADD_OUT(__bf16, half_t);
+    } else {
+        if (x1_dtype == JF_FP_F32) JF_ADD_OUT(float, float);
+        if (x1_dtype == JF_FP_F16) JF_ADD_OUT(half_t, float);
+        JF_ADD_OUT(__bf16, float);
+    }
+#undef JF_ADD_OUT
+#undef JF_ADD
+}
+
+size_t jf_add_rowstats_workspace_bytes(int R, int C)
+{
+    if (R <= 0 || C <= 0 || add_in_strips(R, C)) return 0;
+    return (size_t)2 * (C / QB) * R * sizeof(float);
+}
+
+int jf_add_rowstats(const void *x1, int x1_dtype, const int8_t *q2, const void *s2, int R, int C, int scale_dtype, int rounding,
+                    uint64_t seed, uint64_t offset, void *y1, int y1_dtype, int8_t *q, void *s, float *mean, float *rstd, void *workspace,
+                    size_t workspace_bytes, jf_stream_t stream)
+{
+    int rc = check_block_tensor(q2, s2, R, C, scale_dtype);
+    if (rc) return rc;
+    if (!x1 || !y1 || !q || !s || !mean || !rstd) return JF_ERR_NULL;
+    if (!rounding_ok(rounding) || x1_dtype < JF_FP_F16 || x1_dtype > JF_FP_BF16 || y1_dtype < JF_FP_F16 || y1_dtype > JF_FP_BF16) return JF_ERR_ENUM;
+    if (!aligned16(x1) || !aligned16(y1) || !aligned16(q)) return JF_ERR_ALIGN;
+    if (!add_in_strips(R, C)) {
+        if (!workspace || !aligned16(workspace) || workspace_bytes < jf_add_rowstats_workspace_bytes(R, C)) return JF_ERR_WORKSPACE;
+        float *const rowsum = (float *)workspace, *const rowsq = rowsum + (size_t)(C / QB) * R;
+        rc = jf_add(x1, x1_dtype, q2, s2, R, C, scale_dtype, rounding, seed, offset, y1, y1_dtype, q, s, rowsum, rowsq, stream);
+        return rc ? rc : jf_rowstats_finish(rowsum, rowsq, R, C / QB, C, mean, rstd, stream);
+    }
+    if (!device_is_gfx950()) return JF_ERR_DEVICE;
+    const size_t lds = ((size_t)2 * (C / QB) * QB + QB + ADS_WAVES * QB * ADD_PITCH) * sizeof(float);
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return JF_ERR_DEVICE;
+#define JF_ADD(T, ST, OT)                                                                                         \
+    do {                                                                                                          \
+        auto kern = add_strip_kernel<T, ST, OT>;                                                                  \
+        static std::atomic<bool> opted_in[MAX_DEVICES] = {};      /* more than 64 KiB of LDS: once per device */  \
+        if (!opted_in[dev].load(std::memory_order_acquire)) {                                                     \
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
+            if (e != hipSuccess) return (int)e;                                                                   \
+            opted_in[dev].store(true, std::memory_order_release);                                                 \
+        }                                                                                                         \
+        hipLaunchKernelGGL(kern, dim3(R / QB), dim3(WAVE * ADS_WAVES), lds, (hipStream_t)stream, (const T *)x1, q2, (const ST *)s2, R, C, \
+                           rounding, seed, offset, (OT *)y1, q, (ST *)s, mean, rstd);                             \
+        return (int)hipGetLastError();                                                                            \
+    } while (0)
 #define JF_ADD_OUT(T, ST)                                                                                         \
     do {                                                                                                          \
         if (y1_dtype == JF_FP_F32) JF_ADD(T, ST, float);                                                          \

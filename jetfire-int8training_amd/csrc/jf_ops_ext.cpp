@@ -340,11 +340,12 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor, OptTensor> add(const Tensor &x1, c
     c10::DeviceGuard guard(x1.device());
     Tensor y1 = fresh(x1.sizes(), x1.options().dtype(out_dtype));
     Tensor q = fresh(x1.sizes(), q2.options()), s = fresh(scale_shape(x1), s2.options());
-    Tensor rs, rq;
+    Tensor ws;
     OptTensor mean, rstd;
+    size_t nbytes = 0;
     if (with_stats) {
-        rs = fresh({C / QB, R}, x1.options().dtype(torch::kFloat32));          // part-major
-        rq = fresh_like(rs);
+        nbytes = jf_add_rowstats_workspace_bytes((int)R, (int)C);
+        if (nbytes) ws = scratch(x1, nbytes);
         mean = fresh(row_shape(x1), x1.options().dtype(torch::kFloat32));
         rstd = fresh_like(*mean);
     }
@@ -352,14 +353,13 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor, OptTensor> add(const Tensor &x1, c
     {
         pybind11::gil_scoped_release nogil;
         const jf_stream_t st = current_stream(x1);
-        check_rc(jf_add(x1.data_ptr(), xc, (const int8_t *)q2.data_ptr(), s2.data_ptr(), (int)R, (int)C, sc, (int)rounding, so.first,
-                        so.second, y1.data_ptr(), oc, (int8_t *)q.data_ptr(), s.data_ptr(), with_stats ? rs.data_ptr<float>() : nullptr,
-                        with_stats ? rq.data_ptr<float>() : nullptr, st),
-                 "add");
         if (with_stats)
-            check_rc(jf_rowstats_finish(rs.data_ptr<float>(), rq.data_ptr<float>(), (int)R, (int)(C / QB), (int)C,
-                                        mean->data_ptr<float>(), rstd->data_ptr<float>(), st),
-                     "rowstats_finish");
+            check_rc(jf_add_rowstats(x1.data_ptr(), xc, (const int8_t *)q2.data_ptr(), s2.data_ptr(), (int)R, (int)C, sc, (int)rounding, so.first,
+                                     so.second, y1.data_ptr(), oc, (int8_t *)q.data_ptr(), s.data_ptr(), mean->data_ptr<float>(),
+                                     rstd->data_ptr<float>(), nbytes ? ws.data_ptr() : nullptr, nbytes, st), "add");
+        else
+            check_rc(jf_add(x1.data_ptr(), xc, (const int8_t *)q2.data_ptr(), s2.data_ptr(), (int)R, (int)C, sc, (int)rounding, so.first,
+                            so.second, y1.data_ptr(), oc, (int8_t *)q.data_ptr(), s.data_ptr(), nullptr, nullptr, st), "add");
     }
     return std::make_tuple(y1, q, s, mean, rstd);
 }

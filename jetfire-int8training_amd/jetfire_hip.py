@@ -32,6 +32,7 @@ EXPORTS = [
     "jf_igemm_block_q_dequant", "jf_quantize_slabs", "jf_philox_rounds", "jf_block_colsum", "jf_block_colsum_workspace_bytes",
     "jf_attention_fwd", "jf_attention_bwd", "jf_quantize_many", "jf_rowstats_fp", "jf_wgrad_many", "jf_wgrad_many_workspace_bytes",
     "jf_layernorm_fwd_sums", "jf_attention_fwd_q", "jf_attention_bwd_q", "jf_igemm_block_q_add", "jf_linear_bwd", "jf_wgrad_many_dgrad", "jf_wgrad_many_finish",
+    "jf_add_rowstats", "jf_add_rowstats_workspace_bytes",
 ]
 
 _lib = None
@@ -83,6 +84,9 @@ def lib():
         L.jf_igemm_block_q_add.argtypes = [_p, _p, _p, _p, _p, _p, _p, _i, _i, _p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p]
         L.jf_linear_bwd.argtypes = [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _i, _u64, _u64, _p, _i, _i, _p, _sz, _p]
         L.jf_add.argtypes = [_p, _i, _p, _p, _i, _i, _i, _i, _u64, _u64, _p, _i, _p, _p, _p, _p, _p]
+        L.jf_add_rowstats.argtypes = [_p, _i, _p, _p, _i, _i, _i, _i, _u64, _u64, _p, _i, _p, _p, _p, _p, _p, _sz, _p]
+        L.jf_add_rowstats_workspace_bytes.argtypes = [_i, _i]
+        L.jf_add_rowstats_workspace_bytes.restype = _sz
         L.jf_block_colsum_workspace_bytes.argtypes = [_i, _i]
         L.jf_block_colsum_workspace_bytes.restype = _sz
         L.jf_block_colsum.argtypes = [_p, _p, _i, _i, _i, _p, _p, _sz, _p]
@@ -636,6 +640,26 @@ def add(x1, q2, s2, rounding=ROUND_TRUNC, with_stats=False, seed=None, offset=No
     check(lib().jf_add(_ptr(x1), _FP_CODE[x1.dtype], _ptr(q2), _ptr(s2), R, Cc, code, rounding, seed, offset,
                        _ptr(y1), _FP_CODE[out_dtype], _ptr(q), _ptr(s), _ptr(rs), _ptr(rq), _stream()))
     return (y1, q, s, rs, rq) if with_stats else (y1, q, s)
+
+
+def add_rowstats(x1, q2, s2, rounding=ROUND_TRUNC, seed=None, offset=None, out_dtype=torch.float32):
+    """add(..., with_stats=True) and rowstats_finish in one entry point: (y1, q, s, mean, rstd)."""
+    R, Cc, code = _block_tensor(q2, s2, "x2")
+    _need(x1, None, "x1")
+    if x1.dtype not in _FP_CODE or tuple(x1.shape) != (R, Cc):
+        raise RuntimeError("x1 must be a float tensor of the same shape as x2")
+    if out_dtype not in _FP_CODE:
+        raise RuntimeError("out_dtype must be float32, float16 or bfloat16")
+    seed, offset = _rng(rounding, R * Cc, seed, offset, x1.device)
+    y1 = torch.empty((R, Cc), dtype=out_dtype, device=x1.device)
+    q, s = torch.empty_like(q2), torch.empty_like(s2)
+    mean = torch.empty(R, dtype=torch.float32, device=x1.device)
+    rstd = torch.empty_like(mean)
+    nbytes = lib().jf_add_rowstats_workspace_bytes(R, Cc)
+    ws = torch.empty(nbytes, dtype=torch.int8, device=x1.device) if nbytes else None
+    check(lib().jf_add_rowstats(_ptr(x1), _FP_CODE[x1.dtype], _ptr(q2), _ptr(s2), R, Cc, code, rounding, seed, offset, _ptr(y1), _FP_CODE[out_dtype],
+                                _ptr(q), _ptr(s), _ptr(mean), _ptr(rstd), _ptr(ws), nbytes, _stream()))
+    return y1, q, s, mean, rstd
 
 
 def block_colsum(q, s):

@@ -235,6 +235,43 @@ def test_add(jf, oracle, dtype, mode):
     assert np.allclose(m, wy.mean(-1), atol=1e-5) and np.allclose(rstd.cpu().numpy(), 1 / np.sqrt(wy.var(-1)), rtol=1e-4)
 
 
+# one launch: one block, a last round that is not full, the widest row of few strips, the widest of many, as many strips as CUs; two launches:
+# the next width, the widest row and the next one, one strip more
+@pytest.mark.parametrize("R,C", [(32, 32), (64, 608), (96, 1152), (3072, 2048), (8192, 64), (96, 1184), (64, 2048), (3072, 2080), (8224, 64)])
+@pytest.mark.parametrize("x1,out,scale,mode", [(torch.float32, torch.bfloat16, torch.float16, "trunc"), (torch.bfloat16, torch.float32, torch.float32, "stochastic_trunc"),
+                                               (torch.float16, torch.float16, torch.float16, "nearest")])
+def test_add_with_finished_statistics(jf, R, C, x1, out, scale, mode):
+    """Bit for bit the addition and the finishing of its statistics, in place as well; NaN and infinities go where they go there."""
+    g = torch.Generator("cuda").manual_seed(R + C)
+    x = torch.randn((R, C), device="cuda", generator=g).to(x1)
+    x[0, 0], x[1, C - 1], x[2, 5] = float("nan"), float("inf"), float("-inf")
+    q2, s2 = jf.quantize(torch.randn((R, C), device="cuda", generator=g), scale_dtype=scale)
+    kw = dict(rounding=ROUND[mode], seed=7, offset=4, out_dtype=out)
+    y, q, s, rs, rq = jf.add(x, q2, s2, with_stats=True, **kw)
+    want = (y, q, s) + tuple(jf.rowstats_finish(rs, rq, C))
+    got = jf.add_rowstats(x, q2, s2, **kw)
+    for a, b, name in zip(got, want, ("sum", "codes", "scales", "mean", "rstd")):
+        assert torch.equal(a.view(torch.uint8) if a.dtype != torch.int8 else a, b.view(torch.uint8) if b.dtype != torch.int8 else b), name
+    L, code = jf.lib(), jf.SCALE_F16 if scale == torch.float16 else jf.SCALE_F32
+    nb = L.jf_add_rowstats_workspace_bytes(R, C)
+    ws, mean, rstd = torch.empty(max(nb, 16), dtype=torch.int8, device="cuda"), torch.empty(R, device="cuda"), torch.empty(R, device="cuda")
+    jf.check(L.jf_add_rowstats(jf._ptr(x), jf._FP_CODE[x1], jf._ptr(q2), jf._ptr(s2), R, C, code, ROUND[mode], 7, 4, jf._ptr(y), jf._FP_CODE[out],
+                               jf._ptr(q2), jf._ptr(s2), jf._ptr(mean), jf._ptr(rstd), jf._ptr(ws), nb, jf._stream()))
+    assert torch.equal(q2, want[1]) and torch.equal(s2, want[2]) and torch.equal(mean[3:], want[3][3:])
+
+
+def test_gelu_with_one_and_with_four_blocks_per_wave(jf):
+    """8192 blocks are the most that take a wave each; the rows of a taller tensor get the same bits four blocks to a wave."""
+    R, C = 4096, 2048
+    g = torch.Generator("cuda").manual_seed(3)
+    (q, s), (qg, sg) = (jf.quantize(torch.randn((R + 32, C), device="cuda", generator=g) * a) for a in (2.0, 1e-3))
+    for approx in (jf.GELU_ERF, jf.GELU_TANH):
+        for tall, cut in ((jf.gelu_fwd(q, s, approx, 5e-5), jf.gelu_fwd(q[:R], s[:R // 32], approx, 5e-5)),
+                          (jf.gelu_bwd(q, s, qg, sg, approx, ROUND["stochastic"], 9, 4),
+                           jf.gelu_bwd(q[:R], s[:R // 32], qg[:R], sg[:R // 32], approx, ROUND["stochastic"], 9, 4))):
+            assert torch.equal(tall[0][:R], cut[0]) and torch.equal(tall[1][:R // 32], cut[1])
+
+
 @pytest.mark.parametrize("R,C", [(64, 96), (96, 1600), (32, 2048), (64, 2080)])
 @pytest.mark.parametrize("x1_dtype,out_dtype,scale_dtype", [(torch.float32, torch.float32, torch.float32),
                                                             (torch.bfloat16, torch.bfloat16, torch.float16),
