@@ -1146,7 +1146,7 @@ __global__ __launch_bounds__(NT) void add_kernel(const T *x1, const int8_t *q2, 
     }
 }
 
-// add_kernel and rowstats_finish_kernel as one launch, bit for bit: a workgroup owns a 32-row strip (wave w: column blocks w, w + 16, ..., all
+// add_kernel and rowstats_finish_kernel as one launch, bit for bit: a workgroup owns a 32-row strip (each wave up to four adjacent blocks, all
 // of them requested at once), so that the partial sums of its rows never leave it (add_in_strips).
 constexpr int ADS_WAVES = 16, ADS_BPW = 4;
 template <typename T, typename ST, typename OT>
@@ -1156,15 +1156,15 @@ __global__ __launch_bounds__(WAVE * ADS_WAVES, 4) void add_strip_kernel(const T 
 {
     extern __shared__ __attribute__((aligned(16))) float lds_f[];  // partial sums [2][C/32][32], squares of a row [32], patches
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int SC = C / QB, rb = blockIdx.x, row = rb * QB + (lane >> 1);
+    const int SC = C / QB, rb = blockIdx.x, per = (SC + ADS_WAVES - 1) / ADS_WAVES, row = rb * QB + (lane >> 1);
     float *part = lds_f, *sq = part + 2 * SC * QB, *ypatch = sq + QB + wave * (QB * ADD_PITCH);
     float a[ADS_BPW][16];
     v4i c[ADS_BPW];
     float sc[ADS_BPW];
     static_for<0, ADS_BPW>([&](auto i_c) {
         constexpr int I = decltype(i_c)::value;
-        const int cb = wave + I * ADS_WAVES;
-        if (cb < SC) {
+        const int cb = wave * per + I;
+        if (I < per && cb < SC) {
             const size_t e0 = (size_t)row * C + cb * QB + (lane & 1) * 16;
             Load16<T>::run(x1 + e0, a[I]);
             c[I] = *reinterpret_cast<const v4i *>(q2 + e0);
@@ -1173,8 +1173,8 @@ __global__ __launch_bounds__(WAVE * ADS_WAVES, 4) void add_strip_kernel(const T 
     });
     static_for<0, ADS_BPW>([&](auto i_c) {
         constexpr int I = decltype(i_c)::value;
-        const int cb = wave + I * ADS_WAVES;
-        if (cb >= SC) return;                                      // uniform
+        const int cb = wave * per + I;
+        if (I >= per || cb >= SC) return;                                      // uniform
         const size_t e0 = (size_t)row * C + cb * QB + (lane & 1) * 16;
         float b[16];
         unpack16(c[I], sc[I], b);
@@ -1190,9 +1190,15 @@ __global__ __launch_bounds__(WAVE * ADS_WAVES, 4) void add_strip_kernel(const T 
         }
         store_block_rows(ypatch, b, y1 + (size_t)rb * QB * C + cb * QB, C, lane);
         float scale;
-        *reinterpret_cast<v4i *>(q + e0) = quantize16(b, 0.0f, rounding, seed, offset, e0, &scale);
+        c[I] = quantize16(b, 0.0f, rounding, seed, offset, e0, &scale);
+        if (per < 4) *reinterpret_cast<v4i *>(q + e0) = c[I];
         if (lane == 0) store_scale(s, rb * SC + cb, scale);
     });
+    if (per == 4 && wave * 4 < SC) {                               // four adjacent blocks: the codes in whole 128-byte lines
+        unsigned char *const lines = reinterpret_cast<unsigned char *>(ypatch);
+        static_for<0, ADS_BPW>([&](auto i_c) { group_put(lines, lane, decltype(i_c)::value, c[decltype(i_c)::value]); });
+        group_store_lines(lines, lane, q, rb, wave, C);
+    }
     __syncthreads();
     float acc = 0.0f;                                              // threads 0..31: sums, 32..63: squares, in ascending order
     if (threadIdx.x < 2 * QB) {
