@@ -129,9 +129,8 @@ constexpr int WBN = 1;
 // threads of a workgroup: with one block per wave, as many waves again that do nothing but load (see load_loop)
 constexpr int gemm_threads(int WBM, int WGM, int WGN) { return 64 * WGM * WGN * (WBM == 1 ? 2 : 1); }
 constexpr int TABLE_KB = 512;                        // K blocks a wave's table of scale products holds (WBM = 1)
-// LDS of a workgroup: the operand ring; per-wave scale and product patches or tables; from gelu_lds_at on what the GELU tables of the
-// epilogue need beyond those (WBM = 2: the forward's byte tables, 256 bytes per wave; WBM = 1: both, 1280 bytes).  Epilogues that go
-// through LDS use the ring.
+// LDS of a workgroup: the operand ring; per-wave scale and product patches or tables; from gelu_lds_at on the GELU tables of the epilogue where
+// they don't fit into those (WBM = 1: 1 KB per wave).  Epilogues that go through LDS use the ring.
 constexpr int SPLIT_GROUP = 8 * ROW_BYTES + 64;       // SPLIT: bytes from one 8-row group of a stage to the next
 constexpr int gelu_lds_at(int WBM, int WGM, int WGN, int NSTAGE)
 {
@@ -144,7 +143,7 @@ constexpr int SPLIT_RING = 6;                        // stages: at 0.23 us each,
 constexpr int SPLIT_LDS = SPLIT_RING_AT + SPLIT_RING * 12 * SPLIT_GROUP;
 constexpr int gemm_lds(int EPI, int WBM, int WGM, int WGN, int NSTAGE)
 {
-    const int tables = (WBM == 1 ? (EPI == EPI_QG || EPI == EPI_QB) * 1280 : (EPI == EPI_QG) * 256) * WGM * WGN;
+    const int tables = WBM == 1 ? (EPI == EPI_QG || EPI == EPI_QB) * 1024 * WGM * WGN : 0;
     const int used = gelu_lds_at(WBM, WGM, WGN, NSTAGE) + tables, patch = WGM * WGN * QB * EPI_LD * (int)sizeof(float);
     return used > patch ? used : patch;
 }
@@ -1173,9 +1172,11 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
     const int rrow = QUANT ? lane & 31 : lane >> 1, rcol = (QUANT ? lane >> 5 : lane & 1) * 16;
-    // GELU tables of the wave: its scale patch (nothing is on its way there any more) and, for the byte table, a piece of its own
-    float *const gelu_tab = SPLIT > 1 ? reinterpret_cast<float *>(ring_lds) + wave * 320 : TABLE ? reinterpret_cast<float *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 320 : reinterpret_cast<float *>(scale_patch);
-    int *const gelu_qtab = TABLE ? reinterpret_cast<int *>(gelu_tab + 256) : reinterpret_cast<int *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 64;
+    // GELU table of the wave: its scale patch (nothing is on its way there any more) or a piece of its own.  The forward's byte table is written
+    // over it: by then every lane has read its entries.
+    float *const gelu_tab = SPLIT > 1 ? reinterpret_cast<float *>(ring_lds) + wave * 256
+                          : TABLE ? reinterpret_cast<float *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 256 : reinterpret_cast<float *>(scale_patch);
+    int *const gelu_qtab = reinterpret_cast<int *>(gelu_tab);
     if (EPI == EPI_QG || EPI == EPI_QB) JF_WAIT_VMCNT(0);
     const float biasmax = (QUANT && p.biasmax) ? p.biasmax[0] : 0.0f;
     float gelu_f0 = 0.0f;                                     // gelu(+0), evaluated on the device like every table entry
@@ -1849,11 +1850,12 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs
     // 128x128 tiles would be alone on many of their CUs, and a SIMD's waves belong to workgroups that do not wait for each other.  us,
     // 128x128 | 64x128: 7168x768x768 (336 big tiles) 15.3 | 12.8, 8192x768x768 (384) 15.4 | 13.1, x3072 43.6 | 41.0, 768x8192x2048 (384) 30.3 |
     // 27.8, 3072x1024x4096 (192) 37.5 | 34.9, 2048x1600x1600 (208) 17.6 | 16.9, 1248x2304x768 (180) 10.7 | 10.3; two rounds of them: 2560x2560x2560
-    // (400) 37.1 | 47.4.  Not with the GELU forward behind it, whose byte tables leave room for two workgroups only; with its backward,
-    // the longest epilogue, above one big tile per CU: 2048x3072x768 (384) 22.0 | 19.8, 1248x3072x768 (240) 15.2 | 15.6.
-    if constexpr (EPI == EPI_Q || EPI == EPI_QB || EPI == EPI_QD || EPI == EPI_QA) {
+    // (400) 37.1 | 47.4.  With a GELU behind it, the longest epilogues, above one big tile per CU: backward 2048x3072x768 (384) 22.0 | 19.8,
+    // 1248x3072x768 (240) 15.2 | 15.6, forward 2048x3072x768 18.8 | 18.0, 3072x2048x512 (384) 16.1 | 14.9, 4096x1536x768 (384) 19.0 | 18.1, 1248x3072x768
+    // 13.9 | 14.0, 640x6400x1600 (250) 20.7 | 21.8.
+    if constexpr (EPI == EPI_Q || EPI == EPI_QB || EPI == EPI_QD || EPI == EPI_QA || EPI == EPI_QG) {
         const long tiles_n = (a.N + 127) / 128;
-        if ((a.M + 63) / 64 * tiles_n <= 3L * cu_count() && (EPI != EPI_QB || (a.M + 127) / 128 * tiles_n > cu_count()))
+        if ((a.M + 63) / 64 * tiles_n <= 3L * cu_count() && ((EPI != EPI_QB && EPI != EPI_QG) || (a.M + 127) / 128 * tiles_n > cu_count()))
             return launch_gemm_cfg<EPI, ST, 2, 1, 4, 2, 3, BKN>(a, st);
     }
     return launch_gemm_cfg<EPI, ST, 2, 2, 4, 2, 2, BKN>(a, st);

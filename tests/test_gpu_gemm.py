@@ -658,6 +658,13 @@ def test_both_gradients_with_tiles_that_two_waves_share(jf, R, C_in, C_out, f16)
         test_both_gradients_of_a_linear_layer_in_one_launch(jf, R, C_in, C_out, 0, f16, quantize)
 
 
+# 64x128 tiles with a GELU behind them: the fewest and the most big tiles that they take the place of, one row of tiles less (128x128), the last row
+# and column of tiles ragged
+@pytest.mark.parametrize("M,N,K", [(4096, 1056, 96), (2080, 2080, 32), (2016, 2976, 160), (2048, 2048, 64)])
+def test_gelu_in_the_64_row_tiles(jf, oracle, M, N, K):
+    test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K)
+
+
 # 425 tiles of 128x128 (825 of 64x128, which would not all be resident), the last row and column of them ragged: every ring fill
 @pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 288, 384, 416])
 def test_the_large_tiles_at_every_ring_fill(jf, oracle, K):
