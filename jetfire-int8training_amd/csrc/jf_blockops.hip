@@ -472,6 +472,10 @@ void gelu_bwd_kernel(const int8_t *qx, const ST *sx, const int8_t *qg, const ST 
 // STATS: mean and rstd are not given but follow from a residual add's partial row sums (rowsum, rowsq: [C/32][R]), added here
 // in the order of rowstats_finish_kernel and written by the workgroups of the first column blocks.  Every workgroup adds its
 // own 64 rows' sums again, 2 C/32 floats per row out of the L2: less than the launch of its own that this takes the place of.
+// The sums are what bounds it then, 42 MB at 8192x1600.  Workgroups are dealt round-robin to the 8 XCDs, so in plain order every
+// XCD fetched all rows' sums into its L2; with a row group's workgroups on one XCD each fetches an eighth.  us, plain order | runs per
+// XCD: 8192x1600 15.0 | 12.3 (8.4 without the sums), 12288x768 9.15 | 8.68; 4096x1024 (512 workgroups) 5.18 | 5.15, 1024x256 4.12 | 4.27:
+// few workgroups keep the plain order.  (24 or 32 terms on their way at once instead of 16 cost registers: 8192x1600 14.1 and 16.1.)
 constexpr int CW_ROWS = 2;
 struct RowSums {
     const float *rowsum, *rowsq;
@@ -485,7 +489,12 @@ __global__ __launch_bounds__(NT) void layernorm_fwd_kernel(const int8_t *q, cons
     __shared__ __attribute__((aligned(16))) unsigned char line_patches[2 * QB * LINE_PITCH];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int SC = C / QB, RB = R / QB, S4 = (SC + WPB - 1) / WPB;
-    const int cg = blockIdx.x % S4, grp = blockIdx.x / S4;
+    int work = blockIdx.x;
+    if (STATS && gridDim.x > 512) {                            // one contiguous run of the work per XCD
+        const int per = gridDim.x >> 3, rem = gridDim.x & 7, xcd = blockIdx.x & 7;
+        work = xcd * per + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+    }
+    const int cg = work % S4, grp = work / S4;
     GroupLineStore lines(line_patches, lane, wave);
     // a wave of the last, partial group of column blocks computes its neighbour's block again (and keeps none of it):
     // it is needed for the whole-line stores of the group's rows

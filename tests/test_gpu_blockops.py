@@ -509,6 +509,11 @@ def test_layernorm_from_partial_row_sums(jf, oracle, R, C, f16, with_beta):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("R,C", [(10912, 384), (4096, 1056)])    # 513 workgroups, one XCD's run longer than the others', a half group of rows; 576, an eighth each
+def test_layernorm_from_partial_row_sums_with_a_run_per_xcd(jf, oracle, R, C):
+    test_layernorm_from_partial_row_sums(jf, oracle, R, C, True, True)
+
+
 def test_results_are_seen_by_a_dispatch_mode():
     """Results are allocated without the dispatcher, except where something listens to it; the values do not depend on it."""
     from Nonlinear import int8_quantize
