@@ -4,6 +4,7 @@
   libjetfire_prof.so       hipcc, gfx950 only: measurement aids (include/jetfire_prof.h): the phase-recording build of
                            the GEMM kernel (the same source, -DJF_PROF_LIB) and register-only calibration loops;
                            used by the benchmark, not by the operators
+  libjetfire_tls.so        one thread-local variable, loaded by the extension at its first launch (csrc/jf_tls.c)
   BlockQuantizeCUDA*.so    host C++ (g++): the PyTorch extension with the reference's module name and
                            function signatures (JetfireGEMMKernel/setup.py:13, bindings.cpp:6-35), plus the
                            submodule BlockQuantizeCUDA.jetfire with every other operator of the path; it is
@@ -68,6 +69,7 @@ def build_hip():
     return HIP_LIB
 
 
+TLS_LIB = os.path.join(HERE, "libjetfire_tls.so")
 TORCH_SOURCES = ["bqc_ext.cpp", "jf_ops_ext.cpp", "jf_block_ext.cpp"]
 
 
@@ -97,9 +99,10 @@ def build_torch():
     for cmd, obj, proc in jobs:
         if proc.wait() != 0:
             raise subprocess.CalledProcessError(proc.returncode, cmd)
+    _run(["gcc", "-O2", "-Wall", "-fPIC", "-shared", "-o", TLS_LIB, os.path.join(CSRC, "jf_tls.c")])
     _run(["g++", "-shared", "-o", out] + [obj for _, obj, _ in jobs] + [
         "-L" + torch_lib, "-L" + HERE, "-L" + os.path.join(ROCM, "lib"),
-        "-ltorch", "-ltorch_cpu", "-lc10", "-ltorch_hip", "-lc10_hip", "-ltorch_python", "-ljetfire_hip", "-lamdhip64",
+        "-ltorch", "-ltorch_cpu", "-lc10", "-ltorch_hip", "-lc10_hip", "-ltorch_python", "-ljetfire_hip", "-lamdhip64", "-ldl",
         "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + torch_lib, "-Wl,-rpath," + os.path.join(ROCM, "lib"),
     ])
     return out

@@ -3,6 +3,8 @@ import ctypes
 import os
 import re
 
+import pytest
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
@@ -52,6 +54,26 @@ def test_measurement_library_is_separate(jf):
     for n in names:
         assert hasattr(prof, n), n
         assert not hasattr(main, n), f"{n} belongs to the measurement library"
+
+
+def test_the_thread_local_library_is_read_by_any_thread():
+    import threading
+    lib = ctypes.CDLL(os.path.join(ROOT, "jetfire-int8training_amd", "libjetfire_tls.so"))
+    threads = [threading.Thread(target=lib.jf_tls_read) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    lib.jf_tls_read()
+
+
+@pytest.mark.gpu
+def test_the_extension_loads_the_thread_local_library_at_its_first_launch():
+    import torch
+    import Nonlinear
+    q, s = Nonlinear.int8_quantize(torch.ones(32, 32, device="cuda"), 32)
+    assert (q == 127).all() and s.item() == torch.tensor(1 / 127, dtype=torch.float16).item()
+    assert "libjetfire_tls.so" in open("/proc/self/maps").read()
 
 
 def test_argument_errors_without_gpu(jf):
