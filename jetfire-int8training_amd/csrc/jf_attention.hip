@@ -25,7 +25,7 @@
 // 27.7 | 23.6; 4 x 256 x 4 7.8 | 7.0, 21.1 | 18.4.  Errors against float64 are the same before and with that, the gradients of keys
 // that rise along the sequence 2 % smaller.
 // The gradient is two kernels (dQ by query, dK/dV by key: 12 + 16 MFMAs per tile instead of 20) so that every sum has one owner and a
-// fixed order: no atomics, the same bits on every run.
+// fixed order: no atomics, the same bits on every run.  Where few workgroups leave CUs idle the two run in one launch.
 #include "jf_device.hpp"
 
 #pragma clang diagnostic ignored "-Winline-asm"     // M0 appears in clobber lists on purpose
@@ -43,7 +43,7 @@ struct AttnArgs {
     half_t *out;                    // [B*T, C]                                           (forward)
     half_t *gq, *gk, *gv;           // [B*T, ldg]                                         (gradient kernels)
     float *lse;                     // [B*H, T]: log2 of the row sum of exp2(scale * log2(e) * s)
-    float *delta;                   // [B*H, T]: minus the sum over D of o * go (left by the dQ kernel, read by the dK/dV kernel)
+    float *delta;                   // [B*H, T]: minus the sum over D of o * go (left by dQ, read by the dK/dV kernel)
     int ld, ldg, B, H, T;
     float scale;                    // of the scores
     int8_t *cq;                     // codes and scales of the result [B*T, C] or of the gradients [B*T, 3C] (kernels with QUANT)
@@ -63,9 +63,9 @@ constexpr int WG_ROWS = 32 * NW;
 
 // Workgroup -> (head, block of rows).  Workgroups are dealt to the 8 XCDs in turn: the blocks of one head stay on one XCD
 // (its K and V are read by all of them), and the longest blocks start first.
-__device__ __forceinline__ bool attn_work(const AttnArgs &a, int nblk, bool longest_is_last, int &bh, int &blk)
+__device__ __forceinline__ bool attn_work(const AttnArgs &a, int wg, int nblk, bool longest_is_last, int &bh, int &blk)
 {
-    const int per = (a.B * a.H + 7) / 8, x = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int per = (a.B * a.H + 7) / 8, x = wg & 7, j = wg >> 3;
     bh = (j % per) * 8 + x;
     blk = j / per;
     if (longest_is_last) blk = nblk - 1 - blk;
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_fwd_kernel(AttnArgs a)
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int nblk = (a.T + WG_ROWS - 1) / WG_ROWS;
     int bh, blk;
-    if (!attn_work(a, nblk, true, bh, blk)) return;
+    if (!attn_work(a, blockIdx.x, nblk, true, bh, blk)) return;
     const int b = bh / a.H, head = bh - b * a.H;
     const size_t first = (size_t)b * a.T * a.ld + (size_t)head * D;
     const half_t *kp = a.k + first, *vp = a.v + first;
@@ -360,16 +360,14 @@ __global__ __launch_bounds__(64 * NW, 4) void attn_fwd_kernel(AttnArgs a)
 // 25 heads 131.6 | 129.4 (on another card than the figures above).  But where it fills the chip, the chip then lowers its clock for everything around it (1.99 -> 1.91 GHz in the
 // GEMMs of a training step, read from their clock counters, for as long as the steps go on): three GPT-2 XL blocks 5809 | 5959 us a step,
 // three of GPT-2 small 2860 | 2900, three 1024 wide over 8 x 512 tokens 1641 | 1685; two blocks 768 wide over 2 x 1024 tokens 614 | 606.
-// So it is taken while no CU has more than one workgroup of it.
-template <int D, bool QUANT, bool EARLY>
-__global__ __launch_bounds__(64 * NW, EARLY ? 3 : 4) void attn_dq_kernel(AttnArgs a)
+// So it is taken while no CU has more than one workgroup of it, and in attn_grad_kernel.
+template <int D, bool QUANT, bool EARLY> __device__ __forceinline__ void attn_dq(const AttnArgs &a, int wg, unsigned char *smem)
 {
     using IO = TileIO<D>;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int nblk = (a.T + WG_ROWS - 1) / WG_ROWS;
     int bh, blk;
-    if (!attn_work(a, nblk, true, bh, blk)) return;
+    if (!attn_work(a, wg, nblk, true, bh, blk)) return;
     const int b = bh / a.H, head = bh - b * a.H;
     const size_t first = (size_t)b * a.T * a.ld + (size_t)head * D;
     const half_t *kp = a.k + first, *vp = a.v + first;
@@ -456,17 +454,19 @@ __global__ __launch_bounds__(64 * NW, EARLY ? 3 : 4) void attn_dq_kernel(AttnArg
     }
 }
 
-// dK and dV by blocks of keys
-template <int D, bool QUANT>
-__global__ __launch_bounds__(64 * NW, 2) void attn_dkv_kernel(AttnArgs a)
+// dK and dV by blocks of keys.  OWN: delta is not read but formed here, for all queries of the block's tiles before the first of them (the
+// same operations in the same order as in attn_dq: the same bits).
+constexpr int DKV_STAT = 2 * 2 * ATT_ROWS * 4;                 // bytes of LDS behind the tiles: lse, delta of a tile's queries, twice
+constexpr int OWN_ROWS = 4096;                                 // queries of a sequence with OWN: 16 KB more
+template <int D, bool QUANT, bool OWN> __device__ __forceinline__ void attn_dkv(const AttnArgs &a, int wg, unsigned char *smem)
 {
     using IO = TileIO<D>;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[2][2 * IO::TILE];
-    __shared__ __attribute__((aligned(16))) float stat[2][2][ATT_ROWS];        // lse, delta of the tile's queries
+    float(*const stat)[2][ATT_ROWS] = reinterpret_cast<float(*)[2][ATT_ROWS]>(smem + 4 * IO::TILE);
+    float *const own = reinterpret_cast<float *>(smem + 4 * IO::TILE + DKV_STAT);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int nblk = (a.T + WG_ROWS - 1) / WG_ROWS;
     int bh, blk;
-    if (!attn_work(a, nblk, false, bh, blk)) return;
+    if (!attn_work(a, wg, nblk, false, bh, blk)) return;
     const int b = bh / a.H, head = bh - b * a.H;
     const size_t first = (size_t)b * a.T * a.ld + (size_t)head * D;
     const half_t *qp = a.q + first, *gp = a.go + (size_t)b * a.T * (a.H * D) + (size_t)head * D;
@@ -486,8 +486,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dkv_kernel(AttnArgs a)
             const int r = t * ATT_ROWS + (int)l;
             const unsigned off = (unsigned)(r < a.T ? r : a.T - 1) * 4u, dst = stat_lds + (t & 1) * (2 * ATT_ROWS * 4);
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(lsep), "s"(dst) : "memory", "m0");
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-                         ::"v"(off), "s"(dlp), "s"(dst + ATT_ROWS * 4) : "memory", "m0");
+            if constexpr (!OWN)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                             ::"v"(off), "s"(dlp), "s"(dst + ATT_ROWS * 4) : "memory", "m0");
         }
     };
     load(t0);
@@ -500,6 +501,25 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dkv_kernel(AttnArgs a)
             vv[kk] = *reinterpret_cast<const h8 *>(vs + 16 * kk);
         }
     }
+    if constexpr (OWN) {
+        for (int r = t0 * ATT_ROWS + 32 * wave; r < a.T; r += 32 * NW) {
+            const size_t row = ((size_t)b * a.T + r + (lane & 31)) * (a.H * D) + head * D + 8 * h;
+            h8 o[D / 16], go[D / 16];
+            float dl = 0.0f;
+#pragma unroll
+            for (int kk = 0; kk < D / 16; ++kk) {
+                go[kk] = *reinterpret_cast<const h8 *>(a.go + row + 16 * kk);
+                o[kk] = *reinterpret_cast<const h8 *>(a.o + row + 16 * kk);
+            }
+#pragma unroll
+            for (int kk = 0; kk < D / 16; ++kk)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) dl = __builtin_fmaf((float)o[kk][j], (float)go[kk][j], dl);
+            dl = half_sum(dl);
+            if (h == 0) own[r - t0 * ATT_ROWS + (lane & 31)] = -dl;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // (the barrier is the first tile's)
+    }
     const float c = a.scale * 1.44269504f;
     v16f dk[D / 32], dv[D / 32];
 #pragma unroll
@@ -510,7 +530,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dkv_kernel(AttnArgs a)
         attn_tile_ready();
         if (t + 1 < nt) load(t + 1);
         const typename IO::At at = io.at(lds + (t & 1) * 2 * IO::TILE);
-        const float *st_l = stat[t & 1][0], *st_d = stat[t & 1][1];
+        const float *st_l = stat[t & 1][0], *st_d = OWN ? own + (t - t0) * ATT_ROWS : stat[t & 1][1];
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub) {
             const int q0 = t * ATT_ROWS + sub * ATT_SUB;
@@ -578,6 +598,31 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dkv_kernel(AttnArgs a)
     }
 }
 
+template <int D, bool QUANT, bool EARLY> __global__ __launch_bounds__(64 * NW, EARLY ? 3 : 4) void attn_dq_kernel(AttnArgs a)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char smem[4 * TileIO<D>::TILE];
+    attn_dq<D, QUANT, EARLY>(a, blockIdx.x, smem);
+}
+template <int D, bool QUANT> __global__ __launch_bounds__(64 * NW, 2) void attn_dkv_kernel(AttnArgs a)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char smem[4 * TileIO<D>::TILE + DKV_STAT];
+    attn_dkv<D, QUANT, false>(a, blockIdx.x, smem);
+}
+// Both in one launch: dK and dV first, the longer of the two.  Where few workgroups leave most of the chip idle each is as long as its
+// longest chain of tiles, so side by side they take little more than one of them; the price is that dK/dV forms delta itself (a pass over o and
+// its gradient) and dQ runs with dK/dV's 190 registers.  us with codes, two launches | one, by workgroups of each: 4 heads of 256 rows (8) 18.3 | 12.6, 16 of
+// 256 (32) 18.6 | 12.8, 32 wide 13.0 | 8.8, 36 of 416 (144) 24.2 | 19.5, 24 of 1024 (192) 44.6 | 36.8, 4 of 2048 (64) 72.7 | 55.0, 8 of 4096 (256) 134.5 |
+// 115.7, 36 of 1024 (288) 48.7 | 37.1, 48 of 1024 (384) 51.0 | 46.6, 96 of 512 (384) 34.9 | 31.9; beyond one and a half per CU 60 of 1024 (480)
+// 57.6 | 57.8, 144 of 416 (576) 36.6 | 37.2, 144 of 1024 (1152) 106.0 | 117.5, 200 of 1024 (1600) 141.7 | 158.8.  In a training step (three blocks 768 wide, 288 and
+// 384 workgroups) 1156 | 1114, 1293 | 1259, with 8 x 512 tokens 1225 | 1212.
+template <int D, bool QUANT> __global__ __launch_bounds__(64 * NW, 2) void attn_grad_kernel(AttnArgs a)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char smem[4 * TileIO<D>::TILE + DKV_STAT + OWN_ROWS * 4];
+    const int half = gridDim.x / 2, wg = blockIdx.x;
+    if (wg < half) attn_dkv<D, QUANT, true>(a, wg, smem);
+    else attn_dq<D, QUANT, true>(a, wg - half, smem);
+}
+
 static int attn_check(const void *q, const void *k, const void *v, int ld, int B, int H, int T, int D, float scale)
 {
     if (!q || !k || !v) return JF_ERR_NULL;
@@ -590,15 +635,18 @@ static int attn_check(const void *q, const void *k, const void *v, int ld, int B
     return device_is_gfx950() ? JF_OK : JF_ERR_DEVICE;
 }
 
-static void attn_launch(void (*kernel)(AttnArgs), const AttnArgs &a, hipStream_t st)
+static void attn_launch(void (*kernel)(AttnArgs), const AttnArgs &a, hipStream_t st, unsigned parts = 1)
 {
     const unsigned grid = 8u * ((a.B * a.H + 7) / 8) * ((a.T + WG_ROWS - 1) / WG_ROWS);
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * NW), 0, st, a);
+    hipLaunchKernelGGL(kernel, dim3(parts * grid), dim3(64 * NW), 0, st, a);
 }
-template <int D, bool QUANT> static void attn_launch_dq(const AttnArgs &a, hipStream_t st)
+template <int D, bool QUANT> static void attn_launch_grad(const AttnArgs &a, hipStream_t st)
 {
-    const bool alone = (long)a.B * a.H * ((a.T + WG_ROWS - 1) / WG_ROWS) <= cu_count();   // (see the kernel)
+    const long wgs = (long)a.B * a.H * ((a.T + WG_ROWS - 1) / WG_ROWS), cus = cu_count();
+    if (2 * wgs <= 3 * cus && a.T <= OWN_ROWS) return attn_launch(attn_grad_kernel<D, QUANT>, a, st, 2);   // (see the kernels)
+    const bool alone = wgs <= cus;
     attn_launch(alone ? attn_dq_kernel<D, QUANT, true> : attn_dq_kernel<D, QUANT, false>, a, st);
+    attn_launch(attn_dkv_kernel<D, QUANT>, a, st);
 }
 
 }  // namespace jf
@@ -636,13 +684,8 @@ static int attention_bwd(const void *q, const void *k, const void *v, int ld, co
     a.gq = (half_t *)gq; a.gk = (half_t *)gk; a.gv = (half_t *)gv; a.ldg = ldg; a.B = B; a.H = H; a.T = T; a.scale = scale;
     a.cq = codes; a.cs = (half_t *)scales; a.seed = seed; a.offset = offset;
     hipStream_t st = (hipStream_t)stream;
-    if (D == 64) {
-        codes ? attn_launch_dq<64, true>(a, st) : attn_launch_dq<64, false>(a, st);
-        attn_launch(codes ? attn_dkv_kernel<64, true> : attn_dkv_kernel<64, false>, a, st);
-    } else {
-        codes ? attn_launch_dq<32, true>(a, st) : attn_launch_dq<32, false>(a, st);
-        attn_launch(codes ? attn_dkv_kernel<32, true> : attn_dkv_kernel<32, false>, a, st);
-    }
+    if (D == 64) codes ? attn_launch_grad<64, true>(a, st) : attn_launch_grad<64, false>(a, st);
+    else codes ? attn_launch_grad<32, true>(a, st) : attn_launch_grad<32, false>(a, st);
     return (int)hipGetLastError();
 }
 

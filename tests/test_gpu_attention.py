@@ -177,3 +177,24 @@ def test_scores_of_minus_infinity_count_for_nothing(D, keys):
     finite = want.isfinite().all(1)
     assert finite.sum() >= 64 and not out.cpu()[~finite].isfinite().any()
     assert rel(out.cpu()[finite], want[finite]) < 1e-3
+
+
+# both gradients in one launch (up to one and a half workgroups per CU, sequences of up to 4096 rows) against the two launches that many copies
+# of the same sequences take: one workgroup, waves without rows, ragged last tiles, the most workgroups, the longest sequence; and one row block more
+@pytest.mark.parametrize("B,H,T,D,copies", [(1, 1, 32, 64, 385), (1, 3, 96, 32, 130), (3, 4, 416, 64, 9), (3, 16, 1024, 64, 2), (2, 1, 4096, 32, 7), (1, 1, 4128, 64, 1)])
+def test_both_gradients_in_one_launch(B, H, T, D, copies):
+    import BlockQuantizeCUDA as BQC
+    jf, C = BQC.jetfire, H * D
+    print(f"case B={B} H={H} T={T} D={D}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    qkv = torch.randn(B * T, 3 * C, device="cuda", generator=gen).half()
+    g = (torch.randn(B * T, C, device="cuda", generator=gen) * 1e-2).half()
+    out, lse = jf.attention_fwd(*qkv.split(C, dim=1), B, H)
+    grads = jf.attention_bwd(*qkv.split(C, dim=1), out, lse, g, B, H)
+    qg, sg = jf.attention_bwd_q(*qkv.split(C, dim=1), out, lse, g, B, H, 3, 40)
+    wq, ws, _ = jf.quantize(grads, jf.ROUND_STOCHASTIC, torch.float16, False, 0.0, 3, 40)
+    assert torch.equal(qg, wq) and torch.equal(sg, ws)
+    many = jf.attention_bwd(*qkv.repeat(copies, 1).split(C, dim=1), out.repeat(copies, 1), lse.repeat(copies, 1).reshape(-1, T).contiguous(),
+                            g.repeat(copies, 1), copies * B, H)
+    for part in many.split(B * T):
+        assert torch.equal(part, grads)
