@@ -805,7 +805,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         // K blocks 2 pair, 2 pair + 1 of a stage into register set `pair`; extra: run-time offsets of operands and products
         auto fetch_pair = [&](auto pair_c, auto slot_c, unsigned extra, unsigned extra_tab) {
             constexpr int PAIR = decltype(pair_c)::value, SLOT = decltype(slot_c)::value, SB = SLOT * STAGE_BYTES;
-            static_assert(SPLIT > 1 || NSTAGE * STAGE_BYTES <= 65536, "offsets of 16 bits");
+            static_assert(SPLIT > 1 || (NSTAGE - 1) * STAGE_BYTES + (BKN ? (KB_STAGE - 1) * 4096 + 1024 : 0) < 65536, "offsets of 16 bits");
             v2f &t = pr[PAIR];
             const unsigned pt = tab + extra_tab;
             asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(t) : "v"(pt), "n"(SLOT * KB_STAGE * 4 + 8 * PAIR));
@@ -1822,6 +1822,16 @@ static void wgrad_group_plan(int n, const int *M, const int *N, int K, WgradPlan
 // 6.1 | 6.1, x2304 10.8 | 9.5; with two per CU 1248x768x768 (468) 5.8 | 6.5, 1024x1024x1024 (512) 6.6 | 7.4, 1280x768x2304 (480) 10.4 | 11.2.
 static long split_tiles(int M, int N) { return (long)(M / QB) * ((N + 63) / 64); }
 static bool split_tiles_resident(int M, int N, int K) { return K <= TABLE_KB * QB && split_tiles(M, N) <= (long)cu_count(); }
+// 64x128 tiles, one block per wave (eight waves that multiply, eight that load): where one workgroup per CU holds them all, but not one of 32x128
+// each.  Both put two waves that multiply on a SIMD, but this one loads 6 KB per K block instead of 10, and what a CU can load is what
+// two workgroups of 32x128 wait for.  us, 32x128 | these: 2048x768x768 7.25 | 6.98, x3072 16.6 | 15.7, 864x1824x3200 (210) 17.5 | 15.9, B as [K,N] 21.0 | 17.5,
+// 640x3072x1600 (240) 12.3 | 10.9, 1024x2048x3200 (256) 19.9 | 17.9, 1664x768x768 (156) 7.19 | 6.64, 4128x256x768 (130) 7.08 | 6.78, 1056x1024x96 (136)
+// 4.62 | 4.51, x3072 15.7 | 16.0.  A ring three deep instead of two: 2048x768x768 7.00, x3072 16.6, 1024x2048x3200 18.7.
+static bool tall_tiles_resident(int M, int N, int K)
+{
+    const long cus = cu_count(), cols = (N + 127) / 128;
+    return K <= TABLE_KB * QB && (M + 63) / 64 * cols <= cus && (M + 31) / 32 * cols > cus;
+}
 static bool small_tiles_resident(int M, int N, int K)          // 32x128 tiles, two workgroups per CU
 {
     return K <= TABLE_KB * QB && (long)((M + 31) / 32) * ((N + 127) / 128) <= 2L * cu_count();
@@ -1840,6 +1850,8 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs
 {
     if constexpr (EPI != EPI_S32) {
         if constexpr (EPI != EPI_FP) { if (split_tiles_resident(a.M, a.N, a.K)) return launch_gemm_split<EPI, ST, BKN>(a, st); }
+        if (a.splits <= 1 && tall_tiles_resident(a.M, a.N, a.K))
+            return launch_gemm_cfg<EPI, ST, 1, 2, 4, 2, 1, BKN>(a, st);
         if (a.splits <= 1 && small_tiles_resident(a.M, a.N, a.K))
             return launch_gemm_cfg<EPI, ST, 1, 1, 4, 3, 2, BKN>(a, st);
     }

@@ -642,6 +642,25 @@ def test_tiles_whose_blocks_two_waves_share(jf, oracle, M, N, K):
     test_quantised_with_residual_addition(jf, oracle, M, N, K, torch.bfloat16, torch.float32, True, True)
 
 
+# 64x128 tiles with one block per wave (up to one per CU, more than one of 32x128 each): few, the last row of them half empty, at fills of the two-deep
+# ring and lengths of its last stage; many, columns that end inside a tile; all 256; one row of tiles more
+@pytest.mark.parametrize("M,N,K", [(1056, 1024, k) for k in (32, 96, 128, 160, 288, 416)] + [(1760, 1056, 448), (2048, 1024, 64), (2080, 1024, 96)])
+def test_tiles_of_64_rows_with_one_block_per_wave(jf, oracle, M, N, K):
+    test_both_tile_sizes_at_every_ring_fill(jf, oracle, M, N, K)
+    test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K)       # (every other epilogue)
+    test_quantised_with_residual_addition(jf, oracle, M, N, K, torch.bfloat16, torch.float32, True, True)
+
+
+def test_the_longest_row_of_the_tiles_of_64_rows(jf):
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    a, sa = jf.quantize(torch.randn(1056, 16384, device="cuda", generator=gen))
+    b, sb = jf.quantize(torch.randn(1024, 16384, device="cuda", generator=gen))
+    q, s = jf.igemm_block_q(a, b, sa.t().contiguous(), sb.t().contiguous(), jf.B_NK)
+    for r in range(0, 1056, 352):                                # (parts of 32x64 tiles)
+        qp, sp = jf.igemm_block_q(a[r:r + 352], b, sa[r // 32:r // 32 + 11].t().contiguous(), sb.t().contiguous(), jf.B_NK)
+        assert torch.equal(q[r:r + 352], qp) and torch.equal(s[r // 32:r // 32 + 11], sp)
+
+
 # the residual addition in the epilogue of every larger tile: 128x128 with ragged rows and columns, both sizes in one launch, 64x128; one K block
 # and a short last stage
 @pytest.mark.parametrize("M,N,K,x1,y", [(2080, 3104, 32, torch.float32, torch.float32), (2080, 3104, 160, torch.bfloat16, torch.bfloat16),
