@@ -49,6 +49,29 @@ template <> struct Load16<__bf16> {
     }
 };
 
+// acc + p[0] + p[stride] + ... of n terms in ascending order, STEP of them on their way at once.  (A loop that the compiler unrolls leaves a
+// remainder that waits for every term by itself.  Absent terms count as +0, which changes no bit of a sum that starts from +0.)
+template <int STEP> __device__ __forceinline__ float sum_ascending(const float *p, int n, size_t stride)
+{
+    float acc = 0.0f;
+    int j = 0;
+    for (; j + STEP <= n; j += STEP) {
+        float v[STEP];
+#pragma unroll
+        for (int i = 0; i < STEP; ++i) v[i] = p[(size_t)(j + i) * stride];
+#pragma unroll
+        for (int i = 0; i < STEP; ++i) acc = acc + v[i];
+    }
+    if (j < n) {
+        float v[STEP];
+#pragma unroll
+        for (int i = 0; i < STEP; ++i) v[i] = p[(size_t)(j + i < n ? j + i : n - 1) * stride];
+#pragma unroll
+        for (int i = 0; i < STEP; ++i) acc = acc + (j + i < n ? v[i] : 0.0f);
+    }
+    return acc;
+}
+
 __device__ __forceinline__ void store16_f32(float *p, const float x[16])
 {
 #pragma unroll
@@ -268,8 +291,10 @@ template <typename T, typename ST> __global__ __launch_bounds__(NT) void quantiz
 }
 
 // Mean and 1/sqrt(biased variance) of the rows of a floating tensor (the LayerNorm statistics of a stack's input,
-// qmodel.py:429-430: two reductions of torch and a square root there).  One wave per row; the second pass over the row, for
-// the variance about the mean, comes out of the caches.
+// qmodel.py:429-430: two reductions of torch and a square root there).  One wave per row.  What bounds it is the
+// round trips of a row's pieces: rows of three to eight pieces are read once, all of them at once, and held for the variance about the mean (us, piece by
+// piece and twice | so: 8192x1600 float 16.3 | 9.5, bfloat16 6.2 | 5.0, 12288x768 float 7.8 | 6.4); shorter ones gain nothing (1024x256 2.4 | 2.7) and are
+// read twice like longer ones, the second time out of the caches.
 template <typename T> __global__ __launch_bounds__(NT) void rowstats_fp_kernel(const T *x, int R, int C, float *mean, float *rstd)
 {
     const int lane = threadIdx.x & 63, row = blockIdx.x * WPB + (threadIdx.x >> 6);
@@ -282,20 +307,42 @@ template <typename T> __global__ __launch_bounds__(NT) void rowstats_fp_kernel(c
 #pragma unroll
         for (int i = 0; i < PER; ++i) f[i] = (float)t[i];
     };
-    float s = 0.0f;
-    for (int c = lane * PER; c < C; c += WAVE * PER) {
-        float f[PER];
-        piece(c, f);
+    float s = 0.0f, v = 0.0f, mu;
+    constexpr int HELD = 8;
+    if (C > 2 * WAVE * PER && C <= HELD * WAVE * PER) {
+        v4i t[HELD];
+        const int whole = C / (WAVE * PER);                        // pieces that every lane has; of the next one the first lanes
+        const bool more = (whole * WAVE + lane) * PER < C;
 #pragma unroll
-        for (int i = 0; i < PER; ++i) s = s + f[i];
-    }
-    const float mu = wave_sum(s) / (float)C;
-    float v = 0.0f;
-    for (int c = lane * PER; c < C; c += WAVE * PER) {
-        float f[PER];
-        piece(c, f);
+        for (int k = 0; k < HELD; ++k)
+            if (k < whole || (k == whole && more)) t[k] = *reinterpret_cast<const v4i *>(p + (k * WAVE + lane) * PER);
 #pragma unroll
-        for (int i = 0; i < PER; ++i) { const float d = f[i] - mu; v = __builtin_fmaf(d, d, v); }
+        for (int k = 0; k < HELD; ++k)
+            if (k < whole || (k == whole && more)) {
+#pragma unroll
+                for (int i = 0; i < PER; ++i) s = s + (float)reinterpret_cast<const T *>(&t[k])[i];
+            }
+        mu = wave_sum(s) / (float)C;
+#pragma unroll
+        for (int k = 0; k < HELD; ++k)
+            if (k < whole || (k == whole && more)) {
+#pragma unroll
+                for (int i = 0; i < PER; ++i) { const float d = (float)reinterpret_cast<const T *>(&t[k])[i] - mu; v = __builtin_fmaf(d, d, v); }
+            }
+    } else {
+        for (int c = lane * PER; c < C; c += WAVE * PER) {
+            float f[PER];
+            piece(c, f);
+#pragma unroll
+            for (int i = 0; i < PER; ++i) s = s + f[i];
+        }
+        mu = wave_sum(s) / (float)C;
+        for (int c = lane * PER; c < C; c += WAVE * PER) {
+            float f[PER];
+            piece(c, f);
+#pragma unroll
+            for (int i = 0; i < PER; ++i) { const float d = f[i] - mu; v = __builtin_fmaf(d, d, v); }
+        }
     }
     const float var = wave_sum(v) / (float)C;
     if (lane == 0) { mean[row] = mu; rstd[row] = 1.0f / __builtin_sqrtf(var); }
@@ -475,7 +522,8 @@ void gelu_bwd_kernel(const int8_t *qx, const ST *sx, const int8_t *qg, const ST 
 // The sums are what bounds it then, 42 MB at 8192x1600.  Workgroups are dealt round-robin to the 8 XCDs, so in plain order every
 // XCD fetched all rows' sums into its L2; with a row group's workgroups on one XCD each fetches an eighth.  us, plain order | runs per
 // XCD: 8192x1600 15.0 | 12.3 (8.4 without the sums), 12288x768 9.15 | 8.68; 4096x1024 (512 workgroups) 5.18 | 5.15, 1024x256 4.12 | 4.27:
-// few workgroups keep the plain order.  (24 or 32 terms on their way at once instead of 16 cost registers: 8192x1600 14.1 and 16.1.)
+// few workgroups keep the plain order.  (24 or 32 terms on their way at once instead of 16 cost registers: 8192x1600 14.1 and 16.1.)  The
+// last ones, up to 15, at once as well: 1248x768 4.66 -> 4.22, 256x864 4.75 -> 4.10, 12288x768 8.62 -> 8.27, 8192x1600 11.9 -> 12.0.
 constexpr int CW_ROWS = 2;
 struct RowSums {
     const float *rowsum, *rowsq;
@@ -526,8 +574,7 @@ __global__ __launch_bounds__(NT) void layernorm_fwd_kernel(const int8_t *q, cons
         float acc = 0.0f;
         if (which < 2) {
             const float *src = (which ? rsum.rowsq : rsum.rowsum) + (row < R ? row : R - 1);
-#pragma unroll 16
-            for (int j = 0; j < SC; ++j) acc = acc + src[(size_t)j * R];
+            acc = sum_ascending<16>(src, SC, R);
             stat[which][r] = acc;
         }
         __syncthreads();
@@ -897,6 +944,9 @@ __global__ __launch_bounds__(WAVE * LNB_DX_WAVES) void layernorm_bwd_dx_kernel(
 // column sums is a quarter of the work), each finishes every pieces-th of its waves' blocks.  us with the residual add, stochastic, 16
 // waves and one workgroup per strip | now: 256x2048 29.4 | 13.5, 64x1024 16.3 | 10.4, 1248x1120 17.8 | 10.9, 2048x768 13.0 | 10.7, 4096x1024
 // 17.9 | 13.0, 3072x1280 20.7 | 15.4 (pieces); 12288x768 27.8 | 26.3, 8224x768 25.9 | 24.1 (eight waves).
+// Scales are requested as bits and converted behind the first barrier: the conversion of a value that is requested under a condition is moved to the
+// request, and each block's requests then waited for those of the one before (with dgamma's finishing launch, 12288x768 29.3 | 28.7, 16384x768 29.5 | 28.1,
+// 8192x1600 33.1 | 32.8).
 constexpr int LNS_WAVES = 16, LNS_BPW = 4;
 constexpr int LNS_PATCH_ADD = QB * ADD_PITCH;      // floats per wave: the sum's patch, also used for the column sums
 static_assert(LNS_PATCH_ADD >= COLSUM_PATCH, "one patch per wave serves both");
@@ -914,7 +964,7 @@ __global__ __launch_bounds__(WAVE * WAVES, 4) void layernorm_bwd_strip_kernel(
     float *cpatch = cs + 2 * QB + wave * (ADD ? LNS_PATCH_ADD : COLSUM_PATCH);   // (only with WANT_DW or ADD)
     const int row = rb * QB + (lane >> 1);
     v4i cx[LNS_BPW], cg[LNS_BPW];
-    float scx[LNS_BPW], scg[LNS_BPW];
+    uint32_t scx[LNS_BPW], scg[LNS_BPW];
     static_for<0, LNS_BPW>([&](auto i_c) {
         constexpr int I = decltype(i_c)::value;
         const int cb = wave + I * WAVES;
@@ -922,14 +972,16 @@ __global__ __launch_bounds__(WAVE * WAVES, 4) void layernorm_bwd_strip_kernel(
             const size_t e0 = (size_t)row * C + cb * QB + (lane & 1) * 16;
             cx[I] = *reinterpret_cast<const v4i *>(qx + e0);
             cg[I] = *reinterpret_cast<const v4i *>(qg + e0);
-            scx[I] = load_scale(sx, rb * SC + cb);
-            scg[I] = load_scale(sg, rb * SC + cb);
+            scx[I] = scale_bits(sx, rb * SC + cb);
+            scg[I] = scale_bits(sg, rb * SC + cb);
         }
     });
     const float mu = mean[row], rs = rstd[row];
     for (int c = threadIdx.x * 4; c < C; c += WAVE * WAVES * 4)
         *reinterpret_cast<v4f *>(gl + c) = *reinterpret_cast<const v4f *>(gamma + c);
     __syncthreads();
+#pragma unroll
+    for (int i = 0; i < LNS_BPW; ++i) asm volatile("" : "+v"(scx[i]), "+v"(scg[i]));      // (converted behind the barrier, not at the request)
     const float b = -(mu * rs);
     // phase 1: block partials of the two row sums; column sums of the strip
     static_for<0, LNS_BPW>([&](auto i_c) {
@@ -937,7 +989,7 @@ __global__ __launch_bounds__(WAVE * WAVES, 4) void layernorm_bwd_strip_kernel(
         const int cb = wave + I * WAVES;
         if (cb >= SC) return;                                      // uniform
         const int col = cb * QB + (lane & 1) * 16;
-        const float a = scx[I] * rs, sgk = scg[I];
+        const float a = scale_of_bits<ST>(scx[I]) * rs, sgk = scale_of_bits<ST>(scg[I]);
         float x[16], g[16], w[16];
         Load16<float>::run(gl + col, w);
         codes_to_float16(cx[I], x);
@@ -996,7 +1048,7 @@ __global__ __launch_bounds__(WAVE * WAVES, 4) void layernorm_bwd_strip_kernel(
         if (cb >= SC || !own(I)) return;                           // uniform
         const int col = cb * QB + (lane & 1) * 16;
         const size_t e0 = (size_t)row * C + col;
-        const float a = scx[I] * rs, sgk = scg[I];
+        const float a = scale_of_bits<ST>(scx[I]) * rs, sgk = scale_of_bits<ST>(scg[I]);
         float x[16], g[16], w[16];
         v4i raw[4];                                                // (ADD) the lane's 16 values of x1 as they lie in memory
         if (ADD) {
@@ -1167,17 +1219,17 @@ __global__ __launch_bounds__(WAVE * ADS_WAVES, 4) void add_strip_kernel(const T 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int SC = C / QB, rb = blockIdx.x, per = (SC + ADS_WAVES - 1) / ADS_WAVES, row = rb * QB + (lane >> 1);
     float *part = lds_f, *sq = part + 2 * SC * QB, *ypatch = sq + QB + wave * (QB * ADD_PITCH);
-    float a[ADS_BPW][16];
-    v4i c[ADS_BPW];
-    float sc[ADS_BPW];
+    v4i a[ADS_BPW][sizeof(T)], c[ADS_BPW];                         // the lane's 16 values of x1 as they lie in memory, its codes
+    uint32_t sc[ADS_BPW];
     static_for<0, ADS_BPW>([&](auto i_c) {
         constexpr int I = decltype(i_c)::value;
         const int cb = wave * per + I;
         if (I < per && cb < SC) {
             const size_t e0 = (size_t)row * C + cb * QB + (lane & 1) * 16;
-            Load16<T>::run(x1 + e0, a[I]);
+#pragma unroll
+            for (int k = 0; k < (int)sizeof(T); ++k) a[I][k] = reinterpret_cast<const v4i *>(x1 + e0)[k];
             c[I] = *reinterpret_cast<const v4i *>(q2 + e0);
-            sc[I] = load_scale(s2, rb * SC + cb);
+            sc[I] = scale_bits(s2, rb * SC + cb);
         }
     });
     static_for<0, ADS_BPW>([&](auto i_c) {
@@ -1185,10 +1237,16 @@ __global__ __launch_bounds__(WAVE * ADS_WAVES, 4) void add_strip_kernel(const T 
         const int cb = wave * per + I;
         if (I >= per || cb >= SC) return;                                      // uniform
         const size_t e0 = (size_t)row * C + cb * QB + (lane & 1) * 16;
-        float b[16];
-        unpack16(c[I], sc[I], b);
+        float b[16], x[16];
+        // (opaque, here as in layernorm_bwd_strip_kernel: a conversion of a value requested under a condition is moved to the request,
+        // which then waits for it before the next block's is made)
 #pragma unroll
-        for (int k = 0; k < 16; ++k) b[k] = a[I][k] + b[k];
+        for (int k = 0; k < (int)sizeof(T); ++k) asm volatile("" : "+v"(a[I][k]));
+        asm volatile("" : "+v"(sc[I]));
+        Load16<T>::run(reinterpret_cast<const T *>(a[I]), x);
+        unpack16(c[I], scale_of_bits<ST>(sc[I]), b);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) b[k] = x[k] + b[k];
         float t1 = 0.0f, t2 = 0.0f;
 #pragma unroll
         for (int k = 0; k < 16; ++k) { t1 = t1 + b[k]; t2 = __builtin_fmaf(b[k], b[k], t2); }
@@ -1259,7 +1317,8 @@ static inline bool rounding_ok(int r) { return r >= JF_ROUND_NEAREST && r <= JF_
 using namespace jf;
 
 // mean and 1/sqrt(variance) of every row from its per-32-column partial sums (rowsum, rowsq: [parts][R], what add_kernel
-// leaves): the partials are added in ascending order, var = E[y^2] - mean^2, no epsilon (add_mean_var.py:219-221).
+// leaves): the partials are added in ascending order, var = E[y^2] - mean^2, no epsilon (add_mean_var.py:219-221).  A thread's requests, up to eight
+// of either array, go out together: one after the other | so, us: 8192x1600 3.45 | 3.0, 96x4096 5.1 | 3.8, 12288x768 2.75 | 2.8.
 constexpr int RSF_ROWS = 32;                       // rows per workgroup
 __global__ __launch_bounds__(256) void rowstats_finish_kernel(const float *rowsum, const float *rowsq, int R, int parts,
                                                               float n, float *mean, float *rstd)
@@ -1270,12 +1329,21 @@ __global__ __launch_bounds__(256) void rowstats_finish_kernel(const float *rowsu
     const int r0 = blockIdx.x * RSF_ROWS;
     const int rows = (R - r0) < RSF_ROWS ? (R - r0) : RSF_ROWS;
     const int count = parts * RSF_ROWS;
-    for (int i = threadIdx.x; i < count; i += 256) {
-        const int j = i / RSF_ROWS, r = i % RSF_ROWS;
-        if (r < rows) {
-            rsf_lds[i] = rowsum[(size_t)j * R + r0 + r];
-            rsf_lds[count + i] = rowsq[(size_t)j * R + r0 + r];
-        }
+    const int r_in = threadIdx.x % RSF_ROWS, from = r0 + (r_in < rows ? r_in : 0);
+    for (int j0 = threadIdx.x / RSF_ROWS; j0 < parts; j0 += 64) {     // 64 parts at once, eight of each array on their way per thread
+        float v[8], w[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (j0 + 8 * i < parts) {
+                const size_t at = (size_t)(j0 + 8 * i) * R + from;
+                v[i] = rowsum[at]; w[i] = rowsq[at];
+            }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (j0 + 8 * i < parts) {
+                rsf_lds[(j0 + 8 * i) * RSF_ROWS + r_in] = v[i];
+                rsf_lds[count + (j0 + 8 * i) * RSF_ROWS + r_in] = w[i];
+            }
     }
     __syncthreads();
     const int row = threadIdx.x & (RSF_ROWS - 1), which = threadIdx.x / RSF_ROWS;     // which: 0 = sums, 1 = squares

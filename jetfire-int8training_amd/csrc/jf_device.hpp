@@ -36,6 +36,14 @@ template <int I, int N, typename F> __device__ __forceinline__ void static_for(F
 // ---------------------------------------------------------------------------------------------
 // scale element access: binary16 or binary32 behind one template parameter
 template <typename ST> __device__ __forceinline__ float load_scale(const ST *p, int i) { return (float)p[i]; }
+// the same in two steps: the bits now, their value later
+__device__ __forceinline__ uint32_t scale_bits(const half_t *p, int i) { return reinterpret_cast<const uint16_t *>(p)[i]; }
+__device__ __forceinline__ uint32_t scale_bits(const float *p, int i) { return reinterpret_cast<const uint32_t *>(p)[i]; }
+template <typename ST> __device__ __forceinline__ float scale_of_bits(uint32_t b)
+{
+    if constexpr (sizeof(ST) == 2) return (float)__builtin_bit_cast(half_t, (uint16_t)b);
+    else return __uint_as_float(b);
+}
 template <typename ST> __device__ __forceinline__ void store_scale(ST *p, int i, float v) { p[i] = (ST)v; }
 
 // ---------------------------------------------------------------------------------------------

@@ -260,6 +260,36 @@ def test_add_with_finished_statistics(jf, R, C, x1, out, scale, mode):
     assert torch.equal(q2, want[1]) and torch.equal(s2, want[2]) and torch.equal(mean[3:], want[3][3:])
 
 
+# parts of one and of several requests per thread, a last round of eight that is not full, more than 64; rows that end inside a workgroup
+@pytest.mark.parametrize("R,parts", [(32, 1), (40, 8), (96, 9), (64, 63), (72, 64), (32, 65), (33, 131)])
+def test_finishing_the_row_sums(jf, R, parts):
+    rng = np.random.default_rng(R + parts)
+    rs, rq = rng.standard_normal((parts, R)).astype(np.float32), (rng.random((parts, R)) * 1000).astype(np.float32)
+    n = np.float32(parts * 32)
+    a, b = np.zeros(R, np.float32), np.zeros(R, np.float32)
+    for p in range(parts):
+        a, b = a + rs[p], b + rq[p]
+    m = a / n
+    mean, rstd = jf.rowstats_finish(dev(rs), dev(rq), parts * 32)
+    same(mean, m, "mean")
+    same(rstd, np.float32(1) / np.sqrt(b / n - m * m), "rstd")
+
+
+# rows of up to two pieces per lane, of three (the last one of a few lanes), of eight, and longer
+@pytest.mark.parametrize("dtype,C", [(torch.float32, c) for c in (32, 512, 544, 2016, 2048, 2080)] + [(torch.bfloat16, c) for c in (1024, 1056, 4096, 4128)] + [(torch.float16, 1088)])
+def test_row_statistics_of_a_floating_tensor(dtype, C):
+    import BlockQuantizeCUDA as BQC
+    g = torch.Generator("cuda").manual_seed(C)
+    x = (torch.randn((2, 32, C), device="cuda", generator=g) + 0.5).to(dtype)
+    mean, rstd = BQC.jetfire.rowstats_fp(x)
+    d = x.double()
+    # a lane adds at most C/64 + 4 terms in sequence and the wave six levels of them: (C/64 + 10) roundings of 2^-24 of the sum of |x|
+    bound = (C / 64 + 10) * 2.0 ** -24 * d.abs().mean(-1) + 2.0 ** -24 * d.mean(-1).abs()
+    assert ((mean.double() - d.mean(-1)).abs() <= bound).all()
+    want = torch.rsqrt(d.var(-1, unbiased=False))
+    assert ((rstd.double() - want).abs() <= (C / 64 + 16) * 2.0 ** -24 * want).all()
+
+
 def test_gelu_with_one_and_with_four_blocks_per_wave(jf):
     """8192 blocks are the most that take a wave each; the rows of a taller tensor get the same bits four blocks to a wave."""
     R, C = 4096, 2048
