@@ -291,8 +291,8 @@ int jf_add(const void *x1, int x1_dtype, const int8_t *q2, const void *s2, int R
            int scale_dtype, int rounding, uint64_t seed, uint64_t offset,
            void *y1, int y1_dtype, int8_t *q, void *s, float *rowsum, float *rowsq, jf_stream_t stream);
 
-/* jf_add followed by jf_rowstats_finish (mean and rstd [R] instead of the partial sums), bit for bit; as one kernel where a
- * workgroup per 32-row strip is the faster way.  workspace: jf_add_rowstats_workspace_bytes (0 there).  (q, s) may be (q2, s2). */
+/* jf_add followed by jf_rowstats_finish (mean and rstd [R] instead of the partial sums), bit for bit; as one kernel where that is
+ * the faster way.  workspace: jf_add_rowstats_workspace_bytes (0 for some shapes).  (q, s) may be (q2, s2). */
 size_t jf_add_rowstats_workspace_bytes(int R, int C);
 int jf_add_rowstats(const void *x1, int x1_dtype, const int8_t *q2, const void *s2, int R, int C, int scale_dtype, int rounding,
                     uint64_t seed, uint64_t offset, void *y1, int y1_dtype, int8_t *q, void *s, float *mean, float *rstd,

@@ -1207,6 +1207,25 @@ __global__ __launch_bounds__(NT) void add_kernel(const T *x1, const int8_t *q2, 
     }
 }
 
+// The rows of strip rb from their blocks' partial sums in LDS (part: [2][C/32][32], written by the whole workgroup), in ascending order as in
+// rowstats_finish_kernel; threads 0..31: sums, 32..63: squares.
+__device__ __forceinline__ void finish_strip_rows(const float *part, float *sq, int SC, int C, int rb, float *mean, float *rstd)
+{
+    __syncthreads();
+    float acc = 0.0f;
+    if (threadIdx.x < 2 * QB) {
+        const float *p = part + (threadIdx.x >> 5) * SC * QB + (threadIdx.x & 31);
+        for (int j = 0; j < SC; ++j) acc = acc + p[j * QB];
+        if (threadIdx.x >= QB) sq[threadIdx.x & 31] = acc;
+    }
+    __syncthreads();
+    if (threadIdx.x < QB) {
+        const float n = (float)C, m = acc / n, var = sq[threadIdx.x] / n - m * m;
+        mean[rb * QB + threadIdx.x] = m;
+        rstd[rb * QB + threadIdx.x] = 1.0f / __builtin_sqrtf(var);
+    }
+}
+
 // add_kernel and rowstats_finish_kernel as one launch, bit for bit: a workgroup owns a 32-row strip (each wave up to four adjacent blocks, all
 // of them requested at once), so that the partial sums of its rows never leave it (add_in_strips).
 constexpr int ADS_WAVES = 16, ADS_BPW = 4;
@@ -1266,19 +1285,72 @@ __global__ __launch_bounds__(WAVE * ADS_WAVES, 4) void add_strip_kernel(const T 
         static_for<0, ADS_BPW>([&](auto i_c) { group_put(lines, lane, decltype(i_c)::value, c[decltype(i_c)::value]); });
         group_store_lines(lines, lane, q, rb, wave, C);
     }
-    __syncthreads();
-    float acc = 0.0f;                                              // threads 0..31: sums, 32..63: squares, in ascending order
-    if (threadIdx.x < 2 * QB) {
-        const float *p = part + (threadIdx.x >> 5) * SC * QB + (threadIdx.x & 31);
-        for (int j = 0; j < SC; ++j) acc = acc + p[j * QB];
-        if (threadIdx.x >= QB) sq[threadIdx.x & 31] = acc;
+    finish_strip_rows(part, sq, SC, C, rb, mean, rstd);
+}
+
+// The same with the statistics beside the addition instead of before it: the first R/32 workgroups form the row sums of a strip each and nothing
+// else, the waves of the others add and quantise a block each.  The inputs are read twice, but no strip waits for the quantisation of
+// its blocks and the blocks spread over the chip (add_beside_sums).  No result may lie on an operand.  What bounds it is one chain: request, sum
+// of a row's terms, division; 1248x1120 8.2 -> 5.0 us.
+template <typename T, typename ST, typename OT>
+__global__ __launch_bounds__(WAVE * ADS_WAVES, 4) void add_beside_sums_kernel(const T *x1, const int8_t *q2, const ST *s2, int R, int C,
+                                                                              int rounding, uint64_t seed, uint64_t offset, OT *y1, int8_t *q,
+                                                                              ST *s, float *mean, float *rstd)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds_f[];  // partial sums [2][C/32][32], squares of a row [32]; or patches
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int SC = C / QB, strips = R / QB;
+    if ((int)blockIdx.x >= strips) {
+        const int at = ((int)blockIdx.x - strips) * ADS_WAVES + wave;
+        if (at >= strips * SC) return;
+        const int rb = at / SC, cb = at - rb * SC;
+        const size_t e0 = (size_t)(rb * QB + (lane >> 1)) * C + cb * QB + (lane & 1) * 16;
+        float x[16], b[16];
+        Load16<T>::run(x1 + e0, x);
+        unpack16(*reinterpret_cast<const v4i *>(q2 + e0), load_scale(s2, rb * SC + cb), b);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) b[k] = x[k] + b[k];
+        store_block_rows(lds_f + wave * (QB * ADD_PITCH), b, y1 + (size_t)rb * QB * C + cb * QB, C, lane);
+        float scale;
+        *reinterpret_cast<v4i *>(q + e0) = quantize16(b, 0.0f, rounding, seed, offset, e0, &scale);
+        if (lane == 0) store_scale(s, rb * SC + cb, scale);
+        return;
     }
-    __syncthreads();
-    if (threadIdx.x < QB) {
-        const float n = (float)C, m = acc / n, var = sq[threadIdx.x] / n - m * m;
-        mean[rb * QB + threadIdx.x] = m;
-        rstd[rb * QB + threadIdx.x] = 1.0f / __builtin_sqrtf(var);
-    }
+    const int rb = blockIdx.x;
+    float *const part = lds_f;
+    v4i a[ADS_BPW][sizeof(T)], c[ADS_BPW];
+    uint32_t sc[ADS_BPW];
+    static_for<0, ADS_BPW>([&](auto i_c) {
+        constexpr int I = decltype(i_c)::value;
+        const int cb = wave + I * ADS_WAVES;
+        if (cb < SC) {
+            const size_t e0 = (size_t)(rb * QB + (lane >> 1)) * C + cb * QB + (lane & 1) * 16;
+#pragma unroll
+            for (int k = 0; k < (int)sizeof(T); ++k) a[I][k] = reinterpret_cast<const v4i *>(x1 + e0)[k];
+            c[I] = *reinterpret_cast<const v4i *>(q2 + e0);
+            sc[I] = scale_bits(s2, rb * SC + cb);
+        }
+    });
+    static_for<0, ADS_BPW>([&](auto i_c) {
+        constexpr int I = decltype(i_c)::value;
+        const int cb = wave + I * ADS_WAVES;
+        if (cb >= SC) return;                                      // uniform
+        float x[16], b[16];
+#pragma unroll
+        for (int k = 0; k < (int)sizeof(T); ++k) asm volatile("" : "+v"(a[I][k]));      // (see add_strip_kernel)
+        asm volatile("" : "+v"(sc[I]));
+        Load16<T>::run(reinterpret_cast<const T *>(a[I]), x);
+        unpack16(c[I], scale_of_bits<ST>(sc[I]), b);
+        float t1 = 0.0f, t2 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) { const float y = x[k] + b[k]; t1 = t1 + y; t2 = __builtin_fmaf(y, y, t2); }
+        const float o1 = __shfl_xor(t1, 1, WAVE), o2 = __shfl_xor(t2, 1, WAVE);
+        if ((lane & 1) == 0) {
+            part[cb * QB + (lane >> 1)] = t1 + o1;
+            part[(SC + cb) * QB + (lane >> 1)] = t2 + o2;
+        }
+    });
+    finish_strip_rows(part, part + 2 * SC * QB, SC, C, rb, mean, rstd);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1363,15 +1435,24 @@ __global__ __launch_bounds__(256) void rowstats_finish_kernel(const float *rowsu
     }
 }
 
-// Where one workgroup per strip takes the place of two launches (jf_add_rowstats): a CU to itself for every strip, and either few blocks in
-// a row or enough strips to occupy the chip.  us, two launches | one, bfloat16 in and out (float): 32x128 4.5 | 3.1, 512x1024 6.7 | 7.0 (6.7 | 7.4),
-// 1248x1120 7.6 | 7.3 (8.1 | 8.5), 2048x768 7.1 | 5.9, 4096x1024 9.4 | 8.8, 8192x768 11.6 | 8.4, 8192x1600 21.0 | 16.4 (28.0 | 22.3), 4096x2048 16.3 |
-// 15.9; on the other side of the line 1248x1536 8.4 | 9.9, 2048x1600 10.4 | 10.9, 256x2048 8.1 | 11.8.  (A launch and two allocations less are
-// another 5 us of the host.)
+// How jf_add_rowstats adds: with the row sums beside it, in strips, or in two launches (add_kernel, rowstats_finish_kernel).
+// Beside it where all its workgroups have a CU each, unless a row is narrow (a wave of a strip then has one block anyway) or so wide that the row sums
+// take longer than the two launches.  us, two launches | strips | beside, bfloat16 in and out (float): 32x128 4.8 | 3.2 | 2.7, 32x1024 5.3 | 6.6 | 4.0 (5.4 |
+// 7.3 | 4.7), 1024x512 5.9 | 4.5 | 3.9, 1248x1120 6.8 | 8.2 | 5.0 (7.3 | 9.6 | 6.2), 2048x768 6.9 | 6.6 | 4.4 (7.4 | 7.7 | 5.3), 2048x1280 7.7 | 10.0 | 6.1 (9.1 |
+// 11.5 | 7.9), 1248x1536 7.2 | 10.2 | 6.1 (7.9 | 11.8 | 7.9); beyond the line 1024x128 5.4 | 3.6 | 3.7 (5.4 | 3.6 | 4.1), 1024x256 5.6 | 3.7 | 3.8 (5.5 | 3.9 | 4.1),
+// 1024x2048 7.4 | 12.7 | 7.3 (8.0 | 14.6 | 10.0), 4096x768 (320 workgroups) 7.9 | 7.4 | 7.1 (9.1 | 9.0 | 9.8), 8192x768 11.2 | 9.3 | 11.7 (14.8 | 12.1 | 16.5).
+// In strips where the row is narrow or the strips are many: 4096x256 6.0 | 4.1, 4096x1024 8.7 | 9.1 (11.2 | 10.4), 6144x1600 16.2 | 16.1 (21.1 | 18.5), 8192x1600 19.5 |
+// 17.7 (26.6 | 21.6); beyond 4096x1280 10.2 | 12.0 (12.7 | 14.2), 4096x2048 14.4 | 16.6 (18.1 | 20.1).
+static long add_beside_sums_workgroups(int R, int C) { return R / QB + ((long)(R / QB) * (C / QB) + ADS_WAVES - 1) / ADS_WAVES; }
+static bool add_beside_sums(int R, int C)
+{
+    const int strips = R / QB, blocks = C / QB;
+    return (blocks > 8 || strips == 1) && blocks <= 48 && add_beside_sums_workgroups(R, C) <= cu_count();
+}
 static bool add_in_strips(int R, int C)
 {
     const int strips = R / QB, blocks = C / QB, cus = cu_count();
-    return blocks <= ADS_WAVES * ADS_BPW && strips <= cus && (blocks <= 36 || 8 * strips >= 3 * cus);
+    return blocks <= ADS_WAVES * ADS_BPW && strips <= cus && (blocks <= 32 || 4 * strips >= 3 * cus);
 }
 
 #define JF_LAUNCH(kern, grid, smem, st, ...)                         \
@@ -1820,26 +1901,44 @@ int jf_add_rowstats(const void *x1, int x1_dtype, const int8_t *q2, const void *
     if (!x1 || !y1 || !q || !s || !mean || !rstd) return JF_ERR_NULL;
     if (!rounding_ok(rounding) || x1_dtype < JF_FP_F16 || x1_dtype > JF_FP_BF16 || y1_dtype < JF_FP_F16 || y1_dtype > JF_FP_BF16) return JF_ERR_ENUM;
     if (!aligned16(x1) || !aligned16(y1) || !aligned16(q)) return JF_ERR_ALIGN;
-    if (!add_in_strips(R, C)) {
+    const bool strips = add_in_strips(R, C);
+    bool beside = add_beside_sums(R, C);
+    if (beside) {                                                  // (a workgroup reads what another one writes where a result lies on an operand)
+        const size_t n = (size_t)R * C, ns = n / (QB * QB) * (scale_dtype == JF_SCALE_F16 ? 2 : 4);
+        const auto width = [](int t) -> size_t { return t == JF_FP_F32 ? 4 : 2; };
+        const auto overlap = [](const void *a, size_t na, const void *b, size_t nb) {
+            const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+            return x < y + nb && y < x + na;
+        };
+        const void *const out[] = {y1, q, s, mean, rstd}, *const in[] = {x1, q2, s2};
+        const size_t osize[] = {n * width(y1_dtype), n, ns, (size_t)R * 4, (size_t)R * 4}, isize[] = {n * width(x1_dtype), n, ns};
+        for (int i = 0; i < 5; ++i)
+            for (int j = 0; j < 3; ++j) beside = beside && !overlap(out[i], osize[i], in[j], isize[j]);
+    }
+    if (!strips) {
         if (!workspace || !aligned16(workspace) || workspace_bytes < jf_add_rowstats_workspace_bytes(R, C)) return JF_ERR_WORKSPACE;
+    }
+    if (!strips && !beside) {
         float *const rowsum = (float *)workspace, *const rowsq = rowsum + (size_t)(C / QB) * R;
         rc = jf_add(x1, x1_dtype, q2, s2, R, C, scale_dtype, rounding, seed, offset, y1, y1_dtype, q, s, rowsum, rowsq, stream);
         return rc ? rc : jf_rowstats_finish(rowsum, rowsq, R, C / QB, C, mean, rstd, stream);
     }
     if (!device_is_gfx950()) return JF_ERR_DEVICE;
-    const size_t lds = ((size_t)2 * (C / QB) * QB + QB + ADS_WAVES * QB * ADD_PITCH) * sizeof(float);
+    const size_t sums = (size_t)2 * (C / QB) * QB + QB, patches = ADS_WAVES * QB * ADD_PITCH;
+    const size_t lds = (beside ? (sums > patches ? sums : patches) : sums + patches) * sizeof(float);
+    const int grid = beside ? (int)add_beside_sums_workgroups(R, C) : R / QB;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return JF_ERR_DEVICE;
 #define JF_ADD(T, ST, OT)                                                                                         \
     do {                                                                                                          \
-        auto kern = add_strip_kernel<T, ST, OT>;                                                                  \
-        static std::atomic<bool> opted_in[MAX_DEVICES] = {};      /* more than 64 KiB of LDS: once per device */  \
-        if (!opted_in[dev].load(std::memory_order_acquire)) {                                                     \
+        auto kern = beside ? add_beside_sums_kernel<T, ST, OT> : add_strip_kernel<T, ST, OT>;                     \
+        static std::atomic<bool> opted_in[2][MAX_DEVICES] = {};   /* more than 64 KiB of LDS: once per device */  \
+        if (!opted_in[beside][dev].load(std::memory_order_acquire)) {                                             \
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
             if (e != hipSuccess) return (int)e;                                                                   \
-            opted_in[dev].store(true, std::memory_order_release);                                                 \
+            opted_in[beside][dev].store(true, std::memory_order_release);                                         \
         }                                                                                                         \
-        hipLaunchKernelGGL(kern, dim3(R / QB), dim3(WAVE * ADS_WAVES), lds, (hipStream_t)stream, (const T *)x1, q2, (const ST *)s2, R, C, \
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(WAVE * ADS_WAVES), lds, (hipStream_t)stream, (const T *)x1, q2, (const ST *)s2, R, C, \
                            rounding, seed, offset, (OT *)y1, q, (ST *)s, mean, rstd);                             \
         return (int)hipGetLastError();                                                                            \
     } while (0)

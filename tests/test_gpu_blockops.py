@@ -235,9 +235,10 @@ def test_add(jf, oracle, dtype, mode):
     assert np.allclose(m, wy.mean(-1), atol=1e-5) and np.allclose(rstd.cpu().numpy(), 1 / np.sqrt(wy.var(-1)), rtol=1e-4)
 
 
-# one launch: one block, a last round that is not full, the widest row of few strips, the widest of many, as many strips as CUs; two launches:
-# the next width, the widest row and the next one, one strip more
-@pytest.mark.parametrize("R,C", [(32, 32), (64, 608), (96, 1152), (3072, 2048), (8192, 64), (96, 1184), (64, 2048), (3072, 2080), (8224, 64)])
+# beside the row sums: one block, a strip alone and the narrowest row of two, the widest row, a workgroup on every CU (256); in strips: a narrow row, one
+# workgroup more, the widest of many, as many strips as CUs; two launches: the next width of few strips, fewer strips, one row of blocks wider, one strip more
+@pytest.mark.parametrize("R,C", [(32, 32), (32, 256), (64, 288), (96, 1536), (4096, 512), (64, 256), (4128, 512), (6144, 2048), (8192, 64), (96, 1568), (6112, 2048),
+                                 (6144, 2080), (8224, 64)])
 @pytest.mark.parametrize("x1,out,scale,mode", [(torch.float32, torch.bfloat16, torch.float16, "trunc"), (torch.bfloat16, torch.float32, torch.float32, "stochastic_trunc"),
                                                (torch.float16, torch.float16, torch.float16, "nearest")])
 def test_add_with_finished_statistics(jf, R, C, x1, out, scale, mode):
