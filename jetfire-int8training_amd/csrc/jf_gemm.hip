@@ -149,7 +149,7 @@ constexpr int gemm_lds(int EPI, int WBM, int WGM, int WGN, int NSTAGE)
 }
 // NSTAGE = depth of the LDS ring (one stage being computed, NSTAGE-1 in flight); WGPC = workgroups per CU
 // (the second launch bound counts waves per SIMD: WGPC workgroups of WGM*WGN waves over 4 SIMDs).
-// AKM = 1: A is [K, lda] (M-contiguous rows), staged and read like a [K,N] B operand (below).
+// AKM = 1: A is [K, lda] (M-contiguous rows), staged and read like a [K,N] B operand (below); lower tiles than 128 rows stage the whole lines.
 // BKN = 0: B is [N, ldb] (K-contiguous rows, like A).  BKN = 1: B is [K, ldb] (N-contiguous rows); its tile is staged
 // as it lies in memory and the K-contiguous MFMA operand is produced by the transposing LDS read of gfx950.
 static int pace_of(long wgs, long slots, int k_per_wg);
@@ -174,18 +174,18 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     }
     constexpr int NW = WGM * WGN;
     constexpr int BM = QB * WBM * WGM, BN = QB * WBN * WGN;
+    constexpr int AM = AKM ? ROW_BYTES : BM;                 // rows of A that a stage holds: whole 128-byte lines of a [K,M] operand, whatever the tile's height
     constexpr int GROUP_BYTES = SPLIT > 1 ? SPLIT_GROUP : 8 * ROW_BYTES;
-    constexpr int A_BYTES = BM / 8 * GROUP_BYTES;            // one stage of A
-    constexpr int STAGE_BYTES = (BM + BN) / 8 * GROUP_BYTES;
-    constexpr int GROUPS = (BM + BN) / 8;                    // 8-row groups (1 KiB each) per stage
+    constexpr int A_BYTES = AM / 8 * GROUP_BYTES;            // one stage of A
+    constexpr int STAGE_BYTES = (AM + BN) / 8 * GROUP_BYTES;
+    constexpr int GROUPS = (AM + BN) / 8;                    // 8-row groups (1 KiB each) per stage
     constexpr int LW = SPLIT > 1 ? 4 : NW;                   // waves that load
     constexpr int LPW = GROUPS / LW;                         // LDS-direct loads per wave per stage
     static_assert(GROUPS % LW == 0, "stage must split evenly over the waves");
     static_assert(NSTAGE >= 2 && NSTAGE <= 5, "ring depth");
     static_assert(SPLIT == 1 || (SPLIT == 2 && WBM == 1 && WGM == 1 && WGN == 2), "32x64 tiles");
     static_assert(SPLIT > 1 || !BKN || (BN == ROW_BYTES && WBN == 1), "a staged [K,N] row is one 128-byte LDS row");
-    static_assert(WBM == 2 || !AKM, "one block per wave: A as [M,K] only");
-    static_assert(!AKM || BM == ROW_BYTES, "a staged [K,M] row is one 128-byte LDS row");
+    static_assert(!AKM || ROW_BYTES % BM == 0, "a staged [K,M] row is one 128-byte LDS row");
     // The epilogues that requantise want a lane to hold 16 consecutive columns of a row.  They form the transposed product (B block
     // times A block, the same integers): its registers run along the columns, see the epilogue.
     constexpr bool QUANT = EPI == EPI_Q || EPI == EPI_QG || EPI == EPI_QB || EPI == EPI_QD || EPI == EPI_QA;
@@ -235,7 +235,8 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     // operands lie 64 bytes from those of the one two before)
     const int gchunk = SPLIT > 1 ? (lane & 7) ^ ((lane >> 4) & 3) : (lane & 7) ^ (((load_wave & 1) * 4 + (lane >> 4)) & 7);     // global chunk this lane fetches
     // A as [K,M]: as for B as [K,N] below (8 K rows x 128 M bytes per load, slot c' of row r holds chunk c' ^ r)
-    const int km_chunk = (m0 + (((lane & 7) ^ lrow) << 4)) < p.M ? ((lane & 7) ^ lrow) : 0;
+    const int m0_line = AKM ? m0 & ~(AM - 1) : m0;            // (first column of the lines)
+    const int km_chunk = (m0_line + (((lane & 7) ^ lrow) << 4)) < p.M ? ((lane & 7) ^ lrow) : 0;
     const unsigned loff_a = AKM ? (unsigned)lrow * (unsigned)p.lda + km_chunk * 16
                                 : (unsigned)lrow * (unsigned)p.lda + gchunk * 16;
     // B as [K,N]: a load moves 8 K rows x 128 N bytes (group g of a stage = K rows 8g .. 8g+7 of the stage).  Slot c'
@@ -253,14 +254,14 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
 #pragma unroll
     for (int j = 0; j < LPW; ++j) {
         const int grp = load_wave + j * LW;
-        is_a[j] = grp < BM / 8;
+        is_a[j] = grp < AM / 8;
         if (BKN && !is_a[j]) {
-            const int k0 = (grp - BM / 8) * KN_ROWS;                     // K row of the stage (redirected at issue time if beyond K)
+            const int k0 = (grp - AM / 8) * KN_ROWS;                     // K row of the stage (redirected at issue time if beyond K)
             gbase[j] = p.B + (size_t)k0 * (size_t)p.ldb + n0;
         } else if (AKM && is_a[j]) {
-            gbase[j] = p.A + (size_t)(grp * 8) * (size_t)p.lda + m0;
+            gbase[j] = p.A + (size_t)(grp * 8) * (size_t)p.lda + m0_line;
         } else {
-            int r0 = (is_a[j] ? m0 : n0) + (is_a[j] ? grp : grp - BM / 8) * 8;
+            int r0 = (is_a[j] ? m0 : n0) + (is_a[j] ? grp : grp - AM / 8) * 8;
             if (r0 >= (is_a[j] ? p.M : p.N)) r0 = is_a[j] ? m0 : n0;   // groups of a partial tile: any valid group
             gbase[j] = (is_a[j] ? p.A : p.B) + (size_t)r0 * (size_t)(is_a[j] ? p.lda : p.ldb);
         }
@@ -298,7 +299,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     auto make_table = [&] {
         const int mi = m0 / QB + wm < SM ? m0 / QB + wm : SM - 1, ni = n0 / QB + wn < SN ? n0 / QB + wn : SN - 1;
         const ST *ta = reinterpret_cast<const ST *>(p.sa) + (size_t)mi * p.sa_is, *tb = reinterpret_cast<const ST *>(p.sb) + (size_t)ni * p.sb_is;
-        for (int k = lane + WAVE * part; k < nkb; k += WAVE * SPLIT) table[k] = (SPLIT > 1 ? -1.0f : 1.0f) * ((float)ta[(size_t)k * p.sa_ks] * (float)tb[(size_t)k * p.sb_ks]) * 67108864.0f;
+        for (int k = lane + WAVE * part; k < nkb; k += WAVE * SPLIT) table[k] = (SPLIT > 1 ? -1.0f : 1.0f) * ((float)ta[(size_t)(k + kb_base) * p.sa_ks] * (float)tb[(size_t)(k + kb_base) * p.sb_ks]) * 67108864.0f;
     };
     // the scales of the next stage (one after the other) into ring slot `slot`; K blocks beyond the last: the last one again
     auto issue_scales = [&](auto slot_c) {
@@ -335,8 +336,8 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         asm volatile("ds_write_b32 %0, %1 offset:%2" ::"v"(dst), "v"(t), "n"(decltype(slot_c)::value * SC_SLOT) : "memory");
     };
 
-    constexpr int A_LOADS = (BM / 8) / LW;                    // loads 0 .. A_LOADS-1 of a wave fetch A rows, the rest B rows
-    static_assert((BM / 8) % LW == 0, "a load instruction fetches rows of one operand");
+    constexpr int A_LOADS = (AM / 8) / LW;                    // loads 0 .. A_LOADS-1 of a wave fetch A rows, the rest B rows
+    static_assert((AM / 8) % LW == 0, "a load instruction fetches rows of one operand");
     // FULL: the stage has all KB_STAGE K blocks (every stage but a short last one)
     auto issue_stage_as = [&](int stage, unsigned slot, auto full_c) {       // slot: stage % NSTAGE
         constexpr bool FULL = decltype(full_c)::value;
@@ -357,7 +358,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                 base = gbase[j];
                 gbase[j] += (size_t)(KB_STAGE * QB) * (size_t)p.ldb;
                 // K rows of a missing K block: the stage's first group again
-                if (!FULL && kb0 * QB + (grp - BM / 8) * KN_ROWS >= p.K) base -= (size_t)((grp - BM / 8) * KN_ROWS) * (size_t)p.ldb;
+                if (!FULL && kb0 * QB + (grp - AM / 8) * KN_ROWS >= p.K) base -= (size_t)((grp - AM / 8) * KN_ROWS) * (size_t)p.ldb;
             } else if (AKM && j < A_LOADS) {
                 base = gbase[j];
                 gbase[j] += (size_t)(KB_STAGE * QB) * (size_t)p.lda;
@@ -402,7 +403,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
 #pragma unroll
     for (int i = 0; i < WBM; ++i) {
         const int g = lane >> 4, r = lane & 15, rho = r >> 1;
-        const int c = 2 * (wm * WBM + i) + (g & 1);
+        const int c = 2 * ((m0 - m0_line) / QB + wm * WBM + i) + (g & 1);
         fa_km[i] = AKM ? (unsigned)(uintptr_t)lds + (g >> 1) * 2048 + ((rho * 8 + (c ^ rho)) << 4) + 8 * (r & 1) : 0u;
     }
     // product patch of this wave: a uniform address, parked in a vector register once (LDS reads take a VGPR address)
@@ -812,8 +813,15 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
             static_for<0, 2>([&](auto i_c) {
                 constexpr int I = decltype(i_c)::value, kb = 2 * PAIR + I;
                 v4i &a = fa2[PAIR][I], &b = fb2[PAIR][I];
-                const unsigned pa = fa_u[kb] + extra, pb = (BKN ? fb_kn : fb_u[kb]) + extra;
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(a) : "v"(pa), "n"(SB));
+                const unsigned pa = (AKM ? fa_km[0] : fa_u[kb]) + extra, pb = (BKN ? fb_kn : fb_u[kb]) + extra;
+                if (AKM) {
+                    v2i lo, hi;
+                    asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(lo) : "v"(pa), "n"(SB + kb * 4096));
+                    asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(hi) : "v"(pa), "n"(SB + kb * 4096 + 1024));
+                    a = v4i{lo.x, lo.y, hi.x, hi.y};
+                } else {
+                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(a) : "v"(pa), "n"(SB));
+                }
                 if (BKN) {
                     v2i lo, hi;
                     asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(lo) : "v"(pb), "n"(SB + kb * 4096));
@@ -1462,7 +1470,7 @@ struct GemmGroup {
     int end[WGRAD_MAX];       // first workgroup behind problem k, of an XCD's: ceil(work / 8) for each problem
     int n;
 };
-template <typename ST> __device__ __forceinline__ void wgrad_group_body(const GemmGroup &grp, const int wg)
+template <typename ST, bool SMALL> __device__ __forceinline__ void wgrad_group_body(const GemmGroup &grp, const int wg)
 {
     const int xcd = wg & 7, at = wg >> 3;
     int k = 0, begin = 0;
@@ -1471,9 +1479,11 @@ template <typename ST> __device__ __forceinline__ void wgrad_group_body(const Ge
         if (i < grp.n && at >= grp.end[i - 1]) { k = i; begin = grp.end[i - 1]; }
     const GemmArgs &p = grp.g[k];
     const int logical = logical_workgroup(p.tiles_m * p.tiles_n * p.splits, (at - begin) * 8 + xcd);
-    if (logical >= 0) igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0, 1>(p, logical);
+    if (logical < 0) return;
+    if constexpr (SMALL) igemm_body<EPI_FP, ST, 1, 1, 4, 2, 2, 1, 1, 0>(p, logical);
+    else igemm_body<EPI_FP, ST, 2, 2, 4, 2, 2, 1, 1, 0, 1>(p, logical);
 }
-template <typename ST> __global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp) { wgrad_group_body<ST>(grp, blockIdx.x); }
+template <typename ST> __global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp) { wgrad_group_body<ST, false>(grp, blockIdx.x); }
 
 // An activation gradient (EPI_Q or EPI_QD, B as [K,N]; 32x128 or 128x128 tiles), then weight gradients, in one launch: both gradients of
 // a linear layer, or the last one of a block with all of the block's weight gradients.
@@ -1482,7 +1492,7 @@ struct GemmBackward {
     GemmArgs x;
     GemmGroup w;
 };
-template <int EPI, typename ST, int TILE> __global__ __launch_bounds__(512, 4) void igemm_backward_kernel(GemmBackward b)
+template <int EPI, typename ST, int TILE, bool SMALL_W> __global__ __launch_bounds__(512, 4) void igemm_backward_kernel(GemmBackward b)
 {
     const int work_x = b.x.tiles_m * b.x.tiles_n, first_w = (work_x + 7) & ~7;      // (both parts are dealt to the XCDs from the first one on)
     const int wg = blockIdx.x;
@@ -1490,7 +1500,7 @@ template <int EPI, typename ST, int TILE> __global__ __launch_bounds__(512, 4) v
         const int logical = logical_workgroup(work_x, wg);
         if (logical >= 0) igemm_body<EPI, ST, TILE == TILE_128x128 ? 2 : 1, TILE == TILE_128x128 ? 2 : 1, TILE == TILE_32x64 ? 2 : 4, TILE == TILE_32x128 ? 3 : 2, 2, 1, 0, 0, 0, TILE == TILE_32x64 ? 2 : 1>(b.x, logical);
     } else {
-        wgrad_group_body<ST>(b.w, wg - first_w);
+        wgrad_group_body<ST, SMALL_W>(b.w, wg - first_w);
     }
 }
 
@@ -1899,19 +1909,29 @@ template <int EPI, typename ST> int launch_gemm(const GemmArgs &a, hipStream_t s
 
 #ifndef JF_PROF_LIB
 // x: as for a launch of its own; w: w_wgs workgroups, the longest of them k_per_part deep.
-template <int EPI, typename ST, int TILE> static int launch_backward(const GemmArgs &x, const GemmGroup &w, long w_wgs, int k_per_part, hipStream_t st)
+template <int EPI, typename ST, int TILE, bool SMALL_W = false> static int launch_backward(const GemmArgs &x, const GemmGroup &w, long w_wgs, int k_per_part, hipStream_t st)
 {
     GemmBackward b = {x, w};
+    if (SMALL_W) {
+        long at = 0;
+        for (int i = 0; i < w.n; ++i) {
+            b.w.g[i].tiles_m = w.g[i].M / QB;
+            at += ((long)b.w.g[i].tiles_m * b.w.g[i].tiles_n * w.g[i].splits + 7) / 8;
+            b.w.end[i] = (int)at;
+        }
+        w_wgs = at * 8;
+    }
     constexpr bool BIG = TILE == TILE_128x128;
     constexpr int BN = TILE == TILE_32x64 ? 64 : 128;
     b.x.tiles_m = BIG ? (x.M + 127) / 128 : x.M / QB; b.x.tiles_n = (x.N + BN - 1) / BN; b.x.splits = 1;
     const long x_wgs = ((long)b.x.tiles_m * b.x.tiles_n + 7) & ~7L;
     b.x.pace = !BIG ? (int)PACE_HARDWARE : pace_of(x_wgs + w_wgs, 2L * cu_count(), std::max(x.K, k_per_part));
-    for (int i = 0; i < w.n; ++i) b.w.g[i].pace = b.x.pace;
-    constexpr int SX = BIG ? gemm_lds(EPI, 2, 2, 4, 2) : TILE == TILE_32x128 ? gemm_lds(EPI, 1, 1, 4, 3) : SPLIT_LDS, SW = gemm_lds(EPI_FP, 2, 2, 4, 2), SMEM = SX > SW ? SX : SW;
+    for (int i = 0; i < w.n; ++i) b.w.g[i].pace = SMALL_W ? (int)PACE_HARDWARE : b.x.pace;
+    constexpr int SX = BIG ? gemm_lds(EPI, 2, 2, 4, 2) : TILE == TILE_32x128 ? gemm_lds(EPI, 1, 1, 4, 3) : SPLIT_LDS;
+    constexpr int SW = SMALL_W ? 2 * 2 * 128 * ROW_BYTES + 4 * (TABLE_KB + KB_STAGE) * 4 : gemm_lds(EPI_FP, 2, 2, 4, 2), SMEM = SX > SW ? SX : SW;
     static std::atomic<bool> opted_in[MAX_DEVICES] = {};
-    if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_backward_kernel<EPI, ST, TILE>), SMEM, opted_in)) return rc;
-    hipLaunchKernelGGL((igemm_backward_kernel<EPI, ST, TILE>), dim3((unsigned)(x_wgs + w_wgs)), dim3(512), SMEM, st, b);
+    if (int rc = allow_lds(reinterpret_cast<const void *>(igemm_backward_kernel<EPI, ST, TILE, SMALL_W>), SMEM, opted_in)) return rc;
+    hipLaunchKernelGGL((igemm_backward_kernel<EPI, ST, TILE, SMALL_W>), dim3((unsigned)(x_wgs + w_wgs)), dim3(512), SMEM, st, b);
     return (int)hipGetLastError();
 }
 // One launch for an activation gradient and weight gradients: neither needs the other's result, small ones leave most of the chip
@@ -1922,6 +1942,10 @@ template <int EPI, typename ST, int TILE> static int launch_backward(const GemmA
 //   2048x1024x4096 55.5 | 52.5 (128x128: 59.0), 1024x1600x6400 65.7 | 56.7 (62.5);
 //   128x128: 2048x768x768 23.6 | 19.4 (32x128: 21.3), 1024x2048x1024 31.8 | 25.8 (28.5), 4096x768x768 35.0 | 26.0, 4096x1024x4096 84.4 | 78.3,
 //   12288x768x3072 127.5 | 119.4, 8192x1024x4096 141.4 | 138.2.
+// The weight gradients in 128x128 tiles, except where one workgroup per CU holds all of the launch with theirs in 32x128 tiles, one block per wave: a
+// turn of those is 0.1 us per K block where a 128x128 tile alone on its CU takes 0.27.  us, 128x128 | 32x128: 480x736x160 8.6 | 5.5, 512x512x512
+// 8.7 | 5.6, 64x256x256 4.8 | 4.3, 480x192x2080 8.9 | 8.4, and with K splits 1024x256x1024 11.7 | 9.1, 4096x128x512 12.9 | 9.9; two per CU
+// 256x1024x1024 7.3 | 8.6, 512x1024x1024 9.7 | 11.2, 2048x256x768 12.4 | 13.8.
 // Above three 128x128 tiles of the activation gradient per CU the rounds even out by themselves: 4096x4096x1024 (1024) 86.1 | 83.7,
 // 8192x1600x4800 (832) 248.7 | 263.2, 8192x6400x1600 (3200) 359.4 | 363.9, 4096x4096x4096 (1024) 259.0 | 260.8.
 static bool backward_in_one_launch(int R, int C_in, long w_wgs)
@@ -1930,6 +1954,17 @@ static bool backward_in_one_launch(int R, int C_in, long w_wgs)
 }
 template <int EPI, typename ST> int launch_backward_any(const GemmArgs &x, const GemmGroup &w, long w_wgs, int k_per_part, hipStream_t st)
 {
+    if (x.K <= TABLE_KB * QB) {                                // weight gradients in 32x128 tiles
+        const long cus = cu_count(), narrow = split_tiles(x.M, x.N), wide = (long)(x.M / QB) * ((x.N + 127) / 128);
+        long small_w = 0;
+        for (int i = 0; i < w.n && small_w <= cus; ++i) {
+            const GemmArgs &a = w.g[i];
+            const bool fits = !a.fold_kb && (a.splits > 1 ? a.kb_per_split : a.K / QB) <= TABLE_KB;
+            small_w += fits ? (long)(a.M / QB) * a.tiles_n * a.splits : cus + 1;
+        }
+        if (narrow + small_w <= cus) return launch_backward<EPI, ST, TILE_32x64, true>(x, w, w_wgs, k_per_part, st);
+        if (wide + small_w <= cus) return launch_backward<EPI, ST, TILE_32x128, true>(x, w, w_wgs, k_per_part, st);
+    }
     if (split_tiles_resident(x.M, x.N, x.K) && split_tiles(x.M, x.N) + w_wgs <= cu_count())
         return launch_backward<EPI, ST, TILE_32x64>(x, w, w_wgs, k_per_part, st);
     const bool small = small_tiles_resident(x.M, x.N, x.K) && (x.K > 2048 || (long)(x.M / QB) * ((x.N + 127) / 128) <= cu_count());

@@ -684,6 +684,33 @@ def test_gelu_in_the_64_row_tiles(jf, oracle, M, N, K):
     test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K)
 
 
+# weight gradients in 32x128 tiles beside the activation gradient, up to one workgroup per CU (256): columns of the gradient that end inside a staged
+# line, every length of the last stage, K splits with a short last part; 256 workgroups with 32x64 tiles of the activation gradient, one row of tiles
+# more (its 32x128 tiles), and too many for either
+@pytest.mark.parametrize("R,C_in,C_out", [(r, 160, 288) for r in (32, 64, 96, 128, 160, 288, 416)] + [(1056, 128, 256), (2048, 96, 544), (480, 512, 1088), (480, 512, 1120), (480, 512, 2080)])
+def test_weight_gradients_in_tiles_of_32_rows(jf, R, C_in, C_out):
+    test_both_gradients_of_a_linear_layer_in_one_launch(jf, R, C_in, C_out, 0, True, True)
+    test_both_gradients_of_a_linear_layer_in_one_launch(jf, R, C_in, C_out, 1, False, False)
+
+
+def test_extreme_scales_in_the_weight_gradients_of_32_rows(jf):
+    """Products of scales beyond 2^102: the blocks they touch are formed again from memory, also of a later K split."""
+    rng = np.random.default_rng(1)
+    R, C_in, C_out = 1056, 128, 160
+    g, x, w = dev(rand_codes(rng, (R, C_out))), dev(rand_codes(rng, (R, C_in))), dev(rand_codes(rng, (C_out, C_in)))
+    sg, sx, sw = (torch.ones((r // 32, c // 32), device="cuda") for r, c in ((R, C_out), (R, C_in), (C_out, C_in)))
+    # (2^104 times a block product, below 32 * 128^2 = 2^19, is finite)
+    sg[1, 2], sx[1, 1], sg[30, 0], sx[30, 3] = 2.0 ** 52, 2.0 ** 52, 2.0 ** 53, 2.0 ** 51
+    dx, ds, dw = torch.empty_like(x), torch.empty_like(sx), torch.empty((C_out, C_in), device="cuda")
+    L, p = jf.lib(), jf._ptr
+    for splitk in (0, 1):
+        nb = L.jf_igemm_block_fp_workspace_bytes(C_out, C_in, R, jf.B_KN, splitk)
+        ws = torch.empty(max(nb, 16), dtype=torch.int8, device="cuda")
+        jf.check(L.jf_linear_bwd(p(x), p(sx), p(g), p(sg), p(w), p(sw), R, C_in, C_out, jf.SCALE_F32, p(dx), p(ds), jf.FP_F16, 1, 8, p(dw), jf.FP_F32, splitk, p(ws), nb, jf._stream()))
+        want = jf.igemm_block_fp(g, x, sg, sx, jf.B_KN, torch.float32, jf.A_KM, splitk)
+        assert torch.isfinite(want).all() and torch.equal(dw, want)
+
+
 # 425 tiles of 128x128 (825 of 64x128, which would not all be resident), the last row and column of them ragged: every ring fill
 @pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 288, 384, 416])
 def test_the_large_tiles_at_every_ring_fill(jf, oracle, K):
