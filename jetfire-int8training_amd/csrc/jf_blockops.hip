@@ -248,42 +248,61 @@ __global__ __launch_bounds__(NT) void quantize_kernel(QuantSrc src, int R, int C
     }
 }
 
+// The plain case, one tensor that lies as the result does and no transposed copy: workgroup (group of four column blocks, row block).  What
+// bounds a small launch is one chain, and its first link was the general kernel's way to the first request: 300 instructions of divisions and cases, each
+// executed once and fetched for it (27 ns per 64 bytes).  Here it is 38.  us, general | this: 32x768 binary16 2.98 | 2.54, 2304x768 float 3.67 | 3.19,
+// 512x2304 binary16 stochastic 3.90 | 3.38, 864x3200 3.88 | 3.36, 12288x768 float 9.15 | 8.38, 8192x1600 bfloat16 stochastic 11.2 | 9.3, 8192x6400 float 40.0 | 39.9.
+template <typename T, typename ST>
+__global__ __launch_bounds__(NT) void quantize_plain_kernel(const T *x, int C, int8_t *q, ST *s, int rounding, uint64_t seed, uint64_t offset, float amax_eps)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char line_patches[2 * QB * LINE_PITCH];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int SC = C / QB, cg = blockIdx.x, rb = blockIdx.y, cb = cg * WPB + wave;
+    GroupLineStore lines(line_patches, lane, wave);
+    v4i codes = {0, 0, 0, 0};
+    if (cb < SC) {                                                 // wave-uniform (the others: the barrier only)
+        const size_t e0 = (size_t)(rb * QB + (lane >> 1)) * C + cb * QB + (lane & 1) * 16;
+        float v[16], scale;
+        Load16<T>::run(x + e0, v);
+        codes = quantize16(v, amax_eps, rounding, seed, offset, e0, &scale);
+        if (lane == 0) store_scale(s, rb * SC + cb, scale);
+    }
+    lines.store(codes, q, rb, cg, C);
+}
+
 // quantize.py:33-117 of up to QMANY_MAX tensors of one type in one launch, round to nearest: the weights of a block, quantised
 // after every optimizer step.  (Four launches for a GPT-2 small block take 23 us, most of it ramp and drain; a 256-wide block
-// spends 16 us on four tensors that need 2.)
+// spends 16 us on four tensors that need 2.  The tensor of a group by counting and one indexed read of its fields, instead of a case for each, and without
+// a second division: 6.8 | 6.05 and 3.17 | 3.07 us.)
 constexpr int QMANY_MAX = 8;
 struct QuantMany {
     const void *x[QMANY_MAX];
     int8_t *q[QMANY_MAX];
     void *s[QMANY_MAX];
     int C[QMANY_MAX];
-    int end[QMANY_MAX];      // first group (four column blocks of a row block) behind tensor k
-    int n;
+    int begin[QMANY_MAX], end[QMANY_MAX];      // first group (four column blocks of a row block) of tensor k, and behind it (behind the last tensor: INT_MAX)
+    int groups;
 };
 template <typename T, typename ST> __global__ __launch_bounds__(NT) void quantize_many_kernel(QuantMany m)
 {
     __shared__ __attribute__((aligned(16))) unsigned char line_patches[2 * QB * LINE_PITCH];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     GroupLineStore lines(line_patches, lane, wave);
-    for (int g = blockIdx.x; g < m.end[m.n - 1]; g += gridDim.x) {
-        int k = 0, begin = 0;
-        const T *x = reinterpret_cast<const T *>(m.x[0]);
-        int8_t *q = m.q[0];
-        ST *s = reinterpret_cast<ST *>(m.s[0]);
-        int C = m.C[0];
+    for (int g = blockIdx.x; g < m.groups; g += gridDim.x) {
+        int k = 0;
 #pragma unroll
-        for (k = 1; k < QMANY_MAX; ++k)
-            if (k < m.n && g >= m.end[k - 1]) {
-                begin = m.end[k - 1]; C = m.C[k];
-                x = reinterpret_cast<const T *>(m.x[k]); q = m.q[k]; s = reinterpret_cast<ST *>(m.s[k]);
-            }
+        for (int i = 0; i < QMANY_MAX - 1; ++i) k += g >= m.end[i];     // (no group lies behind the last tensor)
+        const T *x = reinterpret_cast<const T *>(m.x[k]);
+        int8_t *q = m.q[k];
+        ST *s = reinterpret_cast<ST *>(m.s[k]);
+        const int C = m.C[k], begin = m.begin[k];
         const int SC = C / QB, G4 = (SC + WPB - 1) / WPB, rb = (g - begin) / G4, cg = (g - begin) - rb * G4, cb = cg * WPB + wave;
         v4i codes = {0, 0, 0, 0};
         if (cb < SC) {                                             // wave-uniform
-            BlockPos pos(rb * SC + cb, SC, C, lane);
+            const size_t e0 = (size_t)(rb * QB + (lane >> 1)) * C + cb * QB + (lane & 1) * 16;
             float v[16], scale;
-            Load16<T>::run(x + pos.e0, v);
-            codes = quantize16(v, 0.0f, JF_ROUND_NEAREST, 0, 0, pos.e0, &scale);
+            Load16<T>::run(x + e0, v);
+            codes = quantize16(v, 0.0f, JF_ROUND_NEAREST, 0, 0, e0, &scale);
             if (lane == 0) store_scale(s, rb * SC + cb, scale);
         }
         lines.store(codes, q, rb, cg, C);
@@ -1475,10 +1494,14 @@ int jf_quantize(const void *x, int x_dtype, int R, int C, int8_t *q, void *s, in
     hipStream_t st = (hipStream_t)stream;
     const int groups = quantize_groups(R, C, qT != nullptr);
     const int grid = groups < 256 * 32 ? groups : 256 * 32;       // (a multiple of 32, which the transposed walk needs)
+    const bool plain = !qT && R / QB <= 65535;
     QuantSrc src = {};
     src.x[0] = x; src.ldx[0] = C; src.end[0] = C; src.n = 1;
 #define JF_Q(T, ST)                                                                                          \
-    JF_LAUNCH((quantize_kernel<T, ST>), grid, 0, st, src, R, C, q, (ST *)s, qT, rounding, seed, offset, amax_eps)
+    do {                                                                                                     \
+        if (plain) JF_LAUNCH((quantize_plain_kernel<T, ST>), dim3((C / QB + WPB - 1) / WPB, R / QB), 0, st, (const T *)x, C, q, (ST *)s, rounding, seed, offset, amax_eps); \
+        JF_LAUNCH((quantize_kernel<T, ST>), grid, 0, st, src, R, C, q, (ST *)s, qT, rounding, seed, offset, amax_eps); \
+    } while (0)
     if (scale_dtype == JF_SCALE_F16) {
         if (x_dtype == JF_FP_F32) JF_Q(float, half_t);
         if (x_dtype == JF_FP_F16) JF_Q(half_t, half_t);
@@ -1504,11 +1527,13 @@ int jf_quantize_many(int n, const void *const *x, const int *R, const int *C, in
         if (rc) return rc;
         if (!x[k]) return JF_ERR_NULL;
         if (!aligned16(x[k])) return JF_ERR_ALIGN;
+        m.begin[k] = (int)groups;
         groups += quantize_groups(R[k], C[k], false);
         if (groups > 0x7fffffffL) return JF_ERR_SHAPE;
         m.x[k] = x[k]; m.q[k] = q[k]; m.s[k] = s[k]; m.C[k] = C[k]; m.end[k] = (int)groups;
     }
-    m.n = n;
+    for (int k = n - 1; k < QMANY_MAX; ++k) m.end[k] = 0x7fffffff;
+    m.groups = (int)groups;
     hipStream_t st = (hipStream_t)stream;
     const int grid = (int)(groups < 256L * 32 ? groups : 256L * 32);
 #define JF_QM(T, ST) JF_LAUNCH((quantize_many_kernel<T, ST>), grid, 0, st, m)

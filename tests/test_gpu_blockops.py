@@ -261,6 +261,15 @@ def test_add_with_finished_statistics(jf, R, C, x1, out, scale, mode):
     assert torch.equal(q2, want[1]) and torch.equal(s2, want[2]) and torch.equal(mean[3:], want[3][3:])
 
 
+def test_quantising_more_row_blocks_than_a_grid_dimension_holds(jf):
+    """65535 row blocks are the most of the plain kernel; one more takes the general one: the same codes, and as many as the parts of the tensor have."""
+    x = torch.randn((65536 * 32, 32), device="cuda", generator=torch.Generator("cuda").manual_seed(5)).half()
+    q, s = jf.quantize(x, rounding=ROUND["stochastic"], seed=3, offset=8)
+    for rows in (65535 * 32, 96):
+        qp, sp = jf.quantize(x[:rows], rounding=ROUND["stochastic"], seed=3, offset=8)
+        assert torch.equal(q[:rows], qp) and torch.equal(s[:rows // 32], sp)
+
+
 # parts of one and of several requests per thread, a last round of eight that is not full, more than 64; rows that end inside a workgroup
 @pytest.mark.parametrize("R,parts", [(32, 1), (40, 8), (96, 9), (64, 63), (72, 64), (32, 65), (33, 131)])
 def test_finishing_the_row_sums(jf, R, parts):
