@@ -1611,21 +1611,24 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 // A launch of 128x128 tiles that begins a short last round (of one workgroup per CU, or of two) takes that round's part of M as 32x128
 // tiles, in the same launch: tiles left alone on their CUs run at two thirds of the rate and leave most of the chip idle for the whole
 // length of a tile.  Rows of 128x128 tiles if so, else 0.  The line: after two big tiles per CU up to two small ones each (all of
-// them resident at once), after one, four or six one small one each.  us, 128x128 | mixed:
+// them resident at once), after one or three to seven one small one each.  us, 128x128 | mixed:
 //   768 wide, K = 3072: 5504 rows (258 tiles) 39.8 | 32.0, 6144 (288) 42.2 | 33.5, 12288 (576) 72.4 | 61.9; K = 768: 2048x2304 (288)
 //   15.4 | 11.5, 12288x768 23.2 | 21.6; K = 1536: 11008 rows (516) 41.2 | 32.8, 13312 (624) 38.8 | 35.3, 22016 (1032) 63.0 | 56.3;
 //   11008x2304x768 (1548) 50.6 | 45.9; 4224x1024x4096 (264) 52.1 | 43.0.
 // Beyond it: 13824x768x1536 (648 tiles) 38.8 | 39.0, 15360 (720) 39.4 | 42.5, 8192x768x3072 (384) 43.5 | 47.5, 24576x768x1536 (1152)
 // 61.7 | 61.8, 11264x3072x768 (2112) 63.0 | 62.3.
-// After three and after five the rule takes none, which is right for GPT-2 XL's 832 tiles only (640 rows behind three, 260 small tiles):
-// 8192x1600x1600 48.7 | 51.7, x4800 123.6 | 128.8, x6400 157.2 | 162.9.  With fewer behind them a mix would win there too: behind three
-// 16640x768x1536 (780) 46.3 | 41.1, 17408x768x1536 (816) 47.1 | 42.2, x3072 84.9 | 77.8; behind five 27648x768x1536 (1296) 73.5 | 64.5,
-// 12800x1600x6400 (1300) 265.2 | 254.6, 7040x3072x768 (1320) 42.5 | 37.8.
+// After three, five and seven, where half of the slots go on with a big tile, one small one each as well, for rows of K up to 8192.
+// Behind three 17024x768x768 (798) 28.3 | 27.2, with the GELU backward 40.7 | 36.1, x3072 84.1 | 77.3, 7680x1600x1600 (780) 47.4 | 44.6, 8064x1600x6400
+// (819, 208 small) 160.9 | 158.8, 13312x1024x4096 (832, 256 small) 111.1 | 108.9, 17408x768x8192 208 | 195, x96 12.9 | 12.3; behind five 27648x768x1536 (1296) 73.5 |
+// 67.3, 5376x4096x1024 (1344, 256 small) 55.3 | 52.8; behind seven 38400x768x768 (1800) 58.7 | 54.3, 9600x3072x768 (1800)
+// 56.7 | 54.4, 17920x1600x6400 (1820) 344.9 | 336.4, 18048x1600x256 (1833, 208 small) 29.8 | 30.3.  A longer row: 8064x1600x12800 313 | 322.  More than one
+// small tile each: 8192x1600x1600 (832 tiles, 260 small) 49.7 | 53.2, x4800 126.6 | 130.9, 13184x1600x1600 (1339, 260) 76.9 | 76.4.
 static int mixed_big_rows(int M, int N, int K)
 {
     const int rows = (M + 127) / 128, tiles_n = (N + 127) / 128, cus = cu_count();
     if (K > TABLE_KB * QB) return 0;
-    for (const int rounds : {1, 2, 4, 6}) {                    // big tiles per CU
+    for (int rounds = 1; rounds <= 7; rounds++) {              // big tiles per CU
+        if (rounds >= 3 && rounds % 2 && K > 8192) continue;
         const int big = rounds * cus / tiles_n;
         const long small = (long)((M - big * 128) / QB) * tiles_n;
         if (big < rows && big * tiles_n > (rounds - 1) * cus && small <= (rounds == 2 ? 2L : 1L) * cus) return big;

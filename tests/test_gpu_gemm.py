@@ -742,6 +742,14 @@ def test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K):
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+# behind three big tiles per CU one row block of small ones, columns that end inside a tile; as many as CUs, and one row block more (128x128 only);
+# behind five the fewest and the most; behind seven
+@pytest.mark.parametrize("M,N,K", [(16416, 736, 160), (13312, 1024, 32), (13344, 1024, 32), (27296, 768, 32), (5376, 4096, 96), (7328, 4096, 32)])
+def test_two_tile_sizes_behind_odd_rounds(jf, oracle, M, N, K):
+    test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K)
+    test_quantised_with_residual_addition(jf, oracle, M, N, K, torch.bfloat16, torch.float32, True, True)
+
+
 @pytest.mark.parametrize("K", [32, 480, 512, 1056])               # one K block, the longest without and the shortest with a K split, a ragged split
 @pytest.mark.parametrize("widths", [[(96, 32)], [(384, 160), (128, 160), (512, 128), (32, 544)]])
 @pytest.mark.parametrize("f16,out", [(True, torch.float32), (False, torch.bfloat16)])
