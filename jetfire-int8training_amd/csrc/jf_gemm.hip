@@ -1610,7 +1610,7 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 
 // A launch of 128x128 tiles that begins a short last round (of one workgroup per CU, or of two) takes that round's part of M as 32x128
 // tiles, in the same launch: tiles left alone on their CUs run at two thirds of the rate and leave most of the chip idle for the whole
-// length of a tile.  Rows of 128x128 tiles if so, else 0.  The line: after two big tiles per CU up to two small ones each (all of
+// length of a tile.  Rows of 128x128 tiles if so, else 0.  The line: after two (or four) big tiles per CU up to two small ones each (all of
 // them resident at once), after one or three to seven one small one each.  us, 128x128 | mixed:
 //   768 wide, K = 3072: 5504 rows (258 tiles) 39.8 | 32.0, 6144 (288) 42.2 | 33.5, 12288 (576) 72.4 | 61.9; K = 768: 2048x2304 (288)
 //   15.4 | 11.5, 12288x768 23.2 | 21.6; K = 1536: 11008 rows (516) 41.2 | 32.8, 13312 (624) 38.8 | 35.3, 22016 (1032) 63.0 | 56.3;
@@ -1623,15 +1623,19 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 // 67.3, 5376x4096x1024 (1344, 256 small) 55.3 | 52.8; behind seven 38400x768x768 (1800) 58.7 | 54.3, 9600x3072x768 (1800)
 // 56.7 | 54.4, 17920x1600x6400 (1820) 344.9 | 336.4, 18048x1600x256 (1833, 208 small) 29.8 | 30.3.  A longer row: 8064x1600x12800 313 | 322.  More than one
 // small tile each: 8192x1600x1600 (832 tiles, 260 small) 49.7 | 53.2, x4800 126.6 | 130.9, 13184x1600x1600 (1339, 260) 76.9 | 76.4.
+// Up to two small ones each also behind four where a small tile is long enough: 23168x768x3072 (1086, 264 small) 123.2 | 115.2, 24192x768x3072
+// (1134, 456) 124.4 | 120.8, 10752x1600x1600 (1092, 312) 69.7 | 66.1, 11136x1600x6400 (1131, 468) 244.7 | 231.1, 5888x3072x1536 (1104, 384) 66.7 | 66.2; K = 768
+// 24192 rows 39.8 | 41.4, 5760x3072 (288 small) 40.5 | 40.1; behind six 34560x768x1536 (336) 93.9 | 93.4, 16128x1600x1600 (416) 95.4 | 98.6.
 static int mixed_big_rows(int M, int N, int K)
 {
     const int rows = (M + 127) / 128, tiles_n = (N + 127) / 128, cus = cu_count();
     if (K > TABLE_KB * QB) return 0;
     for (int rounds = 1; rounds <= 7; rounds++) {              // big tiles per CU
         if (rounds >= 3 && rounds % 2 && K > 8192) continue;
+        const bool two = rounds == 2 || (rounds == 4 && K >= 1536 && K <= 8192);
         const int big = rounds * cus / tiles_n;
         const long small = (long)((M - big * 128) / QB) * tiles_n;
-        if (big < rows && big * tiles_n > (rounds - 1) * cus && small <= (rounds == 2 ? 2L : 1L) * cus) return big;
+        if (big < rows && big * tiles_n > (rounds - 1) * cus && small <= (two ? 2L : 1L) * cus) return big;
     }
     return 0;
 }
