@@ -1611,13 +1611,13 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 // A launch of 128x128 tiles that begins a short last round (of one workgroup per CU, or of two) takes that round's part of M as 32x128
 // tiles, in the same launch: tiles left alone on their CUs run at two thirds of the rate and leave most of the chip idle for the whole
 // length of a tile.  Rows of 128x128 tiles if so, else 0.  The line: after two (or four) big tiles per CU up to two small ones each (all of
-// them resident at once), after one or three to seven one small one each.  us, 128x128 | mixed:
+// them resident at once), otherwise one small one each.  us, 128x128 | mixed:
 //   768 wide, K = 3072: 5504 rows (258 tiles) 39.8 | 32.0, 6144 (288) 42.2 | 33.5, 12288 (576) 72.4 | 61.9; K = 768: 2048x2304 (288)
 //   15.4 | 11.5, 12288x768 23.2 | 21.6; K = 1536: 11008 rows (516) 41.2 | 32.8, 13312 (624) 38.8 | 35.3, 22016 (1032) 63.0 | 56.3;
 //   11008x2304x768 (1548) 50.6 | 45.9; 4224x1024x4096 (264) 52.1 | 43.0.
 // Beyond it: 13824x768x1536 (648 tiles) 38.8 | 39.0, 15360 (720) 39.4 | 42.5, 8192x768x3072 (384) 43.5 | 47.5, 24576x768x1536 (1152)
-// 61.7 | 61.8, 11264x3072x768 (2112) 63.0 | 62.3.
-// After three, five and seven, where half of the slots go on with a big tile, one small one each as well, for rows of K up to 8192.
+// 61.7 | 61.8, 11264x3072x768 (2112, behind eight) 63.0 | 62.3.
+// After three, five and so on, where half of the slots go on with a big tile, for rows of K up to 8192 only.
 // Behind three 17024x768x768 (798) 28.3 | 27.2, with the GELU backward 40.7 | 36.1, x3072 84.1 | 77.3, 7680x1600x1600 (780) 47.4 | 44.6, 8064x1600x6400
 // (819, 208 small) 160.9 | 158.8, 13312x1024x4096 (832, 256 small) 111.1 | 108.9, 17408x768x8192 208 | 195, x96 12.9 | 12.3; behind five 27648x768x1536 (1296) 73.5 |
 // 67.3, 5376x4096x1024 (1344, 256 small) 55.3 | 52.8; behind seven 38400x768x768 (1800) 58.7 | 54.3, 9600x3072x768 (1800)
@@ -1626,11 +1626,14 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 // Up to two small ones each also behind four where a small tile is long enough: 23168x768x3072 (1086, 264 small) 123.2 | 115.2, 24192x768x3072
 // (1134, 456) 124.4 | 120.8, 10752x1600x1600 (1092, 312) 69.7 | 66.1, 11136x1600x6400 (1131, 468) 244.7 | 231.1, 5888x3072x1536 (1104, 384) 66.7 | 66.2; K = 768
 // 24192 rows 39.8 | 41.4, 5760x3072 (288 small) 40.5 | 40.1; behind six 34560x768x1536 (336) 93.9 | 93.4, 16128x1600x1600 (416) 95.4 | 98.6.
+// With more rounds the gain falls slowly: behind eight 11008x3072x768 (2064) 68.2 | 63.8, 20608x1600x6400 (2093) 409 | 405, nine 12544x3072x3072 (2352) 235 | 220,
+// ten 13696x3072x1600 (2568) 146.3 | 136.6, twelve 16512x3072x768 (3096) 90.8 | 86.5, sixteen 21888x3072x3072 (4104) 401 | 382.
 static int mixed_big_rows(int M, int N, int K)
 {
     const int rows = (M + 127) / 128, tiles_n = (N + 127) / 128, cus = cu_count();
     if (K > TABLE_KB * QB) return 0;
-    for (int rounds = 1; rounds <= 7; rounds++) {              // big tiles per CU
+    const int last = (int)((long)rows * tiles_n / cus);
+    for (int rounds = last > 3 ? last - 2 : 1; rounds <= last; rounds++) {      // big tiles per CU
         if (rounds >= 3 && rounds % 2 && K > 8192) continue;
         const bool two = rounds == 2 || (rounds == 4 && K >= 1536 && K <= 8192);
         const int big = rounds * cus / tiles_n;

@@ -743,10 +743,10 @@ def test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K):
 
 
 # behind three big tiles per CU one row block of small ones, columns that end inside a tile; as many as CUs, and one row block more (128x128 only);
-# behind five the fewest and the most; behind seven; behind four close to two per CU, and one row block more
-@pytest.mark.parametrize("M,N,K", [(16416, 736, 160), (13312, 1024, 32), (13344, 1024, 32), (27296, 768, 32), (5376, 4096, 96), (7328, 4096, 32),
+# behind five the fewest and the most; behind seven and nine; behind four close to two per CU, and one row block more
+@pytest.mark.parametrize("M,N,K", [(16416, 736, 160), (13312, 1024, 32), (13344, 1024, 32), (27296, 768, 32), (5376, 4096, 96), (7328, 4096, 32), (12320, 3072, 32),
                                    (6048, 3072, 1536), (6080, 3072, 1536)])
-def test_two_tile_sizes_behind_three_to_seven(jf, oracle, M, N, K):
+def test_two_tile_sizes_behind_three_and_more(jf, oracle, M, N, K):
     test_two_tile_sizes_in_one_launch(jf, oracle, M, N, K)
     test_quantised_with_residual_addition(jf, oracle, M, N, K, torch.bfloat16, torch.float32, True, True)
 
