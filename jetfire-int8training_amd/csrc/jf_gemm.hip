@@ -293,7 +293,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         s_step = (unsigned)(KB_STAGE * ks) * (unsigned)sizeof(ST);
     }
     // WBM = 1: all of a block's products at once, before the main loop, into a table of the wave: lane l those of the K blocks l,
-    // l + 64, ...
+    // l + 64, ...  (SPLIT: a table of the block, which its waves fill and read together)
     constexpr bool TABLE = WBM == 1;
     float *const table = reinterpret_cast<float *>(smem + (SPLIT > 1 ? 0 : NSTAGE * STAGE_BYTES)) + wave * ((nkb + KB_STAGE - 1) / KB_STAGE * KB_STAGE + KB_STAGE);
     auto make_table = [&] {
@@ -653,8 +653,13 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
     };
     using c0 = std::integral_constant<int, 0>;
     if constexpr (TABLE) {
-        if (!loader) make_table();
-        else if (SPLIT > 1) wait_behind(SPLIT_RING < nstages ? SPLIT_RING - 1 : nstages - 1);
+        if (!loader) {
+            make_table();
+            if constexpr (SPLIT > 1) {                         // the waves of a block share its table: each one's part is written before the barrier
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+            }
+        } else if (SPLIT > 1) wait_behind(SPLIT_RING < nstages ? SPLIT_RING - 1 : nstages - 1);
         else wait_stage(NSTAGE - 1, std::integral_constant<int, NSTAGE - 1>{});           // stage 0 has landed
         if constexpr (EPI == EPI_QA) { if (!loader && m0 + wm * QB < p.M && n0 + wn * QB < p.N) fetch_x1(0); }
     } else {

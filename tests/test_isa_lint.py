@@ -4,7 +4,8 @@ The scale-accumulate MFMA of csrc/jf_gemm.hip is written as inline asm (its accu
 constant), so the compiler's hazard recogniser does not know it is an MFMA.  A vector instruction that reads or
 writes an MFMA's destination registers needs up to 19 wait states after the MFMA issues; the kernel guarantees
 them by program order (the result is consumed one accumulation later).  This test compiles the file to assembly
-and verifies that guarantee for every such MFMA in every instantiation, and that neither these kernels nor those of
+and verifies that guarantee for every such MFMA in every instantiation, that the table of scale products which two waves
+fill together is written before the barrier behind it, and that neither these kernels nor those of
 csrc/jf_attention.hip spill in their main loops."""
 import os
 import re
@@ -76,6 +77,61 @@ def test_asm_mfma_results_are_not_touched_too_early(gemm_isa):
             assert not (_regs(t) & dst), f"line {i + 1}: {code.strip()!r} -> line {j}: {t!r} touches its destination"
             ws += 1
     assert found >= 16, "the scale-accumulate MFMAs were not found (did the kernel change?)"
+
+
+def _functions(lines):
+    """(number of the first line, the instructions and labels) of every function."""
+    start = None
+    for i, line in enumerate(lines):
+        if re.match(r"_Z\w+:", line):
+            start = i + 1
+        elif start is not None and line.startswith(".Lfunc_end"):
+            yield start + 1, [t.split(";")[0].strip() for t in lines[start:i]]
+            start = None
+
+
+def _successors(body):
+    label = {t[:-1]: i for i, t in enumerate(body) if t.endswith(":")}
+    out = []
+    for i, t in enumerate(body):
+        assert not t.startswith(("s_setpc", "s_swappc", "s_call")), t
+        m = re.match(r"s_(c?)branch\w*\s+(\S+)", t)
+        out.append(([label[m.group(2)]] if m else []) + ([i + 1] if not t.startswith(("s_branch", "s_endpgm")) and i + 1 < len(body) else []))
+    return out
+
+
+def _barriers_behind_pending_table_writes(lines):
+    """Number of the kernels whose blocks two waves share (they alone use v_mfma_i32_16x16x32_i8), and the lines of the barriers that
+    one of a block's waves can reach while its writes to their common table of scale products are outstanding.  The factors of that
+    table, and of no other, are negated: times -2^26, 0xcc800000.  A barrier does not wait for LDS writes, and those of different waves
+    are not kept in order: without lgkmcnt(0) in front of it the other wave may read what was there before."""
+    kernels, bad = 0, []
+    for at, body in _functions(lines):
+        if not any("v_mfma_i32_16x16x32_i8" in t for t in body):
+            continue
+        kernels += 1
+        writes = []
+        for i, t in enumerate(body):
+            m = re.match(r"v_mul_f32\S* (v\d+), 0xcc800000, ", t)
+            if m:
+                assert re.match(r"ds_write_b32 v\d+, %s$" % m.group(1), body[i + 1]), f"line {at + i}: a factor of the table goes elsewhere"
+                writes.append(i + 1)
+        assert writes, f"line {at}: the table's writes were not found (did the kernel change?)"
+        succ, seen, todo = _successors(body), set(), [i + 1 for i in writes]
+        while todo:
+            i = todo.pop()
+            if i in seen or re.match(r"s_waitcnt .*lgkmcnt\(0\)", body[i]):
+                continue
+            seen.add(i)
+            todo += succ[i]
+        bad += [at + i for i in sorted(seen) if body[i].startswith("s_barrier")]
+    return kernels, bad
+
+
+def test_tables_of_two_waves_are_written_before_the_barrier(gemm_isa):
+    kernels, bad = _barriers_behind_pending_table_writes(gemm_isa)
+    assert kernels >= 14, "the kernels whose blocks two waves share were not found"
+    assert not bad, f"barriers with LDS writes of the shared table outstanding: lines {bad}"
 
 
 def _no_scratch_in_loops(lines):
