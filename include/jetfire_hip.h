@@ -361,7 +361,8 @@ int jf_attention_fwd_q(const void *q, const void *k, const void *v, int ld, int 
 
 
 /* Its gradients: gq, gk, gv ([B*T, ldg], laid out like q, k, v) from gout [B*T, H*D] and the forward's out and lse.
- * delta: [B*H, T] fp32 scratch.  Every sum has one owner and a fixed order: the same bits on every run. */
+ * delta: [B*H, T] fp32 scratch.  Every sum has one owner and a fixed order: the same bits on every run.  gq may be out, and each of gk and gv
+ * one of out, k and v, where their rows lie alike; no other result overlaps an operand. */
 int jf_attention_bwd(const void *q, const void *k, const void *v, int ld, const void *out, const void *gout, const float *lse,
                      int B, int H, int T, int D, float scale, void *gq, void *gk, void *gv, int ldg, float *delta,
                      jf_stream_t stream);

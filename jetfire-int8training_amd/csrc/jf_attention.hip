@@ -615,6 +615,8 @@ template <int D, bool QUANT> __global__ __launch_bounds__(64 * NW, 2) void attn_
 // 115.7, 36 of 1024 (288) 48.7 | 37.1, 48 of 1024 (384) 51.0 | 46.6, 96 of 512 (384) 34.9 | 31.9; beyond one and a half per CU 60 of 1024 (480)
 // 57.6 | 57.8, 144 of 416 (576) 36.6 | 37.2, 144 of 1024 (1152) 106.0 | 117.5, 200 of 1024 (1600) 141.7 | 158.8.  In a training step (three blocks 768 wide, 288 and
 // 384 workgroups) 1156 | 1114, 1293 | 1259, with 8 x 512 tokens 1225 | 1212.
+// Every operand is read to the end by one half or the other, so a gradient that lies on an operand (dQ on out, dK and dV on out, k or v: what the two
+// launches allow) takes the two launches.
 template <int D, bool QUANT> __global__ __launch_bounds__(64 * NW, 2) void attn_grad_kernel(AttnArgs a)
 {
     __shared__ __attribute__((aligned(16))) unsigned char smem[4 * TileIO<D>::TILE + DKV_STAT + OWN_ROWS * 4];
@@ -640,10 +642,24 @@ static void attn_launch(void (*kernel)(AttnArgs), const AttnArgs &a, hipStream_t
     const unsigned grid = 8u * ((a.B * a.H + 7) / 8) * ((a.T + WG_ROWS - 1) / WG_ROWS);
     hipLaunchKernelGGL(kernel, dim3(parts * grid), dim3(64 * NW), 0, st, a);
 }
+// Whether a result of the gradient kernels lies on one of their operands (as ranges of memory: two columns of one matrix count).
+static bool attn_grad_overlaps(const AttnArgs &a, int D)
+{
+    const size_t rows = (size_t)a.B * a.T, C = (size_t)a.H * D, row = a.H * sizeof(float) * rows;
+    struct Range { const void *p; size_t n; };
+    const auto matrix = [&](const half_t *p, int ld) { return Range{p, p ? ((rows - 1) * ld + C) * sizeof(half_t) : 0}; };
+    const Range in[] = {matrix(a.q, a.ld), matrix(a.k, a.ld), matrix(a.v, a.ld), matrix(a.o, (int)C), matrix(a.go, (int)C), {a.lse, row}};
+    const Range out[] = {matrix(a.gq, a.ldg), matrix(a.gk, a.ldg), matrix(a.gv, a.ldg), {a.delta, row},
+                         {a.cq, a.cq ? rows * 3 * C : 0}, {a.cs, a.cq ? rows / QB * (3 * C / QB) * sizeof(half_t) : 0}};
+    for (const Range &x : out)
+        for (const Range &y : in)
+            if ((uintptr_t)x.p < (uintptr_t)y.p + y.n && (uintptr_t)y.p < (uintptr_t)x.p + x.n) return true;
+    return false;
+}
 template <int D, bool QUANT> static void attn_launch_grad(const AttnArgs &a, hipStream_t st)
 {
     const long wgs = (long)a.B * a.H * ((a.T + WG_ROWS - 1) / WG_ROWS), cus = cu_count();
-    if (2 * wgs <= 3 * cus && a.T <= OWN_ROWS) return attn_launch(attn_grad_kernel<D, QUANT>, a, st, 2);   // (see the kernels)
+    if (2 * wgs <= 3 * cus && a.T <= OWN_ROWS && !attn_grad_overlaps(a, D)) return attn_launch(attn_grad_kernel<D, QUANT>, a, st, 2);   // (see the kernels)
     const bool alone = wgs <= cus;
     attn_launch(alone ? attn_dq_kernel<D, QUANT, true> : attn_dq_kernel<D, QUANT, false>, a, st);
     attn_launch(attn_dkv_kernel<D, QUANT>, a, st);

@@ -198,3 +198,29 @@ def test_both_gradients_in_one_launch(B, H, T, D, copies):
                             g.repeat(copies, 1), copies * B, H)
     for part in many.split(B * T):
         assert torch.equal(part, grads)
+
+
+# gradients that lie where operands were (the kernels of one launch read those to the end) or between the columns of the operands' matrix
+@pytest.mark.parametrize("B,H,T,D", [(1, 1, 32, 64), (3, 4, 416, 64), (2, 16, 1024, 32)])
+def test_gradients_in_the_place_of_operands(jf, B, H, T, D):
+    import BlockQuantizeCUDA as BQC
+    C, p = H * D, jf._ptr
+    print(f"case B={B} H={H} T={T} D={D}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    wide = torch.randn(B * T, 6 * C, device="cuda", generator=gen).half()
+    g = (torch.randn(B * T, C, device="cuda", generator=gen) * 1e-2).half()
+    q, k, v = (wide[:, i * C:(i + 1) * C].contiguous() for i in range(3))
+    out, lse = BQC.jetfire.attention_fwd(q, k, v, B, H)
+    want = BQC.jetfire.attention_bwd(q, k, v, out, lse, g, B, H)
+    delta = torch.empty(B * H, T, device="cuda")
+
+    def bwd(q, k, v, ld, out, gq, gk, gv, ldg):
+        jf.check(jf.lib().jf_attention_bwd(p(q), p(k), p(v), ld, p(out), p(g), p(lse), B, H, T, D, D ** -0.5, p(gq), p(gk), p(gv), ldg, p(delta), jf._stream()))
+        return torch.cat((gq, gk, gv), dim=1)
+
+    part = [wide[:, i * C:(i + 1) * C] for i in range(6)]
+    assert torch.equal(bwd(*part[:3], 6 * C, out, *part[3:], 6 * C), want)
+    o, spare = out.clone(), torch.empty_like(out)
+    assert torch.equal(bwd(q, k, v, C, o, spare, o, torch.empty_like(v), C), want)
+    o, kk, vv = out.clone(), k.clone(), v.clone()
+    assert torch.equal(bwd(q, kk, vv, C, o, o, vv, kk, C), want)
