@@ -1191,6 +1191,16 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
                           : TABLE ? reinterpret_cast<float *>(smem + gelu_lds_at(WBM, WGM, WGN, NSTAGE)) + wave * 256 : reinterpret_cast<float *>(scale_patch);
     int *const gelu_qtab = reinterpret_cast<int *>(gelu_tab);
     if (EPI == EPI_QG || EPI == EPI_QB) JF_WAIT_VMCNT(0);
+    if constexpr (EPI == EPI_QB && WBM == 2) {
+        // Read again (these kernels' first argument): held over the main loop they are scalar registers that it has to do without, and what
+        // it then parks in lanes costs the 64x128 tiles four vector instructions per K block.  us, held | read again: 1600x3680x1024 24.2 | 23.4,
+        // 2048x3072x768 20.4 | 20.0, 1664x3072x2048 33.6 | 32.8, 7040x768x3040 45.3 | 44.4.
+        typedef const __attribute__((address_space(4))) GemmArgs *KernelArgs;
+        KernelArgs again = (KernelArgs)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(again));
+        p.seed = again->seed; p.offset = again->offset; p.seed2 = again->seed2; p.offset2 = again->offset2;
+        p.rounding = again->rounding; p.rounding2 = again->rounding2; p.gelu_approx = again->gelu_approx;
+    }
     const float biasmax = (QUANT && p.biasmax) ? p.biasmax[0] : 0.0f;
     float gelu_f0 = 0.0f;                                     // gelu(+0), evaluated on the device like every table entry
     if (EPI == EPI_QG) {

@@ -80,13 +80,14 @@ def test_asm_mfma_results_are_not_touched_too_early(gemm_isa):
 
 
 def _functions(lines):
-    """(number of the first line, the instructions and labels) of every function."""
+    """(number of the first line, name, instructions and labels) of every function."""
     start = None
     for i, line in enumerate(lines):
-        if re.match(r"_Z\w+:", line):
-            start = i + 1
+        m = re.match(r"(_Z\w+):", line)
+        if m:
+            start, name = i + 1, m.group(1)
         elif start is not None and line.startswith(".Lfunc_end"):
-            yield start + 1, [t.split(";")[0].strip() for t in lines[start:i]]
+            yield start + 1, name, [t.split(";")[0].strip() for t in lines[start:i]]
             start = None
 
 
@@ -106,7 +107,7 @@ def _barriers_behind_pending_table_writes(lines):
     table, and of no other, are negated: times -2^26, 0xcc800000.  A barrier does not wait for LDS writes, and those of different waves
     are not kept in order: without lgkmcnt(0) in front of it the other wave may read what was there before."""
     kernels, bad = 0, []
-    for at, body in _functions(lines):
+    for at, _, body in _functions(lines):
         if not any("v_mfma_i32_16x16x32_i8" in t for t in body):
             continue
         kernels += 1
@@ -132,6 +133,31 @@ def test_tables_of_two_waves_are_written_before_the_barrier(gemm_isa):
     kernels, bad = _barriers_behind_pending_table_writes(gemm_isa)
     assert kernels >= 14, "the kernels whose blocks two waves share were not found"
     assert not bad, f"barriers with LDS writes of the shared table outstanding: lines {bad}"
+
+
+def _scalars_parked_in_main_loops(lines):
+    """Number of the loops over two stages of two blocks per wave (16 products) in kernels of one tile size, and the lines of those that write
+    scalar values to lanes of a vector register: four more vector instructions per K block cost 3 %."""
+    loops, bad = 0, []
+    for at, name, body in _functions(lines):
+        if "igemm_nt_kernel" not in name:
+            continue
+        label = {t[:-1]: i for i, t in enumerate(body) if t.endswith(":")}
+        for i, t in enumerate(body):
+            m = re.match(r"s_c?branch\w*\s+(\S+)", t)
+            if m and label[m.group(1)] < i:
+                loop = body[label[m.group(1)]:i]
+                if sum(t.startswith("v_mfma") for t in loop) == 16:
+                    loops += 1
+                    if any(t.startswith("v_writelane") for t in loop):
+                        bad.append(at + i)
+    return loops, bad
+
+
+def test_main_loops_park_no_scalars(gemm_isa):
+    loops, bad = _scalars_parked_in_main_loops(gemm_isa)
+    assert loops >= 60, "the main loops were not found"
+    assert not bad, f"scalar values written to lanes inside the loops that end at lines {bad}"
 
 
 def _no_scratch_in_loops(lines):
