@@ -50,7 +50,9 @@ template <> struct Load16<__bf16> {
 };
 
 // acc + p[0] + p[stride] + ... of n terms in ascending order, STEP of them on their way at once.  (A loop that the compiler unrolls leaves a
-// remainder that waits for every term by itself.  Absent terms count as +0, which changes no bit of a sum that starts from +0.)
+// remainder that waits for every term by itself.  Absent terms count as +0, which changes no bit of a sum that starts from +0.  The remainder
+// in four, eight or STEP: every term costs an addition in the chain, absent or not.  LayerNorm from 17 sums per row, us, in STEP | so: 768x544 4.84 | 4.60,
+// 1056x1056 5.00 | 4.82.)
 template <int STEP> __device__ __forceinline__ float sum_ascending(const float *p, int n, size_t stride)
 {
     float acc = 0.0f;
@@ -62,13 +64,17 @@ template <int STEP> __device__ __forceinline__ float sum_ascending(const float *
 #pragma unroll
         for (int i = 0; i < STEP; ++i) acc = acc + v[i];
     }
-    if (j < n) {
-        float v[STEP];
+    auto rest = [&](auto n_c) {
+        constexpr int N = decltype(n_c)::value;
+        float v[N];
 #pragma unroll
-        for (int i = 0; i < STEP; ++i) v[i] = p[(size_t)(j + i < n ? j + i : n - 1) * stride];
+        for (int i = 0; i < N; ++i) v[i] = p[(size_t)(j + i < n ? j + i : n - 1) * stride];
 #pragma unroll
-        for (int i = 0; i < STEP; ++i) acc = acc + (j + i < n ? v[i] : 0.0f);
-    }
+        for (int i = 0; i < N; ++i) acc = acc + (j + i < n ? v[i] : 0.0f);
+    };
+    if (n - j > 8) rest(std::integral_constant<int, STEP>{});
+    else if (n - j > 4) rest(std::integral_constant<int, 8>{});
+    else if (n - j > 0) rest(std::integral_constant<int, 4>{});
     return acc;
 }
 
@@ -542,7 +548,7 @@ void gelu_bwd_kernel(const int8_t *qx, const ST *sx, const int8_t *qg, const ST 
 // XCD fetched all rows' sums into its L2; with a row group's workgroups on one XCD each fetches an eighth.  us, plain order | runs per
 // XCD: 8192x1600 15.0 | 12.3 (8.4 without the sums), 12288x768 9.15 | 8.68; 4096x1024 (512 workgroups) 5.18 | 5.15, 1024x256 4.12 | 4.27:
 // few workgroups keep the plain order.  (24 or 32 terms on their way at once instead of 16 cost registers: 8192x1600 14.1 and 16.1.)  The
-// last ones, up to 15, at once as well: 1248x768 4.66 -> 4.22, 256x864 4.75 -> 4.10, 12288x768 8.62 -> 8.27, 8192x1600 11.9 -> 12.0.
+// last ones, up to 15, together as well: 1248x768 4.66 -> 4.22, 256x864 4.75 -> 4.10, 12288x768 8.62 -> 8.27, 8192x1600 11.9 -> 12.0.
 constexpr int CW_ROWS = 2;
 struct RowSums {
     const float *rowsum, *rowsq;

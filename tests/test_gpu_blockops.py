@@ -554,6 +554,12 @@ def test_layernorm_from_partial_row_sums_with_a_run_per_xcd(jf, oracle, R, C):
     test_layernorm_from_partial_row_sums(jf, oracle, R, C, True, True)
 
 
+# sums of 16 terms and a remainder of none, up to four, up to eight, up to fifteen; of a remainder alone
+@pytest.mark.parametrize("terms", [4, 8, 9, 15, 16, 17, 20, 21, 24, 25, 31])
+def test_layernorm_from_any_number_of_partial_sums(jf, oracle, terms):
+    test_layernorm_from_partial_row_sums(jf, oracle, 64, 32 * terms, True, True)
+
+
 def test_results_are_seen_by_a_dispatch_mode():
     """Results are allocated without the dispatcher, except where something listens to it; the values do not depend on it."""
     from Nonlinear import int8_quantize
