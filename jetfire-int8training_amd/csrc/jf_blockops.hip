@@ -1415,7 +1415,8 @@ using namespace jf;
 
 // mean and 1/sqrt(variance) of every row from its per-32-column partial sums (rowsum, rowsq: [parts][R], what add_kernel
 // leaves): the partials are added in ascending order, var = E[y^2] - mean^2, no epsilon (add_mean_var.py:219-221).  A thread's requests, up to eight
-// of either array, go out together: one after the other | so, us: 8192x1600 3.45 | 3.0, 96x4096 5.1 | 3.8, 12288x768 2.75 | 2.8.
+// of either array, go out together: one after the other | so, us: 8192x1600 3.45 | 3.0, 96x4096 5.1 | 3.8.  Up to two where
+// there are no more, the code of the others is only passed over: 32x192 in rounds of eight 3.10, of two 2.77 (one after the other 2.79).
 constexpr int RSF_ROWS = 32;                       // rows per workgroup
 __global__ __launch_bounds__(256) void rowstats_finish_kernel(const float *rowsum, const float *rowsq, int R, int parts,
                                                               float n, float *mean, float *rstd)
@@ -1427,21 +1428,26 @@ __global__ __launch_bounds__(256) void rowstats_finish_kernel(const float *rowsu
     const int rows = (R - r0) < RSF_ROWS ? (R - r0) : RSF_ROWS;
     const int count = parts * RSF_ROWS;
     const int r_in = threadIdx.x % RSF_ROWS, from = r0 + (r_in < rows ? r_in : 0);
-    for (int j0 = threadIdx.x / RSF_ROWS; j0 < parts; j0 += 64) {     // 64 parts at once, eight of each array on their way per thread
-        float v[8], w[8];
+    auto take = [&](auto n_c) {                                       // 8 N parts at once, N of each array on their way per thread
+        constexpr int N = decltype(n_c)::value;
+        for (int j0 = threadIdx.x / RSF_ROWS; j0 < parts; j0 += 8 * N) {
+            float v[N], w[N];
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (j0 + 8 * i < parts) {
-                const size_t at = (size_t)(j0 + 8 * i) * R + from;
-                v[i] = rowsum[at]; w[i] = rowsq[at];
-            }
+            for (int i = 0; i < N; ++i)
+                if (j0 + 8 * i < parts) {
+                    const size_t at = (size_t)(j0 + 8 * i) * R + from;
+                    v[i] = rowsum[at]; w[i] = rowsq[at];
+                }
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (j0 + 8 * i < parts) {
-                rsf_lds[(j0 + 8 * i) * RSF_ROWS + r_in] = v[i];
-                rsf_lds[count + (j0 + 8 * i) * RSF_ROWS + r_in] = w[i];
-            }
-    }
+            for (int i = 0; i < N; ++i)
+                if (j0 + 8 * i < parts) {
+                    rsf_lds[(j0 + 8 * i) * RSF_ROWS + r_in] = v[i];
+                    rsf_lds[count + (j0 + 8 * i) * RSF_ROWS + r_in] = w[i];
+                }
+        }
+    };
+    if (parts <= 16) take(std::integral_constant<int, 2>{});
+    else take(std::integral_constant<int, 8>{});
     __syncthreads();
     const int row = threadIdx.x & (RSF_ROWS - 1), which = threadIdx.x / RSF_ROWS;     // which: 0 = sums, 1 = squares
     float acc = 0.0f;

@@ -270,8 +270,8 @@ def test_quantising_more_row_blocks_than_a_grid_dimension_holds(jf):
         assert torch.equal(q[:rows], qp) and torch.equal(s[:rows // 32], sp)
 
 
-# parts of one and of several requests per thread, a last round of eight that is not full, more than 64; rows that end inside a workgroup
-@pytest.mark.parametrize("R,parts", [(32, 1), (40, 8), (96, 9), (64, 63), (72, 64), (32, 65), (33, 131)])
+# parts of one and of two requests per thread, of up to eight, a last round of eight that is not full, more than 64; rows that end inside a workgroup
+@pytest.mark.parametrize("R,parts", [(32, 1), (40, 8), (96, 9), (40, 16), (32, 17), (64, 63), (72, 64), (32, 65), (33, 131)])
 def test_finishing_the_row_sums(jf, R, parts):
     rng = np.random.default_rng(R + parts)
     rs, rq = rng.standard_normal((parts, R)).astype(np.float32), (rng.random((parts, R)) * 1000).astype(np.float32)
