@@ -1971,6 +1971,9 @@ template <int EPI, typename ST, int TILE, bool SMALL_W = false> static int launc
 // turn of those is 0.1 us per K block where a 128x128 tile alone on its CU takes 0.27.  us, 128x128 | 32x128: 480x736x160 8.6 | 5.5, 512x512x512
 // 8.7 | 5.6, 64x256x256 4.8 | 4.3, 480x192x2080 8.9 | 8.4, and with K splits 1024x256x1024 11.7 | 9.1, 4096x128x512 12.9 | 9.9; two per CU
 // 256x1024x1024 7.3 | 8.6, 512x1024x1024 9.7 | 11.2, 2048x256x768 12.4 | 13.8.
+// The activation gradient in 32x64 tiles beside 128x128 ones where its chain over K is the longer one: at three times as many K blocks 32x128 tiles
+// (218 cycles each) and the weight gradients (0.27 us) take equally long.  32x128 | 32x64: 800x256x3680 16.8 | 13.1, 576x448x2304 12.4 | 11.0, 480x416x2304 12.1 |
+// 10.0, 1024x256x2080 15.3 | 13.9, 1088x256x2016 15.0 | 14.1; not beyond the line 352x992x1056 9.2 | 9.6, 480x672x1024 9.8 | 10.1, 64x5120x192 6.15 | 6.26.
 // Above three 128x128 tiles of the activation gradient per CU the rounds even out by themselves: 4096x4096x1024 (1024) 86.1 | 83.7,
 // 8192x1600x4800 (832) 248.7 | 263.2, 8192x6400x1600 (3200) 359.4 | 363.9, 4096x4096x4096 (1024) 259.0 | 260.8.
 static bool backward_in_one_launch(int R, int C_in, long w_wgs)
@@ -1990,7 +1993,7 @@ template <int EPI, typename ST> int launch_backward_any(const GemmArgs &x, const
         if (narrow + small_w <= cus) return launch_backward<EPI, ST, TILE_32x64, true>(x, w, w_wgs, k_per_part, st);
         if (wide + small_w <= cus) return launch_backward<EPI, ST, TILE_32x128, true>(x, w, w_wgs, k_per_part, st);
     }
-    if (split_tiles_resident(x.M, x.N, x.K) && split_tiles(x.M, x.N) + w_wgs <= cu_count())
+    if (x.K > 3 * k_per_part && split_tiles_resident(x.M, x.N, x.K) && split_tiles(x.M, x.N) + w_wgs <= cu_count())
         return launch_backward<EPI, ST, TILE_32x64>(x, w, w_wgs, k_per_part, st);
     const bool small = small_tiles_resident(x.M, x.N, x.K) && (x.K > 2048 || (long)(x.M / QB) * ((x.N + 127) / 128) <= cu_count());
     if (small) return launch_backward<EPI, ST, TILE_32x128>(x, w, w_wgs, k_per_part, st);

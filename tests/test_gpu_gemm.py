@@ -686,8 +686,9 @@ def test_gelu_in_the_64_row_tiles(jf, oracle, M, N, K):
 
 # weight gradients in 32x128 tiles beside the activation gradient, up to one workgroup per CU (256): columns of the gradient that end inside a staged
 # line, every length of the last stage, K splits with a short last part; 256 workgroups with 32x64 tiles of the activation gradient, one row of tiles
-# more (its 32x128 tiles), and too many for either
-@pytest.mark.parametrize("R,C_in,C_out", [(r, 160, 288) for r in (32, 64, 96, 128, 160, 288, 416)] + [(1056, 128, 256), (2048, 96, 544), (480, 512, 1088), (480, 512, 1120), (480, 512, 2080)])
+# more (its 32x128 tiles), and too many for either (128x128 beside 32x64 tiles); three times as many K blocks of the activation gradient as of the weight
+# gradient (128x128 beside 32x128) and one more (beside 32x64)
+@pytest.mark.parametrize("R,C_in,C_out", [(r, 160, 288) for r in (32, 64, 96, 128, 160, 288, 416)] + [(1056, 128, 256), (2048, 96, 544), (480, 512, 1088), (480, 512, 1120), (480, 512, 2080), (352, 992, 1056), (352, 992, 1088)])
 def test_weight_gradients_in_tiles_of_32_rows(jf, R, C_in, C_out):
     test_both_gradients_of_a_linear_layer_in_one_launch(jf, R, C_in, C_out, 0, True, True)
     test_both_gradients_of_a_linear_layer_in_one_launch(jf, R, C_in, C_out, 1, False, False)
