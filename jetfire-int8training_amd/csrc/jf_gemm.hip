@@ -1861,7 +1861,11 @@ static bool split_tiles_resident(int M, int N, int K) { return K <= TABLE_KB * Q
 // each.  Both put two waves that multiply on a SIMD, but this one loads 6 KB per K block instead of 10, and what a CU can load is what
 // two workgroups of 32x128 wait for.  us, 32x128 | these: 2048x768x768 7.25 | 6.98, x3072 16.6 | 15.7, 864x1824x3200 (210) 17.5 | 15.9, B as [K,N] 21.0 | 17.5,
 // 640x3072x1600 (240) 12.3 | 10.9, 1024x2048x3200 (256) 19.9 | 17.9, 1664x768x768 (156) 7.19 | 6.64, 4128x256x768 (130) 7.08 | 6.78, 1056x1024x96 (136)
-// 4.62 | 4.51, x3072 15.7 | 16.0.  A ring three deep instead of two: 2048x768x768 7.00, x3072 16.6, 1024x2048x3200 18.7.
+// 4.62 | 4.51.  A ring three deep instead of two: 2048x768x768 7.00, x3072 16.6, 1024x2048x3200 18.7.  Over 3400 drawn sizes these are 5 % faster,
+// 2 to 4 % for K up to 256, 5 to 8 % above 512.  Single long rows lose with no size, pitch or layout that tells them from their neighbours: 1056x1024x6240 with B as
+// [K,N] 30.1 | 33.6, 3328x288x4416 22.0 | 25.6, but 1056x1024x3072 16.5 | 16.4, 1024x1600x6400 7 % and 544x1984x5600 5 % faster; 34 of the 3400 by more than 2 %.
+// Short rows stay with 32x128 where the epilogue is a large part: float results up to K = 256 (2048x544x256 5.7 | 6.0, 1024x1088x224 3 % slower), the
+// GELU backward up to 128 (1664x544x128 2.5 % slower).
 static bool tall_tiles_resident(int M, int N, int K)
 {
     const long cus = cu_count(), cols = (N + 127) / 128;
@@ -1885,7 +1889,7 @@ template <int EPI, typename ST, int BKN> static int launch_gemm_b(const GemmArgs
 {
     if constexpr (EPI != EPI_S32) {
         if constexpr (EPI != EPI_FP) { if (split_tiles_resident(a.M, a.N, a.K)) return launch_gemm_split<EPI, ST, BKN>(a, st); }
-        if (a.splits <= 1 && tall_tiles_resident(a.M, a.N, a.K))
+        if (a.splits <= 1 && a.K > (EPI == EPI_FP ? 256 : EPI == EPI_QB ? 128 : 0) && tall_tiles_resident(a.M, a.N, a.K))
             return launch_gemm_cfg<EPI, ST, 1, 2, 4, 2, 1, BKN>(a, st);
         if (a.splits <= 1 && small_tiles_resident(a.M, a.N, a.K))
             return launch_gemm_cfg<EPI, ST, 1, 1, 4, 3, 2, BKN>(a, st);
