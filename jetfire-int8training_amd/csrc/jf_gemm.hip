@@ -661,7 +661,7 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
             }
         } else if (SPLIT > 1) wait_behind(SPLIT_RING < nstages ? SPLIT_RING - 1 : nstages - 1);
         else wait_stage(NSTAGE - 1, std::integral_constant<int, NSTAGE - 1>{});           // stage 0 has landed
-        if constexpr (EPI == EPI_QA) { if (!loader && m0 + wm * QB < p.M && n0 + wn * QB < p.N) fetch_x1(0); }
+        if constexpr (EPI == EPI_QA) { if (!loader && part == 0 && m0 + wm * QB < p.M && n0 + wn * QB < p.N) fetch_x1(0); }   // (the wave that goes on to the epilogue)
     } else {
         if (NSTAGE - 1 >= nstages) JF_WAIT_VMCNT(0);
         else JF_WAIT_VMCNT((NSTAGE - 1) * LOADS - (EPI != EPI_S32 ? 1 : 0));      // stage 0 and the scales of stage 1 have landed
