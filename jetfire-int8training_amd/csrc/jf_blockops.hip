@@ -1473,7 +1473,7 @@ __global__ __launch_bounds__(256) void rowstats_finish_kernel(const float *rowsu
 // 11.5 | 7.9), 1248x1536 7.2 | 10.2 | 6.1 (7.9 | 11.8 | 7.9); beyond the line 1024x128 5.4 | 3.6 | 3.7 (5.4 | 3.6 | 4.1), 1024x256 5.6 | 3.7 | 3.8 (5.5 | 3.9 | 4.1),
 // 1024x2048 7.4 | 12.7 | 7.3 (8.0 | 14.6 | 10.0), 4096x768 (320 workgroups) 7.9 | 7.4 | 7.1 (9.1 | 9.0 | 9.8), 8192x768 11.2 | 9.3 | 11.7 (14.8 | 12.1 | 16.5).
 // In strips where the row is narrow or the strips are many: 4096x256 6.0 | 4.1, 4096x1024 8.7 | 9.1 (11.2 | 10.4), 6144x1600 16.2 | 16.1 (21.1 | 18.5), 8192x1600 19.5 |
-// 17.7 (26.6 | 21.6); beyond 4096x1280 10.2 | 12.0 (12.7 | 14.2), 4096x2048 14.4 | 16.6 (18.1 | 20.1).
+// 17.7 (26.6 | 21.6); beyond 4096x1280 10.2 | 12.0 (12.7 | 14.2), 4096x2048 14.4 | 16.6 (18.1 | 20.1).  Either needs no workspace.
 static long add_beside_sums_workgroups(int R, int C) { return R / QB + ((long)(R / QB) * (C / QB) + ADS_WAVES - 1) / ADS_WAVES; }
 static bool add_beside_sums(int R, int C)
 {
@@ -1925,7 +1925,7 @@ int jf_add(const void *x1, int x1_dtype, const int8_t *q2, const void *s2, int R
 
 size_t jf_add_rowstats_workspace_bytes(int R, int C)
 {
-    if (R <= 0 || C <= 0 || add_in_strips(R, C)) return 0;
+    if (R <= 0 || C <= 0 || add_in_strips(R, C) || add_beside_sums(R, C)) return 0;
     return (size_t)2 * (C / QB) * R * sizeof(float);
 }
 
@@ -1938,9 +1938,9 @@ int jf_add_rowstats(const void *x1, int x1_dtype, const int8_t *q2, const void *
     if (!x1 || !y1 || !q || !s || !mean || !rstd) return JF_ERR_NULL;
     if (!rounding_ok(rounding) || x1_dtype < JF_FP_F16 || x1_dtype > JF_FP_BF16 || y1_dtype < JF_FP_F16 || y1_dtype > JF_FP_BF16) return JF_ERR_ENUM;
     if (!aligned16(x1) || !aligned16(y1) || !aligned16(q)) return JF_ERR_ALIGN;
-    const bool strips = add_in_strips(R, C);
     bool beside = add_beside_sums(R, C);
-    if (beside) {                                                  // (a workgroup reads what another one writes where a result lies on an operand)
+    const bool strips = beside || add_in_strips(R, C);
+    if (beside) {                                                  // (a workgroup reads what another one writes where a result lies on an operand: in strips then)
         const size_t n = (size_t)R * C, ns = n / (QB * QB) * (scale_dtype == JF_SCALE_F16 ? 2 : 4);
         const auto width = [](int t) -> size_t { return t == JF_FP_F32 ? 4 : 2; };
         const auto overlap = [](const void *a, size_t na, const void *b, size_t nb) {
@@ -1954,8 +1954,6 @@ int jf_add_rowstats(const void *x1, int x1_dtype, const int8_t *q2, const void *
     }
     if (!strips) {
         if (!workspace || !aligned16(workspace) || workspace_bytes < jf_add_rowstats_workspace_bytes(R, C)) return JF_ERR_WORKSPACE;
-    }
-    if (!strips && !beside) {
         float *const rowsum = (float *)workspace, *const rowsq = rowsum + (size_t)(C / QB) * R;
         rc = jf_add(x1, x1_dtype, q2, s2, R, C, scale_dtype, rounding, seed, offset, y1, y1_dtype, q, s, rowsum, rowsq, stream);
         return rc ? rc : jf_rowstats_finish(rowsum, rowsq, R, C / QB, C, mean, rstd, stream);
