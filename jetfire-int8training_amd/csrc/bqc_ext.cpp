@@ -20,12 +20,13 @@ void register_block(pybind11::module &m);           // jf_block_ext.cpp
 
 void thread_locals_up_to_date()
 {
-    static void (*const read)() = []() -> void (*)() {
+    using Read = const volatile char *(*)();
+    static const Read read = []() -> Read {
         Dl_info here;
         if (!dladdr(reinterpret_cast<void *>(&thread_locals_up_to_date), &here)) return nullptr;
         const std::string file(here.dli_fname);               // the extension's own: the library lies beside it
         void *lib = dlopen((file.substr(0, file.rfind('/') + 1) + "libjetfire_tls.so").c_str(), RTLD_NOW | RTLD_LOCAL);
-        return lib ? reinterpret_cast<void (*)()>(dlsym(lib, "jf_tls_read")) : nullptr;
+        return lib ? reinterpret_cast<Read>(dlsym(lib, "jf_tls_read")) : nullptr;
     }();
     if (read) read();
 }

@@ -1,7 +1,8 @@
-/* libjetfire_tls.so: one thread-local variable, see thread_locals_up_to_date() in bqc_common.h */
+/* libjetfire_tls.so: one thread-local variable, see thread_locals_up_to_date() in bqc_common.h.  Returns where the calling thread's lies. */
 static __thread volatile char here;
 
-void jf_tls_read(void)
+const volatile char *jf_tls_read(void)
 {
     (void)here;
+    return &here;
 }

@@ -57,14 +57,24 @@ def test_measurement_library_is_separate(jf):
 
 
 def test_the_thread_local_library_is_read_by_any_thread():
+    """Every thread has a variable of its own there."""
     import threading
     lib = ctypes.CDLL(os.path.join(ROOT, "jetfire-int8training_amd", "libjetfire_tls.so"))
-    threads = [threading.Thread(target=lib.jf_tls_read) for _ in range(4)]
+    lib.jf_tls_read.restype = ctypes.c_void_p
+    seen, all_there = [], threading.Barrier(4)
+
+    def read():
+        seen.append(lib.jf_tls_read())
+        all_there.wait(60)                                           # (alive together: the memory of a thread that ended is used again)
+
+    threads = [threading.Thread(target=read) for _ in range(4)]
     for t in threads:
         t.start()
     for t in threads:
         t.join()
-    lib.jf_tls_read()
+    seen.append(lib.jf_tls_read())
+    assert len(seen) == 5 and all(seen) and len(set(seen)) >= 4      # (this thread's may take the place of one that ended)
+    assert lib.jf_tls_read() == seen[-1]
 
 
 @pytest.mark.gpu

@@ -180,8 +180,8 @@ def test_scores_of_minus_infinity_count_for_nothing(D, keys):
 
 
 # both gradients in one launch (up to one and a half workgroups per CU, sequences of up to 4096 rows) against the two launches that many copies
-# of the same sequences take: one workgroup, waves without rows, ragged last tiles, the most workgroups, the longest sequence; and one row block more
-@pytest.mark.parametrize("B,H,T,D,copies", [(1, 1, 32, 64, 385), (1, 3, 96, 32, 130), (3, 4, 416, 64, 9), (3, 16, 1024, 64, 2), (2, 1, 4096, 32, 7), (1, 1, 4128, 64, 1)])
+# of the same sequences take: one workgroup, waves without rows, ragged last tiles, the most workgroups, the longest sequence
+@pytest.mark.parametrize("B,H,T,D,copies", [(1, 1, 32, 64, 385), (1, 3, 96, 32, 130), (3, 4, 416, 64, 9), (3, 16, 1024, 64, 2), (2, 1, 4096, 32, 7)])
 def test_both_gradients_in_one_launch(B, H, T, D, copies):
     import BlockQuantizeCUDA as BQC
     jf, C = BQC.jetfire, H * D
@@ -198,6 +198,25 @@ def test_both_gradients_in_one_launch(B, H, T, D, copies):
                             g.repeat(copies, 1), copies * B, H)
     for part in many.split(B * T):
         assert torch.equal(part, grads)
+
+
+def test_one_row_block_more_than_one_launch_takes():
+    """4128 rows take the two launches.  With no gradient behind row 4095 they return what the one launch returns for the first 4096 rows."""
+    import BlockQuantizeCUDA as BQC
+    jf, T, D = BQC.jetfire, 4128, 64
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    qkv = torch.randn(T, 3 * D, device="cuda", generator=gen).half()
+    g = (torch.randn(T, D, device="cuda", generator=gen) * 1e-2).half()
+    out, lse = jf.attention_fwd(*qkv.split(D, dim=1), 1, 1)
+    grads = jf.attention_bwd(*qkv.split(D, dim=1), out, lse, g, 1, 1)
+    want, want_g = reference(qkv, g, 1, 1, T, D)
+    assert rel(out, want) < 1e-3
+    for i in range(3):
+        assert rel(grads[:, i * D:(i + 1) * D], want_g[:, i * D:(i + 1) * D]) < 2e-3, i
+    g[4096:] = 0
+    long = jf.attention_bwd(*qkv.split(D, dim=1), out, lse, g, 1, 1)
+    short = jf.attention_bwd(*qkv[:4096].split(D, dim=1), out[:4096].contiguous(), lse.view(1, T)[:, :4096].contiguous(), g[:4096].contiguous(), 1, 1)
+    assert torch.equal(long[:4096], short) and not long[4096:, :D].any()
 
 
 # gradients that lie where operands were (the kernels of one launch read those to the end) or between the columns of the operands' matrix
