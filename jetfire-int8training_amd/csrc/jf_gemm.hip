@@ -907,9 +907,9 @@ __device__ __forceinline__ void igemm_body(const GemmArgs &p_in, const int logic
         });
     };
     // SPLIT.  With fewer blocks than SIMDs the vector ALU idles for half of table_loop: a wave alone on its SIMD issues every 4.1 cycles,
-    // and 32 vector instructions per K block in one chain are what the launch waits for.  Two or four waves share a block: each forms the
+    // and 32 vector instructions per K block in one chain are what the launch waits for.  Two waves share a block: each forms the
     // products of 16 rows and STRIPS x 16 columns (v_mfma_i32_16x16x32_i8: the same integers) and accumulates them in the same chain over
-    // K, 16 or 8 vector instructions per K block.  One turn per stage, and nothing unrolled beyond two of them: code that is executed once
+    // K, 16 vector instructions per K block.  One turn per stage, and nothing unrolled beyond two of them: code that is executed once
     // costs an instruction fetch per 64 bytes.
     constexpr int STRIPS = 2;
     auto split_loop = [&] {
@@ -1500,7 +1500,7 @@ template <typename ST, bool SMALL> __device__ __forceinline__ void wgrad_group_b
 }
 template <typename ST> __global__ __launch_bounds__(512, 4) void igemm_wgrad_group_kernel(GemmGroup grp) { wgrad_group_body<ST, false>(grp, blockIdx.x); }
 
-// An activation gradient (EPI_Q or EPI_QD, B as [K,N]; 32x128 or 128x128 tiles), then weight gradients, in one launch: both gradients of
+// An activation gradient (EPI_Q or EPI_QD, B as [K,N]; 32x64, 32x128 or 128x128 tiles), then weight gradients, in one launch: both gradients of
 // a linear layer, or the last one of a block with all of the block's weight gradients.
 enum BackwardTile { TILE_128x128, TILE_32x128, TILE_32x64 };   // of the activation gradient
 struct GemmBackward {
