@@ -134,8 +134,9 @@ inline int check_scales(const torch::Tensor &SX, const torch::Tensor &SW, const 
 // and the runtime read such variables in every allocation and launch: 12 to 14 % of the calling thread's time in launch-bound calls, 16 % of
 // autograd's.  So a library with one such variable (jf_tls.c) is loaded at the first launch, when the runtime has started, and read here by
 // every thread that launches.  Nothing else depends on it: where it cannot be loaded, or another library comes later, all goes the slow way
-// as before.  Host time, us, before | after: one linear layer 5.8 | 5.2, five launches of a linear layer in both directions 31.5 | 27.4, six Nonlinear operators
-// 47.6 | 40.5, a training step of two 256-wide blocks 431 to 476 | 297 to 425.
+// as before.  Host time of a pass, us, without it | with it, six processes of each in turn, like compared with like (processes fall into two groups): one
+// linear layer 5.0 | 4.35, a linear layer in both directions 28.0 | 24.5 and 33.7 | 30.7, six Nonlinear operators 44.6 | 37.4 and 52.5 | 46.6, a training step of
+// two 256-wide blocks 461 | 419.
 void thread_locals_up_to_date();
 
 // The stream that a kernel on `t` is launched on; asked for once per operator.

@@ -1636,7 +1636,7 @@ static int launch_gemm_cfg(const GemmArgs &a, hipStream_t st)
 // Behind three 17024x768x768 (798) 28.3 | 27.2, with the GELU backward 40.7 | 36.1, x3072 84.1 | 77.3, 7680x1600x1600 (780) 47.4 | 44.6, 8064x1600x6400
 // (819, 208 small) 160.9 | 158.8, 13312x1024x4096 (832, 256 small) 111.1 | 108.9, 17408x768x8192 208 | 195, x96 12.9 | 12.3; behind five 27648x768x1536 (1296) 73.5 |
 // 67.3, 5376x4096x1024 (1344, 256 small) 55.3 | 52.8; behind seven 38400x768x768 (1800) 58.7 | 54.3, 9600x3072x768 (1800)
-// 56.7 | 54.4, 17920x1600x6400 (1820) 344.9 | 336.4, 18048x1600x256 (1833, 208 small) 29.8 | 30.3.  A longer row: 8064x1600x12800 313 | 322.  More than one
+// 56.7 | 54.4, 17920x1600x6400 (1820) 344.9 | 336.4, 18048x1600x256 (1833, 208 small) 30.2 | 28.4.  A longer row: 8064x1600x12800 313 | 322.  More than one
 // small tile each: 8192x1600x1600 (832 tiles, 260 small) 49.7 | 53.2, x4800 126.6 | 130.9, 13184x1600x1600 (1339, 260) 76.9 | 76.4.
 // Up to two small ones each also behind four where a small tile is long enough: 23168x768x3072 (1086, 264 small) 123.2 | 115.2, 24192x768x3072
 // (1134, 456) 124.4 | 120.8, 10752x1600x1600 (1092, 312) 69.7 | 66.1, 11136x1600x6400 (1131, 468) 244.7 | 231.1, 5888x3072x1536 (1104, 384) 66.7 | 66.2; K = 768
